@@ -1,10 +1,10 @@
 // True float32 matrix product C[M,N] = A[M,K] * B[N,K]^T (+ bias[N]), both
 // operands K-contiguous (activations times a weight in [out, in] layout).
-// Plain FMA on the vector ALU, float32 accumulation in a fixed K order that
-// does not depend on M: no matrix-core instruction, so no reduced-precision
-// mode can slip in.  64x64 output tile per block of 256 threads, K in steps
-// of 16 through LDS; any M, N, K.  Up to 16 rows of A with K a multiple of four take a
-// weight-streaming variant (below) instead.
+// float32 products and float32 accumulation throughout, in an order that depends
+// on K alone within a variant.  Up to 16 rows of A (64 where K is 1,024 or more) stream the
+// weight past registers on the vector ALU; more rows are tiled on the matrix cores'
+// float32 instruction, whose products and sums are not rounded to anything narrower;
+// operands that are not 16-byte aligned rows take the plain 64x64 tile.
 #include "common.h"
 #include <algorithm>
 
@@ -26,8 +26,6 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(
   // loader: thread -> (row = tid / 4, k quad = tid % 4)
   const int lrow = tid / 4;
   const int lk = (tid % 4) * 4;
-  const bool vec_ok = (K % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) &&
-                      ((((uintptr_t)A) & 15) == 0) && ((((uintptr_t)B) & 15) == 0);
 
   float acc[4][4];
 #pragma unroll
@@ -43,23 +41,13 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(
     const int kk = k0 + lk;
     if (am < M) {
       const float* p = A + (size_t)am * lda + kk;
-      if (vec_ok && kk + 3 < K) {
-        const float4 v = *(const float4*)p;
-        a[0] = v.x; a[1] = v.y; a[2] = v.z; a[3] = v.w;
-      } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) if (kk + i < K) a[i] = p[i];
-      }
+      for (int i = 0; i < 4; ++i) if (kk + i < K) a[i] = p[i];
     }
     if (bn < N) {
       const float* p = B + (size_t)bn * ldb + kk;
-      if (vec_ok && kk + 3 < K) {
-        const float4 v = *(const float4*)p;
-        b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
-      } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) if (kk + i < K) b[i] = p[i];
-      }
+      for (int i = 0; i < 4; ++i) if (kk + i < K) b[i] = p[i];
     }
     __syncthreads();  // previous tile fully consumed
 #pragma unroll
@@ -274,6 +262,184 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_rows_resident_f32_kernel(
   }
 }
 
+// ---- more rows than a decode step: matrix cores ----------------------------------------------------------------
+//
+// The float32 MFMA 16x16x4 multiplies and adds in float32 (no bfloat16 or tf32 form), 256 flops a clock and CU like
+// the vector ALU's FMAs, but an operand that is read from LDS once feeds a whole row of a 16x16 tile: the plain tile
+// above needs an LDS read for every two FMAs a thread does, and that is what bound it.
+// Block = 32 MI rows of A x 32 NI rows of B, KG groups of four waves (2 x 2 of 16 MI x 16 NI each).  K is walked in
+// steps of BK through STAGES buffers in LDS, a share of a step for each group, whose sums meet at the end in the order
+// of the groups: with two to four waves a SIMD one wave's reads of LDS and its wait at the step's barrier pass behind
+// the others' MFMAs (one group, 700 x 4,096 x 1,024: 83 us, two 68), and shorter chains of sums round less.  A
+// tile comes by `global_load_lds_dwordx4` straight from memory, STAGES - 1 steps ahead, waited for by count, one barrier
+// a step.  A lane (r = lane % 16, q = lane / 16) reads a chunk of four neighbouring k of its row, which are the operands
+// of four MFMAs: MFMA s of a sixteen of K adds the products at k = 4 q + s for q = 0..3, for A and B alike.
+// Measured on one MI355X, plain tile -> this, us, for 700 rows: N = 4,096, K = 1,024 108 -> 68; N = 1,024, K = 2,048
+// 133 -> 41; N = 6,144, K = 1,024 150 -> 105; N = 1,024, K = 3,072 190 -> 57; for 2,048 rows, N = 6,144, K = 2,560
+// 870 -> 556 (116 TFLOP/s; the chip's large products reach 154).  What is left is the last, partly filled round of
+// blocks and the waits at the steps' barriers.  Staging through registers instead (the compiler then counts the LDS
+// reads' waits itself) was slower everywhere: 44 to 58 us where this takes 41.
+typedef __attribute__((ext_vector_type(4))) float floatx4;
+
+#define FE_XCDS 8
+// wait until at most n of this wave's vector memory operations are outstanding
+#define FE_WAIT_VMEM(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | ((((n) >> 4) & 0x3) << 14) | (0x7 << 4) | (0xF << 8))
+
+__device__ __forceinline__ void load_to_lds(const void* global, void* lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
+                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+// COUNT times 16 bytes from LDS byte address `at`, STEP bytes apart, arrived when this returns (the compiler's own
+// reads of LDS would wait for every load into LDS that is under way, too)
+template <int COUNT, int STEP>
+__device__ __forceinline__ void lds_read_rows(unsigned int at, floatx4* v) {
+  if constexpr (COUNT == 1) asm volatile("ds_read_b128 %0, %1\n s_waitcnt lgkmcnt(0)" : "=&v"(v[0]) : "v"(at) : "memory");
+  if constexpr (COUNT == 2)
+    asm volatile("ds_read_b128 %0, %2\n ds_read_b128 %1, %2 offset:%3\n s_waitcnt lgkmcnt(0)"
+                 : "=&v"(v[0]), "=&v"(v[1]) : "v"(at), "n"(STEP) : "memory");
+  if constexpr (COUNT == 4)
+    asm volatile("ds_read_b128 %0, %4\n ds_read_b128 %1, %4 offset:%5\n ds_read_b128 %2, %4 offset:%6\n"
+                 " ds_read_b128 %3, %4 offset:%7\n s_waitcnt lgkmcnt(0)"
+                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(at), "n"(STEP), "n"(2 * STEP), "n"(3 * STEP) : "memory");
+}
+
+template <int MI, int NI, int STAGES, int KG, int BK>
+__global__ __launch_bounds__(256 * KG) void gemm_tile_f32_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias, float* __restrict__ C,
+    int M, int N, int K, long long lda, long long ldb, long long ldc, int tiles_m, int tiles, int wide_store) {
+  constexpr int BM = 32 * MI, BN = 32 * NI, CH = BK / 4, T = BK / (16 * KG);      // 16-byte chunks a row; sixteens of K a wave and step
+  constexpr int LOADS = (BM + BN) * CH / (256 * KG);                              // loads a wave and step
+  static_assert(T >= 1 && (BM + BN) * CH % (256 * KG) == 0, "every wave loads as much as every other");
+  static_assert(STAGES * (BM + BN) * BK >= (KG - 1) * BM * BN, "the groups' sums meet in the same LDS");
+  __shared__ __attribute__((aligned(16))) floatx4 lds[STAGES * (BM + BN) * CH];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Block b runs on XCD b % 8.  An XCD takes a run of neighbouring tiles, rows of A fastest, so that the blocks that
+  // share rows of B find them in their L2.
+  const int xcd = blockIdx.x % FE_XCDS, per = tiles / FE_XCDS, more = tiles % FE_XCDS;
+  const int tile = xcd * per + min(xcd, more) + blockIdx.x / FE_XCDS;
+  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+  // the unit of a row that holds a chunk: sixteen lanes that read one chunk of sixteen rows touch every bank once
+  auto swizzle = [](int row) { return CH == 8 ? (row >> 1) & 7 : row & 15; };
+
+  const float* from[LOADS];      // this lane's row of each of the wave's loads (A's rows, then B's)
+  int chunk[LOADS];              // ... and its place in that row
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int unit = (wave * LOADS + i) * 64 + lane, row = unit / CH;
+    from[i] = row < BM ? A + (size_t)min(m0 + row, M - 1) * lda : B + (size_t)min(n0 + row - BM, N - 1) * ldb;
+    chunk[i] = ((unit % CH) ^ swizzle(row)) * 4;
+  }
+  const int steps = (K + BK - 1) / BK;
+  auto load = [&](int step, int stage) {       // past the end the last step again, so that the waits can count; chunks beyond K read the row's first
+    const int k0 = min(step, steps - 1) * BK;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      load_to_lds(from[i] + (k0 + chunk[i] < K ? k0 + chunk[i] : 0), &lds[stage * (BM + BN) * CH + (wave * LOADS + i) * 64]);
+  };
+
+  const int r = lane & 15, q = lane >> 4, group = wave >> 2, wm = wave & 1, wn = (wave >> 1) & 1;
+  const unsigned int base = (unsigned int)(size_t)(const __attribute__((address_space(3))) char*)&lds[0];
+  const unsigned int a_at = base + (wm * 16 * MI + r) * BK * 4, b_at = base + (BM + wn * 16 * NI + r) * BK * 4;
+  floatx4 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  auto multiply = [&](int stage, int k0, bool partial) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int c = 4 * (group * T + t) + q;
+      const unsigned int at = stage * ((BM + BN) * BK * 4) + ((c ^ swizzle(r)) * 16);
+      floatx4 a[MI], b[NI];
+      lds_read_rows<MI, BK * 64>(a_at + at, a);
+      lds_read_rows<NI, BK * 64>(b_at + at, b);
+      if (partial && k0 + c * 4 >= K) {      // chunks beyond K: nothing of either operand
+#pragma unroll
+        for (int i = 0; i < MI; ++i) a[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NI; ++j) b[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][s], a[i][s], acc[i][j], 0, 0, 0);
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s) load(s, s);
+  const int whole = K / BK;
+  int stage = 0, fill = STAGES - 1;
+  for (int step = 0; step < steps; ++step) {
+    FE_WAIT_VMEM(LOADS * (STAGES - 2));      // this wave's share of the step's tile has landed ...
+    __builtin_amdgcn_s_barrier();            // ... and everyone's; everyone is done with the buffer that is filled next
+    asm volatile("" ::: "memory");
+    load(step + STAGES - 1, fill);
+    if (step < whole) multiply(stage, step * BK, false);
+    else multiply(stage, step * BK, true);
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+    fill = fill + 1 == STAGES ? 0 : fill + 1;
+  }
+  FE_WAIT_VMEM(0);       // the loads past the end have landed: the LDS is free
+  if constexpr (KG > 1) {       // the groups' sums, added in the order of the groups
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (group > 0) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) lds[(((group - 1) * 4 + (wave & 3)) * MI * NI + i * NI + j) * 64 + lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; ++g)
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] += lds[(((g - 1) * 4 + wave) * MI * NI + i * NI + j) * 64 + lane];
+  }
+
+  // lane (r, q) holds rows of B n0 + 16 j + 4 q .. + 3 for row of A m0 + 16 i + r: four neighbouring columns of C
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = m0 + (wm * MI + i) * 16 + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int n = n0 + (wn * NI + j) * 16 + 4 * q;
+      float* dst = C + (size_t)m * ldc + n;
+      if (wide_store && n + 3 < N) {
+        floatx4 v = acc[i][j];
+        if (bias) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += bias[n + e];
+        }
+        *(floatx4*)dst = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) dst[e] = acc[i][j][e] + (bias ? bias[n + e] : 0.f);
+      }
+    }
+  }
+}
+
+template <int MI, int NI, int STAGES, int KG, int BK>
+static int launch_tile_f32(const float* A, const float* B, const float* bias, float* C, int M, int N, int K, long long lda,
+                           long long ldb, long long ldc, hipStream_t stream) {
+  const long long tiles_m = (M + 32 * MI - 1) / (32 * MI), tiles = tiles_m * ((N + 32 * NI - 1) / (32 * NI));
+  if (tiles > 0x7fffffffLL) return FE_BAD_ARGUMENT;
+  const int wide_store = ldc % 4 == 0 && (((uintptr_t)C) & 15) == 0;
+  gemm_tile_f32_kernel<MI, NI, STAGES, KG, BK><<<dim3((unsigned)tiles), 256 * KG, 0, stream>>>(
+      A, B, bias, C, M, N, K, lda, ldb, ldc, (int)tiles_m, (int)tiles, wide_store);
+  return fe_check_launch();
+}
+
 #define FE_ROWS_F32_MAX 16     // most rows of A that the weight-streaming variant takes
 #define FE_ROWS_F32_RESIDENT_MAX 64   // most rows of A that go through the variant with A in registers, eight at a time
 
@@ -308,6 +474,18 @@ extern "C" int fe_gemm_nt_f32(const float* A, const float* B, const float* bias,
     else if (M <= 8) gemm_rows_f32_kernel<8, 4><<<dim3((N + 3) / 4, 1), 256, 0, stream>>>(A, B, bias, C, M, N, K, lda, ldb, ldc);   // measured: four rows of B a block beat eight (more waves in flight)
     else gemm_rows_f32_kernel<16, 4><<<dim3((N + 3) / 4, 1), 256, 0, stream>>>(A, B, bias, C, M, N, K, lda, ldb, ldc);
     return fe_check_launch();
+  }
+  if (aligned) {
+    // The tile that loads the fullest CU least: a launch takes as long as the CU with the most tiles, so smaller tiles
+    // win where larger ones leave CUs idle or start a round of few blocks; a small tile takes somewhat longer for its
+    // area (more bytes from LDS and L2 a product).  The factors are fitted to fourteen shapes of 70 to 2,048 rows, where
+    // the rule picks the fastest of the three or one within 2 % of it.
+    auto rounds = [](long long tiles) { return (double)((tiles + 255) / 256); };
+    const long long m64 = (M + 63) / 64, m32 = (M + 31) / 32, n64 = (N + 63) / 64, n32 = (N + 31) / 32;
+    const double large = 4.0 * rounds(m64 * n64), half = 2.24 * rounds(m64 * n32), small = 1.22 * rounds(m32 * n32);
+    if (large <= half && large <= small) return launch_tile_f32<2, 2, 2, 2, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
+    if (half <= small) return launch_tile_f32<2, 1, 3, 2, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
+    return launch_tile_f32<1, 1, 4, 4, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
   }
   const long long grid_y = (M + TILE_M - 1) / TILE_M;
   if (grid_y > 65535) return FE_BAD_ARGUMENT;

@@ -197,7 +197,8 @@ def stream_read(data: Tensor, sink: Tensor) -> None:
 # ------------------------------------------------------------ matrix products
 
 def gemm_nt_f32(a: Tensor, b: Tensor, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
-    """out[M, N] = a[M, K] @ b[N, K]^T (+ bias), true float32 (FMA, no matrix cores)."""
+    """out[M, N] = a[M, K] @ b[N, K]^T (+ bias), true float32: FMAs, and beyond the rows of a decode step
+    the matrix cores' float32 instruction, whose products and sums stay in 32 bits."""
     _gpu(a, "a", torch.float32, contiguous=False)
     _gpu(b, "b", torch.float32, contiguous=False)
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[1]:

@@ -155,6 +155,25 @@ def test_gemm_f32(ops, m, n, k):
             assert torch.equal(part, got[:rows])
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 1, 4), (65, 31, 60), (96, 33, 64), (97, 65, 68), (128, 64, 1024), (129, 4095, 132),   # edges of the tiles, K across a step
+                                   (70, 6145, 260), (250, 2049, 516), (703, 4097, 192)])      # the three tiles, in full and broken rounds
+def test_gemm_f32_tiles(ops, m, n, k):
+    """More rows than a decode step, on the matrix cores: within the bound that any order of k float32 products and
+    sums keeps, |error| <= 2 k 2^-24 sum |a||b|; a row with an infinity spoils itself only; rows with a stride."""
+    g = torch.Generator().manual_seed(m * 31 + n)
+    a, b, bias = rand(g, m, k + 4).to(DEV), rand(g, n, k + 8).to(DEV), rand(g, n).to(DEV)
+    a[m // 2, k - 1] = math.inf
+    got = ops.gemm_nt_f32(a[:, :k], b[:, :k], bias)
+    want = a[:, :k].double() @ b[:, :k].double().t() + bias.double()
+    most = (a[:, :k].double().abs() @ b[:, :k].double().abs().t() + bias.double().abs()) * (2 * k + 2) * 2.0 ** -24
+    finite = torch.ones(m, dtype=torch.bool, device=DEV)
+    finite[m // 2] = False
+    assert bool(((got.double() - want).abs() <= most)[finite].all())
+    assert torch.equal(got[m // 2].double(), want[m // 2])        # +-inf, by the sign of b's last number
+    again = ops.gemm_nt_f32(a[:, :k], b[:, :k], bias)
+    assert torch.equal(got, again)
+
+
 def test_gemm_f32_is_true_float32(ops):
     # operands whose product needs more than bfloat16's or tf32's mantissa
     a = torch.tensor([[1.0 + 2**-20, 1.0]])

@@ -833,12 +833,16 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
         if chunk is not None and chunk < 1:
             raise KernelError("chunk must be positive")
 
+    def runs_scratch(longest: int):
+        """Runs that a row's keys are cut into, and the scratch in which they meet."""
+        runs = generic_splits(num_seqs, kv_heads, groups, longest, head_dim, max_ctx)
+        if runs == 1:
+            return 1, None, None
+        return (runs, torch.empty((runs, tokens, q_heads * head_dim), dtype=torch.float32, device=q.device),
+                torch.empty((runs, tokens, q_heads, 2), dtype=torch.float32, device=q.device))
+
     def general(min_q: int, max_q: int) -> None:
-        runs = generic_splits(num_seqs, kv_heads, groups, min(max_q, max_q_len), head_dim, max_ctx)
-        part_acc = part_ml = None
-        if runs > 1:
-            part_acc = torch.empty((runs, tokens, q_heads * head_dim), dtype=torch.float32, device=q.device)
-            part_ml = torch.empty((runs, tokens, q_heads, 2), dtype=torch.float32, device=q.device)
+        runs, part_acc, part_ml = runs_scratch(min(max_q, max_q_len))
         _call("attention_generic", "fe_paged_attention_generic", _ptr(q), c_longlong(q_stride),
               _ptr(key_pages), _ptr(value_pages), _ptr(out), c_longlong(out.stride(0)),
               c_int(_code(q.dtype)), _ptr(cu_q), _ptr(ctx_len), _ptr(block_table),
@@ -880,7 +884,17 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
               c_int(max_q_len), c_int(kv_heads), c_int(groups), c_int(head_dim), c_int(block_size),
               c_int(num_blocks), c_int(window or 0), *mask, c_float(scale), *cap, c_int(PREFILL_KEY_GROUPS), c_int(PREFILL_ROW_SETS),
               c_int(tokens), _stream())
-    # whatever the two fast kernels did not take: single tokens go to the vector-ALU decode kernel where
+    # float32 portions at the fast kernels' head sizes: the matrix cores' float32 instruction
+    if (any_longer and q.dtype == torch.float32 and head_dim in (64, 128) and block_size >= 4 and block_size & (block_size - 1) == 0
+            and q_stride % 4 == 0 and q.data_ptr() % 16 == 0 and key_pages.data_ptr() % 16 == 0 and value_pages.data_ptr() % 16 == 0):
+        runs, part_acc, part_ml = runs_scratch(max_q_len)
+        _call("attention_f32", "fe_paged_attention_prefill_f32", _ptr(q), c_longlong(q_stride),
+              _ptr(key_pages), _ptr(value_pages), _ptr(out), c_longlong(out.stride(0)), _ptr(cu_q), _ptr(ctx_len),
+              _ptr(block_table), c_int(block_table.stride(0)), c_int(num_seqs), c_int(max_q_len), c_int(kv_heads),
+              c_int(groups), c_int(head_dim), c_int(block_size), c_int(num_blocks), c_int(window or 0), c_float(scale),
+              c_int(runs), _ptr(part_acc), _ptr(part_ml), c_int(tokens), _stream())
+        fast_prefill = True
+    # whatever the fast kernels did not take: single tokens go to the vector-ALU decode kernel where
     # it can read four elements at a time, the rest to the general kernel
     single_left = any_single and not fast_decode
     longer_left = any_longer and not fast_prefill
@@ -1067,7 +1081,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_tile", "qk_rope", "attention_generic", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

@@ -385,6 +385,34 @@ def test_paged_attention_window(ops, window):
     torch.testing.assert_close(got, want, atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,block_size,window", [
+    (4, 2, 128, 16, None), (5, 1, 64, 4, None), (3, 3, 128, 64, 37), (16, 8, 128, 16, 1), (8, 1, 64, 8, 200)])
+def test_float32_portions_on_the_matrix_cores(ops, q_heads, kv_heads, head_dim, block_size, window):
+    """Portions of 2 to 70 tokens at the edges of the row tiles and key units, single tokens beside them, an empty
+    sequence, slots that no token owns filled with NaN; the same with the keys of few rows cut into runs."""
+    g = torch.Generator().manual_seed(head_dim + block_size)
+    for seqs, cuts in (([(0, 70), (31, 2), (9, 1), (5, 16), (0, 17), (127, 33), (0, 2), (64, 64)], False), ([(1500, 3), (700, 2)], True)):
+        q, kp, vp, cu, ctx, table = _attention_case(g, torch.float32, seqs, q_heads, kv_heads, head_dim, block_size)
+        clean = refs.paged_attention(q, kp, vp, torch.empty(q.shape[0], q_heads * head_dim), cu, ctx, table, num_seqs=len(seqs),
+                                     max_q_len=70, q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, scale=head_dim ** -0.5, window=window)
+        owned = torch.zeros(kp.shape[0], block_size, dtype=torch.bool)
+        for s, (before, count) in enumerate(seqs):
+            for j in range(before + count):
+                owned[table[s, j // block_size], j % block_size] = True
+        kp[(~owned)[:, None, :, None].expand_as(kp)] = math.nan
+        vp[(~owned)[:, None, None, :].expand_as(vp)] = math.nan
+        n = len(seqs)
+        cu = torch.cat([cu, cu[-1:]]).to(DEV)                    # one more sequence, without tokens
+        ctx = torch.cat([ctx, torch.zeros(1, dtype=torch.int32)]).to(DEV)
+        table = torch.cat([table, torch.full_like(table[:1], -1)]).to(DEV)
+        if cuts:
+            assert ops.generic_splits(n + 1, kv_heads, q_heads // kv_heads, 3, head_dim, 1503) > 1
+        got = ops.paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), torch.empty(q.shape[0], q_heads * head_dim, device=DEV), cu, ctx, table,
+                                  num_seqs=n + 1, max_q_len=max(c for _, c in seqs), q_heads=q_heads, kv_heads=kv_heads,
+                                  head_dim=head_dim, scale=head_dim ** -0.5, window=window, max_ctx=1503 if cuts else None)
+        torch.testing.assert_close(got.cpu(), clean, atol=1e-5, rtol=1e-5)
+
+
 def test_paged_attention_is_library_attention(ops):
     # whole prompt, nothing cached: the library's causal attention after group expansion
     # (the reference pins its own kernels the same way, tests/test_kernels.py:91-105)

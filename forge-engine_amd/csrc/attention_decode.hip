@@ -534,8 +534,6 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   // a launch at 8 sequences); a cache-wide fence serialises across all blocks (0.3 us per block).
   // The counter goes back to zero for the next launch.
   __shared__ int is_last;
-  __shared__ float scale_s[GMAX][64];   // weight of each split per query row
-  __shared__ float inv_l[GMAX];
   __builtin_amdgcn_s_waitcnt((0x0) | (0x7 << 4) | (0xF << 8));    // vmcnt(0): this wave's stores have been acknowledged
   __syncthreads();
   if (tid == 0) {
@@ -560,25 +558,40 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     }
     return;
   }
-  if (tid < groups) {
-    const int g = tid;
-    float m_tot = -INFINITY;
-    for (int sp = 0; sp < splits; ++sp) m_tot = fmaxf(m_tot, load_agent(&part_ml[((first_part + sp) * groups + g) * 2]));
-    float l = 0.f;
-    for (int sp = 0; sp < splits; ++sp) {
-      const float f = m_tot > -INFINITY ? __builtin_amdgcn_exp2f(load_agent(&part_ml[((first_part + sp) * groups + g) * 2]) - m_tot) : 0.f;
-      scale_s[g][sp] = f;
-      l += f * load_agent(&part_ml[((first_part + sp) * groups + g) * 2 + 1]);
-    }
-    if (sink) l += __builtin_amdgcn_exp2f(sink[hk * groups + g] * 1.4426950408889634f - m_tot);
-    inv_l[g] = l > 0.f ? 1.f / l : 0.f;
-  }
-  __syncthreads();
-  for (int e = tid; e < groups * D; e += 256) {
+  // more: rounds of sixteen, each round's loads all in flight at once, the rounds' shares brought to one maximum as they
+  // come (one sequence of 8,000 keys in 32 runs: 17.8 us a launch, 27.6 with the statistics read one after the other)
+  for (int e = 2 * tid; e < groups * D; e += 512) {
     const int g = e / D, d = e - g * D;
-    float ov = 0.f;
-    for (int sp = 0; sp < splits; ++sp) ov += scale_s[g][sp] * load_agent(&part_o[((first_part + sp) * groups + g) * D + d]);
-    out[(size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d] = float_to_bf16(ov * inv_l[g]);
+    float m_tot = -INFINITY, l_tot = 0.f, ov0 = 0.f, ov1 = 0.f;
+    for (int base = 0; base < splits; base += 16) {
+      float m[16], l[16];
+      unsigned long long o[16];
+#pragma unroll
+      for (int sp = 0; sp < 16; ++sp) {
+        const size_t row = (first_part + min(base + sp, splits - 1)) * groups + g;
+        m[sp] = load_agent(&part_ml[row * 2]);
+        l[sp] = load_agent(&part_ml[row * 2 + 1]);
+        o[sp] = __hip_atomic_load((const unsigned long long*)&part_o[row * D + d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      float m_new = m_tot;
+#pragma unroll
+      for (int sp = 0; sp < 16; ++sp) m_new = fmaxf(m_new, m[sp]);
+      const float m_use = m_new > -INFINITY ? m_new : 0.f;
+      const float corr = __builtin_amdgcn_exp2f(m_tot - m_use);
+      l_tot *= corr; ov0 *= corr; ov1 *= corr;
+#pragma unroll
+      for (int sp = 0; sp < 16; ++sp) {
+        const float f = base + sp < splits ? __builtin_amdgcn_exp2f(m[sp] - m_use) : 0.f;
+        l_tot += f * l[sp];
+        ov0 += f * __uint_as_float((unsigned int)o[sp]);
+        ov1 += f * __uint_as_float((unsigned int)(o[sp] >> 32));
+      }
+      m_tot = m_new;
+    }
+    if (sink) l_tot += __builtin_amdgcn_exp2f(sink[hk * groups + g] * 1.4426950408889634f - m_tot);
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    *(unsigned int*)(out + (size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d) =
+        (unsigned int)float_to_bf16(ov0 * inv) | ((unsigned int)float_to_bf16(ov1 * inv) << 16);
   }
 }
 

@@ -24,6 +24,7 @@
 //   and receives D[m = 4*(l / 16) + i][n = l % 16].
 #include "common.h"
 #include "gate_act.h"
+#include "gemm_lds.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
@@ -245,9 +246,11 @@ __global__ __launch_bounds__(64 * WPB, 2) void gemm_wide_kernel(
 // few rows want a small tile; ending 2 takes tiles of 64 and 128 only).  block_rows = 64 or 32: the weight rows (gate/up ending: output
 // columns) a block of four or two waves takes; 32 gives a launch of few blocks twice as many; 128 (eight
 // waves, plain endings) halves how often x is read.
+// lds_tile >= 0: endings 0 to 2 with both operands through LDS instead, in the tile that gemm_lds.h lists under that number
+// (row_tile and block_rows do not count then).
 extern "C" int fe_gemm_wide(const void* x, const void* w, void* out, int M, int N, int K, long long ldw,
                             long long ldo, int ending, int parts, long long part_stride, int row_tile,
-                            int block_rows, int activation, hipStream_t stream) {
+                            int block_rows, int lds_tile, int activation, hipStream_t stream) {
   if (M < 1) return FE_OK;
   GateAct act;
   if (!gate_act(activation, &act)) return FE_BAD_ARGUMENT;
@@ -256,6 +259,10 @@ extern "C" int fe_gemm_wide(const void* x, const void* w, void* out, int M, int 
   if (ending < EPI_PARTS || ending > EPI_SWIGLU_HALF) return FE_BAD_ARGUMENT;
   if (parts < 1 || parts > 64 || (ending != EPI_PARTS && parts != 1)) return FE_BAD_ARGUMENT;
   if (parts > 1 && part_stride < (long long)M * ldo) return FE_BAD_ARGUMENT;
+  if (lds_tile >= 0) {
+    if (ending == EPI_SWIGLU_HALF) return FE_BAD_ARGUMENT;
+    return through_lds::launch(x, w, out, M, N, K, ldw, ldo, ending, parts, part_stride, lds_tile, act, stream);
+  }
   const int steps = K / WSTEP;
   const int per_part = (steps + parts - 1) / parts;
   if (row_tile != 16 && row_tile != 32 && row_tile != 64 && row_tile != 128) return FE_BAD_ARGUMENT;

@@ -8,6 +8,7 @@ implementation: without a GPU or without the compiled library a call raises.
 
 from __future__ import annotations
 
+import functools
 import threading
 from ctypes import c_double, c_float, c_int, c_longlong, c_void_p
 
@@ -327,6 +328,9 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
     if (bias is None and _skinny_fits(x, weight) and out_dtype in (torch.float32, torch.bfloat16)
             and not (out_dtype == torch.bfloat16 and _few_rows_to_library(x, weight))):
         return gemm_skinny(x, weight, "f32" if out_dtype == torch.float32 else "bf16")
+    if bias is None and out_dtype == torch.bfloat16 and _lds_fits(x, weight) and _lds_store_pays(x.shape[0], *weight.shape):
+        tile, _ = lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])
+        return gemm_lds(x, weight, "bf16", tile=tile)
     if (bias is None and out_dtype == torch.bfloat16 and _wide_fits(x, weight, WIDE_STORE_MAX_ROWS, SKINNY_MAX_ROWS + 1)
             and _wide_store_pays(x.shape[0], weight.shape[0], weight.shape[1])):
         rows = x.shape[0]        # up to 64 rows: blocks of 32 weight rows, so that the launch has twice the blocks
@@ -445,7 +449,7 @@ def gemm_wide(x: Tensor, weight: Tensor, ending: str = "bf16", parts: int = 1, r
         raise KernelError(f"no ending {ending!r} with {parts} parts")
     _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
           c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
-          c_int(row_tile or (16 if m <= 16 else 64 if m <= 64 else 128)), c_int(block_rows), _gate_act(act), _stream())
+          c_int(row_tile or (16 if m <= 16 else 64 if m <= 64 else 128)), c_int(block_rows), c_int(-1), _gate_act(act), _stream())
     return out
 
 
@@ -463,6 +467,102 @@ def _wide_parts(m: int, n: int, k: int, block_rows: int = 64, most: int = 16) ->
         if fill > best_fill + 1e-9:
             best, best_fill = parts, fill
     return -(-steps // -(-steps // best))
+
+
+# The product for portions with both operands through LDS (``gemm_lds``), 17 rows and more: its tiles (rows of x, weight rows,
+# blocks a CU holds at a time) with the microseconds a 64-step of K takes a CU that holds one block and two (or, where it
+# holds one at a time, one after the other).
+LDS_TILES = ((32, 32, 2, 0.151, 0.256), (64, 32, 1, 0.191, 0.382), (64, 64, 2, 0.212, 0.348), (64, 80, 1, 0.303, 0.606),
+             (64, 96, 2, 0.292, 0.451), (128, 64, 1, 0.317, 0.634), (128, 128, 1, 0.510, 1.02), (128, 160, 1, 0.630, 1.26), (32, 64, 2, 0.202, 0.378))
+LDS_MIN_K = 1024               # measured from this K on ...
+LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
+
+
+@functools.lru_cache(maxsize=4096)
+def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, consumer_us: float = 0.0) -> tuple[int, int]:
+    """(tile, parts of K) for ``gemm_lds``: the least of what a launch is predicted to take.  A block's steps take its CU
+    what the table says, the chip reads the weight at 5.4 TB/s (slower with fewer blocks than CUs) and pulls 20 TB/s of
+    tiles at best; whichever is slowest bounds the launch.  Fitted to 3,300 launches (25 weights of 1,024 to 17,408 rows,
+    17 to 1,024 rows of x, every tile, 1 to 8 parts): the picks take 1 % longer than the best of these tiles.
+    ``consumer_us``: what each part costs the consumer that adds them up."""
+    steps = k // 64
+    best = None
+    for tile, (rows, columns, held, one, two) in enumerate(LDS_TILES):
+        for parts in range(1, max(1, min(most_parts, steps // 4)) + 1):
+            tiles = -(-m // rows) * -(-weight_rows // columns) * parts
+            rounds = -(-tiles // 256)
+            step = one * rounds if held == 1 or rounds == 1 else two * -(-rounds // 2)
+            part_steps = -(-steps // parts)
+            bounds = (part_steps * step, weight_rows * k * 2 * 1.84e-7 * (256 / min(256, tiles)) ** 0.35,
+                      tiles * part_steps * (rows + columns) * 128 * 4.9e-8)
+            us = sum(b ** 4 for b in bounds) ** 0.25 + parts * (m * bytes_out * 3.1e-7 + consumer_us)
+            if best is None or us < best[0]:
+                best = (us, tile, parts)
+    return best[1], best[2]
+
+
+def _lds_fits(x: Tensor, weight: Tensor) -> bool:
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+            and x.shape[0] > SKINNY_MAX_ROWS and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
+            and x.shape[1] >= LDS_MIN_K and x.shape[1] % 64 == 0 and weight.shape[0] >= LDS_MIN_WEIGHT_ROWS
+            and weight.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
+    """(tile, parts) of a float32 update, or None where another product is the better one.  Up to 64 rows: weights of up to
+    2,048 x 4,096 by the plan (1,024 x 2,048 at 64 rows 6.5 -> 4.9 us), larger ones in the parts that fill the chip with
+    blocks of 64 weight rows (2,560 x 9,728 14.6 -> 12.9, 4,096 x 12,288 25.9 -> 23.4, at 32 rows 13.1 -> 11.6 and 22.8 ->
+    20.9).  Up to 384 rows all by the plan, and up to 1,024 through weights whose K is at least twice their rows, which the
+    matrix library cuts into too few blocks (512 rows: 2,560 x 9,728 48 -> 33, 5,120 x 17,408 169 -> 86)."""
+    if rows <= MID_ROWS and not (weight_rows <= 2048 and k <= 4096):
+        if weight_rows > WIDE_MAX_WEIGHT_ROWS:
+            return None
+        return (8 if rows <= 32 else 2), _wide_parts(rows, weight_rows, k)
+    if rows <= 384 or (rows <= 1024 and k >= 2 * weight_rows):
+        return lds_plan(rows, weight_rows, k, 4 * weight_rows, 8, 0.15 + rows * weight_rows * 8e-7)    # (a part's read by the norm: 5 TB/s)
+    return None
+
+
+def _lds_store_pays(rows: int, weight_rows: int, k: int) -> bool:
+    """Products that store bfloat16: up to 256 rows, 512 through weights of up to 4,096 rows (beyond, the library ties or
+    wins: 6,144 x 2,560 at 320 rows 18.6 against 19.9 us), weights of 2,048 rows (1,024: 7.7 against 8.4 us at 192 rows) to
+    50 MB (10,240 x 5,120 at 64 rows 32.6 against 33.9)."""
+    return weight_rows >= 2048 and weight_rows * k <= 26_000_000 and rows <= (512 if weight_rows <= 4096 else 256)
+
+
+def _lds_gate_pays(rows: int, columns: int) -> bool:
+    """Gate/up products: where tiles of 128 x 160 make one round of the chip (3,072 columns up to 700 rows: 22 -> 20 us, 6,144
+    up to 384: 33 -> 30, 9,728 up to 256: 54 -> 42, 12,288 up to 128); with a second round the matrix library's larger
+    tiles win (9,728 columns at 320 rows: 50 against 59 us)."""
+    return -(-rows // 128) * -(-2 * columns // 160) <= WIDE_CUS
+
+
+def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu") -> Tensor:
+    """x @ weight^T for bfloat16 rows: ``"parts"`` float32 partial sums [parts, M, N] over runs of whole 64-steps of K,
+    ``"bf16"`` [M, N], or ``"gated"``: act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first; ``act`` as in
+    ``swiglu``).  ``tile``: the block's, see ``LDS_TILES``."""
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(weight, "weight", torch.bfloat16, contiguous=False)
+    if (x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1] or x.shape[1] % 64 or weight.stride(1) != 1
+            or weight.stride(0) % 8 or not 1 <= parts <= 64 or x.data_ptr() % 16 or weight.data_ptr() % 16):
+        raise KernelError("the product through LDS takes contiguous bfloat16 rows, K a multiple of 64, at most 64 parts")
+    m, k = x.shape
+    n = weight.shape[0]
+    if ending == "parts":
+        out = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
+        code, cols = 0, n
+    elif ending in ("bf16", "gated") and parts == 1 and (ending == "bf16" or n % 2 == 0):
+        cols = n if ending == "bf16" else n // 2
+        out = torch.empty((m, cols), dtype=torch.bfloat16, device=x.device)
+        code = 1 if ending == "bf16" else 2
+    else:
+        raise KernelError(f"no ending {ending!r} with {parts} parts")
+    if not 0 <= tile < len(LDS_TILES):
+        raise KernelError(f"no tile {tile}")
+    _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
+          c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
+          c_int(64), c_int(64), c_int(tile), _gate_act(act), _stream())
+    return out
 
 
 def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream: Tensor | None = None) -> Tensor | None:
@@ -486,6 +586,10 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
                             UPDATE_SPLIT_BLOCKS // tiles))
         splits = -(-steps // -(-steps // splits))        # parts of equal length, none empty
         return gemm_skinny(x, weight, "f32", tiles=1, waves=4, splits=splits)
+    if plain_bf16 and _lds_fits(x, weight):
+        plan = _lds_update(x.shape[0], *weight.shape)
+        if plan is not None:
+            return gemm_lds(x, weight, "parts", plan[1], plan[0])
     if plain_bf16 and _wide_fits(x, weight, MID_ROWS, SKINNY_MAX_ROWS + 1):
         # 17 to 64 rows: one tile of x a block, the parts of K that fill the CUs; measured at 64 rows against
         # the product below: output projection 9.2 against 11.1 us (hidden size 4096: 10.6 against 12.5),
@@ -535,6 +639,10 @@ def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
         return gemm_wide(x, weight, "parts", parts, row_tile=16, block_rows=32)
     if _skinny_fits(x, weight) and rows <= FEW_ROWS:
         return gemm_skinny(x, weight, "f32", tiles=1, waves=4, splits=IN_PARTS_FEW_ROWS)
+    if rows <= MID_ROWS and _lds_fits(x, weight) and weight.shape[0] * weight.shape[1] <= 26_000_000:
+        # (6144 x 2560 at 64 rows 10.5 -> 9.4 us, 4096 x 1024 6.5 -> 5.8; at 17 rows level)
+        tile, parts = lds_plan(rows, weight.shape[0], weight.shape[1], 4 * weight.shape[0], 4, 0.15 + rows * weight.shape[0] * 8e-7)
+        return gemm_lds(x, weight, "parts", parts, tile)
     if (_mid_fits(x, weight) and weight.shape[0] <= WIDE_MAX_WEIGHT_ROWS
             and weight.shape[0] * weight.shape[1] * weight.element_size() <= MID_IN_PARTS_MAX_WEIGHT_BYTES):
         # (a weight of 10240 rows, K = 5120: 30 us at 32 rows against the library's 26; 7168 rows: 18 against 20;
@@ -592,6 +700,9 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tenso
             and x.data_ptr() % 16 == 0 and gate_up_weight.data_ptr() % 16 == 0
             and gate_up_weight.shape[0] * gate_up_weight.stride(0) < 2 ** 32 and rows * x.shape[1] < 2 ** 32):
         return gemm_gated(x, gate_up_weight, shape=3, act=act)
+    if (gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight) and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2)):
+        tile, _ = lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])
+        return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
     to_library = (2 <= rows <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
                   and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
     paired_fits = (rows <= MID_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16

@@ -898,6 +898,62 @@ def test_linear_swiglu_routes_by_rows(ops, monkeypatch):
         torch.testing.assert_close(got, refs.linear_swiglu(x, weight).float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("tile", range(9))
+@pytest.mark.parametrize("m,n,k,parts", [(1, 8, 64, 1), (31, 33, 128, 2), (64, 80, 192, 2), (65, 97, 640, 3), (129, 161, 1024, 5), (257, 330, 704, 4)])
+def test_gemm_lds(ops, tile, m, n, k, parts):
+    """Every tile at its edges and remainders, K in equal and unequal parts (and one without steps), a weight that is a slice
+    of a wider one.  float32 parts against the exact products of the bfloat16 operands: |error| <= 2 k 2^-24 sum |a||b|."""
+    g = torch.Generator().manual_seed(m + n)
+    x = rand(g, m, k, dtype=torch.bfloat16).to(DEV)
+    w = rand(g, 2 * n, k + 64, dtype=torch.bfloat16, scale=0.05).to(DEV)[:, :k]
+    exact = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * (2 * k + 2 * parts) * 2.0 ** -24
+    got = ops.gemm_lds(x, w, "parts", parts, tile)
+    assert got.shape == (parts, m, 2 * n) and bool(((got.double().sum(0) - exact).abs() <= bound + 1e-30).all())
+    steps, per = k // 64, -(-(k // 64) // parts)
+    for part in range(parts):
+        at = slice(64 * min(steps, part * per), 64 * min(steps, (part + 1) * per))
+        assert bool(((got[part].double() - x[:, at].double() @ w[:, at].double().t()).abs() <= bound + 1e-30).all())
+    stored = ops.gemm_lds(x, w, "bf16", tile=tile)
+    assert bool(((stored.double() - exact).abs() <= bound + exact.abs() * 2.0 ** -8).all())      # one rounding on top
+    for act in ("silu", "gelu_tanh"):
+        gated = ops.gemm_lds(x, w, "gated", tile=tile, act=act).float()
+        both = exact.float()
+        torch.testing.assert_close(gated, ops.swiglu(both.contiguous(), torch.empty(m, n, device=DEV), act), atol=2e-2, rtol=2e-2)
+    one_row = ops.gemm_lds(x[:1].contiguous(), w, "parts", parts, tile)
+    assert torch.equal(one_row[:, 0], got[:, 0])                 # a row's sums do not depend on the rows beside it
+
+
+def test_gemm_lds_refuses_and_plans(ops, monkeypatch):
+    x = torch.zeros(70, 1024, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(4096, 1024, dtype=torch.bfloat16, device=DEV)
+    for bad in (lambda: ops.gemm_lds(x, w, "bf16", 2), lambda: ops.gemm_lds(x, w, "parts", 65), lambda: ops.gemm_lds(x, w[:, :1000], "parts"),
+                lambda: ops.gemm_lds(x, w, "swiglu"), lambda: ops.gemm_lds(x, w, "bf16", tile=9), lambda: ops.gemm_lds(x, w[:, :960], "bf16"),
+                lambda: ops.gemm_lds(x, w.float(), "bf16")):
+        with pytest.raises(ops.KernelError):
+            bad()
+    # what takes a size: rows, weight rows, K at both sides of every line
+    taken = []
+    real = ops.gemm_lds
+    monkeypatch.setattr(ops, "gemm_lds", lambda *a, **kw: taken.append("lds") or real(*a, **kw))
+    g = torch.Generator().manual_seed(9)
+    for rows, n, k, kind, own in ((17, 4096, 1024, "store", True), (16, 4096, 1024, "store", False), (512, 4096, 1024, "store", True),
+                                  (513, 4096, 1024, "store", False), (257, 4160, 1024, "store", False), (256, 4160, 1024, "store", True),
+                                  (100, 1984, 1024, "store", False), (17, 512, 2048, "update", True), (1024, 512, 1024, "update", True),
+                                  (1025, 512, 1024, "update", False), (400, 1024, 1024, "update", False), (384, 1024, 1024, "update", True),
+                                  (64, 512, 8256, "update", True), (40, 8256, 1024, "update", False), (130, 448, 1024, "update", False),
+                                  (768, 3072, 1024, "gate", True), (769, 3072, 1024, "gate", False), (100, 3072, 960, "gate", False)):
+        x = rand(g, rows, k, dtype=torch.bfloat16).to(DEV)
+        w = rand(g, n * (2 if kind == "gate" else 1), k, dtype=torch.bfloat16, scale=0.02).to(DEV)
+        taken.clear()
+        got = {"store": ops.linear, "update": ops.linear_update, "gate": ops.linear_swiglu}[kind](x, w)
+        assert bool(taken) == own, (rows, n, k, kind, taken)
+        want = x.float() @ w.float().t()
+        if kind == "gate":
+            want = want[:, :n] / (1 + torch.exp(-want[:, :n])) * want[:, n:]
+        torch.testing.assert_close((got.sum(0) if got.dim() == 3 else got).float(), want, atol=2e-2, rtol=2e-2)
+
+
 def test_gemm_wide_refuses_and_routes(ops, monkeypatch):
     x = torch.zeros(70, 200, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(64, 200, dtype=torch.bfloat16, device=DEV)

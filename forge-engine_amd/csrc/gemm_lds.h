@@ -25,62 +25,26 @@
 #pragma once
 #include "common.h"
 #include "gate_act.h"
+#include "lds_tile.h"
 
 namespace through_lds {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float floatx4;
-typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
+using lds_tile::floatx4;
+using lds_tile::uintx4;
+using lds_tile::KSTEP;
 
-constexpr int KSTEP = 64;          // elements of K a step
 constexpr int XCDS = 8;
 constexpr int END_PARTS = 0, END_BF16 = 1, END_GATED = 2;
 
-// wait until at most n of this wave's vector memory operations are outstanding (n < 64)
-#define FE_WAIT_VMEM(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | ((((n) >> 4) & 0x3) << 14) | (0x7 << 4) | (0xF << 8))
-
-__device__ __forceinline__ void load_to_lds(const void* global, void* lds) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
-                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
-}
-
-// 16 bytes from LDS byte address `at` + OFFSET (a constant below 65536); nothing waits for them here (the compiler's own
-// reads of LDS would wait for every load into LDS that is under way, too)
-template <int OFFSET>
-__device__ __forceinline__ uintx4 lds_read16(unsigned int at) {
-  uintx4 v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFFSET) : "memory");
-  return v;
-}
-// COUNT fragments of sixteen rows, 2,048 bytes apart
-template <int COUNT, int FROM = 0>
-__device__ __forceinline__ void lds_read_rows(unsigned int at, uintx4* v) {
-  if constexpr (FROM < COUNT) {
-    v[FROM] = lds_read16<2048 * FROM>(at);
-    lds_read_rows<COUNT, FROM + 1>(at, v);
-  }
-}
-// every read of LDS of this wave has arrived; `v` are the registers that the wait is for
-template <int COUNT>
-__device__ __forceinline__ void lds_arrived(uintx4* v) {
-#pragma unroll
-  for (int i = 0; i < COUNT; ++i) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[i]));
-}
-
-// LDS holds a step of a tile as [row][8 chunks of 16 bytes], x's rows and then the weight's, chunk c of row j at position
-// c ^ (j % 8): the lanes that a 16-byte read serves in one cycle then hit different bank groups (no conflicts counted).
 // With the gated ending a fragment of sixteen weight rows is eight gate rows and the eight up rows of the same columns.
 template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
     long long ldw, long long ldo, int tiles_m, int tiles_n, int parts, int steps_per_part, long long part_stride,
     long long up_offset, GateAct act) {
-  constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, WAVES = WM * WN * KG, T = 2 / KG;
-  constexpr int GROUPS = (BM + BN) / 8, LOADS = GROUPS / WAVES, MORE = GROUPS % WAVES;   // groups of eight rows: one load of a wave each
-  constexpr int STAGE = (BM + BN) * 8;              // 16-byte units of a stage
+  constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN;
   constexpr int COLUMNS = END == END_GATED ? BN / 2 : BN;
   extern __shared__ __attribute__((aligned(16))) uintx4 lds[];     // [STAGES][BM + BN rows][8]
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Block b runs on XCD b % 8.  An XCD takes a run of neighbouring tiles, rows of x fastest, so that the blocks that
   // share weight rows find them in their L2.
   const int tiles = tiles_m * tiles_n * parts;
@@ -91,111 +55,16 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
   const int n0 = tile % tiles_n * COLUMNS, part = tile / tiles_n;
   const int steps = K / KSTEP, first = part * steps_per_part, last = min(steps, first + steps_per_part);
 
-  // this lane's place in each of the wave's loads; rows beyond M and N read the last row again (never stored)
-  const bf16_t* from[LOADS + 1];
-#pragma unroll
-  for (int i = 0; i <= LOADS; ++i) {
-    const int row = min((wave + WAVES * i) * 8 + (lane >> 3), BM + BN - 1);
-    const int chunk = (lane & 7) ^ (row & 7);
-    if (row < BM) from[i] = x + (size_t)min(m0 + row, M - 1) * K + chunk * 8;
-    else {
-      const int j = row - BM;
-      if (END == END_GATED) from[i] = w + (size_t)min(n0 + (j >> 4) * 8 + (j & 7), N - 1) * ldw + ((j & 8) ? up_offset : 0) + chunk * 8;
-      else from[i] = w + (size_t)min(n0 + j, N - 1) * ldw + chunk * 8;
-    }
-  }
-  auto load = [&](int step, int stage) {       // past the end the last step again, so that the waits can count
-    const int k0 = min(step, last - 1) * KSTEP;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_to_lds(from[i] + k0, &lds[stage * STAGE + (wave + WAVES * i) * 64]);
-    if (MORE > 0 && wave < MORE) load_to_lds(from[LOADS] + k0, &lds[stage * STAGE + (wave + WAVES * LOADS) * 64]);
+  // rows beyond M and N read the last row again (never stored)
+  auto row_of = [&](int row) -> const bf16_t* {
+    if (row < BM) return x + (size_t)min(m0 + row, M - 1) * K;
+    const int j = row - BM;
+    if (END == END_GATED) return w + (size_t)min(n0 + (j >> 4) * 8 + (j & 7), N - 1) * ldw + ((j & 8) ? up_offset : 0);
+    return w + (size_t)min(n0 + j, N - 1) * ldw;
   };
-  const int r = lane & 15, q = lane >> 4, group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  const unsigned int base = (unsigned int)(size_t)(const __attribute__((address_space(3))) char*)&lds[0];
-  const unsigned int x_at = base + (wm * 16 * MI + r) * 128, w_at = base + (BM + wn * 16 * NI + r) * 128;
   floatx4 acc[MI][NI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NI; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  if (first < last) {
-    uintx4 a0[MI], b0[NI], a1[MI], b1[NI];
-    auto fragments = [&](int stage, int t, uintx4* a, uintx4* b) {
-      const unsigned int at = stage * (STAGE * 16) + (((4 * (group * T + t) + q) ^ (r & 7)) * 16);
-      lds_read_rows<MI>(x_at + at, a);
-      lds_read_rows<NI>(w_at + at, b);
-    };
-    auto multiply = [&](const uintx4* a, const uintx4* b) {
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b[j]), __builtin_bit_cast(bf16x8, a[i]), acc[i][j], 0, 0, 0);
-    };
-    int stage = 0;
-    // a half: the next half's fragments are requested, then this half's are multiplied
-    auto half = [&](int step, bool ends_step, int t_next, const uintx4* a, const uintx4* b, uintx4* a_next, uintx4* b_next) {
-      int from_stage = stage;
-      if (ends_step) {
-        // this wave's share of the next step has landed, and behind the barrier everyone's; everyone has read all of
-        // this step, whose buffer is filled again
-        if (MORE > 0 && wave < MORE) FE_WAIT_VMEM((LOADS + 1) * (STAGES - 2));
-        else FE_WAIT_VMEM(LOADS * (STAGES - 2));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        load(step + STAGES, stage);
-        stage = stage + 1 == STAGES ? 0 : stage + 1;
-        from_stage = stage;
-      }
-      fragments(from_stage, t_next, a_next, b_next);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(a, b);
-      __builtin_amdgcn_sched_barrier(0);
-      lds_arrived<MI>(a_next);
-      lds_arrived<NI>(b_next);
-    };
-#pragma unroll
-    for (int s = 0; s < STAGES; ++s) load(first + s, s);
-    if (MORE > 0 && wave < MORE) FE_WAIT_VMEM((LOADS + 1) * (STAGES - 1));
-    else FE_WAIT_VMEM(LOADS * (STAGES - 1));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    fragments(0, 0, a0, b0);
-    lds_arrived<MI>(a0);
-    lds_arrived<NI>(b0);
-    if constexpr (T == 2) {
-      for (int step = first; step < last; ++step) {
-        half(step, false, 1, a0, b0, a1, b1);
-        half(step, true, 0, a1, b1, a0, b0);
-      }
-    } else {
-      int step = first;
-      for (; step + 1 < last; step += 2) {
-        half(step, true, 0, a0, b0, a1, b1);
-        half(step + 1, true, 0, a1, b1, a0, b0);
-      }
-      if (step < last) half(step, true, 0, a0, b0, a1, b1);
-    }
-    FE_WAIT_VMEM(0);
-  }
-  if constexpr (KG > 1) {
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    floatx4* meet = (floatx4*)lds;
-    if (group > 0) {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) meet[((wave % (WM * WN)) * MI * NI + i * NI + j) * 64 + lane] = acc[i][j];
-    }
-    __syncthreads();
-    if (group > 0) return;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NI; ++j) acc[i][j] += meet[(wave * MI * NI + i * NI + j) * 64 + lane];
-  }
+  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, false>(lds, row_of, first, last, K, acc)) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4, wm = wave % WM, wn = wave / WM;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int m = m0 + (wm * MI + i) * 16 + r;
@@ -240,29 +109,14 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
   }
 }
 
-// The fragments' reads are waited for by hand: a build that spills registers would move values that are still in flight,
-// and is never launched.  Also raises the kernel's LDS limit.  0: not yet asked, 1: fit, -1: refused.
-static int fit_to_launch(const void* kernel, size_t lds_bytes, int* checked) {
-  if (*checked == 0) {
-    hipFuncAttributes attributes;
-    if (hipFuncGetAttributes(&attributes, kernel) != hipSuccess) return FE_LAUNCH_FAILED;
-    if (attributes.localSizeBytes != 0) { *checked = -1; return FE_BAD_ARGUMENT; }
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
-      return FE_LAUNCH_FAILED;
-    *checked = 1;                 // (a race here only repeats the calls)
-  }
-  return *checked < 0 ? FE_BAD_ARGUMENT : FE_OK;
-}
-
 template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END>
 static int launch_tile(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int parts,
                        long long part_stride, GateAct act, hipStream_t stream) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, COLUMNS = END == END_GATED ? BN / 2 : BN;
-  constexpr size_t bytes = (size_t)STAGES * (BM + BN) * 128;
-  static_assert(bytes <= 160 * 1024 && bytes >= (size_t)(KG - 1) * BM * BN * 4, "LDS of a CU");
+  constexpr size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES;
   static int checked = 0;
   auto kernel = gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END>;
-  const int fit = fit_to_launch((const void*)kernel, bytes, &checked);
+  const int fit = lds_tile::fit_to_launch((const void*)kernel, bytes, &checked);
   if (fit != FE_OK) return fit;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + COLUMNS - 1) / COLUMNS;
   if (tiles_m * tiles_n * parts > 0x7fffffffLL) return FE_BAD_ARGUMENT;

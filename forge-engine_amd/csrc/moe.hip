@@ -17,11 +17,10 @@
 //
 // The grouped products tile the sorted rows within an expert (a tile never spans two experts).  float32, and
 // bfloat16 with K no multiple of 32: 32 rows x 64 columns a block, K through LDS in steps of 32, FMA.  bfloat16:
-// MFMA 16x16x32 over 64 rows x 64 columns with the weight straight into the operands (steps of few rows: a
-// decode step streams every expert's weight once), or 64 rows x 128 columns with the weight tile through LDS like
-// the rows (steps of many rows).  A launch has as many row-tile slots as the pairs could need at worst (pairs /
+// MFMA 16x16x32 over tiles of 32 x 64 to 256 x 128 with rows and weight straight from memory in LDS.  A launch has as many row-tile slots as the pairs could need at worst (pairs /
 // rows a tile + experts); a block whose slot lies beyond the tiles there are returns at once.
 #include "common.h"
+#include "lds_tile.h"
 
 // One thread per token over its row of router logits z [T, E] (float32, the product comes from the
 // caller): bias added, the `top` largest chosen one after the other (the largest first; among equals
@@ -335,324 +334,161 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
   }
 }
 
-// The same two products on the matrix cores, for bfloat16 with K a multiple of 32: a block takes 64 sorted
-// rows of one expert and 64 output columns (MODE 0: 64 gate columns and their 64 up columns), K in steps
-// of 32.  The rows go through LDS (two stages, one barrier a step; rows 80 bytes apart so that the
-// 16-byte reads of a fragment spread over the banks), the weight goes straight from memory into the
-// MFMA operand: wave w owns columns 16 w .. 16 w + 15 and all four 16-row tiles.  Both operands of the
-// next step are requested before this step's products.  A result lane holds rows 4 (lane / 16) + i of a
-// tile at column lane % 16.
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float floatx4;
-typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
-#define TM 64
-#define TN 64
-#define TK 32
-#define TPAD 40
+// The same two products on the matrix cores, for bfloat16 with K a multiple of 32: the tile product of lds_tile.h, a tile's rows
+// gathered through the sorted pairs, its weight rows the expert's; rows and weight go straight from memory into LDS, several
+// steps of 64 ahead.  (MODE 0: a fragment of sixteen weight rows is eight gate rows and the eight up rows of the same columns.)
+// Blocks go to the eight dies (XCDs, each with an L2 of its own) in turn by their index.  The row tiles of one expert
+// under one column tile read the same part of the weight, so they are made neighbours in the order of work (the row
+// slot runs fastest) and a die takes a run of that order: a weight tile comes from memory once for all its row tiles.
+using lds_tile::floatx4;
+using lds_tile::uintx4;
 
-// A barrier that orders the block's LDS traffic only: the loads from global memory that are under way for
-// later steps stay under way (a barrier that fences every address space waits for all of them, and the
-// operands requested steps ahead would arrive no earlier than those of the step at hand).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+// find_tile by the lanes of a wave: experts 64 at a time, a lane one of them; every lane gets the answer
+template <int ROWS>
+__device__ __forceinline__ bool find_tile_by_lanes(const int* __restrict__ offsets, int E, int slot, int& expert, int& row0, int& row_end) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = min(e0 + lane, E - 1);
+    const int begin = offsets[e], end = offsets[e + 1];
+    int upto = e0 + lane < E ? (end - begin + ROWS - 1) / ROWS : 0;      // tiles of this lane's expert, then of all up to it
+    const int mine = upto;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+      const int below = __shfl_up(upto, offset, FE_WAVE);
+      if (lane >= offset) upto += below;
+    }
+    const unsigned long long past = __ballot(slot < before + upto);
+    if (past) {
+      const int at = __ffsll((long long)past) - 1;
+      expert = e0 + at;
+      const int first = __shfl(begin, at, FE_WAVE), tile = slot - before - (__shfl(upto, at, FE_WAVE) - __shfl(mine, at, FE_WAVE));
+      row0 = first + tile * ROWS;
+      row_end = __shfl(end, at, FE_WAVE);
+      return true;
+    }
+    before += __shfl(upto, 63, FE_WAVE);
+  }
+  return false;
 }
 
-template <int MODE, int NT, int MT>
-__global__ __launch_bounds__(256) void moe_grouped_mfma_kernel(
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, int MODE>
+__global__ __launch_bounds__(64 * WM * WN * KG) void moe_lds_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ offsets,
     const int* __restrict__ order, const float* __restrict__ pair_weight, bf16_t* __restrict__ act,
     float* __restrict__ out, int E, int N, int K, int top, int tokens, float limit, float alpha, int form,
     const float* __restrict__ extra, int extra_parts, int slots, int column_tiles) {
-  // NT: groups of 16 columns a wave (a block takes 64 NT columns); MT: tiles of 16 rows a wave (a block takes
-  // 16 MT rows, every wave all of them).  Steps of few rows launch <MODE, 1, 4>: many blocks, each streaming
-  // its part of the weight.  For steps of many rows the larger shapes of this kernel were measured and lost to
-  // the kernel below, whose weight tile goes through LDS (<MODE, 2, 4>: 3.80 against 3.67 ms for a prompt of 2,048
-  // tokens at a width of 2,048; <MODE, 2, 8> at 4,096: 9.9 against 9.6 ms; eight waves over 128 rows, the second
-  // four asking for the weight fragments of the first four: 4.3 ms at 2,048).
-  constexpr int ROWS = 16 * MT;
-  constexpr int AL = ROWS / 64;          // 16-byte pieces of a step's rows a thread brings
-  __shared__ __attribute__((aligned(16))) bf16_t As[2][ROWS][TPAD];
-  __shared__ int pair_of[ROWS];
-  // Blocks go to the eight dies (XCDs, each with an L2 of its own) in turn by their index.  The row tiles of
-  // one expert under one column tile read the same part of the weight, so they are made neighbours in the
-  // order of work (the row slot runs fastest) and a die takes a run of that order: block b works on item
-  // (b % 8) * ceil(items / 8) + b / 8, and a weight tile comes from memory once for all its row tiles.
+  constexpr int TILE_ROWS = 16 * MI * WM, TILE_COLS = 16 * NI * WN, COLUMNS = MODE == 0 ? TILE_COLS / 2 : TILE_COLS;
+  extern __shared__ __attribute__((aligned(16))) uintx4 lds[];
   const int items = slots * column_tiles;
   const int per_die = (items + 7) / 8;
   const int item = (int)(blockIdx.x % 8) * per_die + (int)(blockIdx.x / 8);
   if (item >= items) return;
   int expert, row0, row_end;
-  if (!find_tile<ROWS>(offsets, E, item % slots, expert, row0, row_end)) return;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, lr = lane % 16, lq = lane / 16;
-  const int n0 = (item / slots) * (TN * NT);
-  for (int r = tid; r < ROWS; r += 256) pair_of[r] = row0 + r < row_end ? order[row0 + r] : -1;
-  __syncthreads();
-  // this thread's 16-byte pieces of a step's rows: rows tid / 4 + 64 j, k chunk tid % 4
-  const int my_chunk = tid % 4;
-  int my_row[AL];
-  bool my_live[AL];
-  const bf16_t* a_at[AL];
-#pragma unroll
-  for (int j = 0; j < AL; ++j) {
-    my_row[j] = tid / 4 + 64 * j;
-    const int pair = pair_of[my_row[j]];
-    my_live[j] = pair >= 0;
-    const size_t src = pair < 0 ? 0 : (MODE != 1 ? (size_t)(pair / top) : (size_t)(row0 + my_row[j]));
-    a_at[j] = a + src * K + my_chunk * 8;
-  }
-  const size_t w_rows = MODE == 0 ? 2 * (size_t)N : (size_t)N;
-  int n[NT];
-  const bf16_t* wg_at[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    n[nt] = n0 + (wave * NT + nt) * 16 + lr;
-    wg_at[nt] = w + ((size_t)expert * w_rows + min(n[nt], N - 1)) * K + lq * 8;
-  }
-  const size_t up_offset = MODE == 0 ? (size_t)N * K : 0;
-  floatx4 acc_g[NT][MT], acc_u[NT][MT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc_g[nt][mt] = acc_u[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const uintx4 zero = {0u, 0u, 0u, 0u};
-  // Step s has its operands in register set s % DEPTH, requested DEPTH steps ahead (a step's arithmetic is far
-  // shorter than a trip to memory, and a launch of few blocks keeps the memory busy only through what each
-  // block has in flight).  The rows of step s + 1 go into the other LDS stage while step s multiplies; one
-  // barrier a step.  Whole rounds of DEPTH steps are straight-line code; steps beyond the last fetch the last
-  // step's operands again, so that no load stands under a branch.
-  constexpr int DEPTH = MT > 4 ? 2 : 4;
-  const int steps = K / TK;
-  uintx4 a_reg[DEPTH][AL], wg_reg[DEPTH][NT], wu_reg[DEPTH][NT];
-  auto fetch = [&](int step, int set) {
-    const int at = min(step, steps - 1) * TK;
-#pragma unroll
-    for (int j = 0; j < AL; ++j) a_reg[set][j] = *(const uintx4*)(a_at[j] + at);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      wg_reg[set][nt] = *(const uintx4*)(wg_at[nt] + at);
-      if (MODE == 0) wu_reg[set][nt] = *(const uintx4*)(wg_at[nt] + up_offset + at);
+  if (!find_tile_by_lanes<TILE_ROWS>(offsets, E, item % slots, expert, row0, row_end)) return;
+  const int n0 = (item / slots) * COLUMNS;
+  const bf16_t* w_expert = w + (size_t)expert * (MODE == 0 ? 2 * (size_t)N : (size_t)N) * K;
+  auto row_of = [&](int row) -> const bf16_t* {      // rows beyond the expert's and columns beyond N: the last again, never stored
+    if (row < TILE_ROWS) {
+      const int sorted = min(row0 + row, row_end - 1);
+      return a + (size_t)(MODE != 1 ? order[sorted] / top : sorted) * K;
     }
+    const int j = row - TILE_ROWS;
+    if (MODE == 0) return w_expert + ((size_t)min(n0 + (j >> 4) * 8 + (j & 7), N - 1) + ((j & 8) ? N : 0)) * K;
+    return w_expert + (size_t)min(n0 + j, N - 1) * K;
   };
-  auto multiply = [&](int stage, int set) {
+  floatx4 acc[MI][NI];
+  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, true>(lds, row_of, 0, (K + lds_tile::KSTEP - 1) / lds_tile::KSTEP, K, acc)) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4, wm = wave % WM, wn = wave / WM;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const bf16x8 rows = *(const bf16x8*)&As[stage][mt * 16 + lr][lq * 8];
+  for (int i = 0; i < MI; ++i) {
+    const int row = row0 + (wm * MI + i) * 16 + r;
+    const bool live = row < row_end;
+    const int pair = live ? order[row] : 0;
+    const float weight = pair_weight ? pair_weight[pair] : 1.f;
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        acc_g[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows, __builtin_bit_cast(bf16x8, wg_reg[set][nt]), acc_g[nt][mt], 0, 0, 0);
-        if (MODE == 0)
-          acc_u[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows, __builtin_bit_cast(bf16x8, wu_reg[set][nt]), acc_u[nt][mt], 0, 0, 0);
-      }
-    }
-  };
-  auto stash = [&](int stage, int set) {
+    for (int j = 0; j < NI; ++j) {
+      if constexpr (MODE != 1) {
+        float y[4];
 #pragma unroll
-    for (int j = 0; j < AL; ++j) *(uintx4*)&As[stage][my_row[j]][my_chunk * 8] = my_live[j] ? a_reg[set][j] : zero;
-  };
-#pragma unroll
-  for (int u = 0; u < DEPTH; ++u) fetch(u, u);
-  stash(0, 0);
-  lds_barrier();
-  int step = 0;
-  for (; step + DEPTH <= steps; step += DEPTH) {
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-      multiply(u & 1, u);
-      stash((u + 1) & 1, (u + 1) % DEPTH);
-      fetch(step + u + DEPTH, u);
-      lds_barrier();
-    }
-  }
-  const int left = steps - step;       // 0 .. DEPTH - 1, the same for every thread
-#pragma unroll
-  for (int u = 0; u < DEPTH - 1; ++u)
-    if (u < left) {
-      multiply(u & 1, u);
-      stash((u + 1) & 1, (u + 1) % DEPTH);
-      lds_barrier();
-    }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    if (n[nt] >= N) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = mt * 16 + lq * 4 + i;
-        const int pair = pair_of[r];
-        if (pair < 0) continue;
-        if (MODE != 1) {
-          act[(size_t)(row0 + r) * N + n[nt]] = float_to_bf16(gated(acc_g[nt][mt][i], acc_u[nt][mt][i], limit, alpha, form, pair_weight ? pair_weight[pair] : 1.f));
-        } else {
-          const int token = pair / top, choice = pair - token * top;
-          out[((size_t)choice * tokens + token) * N + n[nt]] = with_extra(
-              acc_g[nt][mt][i] * (pair_weight ? pair_weight[pair] : 1.f), choice, extra, extra_parts, (size_t)tokens * N, (size_t)token * N + n[nt]);
+        for (int e = 0; e < 4; ++e) {
+          // (MODE 0: lanes q = 0, 1 hold gate columns 4 q .. + 3 of the fragment's eight, lanes q = 2, 3 the up columns of lane - 32)
+          float up = 0.f;
+          if constexpr (MODE == 0)
+            up = __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i][j][e]), __float_as_uint(acc[i][j][e]), false, false)[1]);
+          y[e] = gated(acc[i][j][e], up, limit, alpha, form, weight);
         }
+        const int n = n0 + (wn * NI + j) * (MODE == 0 ? 8 : 16) + 4 * (MODE == 0 ? q & 1 : q);
+        if (!live || (MODE == 0 && q >= 2)) continue;
+        bf16_t* to = act + (size_t)row * N + n;
+        if (n + 3 < N && (N & 3) == 0 && ((uintptr_t)act & 7) == 0)
+          *(uint2*)to = make_uint2((unsigned)float_to_bf16(y[0]) | ((unsigned)float_to_bf16(y[1]) << 16),
+                                   (unsigned)float_to_bf16(y[2]) | ((unsigned)float_to_bf16(y[3]) << 16));
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) to[e] = float_to_bf16(y[e]);
+      } else {
+        const int n = n0 + (wn * NI + j) * 16 + 4 * q;
+        if (!live) continue;
+        const int token = pair / top, choice = pair - token * top;
+        float* to = out + ((size_t)choice * tokens + token) * N + n;
+        floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[e] = n + e < N ? with_extra(acc[i][j][e] * weight, choice, extra, extra_parts, (size_t)tokens * N, (size_t)token * N + n + e) : 0.f;
+        if (n + 3 < N && (N & 3) == 0 && ((uintptr_t)out & 15) == 0) *(floatx4*)to = v;
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) to[e] = v[e];
       }
+    }
   }
 }
 
-// The shape for steps of many rows: the weight tile goes through LDS as the rows do.  Straight into the MFMA
-// operand, a lane asks for 16 bytes of a weight row of its own, and the 64 lanes of a load are 64 accesses of
-// the CU's L1 (measured: 80 million a launch, 312,000 a CU in 473,000 cycles, with the matrix cores busy 14 %);
-// here four neighbouring lanes bring 64 neighbouring bytes of one weight row, a quarter of the accesses, and every
-// wave reads its fragments out of LDS.  Block = 64 rows x 128 columns (MODE 0: and their 128 up columns), K in
-// steps of 32, two stages, operands requested DEPTH steps ahead, one LDS-only barrier a step.  (Rows of 64 bytes
-// with their 16-byte pieces exchanged by the row's number, instead of rows 80 bytes apart, took the bank conflicts
-// from 20 million cycles a launch to none and the launch from 179 to 181 us: they were not what it waits for.
-// Rows and weight tile straight from global memory into LDS (`global_load_lds_dwordx4`, no staging registers,
-// three and four steps deep) gave 3.85 instead of 3.64 ms for a prompt of 2,048 tokens at a width of 2,048.  With
-// the products taken out of this kernel its loads, LDS stores and barriers alone take 124 of the 174 us, and with
-// every block reading the same hot tile 151: neither the depth of the prefetch nor where the bytes come from
-// is what bounds it.  Blocks of 128 rows in this shape need the registers of a whole SIMD a wave: 4.25 ms.)
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, int MODE>
+static int launch_moe_tile(const bf16_t* a, const bf16_t* w, const int* offsets, const int* order, const float* pair_weight,
+                           bf16_t* act, float* out, int experts, int N, int K, int top, int tokens, float limit, float alpha,
+                           int form, const float* extra, int extra_parts, hipStream_t stream) {
+  constexpr int TILE_ROWS = 16 * MI * WM, TILE_COLS = 16 * NI * WN, COLUMNS = MODE == 0 ? TILE_COLS / 2 : TILE_COLS;
+  constexpr size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES;
+  static int checked = 0;
+  auto kernel = moe_lds_kernel<MI, NI, WM, WN, KG, STAGES, MODE>;
+  const int fit = lds_tile::fit_to_launch((const void*)kernel, bytes, &checked);
+  if (fit != FE_OK) return fit;
+  const long long pairs = (long long)tokens * top, slots = pairs / TILE_ROWS + experts, tiles = ((long long)N + COLUMNS - 1) / COLUMNS;
+  const long long blocks = (slots * tiles + 7) / 8 * 8;
+  if (blocks > 0x7fffffffLL) return FE_BAD_ARGUMENT;
+  kernel<<<(unsigned)blocks, 64 * WM * WN * KG, bytes, stream>>>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens,
+                                                                 limit, alpha, form, extra, extra_parts, (int)slots, (int)tiles);
+  return fe_check_launch();
+}
+
+// Which tile (rows x weight rows) a launch takes, by the rows an expert gets on average: few rows want many blocks with deep
+// buffers, each streaming its part of the weight (what bounds them is the weight's bytes), many rows want every weight row read
+// for more of them (what bounds them is the lines that a CU's L1 can wait for, see gemm_lds.h).  Measured on one MI355X, both
+// products and the plan, us, 8 experts as wide as the model, 2 a token (weight straight in registers, or staged through them
+// from 1,024 pairs on -> this): width 2,048 with 1 / 8 / 32 / 100 / 300 / 1,500 / 3,000 tokens 40 -> 26, 57 -> 48, 85 -> 56,
+// 93 -> 64, 98 -> 77, 228 -> 141, 379 -> 270; width 1,024 25 -> 18, 27 -> 19, 28 -> 22, 30 -> 23, 35 -> 27, 73 -> 63, 132 -> 100.
+// At 300 tokens (75 rows an expert) 64 x 64 takes 27 and 77 us, 64 x 128 31 and 72, 32 x 64 32 and 89; at 1,500 (375 rows)
+// 64 x 128 61 and 165, 128 x 128 76 and 199, 256 x 128 63 and 141.
 template <int MODE>
-__global__ __launch_bounds__(256) void moe_grouped_staged_kernel(
-    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ offsets,
-    const int* __restrict__ order, const float* __restrict__ pair_weight, bf16_t* __restrict__ act,
-    float* __restrict__ out, int E, int N, int K, int top, int tokens, float limit, float alpha, int form,
-    const float* __restrict__ extra, int extra_parts, int slots, int column_tiles) {
-  constexpr int COLS = 128, MATS = MODE == 0 ? 2 : 1, NT = 2, MT = 4;
-  __shared__ __attribute__((aligned(16))) bf16_t As[2][TM][TPAD];
-  __shared__ __attribute__((aligned(16))) bf16_t Ws[2][MATS][COLS][TPAD];
-  __shared__ int pair_of[TM];
-  const int items = slots * column_tiles;
-  const int per_die = (items + 7) / 8;
-  const int item = (int)(blockIdx.x % 8) * per_die + (int)(blockIdx.x / 8);
-  if (item >= items) return;
-  int expert, row0, row_end;
-  if (!find_tile<TM>(offsets, E, item % slots, expert, row0, row_end)) return;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, lr = lane % 16, lq = lane / 16;
-  const int n0 = (item / slots) * COLS;
-  if (tid < TM) pair_of[tid] = row0 + tid < row_end ? order[row0 + tid] : -1;
-  __syncthreads();
-  // a thread's 16-byte pieces of a step: row tid / 4 of the rows, weight rows tid / 4 and tid / 4 + 64 of each
-  // matrix, k chunk tid % 4
-  const int my_row = tid / 4, my_chunk = tid % 4;
-  const int my_pair = pair_of[my_row];
-  const size_t src = my_pair < 0 ? 0 : (MODE != 1 ? (size_t)(my_pair / top) : (size_t)(row0 + my_row));
-  const bf16_t* a_at = a + src * K + my_chunk * 8;
-  const size_t w_rows = MODE == 0 ? 2 * (size_t)N : (size_t)N;
-  const bf16_t* w_at[MATS][2];
-#pragma unroll
-  for (int m = 0; m < MATS; ++m)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      w_at[m][j] = w + ((size_t)expert * w_rows + (size_t)m * N + min(n0 + my_row + 64 * j, N - 1)) * K + my_chunk * 8;
-  floatx4 acc[MATS][NT][MT];
-#pragma unroll
-  for (int m = 0; m < MATS; ++m)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[m][nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const uintx4 zero = {0u, 0u, 0u, 0u};
-  constexpr int DEPTH = MODE == 0 ? 2 : 4;      // with two matrices the registers hold two steps' operands beside the sums
-  const int steps = K / TK;
-  uintx4 a_reg[DEPTH], w_reg[DEPTH][MATS][2];
-  auto fetch = [&](int step, int set) {
-    const int at = min(step, steps - 1) * TK;
-    a_reg[set] = *(const uintx4*)(a_at + at);
-#pragma unroll
-    for (int m = 0; m < MATS; ++m)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) w_reg[set][m][j] = *(const uintx4*)(w_at[m][j] + at);
-  };
-  auto stash = [&](int stage, int set) {
-    *(uintx4*)&As[stage][my_row][my_chunk * 8] = my_pair < 0 ? zero : a_reg[set];
-#pragma unroll
-    for (int m = 0; m < MATS; ++m)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) *(uintx4*)&Ws[stage][m][my_row + 64 * j][my_chunk * 8] = w_reg[set][m][j];
-  };
-  auto multiply = [&](int stage) {
-    bf16x8 cols[MATS][NT];
-#pragma unroll
-    for (int m = 0; m < MATS; ++m)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) cols[m][nt] = *(const bf16x8*)&Ws[stage][m][(wave * NT + nt) * 16 + lr][lq * 8];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const bf16x8 rows = *(const bf16x8*)&As[stage][mt * 16 + lr][lq * 8];
-#pragma unroll
-      for (int m = 0; m < MATS; ++m)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          acc[m][nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows, cols[m][nt], acc[m][nt][mt], 0, 0, 0);
-    }
-  };
-#pragma unroll
-  for (int u = 0; u < DEPTH; ++u) fetch(u, u);
-  stash(0, 0);
-  lds_barrier();
-  int step = 0;
-  for (; step + DEPTH <= steps; step += DEPTH) {
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-      // set u went into LDS during the step before: its registers are free, and what is asked for now has
-      // this step's products and the next step's to arrive in
-      fetch(step + u + DEPTH, u);
-      multiply(u & 1);
-      stash((u + 1) & 1, (u + 1) % DEPTH);
-      lds_barrier();
-    }
-  }
-  const int left = steps - step;
-#pragma unroll
-  for (int u = 0; u < DEPTH - 1; ++u)
-    if (u < left) {
-      multiply(u & 1);
-      stash((u + 1) & 1, (u + 1) % DEPTH);
-      lds_barrier();
-    }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = n0 + (wave * NT + nt) * 16 + lr;
-    if (n >= N) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = mt * 16 + lq * 4 + i;
-        const int pair = pair_of[r];
-        if (pair < 0) continue;
-        if (MODE != 1) {
-          act[(size_t)(row0 + r) * N + n] = float_to_bf16(gated(acc[0][nt][mt][i], acc[MATS - 1][nt][mt][i], limit, alpha, form, pair_weight ? pair_weight[pair] : 1.f));
-        } else {
-          const int token = pair / top, choice = pair - token * top;
-          out[((size_t)choice * tokens + token) * N + n] = with_extra(
-              acc[0][nt][mt][i] * (pair_weight ? pair_weight[pair] : 1.f), choice, extra, extra_parts, (size_t)tokens * N, (size_t)token * N + n);
-        }
-      }
-  }
+static int launch_moe(const bf16_t* a, const bf16_t* w, const int* offsets, const int* order, const float* pair_weight,
+                      bf16_t* act, float* out, int experts, int N, int K, int top, int tokens, float limit, float alpha,
+                      int form, const float* extra, int extra_parts, hipStream_t stream) {
+  const long long each = (long long)tokens * top / experts;
+#define FE_GO(...) return launch_moe_tile<__VA_ARGS__, MODE>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens, \
+                                                             limit, alpha, form, extra, extra_parts, stream)
+  if (each <= 32) FE_GO(1, 2, 2, 2, 2, 6);       // 32 x 64
+  if (each <= 96) FE_GO(2, 2, 2, 2, 2, 4);       // 64 x 64
+  if (each < 256) FE_GO(2, 4, 2, 2, 2, 3);       // 64 x 128
+  FE_GO(4, 4, 4, 2, 1, 3);                       // 256 x 128
+#undef FE_GO
 }
-
-// Two groups of columns a wave from this many pairs on (the launch then still has blocks enough).
-#define WIDE_COLUMNS_MIN_PAIRS 1024
-
-// blocks of a launch: the items rounded up to a whole number a die
-static unsigned mfma_blocks(int slots, int column_tiles) { return (unsigned)(((long long)slots * column_tiles + 7) / 8 * 8); }
-
-// Which shape a launch takes: from WIDE_COLUMNS_MIN_PAIRS pairs on the one whose weight tile goes through LDS
-// (a prompt of 2,048 tokens at a width of 2,048: 3.80 -> 3.67 ms against the direct shape with two column groups
-// a wave; at 4,096: 10.0 -> 9.6 ms, where the direct shape with blocks of 128 rows reached 9.9), below that the
-// direct shape with one column group a wave, which streams the weight at 3 to 4.7 TB/s in a decode step.
-#define MFMA_LAUNCH(MODE, COLUMNS, A, W, PW, ACT, OUT, N_, K_, LIMIT, ALPHA, FORM, EXTRA, EXTRA_PARTS)                        \
-  do {                                                                                                                   \
-    const bool wide = pairs >= WIDE_COLUMNS_MIN_PAIRS;                                                                   \
-    const int slots = (int)(pairs / TM + experts);                                                                       \
-    const int tiles = ((COLUMNS) + (wide ? 2 : 1) * TN - 1) / ((wide ? 2 : 1) * TN);                                      \
-    if (wide)                                                                                                            \
-      moe_grouped_staged_kernel<MODE><<<mfma_blocks(slots, tiles), 256, 0, stream>>>(                                    \
-          A, W, offsets, order, PW, ACT, OUT, experts, N_, K_, top, tokens, LIMIT, ALPHA, FORM, EXTRA, EXTRA_PARTS, slots, tiles); \
-    else                                                                                                                 \
-      moe_grouped_mfma_kernel<MODE, 1, 4><<<mfma_blocks(slots, tiles), 256, 0, stream>>>(                                \
-          A, W, offsets, order, PW, ACT, OUT, experts, N_, K_, top, tokens, LIMIT, ALPHA, FORM, EXTRA, EXTRA_PARTS, slots, tiles); \
-  } while (0)
 
 static bool mfma_fits(const void* a, const void* w, int K) {
-  return K % TK == 0 && ((((uintptr_t)a) | ((uintptr_t)w)) & 15) == 0;
+  return K % 32 == 0 && ((((uintptr_t)a) | ((uintptr_t)w)) & 15) == 0;
 }
 
 extern "C" int fe_moe_gate_up(const void* x, const void* gate_up, int dtype, const int* offsets, const int* order, void* act,
@@ -669,7 +505,8 @@ extern "C" int fe_moe_gate_up(const void* x, const void* gate_up, int dtype, con
       moe_grouped_kernel<float, 2><<<grid, 256, 0, stream>>>((const float*)x, (const float*)gate_up, offsets, order, input_weight,
                                                              (float*)act, nullptr, experts, inner, hidden, top, tokens, limit, alpha, form, nullptr, 0);
     else if (dtype == FE_BF16 && mfma_fits(x, gate_up, hidden)) {
-      MFMA_LAUNCH(2, inner, (const bf16_t*)x, (const bf16_t*)gate_up, input_weight, (bf16_t*)act, nullptr, inner, hidden, limit, alpha, form, nullptr, 0);
+      return launch_moe<2>((const bf16_t*)x, (const bf16_t*)gate_up, offsets, order, input_weight, (bf16_t*)act, nullptr, experts, inner, hidden, top,
+                           tokens, limit, alpha, form, nullptr, 0, stream);
     } else if (dtype == FE_BF16)
       moe_grouped_kernel<bf16_t, 2><<<grid, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)gate_up, offsets, order, input_weight,
                                                               (bf16_t*)act, nullptr, experts, inner, hidden, top, tokens, limit,
@@ -682,7 +519,8 @@ extern "C" int fe_moe_gate_up(const void* x, const void* gate_up, int dtype, con
     moe_grouped_kernel<float, 0><<<grid, 256, 0, stream>>>((const float*)x, (const float*)gate_up, offsets, order, input_weight,
                                                            (float*)act, nullptr, experts, inner, hidden, top, tokens, limit, alpha, form, nullptr, 0);
   else if (dtype == FE_BF16 && mfma_fits(x, gate_up, hidden)) {
-    MFMA_LAUNCH(0, inner, (const bf16_t*)x, (const bf16_t*)gate_up, input_weight, (bf16_t*)act, nullptr, inner, hidden, limit, alpha, form, nullptr, 0);
+    return launch_moe<0>((const bf16_t*)x, (const bf16_t*)gate_up, offsets, order, input_weight, (bf16_t*)act, nullptr, experts, inner, hidden, top,
+                         tokens, limit, alpha, form, nullptr, 0, stream);
   } else if (dtype == FE_BF16)
     moe_grouped_kernel<bf16_t, 0><<<grid, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)gate_up, offsets, order, input_weight,
                                                             (bf16_t*)act, nullptr, experts, inner, hidden, top, tokens, limit,
@@ -704,7 +542,8 @@ extern "C" int fe_moe_down(const void* act, const void* down, int dtype, const i
                                                            nullptr, out, experts, hidden, inner, top, tokens, 0.f, 0.f, 0, extra,
                                                            extra_parts);
   else if (dtype == FE_BF16 && mfma_fits(act, down, inner)) {
-    MFMA_LAUNCH(1, hidden, (const bf16_t*)act, (const bf16_t*)down, pair_weight, nullptr, out, hidden, inner, 0.f, 0.f, 0, extra, extra_parts);
+    return launch_moe<1>((const bf16_t*)act, (const bf16_t*)down, offsets, order, pair_weight, nullptr, out, experts, hidden, inner, top, tokens, 0.f, 0.f,
+                         0, extra, extra_parts, stream);
   } else if (dtype == FE_BF16)
     moe_grouped_kernel<bf16_t, 1><<<grid, 256, 0, stream>>>((const bf16_t*)act, (const bf16_t*)down, offsets, order, pair_weight,
                                                             nullptr, out, experts, hidden, inner, top, tokens, 0.f, 0.f, 0, extra,

@@ -170,6 +170,44 @@ def test_mixture_of_experts_kernels(tokens, hidden, experts, top, inner, dtype):
     close(ops.linear_gated(x.to(DEV), shared.to(DEV), limit=0.8, alpha=1.702), refs.linear_gated(x, shared, limit=0.8, alpha=1.702), dtype)
 
 
+@pytest.mark.parametrize("tokens,hidden,experts,top,inner", [
+    (3, 96, 130, 2, 33), (40, 128, 70, 3, 100),                 # more experts than a wave has lanes, few rows each
+    (65, 160, 2, 1, 70), (150, 64, 3, 2, 130),                  # 32 to 100 rows an expert
+    (190, 224, 2, 2, 129), (300, 96, 1, 1, 260),                # 190 and 300: the wider tiles
+    (1030, 192, 4, 1, 34)])
+@pytest.mark.parametrize("weight_input", [False, True])
+def test_grouped_products_tiles(tokens, hidden, experts, top, inner, weight_input):
+    """Every tile of the grouped products, rows and columns beside its edges, K ending in half a step, some experts without
+    rows: against the same products in 64 bits, with the middle rounded to bfloat16 as the kernels round it."""
+    from forge_engine_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(tokens + inner)
+
+    def draw(*shape, scale=1.0):
+        return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
+
+    x, gate_up, down = draw(tokens, hidden), draw(experts, 2 * inner, hidden, scale=hidden ** -0.5), draw(experts, hidden, inner, scale=inner ** -0.5)
+    chosen = torch.rand(tokens, experts, generator=g, device=DEV).argsort(1)[:, :top].int()
+    if experts > 1:
+        chosen[chosen == experts - 1] = 0 if top == 1 else experts - 1      # (one choice a token: the last expert gets nothing)
+    weights = torch.rand(tokens, top, generator=g, device=DEV)
+    got = ops.moe_experts(x, chosen, weights, gate_up, down, torch.full((top, tokens, hidden), float("nan"), device=DEV), limit=2.0,
+                          alpha=1.702, weight_input=weight_input)
+    want = torch.zeros(top, tokens, hidden, dtype=torch.float64, device=DEV)
+    for k in range(top):
+        for e in chosen[:, k].unique().tolist():
+            mine = (chosen[:, k] == e).nonzero().flatten()
+            both = x[mine].double() @ gate_up[e].double().t()
+            w = weights[mine, k, None].double()
+            if weight_input:
+                both = both * w
+            gate, up = both[:, :inner].clamp(max=2.0), both[:, inner:].clamp(-2.0, 2.0)
+            act = (gate * torch.sigmoid(1.702 * gate) * (up + 1.0)).float().bfloat16().double()
+            want[k, mine] = act @ down[e].double().t() * (1.0 if weight_input else w)
+    # the middle may round the other way where a float32 sum lies beside a tie: 2^-8 of one of `inner` terms of size inner^-0.5 each
+    torch.testing.assert_close(got.double(), want, atol=2e-2, rtol=1e-3)
+    assert float((got.double() - want).norm() / want.norm()) < 1e-3
+
+
 # ------------------------------------------------------------------ the model
 
 @pytest.fixture(scope="module")

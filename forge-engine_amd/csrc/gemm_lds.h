@@ -1,5 +1,5 @@
-// The product for portions (gemm_wide.hip) with both operands in LDS: dozens to hundreds of rows of x (many requests
-// decoding, a portion of a prompt):
+// The product for portions (gemm_wide.hip) with both operands in LDS: one to hundreds of rows of x (requests decoding, a
+// portion of a prompt):
 //   out[M, N] = x[M, K] * W[N, K]^T
 // with one of three endings: float32 partial sums over parts of K ([parts][M, N]; the consumer, the next norm or the
 // attention launch, adds them in order), bfloat16, or act(gate) * up as bfloat16 for a fused gate/up weight.
@@ -19,6 +19,13 @@
 // 21 -> 15; down projection of 2,560 x 9,728 at 64 / 256 / 512 rows 14.6 -> 12, 25.5 -> 22, 48 -> 32; gate/up of
 // 3,072 x 1,024 at 384 rows 18.0 -> 13.5.  Starting the blocks' walks over K at different places changes nothing (no
 // memory channel is hot), nor do four stages instead of three.  From 1,500 rows on the matrix library is ahead.
+//
+// Up to 16 rows of x, tiles of 16 rows with one fragment a wave: the weight's bytes are nearly all of the tile's, so the widths
+// (16 to 80 weight rows) only choose how evenly the CUs share them, and 8 to 12 stages keep 64 KB and more of a CU's share in
+// flight; the kernels with the weight in registers had a wave's two to four steps, and read x again for every 16 weight rows
+// (gemm_skinny) or gave a block 64 weight rows whatever the weight (gemm_wide).  8 rows, before -> this: gate/up of 3,072 x
+// 1,024 8.3 -> 5.7, of 6,144 x 2,048 14.4 -> 12.8, of 9,728 x 2,560 22.4 -> 21.1; updates of 1,024 x 2,048 5.0 -> 3.1,
+// of 2,560 x 9,728 12.2 -> 11.6; q/k/v of 4,096 x 1,024 4.7 -> 4.2; 6,144 x 2,048 stored 9.2 -> 7.7.
 //
 // MFMA 16x16x32 bf16 with A = W (16 weight rows), B = x^T (16 rows of x): lane l (r = l % 16, q = l / 16) supplies row r,
 // k = 8 q .. + 8 of either and receives D[weight row 4 q + i][row of x r]: four neighbouring output columns of a row.
@@ -129,7 +136,7 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
 
 // Operands and endings as fe_gemm_wide's (ending 0: parts, 1: bfloat16, 2: gated); the caller has checked them.
 // tile: rows of x x weight rows a block takes: 0: 32 x 32, 1: 64 x 32, 2: 64 x 64, 3: 64 x 80, 4: 64 x 96, 5: 128 x 64,
-//   6: 128 x 128, 7: 128 x 160, 8: 32 x 64.
+//   6: 128 x 128, 7: 128 x 160, 8: 32 x 64, 9 to 13: 16 x 16, 32, 48, 64, 80.
 // FE_BAD_ARGUMENT also if the library was built with registers spilled to scratch memory: the kernel then never runs.
 static int launch(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
                   int parts, long long part_stride, int tile, GateAct act, hipStream_t stream) {
@@ -150,6 +157,11 @@ static int launch(const void* x, const void* w, void* out, int M, int N, int K, 
     FE_TILE(6, 4, 4, 2, 2, 2, 4)
     FE_TILE(7, 4, 5, 2, 2, 2, 3)
     FE_TILE(8, 1, 2, 2, 2, 2, 6)
+    FE_TILE(9, 1, 1, 1, 1, 2, 12)
+    FE_TILE(10, 1, 1, 1, 2, 2, 12)
+    FE_TILE(11, 1, 1, 1, 3, 2, 9)
+    FE_TILE(12, 1, 1, 1, 4, 2, 8)
+    FE_TILE(13, 1, 1, 1, 5, 2, 10)
   }
 #undef FE_TILE
 #undef FE_END

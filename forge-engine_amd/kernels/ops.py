@@ -268,7 +268,9 @@ def gemm_skinny(x: Tensor, weight: Tensor, epilogue: str = "bf16", tiles: int = 
     return out
 
 
-# Which kernel takes a product of up to 16 rows, measured in the decode step at the sizes of Qwen3-4B, 8B and 32B
+# Up to 16 rows of x the product through LDS (``gemm_lds``, below) goes first wherever it fits (K of at least 1,024 in whole
+# 64-steps, 512 weight rows) and wins: see ``_lds_update``, ``_lds_store_pays``, ``_lds_gate_pays`` and ``linear_in_parts``.
+# Which kernel takes the rest, measured in the decode step at the sizes of Qwen3-4B, 8B and 32B
 # (hidden 2560 / 4096 / 5120; milliseconds a step before -> after at the batch named).  The kernels for up to 16
 # rows (`fe_gemm_skinny`) were shaped at 8 rows of the 4B sizes; the product for portions (`fe_gemm_wide`: a tile
 # of 16 rows of x in LDS, 64 weight rows a block, K in the parts that fill the CUs) turned out faster for:
@@ -312,7 +314,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
 
     float32 weights go through the true float32 kernel (a weight stored in
     32-bit stays 32-bit even in a bfloat16 model; the activation is widened).
-    bfloat16: up to 16 rows take the weight-streaming kernel and up to 256 rows the
+    bfloat16: up to 16 rows take the weight-streaming kernel or, like up to 256 rows, the
     product for portions, where the measurements above and below say they win; the
     rest is the platform's matrix library's, which the reference uses for every
     projection (its nn.Linear calls, qwen3.py:115-122,215-223).
@@ -325,12 +327,13 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
         return y if out_dtype == torch.float32 else y.to(out_dtype)
     if x.dtype != weight.dtype:
         raise KernelError(f"activation {x.dtype} does not match weight {weight.dtype}")
-    if (bias is None and _skinny_fits(x, weight) and out_dtype in (torch.float32, torch.bfloat16)
-            and not (out_dtype == torch.bfloat16 and _few_rows_to_library(x, weight))):
-        return gemm_skinny(x, weight, "f32" if out_dtype == torch.float32 else "bf16")
-    if bias is None and out_dtype == torch.bfloat16 and _lds_fits(x, weight) and _lds_store_pays(x.shape[0], *weight.shape):
+    to_library = out_dtype == torch.bfloat16 and _few_rows_to_library(x, weight)
+    if (bias is None and out_dtype == torch.bfloat16 and not to_library and _lds_fits(x, weight)
+            and _lds_store_pays(x.shape[0], *weight.shape)):
         tile, _ = lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])
         return gemm_lds(x, weight, "bf16", tile=tile)
+    if bias is None and _skinny_fits(x, weight) and out_dtype in (torch.float32, torch.bfloat16) and not to_library:
+        return gemm_skinny(x, weight, "f32" if out_dtype == torch.float32 else "bf16")
     if (bias is None and out_dtype == torch.bfloat16 and _wide_fits(x, weight, WIDE_STORE_MAX_ROWS, SKINNY_MAX_ROWS + 1)
             and _wide_store_pays(x.shape[0], weight.shape[0], weight.shape[1])):
         rows = x.shape[0]        # up to 64 rows: blocks of 32 weight rows, so that the launch has twice the blocks
@@ -469,11 +472,12 @@ def _wide_parts(m: int, n: int, k: int, block_rows: int = 64, most: int = 16) ->
     return -(-steps // -(-steps // best))
 
 
-# The product for portions with both operands through LDS (``gemm_lds``), 17 rows and more: its tiles (rows of x, weight rows,
-# blocks a CU holds at a time) with the microseconds a 64-step of K takes a CU that holds one block and two (or, where it
-# holds one at a time, one after the other).
+# The product for portions with both operands through LDS (``gemm_lds``): its tiles (rows of x, weight rows, blocks a CU holds
+# at a time) with the microseconds a 64-step of K takes a CU that holds one block and two (or, where it holds one at a time,
+# one after the other).  Tiles of 16 rows serve up to 16 rows of x, the others more.
 LDS_TILES = ((32, 32, 2, 0.151, 0.256), (64, 32, 1, 0.191, 0.382), (64, 64, 2, 0.212, 0.348), (64, 80, 1, 0.303, 0.606),
-             (64, 96, 2, 0.292, 0.451), (128, 64, 1, 0.317, 0.634), (128, 128, 1, 0.510, 1.02), (128, 160, 1, 0.630, 1.26), (32, 64, 2, 0.202, 0.378))
+             (64, 96, 2, 0.292, 0.451), (128, 64, 1, 0.317, 0.634), (128, 128, 1, 0.510, 1.02), (128, 160, 1, 0.630, 1.26), (32, 64, 2, 0.202, 0.378),
+             (16, 16, 2, 0.073, 0.117), (16, 32, 2, 0.116, 0.247), (16, 48, 2, 0.143, 0.334), (16, 64, 2, 0.168, 0.444), (16, 80, 1, 0.220, 0.440))
 LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
 
@@ -483,19 +487,25 @@ def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int =
     """(tile, parts of K) for ``gemm_lds``: the least of what a launch is predicted to take.  A block's steps take its CU
     what the table says, the chip reads the weight at 5.4 TB/s (slower with fewer blocks than CUs) and pulls 20 TB/s of
     tiles at best; whichever is slowest bounds the launch.  Fitted to 3,300 launches (25 weights of 1,024 to 17,408 rows,
-    17 to 1,024 rows of x, every tile, 1 to 8 parts): the picks take 1 % longer than the best of these tiles.
+    17 to 1,024 rows of x, every tile, 1 to 8 parts): the picks take 1 % longer than the best of these tiles.  Up to 16 rows
+    the reading rate, the tiles' rate and the cost of a part have values of their own (4,500 launches, 27 weights of 512 to
+    34,816 rows, 1 to 16 rows of x: the picks take 2 % longer than the best in parts, 0.3 % whole).
     ``consumer_us``: what each part costs the consumer that adds them up."""
     steps = k // 64
     best = None
+    few = m <= SKINNY_MAX_ROWS
+    read, alone, pull, store = (1.74e-7, 0.27, 8.8e-8, 1.33e-6) if few else (1.84e-7, 0.35, 4.9e-8, 3.1e-7)
     for tile, (rows, columns, held, one, two) in enumerate(LDS_TILES):
+        if few != (rows == 16):
+            continue
         for parts in range(1, max(1, min(most_parts, steps // 4)) + 1):
             tiles = -(-m // rows) * -(-weight_rows // columns) * parts
             rounds = -(-tiles // 256)
             step = one * rounds if held == 1 or rounds == 1 else two * -(-rounds // 2)
             part_steps = -(-steps // parts)
-            bounds = (part_steps * step, weight_rows * k * 2 * 1.84e-7 * (256 / min(256, tiles)) ** 0.35,
-                      tiles * part_steps * (rows + columns) * 128 * 4.9e-8)
-            us = sum(b ** 4 for b in bounds) ** 0.25 + parts * (m * bytes_out * 3.1e-7 + consumer_us)
+            bounds = (part_steps * step, weight_rows * k * 2 * read * (256 / min(256, tiles)) ** alone,
+                      tiles * part_steps * (rows + columns) * 128 * pull)
+            us = sum(b ** 4 for b in bounds) ** 0.25 + parts * (m * bytes_out * store + consumer_us + 0.05 * few)
             if best is None or us < best[0]:
                 best = (us, tile, parts)
     return best[1], best[2]
@@ -503,18 +513,23 @@ def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int =
 
 def _lds_fits(x: Tensor, weight: Tensor) -> bool:
     return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
-            and x.shape[0] > SKINNY_MAX_ROWS and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
+            and x.shape[0] > 0 and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
             and x.shape[1] >= LDS_MIN_K and x.shape[1] % 64 == 0 and weight.shape[0] >= LDS_MIN_WEIGHT_ROWS
             and weight.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
-    """(tile, parts) of a float32 update, or None where another product is the better one.  Up to 64 rows: weights of up to
+    """(tile, parts) of a float32 update, or None where another product is the better one.  Up to 16 rows: weights of up to
+    3,072 rows (1,024 x 3,072 at 1 row 5.8 -> 3.7 us, 2,560 x 4,096 at 8 rows 7.0 -> 6.6) and others whose K is at least twice
+    their rows (4,096 x 12,288 at 1 row 21.3 -> 19.7); beside them the products below tie or win (4,096 x 4,096 at 1 row 8.5
+    against 9.4, 8,192 x 4,096 15.0 against 16.7).  Up to 64 rows: weights of up to
     2,048 x 4,096 by the plan (1,024 x 2,048 at 64 rows 6.5 -> 4.9 us), larger ones in the parts that fill the chip with
     blocks of 64 weight rows (2,560 x 9,728 14.6 -> 12.9, 4,096 x 12,288 25.9 -> 23.4, at 32 rows 13.1 -> 11.6 and 22.8 ->
     20.9).  Up to 384 rows all by the plan, and up to 1,024 through weights whose K is at least twice their rows, which the
     matrix library cuts into too few blocks (512 rows: 2,560 x 9,728 48 -> 33, 5,120 x 17,408 169 -> 86)."""
-    if rows <= MID_ROWS and not (weight_rows <= 2048 and k <= 4096):
+    if rows <= SKINNY_MAX_ROWS and not (weight_rows <= 3072 or k >= 2 * weight_rows):
+        return None
+    if SKINNY_MAX_ROWS < rows <= MID_ROWS and not (weight_rows <= 2048 and k <= 4096):
         if weight_rows > WIDE_MAX_WEIGHT_ROWS:
             return None
         return (8 if rows <= 32 else 2), _wide_parts(rows, weight_rows, k)
@@ -524,16 +539,25 @@ def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
 
 
 def _lds_store_pays(rows: int, weight_rows: int, k: int) -> bool:
-    """Products that store bfloat16: up to 256 rows, 512 through weights of up to 4,096 rows (beyond, the library ties or
+    """Products that store bfloat16.  Up to 8 rows where K is 2,048 and more and the weight has up to 8,192 rows, from five rows
+    (8 rows: 6,144 x 2,048 9.2 -> 7.7 us, 2,048 x 2,048 5.5 -> 5.4, but 4,096 x 1,024 4.23 -> 4.28 and 12,288 x 2,048 12.4 ->
+    12.8; 4 rows: 2,048 x 2,048 5.2 -> 5.4), 9 to 16 rows always (1,024 x 1,024 3.9 -> 3.7, 6,144 x 2,560 14.7 -> 9.6).
+    Beyond, up to 256 rows, 512 through weights of up to 4,096 rows (beyond, the library ties or
     wins: 6,144 x 2,560 at 320 rows 18.6 against 19.9 us), weights of 2,048 rows (1,024: 7.7 against 8.4 us at 192 rows) to
     50 MB (10,240 x 5,120 at 64 rows 32.6 against 33.9)."""
+    if rows <= SKINNY_MAX_ROWS:
+        return rows > 8 or (rows > 4 and k >= 2048 and weight_rows <= 8192)
     return weight_rows >= 2048 and weight_rows * k <= 26_000_000 and rows <= (512 if weight_rows <= 4096 else 256)
 
 
-def _lds_gate_pays(rows: int, columns: int) -> bool:
-    """Gate/up products: where tiles of 128 x 160 make one round of the chip (3,072 columns up to 700 rows: 22 -> 20 us, 6,144
+def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
+    """Gate/up products.  Up to 16 rows all (1 row: 3,072 columns of K = 1,024 7.9 -> 5.5 us, 9,728 of 2,560 21.9 -> 21.0,
+    17,408 of 5,120 70.8 -> 62.6) but the weights of K = 4,096 at up to four rows, whose blocks keep x in registers (1 row:
+    12,288 columns 37.4 against 38.9, 4,096 columns 15.6 against 16.8).  Beyond, where tiles of 128 x 160 make one round of the chip (3,072 columns up to 700 rows: 22 -> 20 us, 6,144
     up to 384: 33 -> 30, 9,728 up to 256: 54 -> 42, 12,288 up to 128); with a second round the matrix library's larger
     tiles win (9,728 columns at 320 rows: 50 against 59 us)."""
+    if rows <= SKINNY_MAX_ROWS:
+        return rows > 4 or not (GATE_HALF_FEW_ROWS_MAX_K < k <= 4096 and columns >= 4096)
     return -(-rows // 128) * -(-2 * columns // 160) <= WIDE_CUS
 
 
@@ -574,6 +598,10 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     plain_bf16 = bias is None and weight.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
+    if plain_bf16 and _lds_fits(x, weight):
+        plan = _lds_update(x.shape[0], *weight.shape)
+        if plan is not None:
+            return gemm_lds(x, weight, "parts", plan[1], plan[0])
     if plain_bf16 and FEW_ROWS_UPDATE < x.shape[0] <= SKINNY_MAX_ROWS and _wide_fits(x, weight, SKINNY_MAX_ROWS, 1):
         # a tile of 16 rows of x: a tile's rows beyond M are fetched and multiplied like the others (with tiles of
         # 64 rows: 4B, batch 16: 3.05 -> 3.00 ms; 32B: 15.4 -> 14.9; tiles of 32 rows for 17 to 32 rows lose 2 to 6 %)
@@ -586,10 +614,6 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
                             UPDATE_SPLIT_BLOCKS // tiles))
         splits = -(-steps // -(-steps // splits))        # parts of equal length, none empty
         return gemm_skinny(x, weight, "f32", tiles=1, waves=4, splits=splits)
-    if plain_bf16 and _lds_fits(x, weight):
-        plan = _lds_update(x.shape[0], *weight.shape)
-        if plan is not None:
-            return gemm_lds(x, weight, "parts", plan[1], plan[0])
     if plain_bf16 and _wide_fits(x, weight, MID_ROWS, SKINNY_MAX_ROWS + 1):
         # 17 to 64 rows: one tile of x a block, the parts of K that fill the CUs; measured at 64 rows against
         # the product below: output projection 9.2 against 11.1 us (hidden size 4096: 10.6 against 12.5),
@@ -632,6 +656,12 @@ def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
     rows = x.shape[0]
     if _few_rows_to_library(x, weight):
         return None
+    if (rows <= SKINNY_MAX_ROWS and _lds_fits(x, weight)
+            and (rows > FEW_ROWS_IN_PARTS or weight.shape[0] <= (6144 if weight.shape[1] >= 2048 else 4096))):
+        # (8 rows: 4,096 x 1,024 4.7 -> 4.2 us, 6,144 x 2,560 8.6 -> 8.4, 4,096 x 4,096 10.8 -> 9.4; up to four rows through a
+        # larger weight the kernels below tie or win: 6,144 x 1,024 at 1 row 4.9 against 5.4, 8,192 x 4,096 15.9 against 16.7)
+        tile, parts = lds_plan(rows, weight.shape[0], weight.shape[1], 4 * weight.shape[0], 4, 0.15 + rows * weight.shape[0] * 8e-7)
+        return gemm_lds(x, weight, "parts", parts, tile)
     if FEW_ROWS_IN_PARTS < rows <= SKINNY_MAX_ROWS and _wide_fits(x, weight, SKINNY_MAX_ROWS, 1):
         # blocks of 32 weight rows in up to four parts of K (768 blocks for 6144 weight rows): 1 % of the step
         # at 6 to 16 rows against the kernels below (4B, batch 8: 2.74 -> 2.71 ms; 8B: 3.93 -> 3.89)
@@ -700,11 +730,12 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tenso
             and x.data_ptr() % 16 == 0 and gate_up_weight.data_ptr() % 16 == 0
             and gate_up_weight.shape[0] * gate_up_weight.stride(0) < 2 ** 32 and rows * x.shape[1] < 2 ** 32):
         return gemm_gated(x, gate_up_weight, shape=3, act=act)
-    if (gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight) and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2)):
-        tile, _ = lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])
-        return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
     to_library = (2 <= rows <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
                   and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
+    if (not to_library and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
+            and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])):
+        tile, _ = lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])
+        return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
     paired_fits = (rows <= MID_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16
                    and x.is_contiguous() and gate_up_weight.is_contiguous() and x.shape[1] % 64 == 0
                    and x.shape[1] <= WIDE_GATE_MAX_K and gate_up_weight.shape[0] % 2 == 0

@@ -898,8 +898,8 @@ def test_linear_swiglu_routes_by_rows(ops, monkeypatch):
         torch.testing.assert_close(got, refs.linear_swiglu(x, weight).float(), atol=2e-2, rtol=2e-2)
 
 
-@pytest.mark.parametrize("tile", range(9))
-@pytest.mark.parametrize("m,n,k,parts", [(1, 8, 64, 1), (31, 33, 128, 2), (64, 80, 192, 2), (65, 97, 640, 3), (129, 161, 1024, 5), (257, 330, 704, 4)])
+@pytest.mark.parametrize("tile", range(14))
+@pytest.mark.parametrize("m,n,k,parts", [(1, 8, 64, 1), (16, 41, 1344, 1), (31, 33, 128, 2), (64, 80, 192, 2), (65, 97, 640, 3), (129, 161, 1024, 5), (257, 330, 704, 4)])
 def test_gemm_lds(ops, tile, m, n, k, parts):
     """Every tile at its edges and remainders, K in equal and unequal parts (and one without steps), a weight that is a slice
     of a wider one.  float32 parts against the exact products of the bfloat16 operands: |error| <= 2 k 2^-24 sum |a||b|."""
@@ -928,7 +928,7 @@ def test_gemm_lds_refuses_and_plans(ops, monkeypatch):
     x = torch.zeros(70, 1024, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(4096, 1024, dtype=torch.bfloat16, device=DEV)
     for bad in (lambda: ops.gemm_lds(x, w, "bf16", 2), lambda: ops.gemm_lds(x, w, "parts", 65), lambda: ops.gemm_lds(x, w[:, :1000], "parts"),
-                lambda: ops.gemm_lds(x, w, "swiglu"), lambda: ops.gemm_lds(x, w, "bf16", tile=9), lambda: ops.gemm_lds(x, w[:, :960], "bf16"),
+                lambda: ops.gemm_lds(x, w, "swiglu"), lambda: ops.gemm_lds(x, w, "bf16", tile=14), lambda: ops.gemm_lds(x, w[:, :960], "bf16"),
                 lambda: ops.gemm_lds(x, w.float(), "bf16")):
         with pytest.raises(ops.KernelError):
             bad()
@@ -937,7 +937,12 @@ def test_gemm_lds_refuses_and_plans(ops, monkeypatch):
     real = ops.gemm_lds
     monkeypatch.setattr(ops, "gemm_lds", lambda *a, **kw: taken.append("lds") or real(*a, **kw))
     g = torch.Generator().manual_seed(9)
-    for rows, n, k, kind, own in ((17, 4096, 1024, "store", True), (16, 4096, 1024, "store", False), (512, 4096, 1024, "store", True),
+    for rows, n, k, kind, own in ((17, 4096, 1024, "store", True), (16, 4096, 1024, "store", True), (8, 4096, 1024, "store", False), (8, 8192, 2048, "store", True),
+                                  (8, 8208, 2048, "store", False), (4, 4096, 2048, "store", False), (1, 3072, 1024, "update", True),
+                                  (1, 3088, 1024, "update", False), (16, 3088, 6208, "update", True), (5, 4096, 1024, "parts", True),
+                                  (5, 8192, 1024, "parts", True), (4, 4096, 1024, "parts", True), (4, 4112, 1024, "parts", False),
+                                  (4, 6144, 2048, "parts", True), (1, 512, 1024, "gate", True), (4, 4096, 4096, "gate", False),
+                                  (5, 4096, 4096, "gate", True), (16, 3072, 960, "gate", False), (512, 4096, 1024, "store", True),
                                   (513, 4096, 1024, "store", False), (257, 4160, 1024, "store", False), (256, 4160, 1024, "store", True),
                                   (100, 1984, 1024, "store", False), (17, 512, 2048, "update", True), (1024, 512, 1024, "update", True),
                                   (1025, 512, 1024, "update", False), (400, 1024, 1024, "update", False), (384, 1024, 1024, "update", True),
@@ -946,7 +951,7 @@ def test_gemm_lds_refuses_and_plans(ops, monkeypatch):
         x = rand(g, rows, k, dtype=torch.bfloat16).to(DEV)
         w = rand(g, n * (2 if kind == "gate" else 1), k, dtype=torch.bfloat16, scale=0.02).to(DEV)
         taken.clear()
-        got = {"store": ops.linear, "update": ops.linear_update, "gate": ops.linear_swiglu}[kind](x, w)
+        got = {"store": ops.linear, "update": ops.linear_update, "gate": ops.linear_swiglu, "parts": ops.linear_in_parts}[kind](x, w)
         assert bool(taken) == own, (rows, n, k, kind, taken)
         want = x.float() @ w.float().t()
         if kind == "gate":

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   constexpr int KC = D / 32;        // MFMA k-steps over the head dim (scores)
   constexpr int DT = D / 16;        // 16-dim tiles of the output
   constexpr int PARTS = WAVES + (PREPARE ? 1 : 0);   // partial results that meet in LDS
-  __shared__ float Ow[PARTS][GMAX][D];
+  __shared__ __attribute__((aligned(16))) float Ow[PARTS][GMAX][D];
   __shared__ float Ms[PARTS][GMAX], Ls[PARTS][GMAX];
 
   const int split = blockIdx.x, splits = gridDim.x;
@@ -312,6 +312,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   int kr1 = raw_page((b0 + WAVES) * KEYS + krow);
   int v1 = raw_page((b0 + WAVES) * KEYS + 8 * lq);
   int kr0 = 0;
+  const int new_page = PREPARE ? raw_page(ctx - 1) : 0;      // of the new token
   fetch_keys(b0, checked(kraw0, b0 * KEYS + krow), k0);
 
   // What the requests above brought, while the keys are on their way: the rotation's cosines and
@@ -340,6 +341,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   }
 
   bool extra = false;       // this block also brings the new token's own key and value
+  uintx4 fresh = {0u, 0u, 0u, 0u};     // in the last wave: 8 elements of the new key (lanes below D / 8) or of the new value (the D / 8 after them)
   if constexpr (PREPARE) {
     __syncthreads();        // cos_s, sin_s, raw_s (the keys requested above stay in flight)
     if constexpr (FROM_SUMS) {
@@ -404,14 +406,11 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       __shared__ __attribute__((aligned(16))) bf16_t new_key[D];
       const int sub = lane & (LPH - 1);
       const int role = lane / LPH;               // 0: key, 1: value, others idle (they follow the key's path)
-      const int pos = ctx - 1;
       const bf16_t* row = q + (size_t)q0 * q_stride;
       const size_t k_at = (size_t)(kv_heads * groups + hk) * D, v_at = k_at + (size_t)kv_heads * D;
       uint4 raw;
       if constexpr (FROM_SUMS) raw = *(const uint4*)&raw_s[(groups + (role == 1 ? 1 : 0)) * D + sub * 8];
       else raw = *(const uint4*)(row + (role == 1 ? v_at : k_at) + sub * 8);
-      const int block = table[min(pos >> block_shift, table_last)];
-      const bool writable = block >= 0 && block < num_blocks;     // the host reserves pages before the launch
       const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
       float v[8];
       unpack_bf16x8(w4, v);
@@ -435,23 +434,22 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       }
       uint32_t k4[4];
       pack_bf16x8(r, k4);
-      const size_t page = (size_t)(writable ? block : 0) * kv_heads + hk;
       if (role == 0) {
-        *(uint4*)&new_key[sub * 8] = make_uint4(k4[0], k4[1], k4[2], k4[3]);
-        if (writable)
-          *(uint4*)(const_cast<bf16_t*>(key_pages) + ((page << block_shift) + (pos & block_mask)) * D + sub * 8) =
-              make_uint4(k4[0], k4[1], k4[2], k4[3]);
+        fresh = uintx4{k4[0], k4[1], k4[2], k4[3]};
+        *(uintx4*)&new_key[sub * 8] = fresh;
       } else if (role == 1) {
-        bf16_t* vdst = const_cast<bf16_t*>(value_pages) + ((page * D) << block_shift) + (pos & block_mask);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bf16_t bits = (bf16_t)(e & 1 ? w4[e >> 1] >> 16 : w4[e >> 1] & 0xffffu);
-          if (writable) vdst[(size_t)(sub * 8 + e) << block_shift] = bits;
-          for (int g = 0; g < groups; ++g) Ow[WAVES][g][sub * 8 + e] = bf16_to_float(bits);
+        fresh = __builtin_bit_cast(uintx4, raw);
+        float value[8];
+        unpack_bf16x8(w4, value);
+        for (int g = 0; g < groups; ++g) {
+          *(float4*)&Ow[WAVES][g][sub * 8] = make_float4(value[0], value[1], value[2], value[3]);
+          *(float4*)&Ow[WAVES][g][sub * 8 + 4] = make_float4(value[4], value[5], value[6], value[7]);
         }
       }
+      // new_key is read by other lanes of this wave: a wave's LDS accesses are served in order, so the compiler alone
+      // has to keep them in order (a fence would also wait for the keys under way and for the stores to the pages)
+      asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
-      __threadfence_block();                     // new_key is read by other lanes of this wave
       float dot = 0.f;
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
@@ -469,6 +467,26 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       if (lq == 0 && lr < groups) { Ms[WAVES][lr] = dot * scale_log2; Ls[WAVES][lr] = 1.f; }
     }
   }
+
+  // The new token's key and value go to their pages last of all: a wave's loads and stores are counted together, so the
+  // last wave would wait for these stores (a value's elements lie in as many lines) wherever it next waits for a load.
+  // (Left out altogether from behind its first keys: 38.9 -> 36.4 us at 64 sequences of 706 keys.  Moved here, with the
+  // hardware's rounding to bfloat16: 36.9 -> 35.0 us, one sequence of 217 keys 7.6 -> 7.0.)
+  auto write_pages = [&]() {
+    if constexpr (PREPARE) {
+      constexpr int LPH = D / 8;
+      if (!extra || wave != WAVES - 1 || lane >= 2 * LPH || new_page < 0 || new_page >= num_blocks) return;   // (the host reserves pages before the launch)
+      const int sub = lane & (LPH - 1), slot = (ctx - 1) & block_mask;
+      const size_t page = (size_t)new_page * kv_heads + hk;
+      if (lane < LPH) {
+        *(uintx4*)(const_cast<bf16_t*>(key_pages) + ((page << block_shift) + slot) * D + sub * 8) = fresh;
+      } else {
+        bf16_t* vdst = const_cast<bf16_t*>(value_pages) + ((page * D) << block_shift) + slot;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vdst[(size_t)(sub * 8 + e) << block_shift] = (bf16_t)(e & 1 ? fresh[e >> 1] >> 16 : fresh[e >> 1] & 0xffffu);
+      }
+    }
+  };
 
   for (int b = b0; b < my_last; b += 2 * WAVES) {
     step(b, k0, k1, v0, kr1, kr0);
@@ -519,7 +537,10 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       }
     }
   }
-  if (splits == 1) return;
+  if (splits == 1) {
+    write_pages();
+    return;
+  }
 
   // The block that finishes last among the splits of this (sequence, kv head) merges them.  The
   // parts are written and read with device-scope accesses that go past the per-die L2 caches,
@@ -543,7 +564,10 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     if (is_last) atomicExch(counter, 0);
   }
   __syncthreads();
-  if (!is_last) return;
+  if (!is_last) {
+    write_pages();
+    return;
+  }
   const size_t first_part = ((size_t)seq * kv_heads + hk) * splits;
   if (splits <= 16) {
     // few splits: every thread reads the statistics of its row itself, together with its share
@@ -556,6 +580,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       else if (splits <= 8) *dst = merge_few<8>(part_o, part_ml, first_part, splits, groups, g, D, d, sink2);
       else *dst = merge_few<16>(part_o, part_ml, first_part, splits, groups, g, D, d, sink2);
     }
+    write_pages();
     return;
   }
   // more: rounds of sixteen, each round's loads all in flight at once, the rounds' shares brought to one maximum as they
@@ -593,6 +618,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     *(unsigned int*)(out + (size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d) =
         (unsigned int)float_to_bf16(ov0 * inv) | ((unsigned int)float_to_bf16(ov1 * inv) << 16);
   }
+  write_pages();
 }
 
 static int launch_decode(const void* q, long long q_stride, const void* key_pages, const void* value_pages,

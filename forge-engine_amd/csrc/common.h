@@ -21,13 +21,9 @@ __device__ __forceinline__ float bf16_to_float(bf16_t v) {
   return __uint_as_float(((uint32_t)v) << 16);
 }
 
-// Round to nearest even; NaN stays NaN.
-__device__ __forceinline__ bf16_t float_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)0x7fc0;
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (bf16_t)(u >> 16);
-}
+// Round to nearest even by the hardware's conversion (one instruction for a pair of values; the same bits as the rounding
+// by integer arithmetic for every float that is a number, all 2^32 compared); NaN stays NaN.
+__device__ __forceinline__ bf16_t float_to_bf16(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
 
 __device__ __forceinline__ float load_as_float(const float* p) { return *p; }
 __device__ __forceinline__ float load_as_float(const bf16_t* p) { return bf16_to_float(*p); }

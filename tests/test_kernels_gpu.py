@@ -898,6 +898,26 @@ def test_linear_swiglu_routes_by_rows(ops, monkeypatch):
         torch.testing.assert_close(got, refs.linear_swiglu(x, weight).float(), atol=2e-2, rtol=2e-2)
 
 
+def test_stored_products_round_to_nearest_even(ops):
+    """A product whose float32 sum is exact (one bfloat16 and a smaller one): the stored bfloat16 is torch's rounding of it, at
+    ties, just beside them, across a power of two, at the largest finite value, at infinities and NaN."""
+    g = torch.Generator().manual_seed(3)
+    a = torch.randn(4096, generator=g).bfloat16().float()
+    a[:8] = torch.tensor([3.3895e38, -3.3895e38, float("inf"), -float("inf"), float("nan"), 1.9921875, -1.9921875, 0.0])
+    step = torch.tensor([0.5, 0.498046875, 0.50390625, -0.25, 0.25, -0.251953125, 0.0, 1.0])[torch.randint(0, 8, (4096,), generator=g)]
+    b = torch.where(a.isfinite(), a.abs().clamp(min=1e-30).log2().floor().exp2() * step * 2.0 ** -7, torch.zeros(()))
+    b[:2] = torch.tensor([2.0 ** 119, -(2.0 ** 119)])
+    w = torch.zeros(4096, 128)
+    w[:, 0], w[:, 1] = a, b
+    x = torch.zeros(2, 128)
+    x[:, :2] = 1.0
+    want = (w[:, 0].bfloat16().float() + w[:, 1].bfloat16().float()).bfloat16()
+    for got in (ops.gemm_skinny(x.bfloat16().to(DEV), w.bfloat16().to(DEV)), ops.gemm_lds(x.bfloat16().to(DEV), w.bfloat16().to(DEV), "bf16", tile=9)):
+        for row in got.cpu():
+            assert torch.equal(row.isnan(), want.isnan())
+            assert torch.equal(row.nan_to_num(nan=7.0, posinf=9.0, neginf=-9.0), want.nan_to_num(nan=7.0, posinf=9.0, neginf=-9.0))
+
+
 @pytest.mark.parametrize("tile", range(14))
 @pytest.mark.parametrize("m,n,k,parts", [(1, 8, 64, 1), (16, 41, 1344, 1), (31, 33, 128, 2), (64, 80, 192, 2), (65, 97, 640, 3), (129, 161, 1024, 5), (257, 330, 704, 4)])
 def test_gemm_lds(ops, tile, m, n, k, parts):

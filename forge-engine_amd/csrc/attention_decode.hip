@@ -8,6 +8,7 @@
 //   * grid (key split, kv head, sequence); with few sequences the keys of one
 //     (sequence, head) are split over several blocks so that the chip is full,
 //     and the block that finishes last merges the splits (a counter per (sequence, head));
+//     with a dozen sequences and more, or a few long ones, the splits follow the lengths (find_run);
 //   * inside a block the four waves take 32-key blocks in turn;
 //   * scores transposed, S^T = K Q^T: MFMA 16x16x32 with A = 16 keys (rows) and
 //     B = the G query rows padded to 16 (columns).  The 32 keys of a block feed
@@ -38,6 +39,7 @@ typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
 #define KEYS 32          // keys per block of work
 #define WAVES 4
 #define GMAX 8           // largest group size served
+#define SLOT_LAYER 256   // CUs: blocks that land on a CU of their own
 
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 __device__ __forceinline__ unsigned int pack_bf16(float lo, float hi) {
@@ -98,6 +100,76 @@ struct Prepare {
 };
 #define MAX_SUMS 4
 
+// A wave's sum of ints.
+__device__ __forceinline__ int wave_sum_int(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);    // lane ^ 1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);    // lane ^ 2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);   // 7 - lane within 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true);   // 15 - lane within 16
+  auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+  v = (int)r[0] + (int)r[1];
+  r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+  return __builtin_amdgcn_readfirstlane((int)r[0] + (int)r[1]);
+}
+
+// Key blocks that a sequence's token reads: [first, last).  The token at position ctx - 1 reads the last `window` keys, and of
+// those the ones of its own run of `chunk` positions (runs counted from position 0); cached: keys that come from the pages.
+struct KeyRange {
+  int k_begin, first, last;
+};
+__device__ __forceinline__ KeyRange key_range(int ctx, int cached, int window, int chunk) {
+  int k_begin = window > 0 ? max(0, ctx - window) : 0;
+  if (chunk > 0) k_begin = max(k_begin, (ctx - 1) / chunk * chunk);
+  return {k_begin, k_begin / KEYS, (cached + KEYS - 1) / KEYS};
+}
+
+// Runs by length (launches of up to 64 sequences): every wave finds its block's run from the lengths, one sequence a lane.
+// A sequence is cut into equal runs of at most max(4, ceil(all key blocks / more)) key blocks, so a launch of num_seqs + more
+// blocks a head has one for each; the runs are handed out longest first, which the order of the blocks then balances: the first
+// `layer` blocks of a head land on CUs of their own, the next `layer` beside them, shortest first, what is left goes to
+// the slots that come free first.
+struct Run {
+  int seq, split, splits, part;      // part: where the sequence's partial results begin, in runs of a head
+  int q0, tokens, ctx;               // the sequence's query row, how many it brings, and its length
+};
+__device__ __forceinline__ bool find_run(const int* cu_q, const int* ctx_len, int num_seqs, int more, int own, int window, int chunk,
+                                         int layer, int item, Run* run) {
+  __shared__ int positions[WAVES][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = min(lane, num_seqs - 1);
+  const int q0 = cu_q[i], q1 = cu_q[i + 1], ctx = ctx_len[i];
+  const bool mine = lane < num_seqs && q1 - q0 == 1;
+  const KeyRange range = key_range(ctx, ctx - own, window, chunk);
+  const int blocks = mine ? max(range.last - range.first, 0) : 0;
+  const int target = max((wave_sum_int(blocks) + more - 1) / more, WAVES);
+  const int runs = mine ? max((blocks + target - 1) / target, 1) : 0;
+  const int size = mine ? (blocks + runs - 1) / runs : -1;
+  const int key = size * 64 + lane;
+  const int all = wave_sum_int(runs);
+  if (item >= all) return false;
+  int position = 0;           // runs of longer ones; each wave counts among sixteen sequences
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int other = __builtin_amdgcn_readlane(key, wave * 16 + j), count = __builtin_amdgcn_readlane(runs, wave * 16 + j);
+    position += other > key ? count : 0;
+  }
+  positions[wave][lane] = position;
+  __syncthreads();
+  position = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) position += positions[w][lane];
+  if (item >= layer && item < 2 * layer) item = layer + min(all, 2 * layer) - 1 - item;
+  const int at = __builtin_ctzll(__ballot(mine && position <= item && item < position + runs));
+  run->seq = at;
+  run->splits = __builtin_amdgcn_readlane(runs, at);
+  run->part = __builtin_amdgcn_readlane(position, at);
+  run->split = item - run->part;
+  run->q0 = __builtin_amdgcn_readlane(q0, at);
+  run->tokens = 1;
+  run->ctx = __builtin_amdgcn_readlane(ctx, at);
+  return true;
+}
+
 // MODE 0: finished queries; 1: PREPARE from the projection's bfloat16 output; 2: PREPARE from its
 // float32 partial sums.
 template <int D, int MODE, bool CAP = false, int DIST = 0>
@@ -108,7 +180,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     const int* __restrict__ ctx_len, const int* __restrict__ block_table, int table_stride,
     int kv_heads, int groups, int block_shift, int num_blocks, int window, float scale_log2,
     Prepare prep, int chunk, const float* __restrict__ sink, float cap_ratio, const float* __restrict__ slopes,
-    int bias_span) {
+    int bias_span, int num_seqs, int more) {
   constexpr bool PREPARE = MODE != 0, FROM_SUMS = MODE == 2;
   const int block_size = 1 << block_shift, block_mask = block_size - 1;
   constexpr int KC = D / 32;        // MFMA k-steps over the head dim (scores)
@@ -117,18 +189,21 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   __shared__ __attribute__((aligned(16))) float Ow[PARTS][GMAX][D];
   __shared__ float Ms[PARTS][GMAX], Ls[PARTS][GMAX];
 
-  const int split = blockIdx.x, splits = gridDim.x;
-  const int hk = blockIdx.y, seq = blockIdx.z;
-  const int q0 = cu_q[seq];
-  if (cu_q[seq + 1] - q0 != 1) return;
-  const int ctx = ctx_len[seq];
+  const int hk = blockIdx.y;
+  Run run;
+  if (more > 0) {
+    if (!find_run(cu_q, ctx_len, num_seqs, more, PREPARE, window, chunk, max(SLOT_LAYER / kv_heads, 1), blockIdx.z, &run)) return;
+  } else {
+    const int z = blockIdx.z, q = cu_q[z];
+    run = {z, (int)blockIdx.x, (int)gridDim.x, z * (int)gridDim.x, q, cu_q[z + 1] - q, ctx_len[z]};
+  }
+  const int seq = run.seq, split = run.split, splits = run.splits;
+  const size_t first_part = (size_t)run.part * kv_heads + (size_t)hk * splits;
+  const int q0 = run.q0, ctx = run.ctx;
+  if (run.tokens != 1) return;
   const int cached = PREPARE ? ctx - 1 : ctx;             // keys that the loop below reads from the pages
-  // the token at position ctx - 1 reads the last `window` keys, and of those the ones of its own
-  // run of `chunk` positions (runs counted from position 0)
-  int k_begin = window > 0 ? max(0, ctx - window) : 0;
-  if (chunk > 0) k_begin = max(k_begin, (ctx - 1) / chunk * chunk);
-  const int first = k_begin / KEYS;
-  const int last = (cached + KEYS - 1) / KEYS;            // exclusive
+  const KeyRange range = key_range(ctx, cached, window, chunk);
+  const int k_begin = range.k_begin, first = range.first, last = range.last;
   const int per_split = (last - first + splits - 1) / splits;
   const int my_first = first + split * per_split;
   const int my_last = min(last, my_first + per_split);
@@ -529,7 +604,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       if (sink) l += __builtin_amdgcn_exp2f(sink[hk * groups + g] * 1.4426950408889634f - m_tot);
       out[(size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d] = float_to_bf16(l > 0.f ? ov / l : 0.f);
     } else {
-      const size_t slot = ((size_t)seq * kv_heads + hk) * splits + split;
+      const size_t slot = first_part + split;
       store_agent(&part_o[(slot * groups + g) * D + d], ov);
       if (d == 0) {
         store_agent(&part_ml[(slot * groups + g) * 2], m_tot);        // base-2 exponent units
@@ -568,7 +643,6 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     write_pages();
     return;
   }
-  const size_t first_part = ((size_t)seq * kv_heads + hk) * splits;
   if (splits <= 16) {
     // few splits: every thread reads the statistics of its row itself, together with its share
     // of the partial outputs, so that all loads are in flight at once (same sums, same order)
@@ -637,30 +711,32 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
   if (block_size < 16 || (block_size & (block_size - 1)) || num_blocks < 1 || table_stride < 1) return FE_BAD_ARGUMENT;
   int block_shift = 0;
   while ((1 << block_shift) < block_size) ++block_shift;
-  if (q_stride % 8 || out_stride % 2 || splits < 1 || splits > 64) return FE_BAD_ARGUMENT;
+  if (q_stride % 8 || out_stride % 2 || splits > 64) return FE_BAD_ARGUMENT;
+  const int more = splits < 0 ? -splits : 0;     // runs by length: blocks a head beyond the sequences
+  if (splits == 0 || more > 4096 || (more > 0 && num_seqs > 64)) return FE_BAD_ARGUMENT;
   if ((((uintptr_t)out) & 3) || (((uintptr_t)part_o) & 7)) return FE_BAD_ARGUMENT;   // pairs of outputs, pairs of partial sums
   if ((((uintptr_t)q) | ((uintptr_t)key_pages) | ((uintptr_t)value_pages)) & 15) return FE_BAD_ARGUMENT;
-  if (splits > 1 && (!part_o || !part_ml || !counters)) return FE_BAD_ARGUMENT;
+  if (splits != 1 && (!part_o || !part_ml || !counters)) return FE_BAD_ARGUMENT;
   if (chunk < 0) return FE_BAD_ARGUMENT;
-  dim3 grid(splits, kv_heads, num_seqs);
+  dim3 grid(more > 0 ? 1 : splits, kv_heads, num_seqs + more);
   const float scale_log2 = scale * 1.4426950408889634f;
   const Prepare none = {nullptr, nullptr, nullptr, 0.f, nullptr, 0, 0};
 #define FE_GO(DD, MODE)                                                                                    \
   paged_decode_kernel<DD, MODE><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
       (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, MODE ? *prep : none, chunk, sink, 0.f, nullptr, 0)
+      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, MODE ? *prep : none, chunk, sink, 0.f, nullptr, 0, num_seqs, more)
 #define FE_GO_CAPPED(DD)                                                                                   \
   paged_decode_kernel<DD, 0, true><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
       (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, softcap / scale, nullptr, 0)
+      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, softcap / scale, nullptr, 0, num_seqs, more)
 #define FE_GO_SLOPED(DD)                                                                                   \
   paged_decode_kernel<DD, 0, false, 1><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
       (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, 0.f, slopes, 0)
+      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, 0.f, slopes, 0, num_seqs, more)
 #define FE_GO_TABLE(DD)                                                                                    \
   paged_decode_kernel<DD, 0, false, 2><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
       (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, 0.f, slopes, bias_span)
+      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, 0.f, slopes, bias_span, num_seqs, more)
   if (slopes && bias_span > 0) {
     if (head_dim == 64) FE_GO_TABLE(64);
     else if (head_dim == 128) FE_GO_TABLE(128);
@@ -696,7 +772,9 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
 // Sequences with one query token only; others are left untouched.  Pages: keys
 // [blocks][kv_heads][block_size][D], values transposed [blocks][kv_heads][D][block_size];
 // block_size a power of two >= 16.  splits > 1 (at most 64) needs part_o [num_seqs * kv_heads * splits * groups * head_dim] and
-// part_ml [num_seqs * kv_heads * splits * groups * 2] floats, and counters [num_seqs * kv_heads]
+// part_ml [num_seqs * kv_heads * splits * groups * 2] floats, and counters [num_seqs * kv_heads]; splits = -E (at most
+// 4,096, up to 64 sequences): runs by length, at most num_seqs + E of them a head, which is what part_o and part_ml hold then
+// in place of num_seqs * splits; the counters alike:
 // ints that are zero before the first launch; every launch leaves them zero again.  Launches that
 // share counters must not overlap.
 extern "C" int fe_paged_attention_decode(const void* q, long long q_stride, const void* key_pages,

@@ -858,6 +858,36 @@ def _split_counters(device, count: int) -> Tensor:
     return current.split_counters(device, count)
 
 
+DECODE_SLOTS = 512             # blocks of the decode kernel that the chip holds at a time (heads up to 128), two a CU
+RUNS_BY_LENGTH_MIN_SEQUENCES = 12
+RUNS_BY_LENGTH_LONG = 8192
+
+
+def decode_runs(num_decode: int, num_seqs: int, kv_heads: int, head_dim: int, reach: int) -> int:
+    """The decode launch's ``splits``: ``decode_splits``, or -E for runs by length.  With as many runs for every sequence the
+    launch lasts as long as its longest run, and that depends on where the long ones land; runs by length, found on the
+    device, cut a sequence into runs of at most (all key blocks / E) and order them so that CUs share the keys evenly.
+    Measured at 8 kv heads of 128 (us, splits -> by length): 64 sequences of 130 to 2,000 keys, shuffled 52.4 -> 41.5, falling
+    43.1 -> 41.0, 48: 35.4 -> 29.7, 32: 30.2 -> 23.8, 16: 21.1 -> 17.5, 4 of 6,000 to 16,000 39.7 -> 37.0.  What finding the
+    runs costs shows where lengths are equal (64 of 706 keys 34.8 -> 35.6) and where a launch is latency alone (8 of 200 to
+    1,900 14.9 -> 15.2, 1 of 217 8.3 -> 9.3), so: from twelve sequences, or from three where contexts may be long.  E keeps
+    the runs (about half a run a sequence more than the keys need) within the slots that the chip has at a time: a third
+    round of a few blocks cost 29.9 -> 32.7 at 48 sequences."""
+    if (num_seqs <= 64 and head_dim <= 128 and num_seqs * kv_heads <= DECODE_SLOTS
+            and num_decode >= (3 if reach >= RUNS_BY_LENGTH_LONG else RUNS_BY_LENGTH_MIN_SEQUENCES) and num_decode * kv_heads >= 24):
+        return -max(1, DECODE_SLOTS // kv_heads - 2 * num_decode // 3)
+    return decode_splits(num_decode, kv_heads, reach)
+
+
+def _split_scratch(device, num_seqs: int, kv_heads: int, groups: int, head_dim: int, splits: int):
+    """The decode kernel's partial outputs and statistics (one set a run of a (sequence, kv head)) and its counters."""
+    if splits == 1:
+        return None, None, None
+    runs = (num_seqs * splits if splits > 0 else num_seqs - splits) * kv_heads
+    return (torch.empty(runs * groups * head_dim, dtype=torch.float32, device=device),
+            torch.empty(runs * groups * 2, dtype=torch.float32, device=device), _split_counters(device, num_seqs * kv_heads))
+
+
 def decode_splits(num_decode: int, kv_heads: int, max_ctx: int) -> int:
     """Key splits per (sequence, kv head) for the decode kernel: enough blocks to
     fill the chip, at least four 32-key blocks of work (one per wave) in each."""
@@ -996,12 +1026,9 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
     if any_single and fast_decode:
         if splits is None:
             reach = max_ctx if max_ctx is not None else 16 * 4 * 8
-            splits = decode_splits(num_decode, kv_heads, reach if chunk is None else min(reach, chunk))
-        part_o = part_ml = counters = None
-        if splits > 1:
-            part_o = torch.empty(num_seqs * kv_heads * splits * groups * head_dim, dtype=torch.float32, device=q.device)
-            part_ml = torch.empty(num_seqs * kv_heads * splits * groups * 2, dtype=torch.float32, device=q.device)
-            counters = _split_counters(q.device, num_seqs * kv_heads)
+            reach = reach if chunk is None else min(reach, chunk)
+            splits = decode_runs(num_decode, num_seqs, kv_heads, head_dim, reach)
+        part_o, part_ml, counters = _split_scratch(q.device, num_seqs, kv_heads, groups, head_dim, splits)
         mask = (c_int(chunk or 0), _ptr(sink)) + ((_ptr(slopes),) if slopes is not None else ()) if masked else ()
         if dist_bias is not None:
             mask = (c_int(chunk or 0), _ptr(sink), _ptr(dist_bias), c_int(dist_bias.shape[1]))
@@ -1125,12 +1152,8 @@ def decode_attention_prepare(qkv: Tensor, q_weight: Tensor | None, k_weight: Ten
         raise KernelError("block_table must be [sequences, max_blocks] with unit inner stride")
     groups = q_heads // kv_heads
     if splits is None:
-        splits = decode_splits(num_seqs, kv_heads, max_ctx if max_ctx is not None else 16 * 4 * 8)
-    part_o = part_ml = counters = None
-    if splits > 1:
-        part_o = torch.empty(num_seqs * kv_heads * splits * groups * head_dim, dtype=torch.float32, device=qkv.device)
-        part_ml = torch.empty(num_seqs * kv_heads * splits * groups * 2, dtype=torch.float32, device=qkv.device)
-        counters = _split_counters(qkv.device, num_seqs * kv_heads)
+        splits = decode_runs(num_seqs, num_seqs, kv_heads, head_dim, max_ctx if max_ctx is not None else 16 * 4 * 8)
+    part_o, part_ml, counters = _split_scratch(qkv.device, num_seqs, kv_heads, groups, head_dim, splits)
     _call("attention_decode", "fe_paged_attention_decode_prepare", _ptr(qkv), c_int(sums),
           c_longlong(num_seqs * width), c_longlong(width), _ptr(q_weight),
           _ptr(k_weight), _ptr(inv_freq), c_float(eps), _ptr(key_pages), _ptr(value_pages), _ptr(out),

@@ -1326,6 +1326,63 @@ def test_linear_in_parts(ops):
     assert ops.linear_in_parts(rand(g, 4, 2560).to(DEV), w.float()) is None                        # not bfloat16
 
 
+@pytest.mark.parametrize("more", [1, 7, 48, 300])
+@pytest.mark.parametrize("count,kv_heads,head_dim,window", [(1, 8, 128, 0), (5, 2, 64, 0), (13, 8, 128, 200), (64, 3, 128, 0), (64, 8, 64, 33), (7, 1, 256, 0)])
+def test_decode_attention_in_runs_by_length(ops, count, kv_heads, head_dim, window, more):
+    """Runs that the launch finds from the lengths, against the plain reference: lengths of every size beside one another and
+    equal ones, empty contexts, few and many runs a head, more runs than the first two rounds of the chip; twice on the same
+    counters, the pages with the same bits as with one run."""
+    g = torch.Generator().manual_seed(count + more)
+    contexts = [0, 700, 31, 32, 33, 700, 1, 127, 128, 1500][:count] + torch.randint(0, 400, (max(0, count - 10),), generator=g).tolist()
+    qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq, positions, token_seq = _prepare_case(g, 2 * kv_heads, kv_heads, head_dim, 16, contexts)
+    sizes = dict(q_heads=2 * kv_heads, kv_heads=kv_heads, head_dim=head_dim)
+    more = min(more, 4 * (64 // kv_heads) + 40)
+    outs = []
+    for splits in (1, -more, -more):
+        kp_dev, vp_dev = kp.to(DEV), vp.to(DEV)
+        out = torch.full((count, 2 * kv_heads * head_dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.decode_attention_prepare(qkv.to(DEV), qw.to(DEV), kw.to(DEV), inv_freq.to(DEV), kp_dev, vp_dev, out, cu.to(DEV), ctx.to(DEV),
+                                     table.to(DEV), eps=1e-6, scale=0.1, window=window or None, max_ctx=1501, splits=splits, **sizes)
+        outs.append((out, kp_dev, vp_dev))
+    for out, kp_dev, vp_dev in outs[1:]:
+        # float32 sums in another order, one rounding each: an ulp of bfloat16 at most
+        torch.testing.assert_close(out.float(), outs[0][0].float(), atol=2e-3, rtol=2.0 ** -7)
+        assert torch.equal(kp_dev, outs[0][1]) and torch.equal(vp_dev, outs[0][2]) and torch.equal(out, outs[1][0])
+    refs.qk_norm_rope_write(qkv, qw, kw, inv_freq, positions, token_seq, table, kp, vp, rotary_dim=head_dim, eps=1e-6, **sizes)
+    want = refs.paged_attention(qkv, kp, vp, torch.empty(count, 2 * kv_heads * head_dim, dtype=qkv.dtype), cu, ctx, table, num_seqs=count, max_q_len=1,
+                                scale=0.1, window=window or None, **sizes).float()
+    torch.testing.assert_close(outs[1][0].cpu().float(), want, atol=2e-2, rtol=2e-2)
+
+
+def test_decode_attention_in_runs_by_length_beside_portions(ops):
+    """Sequences that bring more than one token, and none, have no run; the finished queries' kernel, a chunk."""
+    g = torch.Generator().manual_seed(6)
+    seqs = [(600, 1), (40, 9), (0, 1), (33, 1), (900, 1), (10, 3), (64, 1)] + [(50 * i, 1) for i in range(12)]
+    q, kp, vp, cu, ctx, table = _attention_case(g, torch.bfloat16, seqs, 8, 4, 128, 16)
+    tokens = q.shape[0]
+    for chunk in (None, 128):
+        results = []
+        for splits in (1, -5, -100):
+            out = torch.full((tokens, 8 * 128), float("nan"), dtype=torch.bfloat16, device=DEV)
+            ops.paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), out, cu.to(DEV), ctx.to(DEV), table.to(DEV), num_seqs=len(seqs), max_q_len=9,
+                                num_decode=17, q_heads=8, kv_heads=4, head_dim=128, scale=0.1, max_ctx=1024, splits=splits, chunk=chunk)
+            results.append(out.float())
+        for other in results[1:]:
+            torch.testing.assert_close(other, results[0], atol=2e-3, rtol=2.0 ** -7)
+    case = _prepare_case(g, 2, 1, 64, 16, [3] * 65)
+    qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq = (t.to(DEV) for t in case[:9])
+    with pytest.raises(ops.KernelError):                       # a lane a sequence
+        ops.decode_attention_prepare(qkv, qw, kw, inv_freq, kp, vp, torch.empty(65, 128, dtype=torch.bfloat16, device=DEV), cu, ctx, table,
+                                     q_heads=2, kv_heads=1, head_dim=64, eps=1e-6, scale=0.1, max_ctx=64, splits=-4)
+
+
+def test_which_decode_launches_take_runs_by_length(ops):
+    assert ops.decode_runs(64, 64, 8, 128, 2048) == -22 and ops.decode_runs(12, 12, 8, 64, 1024) == -56
+    assert ops.decode_runs(3, 3, 8, 128, 8192) == -62 and ops.decode_runs(12, 20, 2, 128, 512) == -248
+    for other in ((11, 11, 8, 128, 2048), (2, 2, 8, 128, 8192), (3, 3, 4, 128, 8192), (64, 65, 8, 128, 2048), (64, 64, 9, 128, 2048), (32, 32, 8, 256, 2048)):
+        assert ops.decode_runs(*other) == ops.decode_splits(other[0], other[2], other[4])
+
+
 @pytest.mark.parametrize("window", [1, 16, 37, 300])
 def test_decode_attention_that_prepares_with_a_window(ops, window):
     g = torch.Generator().manual_seed(34)

@@ -163,6 +163,7 @@ def add_rows(h: Tensor, delta: Tensor | None, other: Tensor | None = None, shift
 
 
 GATE_ACTS = {"silu": 0, "gelu_tanh": 1}     # FE_GATE_* of csrc/gate_act.h
+GATE_BOUNDED = 2
 
 
 def _gate_act(act: str) -> c_int:
@@ -332,6 +333,10 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
             and _lds_store_pays(x.shape[0], *weight.shape)):
         tile, _ = lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])
         return gemm_lds(x, weight, "bf16", tile=tile)
+    if (bias is None and out_dtype == torch.float32 and x.shape[0] <= MID_ROWS and weight.shape[0] >= LDS_HEAD_WEIGHT_ROWS
+            and weight.shape[1] >= LDS_HEAD_MIN_K and _lds_fits(x, weight)):
+        rows = x.shape[0]          # (hundreds of tiles a CU: the cheapest tile whatever the rounds, not the plan's)
+        return gemm_lds(x, weight, "parts", tile=10 if rows <= 8 else 12 if rows <= 16 else 8 if rows <= 32 else 4)[0]
     if bias is None and _skinny_fits(x, weight) and out_dtype in (torch.float32, torch.bfloat16) and not to_library:
         return gemm_skinny(x, weight, "f32" if out_dtype == torch.float32 else "bf16")
     if (bias is None and out_dtype == torch.bfloat16 and _wide_fits(x, weight, WIDE_STORE_MAX_ROWS, SKINNY_MAX_ROWS + 1)
@@ -452,7 +457,7 @@ def gemm_wide(x: Tensor, weight: Tensor, ending: str = "bf16", parts: int = 1, r
         raise KernelError(f"no ending {ending!r} with {parts} parts")
     _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
           c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
-          c_int(row_tile or (16 if m <= 16 else 64 if m <= 64 else 128)), c_int(block_rows), c_int(-1), _gate_act(act), _stream())
+          c_int(row_tile or (16 if m <= 16 else 64 if m <= 64 else 128)), c_int(block_rows), c_int(-1), _gate_act(act), c_float(0.0), c_float(0.0), _stream())
     return out
 
 
@@ -478,6 +483,11 @@ def _wide_parts(m: int, n: int, k: int, block_rows: int = 64, most: int = 16) ->
 LDS_TILES = ((32, 32, 2, 0.151, 0.256), (64, 32, 1, 0.191, 0.382), (64, 64, 2, 0.212, 0.348), (64, 80, 1, 0.303, 0.606),
              (64, 96, 2, 0.292, 0.451), (128, 64, 1, 0.317, 0.634), (128, 128, 1, 0.510, 1.02), (128, 160, 1, 0.630, 1.26), (32, 64, 2, 0.202, 0.378),
              (16, 16, 2, 0.073, 0.117), (16, 32, 2, 0.116, 0.247), (16, 48, 2, 0.143, 0.334), (16, 64, 2, 0.168, 0.444), (16, 80, 1, 0.220, 0.440))
+# float32 logits, up to 64 rows through a vocabulary's weight (151,936 rows; kernel for few rows or library -> this): K = 2,560
+# 1 row 137 -> 130 us, 8: 151 -> 142, 17: 167 -> 150, 64: 185 -> 183; K = 2,048 1 row 108 -> 108, 8: 119 -> 113, 17: 148 -> 122,
+# 64: 160 -> 149; at K = 1,024 the blocks that keep x in registers win (1 row 53 against 55, 8: 58 against 59).
+LDS_HEAD_WEIGHT_ROWS = 131072
+LDS_HEAD_MIN_K = 2048
 LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
 
@@ -561,10 +571,11 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     return -(-rows // 128) * -(-2 * columns // 160) <= WIDE_CUS
 
 
-def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu") -> Tensor:
+def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu",
+             bounded: tuple[float, float] | None = None) -> Tensor:
     """x @ weight^T for bfloat16 rows: ``"parts"`` float32 partial sums [parts, M, N] over runs of whole 64-steps of K,
     ``"bf16"`` [M, N], or ``"gated"``: act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first; ``act`` as in
-    ``swiglu``).  ``tile``: the block's, see ``LDS_TILES``."""
+    ``swiglu``; ``bounded`` (limit, alpha): ``linear_gated``'s instead).  ``tile``: the block's, see ``LDS_TILES``."""
     _gpu(x, "x", torch.bfloat16)
     _gpu(weight, "weight", torch.bfloat16, contiguous=False)
     if (x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1] or x.shape[1] % 64 or weight.stride(1) != 1
@@ -585,7 +596,8 @@ def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int =
         raise KernelError(f"no tile {tile}")
     _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
           c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
-          c_int(64), c_int(64), c_int(tile), _gate_act(act), _stream())
+          c_int(64), c_int(64), c_int(tile), c_int(GATE_BOUNDED) if bounded else _gate_act(act), c_float(bounded[0] if bounded else 0.0),
+          c_float(bounded[1] if bounded else 0.0), _stream())
     return out
 
 
@@ -719,6 +731,16 @@ GATED_TILE_MAX_ROWS = 4096
 GATED_TILE_MAX_K = 3072
 
 
+def _gate_to_library(x: Tensor, gate_up_weight: Tensor) -> bool:
+    return (2 <= x.shape[0] <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
+            and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
+
+
+def _lds_gate_takes(x: Tensor, gate_up_weight: Tensor) -> bool:
+    return (not _gate_to_library(x, gate_up_weight) and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
+            and _lds_gate_pays(x.shape[0], gate_up_weight.shape[0] // 2, gate_up_weight.shape[1]))
+
+
 def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tensor:
     """act(x Wg^T) * (x Wu^T) for the fused weight [2I, K] (gate rows first); ``act`` as in ``swiglu``."""
     _gpu(x, "x")
@@ -730,10 +752,8 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tenso
             and x.data_ptr() % 16 == 0 and gate_up_weight.data_ptr() % 16 == 0
             and gate_up_weight.shape[0] * gate_up_weight.stride(0) < 2 ** 32 and rows * x.shape[1] < 2 ** 32):
         return gemm_gated(x, gate_up_weight, shape=3, act=act)
-    to_library = (2 <= rows <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
-                  and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
-    if (not to_library and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
-            and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])):
+    to_library = _gate_to_library(x, gate_up_weight)
+    if _lds_gate_takes(x, gate_up_weight):
         tile, _ = lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])
         return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
     paired_fits = (rows <= MID_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16
@@ -2339,7 +2359,12 @@ def moe_experts(x: Tensor, chosen: Tensor | None, weights: Tensor, gate_up: Tens
 
 def linear_gated(x: Tensor, gate_up_weight: Tensor, *, limit: float, alpha: float) -> Tensor:
     """``min(g, limit) * sigmoid(alpha * min(g, limit)) * (clamp(u, -limit, limit) + 1)`` with g and u the two
-    halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype."""
+    halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype.  bfloat16 where
+    ``linear_swiglu`` takes the product through LDS: in its ending, without a launch of its own (4,096 x 2,048 at 8 rows:
+    6.2 + 4.4 us -> 6.2) and without the rounding of g and u."""
+    if (limit > 0.0 and gate_up_weight.dim() == 2 and gate_up_weight.shape[0] % 2 == 0 and _lds_gate_takes(_gpu(x, "x"), _gpu(gate_up_weight, "gate_up_weight", contiguous=False))):
+        tile, _ = lds_plan(x.shape[0], *gate_up_weight.shape, gate_up_weight.shape[0])
+        return gemm_lds(x, gate_up_weight, "gated", tile=tile, bounded=(limit, alpha))
     gate_up = linear(x, gate_up_weight)
     tokens, width = gate_up.shape
     if width % 2 or not limit > 0.0:

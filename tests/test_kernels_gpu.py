@@ -898,6 +898,33 @@ def test_linear_swiglu_routes_by_rows(ops, monkeypatch):
         torch.testing.assert_close(got, refs.linear_swiglu(x, weight).float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 32, 33, 64, 65])
+def test_logits_through_a_vocabulary(ops, rows):
+    """float32 logits at both sides of every line between tiles: sampled columns against 64 bits, |error| <= 2 k 2^-24 sum |a||b|."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, 2048, generator=g, device=DEV).bfloat16()
+    w = torch.empty(131073, 2048, dtype=torch.bfloat16, device=DEV).normal_(generator=g)
+    got = ops.linear(x, w, out_dtype=torch.float32)
+    assert got.shape == (rows, 131073) and got.dtype == torch.float32
+    at = torch.cat([torch.arange(0, 131073, 1009, device=DEV), torch.arange(131073 - 97, 131073, device=DEV)])
+    a, b = x.double(), w[at].double()
+    assert bool(((got[:, at].double() - a @ b.t()).abs() <= (a.abs() @ b.abs().t()) * 2 * 2048 * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("rows", [1, 5, 16, 17, 300])
+def test_linear_gated_in_the_product(ops, rows):
+    """The bounded gate in the product's ending: against 64 bits, one rounding to bfloat16 (and the float32 sums' error at 2 k 2^-24)."""
+    g = torch.Generator().manual_seed(rows)
+    x, w = rand(g, rows, 1024, dtype=torch.bfloat16), rand(g, 2 * 260, 1024, dtype=torch.bfloat16, scale=0.05)
+    got = ops.linear_gated(x.to(DEV), w.to(DEV), limit=0.8, alpha=1.702).double().cpu()
+    both = x.double() @ w.double().t()
+    gate, up = both[:, :260].clamp(max=0.8), both[:, 260:].clamp(-0.8, 0.8)
+    want = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+    torch.testing.assert_close(got, want, atol=2e-3, rtol=2.0 ** -8)
+    with pytest.raises(ops.KernelError):
+        ops.linear_gated(x.to(DEV), w.to(DEV), limit=0.0, alpha=1.0)
+
+
 def test_stored_products_round_to_nearest_even(ops):
     """A product whose float32 sum is exact (one bfloat16 and a smaller one): the stored bfloat16 is torch's rounding of it, at
     ties, just beside them, across a power of two, at the largest finite value, at infinities and NaN."""

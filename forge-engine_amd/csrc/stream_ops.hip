@@ -85,45 +85,78 @@ __device__ __forceinline__ float parts_sum(const float* p, int parts, size_t par
   return d;
 }
 
+// Elements c = threadIdx.x + j * blockDim.x of a row in parts, each the sum of its parts in order, zeros beyond the row.  The loads
+// of four parts and all elements are issued before any is used, none under a condition (an index beyond the row or the parts
+// reads the last one again): at a few rows these kernels take what their chain of dependent loads takes.  The sums are those
+// of parts_sum, bit for bit.
+template <int N>
+__device__ __forceinline__ void held_row(const float* __restrict__ row, int parts, size_t part_stride, int width, float (&u)[N]) {
+  for (int from = 0; from < parts; from += 4) {
+    float v[N][4];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        v[j][p] = row[min((int)(threadIdx.x + j * blockDim.x), width - 1) + min(from + p, parts - 1) * part_stride];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      u[j] = from == 0 ? v[j][0] : u[j] + v[j][0];
+#pragma unroll
+      for (int p = 1; p < 4; ++p) u[j] = from + p < parts ? u[j] + v[j][p] : u[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    if ((int)(threadIdx.x + j * blockDim.x) >= width) u[j] = 0.f;
+}
+
+// Elements a thread holds of a row of up to 8 a thread: 1, 2, 4 or 8; 0: wider.
+static inline int held_elements(int width, int threads) {
+  const int each = (width + threads - 1) / threads;
+  return each <= 1 ? 1 : each <= 2 ? 2 : each <= 4 ? 4 : each <= 8 ? 8 : 0;
+}
+
 // h[r] += u * rsqrt(mean(u^2) + eps) * w, u = the sum of the update's parts; out (if any) = new h.
-// A row of up to 8 elements a thread stays in registers between the two passes (the parts are read
-// once); wider rows are read again.
-template <typename TO, bool HAS_OUT>
+// A row of up to 8 elements a thread (N) stays in registers between the two passes, with the stream's and the weight's
+// elements, which are asked for beside the update's; wider rows (N = 0) are read again.  6 rows of 2,048 in 4 parts: a launch of
+// 6.2 us with loads under conditions, part after part.
+template <typename TO, bool HAS_OUT, int N>
 __global__ __launch_bounds__(ROW_THREADS_FEW) void rmsnorm_update_kernel(
     float* __restrict__ h, const float* __restrict__ update, int parts, size_t part_stride,
     const float* __restrict__ w, float eps, TO* __restrict__ out, int width) {
   __shared__ float scratch[16];
   const size_t base = (size_t)blockIdx.x * width;
   const int threads = blockDim.x;
-  const bool held = width <= 8 * threads;
-  float u[8];
   float ss = 0.f;
-  if (held) {
+  if constexpr (N > 0) {
+    float u[N], before[N], weight[N];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < N; ++j) {
+      const int c = min((int)(threadIdx.x + j * threads), width - 1);
+      before[j] = h[base + c];
+      weight[j] = w[c];
+    }
+    held_row<N>(update + base, parts, part_stride, width, u);
+#pragma unroll
+    for (int j = 0; j < N; ++j) ss += u[j] * u[j];
+    ss = block_sum<true>(ss, scratch);
+    const float inv = rsqrtf(ss / (float)width + eps);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
       const int c = threadIdx.x + j * threads;
-      u[j] = c < width ? parts_sum(update + base + c, parts, part_stride) : 0.f;
-      ss += u[j] * u[j];
+      if (c < width) {
+        const float v = before[j] + u[j] * inv * weight[j];
+        h[base + c] = v;
+        if (HAS_OUT) store_from_float(out + base + c, v);
+      }
     }
   } else {
     for (int c = threadIdx.x; c < width; c += threads) {
       const float v = parts_sum(update + base + c, parts, part_stride);
       ss += v * v;
     }
-  }
-  ss = block_sum<true>(ss, scratch);
-  const float inv = rsqrtf(ss / (float)width + eps);
-  if (held) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int c = threadIdx.x + j * threads;
-      if (c < width) {
-        const float v = h[base + c] + u[j] * inv * w[c];
-        h[base + c] = v;
-        if (HAS_OUT) store_from_float(out + base + c, v);
-      }
-    }
-  } else {
+    ss = block_sum<true>(ss, scratch);
+    const float inv = rsqrtf(ss / (float)width + eps);
     for (int c = threadIdx.x; c < width; c += threads) {
       const float v = h[base + c] + parts_sum(update + base + c, parts, part_stride) * inv * w[c];
       h[base + c] = v;
@@ -136,13 +169,23 @@ extern "C" int fe_rmsnorm_update(float* h, const float* update, int parts, long 
                                  float eps, void* out, int out_dtype, int rows, int width, hipStream_t stream) {
   if (rows <= 0) return FE_OK;
   if (width <= 0 || parts < 1 || parts > 64 || !(eps > 0.f)) return FE_BAD_ARGUMENT;
-  if (out == nullptr || out_dtype < 0)
-    rmsnorm_update_kernel<float, false><<<rows, row_threads(rows, width), 0, stream>>>(h, update, parts, (size_t)part_stride, w, eps, nullptr, width);
-  else if (out_dtype == FE_F32)
-    rmsnorm_update_kernel<float, true><<<rows, row_threads(rows, width), 0, stream>>>(h, update, parts, (size_t)part_stride, w, eps, (float*)out, width);
-  else if (out_dtype == FE_BF16)
-    rmsnorm_update_kernel<bf16_t, true><<<rows, row_threads(rows, width), 0, stream>>>(h, update, parts, (size_t)part_stride, w, eps, (bf16_t*)out, width);
+  const int threads = row_threads(rows, width);
+#define LAUNCH(TO, HAS_OUT, N) \
+  rmsnorm_update_kernel<TO, HAS_OUT, N><<<rows, threads, 0, stream>>>(h, update, parts, (size_t)part_stride, w, eps, (TO*)out, width)
+#define LAUNCH_HELD(TO, HAS_OUT)                       \
+  switch (held_elements(width, threads)) {             \
+    case 1: LAUNCH(TO, HAS_OUT, 1); break;             \
+    case 2: LAUNCH(TO, HAS_OUT, 2); break;             \
+    case 4: LAUNCH(TO, HAS_OUT, 4); break;             \
+    case 8: LAUNCH(TO, HAS_OUT, 8); break;             \
+    default: LAUNCH(TO, HAS_OUT, 0);                   \
+  }
+  if (out == nullptr || out_dtype < 0) { LAUNCH_HELD(float, false); }
+  else if (out_dtype == FE_F32) { LAUNCH_HELD(float, true); }
+  else if (out_dtype == FE_BF16) { LAUNCH_HELD(bf16_t, true); }
   else return FE_BAD_ARGUMENT;
+#undef LAUNCH_HELD
+#undef LAUNCH
   return fe_check_launch();
 }
 
@@ -333,27 +376,59 @@ struct MeanInputs {
   int parts[4];
 };
 
+// N: elements a thread holds of each update (0: they are read again in the second pass).
+template <int N>
 __global__ __launch_bounds__(ROW_THREADS_FEW) void rmsnorm_mean_kernel(MeanInputs in, int count, size_t part_stride,
                                                                    const float* __restrict__ w, float eps,
                                                                    float* __restrict__ out, int width) {
   __shared__ float scratch[4][16];
   const size_t base = (size_t)blockIdx.x * width;
-  float inv[4];
-  for (int b = 0; b < count; ++b) {
-    float ss = 0.f;
-    for (int c = threadIdx.x; c < width; c += blockDim.x) {
-      const float u = parts_sum(in.u[b] + base + c, in.parts[b], part_stride);
-      ss += u * u;
-    }
-    ss = block_sum<true>(ss, scratch[b]);
-    inv[b] = rsqrtf(ss / (float)width + eps);
-  }
   const float share = 1.f / (float)count;
-  for (int c = threadIdx.x; c < width; c += blockDim.x) {
-    float total = 0.f;
-    for (int b = 0; b < count; ++b)
-      total += parts_sum(in.u[b] + base + c, in.parts[b], part_stride) * inv[b] * w[(size_t)b * width + c];
-    out[base + c] = total * share;
+  float inv[4];
+  if constexpr (N > 0) {
+    float u[4][N], weight[4][N];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        weight[b][j] = w[(size_t)min(b, count - 1) * width + min((int)(threadIdx.x + j * blockDim.x), width - 1)];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (b < count) held_row<N>(in.u[b] + base, in.parts[b], part_stride, width, u[b]);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      if (b >= count) break;
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < N; ++j) ss += u[b][j] * u[b][j];
+      ss = block_sum<true>(ss, scratch[b]);
+      inv[b] = rsqrtf(ss / (float)width + eps);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int c = threadIdx.x + j * blockDim.x;
+      float total = 0.f;
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (b < count) total += u[b][j] * inv[b] * weight[b][j];
+      if (c < width) out[base + c] = total * share;
+    }
+  } else {
+    for (int b = 0; b < count; ++b) {
+      float ss = 0.f;
+      for (int c = threadIdx.x; c < width; c += blockDim.x) {
+        const float v = parts_sum(in.u[b] + base + c, in.parts[b], part_stride);
+        ss += v * v;
+      }
+      ss = block_sum<true>(ss, scratch[b]);
+      inv[b] = rsqrtf(ss / (float)width + eps);
+    }
+    for (int c = threadIdx.x; c < width; c += blockDim.x) {
+      float total = 0.f;
+      for (int b = 0; b < count; ++b)
+        total += parts_sum(in.u[b] + base + c, in.parts[b], part_stride) * inv[b] * w[(size_t)b * width + c];
+      out[base + c] = total * share;
+    }
   }
 }
 
@@ -365,35 +440,70 @@ extern "C" int fe_rmsnorm_mean(const float* u0, const float* u1, const float* u2
   MeanInputs in = {{u0, u1, u2, u3}, {p0, p1, p2, p3}};
   for (int b = 0; b < count; ++b)
     if (in.u[b] == nullptr || in.parts[b] < 1 || in.parts[b] > 64) return FE_BAD_ARGUMENT;
-  rmsnorm_mean_kernel<<<rows, row_threads(rows, width), 0, stream>>>(in, count, (size_t)part_stride, w, eps, out, width);
+  const int threads = row_threads(rows, width);
+#define LAUNCH(N) rmsnorm_mean_kernel<N><<<rows, threads, 0, stream>>>(in, count, (size_t)part_stride, w, eps, out, width)
+  switch (held_elements(width, threads)) {
+    case 1: LAUNCH(1); break;
+    case 2: LAUNCH(2); break;
+    case 4: LAUNCH(4); break;
+    default: LAUNCH(0);          // (eight of each would not fit the registers of 1,024 threads)
+  }
+#undef LAUNCH
   return fe_check_launch();
 }
 
 // ---------------------------------------------------------------- PolyNorm
 // out = a z/rms(z) + b z^2/rms(z^2) + c z^3/rms(z^3) + e over a row
-template <typename T>
+// A row of up to 8 elements a thread (N) is held between the passes and read without conditions, and the three sums share one
+// barrier (6 rows of 6,144: a launch of 7.7 us with the row read again and a barrier a sum); wider rows (N = 0) are read again.
+template <typename T, int N>
 __global__ __launch_bounds__(ROW_THREADS_FEW) void polynorm_kernel(const T* __restrict__ z, const float* __restrict__ coeff,
                                                                float eps, T* __restrict__ out, int width) {
   __shared__ float scratch[3][16];
   const size_t base = (size_t)blockIdx.x * width;
+  const float c0 = coeff[0], c1 = coeff[1], c2 = coeff[2], e = coeff[3];
   float s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  for (int c = threadIdx.x; c < width; c += blockDim.x) {
-    const float v = load_as_float(z + base + c);
+  auto add = [&](float v) {
     const float v2 = v * v;
     s1 += v2;
     s2 += v2 * v2;
     s3 += v2 * v2 * v2;
+  };
+  float held[N > 0 ? N : 1];
+  if constexpr (N > 0) {
+    T raw[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) raw[j] = z[base + min((int)(threadIdx.x + j * blockDim.x), width - 1)];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      held[j] = (int)(threadIdx.x + j * blockDim.x) < width ? load_as_float(&raw[j]) : 0.f;
+      add(held[j]);
+    }
+  } else {
+    for (int c = threadIdx.x; c < width; c += blockDim.x) add(load_as_float(z + base + c));
   }
-  s1 = block_sum<true>(s1, scratch[0]);
-  s2 = block_sum<true>(s2, scratch[1]);
-  s3 = block_sum<true>(s3, scratch[2]);
+  const int lane = threadIdx.x & (FE_WAVE - 1), wave = threadIdx.x / FE_WAVE, waves = (blockDim.x + FE_WAVE - 1) / FE_WAVE;
+  s1 = wave_sum_dpp(s1);
+  s2 = wave_sum_dpp(s2);
+  s3 = wave_sum_dpp(s3);
+  if (lane == 0) { scratch[0][wave] = s1; scratch[1][wave] = s2; scratch[2][wave] = s3; }
+  __syncthreads();
+  s1 = s2 = s3 = 0.f;
+  for (int i = 0; i < waves; ++i) { s1 += scratch[0][i]; s2 += scratch[1][i]; s3 += scratch[2][i]; }
   const float n = (float)width;
-  const float a = coeff[0] * rsqrtf(s1 / n + eps), b = coeff[1] * rsqrtf(s2 / n + eps),
-              c3 = coeff[2] * rsqrtf(s3 / n + eps), e = coeff[3];
-  for (int c = threadIdx.x; c < width; c += blockDim.x) {
-    const float v = load_as_float(z + base + c);
+  const float a = c0 * rsqrtf(s1 / n + eps), b = c1 * rsqrtf(s2 / n + eps), c3 = c2 * rsqrtf(s3 / n + eps);
+  auto norm = [&](float v) {
     const float v2 = v * v;
-    store_from_float(out + base + c, a * v + b * v2 + c3 * (v2 * v) + e);
+    return a * v + b * v2 + c3 * (v2 * v) + e;
+  };
+  if constexpr (N > 0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int c = threadIdx.x + j * blockDim.x;
+      if (c < width) store_from_float(out + base + c, norm(held[j]));
+    }
+  } else {
+    for (int c = threadIdx.x; c < width; c += blockDim.x) store_from_float(out + base + c, norm(load_as_float(z + base + c)));
   }
 }
 
@@ -401,11 +511,21 @@ extern "C" int fe_polynorm(const void* z, int dtype, const float* coeff, float e
                            hipStream_t stream) {
   if (rows <= 0) return FE_OK;
   if (width <= 0 || !(eps > 0.f)) return FE_BAD_ARGUMENT;
-  if (dtype == FE_F32)
-    polynorm_kernel<float><<<rows, row_threads(rows, width), 0, stream>>>((const float*)z, coeff, eps, (float*)out, width);
-  else if (dtype == FE_BF16)
-    polynorm_kernel<bf16_t><<<rows, row_threads(rows, width), 0, stream>>>((const bf16_t*)z, coeff, eps, (bf16_t*)out, width);
+  const int threads = row_threads(rows, width);
+#define LAUNCH(T, N) polynorm_kernel<T, N><<<rows, threads, 0, stream>>>((const T*)z, coeff, eps, (T*)out, width)
+#define LAUNCH_HELD(T)                         \
+  switch (held_elements(width, threads)) {     \
+    case 1: LAUNCH(T, 1); break;               \
+    case 2: LAUNCH(T, 2); break;               \
+    case 4: LAUNCH(T, 4); break;               \
+    case 8: LAUNCH(T, 8); break;               \
+    default: LAUNCH(T, 0);                     \
+  }
+  if (dtype == FE_F32) { LAUNCH_HELD(float); }
+  else if (dtype == FE_BF16) { LAUNCH_HELD(bf16_t); }
   else return FE_BAD_ARGUMENT;
+#undef LAUNCH_HELD
+#undef LAUNCH
   return fe_check_launch();
 }
 

@@ -83,6 +83,32 @@ def test_rmsnorm_update(ops, out_dtype, parts, rows, width):
         torch.testing.assert_close(out.cpu().float(), out_ref.float(), **tol(out_dtype))
 
 
+@pytest.mark.parametrize("rows,width", [(2, 256), (513, 257), (513, 513), (6, 1024), (6, 1025), (513, 1025), (6, 2049), (6, 4097), (600, 2049), (6, 8192), (6, 8193)])
+@pytest.mark.parametrize("parts", [1, 4, 5, 9])
+def test_rows_held_in_registers(ops, rows, width, parts):
+    """Both sides of every count of elements a thread holds (256 and 1,024 threads a row), parts that fill no round of four; NaN
+    beside the last element stays in its row."""
+    g = torch.Generator().manual_seed(width + parts)
+    h, update, w = rand(g, rows, width, scale=2.0), rand(g, parts, rows, width), 1.0 + rand(g, width, scale=0.1)
+    update[0, rows - 1, width - 1] = float("nan")
+    h_ref, hd = h.clone(), h.to(DEV)
+    refs.rmsnorm_update(h_ref, update, w, 1e-6, None)
+    ops.rmsnorm_update(hd, update.to(DEV), w.to(DEV), 1e-6, None)
+    torch.testing.assert_close(hd.cpu(), h_ref, atol=2e-5, rtol=2e-5, equal_nan=True)
+    if parts > 1:
+        many = [update[:, : rows - 1].contiguous(), update[:2, : rows - 1].contiguous()] * 2
+        weights = 1.0 + rand(g, 4, width, scale=0.1)
+        want = refs.rmsnorm_mean(many, weights, 1e-6, torch.empty(rows - 1, width))
+        torch.testing.assert_close(ops.rmsnorm_mean(dev(*many), weights.to(DEV), 1e-6, torch.empty(rows - 1, width, device=DEV)).cpu(), want,
+                                   atol=2e-5, rtol=2e-5)
+    coeff = torch.tensor([0.7, -0.4, 0.25, 0.1])
+    for dtype in (torch.float32, torch.bfloat16):
+        z = update[0].to(dtype)
+        want = refs.polynorm(z, coeff, 1e-6, torch.empty_like(z))
+        torch.testing.assert_close(ops.polynorm(z.to(DEV), coeff.to(DEV), 1e-6, torch.empty_like(z, device=DEV)).cpu().float(), want.float(),
+                                   **tol(dtype), equal_nan=True)
+
+
 @pytest.mark.parametrize("count", [1, 2, 4])
 @pytest.mark.parametrize("rows,width", [(5, 40), (129, 1000)])
 def test_rmsnorm_mean(ops, count, rows, width):

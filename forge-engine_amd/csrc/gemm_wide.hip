@@ -247,13 +247,13 @@ __global__ __launch_bounds__(64 * WPB, 2) void gemm_wide_kernel(
 // columns) a block of four or two waves takes; 32 gives a launch of few blocks twice as many; 128 (eight
 // waves, plain endings) halves how often x is read.
 // lds_tile >= 0: endings 0 to 2 with both operands through LDS instead, in the tile that gemm_lds.h lists under that number
-// (row_tile and block_rows do not count then).  limit, alpha: the bounded activation's (gate_act.h).
+// (row_tile and block_rows do not count then).
 extern "C" int fe_gemm_wide(const void* x, const void* w, void* out, int M, int N, int K, long long ldw,
                             long long ldo, int ending, int parts, long long part_stride, int row_tile,
-                            int block_rows, int lds_tile, int activation, float limit, float alpha, hipStream_t stream) {
+                            int block_rows, int lds_tile, int activation, hipStream_t stream) {
   if (M < 1) return FE_OK;
   GateAct act;
-  if (!gate_act(activation, &act, limit, alpha)) return FE_BAD_ARGUMENT;
+  if (!gate_act(activation, &act)) return FE_BAD_ARGUMENT;
   if (N < 1 || K < WSTEP || K % WSTEP || ldw < K || ldw % 8 || ldo < N) return FE_BAD_ARGUMENT;
   if ((((uintptr_t)x) & 15) || (((uintptr_t)w) & 15)) return FE_BAD_ARGUMENT;
   if (ending < EPI_PARTS || ending > EPI_SWIGLU_HALF) return FE_BAD_ARGUMENT;

@@ -163,7 +163,6 @@ def add_rows(h: Tensor, delta: Tensor | None, other: Tensor | None = None, shift
 
 
 GATE_ACTS = {"silu": 0, "gelu_tanh": 1}     # FE_GATE_* of csrc/gate_act.h
-GATE_BOUNDED = 2
 
 
 def _gate_act(act: str) -> c_int:
@@ -457,7 +456,7 @@ def gemm_wide(x: Tensor, weight: Tensor, ending: str = "bf16", parts: int = 1, r
         raise KernelError(f"no ending {ending!r} with {parts} parts")
     _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
           c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
-          c_int(row_tile or (16 if m <= 16 else 64 if m <= 64 else 128)), c_int(block_rows), c_int(-1), _gate_act(act), c_float(0.0), c_float(0.0), _stream())
+          c_int(row_tile or (16 if m <= 16 else 64 if m <= 64 else 128)), c_int(block_rows), c_int(-1), _gate_act(act), _stream())
     return out
 
 
@@ -571,11 +570,10 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     return -(-rows // 128) * -(-2 * columns // 160) <= WIDE_CUS
 
 
-def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu",
-             bounded: tuple[float, float] | None = None) -> Tensor:
+def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu") -> Tensor:
     """x @ weight^T for bfloat16 rows: ``"parts"`` float32 partial sums [parts, M, N] over runs of whole 64-steps of K,
     ``"bf16"`` [M, N], or ``"gated"``: act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first; ``act`` as in
-    ``swiglu``; ``bounded`` (limit, alpha): ``linear_gated``'s instead).  ``tile``: the block's, see ``LDS_TILES``."""
+    ``swiglu``).  ``tile``: the block's, see ``LDS_TILES``."""
     _gpu(x, "x", torch.bfloat16)
     _gpu(weight, "weight", torch.bfloat16, contiguous=False)
     if (x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1] or x.shape[1] % 64 or weight.stride(1) != 1
@@ -596,8 +594,7 @@ def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int =
         raise KernelError(f"no tile {tile}")
     _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
           c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
-          c_int(64), c_int(64), c_int(tile), c_int(GATE_BOUNDED) if bounded else _gate_act(act), c_float(bounded[0] if bounded else 0.0),
-          c_float(bounded[1] if bounded else 0.0), _stream())
+          c_int(64), c_int(64), c_int(tile), _gate_act(act), _stream())
     return out
 
 
@@ -731,16 +728,6 @@ GATED_TILE_MAX_ROWS = 4096
 GATED_TILE_MAX_K = 3072
 
 
-def _gate_to_library(x: Tensor, gate_up_weight: Tensor) -> bool:
-    return (2 <= x.shape[0] <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
-            and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
-
-
-def _lds_gate_takes(x: Tensor, gate_up_weight: Tensor) -> bool:
-    return (not _gate_to_library(x, gate_up_weight) and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
-            and _lds_gate_pays(x.shape[0], gate_up_weight.shape[0] // 2, gate_up_weight.shape[1]))
-
-
 def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tensor:
     """act(x Wg^T) * (x Wu^T) for the fused weight [2I, K] (gate rows first); ``act`` as in ``swiglu``."""
     _gpu(x, "x")
@@ -752,8 +739,10 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tenso
             and x.data_ptr() % 16 == 0 and gate_up_weight.data_ptr() % 16 == 0
             and gate_up_weight.shape[0] * gate_up_weight.stride(0) < 2 ** 32 and rows * x.shape[1] < 2 ** 32):
         return gemm_gated(x, gate_up_weight, shape=3, act=act)
-    to_library = _gate_to_library(x, gate_up_weight)
-    if _lds_gate_takes(x, gate_up_weight):
+    to_library = (2 <= rows <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
+                  and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
+    if (not to_library and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
+            and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])):
         tile, _ = lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])
         return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
     paired_fits = (rows <= MID_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16
@@ -951,8 +940,11 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
                     window: int | None = None, num_decode: int | None = None,
                     max_ctx: int | None = None, splits: int | None = None, chunk: int | None = None,
                     sink: Tensor | None = None, softcap: float | None = None, slopes: Tensor | None = None,
-                    dist_bias: Tensor | None = None) -> Tensor:
+                    dist_bias: Tensor | None = None, by_length: int | None = None) -> Tensor:
     """Attention of every query token of a mixed batch over its paged keys.
+
+    ``splits``: key runs of every single token's sequence; ``by_length``: runs by length instead, this many a kv head beyond the
+    sequences; neither: ``decode_runs``.
 
     ``chunk`` (a token reads keys of its own run of that many positions only), ``sink``
     (float32 [Hq]: exp(sink_h) joins head h's softmax denominator), ``softcap`` (scores, after
@@ -1047,7 +1039,9 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
         if splits is None:
             reach = max_ctx if max_ctx is not None else 16 * 4 * 8
             reach = reach if chunk is None else min(reach, chunk)
-            splits = decode_runs(num_decode, num_seqs, kv_heads, head_dim, reach)
+            splits = -by_length if by_length else decode_runs(num_decode, num_seqs, kv_heads, head_dim, reach)
+        elif splits < 1:
+            raise KernelError("splits must be at least 1")
         part_o, part_ml, counters = _split_scratch(q.device, num_seqs, kv_heads, groups, head_dim, splits)
         mask = (c_int(chunk or 0), _ptr(sink)) + ((_ptr(slopes),) if slopes is not None else ()) if masked else ()
         if dist_bias is not None:
@@ -1121,14 +1115,15 @@ def decode_attention_prepare(qkv: Tensor, q_weight: Tensor | None, k_weight: Ten
                              key_pages: Tensor, value_pages: Tensor, out: Tensor, cu_q: Tensor, ctx_len: Tensor,
                              block_table: Tensor, *, q_heads: int, kv_heads: int, head_dim: int, eps: float,
                              scale: float, window: int | None = None, max_ctx: int | None = None,
-                             splits: int | None = None) -> Tensor:
+                             splits: int | None = None, by_length: int | None = None) -> Tensor:
     """A step of single tokens only, from the fused projection's output to the attention's
     output in one launch: what ``qk_norm_rope_write`` followed by ``paged_attention`` does for
     such a batch (same bits in the cache; qkv is left as it is).
 
     qkv [B, (Hq + 2 Hkv) D] bfloat16, one row per sequence, or float32 [parts <= 4, B, ...]:
     partial sums of the projection (``linear_in_parts``), added up in order and rounded to
-    bfloat16 inside the kernel.  ctx_len counts the new token, whose position is ctx_len - 1."""
+    bfloat16 inside the kernel.  ctx_len counts the new token, whose position is ctx_len - 1.
+    ``splits`` and ``by_length`` as in ``paged_attention``."""
     width = (q_heads + 2 * kv_heads) * head_dim
     if isinstance(qkv, Tensor) and qkv.dtype == torch.float32:
         _gpu(qkv, "qkv", torch.float32)
@@ -1172,7 +1167,9 @@ def decode_attention_prepare(qkv: Tensor, q_weight: Tensor | None, k_weight: Ten
         raise KernelError("block_table must be [sequences, max_blocks] with unit inner stride")
     groups = q_heads // kv_heads
     if splits is None:
-        splits = decode_runs(num_seqs, num_seqs, kv_heads, head_dim, max_ctx if max_ctx is not None else 16 * 4 * 8)
+        splits = -by_length if by_length else decode_runs(num_seqs, num_seqs, kv_heads, head_dim, max_ctx if max_ctx is not None else 16 * 4 * 8)
+    elif splits < 1:
+        raise KernelError("splits must be at least 1")
     part_o, part_ml, counters = _split_scratch(qkv.device, num_seqs, kv_heads, groups, head_dim, splits)
     _call("attention_decode", "fe_paged_attention_decode_prepare", _ptr(qkv), c_int(sums),
           c_longlong(num_seqs * width), c_longlong(width), _ptr(q_weight),
@@ -2359,12 +2356,7 @@ def moe_experts(x: Tensor, chosen: Tensor | None, weights: Tensor, gate_up: Tens
 
 def linear_gated(x: Tensor, gate_up_weight: Tensor, *, limit: float, alpha: float) -> Tensor:
     """``min(g, limit) * sigmoid(alpha * min(g, limit)) * (clamp(u, -limit, limit) + 1)`` with g and u the two
-    halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype.  bfloat16 where
-    ``linear_swiglu`` takes the product through LDS: in its ending, without a launch of its own (4,096 x 2,048 at 8 rows:
-    6.2 + 4.4 us -> 6.2) and without the rounding of g and u."""
-    if (limit > 0.0 and gate_up_weight.dim() == 2 and gate_up_weight.shape[0] % 2 == 0 and _lds_gate_takes(_gpu(x, "x"), _gpu(gate_up_weight, "gate_up_weight", contiguous=False))):
-        tile, _ = lds_plan(x.shape[0], *gate_up_weight.shape, gate_up_weight.shape[0])
-        return gemm_lds(x, gate_up_weight, "gated", tile=tile, bounded=(limit, alpha))
+    halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype."""
     gate_up = linear(x, gate_up_weight)
     tokens, width = gate_up.shape
     if width % 2 or not limit > 0.0:

@@ -911,20 +911,6 @@ def test_logits_through_a_vocabulary(ops, rows):
     assert bool(((got[:, at].double() - a @ b.t()).abs() <= (a.abs() @ b.abs().t()) * 2 * 2048 * 2.0 ** -24).all())
 
 
-@pytest.mark.parametrize("rows", [1, 5, 16, 17, 300])
-def test_linear_gated_in_the_product(ops, rows):
-    """The bounded gate in the product's ending: against 64 bits, one rounding to bfloat16 (and the float32 sums' error at 2 k 2^-24)."""
-    g = torch.Generator().manual_seed(rows)
-    x, w = rand(g, rows, 1024, dtype=torch.bfloat16), rand(g, 2 * 260, 1024, dtype=torch.bfloat16, scale=0.05)
-    got = ops.linear_gated(x.to(DEV), w.to(DEV), limit=0.8, alpha=1.702).double().cpu()
-    both = x.double() @ w.double().t()
-    gate, up = both[:, :260].clamp(max=0.8), both[:, 260:].clamp(-0.8, 0.8)
-    want = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
-    torch.testing.assert_close(got, want, atol=2e-3, rtol=2.0 ** -8)
-    with pytest.raises(ops.KernelError):
-        ops.linear_gated(x.to(DEV), w.to(DEV), limit=0.0, alpha=1.0)
-
-
 def test_stored_products_round_to_nearest_even(ops):
     """A product whose float32 sum is exact (one bfloat16 and a smaller one): the stored bfloat16 is torch's rounding of it, at
     ties, just beside them, across a power of two, at the largest finite value, at infinities and NaN."""
@@ -1365,11 +1351,11 @@ def test_decode_attention_in_runs_by_length(ops, count, kv_heads, head_dim, wind
     sizes = dict(q_heads=2 * kv_heads, kv_heads=kv_heads, head_dim=head_dim)
     more = min(more, 4 * (64 // kv_heads) + 40)
     outs = []
-    for splits in (1, -more, -more):
+    for form in ({"splits": 1}, {"by_length": more}, {"by_length": more}):
         kp_dev, vp_dev = kp.to(DEV), vp.to(DEV)
         out = torch.full((count, 2 * kv_heads * head_dim), float("nan"), dtype=torch.bfloat16, device=DEV)
         ops.decode_attention_prepare(qkv.to(DEV), qw.to(DEV), kw.to(DEV), inv_freq.to(DEV), kp_dev, vp_dev, out, cu.to(DEV), ctx.to(DEV),
-                                     table.to(DEV), eps=1e-6, scale=0.1, window=window or None, max_ctx=1501, splits=splits, **sizes)
+                                     table.to(DEV), eps=1e-6, scale=0.1, window=window or None, max_ctx=1501, **form, **sizes)
         outs.append((out, kp_dev, vp_dev))
     for out, kp_dev, vp_dev in outs[1:]:
         # float32 sums in another order, one rounding each: an ulp of bfloat16 at most
@@ -1389,18 +1375,19 @@ def test_decode_attention_in_runs_by_length_beside_portions(ops):
     tokens = q.shape[0]
     for chunk in (None, 128):
         results = []
-        for splits in (1, -5, -100):
+        for form in ({"splits": 1}, {"by_length": 5}, {"by_length": 100}):
             out = torch.full((tokens, 8 * 128), float("nan"), dtype=torch.bfloat16, device=DEV)
             ops.paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), out, cu.to(DEV), ctx.to(DEV), table.to(DEV), num_seqs=len(seqs), max_q_len=9,
-                                num_decode=17, q_heads=8, kv_heads=4, head_dim=128, scale=0.1, max_ctx=1024, splits=splits, chunk=chunk)
+                                num_decode=17, q_heads=8, kv_heads=4, head_dim=128, scale=0.1, max_ctx=1024, chunk=chunk, **form)
             results.append(out.float())
         for other in results[1:]:
             torch.testing.assert_close(other, results[0], atol=2e-3, rtol=2.0 ** -7)
     case = _prepare_case(g, 2, 1, 64, 16, [3] * 65)
     qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq = (t.to(DEV) for t in case[:9])
-    with pytest.raises(ops.KernelError):                       # a lane a sequence
-        ops.decode_attention_prepare(qkv, qw, kw, inv_freq, kp, vp, torch.empty(65, 128, dtype=torch.bfloat16, device=DEV), cu, ctx, table,
-                                     q_heads=2, kv_heads=1, head_dim=64, eps=1e-6, scale=0.1, max_ctx=64, splits=-4)
+    for form in ({"by_length": 4}, {"splits": -4}, {"splits": 0}, {"by_length": 5000}):      # a lane a sequence: 65 are too many
+        with pytest.raises(ops.KernelError):
+            ops.decode_attention_prepare(qkv, qw, kw, inv_freq, kp, vp, torch.empty(65, 128, dtype=torch.bfloat16, device=DEV), cu, ctx, table,
+                                         q_heads=2, kv_heads=1, head_dim=64, eps=1e-6, scale=0.1, max_ctx=64, **form)
 
 
 def test_which_decode_launches_take_runs_by_length(ops):

@@ -121,10 +121,10 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
                        long long part_stride, GateAct act, hipStream_t stream) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, COLUMNS = END == END_GATED ? BN / 2 : BN;
   constexpr size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES;
-  static int checked = 0;
+  static std::atomic<bool> raised{false};
   auto kernel = gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END>;
-  const int fit = lds_tile::fit_to_launch((const void*)kernel, bytes, &checked);
-  if (fit != FE_OK) return fit;
+  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, bytes, &raised);
+  if (limit_raised != FE_OK) return limit_raised;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + COLUMNS - 1) / COLUMNS;
   if (tiles_m * tiles_n * parts > 0x7fffffffLL) return FE_BAD_ARGUMENT;
   const int steps = K / KSTEP, per_part = (steps + parts - 1) / parts;
@@ -137,7 +137,6 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
 // Operands and endings as fe_gemm_wide's (ending 0: parts, 1: bfloat16, 2: gated); the caller has checked them.
 // tile: rows of x x weight rows a block takes: 0: 32 x 32, 1: 64 x 32, 2: 64 x 64, 3: 64 x 80, 4: 64 x 96, 5: 128 x 64,
 //   6: 128 x 128, 7: 128 x 160, 8: 32 x 64, 9 to 13: 16 x 16, 32, 48, 64, 80.
-// FE_BAD_ARGUMENT also if the library was built with registers spilled to scratch memory: the kernel then never runs.
 static int launch(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
                   int parts, long long part_stride, int tile, GateAct act, hipStream_t stream) {
 #define FE_END(END, ...) return launch_tile<__VA_ARGS__, END>(x, w, out, M, N, K, ldw, ldo, parts, part_stride, act, stream)

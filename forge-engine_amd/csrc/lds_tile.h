@@ -2,6 +2,7 @@
 // of the other (bfloat16, K contiguous in both), WM x WN waves of 16 MI x 16 NI each, in KG groups that share a step's K.
 #pragma once
 #include "common.h"
+#include <atomic>
 
 namespace lds_tile {
 
@@ -11,35 +12,26 @@ typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
 
 constexpr int KSTEP = 64;          // elements of K a step
 
-// wait until at most n of this wave's vector memory operations are outstanding (n < 64)
-#define FE_WAIT_VMEM(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | ((((n) >> 4) & 0x3) << 14) | (0x7 << 4) | (0xF << 8))
-
-__device__ __forceinline__ void load_to_lds(const void* global, void* lds) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
-                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+// 16 bytes a lane from `global` to LDS byte address `at` + 16 * lane (`at` the same in every lane).  In assembly, because behind the
+// builtin every read of LDS that the compiler forms waits for all loads into LDS that are under way; the statement writes no register,
+// so a load under way has nothing of the compiler's to overwrite.  (The other way round, reads of LDS in assembly that are waited for
+// later, a register that looks free or is copied meanwhile would be lost; that form was as fast: 1,316 products of 1 to 8,192 rows
+// take 0.996 of its time with the compiler's own reads, which it counts and waits for itself.)
+__device__ __forceinline__ void load_to_lds(const void* global, unsigned int at) {
+  unsigned int m0;       // kept: the compiler takes m0 as untouched by a statement
+  asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off\n s_mov_b32 m0, %0"
+               : "=&s"(m0) : "v"(global), "s"(at) : "memory");
 }
-
-// 16 bytes from LDS byte address `at` + OFFSET (a constant below 65536); nothing waits for them here (the compiler's own
-// reads of LDS would wait for every load into LDS that is under way, too)
-template <int OFFSET>
-__device__ __forceinline__ uintx4 lds_read16(unsigned int at) {
-  uintx4 v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFFSET) : "memory");
-  return v;
+// wait until at most PENDING of this wave's loads are outstanding (PENDING < 64; loads of the compiler's in between only make it longer)
+template <int PENDING>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PENDING) : "memory");
 }
-// COUNT fragments of sixteen rows, 2,048 bytes apart
-template <int COUNT, int FROM = 0>
-__device__ __forceinline__ void lds_read_rows(unsigned int at, uintx4* v) {
-  if constexpr (FROM < COUNT) {
-    v[FROM] = lds_read16<2048 * FROM>(at);
-    lds_read_rows<COUNT, FROM + 1>(at, v);
-  }
-}
-// every read of LDS of this wave has arrived; `v` are the registers that the wait is for
-template <int COUNT>
-__device__ __forceinline__ void lds_arrived(uintx4* v) {
-#pragma unroll
-  for (int i = 0; i < COUNT; ++i) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[i]));
+// all of this wave's reads of LDS have arrived, and it goes on when every wave of the block is here
+__device__ __forceinline__ void reads_done_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4));      // lgkmcnt(0), and nothing of the other counters
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 template <int MI, int NI, int WM, int WN, int KG, int STAGES>
@@ -51,9 +43,8 @@ struct Shape {
 
 // Fills acc[i][j] of lane (r = lane % 16, q = lane / 16) of wave (wm, wn) with the products of row 16 (MI wm + i) + r of the first
 // operand and rows 16 (NI wn + j) + 4 q .. + 3 of the second, over 64-steps [first, last) of K (a multiple of 64, or, with
-// HALF_END, of 32).  row_of(j): where
-// row j of the tile begins, the first operand's BM rows, then the second's BN.  Returns whether this wave holds the sums
-// (those of group 0 do); every thread of the block must call it.
+// HALF_END, of 32).  row_of(j): where row j of the tile begins, the first operand's BM rows, then the second's BN.  Returns
+// whether this wave holds the sums (those of group 0 do); every thread of the block must call it.
 //
 // LDS holds a step of a tile as [row][8 chunks of 16 bytes], chunk c of row j at position c ^ (j % 8): the lanes that a 16-byte
 // read serves in one cycle then hit different bank groups (no conflicts counted).  Both operands go there straight from memory
@@ -66,6 +57,7 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
   constexpr int STAGE = (BM + BN) * 8;              // 16-byte units of a stage
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int my_chunk = (lane & 7) ^ (lane >> 3);    // (a group's first row is a multiple of eight)
+  const unsigned int base = __builtin_amdgcn_readfirstlane((unsigned int)(size_t)(const __attribute__((address_space(3))) char*)&lds[0]);
   // this lane's place in each of the wave's loads
   const bf16_t* from[LOADS + 1];
 #pragma unroll
@@ -74,12 +66,12 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
     const int k0 = min(step, last - 1) * KSTEP;
     const int at = k0 + (HALF_END && k0 + KSTEP > K ? my_chunk & 3 : my_chunk) * 8;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_to_lds(from[i] + at, &lds[stage * STAGE + (wave + WAVES * i) * 64]);
-    if (MORE > 0 && wave < MORE) load_to_lds(from[LOADS] + at, &lds[stage * STAGE + (wave + WAVES * LOADS) * 64]);
+    for (int i = 0; i < LOADS; ++i) load_to_lds(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
+    if (MORE > 0 && wave < MORE) load_to_lds(from[LOADS] + at, base + (stage * STAGE + (wave + WAVES * LOADS) * 64) * 16);
   };
   const int r = lane & 15, q = lane >> 4, group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  const unsigned int base = (unsigned int)(size_t)(const __attribute__((address_space(3))) char*)&lds[0];
-  const unsigned int x_at = base + (wm * 16 * MI + r) * 128, w_at = base + (BM + wn * 16 * NI + r) * 128;
+  const uintx4* x_at = lds + (wm * 16 * MI + r) * 8;
+  const uintx4* w_at = lds + (BM + wn * 16 * NI + r) * 8;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -88,9 +80,11 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
   if (first < last) {
     uintx4 a0[MI], b0[NI], a1[MI], b1[NI];
     auto fragments = [&](int stage, int t, uintx4* a, uintx4* b) {
-      const unsigned int at = stage * (STAGE * 16) + (((4 * (group * T + t) + q) ^ (r & 7)) * 16);
-      lds_read_rows<MI>(x_at + at, a);
-      lds_read_rows<NI>(w_at + at, b);
+      const int at = stage * STAGE + ((4 * (group * T + t) + q) ^ (r & 7));
+#pragma unroll
+      for (int i = 0; i < MI; ++i) a[i] = x_at[at + 128 * i];
+#pragma unroll
+      for (int j = 0; j < NI; ++j) b[j] = w_at[at + 128 * j];
     };
     auto multiply = [&](const uintx4* a, const uintx4* b) {
 #pragma unroll
@@ -107,10 +101,9 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
       if (ends_step) {
         // this wave's share of the next step has landed, and behind the barrier everyone's; everyone has read all of
         // this step, whose buffer is filled again
-        if (MORE > 0 && wave < MORE) FE_WAIT_VMEM((LOADS + 1) * (STAGES - 2));
-        else FE_WAIT_VMEM(LOADS * (STAGES - 2));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        if (MORE > 0 && wave < MORE) wait_loads<(LOADS + 1) * (STAGES - 2)>();
+        else wait_loads<LOADS * (STAGES - 2)>();
+        reads_done_barrier();
         load(step + STAGES, stage);
         stage = stage + 1 == STAGES ? 0 : stage + 1;
         from_stage = stage;
@@ -119,18 +112,13 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
       __builtin_amdgcn_sched_barrier(0);
       if (!HALF_END || step * KSTEP + (group * T + t) * 32 < K) multiply(a, b);
       __builtin_amdgcn_sched_barrier(0);
-      lds_arrived<MI>(a_next);
-      lds_arrived<NI>(b_next);
     };
 #pragma unroll
     for (int s = 0; s < STAGES; ++s) load(first + s, s);
-    if (MORE > 0 && wave < MORE) FE_WAIT_VMEM((LOADS + 1) * (STAGES - 1));
-    else FE_WAIT_VMEM(LOADS * (STAGES - 1));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    if (MORE > 0 && wave < MORE) wait_loads<(LOADS + 1) * (STAGES - 1)>();
+    else wait_loads<LOADS * (STAGES - 1)>();
+    reads_done_barrier();
     fragments(0, 0, a0, b0);
-    lds_arrived<MI>(a0);
-    lds_arrived<NI>(b0);
     if constexpr (T == 2) {
       for (int step = first; step < last; ++step) {
         half(step, false, 1, a0, b0, a1, b1);
@@ -144,11 +132,10 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
       }
       if (step < last) half(step, true, 0, a0, b0, a1, b1);
     }
-    FE_WAIT_VMEM(0);
+    wait_loads<0>();
   }
   if constexpr (KG > 1) {
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    reads_done_barrier();
     floatx4* meet = (floatx4*)lds;
     if (group > 0) {
 #pragma unroll
@@ -166,18 +153,13 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
   return true;
 }
 
-// The fragments' reads are waited for by hand: a build that spills registers would move values that are still in flight,
-// and is never launched.  Also raises the kernel's LDS limit.  0: not yet asked, 1: fit, -1: refused.
-static inline int fit_to_launch(const void* kernel, size_t lds_bytes, int* checked) {
-  if (*checked == 0) {
-    hipFuncAttributes attributes;
-    if (hipFuncGetAttributes(&attributes, kernel) != hipSuccess) return FE_LAUNCH_FAILED;
-    if (attributes.localSizeBytes != 0) { *checked = -1; return FE_BAD_ARGUMENT; }
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
-      return FE_LAUNCH_FAILED;
-    *checked = 1;                 // (a race here only repeats the calls)
-  }
-  return *checked < 0 ? FE_BAD_ARGUMENT : FE_OK;
+// Lets a kernel use more LDS than a launch may by default; once a kernel (asked for from several threads at a time it is only
+// done again).
+static inline int raise_lds_limit(const void* kernel, size_t lds_bytes, std::atomic<bool>* raised) {
+  if (raised->load(std::memory_order_relaxed)) return FE_OK;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess) return FE_LAUNCH_FAILED;
+  raised->store(true, std::memory_order_relaxed);
+  return FE_OK;
 }
 
 }  // namespace lds_tile

@@ -453,10 +453,10 @@ static int launch_moe_tile(const bf16_t* a, const bf16_t* w, const int* offsets,
                            int form, const float* extra, int extra_parts, hipStream_t stream) {
   constexpr int TILE_ROWS = 16 * MI * WM, TILE_COLS = 16 * NI * WN, COLUMNS = MODE == 0 ? TILE_COLS / 2 : TILE_COLS;
   constexpr size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES;
-  static int checked = 0;
+  static std::atomic<bool> raised{false};
   auto kernel = moe_lds_kernel<MI, NI, WM, WN, KG, STAGES, MODE>;
-  const int fit = lds_tile::fit_to_launch((const void*)kernel, bytes, &checked);
-  if (fit != FE_OK) return fit;
+  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, bytes, &raised);
+  if (limit_raised != FE_OK) return limit_raised;
   const long long pairs = (long long)tokens * top, slots = pairs / TILE_ROWS + experts, tiles = ((long long)N + COLUMNS - 1) / COLUMNS;
   const long long blocks = (slots * tiles + 7) / 8 * 8;
   if (blocks > 0x7fffffffLL) return FE_BAD_ARGUMENT;

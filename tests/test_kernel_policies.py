@@ -3,9 +3,11 @@ and how many key splits the decode attention takes."""
 
 from __future__ import annotations
 
+import re
+
 import pytest
 
-from forge_engine_amd.kernels import ops
+from forge_engine_amd.kernels import build, ops
 
 
 @pytest.mark.parametrize("steps", [1, 3, 4, 7, 20, 32, 76, 500])
@@ -192,3 +194,17 @@ def test_the_product_that_stores_bfloat16_needs_blocks_enough_beyond_64_rows():
     for rows in (17, 32, 64):
         assert ops._wide_store_pays(rows, 4096, 2048) and ops._wide_store_pays(rows, 7168, 5120)
         assert not ops._wide_store_pays(rows, 8192, 6144)       # 100 MB of weight: the library's
+
+
+@pytest.mark.parametrize("source", ["lds_tile.h", "gemm_lds.h", "moe.hip", "gemm_f32.hip"])
+def test_loads_in_assembly_leave_no_register_in_flight(source):
+    """A load in an assembly statement that writes a register is waited for in the same statement: to the compiler the register is
+    written there and then, and it may copy it or give it away.  (Loads into LDS write no register.)"""
+    text = (build.SOURCE_DIR / source).read_text()
+    statements = [m.group(0) for m in re.finditer(r"asm volatile\(.*?\);", text, re.S)]
+    for statement in statements:
+        code = "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', statement.split(" : ")[0]))
+        if re.search(r"\b(ds_read|ds_load|global_load|buffer_load|flat_load|s_load)", code.replace("global_load_lds_dwordx4", "")):
+            assert re.search(r"s_waitcnt (lgkmcnt|vmcnt)\(0\)$", code), statement
+    if source in ("lds_tile.h", "gemm_f32.hip"):
+        assert statements

@@ -332,8 +332,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
             and _lds_store_pays(x.shape[0], *weight.shape)):
         tile, _ = lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])
         return gemm_lds(x, weight, "bf16", tile=tile)
-    if (bias is None and out_dtype == torch.float32 and x.shape[0] <= MID_ROWS and weight.shape[0] >= LDS_HEAD_WEIGHT_ROWS
-            and weight.shape[1] >= LDS_HEAD_MIN_K and _lds_fits(x, weight)):
+    if bias is None and out_dtype == torch.float32 and _lds_fits(x, weight) and _lds_head_pays(x.shape[0], *weight.shape):
         rows = x.shape[0]          # (hundreds of tiles a CU: the cheapest tile whatever the rounds, not the plan's)
         return gemm_lds(x, weight, "parts", tile=10 if rows <= 8 else 12 if rows <= 16 else 8 if rows <= 32 else 4)[0]
     if bias is None and _skinny_fits(x, weight) and out_dtype in (torch.float32, torch.bfloat16) and not to_library:
@@ -482,10 +481,7 @@ def _wide_parts(m: int, n: int, k: int, block_rows: int = 64, most: int = 16) ->
 LDS_TILES = ((32, 32, 2, 0.151, 0.256), (64, 32, 1, 0.191, 0.382), (64, 64, 2, 0.212, 0.348), (64, 80, 1, 0.303, 0.606),
              (64, 96, 2, 0.292, 0.451), (128, 64, 1, 0.317, 0.634), (128, 128, 1, 0.510, 1.02), (128, 160, 1, 0.630, 1.26), (32, 64, 2, 0.202, 0.378),
              (16, 16, 2, 0.073, 0.117), (16, 32, 2, 0.116, 0.247), (16, 48, 2, 0.143, 0.334), (16, 64, 2, 0.168, 0.444), (16, 80, 1, 0.220, 0.440))
-# float32 logits, up to 64 rows through a vocabulary's weight (151,936 rows; kernel for few rows or library -> this): K = 2,560
-# 1 row 137 -> 130 us, 8: 151 -> 142, 17: 167 -> 150, 64: 185 -> 183; K = 2,048 1 row 108 -> 108, 8: 119 -> 113, 17: 148 -> 122,
-# 64: 160 -> 149; at K = 1,024 the blocks that keep x in registers win (1 row 53 against 55, 8: 58 against 59).
-LDS_HEAD_WEIGHT_ROWS = 131072
+LDS_HEAD_WEIGHT_ROWS = 131072  # float32 logits: see _lds_head_pays
 LDS_HEAD_MIN_K = 2048
 LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
@@ -557,6 +553,21 @@ def _lds_store_pays(rows: int, weight_rows: int, k: int) -> bool:
     if rows <= SKINNY_MAX_ROWS:
         return rows > 8 or (rows > 4 and k >= 2048 and weight_rows <= 8192)
     return weight_rows >= 2048 and weight_rows * k <= 26_000_000 and rows <= (512 if weight_rows <= 4096 else 256)
+
+
+def _lds_head_pays(rows: int, weight_rows: int, k: int) -> bool:
+    """float32 logits, measured at 131,072 to 262,144 weight rows (us, what took them before -> this; below, and at K < 2,048, the
+    blocks that keep x in registers win: 65,536 x 2,048 at 1 row 47 against 55).  Up to 16 rows: 151,936 x 2,560 at 8 rows 147 ->
+    139, x 5,120 at 1 row 278 -> 249; but at K of 4,096 and up to 8 rows those blocks win (131,072: 172 against 189).  17 to 64
+    rows beside the matrix library: at K = 2,048 and 4,096, rows whole 4 KB apart, where the library is slow, always (64 rows:
+    131,072 x 4,096 247 -> 218, 200,064 x 2,048 214 -> 188); else up to 32 rows where the weight's rows are no multiple of the
+    library's tiles of 256 (17 rows: 200,064 x 2,560 327 -> 201, 151,936 x 5,120 326 -> 283; but 256,000 x 2,560 230 against
+    255), and no more beyond (64 rows: 131,072 x 5,120 248 against 280, 151,936 x 5,120 313 against 328)."""
+    if weight_rows < LDS_HEAD_WEIGHT_ROWS or k < LDS_HEAD_MIN_K or rows > MID_ROWS:
+        return False
+    if rows <= SKINNY_MAX_ROWS:
+        return rows > 8 or not 3584 < k <= 4096
+    return (k % 2048 == 0 and k <= 4096) or (rows <= 32 and weight_rows % 256 != 0)
 
 
 def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:

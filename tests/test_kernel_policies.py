@@ -208,3 +208,14 @@ def test_loads_in_assembly_leave_no_register_in_flight(source):
             assert re.search(r"s_waitcnt (lgkmcnt|vmcnt)\(0\)$", code), statement
     if source in ("lds_tile.h", "gemm_f32.hip"):
         assert statements
+
+
+def test_which_logits_go_through_lds():
+    """Both sides of every line (rows, weight rows, K), see the rule."""
+    pays = ops._lds_head_pays
+    for rows, weight_rows, k in ((1, 131072, 2048), (8, 151936, 2560), (8, 131072, 3584), (9, 131072, 4096), (8, 131072, 4160), (16, 151936, 5120),
+                                 (17, 131072, 2048), (64, 256000, 2048), (64, 131072, 4096), (17, 151936, 2560), (32, 200064, 5120)):
+        assert pays(rows, weight_rows, k), (rows, weight_rows, k)
+    for rows, weight_rows, k in ((1, 131071, 2048), (1, 131072, 1984), (1, 151936, 4096), (8, 256000, 4096), (8, 151936, 3648), (65, 131072, 2048),
+                                 (17, 256000, 2560), (17, 131072, 5120), (33, 151936, 2560), (64, 200064, 5120), (17, 131072, 6144), (64, 151936, 6144)):
+        assert not pays(rows, weight_rows, k), (rows, weight_rows, k)

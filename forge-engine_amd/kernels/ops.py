@@ -483,6 +483,7 @@ LDS_TILES = ((32, 32, 2, 0.151, 0.256), (64, 32, 1, 0.191, 0.382), (64, 64, 2, 0
              (16, 16, 2, 0.073, 0.117), (16, 32, 2, 0.116, 0.247), (16, 48, 2, 0.143, 0.334), (16, 64, 2, 0.168, 0.444), (16, 80, 1, 0.220, 0.440))
 LDS_HEAD_WEIGHT_ROWS = 131072  # float32 logits: see _lds_head_pays
 LDS_HEAD_MIN_K = 2048
+LDS_GATE_MAX_ROWS = 1536       # gate/up: measured up to here (4,096 rows, 256 columns of K = 4,096: 28.6 against 43.0 us)
 LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
 
@@ -571,14 +572,38 @@ def _lds_head_pays(rows: int, weight_rows: int, k: int) -> bool:
 
 
 def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
-    """Gate/up products.  Up to 16 rows all (1 row: 3,072 columns of K = 1,024 7.9 -> 5.5 us, 9,728 of 2,560 21.9 -> 21.0,
-    17,408 of 5,120 70.8 -> 62.6) but the weights of K = 4,096 at up to four rows, whose blocks keep x in registers (1 row:
-    12,288 columns 37.4 against 38.9, 4,096 columns 15.6 against 16.8).  Beyond, where tiles of 128 x 160 make one round of the chip (3,072 columns up to 700 rows: 22 -> 20 us, 6,144
-    up to 384: 33 -> 30, 9,728 up to 256: 54 -> 42, 12,288 up to 128); with a second round the matrix library's larger
-    tiles win (9,728 columns at 320 rows: 50 against 59 us)."""
+    """Gate/up products.  What decides is how the plan's blocks fill the chip: a second round of blocks that is not nearly whole costs
+    as much as a whole one, and the plan counts it for less.  us, what took the size before -> this:
+    up to 16 rows all but such rounds (1 row: 3,072 columns of K = 1,024 7.8 -> 5.3, 9,728 of 2,560 21.7 -> 20.5, 17,408 of 5,120
+    70.9 -> 65.2; 346 blocks: 13,824 of 2,560 at 8 rows 28.9 against 33.4), and the weights of K = 4,096 from 4,096 columns at up to
+    four rows and beyond 12,288 at more, whose blocks keep x in registers (1 row: 12,288 columns 37.4 against 38.9, 8 rows: 17,408
+    columns 56.5 against 60.5);
+    17 to 64 rows one round (64 rows: 9,728 of 2,560 28.0 -> 25.2; 344 blocks: 11,008 of 2,048 24.0 against 27.5), from K = 8,192
+    and 8,192 columns on more (32 rows: 14,336 of 8,192 120 -> 92);
+    beyond, where tiles of 128 x 160 would make one round, up to 1,536 rows.  K up to 2,048: all of them (3,072 of 1,024 at 768 rows
+    23.4 -> 20.3, 256 of 1,024 at 1,100 rows 11.5 -> 6.6).  Larger K: to 256 rows one round of the plan's blocks (9,728 of 2,560 at
+    256 rows 52.5 -> 43.0; at 128 rows, 406 blocks, 35.3 against 40.3), but for few columns at K > 5,120 (256 of 8,192 at 80 rows
+    13.5 against 15.5);
+    beyond that either products too small for the library to fill the chip (1,536 of 4,096 at 320 rows 25.1 -> 21.3) or
+    tiles of 128 x 160 that nearly do (4,864 of 4,096 at 320 rows 44.3 -> 39.9; 3,072 of 4,096 at 320 rows 33.6 against 37.7,
+    1,024 of 8,192 at 1,536 rows 59.5 against 70.8)."""
+    weight_rows = 2 * columns
+    tile, _ = lds_plan(rows, weight_rows, k, weight_rows)
+    blocks = -(-rows // LDS_TILES[tile][0]) * -(-weight_rows // LDS_TILES[tile][1])
     if rows <= SKINNY_MAX_ROWS:
-        return rows > 4 or not (GATE_HALF_FEW_ROWS_MAX_K < k <= 4096 and columns >= 4096)
-    return -(-rows // 128) * -(-2 * columns // 160) <= WIDE_CUS
+        if GATE_HALF_FEW_ROWS_MAX_K < k <= 4096 and columns >= 4096 and (rows <= 4 or columns > 12288):
+            return False
+        return blocks <= WIDE_CUS or blocks > 1.6 * WIDE_CUS
+    large_tiles = -(-rows // 128) * -(-weight_rows // 160)
+    if rows > LDS_GATE_MAX_ROWS or large_tiles > WIDE_CUS:
+        return False
+    if rows <= MID_ROWS:
+        return blocks <= WIDE_CUS or (k >= 8192 and columns >= 8192)
+    if k <= 2048:
+        return True
+    if rows <= 256:
+        return blocks <= WIDE_CUS and (columns >= 512 or k <= 5120)
+    return rows * columns <= 600_000 or large_tiles >= 180
 
 
 def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu") -> Tensor:

@@ -219,3 +219,18 @@ def test_which_logits_go_through_lds():
     for rows, weight_rows, k in ((1, 131071, 2048), (1, 131072, 1984), (1, 151936, 4096), (8, 256000, 4096), (8, 151936, 3648), (65, 131072, 2048),
                                  (17, 256000, 2560), (17, 131072, 5120), (33, 151936, 2560), (64, 200064, 5120), (17, 131072, 6144), (64, 151936, 6144)):
         assert not pays(rows, weight_rows, k), (rows, weight_rows, k)
+
+
+def test_which_gated_products_go_through_lds():
+    """Both sides of every line of the rule: the rounds that the planned blocks make, rows, columns, K."""
+    pays = ops._lds_gate_pays
+    taken = ((1, 3072, 1024), (8, 9728, 2560), (8, 17408, 5120), (16, 12288, 5120), (5, 4096, 4096), (5, 12288, 4096),
+             (17, 9728, 2560), (64, 9728, 2560), (32, 14336, 8192), (65, 17408, 5120), (128, 6144, 2048), (256, 9728, 2560), (192, 9728, 2560),
+             (384, 3072, 1024), (700, 3072, 1024), (1536, 256, 1024), (80, 512, 5184), (320, 1536, 4096), (320, 4864, 4096))
+    left = ((8, 13824, 2560), (1, 14336, 2048), (4, 4096, 4096), (8, 17408, 4096), (64, 11008, 2048), (32, 16384, 4096),
+            (128, 9728, 2560), (96, 12288, 4096), (80, 256, 8192), (320, 9728, 2560), (320, 3072, 4096), (1536, 1024, 8192),
+            (1537, 256, 1024), (4096, 256, 4096), (8192, 256, 8192), (769, 3072, 1024))
+    for size in taken:
+        assert pays(*size), size
+    for size in left:
+        assert not pays(*size), size

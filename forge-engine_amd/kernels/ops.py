@@ -526,20 +526,28 @@ def _lds_fits(x: Tensor, weight: Tensor) -> bool:
 
 def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
     """(tile, parts) of a float32 update, or None where another product is the better one.  Up to 16 rows: weights of up to
-    3,072 rows (1,024 x 3,072 at 1 row 5.8 -> 3.7 us, 2,560 x 4,096 at 8 rows 7.0 -> 6.6) and others whose K is at least twice
-    their rows (4,096 x 12,288 at 1 row 21.3 -> 19.7); beside them the products below tie or win (4,096 x 4,096 at 1 row 8.5
-    against 9.4, 8,192 x 4,096 15.0 against 16.7).  Up to 64 rows: weights of up to
+    3,072 rows (1,024 x 3,072 at 1 row 5.8 -> 3.7 us, 2,560 x 4,096 at 8 rows 7.0 -> 6.6) and others of up to 5,120 whose K is at
+    least twice their rows (4,096 x 12,288 at 1 row 21.3 -> 19.7; but 6,144 x 12,288 33.8 against 38.0); beside them the products
+    below tie or win (4,096 x 4,096 at 1 row 8.5 against 9.4, 8,192 x 4,096 15.0 against 16.7).  Up to 64 rows: weights of up to
     2,048 x 4,096 by the plan (1,024 x 2,048 at 64 rows 6.5 -> 4.9 us), larger ones in the parts that fill the chip with
     blocks of 64 weight rows (2,560 x 9,728 14.6 -> 12.9, 4,096 x 12,288 25.9 -> 23.4, at 32 rows 13.1 -> 11.6 and 22.8 ->
-    20.9).  Up to 384 rows all by the plan, and up to 1,024 through weights whose K is at least twice their rows, which the
-    matrix library cuts into too few blocks (512 rows: 2,560 x 9,728 48 -> 33, 5,120 x 17,408 169 -> 86)."""
-    if rows <= SKINNY_MAX_ROWS and not (weight_rows <= 3072 or k >= 2 * weight_rows):
+    20.9).  Up to 256 rows all by the plan.  To 384 rows, beside the matrix library that adds into the stream: weights of up to 3,584
+    rows (320 rows: 3,072 x 4,096 33.7 -> 25.9), to 6,144 from K = 5,120 on (5,120 x 8,192 53.8 -> 46.4; but 4,096 x 4,096 29.9
+    against 32.4, 8,192 x 4,096 42.0 against 53.6), and from twice their rows on.  These last, which the library cuts into too few
+    blocks, also to 640 rows (512 rows: 2,560 x 9,728 55.5 -> 44.1, 5,120 x 17,408 175 -> 107), to 768 through up to 3,584 rows (3,072 x
+    9,728 1.24 times as fast; 4,096 x 8,192 70.5 against 78.2) and to 1,024 through up to 2,560 or from K = 16,384 on (1,024 rows:
+    2,560 x 9,728 85.5 -> 65.3, 5,120 x 25,600 352 -> 283; but 3,072 x 9,728 83.9 against 98.1).  (The times hold the norm that
+    adds the parts.)"""
+    long_k = k >= 2 * weight_rows
+    if rows <= SKINNY_MAX_ROWS and not (weight_rows <= 3072 or (long_k and weight_rows <= 5120)):
         return None
     if SKINNY_MAX_ROWS < rows <= MID_ROWS and not (weight_rows <= 2048 and k <= 4096):
         if weight_rows > WIDE_MAX_WEIGHT_ROWS:
             return None
         return (8 if rows <= 32 else 2), _wide_parts(rows, weight_rows, k)
-    if rows <= 384 or (rows <= 1024 and k >= 2 * weight_rows):
+    if (rows <= 256 or (rows <= 384 and (weight_rows <= 3584 or (weight_rows <= 6144 and k >= 5120)))
+            or (long_k and (rows <= 640 or (rows <= 768 and weight_rows <= 3584)
+                            or (rows <= 1024 and (weight_rows <= 2560 or k >= 16384))))):
         return lds_plan(rows, weight_rows, k, 4 * weight_rows, 8, 0.15 + rows * weight_rows * 8e-7)    # (a part's read by the norm: 5 TB/s)
     return None
 

@@ -234,3 +234,12 @@ def test_which_gated_products_go_through_lds():
         assert pays(*size), size
     for size in left:
         assert not pays(*size), size
+
+
+def test_which_updates_go_through_lds():
+    for size in ((1, 3072, 1024), (16, 5120, 10240), (17, 8192, 4096), (256, 8192, 4096), (384, 3584, 1024), (384, 6144, 5120), (640, 4096, 8192), (768, 3584, 8192),
+                 (1024, 2560, 9728), (1024, 5120, 25600), (384, 8192, 16384)):
+        assert ops._lds_update(*size) is not None, size
+    for size in ((1, 3088, 4096), (1, 6144, 12288), (16, 5120, 10176), (257, 3600, 4096), (320, 4096, 4096), (384, 6144, 5056), (385, 3072, 4096),
+                 (769, 3072, 9728), (641, 3600, 9728), (1025, 2560, 9728), (768, 4096, 8192), (257, 8192, 16320)):
+        assert ops._lds_update(*size) is None, size

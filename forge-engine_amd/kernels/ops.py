@@ -697,6 +697,25 @@ IN_PARTS_FEW_ROWS = 2
 MID_IN_PARTS_MAX_WEIGHT_BYTES = 80 << 20   # 17 to 64 rows in parts of K: a larger weight than this is the library's
 
 
+def _lds_in_parts(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
+    """(tile, parts) of q/k/v in parts, or None where another product is the better one.  5 to 16 rows all (8 rows: 4,096 x 1,024
+    4.7 -> 4.2 us, 6,144 x 2,560 8.6 -> 8.4, 4,096 x 4,096 10.8 -> 9.4); up to four rows through a larger weight the kernels for few
+    rows tie or win (6,144 x 1,024 at 1 row 4.9 against 5.4, x 4,096 11.7 against 12.7, 8,192 x 4,096 15.9 against 16.7).  17 to 64
+    rows, weights of up to 52 MB, one round of the chip (6,144 x 2,560 at 64 rows 10.5 -> 9.4, 4,096 x 1,024 6.5 -> 5.8): a second
+    round that is not whole costs as much as a whole one (6,144 x 2,560 in 384 blocks at 17 / 32 rows 10.0 against 10.9, 10.6
+    against 12.6), unless the weight has more rows than the other product for these takes."""
+    few = rows <= SKINNY_MAX_ROWS
+    if few and rows <= FEW_ROWS_IN_PARTS and weight_rows > (4096 if k < 2048 else 5120 if 3072 <= k <= 4096 else 6144):
+        return None
+    if not few and (rows > MID_ROWS or weight_rows * k > 26_000_000):
+        return None
+    tile, parts = lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, 0.15 + rows * weight_rows * 8e-7)
+    blocks = -(-rows // LDS_TILES[tile][0]) * -(-weight_rows // LDS_TILES[tile][1]) * parts
+    if not few and blocks > WIDE_CUS and weight_rows <= WIDE_MAX_WEIGHT_ROWS:
+        return None
+    return tile, parts
+
+
 def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
     """x @ weight^T as float32 partial sums [parts <= 4, M, N] over parts of K, for a consumer that
     adds them up itself (the decode attention kernel that prepares its own queries and keys);
@@ -709,12 +728,9 @@ def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
     rows = x.shape[0]
     if _few_rows_to_library(x, weight):
         return None
-    if (rows <= SKINNY_MAX_ROWS and _lds_fits(x, weight)
-            and (rows > FEW_ROWS_IN_PARTS or weight.shape[0] <= (6144 if weight.shape[1] >= 2048 else 4096))):
-        # (8 rows: 4,096 x 1,024 4.7 -> 4.2 us, 6,144 x 2,560 8.6 -> 8.4, 4,096 x 4,096 10.8 -> 9.4; up to four rows through a
-        # larger weight the kernels below tie or win: 6,144 x 1,024 at 1 row 4.9 against 5.4, 8,192 x 4,096 15.9 against 16.7)
-        tile, parts = lds_plan(rows, weight.shape[0], weight.shape[1], 4 * weight.shape[0], 4, 0.15 + rows * weight.shape[0] * 8e-7)
-        return gemm_lds(x, weight, "parts", parts, tile)
+    plan = _lds_in_parts(rows, *weight.shape) if _lds_fits(x, weight) else None
+    if plan is not None:
+        return gemm_lds(x, weight, "parts", plan[1], plan[0])
     if FEW_ROWS_IN_PARTS < rows <= SKINNY_MAX_ROWS and _wide_fits(x, weight, SKINNY_MAX_ROWS, 1):
         # blocks of 32 weight rows in up to four parts of K (768 blocks for 6144 weight rows): 1 % of the step
         # at 6 to 16 rows against the kernels below (4B, batch 8: 2.74 -> 2.71 ms; 8B: 3.93 -> 3.89)
@@ -722,10 +738,6 @@ def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
         return gemm_wide(x, weight, "parts", parts, row_tile=16, block_rows=32)
     if _skinny_fits(x, weight) and rows <= FEW_ROWS:
         return gemm_skinny(x, weight, "f32", tiles=1, waves=4, splits=IN_PARTS_FEW_ROWS)
-    if rows <= MID_ROWS and _lds_fits(x, weight) and weight.shape[0] * weight.shape[1] <= 26_000_000:
-        # (6144 x 2560 at 64 rows 10.5 -> 9.4 us, 4096 x 1024 6.5 -> 5.8; at 17 rows level)
-        tile, parts = lds_plan(rows, weight.shape[0], weight.shape[1], 4 * weight.shape[0], 4, 0.15 + rows * weight.shape[0] * 8e-7)
-        return gemm_lds(x, weight, "parts", parts, tile)
     if (_mid_fits(x, weight) and weight.shape[0] <= WIDE_MAX_WEIGHT_ROWS
             and weight.shape[0] * weight.shape[1] * weight.element_size() <= MID_IN_PARTS_MAX_WEIGHT_BYTES):
         # (a weight of 10240 rows, K = 5120: 30 us at 32 rows against the library's 26; 7168 rows: 18 against 20;

@@ -243,3 +243,13 @@ def test_which_updates_go_through_lds():
     for size in ((1, 3088, 4096), (1, 6144, 12288), (16, 5120, 10176), (257, 3600, 4096), (320, 4096, 4096), (384, 6144, 5056), (385, 3072, 4096),
                  (769, 3072, 9728), (641, 3600, 9728), (1025, 2560, 9728), (768, 4096, 8192), (257, 8192, 16320)):
         assert ops._lds_update(*size) is None, size
+
+
+def test_which_projections_in_parts_go_through_lds():
+    for size in ((1, 4096, 1024), (4, 6144, 2048), (4, 6144, 2560), (4, 5120, 4096), (4, 6144, 4160), (5, 8192, 4096), (64, 6144, 2560),
+                 (33, 6144, 2560), (17, 4096, 1024), (32, 4096, 2560), (32, 12288, 1024)):
+        plan = ops._lds_in_parts(*size)
+        assert plan is not None and 1 <= plan[1] <= 4, size      # at most what the attention launch adds up
+    for size in ((1, 4112, 1024), (4, 6144, 4096), (4, 5136, 3072), (1, 6160, 2048), (17, 6144, 2560), (32, 6144, 2560), (32, 6144, 2048),
+                 (24, 3072, 5120), (64, 6144, 4288), (65, 4096, 1024)):
+        assert ops._lds_in_parts(*size) is None, size

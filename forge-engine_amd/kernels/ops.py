@@ -558,10 +558,16 @@ def _lds_store_pays(rows: int, weight_rows: int, k: int) -> bool:
     12.8; 4 rows: 2,048 x 2,048 5.2 -> 5.4), 9 to 16 rows always (1,024 x 1,024 3.9 -> 3.7, 6,144 x 2,560 14.7 -> 9.6).
     Beyond, up to 256 rows, 512 through weights of up to 4,096 rows (beyond, the library ties or
     wins: 6,144 x 2,560 at 320 rows 18.6 against 19.9 us), weights of 2,048 rows (1,024: 7.7 against 8.4 us at 192 rows) to
-    50 MB (10,240 x 5,120 at 64 rows 32.6 against 33.9)."""
+    50 MB (10,240 x 5,120 at 64 rows 32.6 against 33.9).  Not through fewer than 3,584 rows at K > 5,120 beyond 192 rows
+    (3,072 x 6,144 at 256 rows 28.8 against 31.4), nor through more at K >= 2,048 and 321 to 384 rows, which fill the library's
+    tiles (4,096 x 2,048 at 384 rows 14.8 against 16.7; at 320 and 448 rows 15.3 -> 14.8 and 17.1 -> 14.9)."""
     if rows <= SKINNY_MAX_ROWS:
         return rows > 8 or (rows > 4 and k >= 2048 and weight_rows <= 8192)
-    return weight_rows >= 2048 and weight_rows * k <= 26_000_000 and rows <= (512 if weight_rows <= 4096 else 256)
+    if weight_rows < 2048 or weight_rows * k > 26_000_000 or rows > (512 if weight_rows <= 4096 else 256):
+        return False
+    if weight_rows >= 3584:
+        return not (320 < rows <= 384 and weight_rows <= 4096 and k >= 2048)
+    return rows <= 192 or k <= 5120
 
 
 def _lds_head_pays(rows: int, weight_rows: int, k: int) -> bool:

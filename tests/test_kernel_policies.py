@@ -253,3 +253,12 @@ def test_which_projections_in_parts_go_through_lds():
     for size in ((1, 4112, 1024), (4, 6144, 4096), (4, 5136, 3072), (1, 6160, 2048), (17, 6144, 2560), (32, 6144, 2560), (32, 6144, 2048),
                  (24, 3072, 5120), (64, 6144, 4288), (65, 4096, 1024)):
         assert ops._lds_in_parts(*size) is None, size
+
+
+def test_which_stored_products_go_through_lds():
+    for size in ((9, 1024, 1024), (5, 8192, 2048), (17, 2048, 1024), (192, 3072, 8192), (256, 6144, 2560), (512, 4096, 1024), (320, 4096, 2048),
+                 (385, 4096, 2048), (384, 3568, 2048), (384, 4096, 1984), (288, 3584, 6144)):
+        assert ops._lds_store_pays(*size), size
+    for size in ((4, 4096, 2048), (8, 8208, 2048), (8, 4096, 1984), (17, 2032, 1024), (193, 3072, 8192), (257, 4112, 1024), (513, 2048, 1024),
+                 (321, 4096, 2048), (384, 3584, 2048), (288, 3568, 6144), (64, 10240, 5120)):
+        assert not ops._lds_store_pays(*size), size

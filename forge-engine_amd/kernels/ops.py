@@ -488,18 +488,27 @@ LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
 
 
-@functools.lru_cache(maxsize=4096)
-def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, consumer_us: float = 0.0) -> tuple[int, int]:
+def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, summed: bool = False) -> tuple[int, int]:
     """(tile, parts of K) for ``gemm_lds``: the least of what a launch is predicted to take.  A block's steps take its CU
     what the table says, the chip reads the weight at 5.4 TB/s (slower with fewer blocks than CUs) and pulls 20 TB/s of
     tiles at best; whichever is slowest bounds the launch.  Fitted to 3,300 launches (25 weights of 1,024 to 17,408 rows,
     17 to 1,024 rows of x, every tile, 1 to 8 parts): the picks take 1 % longer than the best of these tiles.  Up to 16 rows
     the reading rate, the tiles' rate and the cost of a part have values of their own (4,500 launches, 27 weights of 512 to
     34,816 rows, 1 to 16 rows of x: the picks take 2 % longer than the best in parts, 0.3 % whole).
-    ``consumer_us``: what each part costs the consumer that adds them up."""
+    ``summed``: with what each part costs the consumer that adds them up (its reads at 5 TB/s).
+
+    A plan takes 35 (whole) to 190 us (in parts) to find, which a portion of a new length would pay for every weight; a length
+    makes as many tiles as the next multiple of 32, the smallest tile beyond 16 rows, so that is what plans are kept by (one
+    length in 90 gets another plan than its own, by the prediction 1 % longer)."""
+    return _lds_plan(m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32, weight_rows, k, bytes_out, most_parts, summed)
+
+
+@functools.lru_cache(maxsize=4096)
+def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool) -> tuple[int, int]:
     steps = k // 64
     best = None
     few = m <= SKINNY_MAX_ROWS
+    consumer_us = 0.15 + m * weight_rows * 8e-7 if summed else 0.0
     read, alone, pull, store = (1.74e-7, 0.27, 8.8e-8, 1.33e-6) if few else (1.84e-7, 0.35, 4.9e-8, 3.1e-7)
     for tile, (rows, columns, held, one, two) in enumerate(LDS_TILES):
         if few != (rows == 16):
@@ -548,7 +557,7 @@ def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
     if (rows <= 256 or (rows <= 384 and (weight_rows <= 3584 or (weight_rows <= 6144 and k >= 5120)))
             or (long_k and (rows <= 640 or (rows <= 768 and weight_rows <= 3584)
                             or (rows <= 1024 and (weight_rows <= 2560 or k >= 16384))))):
-        return lds_plan(rows, weight_rows, k, 4 * weight_rows, 8, 0.15 + rows * weight_rows * 8e-7)    # (a part's read by the norm: 5 TB/s)
+        return lds_plan(rows, weight_rows, k, 4 * weight_rows, 8, summed=True)
     return None
 
 
@@ -715,7 +724,7 @@ def _lds_in_parts(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None
         return None
     if not few and (rows > MID_ROWS or weight_rows * k > 26_000_000):
         return None
-    tile, parts = lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, 0.15 + rows * weight_rows * 8e-7)
+    tile, parts = lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, summed=True)
     blocks = -(-rows // LDS_TILES[tile][0]) * -(-weight_rows // LDS_TILES[tile][1]) * parts
     if not few and blocks > WIDE_CUS and weight_rows <= WIDE_MAX_WEIGHT_ROWS:
         return None

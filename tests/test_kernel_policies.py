@@ -262,3 +262,16 @@ def test_which_stored_products_go_through_lds():
     for size in ((4, 4096, 2048), (8, 8208, 2048), (8, 4096, 1984), (17, 2032, 1024), (193, 3072, 8192), (257, 4112, 1024), (513, 2048, 1024),
                  (321, 4096, 2048), (384, 3584, 2048), (288, 3568, 6144), (64, 10240, 5120)):
         assert not ops._lds_store_pays(*size), size
+
+
+def test_plans_are_found_once_for_all_lengths_of_as_many_tiles():
+    """Portions of every length up to 1,024: a plan a weight and multiple of 32, the same for all lengths that make these tiles."""
+    before = ops._lds_plan.cache_info().misses
+    plans = {}
+    for rows in range(17, 1025):
+        plan = ops.lds_plan(rows, 2568, 4160, 4 * 2568, 8, summed=True)
+        assert plans.setdefault(-(-rows // 32), plan) == plan
+    assert ops._lds_plan.cache_info().misses - before <= 32
+    for rows in range(1, 17):                                # (few rows: by the count itself)
+        tile, parts = ops.lds_plan(rows, 2568, 4160, 4 * 2568, 8, summed=True)
+        assert ops.LDS_TILES[tile][0] == 16 and 1 <= parts <= 8

@@ -959,6 +959,19 @@ def decode_runs(num_decode: int, num_seqs: int, kv_heads: int, head_dim: int, re
     return decode_splits(num_decode, kv_heads, reach)
 
 
+def _runs_asked_for(splits: int | None, by_length: int | None) -> int | None:
+    """The decode launch's ``splits`` (negative: runs by length) that a caller asks for; None: neither is given."""
+    if by_length is not None:
+        if splits is not None:
+            raise KernelError("splits and by_length exclude each other")
+        if by_length < 1:
+            raise KernelError("by_length must be at least 1")
+        return -by_length
+    if splits is not None and splits < 1:
+        raise KernelError("splits must be at least 1")
+    return splits
+
+
 def _split_scratch(device, num_seqs: int, kv_heads: int, groups: int, head_dim: int, splits: int):
     """The decode kernel's partial outputs and statistics (one set a run of a (sequence, kv head)) and its counters."""
     if splits == 1:
@@ -1015,7 +1028,7 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
     """Attention of every query token of a mixed batch over its paged keys.
 
     ``splits``: key runs of every single token's sequence; ``by_length``: runs by length instead, this many a kv head beyond the
-    sequences; neither: ``decode_runs``.
+    sequences (at most 64 of them); neither: ``decode_runs``.  Both are for the matrix-core decode kernel; another ignores them.
 
     ``chunk`` (a token reads keys of its own run of that many positions only), ``sink``
     (float32 [Hq]: exp(sink_h) joins head h's softmax denominator), ``softcap`` (scores, after
@@ -1107,12 +1120,11 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
               _ptr(part_ml), c_int(tokens), _stream())
 
     if any_single and fast_decode:
-        if splits is None:
+        runs = _runs_asked_for(splits, by_length)
+        if runs is None:
             reach = max_ctx if max_ctx is not None else 16 * 4 * 8
-            reach = reach if chunk is None else min(reach, chunk)
-            splits = -by_length if by_length else decode_runs(num_decode, num_seqs, kv_heads, head_dim, reach)
-        elif splits < 1:
-            raise KernelError("splits must be at least 1")
+            runs = decode_runs(num_decode, num_seqs, kv_heads, head_dim, reach if chunk is None else min(reach, chunk))
+        splits = runs
         part_o, part_ml, counters = _split_scratch(q.device, num_seqs, kv_heads, groups, head_dim, splits)
         mask = (c_int(chunk or 0), _ptr(sink)) + ((_ptr(slopes),) if slopes is not None else ()) if masked else ()
         if dist_bias is not None:
@@ -1237,10 +1249,8 @@ def decode_attention_prepare(qkv: Tensor, q_weight: Tensor | None, k_weight: Ten
     if block_table.dim() != 2 or block_table.stride(1) != 1:
         raise KernelError("block_table must be [sequences, max_blocks] with unit inner stride")
     groups = q_heads // kv_heads
-    if splits is None:
-        splits = -by_length if by_length else decode_runs(num_seqs, num_seqs, kv_heads, head_dim, max_ctx if max_ctx is not None else 16 * 4 * 8)
-    elif splits < 1:
-        raise KernelError("splits must be at least 1")
+    runs = _runs_asked_for(splits, by_length)
+    splits = runs if runs is not None else decode_runs(num_seqs, num_seqs, kv_heads, head_dim, max_ctx if max_ctx is not None else 16 * 4 * 8)
     part_o, part_ml, counters = _split_scratch(qkv.device, num_seqs, kv_heads, groups, head_dim, splits)
     _call("attention_decode", "fe_paged_attention_decode_prepare", _ptr(qkv), c_int(sums),
           c_longlong(num_seqs * width), c_longlong(width), _ptr(q_weight),

@@ -275,3 +275,10 @@ def test_plans_are_found_once_for_all_lengths_of_as_many_tiles():
     for rows in range(1, 17):                                # (few rows: by the count itself)
         tile, parts = ops.lds_plan(rows, 2568, 4160, 4 * 2568, 8, summed=True)
         assert ops.LDS_TILES[tile][0] == 16 and 1 <= parts <= 8
+
+
+def test_key_runs_that_a_caller_asks_for():
+    assert ops._runs_asked_for(None, None) is None and ops._runs_asked_for(3, None) == 3 and ops._runs_asked_for(None, 5) == -5
+    for bad in ((0, None), (-4, None), (None, 0), (None, -4), (2, 4), (2, 0)):
+        with pytest.raises(ops.KernelError):
+            ops._runs_asked_for(*bad)

@@ -1384,7 +1384,8 @@ def test_decode_attention_in_runs_by_length_beside_portions(ops):
             torch.testing.assert_close(other, results[0], atol=2e-3, rtol=2.0 ** -7)
     case = _prepare_case(g, 2, 1, 64, 16, [3] * 65)
     qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq = (t.to(DEV) for t in case[:9])
-    for form in ({"by_length": 4}, {"splits": -4}, {"splits": 0}, {"by_length": 5000}):      # a lane a sequence: 65 are too many
+    for form in ({"by_length": 4}, {"splits": -4}, {"splits": 0}, {"by_length": 5000}, {"by_length": 0}, {"by_length": -4},
+                 {"splits": 2, "by_length": 4}):      # a lane a sequence: 65 are too many
         with pytest.raises(ops.KernelError):
             ops.decode_attention_prepare(qkv, qw, kw, inv_freq, kp, vp, torch.empty(65, 128, dtype=torch.bfloat16, device=DEV), cu, ctx, table,
                                          q_heads=2, kv_heads=1, head_dim=64, eps=1e-6, scale=0.1, max_ctx=64, **form)

@@ -443,6 +443,19 @@ static int launch_tile_f32(const float* A, const float* B, const float* bias, fl
 #define FE_ROWS_F32_MAX 16     // most rows of A that the weight-streaming variant takes
 #define FE_ROWS_F32_RESIDENT_MAX 64   // most rows of A that go through the variant with A in registers, eight at a time
 
+// The tile (1,000 times its rows of A + its rows of B) that a product of more rows than the few-rows variants takes: the one that
+// loads the fullest CU least.  A launch takes as long as the CU with the most tiles, so smaller tiles win where larger ones leave
+// CUs idle or start a round of few blocks; a small tile takes somewhat longer for its area (more bytes from LDS and L2 a product).
+// The factors are fitted to fourteen shapes of 70 to 2,048 rows, where the rule picks the fastest of the three or one within 2 %
+// of it.
+extern "C" int fe_gemm_nt_f32_tile(int M, int N) {
+  auto rounds = [](long long tiles) { return (double)((tiles + 255) / 256); };
+  const long long m64 = (M + 63LL) / 64, m32 = (M + 31LL) / 32, n64 = (N + 63LL) / 64, n32 = (N + 31LL) / 32;
+  const double large = 4.0 * rounds(m64 * n64), half = 2.24 * rounds(m64 * n32), small = 1.22 * rounds(m32 * n32);
+  if (large <= half && large <= small) return 64064;
+  return half <= small ? 64032 : 32032;
+}
+
 extern "C" int fe_gemm_nt_f32(const float* A, const float* B, const float* bias, float* C,
                               int M, int N, int K, long long lda, long long ldb, long long ldc,
                               hipStream_t stream) {
@@ -476,16 +489,11 @@ extern "C" int fe_gemm_nt_f32(const float* A, const float* B, const float* bias,
     return fe_check_launch();
   }
   if (aligned) {
-    // The tile that loads the fullest CU least: a launch takes as long as the CU with the most tiles, so smaller tiles
-    // win where larger ones leave CUs idle or start a round of few blocks; a small tile takes somewhat longer for its
-    // area (more bytes from LDS and L2 a product).  The factors are fitted to fourteen shapes of 70 to 2,048 rows, where
-    // the rule picks the fastest of the three or one within 2 % of it.
-    auto rounds = [](long long tiles) { return (double)((tiles + 255) / 256); };
-    const long long m64 = (M + 63) / 64, m32 = (M + 31) / 32, n64 = (N + 63) / 64, n32 = (N + 31) / 32;
-    const double large = 4.0 * rounds(m64 * n64), half = 2.24 * rounds(m64 * n32), small = 1.22 * rounds(m32 * n32);
-    if (large <= half && large <= small) return launch_tile_f32<2, 2, 2, 2, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
-    if (half <= small) return launch_tile_f32<2, 1, 3, 2, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
-    return launch_tile_f32<1, 1, 4, 4, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
+    switch (fe_gemm_nt_f32_tile(M, N)) {
+      case 64064: return launch_tile_f32<2, 2, 2, 2, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
+      case 64032: return launch_tile_f32<2, 1, 3, 2, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
+      default: return launch_tile_f32<1, 1, 4, 4, 64>(A, B, bias, C, M, N, K, lda, ldb, ldc, stream);
+    }
   }
   const long long grid_y = (M + TILE_M - 1) / TILE_M;
   if (grid_y > 65535) return FE_BAD_ARGUMENT;

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import kernel_refs as refs
+from forge_engine_amd.kernels import library
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -155,9 +156,11 @@ def test_gemm_f32(ops, m, n, k):
             assert torch.equal(part, got[:rows])
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 1, 4), (65, 31, 60), (96, 33, 64), (97, 65, 68), (128, 64, 1024), (129, 4095, 132),   # edges of the tiles, K across a step
-                                   (70, 6145, 260), (250, 2049, 516), (703, 4097, 192)])      # the three tiles, in full and broken rounds
-def test_gemm_f32_tiles(ops, m, n, k):
+@pytest.mark.parametrize("m,n,k,tile", [(65, 1, 4, 32032), (65, 31, 60, 32032), (96, 33, 64, 32032), (97, 65, 68, 32032), (128, 64, 1024, 32032),
+                                        (129, 4095, 132, 32032), (70, 6145, 260, 32032), (250, 2049, 516, 32032),   # edges of the tiles, K across a step,
+                                        (509, 1021, 1028, 64032), (301, 1023, 324, 64032), (449, 1023, 60, 64032),  # the three tiles with K shorter and
+                                        (703, 4097, 192, 64064), (1021, 1023, 1100, 64064)])                        # longer than their stages
+def test_gemm_f32_tiles(ops, m, n, k, tile):
     """More rows than a decode step, on the matrix cores: within the bound that any order of k float32 products and
     sums keeps, |error| <= 2 k 2^-24 sum |a||b|; a row with an infinity spoils itself only; rows with a stride."""
     g = torch.Generator().manual_seed(m * 31 + n)
@@ -170,6 +173,7 @@ def test_gemm_f32_tiles(ops, m, n, k):
     finite[m // 2] = False
     assert bool(((got.double() - want).abs() <= most)[finite].all())
     assert torch.equal(got[m // 2].double(), want[m // 2])        # +-inf, by the sign of b's last number
+    assert library.load("gemm_f32").fe_gemm_nt_f32_tile(m, n) == tile
     again = ops.gemm_nt_f32(a[:, :k], b[:, :k], bias)
     assert torch.equal(got, again)
 

@@ -1347,8 +1347,8 @@ def test_linear_in_parts(ops):
 @pytest.mark.parametrize("count,kv_heads,head_dim,window", [(1, 8, 128, 0), (5, 2, 64, 0), (13, 8, 128, 200), (64, 3, 128, 0), (64, 8, 64, 33), (7, 1, 256, 0)])
 def test_decode_attention_in_runs_by_length(ops, count, kv_heads, head_dim, window, more):
     """Runs that the launch finds from the lengths, against the plain reference: lengths of every size beside one another and
-    equal ones, empty contexts, few and many runs a head, more runs than the first two rounds of the chip; twice on the same
-    counters, the pages with the same bits as with one run."""
+    equal ones, empty contexts, few and many runs a head (more than the chip has CUs or than a round of the merge takes: see
+    the launches in many runs below); twice on the same counters, the pages with the same bits as with one run."""
     g = torch.Generator().manual_seed(count + more)
     contexts = [0, 700, 31, 32, 33, 700, 1, 127, 128, 1500][:count] + torch.randint(0, 400, (max(0, count - 10),), generator=g).tolist()
     qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq, positions, token_seq = _prepare_case(g, 2 * kv_heads, kv_heads, head_dim, 16, contexts)
@@ -1393,6 +1393,59 @@ def test_decode_attention_in_runs_by_length_beside_portions(ops):
         with pytest.raises(ops.KernelError):
             ops.decode_attention_prepare(qkv, qw, kw, inv_freq, kp, vp, torch.empty(65, 128, dtype=torch.bfloat16, device=DEV), cu, ctx, table,
                                          q_heads=2, kv_heads=1, head_dim=64, eps=1e-6, scale=0.1, max_ctx=64, **form)
+
+
+def _runs_by_length(contexts, own, more, window, chunk):
+    """How many runs each sequence is cut into, as the launch finds it: key blocks of 32 that its token reads, over at most
+    max(4, ceil(all / more)) blocks a run."""
+    blocks = []
+    for ctx in contexts:
+        first = max(0, ctx - window) if window else 0
+        if chunk:
+            first = max(first, (ctx - 1) // chunk * chunk)
+        blocks.append(max(-(-(ctx - own) // 32) - first // 32, 0))
+    target = max(-(-sum(blocks) // more), 4)
+    return [max(-(-b // target), 1) for b in blocks]
+
+
+@pytest.mark.parametrize("kv_heads,contexts,more,window,chunk,layers,most", [
+    (8, [200 + 337 * i % 1000 for i in range(64)], 300, None, None, 9, 7),            # beyond the second round of the chip's CUs
+    (8, [6000, 9000, 7001, 8111], 120, None, None, 4, 36),                            # ... and more runs than one round of the merge
+    (2, [6000, 9000, 7001, 8111], 60, None, None, 1, 18), (4, [9000, 700, 1], 64, 5000, None, 1, 40),
+    (4, [7600, 2561, 2560] + [350 * i + 1 for i in range(17)], 200, None, 2560, 4, 20)])
+def test_decode_attention_in_many_runs_by_length(ops, kv_heads, contexts, more, window, chunk, layers, most):
+    """Launches whose runs go past the first (256 / kv_heads blocks a head land on CUs of their own), second and third layer of
+    blocks, and sequences of more runs than the merge takes in one round; against one run a sequence and the plain reference.
+    What a case reaches is counted on the host."""
+    g = torch.Generator().manual_seed(more)
+    n, layer = len(contexts), 256 // kv_heads
+    for own in (1, 0):
+        runs = _runs_by_length(contexts, own, more, window, chunk)
+        assert -(-sum(runs) // layer) >= layers and max(runs) >= most and sum(runs) <= n + more, (sum(runs), layer, max(runs))
+    sizes = dict(q_heads=2 * kv_heads, kv_heads=kv_heads, head_dim=64)
+    qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq, positions, token_seq = _prepare_case(g, 2 * kv_heads, kv_heads, 64, 16, [c - 1 for c in contexts])
+    dev = [t.to(DEV) for t in (qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq)]
+    queries = dev[0][:, :2 * kv_heads * 64].contiguous()
+    results = {}
+    for form in ({"splits": 1}, {"by_length": more}):
+        out = torch.full((n, 2 * kv_heads * 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.paged_attention(queries, dev[1], dev[2], out, dev[3], dev[4], dev[5], num_seqs=n, max_q_len=1, num_decode=n, scale=0.1, window=window,
+                            chunk=chunk, max_ctx=max(contexts), **form, **sizes)
+        results["finished", len(results)] = out
+        if chunk is None:
+            out = torch.full((n, 2 * kv_heads * 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+            ops.decode_attention_prepare(dev[0], dev[6], dev[7], dev[8], dev[1], dev[2], out, dev[3], dev[4], dev[5], eps=1e-6, scale=0.1,
+                                         window=window, max_ctx=max(contexts), **form, **sizes)
+            results["prepared", len(results)] = out
+            dev[1], dev[2] = kp.to(DEV), vp.to(DEV)          # (the launch wrote the new keys and values)
+    outs = [out.cpu().float() for out in results.values()]
+    per = len(outs) // 2
+    for one, many in zip(outs[:per], outs[per:]):
+        torch.testing.assert_close(many, one, atol=2e-3, rtol=2.0 ** -7)          # float32 sums in another order, one rounding each
+    if chunk is None:
+        want = refs.paged_attention(queries.cpu(), kp, vp, torch.empty(n, 2 * kv_heads * 64, dtype=qkv.dtype), cu, ctx, table, num_seqs=n,
+                                    max_q_len=1, scale=0.1, window=window, **sizes)
+        torch.testing.assert_close(outs[per], want.float(), atol=2e-2, rtol=2e-2)
 
 
 def test_which_decode_launches_take_runs_by_length(ops):

@@ -40,6 +40,7 @@ typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
 #define WAVES 4
 #define GMAX 8           // largest group size served
 #define SLOT_LAYER 256   // CUs: blocks that land on a CU of their own
+#define RUN_LEAST 12     // runs by length: fewest key blocks that a sequence is cut into runs of
 
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 __device__ __forceinline__ unsigned int pack_bf16(float lo, float hi) {
@@ -124,8 +125,9 @@ __device__ __forceinline__ KeyRange key_range(int ctx, int cached, int window, i
 }
 
 // Runs by length (launches of up to 64 sequences): every wave finds its block's run from the lengths, one sequence a lane.
-// A sequence is cut into equal runs of at most max(4, ceil(all key blocks / more)) key blocks, so a launch of num_seqs + more
-// blocks a head has one for each; the runs are handed out longest first, which the order of the blocks then balances: the first
+// A sequence is cut into equal runs of at most max(RUN_LEAST, ceil(all key blocks / more)) key blocks, so a launch of num_seqs + more
+// blocks a head has one for each (a run's start and its part in the merge cost about as much as RUN_LEAST blocks of keys: with
+// runs of down to 4 blocks 32 sequences of 20 to 200 keys took 13.4 us, whole 9.0; 4 of 1,000 to 8,000 16.9 against 16.1); the runs are handed out longest first, which the order of the blocks then balances: the first
 // `layer` blocks of a head land on CUs of their own, the next `layer` beside them, shortest first, what is left goes to
 // the slots that come free first.
 struct Run {
@@ -141,7 +143,7 @@ __device__ __forceinline__ bool find_run(const int* cu_q, const int* ctx_len, in
   const bool mine = lane < num_seqs && q1 - q0 == 1;
   const KeyRange range = key_range(ctx, ctx - own, window, chunk);
   const int blocks = mine ? max(range.last - range.first, 0) : 0;
-  const int target = max((wave_sum_int(blocks) + more - 1) / more, WAVES);
+  const int target = max((wave_sum_int(blocks) + more - 1) / more, RUN_LEAST);
   const int runs = mine ? max((blocks + target - 1) / target, 1) : 0;
   const int size = mine ? (blocks + runs - 1) / runs : -1;
   const int key = size * 64 + lane;

@@ -940,21 +940,28 @@ def _split_counters(device, count: int) -> Tensor:
 
 DECODE_SLOTS = 512             # blocks of the decode kernel that the chip holds at a time (heads up to 128), two a CU
 RUNS_BY_LENGTH_MIN_SEQUENCES = 12
+RUNS_BY_LENGTH_MIN_REACH = 2048
 RUNS_BY_LENGTH_LONG = 8192
 
 
 def decode_runs(num_decode: int, num_seqs: int, kv_heads: int, head_dim: int, reach: int) -> int:
     """The decode launch's ``splits``: ``decode_splits``, or -E for runs by length.  With as many runs for every sequence the
     launch lasts as long as its longest run, and that depends on where the long ones land; runs by length, found on the
-    device, cut a sequence into runs of at most (all key blocks / E) and order them so that CUs share the keys evenly.
-    Measured at 8 kv heads of 128 (us, splits -> by length): 64 sequences of 130 to 2,000 keys, shuffled 52.4 -> 41.5, falling
-    43.1 -> 41.0, 48: 35.4 -> 29.7, 32: 30.2 -> 23.8, 16: 21.1 -> 17.5, 4 of 6,000 to 16,000 39.7 -> 37.0.  What finding the
-    runs costs shows where lengths are equal (64 of 706 keys 34.8 -> 35.6) and where a launch is latency alone (8 of 200 to
-    1,900 14.9 -> 15.2, 1 of 217 8.3 -> 9.3), so: from twelve sequences, or from three where contexts may be long.  E keeps
-    the runs (about half a run a sequence more than the keys need) within the slots that the chip has at a time: a third
-    round of a few blocks cost 29.9 -> 32.7 at 48 sequences."""
-    if (num_seqs <= 64 and head_dim <= 128 and num_seqs * kv_heads <= DECODE_SLOTS
-            and num_decode >= (3 if reach >= RUNS_BY_LENGTH_LONG else RUNS_BY_LENGTH_MIN_SEQUENCES) and num_decode * kv_heads >= 24):
+    device, cut a sequence into runs of at most (all key blocks / E), and no fewer than 12, and order them so that CUs share the
+    keys evenly.
+    Measured at 32 query heads on 8 kv heads of 128 (us, splits -> by length; lengths drawn from a tenth of the longest up, one long
+    one beside others of an eighth, all the longest): up to 2,000 keys 12 sequences 18.2 -> 18.2, 15.9 -> 11.9, 26.8 -> 22.9, 32: 30.1
+    -> 29.3, 25.7 -> 16.3, 42.8 -> 46.1, 64: 59.7 -> 49.6, 30.4 -> 22.2, 98.6 -> 95.2; 4 of up to 16,000 29.5 -> 27.6.  What finding
+    the runs costs, 0.9 us, shows where contexts are short (32 of 1,000 24.4 against 26.8, of 20 to 200 9.0 against 10.1) and where
+    a launch is latency alone (1 of 217 8.3 against 9.3), and with few blocks equal splits are as short (2 kv heads, 16 of 200 to
+    2,000 10.4 against 12.2), so: from twelve sequences and 40 (sequence, kv head) pairs where contexts may reach 2,048, from three
+    and 24 where they may reach 8,192.
+    E keeps the runs (about half a run a sequence more than the keys need) within the slots that the chip has at a time: a
+    third round of a few blocks cost 29.9 -> 32.7 at 48 sequences."""
+    blocks = num_decode * kv_heads
+    long = reach >= RUNS_BY_LENGTH_LONG and num_decode >= 3 and blocks >= 24
+    many = reach >= RUNS_BY_LENGTH_MIN_REACH and num_decode >= RUNS_BY_LENGTH_MIN_SEQUENCES and blocks >= 40
+    if num_seqs <= 64 and head_dim <= 128 and num_seqs * kv_heads <= DECODE_SLOTS and (long or many):
         return -max(1, DECODE_SLOTS // kv_heads - 2 * num_decode // 3)
     return decode_splits(num_decode, kv_heads, reach)
 

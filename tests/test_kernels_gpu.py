@@ -1397,22 +1397,22 @@ def test_decode_attention_in_runs_by_length_beside_portions(ops):
 
 def _runs_by_length(contexts, own, more, window, chunk):
     """How many runs each sequence is cut into, as the launch finds it: key blocks of 32 that its token reads, over at most
-    max(4, ceil(all / more)) blocks a run."""
+    max(12, ceil(all / more)) blocks a run."""
     blocks = []
     for ctx in contexts:
         first = max(0, ctx - window) if window else 0
         if chunk:
             first = max(first, (ctx - 1) // chunk * chunk)
         blocks.append(max(-(-(ctx - own) // 32) - first // 32, 0))
-    target = max(-(-sum(blocks) // more), 4)
+    target = max(-(-sum(blocks) // more), 12)
     return [max(-(-b // target), 1) for b in blocks]
 
 
 @pytest.mark.parametrize("kv_heads,contexts,more,window,chunk,layers,most", [
-    (8, [200 + 337 * i % 1000 for i in range(64)], 300, None, None, 9, 7),            # beyond the second round of the chip's CUs
-    (8, [6000, 9000, 7001, 8111], 120, None, None, 4, 36),                            # ... and more runs than one round of the merge
-    (2, [6000, 9000, 7001, 8111], 60, None, None, 1, 18), (4, [9000, 700, 1], 64, 5000, None, 1, 40),
-    (4, [7600, 2561, 2560] + [350 * i + 1 for i in range(17)], 200, None, 2560, 4, 20)])
+    (8, [200 + 337 * i % 1000 for i in range(64)], 300, None, None, 5, 3),            # beyond the second round of the chip's CUs
+    (8, [6000, 9000, 7001, 8111], 120, None, None, 3, 24),                            # ... and more runs than one round of the merge
+    (2, [6000, 9000, 7001, 8111], 60, None, None, 1, 18), (4, [9000, 700, 1], 64, 7000, None, 1, 19),
+    (4, [16000, 2561, 2560] + [350 * i + 1 for i in range(27)], 400, None, 8192, 4, 20)])
 def test_decode_attention_in_many_runs_by_length(ops, kv_heads, contexts, more, window, chunk, layers, most):
     """Launches whose runs go past the first (256 / kv_heads blocks a head land on CUs of their own), second and third layer of
     blocks, and sequences of more runs than the merge takes in one round; against one run a sequence and the plain reference.
@@ -1449,9 +1449,9 @@ def test_decode_attention_in_many_runs_by_length(ops, kv_heads, contexts, more, 
 
 
 def test_which_decode_launches_take_runs_by_length(ops):
-    assert ops.decode_runs(64, 64, 8, 128, 2048) == -22 and ops.decode_runs(12, 12, 8, 64, 1024) == -56
-    assert ops.decode_runs(3, 3, 8, 128, 8192) == -62 and ops.decode_runs(12, 20, 2, 128, 512) == -248
-    for other in ((11, 11, 8, 128, 2048), (2, 2, 8, 128, 8192), (3, 3, 4, 128, 8192), (64, 65, 8, 128, 2048), (64, 64, 9, 128, 2048), (32, 32, 8, 256, 2048)):
+    assert ops.decode_runs(64, 64, 8, 128, 2048) == -22 and ops.decode_runs(12, 12, 8, 64, 2048) == -56
+    assert ops.decode_runs(3, 3, 8, 128, 8192) == -62 and ops.decode_runs(20, 20, 2, 128, 2048) == -243 and ops.decode_runs(12, 20, 2, 128, 8192) == -248
+    for other in ((11, 11, 8, 128, 2048), (12, 12, 8, 64, 1024), (64, 64, 8, 128, 2047), (12, 20, 2, 128, 2048), (11, 11, 2, 128, 8192), (2, 2, 8, 128, 8192), (3, 3, 4, 128, 8192), (64, 65, 8, 128, 2048), (64, 64, 9, 128, 2048), (32, 32, 8, 256, 2048)):
         assert ops.decode_runs(*other) == ops.decode_splits(other[0], other[2], other[4])
 
 

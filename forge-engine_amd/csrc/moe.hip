@@ -21,6 +21,7 @@
 // rows a tile + experts); a block whose slot lies beyond the tiles there are returns at once.
 #include "common.h"
 #include "lds_tile.h"
+#include <algorithm>
 
 // One thread per token over its row of router logits z [T, E] (float32, the product comes from the
 // caller): bias added, the `top` largest chosen one after the other (the largest first; among equals
@@ -473,17 +474,39 @@ static int launch_moe_tile(const bf16_t* a, const bf16_t* w, const int* offsets,
 // 93 -> 64, 98 -> 77, 228 -> 141, 379 -> 270; width 1,024 25 -> 18, 27 -> 19, 28 -> 22, 30 -> 23, 35 -> 27, 73 -> 63, 132 -> 100.
 // At 300 tokens (75 rows an expert) 64 x 64 takes 27 and 77 us, 64 x 128 31 and 72, 32 x 64 32 and 89; at 1,500 (375 rows)
 // 64 x 128 61 and 165, 128 x 128 76 and 199, 256 x 128 63 and 141.
+// The largest tile also wants steps enough for its start (its three buffers filled, 256 gathered rows) and blocks for most of the
+// CUs: 1,024 x 3,072 of 4 experts at 1,100 tokens, 240 blocks, gate/up 59 us in 256 x 128 against 39 in 64 x 128; 512 x 1,536 at 2,048
+// tokens 49 against 30; 2,048 x 2,048 down at 1,500 tokens 41 in the large tile against 53.  And where the smaller tile's blocks
+// still leave half the chip idle it is the faster one at any number of rows: 64 x 64 of 4 experts at 400 tokens 6.3 us in 32 x 64, 8.0
+// in 64 x 64, 11.3 in 64 x 128.  (Over 1,995 sizes of both products against the kernels before: 1.38 times as fast; at widths of
+// 256 and 512 with many tokens those were up to a quarter faster.)
+// Returned: 1,000 times the tile's rows + its weight rows.  gated: gate and up rows share a tile's weight rows (MODE 0).
+extern "C" int fe_moe_tile(int gated, int tokens, int top, int experts, int N, int K) {
+  const long long pairs = (long long)tokens * top, each = pairs / experts;
+  // blocks that have work, if the experts share the pairs evenly
+  auto busy = [&](int rows, int weight_rows) {
+    const int columns = gated ? weight_rows / 2 : weight_rows;
+    return (pairs + (long long)rows * experts - 1) / ((long long)rows * experts) * std::min((long long)experts, pairs) * ((N + columns - 1) / columns);
+  };
+  const int half_the_chip = 128;
+  if (each >= 256 && K >= (gated ? 2048 : 768) && busy(256, 128) >= 160) return 256128;
+  if (each > 96 && busy(64, 64) > half_the_chip) return 64128;
+  if (each > 32 && busy(32, 64) > half_the_chip) return 64064;
+  return 32064;
+}
+
 template <int MODE>
 static int launch_moe(const bf16_t* a, const bf16_t* w, const int* offsets, const int* order, const float* pair_weight,
                       bf16_t* act, float* out, int experts, int N, int K, int top, int tokens, float limit, float alpha,
                       int form, const float* extra, int extra_parts, hipStream_t stream) {
-  const long long each = (long long)tokens * top / experts;
 #define FE_GO(...) return launch_moe_tile<__VA_ARGS__, MODE>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens, \
                                                              limit, alpha, form, extra, extra_parts, stream)
-  if (each <= 32) FE_GO(1, 2, 2, 2, 2, 6);       // 32 x 64
-  if (each <= 96) FE_GO(2, 2, 2, 2, 2, 4);       // 64 x 64
-  if (each < 256) FE_GO(2, 4, 2, 2, 2, 3);       // 64 x 128
-  FE_GO(4, 4, 4, 2, 1, 3);                       // 256 x 128
+  switch (fe_moe_tile(MODE == 0, tokens, top, experts, N, K)) {
+    case 256128: FE_GO(4, 4, 4, 2, 1, 3);
+    case 64128: FE_GO(2, 4, 2, 2, 2, 3);
+    case 64064: FE_GO(2, 2, 2, 2, 2, 4);
+    default: FE_GO(1, 2, 2, 2, 2, 6);       // 32 x 64
+  }
 #undef FE_GO
 }
 

@@ -174,7 +174,10 @@ def test_mixture_of_experts_kernels(tokens, hidden, experts, top, inner, dtype):
     (3, 96, 130, 2, 33), (40, 128, 70, 3, 100),                 # more experts than a wave has lanes, few rows each
     (65, 160, 2, 1, 70), (150, 64, 3, 2, 130),                  # 32 to 100 rows an expert
     (190, 224, 2, 2, 129), (300, 96, 1, 1, 260),                # 190 and 300: the wider tiles
-    (1030, 192, 4, 1, 34)])
+    (1030, 192, 4, 1, 34),
+    (130, 1440, 3, 1, 2080), (130, 1440, 3, 1, 2083), (130, 1441, 3, 1, 2080),      # blocks enough for 64 x 64
+    (300, 1440, 2, 1, 736), (300, 1440, 2, 1, 739), (300, 1441, 2, 1, 736),         # ... for 64 x 128
+    (1300, 5152, 4, 1, 1312), (1300, 5152, 4, 1, 1315), (1300, 5153, 4, 1, 1312)])  # ... and steps enough for 256 x 128
 @pytest.mark.parametrize("weight_input", [False, True])
 def test_grouped_products_tiles(tokens, hidden, experts, top, inner, weight_input):
     """Every tile of the grouped products, rows and columns beside its edges, K ending in half a step, some experts without
@@ -206,6 +209,21 @@ def test_grouped_products_tiles(tokens, hidden, experts, top, inner, weight_inpu
     # the middle may round the other way where a float32 sum lies beside a tie: 2^-8 of one of `inner` terms of size inner^-0.5 each
     torch.testing.assert_close(got.double(), want, atol=2e-2, rtol=1e-3)
     assert float((got.double() - want).norm() / want.norm()) < 1e-3
+
+
+def test_which_tile_a_grouped_product_takes():
+    """Both sides of every line: rows an expert, blocks, steps, for the gated product and the other; and that the sizes above
+    reach every tile."""
+    from forge_engine_amd.kernels import library
+    tile = library.load("moe").fe_moe_tile
+    for gated, tokens, top, experts, n, k, want in (
+            (1, 130, 1, 3, 2080, 1440, 64064), (0, 130, 1, 3, 1440, 2080, 64064), (1, 300, 1, 2, 736, 1440, 64128), (0, 300, 1, 2, 1440, 736, 64128),
+            (1, 1300, 1, 4, 1312, 5152, 256128), (0, 1300, 1, 4, 5152, 1312, 256128),
+            (1, 32, 1, 1, 65536, 2048, 32064), (1, 33, 1, 1, 65536, 2048, 64064), (1, 96, 1, 1, 65536, 2048, 64064), (1, 97, 1, 1, 65536, 2048, 64128),
+            (1, 255, 1, 1, 65536, 2048, 64128), (1, 256, 1, 1, 65536, 2048, 256128), (1, 256, 1, 1, 65536, 2016, 64128), (0, 256, 1, 1, 65536, 736, 64128),
+            (0, 256, 1, 1, 65536, 768, 256128), (0, 256, 1, 1, 20352, 768, 64128), (0, 256, 1, 1, 20353, 768, 256128),
+            (0, 128, 1, 1, 4096, 768, 64064), (0, 64, 1, 1, 4096, 768, 32064), (0, 64, 1, 1, 4097, 768, 64064), (0, 128, 1, 1, 4097, 768, 64128), (1, 400, 1, 4, 64, 64, 32064)):
+        assert tile(gated, tokens, top, experts, n, k) == want, (gated, tokens, top, experts, n, k)
 
 
 # ------------------------------------------------------------------ the model

@@ -9,6 +9,7 @@
 #define ROW_THREADS 256
 #define ROW_THREADS_FEW 1024   // threads a row when a step has few rows (measured faster up to some hundred rows)
 #define FEW_ROWS 512
+#define CUS 256
 static inline int row_threads(int rows, int width) { return rows <= FEW_ROWS && width >= 1024 ? ROW_THREADS_FEW : ROW_THREADS; }
 
 // ---------------------------------------------------------------- token shift
@@ -86,23 +87,23 @@ __device__ __forceinline__ float parts_sum(const float* p, int parts, size_t par
 }
 
 // Elements c = threadIdx.x + j * blockDim.x of a row in parts, each the sum of its parts in order, zeros beyond the row.  The loads
-// of four parts and all elements are issued before any is used, none under a condition (an index beyond the row or the parts
+// of P parts and all elements are issued before any is used, none under a condition (an index beyond the row or the parts
 // reads the last one again): at a few rows these kernels take what their chain of dependent loads takes.  The sums are those
 // of parts_sum, bit for bit.
-template <int N>
+template <int N, int P>
 __device__ __forceinline__ void held_row(const float* __restrict__ row, int parts, size_t part_stride, int width, float (&u)[N]) {
-  for (int from = 0; from < parts; from += 4) {
-    float v[N][4];
+  for (int from = 0; from < parts; from += P) {
+    float v[N][P];
 #pragma unroll
     for (int j = 0; j < N; ++j)
 #pragma unroll
-      for (int p = 0; p < 4; ++p)
+      for (int p = 0; p < P; ++p)
         v[j][p] = row[min((int)(threadIdx.x + j * blockDim.x), width - 1) + min(from + p, parts - 1) * part_stride];
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       u[j] = from == 0 ? v[j][0] : u[j] + v[j][0];
 #pragma unroll
-      for (int p = 1; p < 4; ++p) u[j] = from + p < parts ? u[j] + v[j][p] : u[j];
+      for (int p = 1; p < P; ++p) u[j] = from + p < parts ? u[j] + v[j][p] : u[j];
     }
   }
 #pragma unroll
@@ -119,8 +120,10 @@ static inline int held_elements(int width, int threads) {
 // h[r] += u * rsqrt(mean(u^2) + eps) * w, u = the sum of the update's parts; out (if any) = new h.
 // A row of up to 8 elements a thread (N) stays in registers between the two passes, with the stream's and the weight's
 // elements, which are asked for beside the update's; wider rows (N = 0) are read again.  6 rows of 2,048 in 4 parts: a launch of
-// 6.2 us with loads under conditions, part after part.
-template <typename TO, bool HAS_OUT, int N>
+// 6.2 us with loads under conditions, part after part.  P: parts asked for at a time.  One where there is one (four times the
+// last one cost 6.3 -> 8.5 us at 512 rows of 6,144), and at eight elements a thread with more rows than CUs, where the
+// registers of four leave room for one block a CU.
+template <typename TO, bool HAS_OUT, int N, int P>
 __global__ __launch_bounds__(ROW_THREADS_FEW) void rmsnorm_update_kernel(
     float* __restrict__ h, const float* __restrict__ update, int parts, size_t part_stride,
     const float* __restrict__ w, float eps, TO* __restrict__ out, int width) {
@@ -136,7 +139,7 @@ __global__ __launch_bounds__(ROW_THREADS_FEW) void rmsnorm_update_kernel(
       before[j] = h[base + c];
       weight[j] = w[c];
     }
-    held_row<N>(update + base, parts, part_stride, width, u);
+    held_row<N, P>(update + base, parts, part_stride, width, u);
 #pragma unroll
     for (int j = 0; j < N; ++j) ss += u[j] * u[j];
     ss = block_sum<true>(ss, scratch);
@@ -170,21 +173,25 @@ extern "C" int fe_rmsnorm_update(float* h, const float* update, int parts, long 
   if (rows <= 0) return FE_OK;
   if (width <= 0 || parts < 1 || parts > 64 || !(eps > 0.f)) return FE_BAD_ARGUMENT;
   const int threads = row_threads(rows, width);
-#define LAUNCH(TO, HAS_OUT, N) \
-  rmsnorm_update_kernel<TO, HAS_OUT, N><<<rows, threads, 0, stream>>>(h, update, parts, (size_t)part_stride, w, eps, (TO*)out, width)
+  const int held = held_elements(width, threads);
+  const bool by_one = parts == 1 || (held == 8 && rows > CUS);
+#define LAUNCH(TO, HAS_OUT, N, P) \
+  rmsnorm_update_kernel<TO, HAS_OUT, N, P><<<rows, threads, 0, stream>>>(h, update, parts, (size_t)part_stride, w, eps, (TO*)out, width)
+#define LAUNCH_PARTS(TO, HAS_OUT, N) if (by_one) LAUNCH(TO, HAS_OUT, N, 1); else LAUNCH(TO, HAS_OUT, N, 4)
 #define LAUNCH_HELD(TO, HAS_OUT)                       \
-  switch (held_elements(width, threads)) {             \
-    case 1: LAUNCH(TO, HAS_OUT, 1); break;             \
-    case 2: LAUNCH(TO, HAS_OUT, 2); break;             \
-    case 4: LAUNCH(TO, HAS_OUT, 4); break;             \
-    case 8: LAUNCH(TO, HAS_OUT, 8); break;             \
-    default: LAUNCH(TO, HAS_OUT, 0);                   \
+  switch (held) {                                      \
+    case 1: LAUNCH_PARTS(TO, HAS_OUT, 1); break;       \
+    case 2: LAUNCH_PARTS(TO, HAS_OUT, 2); break;       \
+    case 4: LAUNCH_PARTS(TO, HAS_OUT, 4); break;       \
+    case 8: LAUNCH_PARTS(TO, HAS_OUT, 8); break;       \
+    default: LAUNCH(TO, HAS_OUT, 0, 1);                \
   }
   if (out == nullptr || out_dtype < 0) { LAUNCH_HELD(float, false); }
   else if (out_dtype == FE_F32) { LAUNCH_HELD(float, true); }
   else if (out_dtype == FE_BF16) { LAUNCH_HELD(bf16_t, true); }
   else return FE_BAD_ARGUMENT;
 #undef LAUNCH_HELD
+#undef LAUNCH_PARTS
 #undef LAUNCH
   return fe_check_launch();
 }
@@ -394,7 +401,7 @@ __global__ __launch_bounds__(ROW_THREADS_FEW) void rmsnorm_mean_kernel(MeanInput
         weight[b][j] = w[(size_t)min(b, count - 1) * width + min((int)(threadIdx.x + j * blockDim.x), width - 1)];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
-      if (b < count) held_row<N>(in.u[b] + base, in.parts[b], part_stride, width, u[b]);
+      if (b < count) held_row<N, 4>(in.u[b] + base, in.parts[b], part_stride, width, u[b]);
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       if (b >= count) break;

@@ -488,23 +488,25 @@ LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
 
 
-def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, summed: bool = False) -> tuple[int, int]:
+def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, summed: bool = False,
+             one_round: bool = False) -> tuple[int, int]:
     """(tile, parts of K) for ``gemm_lds``: the least of what a launch is predicted to take.  A block's steps take its CU
     what the table says, the chip reads the weight at 5.4 TB/s (slower with fewer blocks than CUs) and pulls 20 TB/s of
     tiles at best; whichever is slowest bounds the launch.  Fitted to 3,300 launches (25 weights of 1,024 to 17,408 rows,
     17 to 1,024 rows of x, every tile, 1 to 8 parts): the picks take 1 % longer than the best of these tiles.  Up to 16 rows
     the reading rate, the tiles' rate and the cost of a part have values of their own (4,500 launches, 27 weights of 512 to
     34,816 rows, 1 to 16 rows of x: the picks take 2 % longer than the best in parts, 0.3 % whole).
-    ``summed``: with what each part costs the consumer that adds them up (its reads at 5 TB/s).
+    ``summed``: with what each part costs the consumer that adds them up (its reads at 5 TB/s).  ``one_round``: at most a block a CU
+    (the prediction is kind to a second round that is not whole).
 
     A plan takes 35 (whole) to 190 us (in parts) to find, which a portion of a new length would pay for every weight; a length
     makes as many tiles as the next multiple of 32, the smallest tile beyond 16 rows, so that is what plans are kept by (one
     length in 90 gets another plan than its own, by the prediction 1 % longer)."""
-    return _lds_plan(m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32, weight_rows, k, bytes_out, most_parts, summed)
+    return _lds_plan(m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32, weight_rows, k, bytes_out, most_parts, summed, one_round)
 
 
 @functools.lru_cache(maxsize=4096)
-def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool) -> tuple[int, int]:
+def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool, one_round: bool) -> tuple[int, int]:
     steps = k // 64
     best = None
     few = m <= SKINNY_MAX_ROWS
@@ -515,6 +517,8 @@ def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int,
             continue
         for parts in range(1, max(1, min(most_parts, steps // 4)) + 1):
             tiles = -(-m // rows) * -(-weight_rows // columns) * parts
+            if one_round and tiles > 256:
+                continue
             rounds = -(-tiles // 256)
             step = one * rounds if held == 1 or rounds == 1 else two * -(-rounds // 2)
             part_steps = -(-steps // parts)
@@ -533,6 +537,14 @@ def _lds_fits(x: Tensor, weight: Tensor) -> bool:
             and weight.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
+def _library_fits(weight_rows: int, k: int) -> bool:
+    """Whether the matrix library's tiles fit a weight whole.  Others cost it up to half again, and the lines below, drawn beside
+    it at sizes like those of models (multiples of 256), do not hold for them (us, library against the product through LDS: stored
+    3,864 x 3,008 at 329 rows 29.5 against 18.0; an update of 6,320 x 3,136 at 271 rows 37.9 against 31.8; gate/up of 960 columns,
+    K = 2,880, at 983 rows 30.2 against 21.7)."""
+    return weight_rows % 256 == 0 and k % 256 == 0
+
+
 def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
     """(tile, parts) of a float32 update, or None where another product is the better one.  Up to 16 rows: weights of up to
     3,072 rows (1,024 x 3,072 at 1 row 5.8 -> 3.7 us, 2,560 x 4,096 at 8 rows 7.0 -> 6.6) and others of up to 5,120 whose K is at
@@ -540,13 +552,14 @@ def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
     below tie or win (4,096 x 4,096 at 1 row 8.5 against 9.4, 8,192 x 4,096 15.0 against 16.7).  Up to 64 rows: weights of up to
     2,048 x 4,096 by the plan (1,024 x 2,048 at 64 rows 6.5 -> 4.9 us), larger ones in the parts that fill the chip with
     blocks of 64 weight rows (2,560 x 9,728 14.6 -> 12.9, 4,096 x 12,288 25.9 -> 23.4, at 32 rows 13.1 -> 11.6 and 22.8 ->
-    20.9).  Up to 256 rows all by the plan.  To 384 rows, beside the matrix library that adds into the stream: weights of up to 3,584
-    rows (320 rows: 3,072 x 4,096 33.7 -> 25.9), to 6,144 from K = 5,120 on (5,120 x 8,192 53.8 -> 46.4; but 4,096 x 4,096 29.9
-    against 32.4, 8,192 x 4,096 42.0 against 53.6), and from twice their rows on.  These last, which the library cuts into too few
-    blocks, also to 640 rows (512 rows: 2,560 x 9,728 55.5 -> 44.1, 5,120 x 17,408 175 -> 107), to 768 through up to 3,584 rows (3,072 x
-    9,728 1.24 times as fast; 4,096 x 8,192 70.5 against 78.2) and to 1,024 through up to 2,560 or from K = 16,384 on (1,024 rows:
-    2,560 x 9,728 85.5 -> 65.3, 5,120 x 25,600 352 -> 283; but 3,072 x 9,728 83.9 against 98.1).  (The times hold the norm that
-    adds the parts.)"""
+    20.9).  Up to 256 rows all of up to 8,192 rows, or half their K, by the plan (11,136 x 2,496 at 149 rows .86 of the library's
+    speed).  To 384 rows, beside the matrix library that adds into the stream: weights of up to 3,584 rows (320 rows: 3,072 x 4,096
+    33.7 -> 25.9), to 6,144 from K = 5,120 on (5,120 x 8,192 53.8 -> 46.4; but 4,096 x 4,096 29.9 against 32.4, 8,192 x 4,096 42.0
+    against 53.6), and those whose K is at least twice their rows.  These last, which the library cuts into too few blocks, also
+    to 640 rows (512 rows: 2,560 x 9,728 55.5 -> 44.1, 5,120 x 17,408 175 -> 107), to 768 through up to 3,584 rows (3,072 x 9,728
+    1.24 times as fast; 4,096 x 8,192 70.5 against 78.2) and to 1,024 through up to 2,560 or from K = 16,384 on (1,024 rows: 2,560 x
+    9,728 85.5 -> 65.3, 5,120 x 25,600 352 -> 283; but 3,072 x 9,728 83.9 against 98.1).  (The times hold the norm that adds the
+    parts.)"""
     long_k = k >= 2 * weight_rows
     if rows <= SKINNY_MAX_ROWS and not (weight_rows <= 3072 or (long_k and weight_rows <= 5120)):
         return None
@@ -554,7 +567,9 @@ def _lds_update(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None:
         if weight_rows > WIDE_MAX_WEIGHT_ROWS:
             return None
         return (8 if rows <= 32 else 2), _wide_parts(rows, weight_rows, k)
-    if (rows <= 256 or (rows <= 384 and (weight_rows <= 3584 or (weight_rows <= 6144 and k >= 5120)))
+    if weight_rows > WIDE_MAX_WEIGHT_ROWS and not long_k:
+        return None
+    if (rows <= 256 or (rows <= 384 and (weight_rows <= 3584 or (weight_rows <= 6144 and k >= 5120) or not _library_fits(weight_rows, k)))
             or (long_k and (rows <= 640 or (rows <= 768 and weight_rows <= 3584)
                             or (rows <= 1024 and (weight_rows <= 2560 or k >= 16384))))):
         return lds_plan(rows, weight_rows, k, 4 * weight_rows, 8, summed=True)
@@ -574,6 +589,8 @@ def _lds_store_pays(rows: int, weight_rows: int, k: int) -> bool:
         return rows > 8 or (rows > 4 and k >= 2048 and weight_rows <= 8192)
     if weight_rows < 2048 or weight_rows * k > 26_000_000 or rows > (512 if weight_rows <= 4096 else 256):
         return False
+    if not _library_fits(weight_rows, k):
+        return True
     if weight_rows >= 3584:
         return not (320 < rows <= 384 and weight_rows <= 4096 and k >= 2048)
     return rows <= 192 or k <= 5120
@@ -616,13 +633,13 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     if rows <= SKINNY_MAX_ROWS:
         if GATE_HALF_FEW_ROWS_MAX_K < k <= 4096 and columns >= 4096 and (rows <= 4 or columns > 12288):
             return False
-        return blocks <= WIDE_CUS or blocks > 1.6 * WIDE_CUS
+        return LDS_TILES[tile][2] == 2 or blocks <= WIDE_CUS or blocks > 1.6 * WIDE_CUS      # (a CU holds one block of the widest tile)
     large_tiles = -(-rows // 128) * -(-weight_rows // 160)
     if rows > LDS_GATE_MAX_ROWS or large_tiles > WIDE_CUS:
         return False
     if rows <= MID_ROWS:
         return blocks <= WIDE_CUS or (k >= 8192 and columns >= 8192)
-    if k <= 2048:
+    if k <= 2048 or not _library_fits(weight_rows, k):
         return True
     if rows <= 256:
         return blocks <= WIDE_CUS and (columns >= 512 or k <= 5120)
@@ -716,19 +733,15 @@ def _lds_in_parts(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None
     """(tile, parts) of q/k/v in parts, or None where another product is the better one.  5 to 16 rows all (8 rows: 4,096 x 1,024
     4.7 -> 4.2 us, 6,144 x 2,560 8.6 -> 8.4, 4,096 x 4,096 10.8 -> 9.4); up to four rows through a larger weight the kernels for few
     rows tie or win (6,144 x 1,024 at 1 row 4.9 against 5.4, x 4,096 11.7 against 12.7, 8,192 x 4,096 15.9 against 16.7).  17 to 64
-    rows, weights of up to 52 MB, one round of the chip (6,144 x 2,560 at 64 rows 10.5 -> 9.4, 4,096 x 1,024 6.5 -> 5.8): a second
-    round that is not whole costs as much as a whole one (6,144 x 2,560 in 384 blocks at 17 / 32 rows 10.0 against 10.9, 10.6
-    against 12.6), unless the weight has more rows than the other product for these takes."""
-    few = rows <= SKINNY_MAX_ROWS
-    if few and rows <= FEW_ROWS_IN_PARTS and weight_rows > (4096 if k < 2048 else 5120 if 3072 <= k <= 4096 else 6144):
+    rows, weights of up to 52 MB: one round of the chip (6,144 x 2,560 at 64 rows 10.5 -> 9.4, at 17 10.1 -> 9.5, at 32 10.7 -> 10.4
+    and in 384 blocks 12.6; 4,096 x 1,024 6.5 -> 5.8)."""
+    if rows <= SKINNY_MAX_ROWS:
+        if rows <= FEW_ROWS_IN_PARTS and weight_rows > (4096 if k < 2048 else 5120 if 3072 <= k <= 4096 else 6144):
+            return None
+        return lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, summed=True)
+    if rows > MID_ROWS or weight_rows * k > 26_000_000:
         return None
-    if not few and (rows > MID_ROWS or weight_rows * k > 26_000_000):
-        return None
-    tile, parts = lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, summed=True)
-    blocks = -(-rows // LDS_TILES[tile][0]) * -(-weight_rows // LDS_TILES[tile][1]) * parts
-    if not few and blocks > WIDE_CUS and weight_rows <= WIDE_MAX_WEIGHT_ROWS:
-        return None
-    return tile, parts
+    return lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, summed=True, one_round=True)
 
 
 def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:

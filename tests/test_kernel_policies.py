@@ -224,7 +224,7 @@ def test_which_logits_go_through_lds():
 def test_which_gated_products_go_through_lds():
     """Both sides of every line of the rule: the rounds that the planned blocks make, rows, columns, K."""
     pays = ops._lds_gate_pays
-    taken = ((1, 3072, 1024), (8, 9728, 2560), (8, 17408, 5120), (16, 12288, 5120), (5, 4096, 4096), (5, 12288, 4096),
+    taken = ((1, 3072, 1024), (8, 9728, 2560), (2, 2064, 2432), (983, 960, 2880), (128, 9728, 2496), (8, 17408, 5120), (16, 12288, 5120), (5, 4096, 4096), (5, 12288, 4096),
              (17, 9728, 2560), (64, 9728, 2560), (32, 14336, 8192), (65, 17408, 5120), (128, 6144, 2048), (256, 9728, 2560), (192, 9728, 2560),
              (384, 3072, 1024), (700, 3072, 1024), (1536, 256, 1024), (80, 512, 5184), (320, 1536, 4096), (320, 4864, 4096))
     left = ((8, 13824, 2560), (1, 14336, 2048), (4, 4096, 4096), (8, 17408, 4096), (64, 11008, 2048), (32, 16384, 4096),
@@ -237,30 +237,31 @@ def test_which_gated_products_go_through_lds():
 
 
 def test_which_updates_go_through_lds():
-    for size in ((1, 3072, 1024), (16, 5120, 10240), (17, 8192, 4096), (256, 8192, 4096), (384, 3584, 1024), (384, 6144, 5120), (640, 4096, 8192), (768, 3584, 8192),
+    for size in ((1, 3072, 1024), (16, 5120, 10240), (17, 8192, 4096), (256, 8192, 4096), (384, 3584, 1024), (384, 6144, 5120), (640, 4096, 8192), (768, 3584, 8192), (271, 6320, 3136),
                  (1024, 2560, 9728), (1024, 5120, 25600), (384, 8192, 16384)):
         assert ops._lds_update(*size) is not None, size
-    for size in ((1, 3088, 4096), (1, 6144, 12288), (16, 5120, 10176), (257, 3600, 4096), (320, 4096, 4096), (384, 6144, 5056), (385, 3072, 4096),
-                 (769, 3072, 9728), (641, 3600, 9728), (1025, 2560, 9728), (768, 4096, 8192), (257, 8192, 16320)):
+    for size in ((1, 3088, 4096), (1, 6144, 12288), (16, 5120, 10176), (257, 3840, 4096), (320, 4096, 4096), (384, 6144, 4864), (385, 3072, 4096),
+                 (769, 3072, 9728), (641, 3840, 9728), (1025, 2560, 9728), (768, 4096, 8192), (257, 8192, 16128)):
         assert ops._lds_update(*size) is None, size
 
 
 def test_which_projections_in_parts_go_through_lds():
-    for size in ((1, 4096, 1024), (4, 6144, 2048), (4, 6144, 2560), (4, 5120, 4096), (4, 6144, 4160), (5, 8192, 4096), (64, 6144, 2560),
-                 (33, 6144, 2560), (17, 4096, 1024), (32, 4096, 2560), (32, 12288, 1024)):
-        plan = ops._lds_in_parts(*size)
-        assert plan is not None and 1 <= plan[1] <= 4, size      # at most what the attention launch adds up
-    for size in ((1, 4112, 1024), (4, 6144, 4096), (4, 5136, 3072), (1, 6160, 2048), (17, 6144, 2560), (32, 6144, 2560), (32, 6144, 2048),
-                 (24, 3072, 5120), (64, 6144, 4288), (65, 4096, 1024)):
+    for rows, weight_rows, k in ((1, 4096, 1024), (4, 6144, 2048), (4, 6144, 2560), (4, 5120, 4096), (4, 6144, 4160), (5, 8192, 4096), (64, 6144, 2560),
+                                 (17, 6144, 2560), (32, 6144, 2560), (24, 6144, 4096), (17, 4096, 1024), (32, 12288, 1024), (64, 25344, 1024)):
+        tile, parts = ops._lds_in_parts(rows, weight_rows, k)
+        assert 1 <= parts <= 4                                   # at most what the attention launch adds up
+        if rows > 16:                                            # one round of the chip
+            assert -(-rows // ops.LDS_TILES[tile][0]) * -(-weight_rows // ops.LDS_TILES[tile][1]) * parts <= 256, (rows, weight_rows, k)
+    for size in ((1, 4112, 1024), (4, 6144, 4096), (4, 5136, 3072), (1, 6160, 2048), (64, 6144, 4288), (65, 4096, 1024)):
         assert ops._lds_in_parts(*size) is None, size
 
 
 def test_which_stored_products_go_through_lds():
     for size in ((9, 1024, 1024), (5, 8192, 2048), (17, 2048, 1024), (192, 3072, 8192), (256, 6144, 2560), (512, 4096, 1024), (320, 4096, 2048),
-                 (385, 4096, 2048), (384, 3568, 2048), (384, 4096, 1984), (288, 3584, 6144)):
+                 (385, 4096, 2048), (384, 3568, 2048), (329, 3864, 3008), (384, 4096, 1984), (288, 3584, 6144)):
         assert ops._lds_store_pays(*size), size
     for size in ((4, 4096, 2048), (8, 8208, 2048), (8, 4096, 1984), (17, 2032, 1024), (193, 3072, 8192), (257, 4112, 1024), (513, 2048, 1024),
-                 (321, 4096, 2048), (384, 3584, 2048), (288, 3568, 6144), (64, 10240, 5120)):
+                 (321, 4096, 2048), (384, 3584, 2048), (288, 3328, 6144), (64, 10240, 5120)):
         assert not ops._lds_store_pays(*size), size
 
 

@@ -8,7 +8,7 @@
 //   * grid (key split, kv head, sequence); with few sequences the keys of one
 //     (sequence, head) are split over several blocks so that the chip is full,
 //     and the block that finishes last merges the splits (a counter per (sequence, head));
-//     with a dozen sequences and more, or a few long ones, the splits follow the lengths (find_run);
+//     with a dozen sequences and more, or a few, where contexts may be long, the splits follow the lengths (find_run);
 //   * inside a block the four waves take 32-key blocks in turn;
 //   * scores transposed, S^T = K Q^T: MFMA 16x16x32 with A = 16 keys (rows) and
 //     B = the G query rows padded to 16 (columns).  The 32 keys of a block feed

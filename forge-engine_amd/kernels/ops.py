@@ -269,22 +269,17 @@ def gemm_skinny(x: Tensor, weight: Tensor, epilogue: str = "bf16", tiles: int = 
 
 
 # Up to 16 rows of x the product through LDS (``gemm_lds``, below) goes first wherever it fits (K of at least 1,024 in whole
-# 64-steps, 512 weight rows) and wins: see ``_lds_update``, ``_lds_store_pays``, ``_lds_gate_pays`` and ``linear_in_parts``.
-# Which kernel takes the rest, measured in the decode step at the sizes of Qwen3-4B, 8B and 32B
-# (hidden 2560 / 4096 / 5120; milliseconds a step before -> after at the batch named).  The kernels for up to 16
-# rows (`fe_gemm_skinny`) were shaped at 8 rows of the 4B sizes; the product for portions (`fe_gemm_wide`: a tile
-# of 16 rows of x in LDS, 64 weight rows a block, K in the parts that fill the CUs) turned out faster for:
-# * updates of the stream (output and down projections) from 4 rows (4B, batch 8: 2.83 -> 2.79, batch 16: 3.35 ->
-#   3.17; 8B, batch 8: 4.15 -> 3.96; 32B, batch 16: 18.2 -> 16.3), and faster than the library there (8B, batch 16:
-#   4.39 against 4.45); with up to 3 rows the K-split kernel stays (4B, batch 1: 2.50 against 2.51);
-# * gate/up at K up to 3072, with gate and up rows paired in a wave, at every row count (4B: 2.50 -> 2.48 at batch 1,
-#   2.83 -> 2.79 at batch 8, 3.35 -> 3.28 at batch 16); at K = 4096 the kernel whose blocks keep x in registers wins
-#   (8B, batch 8: 3.94 against 4.15); a weight of more than 40,000 rows goes to the library from 2 rows (32B: 13.86
-#   -> 13.50 at batch 2, 14.75 -> 14.27 at batch 8, 16.35 -> 15.85 at batch 16; a weight of 34,816 rows at the same
-#   K does not: 72 against 78 us at 8 rows);
-# * q/k/v: from 5 rows, in up to four parts that the attention launch adds up (4B, batch 8: 2.74 -> 2.71, batch 16:
-#   3.35 -> 3.31; 8B, batch 16: 4.84 -> 4.70); a weight of more than 64 MB goes to the library from 5 rows (14B,
-#   batch 8: 6.70 -> 6.61; 32B, batch 16: 15.85 -> 15.00 with the other two in place).
+# 64-steps, 512 weight rows) and wins: see ``_lds_update``, ``_lds_store_pays``, ``_lds_gate_pays``, ``_lds_in_parts`` and
+# ``_lds_head_pays``.  What it leaves goes by the lines below: smaller models, K of other lengths, and of larger models
+# * updates through more than 3,072 rows whose K is under twice their rows (8B and 32B: the output projection): the product for
+#   portions (`fe_gemm_wide`: a tile of 16 rows of x in LDS, 64 weight rows a block, K in the parts that fill the CUs) from 4 rows,
+#   with up to 3 rows the kernel for few rows (`fe_gemm_skinny`), K in parts (a decode step at 8B, batch 8, milliseconds: 4.15 ->
+#   3.96; 32B, batch 16: 18.2 -> 16.3);
+# * gate/up of K = 4,096 (8B) at up to four rows: the kernel for few rows, whose blocks keep x in registers; a weight of more than
+#   40,000 rows (32B): the library from 2 rows (13.86 -> 13.50 at batch 2, 14.75 -> 14.27 at batch 8; a weight of 34,816 rows at
+#   the same K does not: 72 against 78 us at 8 rows);
+# * q/k/v up to four rows through larger weights: the kernel for few rows in two parts; from 5 rows a weight of more than 64 MB: the
+#   library (14B, batch 8: 6.70 -> 6.61; 32B, batch 16: 15.85 -> 15.00 with the other two in place).
 FEW_ROWS = 8                        # q/k/v where the product for portions does not fit: up to here the kernel for up to 16 rows
 FEW_ROWS_IN_PARTS = 4               # q/k/v: up to here the kernel for up to 16 rows, then the product for portions in parts
 FEW_ROWS_UPDATE = 3                 # updates of the stream: up to here
@@ -396,18 +391,13 @@ def gemm_mid_parts(x: Tensor, weight: Tensor, parts: int) -> Tensor:
     return out
 
 
-# Measured on MI355X at Qwen3-4B's sizes against the matrix library, per call: the products back to the
-# hidden size (2560 weight rows; K = 4096 / 9728) in parts of K take 10 / 20 us at 128 rows (library 28 / 53),
-# 14 / 30 us at 256 rows (25 / 46), 18 / 41 at 384 (24 / 47) and lose from 512 rows on; the q/k/v product
-# (6144 weight rows) takes 18 - 20 us at 96 and 128 rows in row tiles of 64 and 23 - 26 us at 192 and 256 rows
-# in tiles of 128 (library 24 and 27 - 33), 15 - 16 us at 32 and 64 rows in blocks of 32 weight rows (library
-# 20 - 23); the gate/up product (19456 weight rows) is the library's at every row count above 64 (55 against
-# 52 us at 256 rows).
+# The product for portions with the weight straight in registers, for what the product through LDS (below) does not take: K under
+# 1,024, fewer than 512 weight rows, and, stored, weights of fewer than 2,048 rows or more than 50 MB.  (Measured at Qwen3-4B's
+# sizes, which go through LDS since: the output projection at 256 rows 14 us against the matrix library's 25, the down projection 30
+# against 46, q/k/v 23 - 26 against 27 - 33; it loses from 512 rows on.)
 WIDE_UPDATE_MAX_ROWS = 384     # most rows of x for which a product in parts of K beats the matrix library ...
 WIDE_UPDATE_SURE_ROWS = 256    # ... for weights of up to WIDE_UPDATE_FEW_WEIGHT_ROWS rows; up to this many rows it does for every
-WIDE_UPDATE_FEW_WEIGHT_ROWS = 3072   # weight measured (hidden sizes 2560, 4096, 5120 at 256 rows: output projection 14 / 21 / 45 us
-                                     # against 25 / 26 / 73, down projection 30 / 55 / 146 against 46 / 59 / 178); at 384 rows the
-                                     # hidden sizes 4096 and 5120 are the library's by a tenth
+WIDE_UPDATE_FEW_WEIGHT_ROWS = 3072   # weight measured
 WIDE_STORE_MAX_ROWS = 256      # ... and a product that stores bfloat16
 WIDE_STORE_MIN_BLOCKS = 140    # ... with more than 64 rows, if its launch has at least this many blocks (row tiles x 64 weight
                                # rows): q/k/v of 6144 rows 18-26 against 24-33 us and of 4608 to 5120 rows level with the library,
@@ -689,7 +679,7 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
             return gemm_lds(x, weight, "parts", plan[1], plan[0])
     if plain_bf16 and FEW_ROWS_UPDATE < x.shape[0] <= SKINNY_MAX_ROWS and _wide_fits(x, weight, SKINNY_MAX_ROWS, 1):
         # a tile of 16 rows of x: a tile's rows beyond M are fetched and multiplied like the others (with tiles of
-        # 64 rows: 4B, batch 16: 3.05 -> 3.00 ms; 32B: 15.4 -> 14.9; tiles of 32 rows for 17 to 32 rows lose 2 to 6 %)
+        # 64 rows a step of the 32B sizes at batch 16: 15.4 -> 14.9 ms)
         return gemm_wide(x, weight, "parts", _wide_parts(x.shape[0], weight.shape[0], weight.shape[1]), row_tile=16)
     if (plain_bf16 and _skinny_fits(x, weight)
             and -(-weight.shape[0] // 16) <= UPDATE_SPLIT_MAX_TILES
@@ -700,9 +690,8 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
         splits = -(-steps // -(-steps // splits))        # parts of equal length, none empty
         return gemm_skinny(x, weight, "f32", tiles=1, waves=4, splits=splits)
     if plain_bf16 and _wide_fits(x, weight, MID_ROWS, SKINNY_MAX_ROWS + 1):
-        # 17 to 64 rows: one tile of x a block, the parts of K that fill the CUs; measured at 64 rows against
-        # the product below: output projection 9.2 against 11.1 us (hidden size 4096: 10.6 against 12.5),
-        # down projection 15.1 against 15.3 us (25.0 against 30.2)
+        # 17 to 64 rows where K is shorter than 1,024 or the weight has fewer than 512 rows (the product through LDS takes the
+        # rest): one tile of x a block, the parts of K that fill the CUs
         return gemm_wide(x, weight, "parts", _wide_parts(x.shape[0], weight.shape[0], weight.shape[1]), row_tile=64)
     if plain_bf16 and x.shape[0] > SKINNY_MAX_ROWS and _mid_fits(x, weight):
         steps = -(-weight.shape[1] // 128)
@@ -710,8 +699,8 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
         return gemm_mid_parts(x, weight, _mid_parts(steps, blocks))
     if plain_bf16 and _wide_fits(x, weight, WIDE_UPDATE_MAX_ROWS if weight.shape[0] <= WIDE_UPDATE_FEW_WEIGHT_ROWS
                                  else WIDE_UPDATE_SURE_ROWS):
-        # a long K beside more than 128 rows: blocks of eight waves (128 weight rows share a tile of x) in twice the
-        # parts; measured at K = 9728: 29 against 32 us at 256 rows, 38 against 43 at 384 (at K = 4096 nothing)
+        # (likewise what the product through LDS does not take) a long K beside more than 128 rows: blocks of eight waves (128
+        # weight rows share a tile of x) in twice the parts
         block_rows = 128 if x.shape[0] > 128 and weight.shape[1] >= 8192 else 64
         parts = _wide_parts(x.shape[0], weight.shape[0], weight.shape[1], block_rows)
         return gemm_wide(x, weight, "parts", parts, block_rows=block_rows)
@@ -760,8 +749,8 @@ def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
     if plan is not None:
         return gemm_lds(x, weight, "parts", plan[1], plan[0])
     if FEW_ROWS_IN_PARTS < rows <= SKINNY_MAX_ROWS and _wide_fits(x, weight, SKINNY_MAX_ROWS, 1):
-        # blocks of 32 weight rows in up to four parts of K (768 blocks for 6144 weight rows): 1 % of the step
-        # at 6 to 16 rows against the kernels below (4B, batch 8: 2.74 -> 2.71 ms; 8B: 3.93 -> 3.89)
+        # (what the product through LDS does not take: K of 960, fewer than 512 weight rows) blocks of 32 weight rows in up
+        # to four parts of K
         parts = _wide_parts(rows, weight.shape[0], weight.shape[1], 32, most=4)
         return gemm_wide(x, weight, "parts", parts, row_tile=16, block_rows=32)
     if _skinny_fits(x, weight) and rows <= FEW_ROWS:
@@ -837,7 +826,8 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tenso
         # gate and up rows paired in a wave.  17 to 64 rows (many requests decoding), measured at 32 rows against the
         # matrix library with the gate kernel behind it: 24 against 28 us at 9728 columns of K = 2560, 46 against 50 at
         # 12288 of K = 4096; at K = 5120 the library wins (17408 columns: 85 against 82 us, 25600 columns: 111 against
-        # 96), and from 96 rows on at every size.  Up to 16 rows: see FEW_ROWS above.
+        # 96), and from 96 rows on at every size.  (Sizes that `_lds_gate_pays` leaves, up to 16 rows at K up to
+        # 3,072, and K under 1,024.)
         return gemm_wide(x, gate_up_weight, "swiglu_half", block_rows=_gate_block_columns(gate_up_weight.shape[0] // 2), act=act)
     if _skinny_fits(x, gate_up_weight) and not to_library:
         return gemm_skinny(x, gate_up_weight, "swiglu", act=act)

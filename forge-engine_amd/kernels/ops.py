@@ -951,10 +951,10 @@ def decode_runs(num_decode: int, num_seqs: int, kv_heads: int, head_dim: int, re
     """The decode launch's ``splits``: ``decode_splits``, or -E for runs by length.  With as many runs for every sequence the
     launch lasts as long as its longest run, and that depends on where the long ones land; runs by length, found on the
     device, cut a sequence into runs of at most (all key blocks / E), and no fewer than 12, and order them so that CUs share the
-    keys evenly.
+    keys evenly (one run a CU where that comes out even: equal contexts take the splits' own parts).
     Measured at 32 query heads on 8 kv heads of 128 (us, splits -> by length; lengths drawn from a tenth of the longest up, one long
     one beside others of an eighth, all the longest): up to 2,000 keys 12 sequences 18.2 -> 18.2, 15.9 -> 11.9, 26.8 -> 22.9, 32: 30.1
-    -> 29.3, 25.7 -> 16.3, 42.8 -> 46.1, 64: 59.7 -> 49.6, 30.4 -> 22.2, 98.6 -> 95.2; 4 of up to 16,000 29.5 -> 27.6.  What finding
+    -> 29.3, 25.7 -> 16.3, 50.9 -> 51.9, 64: 59.7 -> 49.6, 30.4 -> 22.2, 98.6 -> 95.2; 4 of up to 16,000 29.5 -> 27.6.  What finding
     the runs costs, 0.9 us, shows where contexts are short (32 of 1,000 24.4 against 26.8, of 20 to 200 9.0 against 10.1) and where
     a launch is latency alone (1 of 217 8.3 against 9.3), and with few blocks equal splits are as short (2 kv heads, 16 of 200 to
     2,000 10.4 against 12.2), so: from twelve sequences and 40 (sequence, kv head) pairs where contexts may reach 2,048, from three

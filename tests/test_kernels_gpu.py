@@ -1395,17 +1395,44 @@ def test_decode_attention_in_runs_by_length_beside_portions(ops):
                                          q_heads=2, kv_heads=1, head_dim=64, eps=1e-6, scale=0.1, max_ctx=64, **form)
 
 
-def _runs_by_length(contexts, own, more, window, chunk):
+def _runs_by_length(contexts, own, more, window, chunk, layer):
     """How many runs each sequence is cut into, as the launch finds it: key blocks of 32 that its token reads, over at most
-    max(12, ceil(all / more)) blocks a run."""
+    max(12, ceil(all / more)) blocks a run; at most ceil(all / layer) + 1 where no more than ``layer`` runs come of that."""
     blocks = []
     for ctx in contexts:
         first = max(0, ctx - window) if window else 0
         if chunk:
             first = max(first, (ctx - 1) // chunk * chunk)
         blocks.append(max(-(-(ctx - own) // 32) - first // 32, 0))
-    target = max(-(-sum(blocks) // more), 12)
+    target, even = max(-(-sum(blocks) // more), 12), -(-sum(blocks) // layer) + 1
+    if even > target and sum(max(-(-b // even), 1) for b in blocks) <= layer:
+        target = even
     return [max(-(-b // target), 1) for b in blocks]
+
+
+@pytest.mark.parametrize("kv_heads,contexts,splits", [
+    (8, [3008] * 8, 4), (8, [6000 + 5 * i for i in range(4)], 8), (4, [1000] * 32, 2), (6, [6000] * 3, 13),
+    (8, [3008] * 7 + [3500], 0), (8, [3008] * 9, 0)])
+def test_decode_attention_in_even_runs(ops, kv_heads, contexts, splits):
+    """Contexts that a run for each CU cuts evenly are cut so, into the bits of as many splits; with one longer, or one sequence
+    more (``splits`` 0), the runs are those for two a CU."""
+    g = torch.Generator().manual_seed(len(contexts))
+    n, layer, more = len(contexts), 256 // kv_heads, 512 // kv_heads - 2 * len(contexts) // 3
+    for own in (1, 0):
+        runs = _runs_by_length(contexts, own, more, None, None, layer)
+        assert runs == [splits] * n if splits else sum(runs) > layer
+    sizes = dict(q_heads=2 * kv_heads, kv_heads=kv_heads, head_dim=64)
+    qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq, _, _ = _prepare_case(g, 2 * kv_heads, kv_heads, 64, 16, [c - 1 for c in contexts])
+    dev = [t.to(DEV) for t in (qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq)]
+    results = []
+    for form in ({"by_length": more}, {"splits": splits or 4}):
+        out = torch.full((n, 2 * kv_heads * 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.decode_attention_prepare(dev[0], dev[6], dev[7], dev[8], dev[1], dev[2], out, dev[3], dev[4], dev[5], eps=1e-6, scale=0.1,
+                                     max_ctx=max(contexts), **form, **sizes)
+        results.append(out)
+    # float32 sums in another order, one rounding each: an ulp of bfloat16 at most
+    torch.testing.assert_close(results[0].float(), results[1].float(), atol=2e-3, rtol=2.0 ** -7)
+    assert torch.equal(*results) == bool(splits)
 
 
 @pytest.mark.parametrize("kv_heads,contexts,more,window,chunk,layers,most", [
@@ -1420,7 +1447,7 @@ def test_decode_attention_in_many_runs_by_length(ops, kv_heads, contexts, more, 
     g = torch.Generator().manual_seed(more)
     n, layer = len(contexts), 256 // kv_heads
     for own in (1, 0):
-        runs = _runs_by_length(contexts, own, more, window, chunk)
+        runs = _runs_by_length(contexts, own, more, window, chunk, layer)
         assert -(-sum(runs) // layer) >= layers and max(runs) >= most and sum(runs) <= n + more, (sum(runs), layer, max(runs))
     sizes = dict(q_heads=2 * kv_heads, kv_heads=kv_heads, head_dim=64)
     qkv, kp, vp, cu, ctx, table, qw, kw, inv_freq, positions, token_seq = _prepare_case(g, 2 * kv_heads, kv_heads, 64, 16, [c - 1 for c in contexts])

@@ -3,6 +3,7 @@
 #pragma once
 #include "common.h"
 #include <atomic>
+#include <type_traits>
 
 namespace lds_tile {
 
@@ -27,6 +28,13 @@ template <int PENDING>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PENDING) : "memory");
 }
+// the same for min(AHEAD, ahead) steps of PER loads each: the counts of a walk's end are known only when it runs, and a wait takes a constant
+template <int PER, int AHEAD>
+__device__ __forceinline__ void wait_steps(int ahead) {
+  if constexpr (AHEAD <= 0) wait_loads<0>();
+  else if (ahead >= AHEAD) wait_loads<PER * AHEAD>();
+  else wait_steps<PER, AHEAD - 1>(ahead);
+}
 // all of this wave's reads of LDS have arrived, and it goes on when every wave of the block is here
 __device__ __forceinline__ void reads_done_barrier() {
   __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4));      // lgkmcnt(0), and nothing of the other counters
@@ -49,7 +57,10 @@ struct Shape {
 // LDS holds a step of a tile as [row][8 chunks of 16 bytes], chunk c of row j at position c ^ (j % 8): the lanes that a 16-byte
 // read serves in one cycle then hit different bank groups (no conflicts counted).  Both operands go there straight from memory
 // (`global_load_lds_dwordx4`), STAGES buffers, all of them in flight; one barrier a step.  A wave requests the fragments of its
-// next half step from LDS before it multiplies those of this one.
+// next half step from LDS before it multiplies those of this one.  The last STAGES steps request nothing (until then they fetched
+// the last step again, so that one constant served every wait: a quarter more requests at K = 2,560 and ten stages, and a block
+// ended when those had landed).  Decode steps: 0.6B, 1 request 947 -> 909 us, 4B, 8 requests 2,532 -> 2,464, 64 requests 4,291 ->
+// 4,245; counting the way down at run time, a chain of branches a step, cost more than it saved (1,058 at 1 request).
 template <int MI, int NI, int WM, int WN, int KG, int STAGES, bool HALF_END, typename RowOf>
 __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, int last, int K, floatx4 (&acc)[MI][NI]) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, WAVES = WM * WN * KG, T = 2 / KG;
@@ -62,8 +73,8 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
   const bf16_t* from[LOADS + 1];
 #pragma unroll
   for (int i = 0; i <= LOADS; ++i) from[i] = row_of(min((wave + WAVES * i) * 8 + (lane >> 3), BM + BN - 1));
-  auto load = [&](int step, int stage) {       // past the end the last step again, so that the waits can count
-    const int k0 = min(step, last - 1) * KSTEP;
+  auto load = [&](int step, int stage) {
+    const int k0 = step * KSTEP;
     const int at = k0 + (HALF_END && k0 + KSTEP > K ? my_chunk & 3 : my_chunk) * 8;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) load_to_lds(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
@@ -94,17 +105,18 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b[j]), __builtin_bit_cast(bf16x8, a[i]), acc[i][j], 0, 0, 0);
     };
     int stage = 0;
-    // a half: the next half's fragments are requested, then this half's are multiplied
-    auto half = [&](int step, bool ends_step, int t_next, const uintx4* a, const uintx4* b, uintx4* a_next, uintx4* b_next) {
+    // a half: the next half's fragments are requested, then this half's are multiplied.
+    auto half = [&](int step, bool ends_step, auto ahead, bool loads, int t_next, const uintx4* a, const uintx4* b, uintx4* a_next, uintx4* b_next) {
       const int t = T == 1 ? 0 : ends_step;
       int from_stage = stage;
       if (ends_step) {
         // this wave's share of the next step has landed, and behind the barrier everyone's; everyone has read all of
         // this step, whose buffer is filled again
-        if (MORE > 0 && wave < MORE) wait_loads<(LOADS + 1) * (STAGES - 2)>();
-        else wait_loads<LOADS * (STAGES - 2)>();
+        constexpr int AHEAD = decltype(ahead)::value;
+        if (MORE > 0 && wave < MORE) wait_loads<(LOADS + 1) * AHEAD>();
+        else wait_loads<LOADS * AHEAD>();
         reads_done_barrier();
-        load(step + STAGES, stage);
+        if (loads) load(step + STAGES, stage);
         stage = stage + 1 == STAGES ? 0 : stage + 1;
         from_stage = stage;
       }
@@ -113,26 +125,49 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
       if (!HALF_END || step * KSTEP + (group * T + t) * 32 < K) multiply(a, b);
       __builtin_amdgcn_sched_barrier(0);
     };
+    const std::integral_constant<int, STAGES - 2> full;
 #pragma unroll
-    for (int s = 0; s < STAGES; ++s) load(first + s, s);
-    if (MORE > 0 && wave < MORE) wait_loads<(LOADS + 1) * (STAGES - 1)>();
-    else wait_loads<LOADS * (STAGES - 1)>();
+    for (int s = 0; s < STAGES; ++s)
+      if (first + s < last) load(first + s, s);
+    if (MORE > 0 && wave < MORE) wait_steps<LOADS + 1, STAGES - 1>(last - 1 - first);
+    else wait_steps<LOADS, STAGES - 1>(last - 1 - first);
     reads_done_barrier();
     fragments(0, 0, a0, b0);
+    int step = first;
     if constexpr (T == 2) {
-      for (int step = first; step < last; ++step) {
-        half(step, false, 1, a0, b0, a1, b1);
-        half(step, true, 0, a1, b1, a0, b0);
+      for (; last - step > STAGES; ++step) {
+        half(step, false, full, true, 1, a0, b0, a1, b1);
+        half(step, true, full, true, 0, a1, b1, a0, b0);
       }
     } else {
-      int step = first;
-      for (; step + 1 < last; step += 2) {
-        half(step, true, 0, a0, b0, a1, b1);
-        half(step + 1, true, 0, a1, b1, a0, b0);
+      for (; last - step > STAGES + 1; step += 2) {
+        half(step, true, full, true, 0, a0, b0, a1, b1);
+        half(step + 1, true, full, true, 0, a1, b1, a0, b0);
       }
-      if (step < last) half(step, true, 0, a0, b0, a1, b1);
+      if ((last - step) % 2 == 0) fragments(stage, 0, a1, b1);      // below, an odd count of steps left finds its fragments in a0
     }
-    wait_loads<0>();
+    // The last STAGES steps (STAGES + 1 where two steps make a round) request nothing, or no further step: fewer and fewer loads
+    // are under way, and a wait takes a constant, so each of them is written out.
+    const int rest = last - step;
+    auto end = [&](auto self, auto left) {
+      constexpr int L = decltype(left)::value;
+      if constexpr (L > 0) {
+        const std::integral_constant<int, (L < STAGES ? (L > 1 ? L - 2 : 0) : STAGES - 2)> ahead;
+        if (rest >= L) {
+          if constexpr (T == 2) {
+            half(last - L, false, ahead, false, 1, a0, b0, a1, b1);
+            if constexpr (L > 1) half(last - L, true, ahead, false, 0, a1, b1, a0, b0);
+            else if (!HALF_END || (last - 1) * KSTEP + (group * T + 1) * 32 < K) multiply(a1, b1);
+          } else {
+            const uintx4 *a = L % 2 ? a0 : a1, *b = L % 2 ? b0 : b1;
+            if constexpr (L > 1) half(last - L, true, ahead, L > STAGES, 0, a, b, L % 2 ? a1 : a0, L % 2 ? b1 : b0);
+            else if (!HALF_END || (last - 1) * KSTEP + group * 32 < K) multiply(a, b);
+          }
+        }
+        self(self, std::integral_constant<int, L - 1>{});
+      }
+    };
+    end(end, std::integral_constant<int, T == 2 ? STAGES : STAGES + 1>{});
   }
   if constexpr (KG > 1) {
     reads_done_barrier();

@@ -961,6 +961,22 @@ def test_gemm_lds(ops, tile, m, n, k, parts):
     assert torch.equal(one_row[:, 0], got[:, 0])                 # a row's sums do not depend on the rows beside it
 
 
+@pytest.mark.parametrize("tile", range(14))
+def test_gemm_lds_walks_of_every_length(ops, tile):
+    """Walks over K of one step to more than two rounds of the buffers (3 to 12 stages), whose last steps are written out one by one:
+    |error| <= 2 k 2^-24 sum |a||b| as above."""
+    g = torch.Generator().manual_seed(tile)
+    m, n = (7, 40) if tile >= 9 else (70, 40)
+    for steps in range(1, 27):
+        k = 64 * steps
+        x = rand(g, m, k, dtype=torch.bfloat16).to(DEV)
+        w = rand(g, 2 * n, k, dtype=torch.bfloat16, scale=0.05).to(DEV)
+        exact = x.double() @ w.double().t()
+        bound = (x.double().abs() @ w.double().abs().t()) * (2 * k + 2) * 2.0 ** -24
+        got = ops.gemm_lds(x, w, "parts", 1, tile)[0]
+        assert bool(((got.double() - exact).abs() <= bound + 1e-30).all()), steps
+
+
 def test_gemm_lds_refuses_and_plans(ops, monkeypatch):
     x = torch.zeros(70, 1024, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(4096, 1024, dtype=torch.bfloat16, device=DEV)

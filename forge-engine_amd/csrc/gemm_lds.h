@@ -43,12 +43,21 @@ using lds_tile::KSTEP;
 constexpr int XCDS = 8;
 constexpr int END_PARTS = 0, END_BF16 = 1, END_GATED = 2;
 
+// Rows whose norm's factor was left out (gemm_update.hip): the sums of row m are multiplied by rsqrt(sum of squares[m][.] / width +
+// eps) before anything else is done with them.  The factors are made from LDS, where the row's 256 partial sums of squares went
+// ahead of the walk over K.
+struct RowFactors {
+  const float* squares;       // [M][256]
+  float width, eps;
+};
+constexpr int SQUARES = 256, SQUARES_PITCH = SQUARES * 4 + 16;      // bytes from row to row in LDS: sixteen rows in different banks
+
 // With the gated ending a fragment of sixteen weight rows is eight gate rows and the eight up rows of the same columns.
-template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END>
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END, bool SCALED>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
     long long ldw, long long ldo, int tiles_m, int tiles_n, int parts, int steps_per_part, long long part_stride,
-    long long up_offset, GateAct act) {
+    long long up_offset, GateAct act, RowFactors factors) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN;
   constexpr int COLUMNS = END == END_GATED ? BN / 2 : BN;
   extern __shared__ __attribute__((aligned(16))) uintx4 lds[];     // [STAGES][BM + BN rows][8]
@@ -69,9 +78,29 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
     if (END == END_GATED) return w + (size_t)min(n0 + (j >> 4) * 8 + (j & 7), N - 1) * ldw + ((j & 8) ? up_offset : 0);
     return w + (size_t)min(n0 + j, N - 1) * ldw;
   };
+  constexpr int STAGE_BYTES = STAGES * (BM + BN) * 128;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4, wm = wave % WM, wn = wave / WM;
+  if constexpr (SCALED) {
+    static_assert(MI == 1 && WM == 1, "rows of x in one tile of sixteen");
+    const unsigned int base = __builtin_amdgcn_readfirstlane((unsigned int)(size_t)(const __attribute__((address_space(3))) char*)&lds[0]);
+    for (int m = __builtin_amdgcn_readfirstlane(wave); m < M; m += WN * KG)
+      lds_tile::load_to_lds(factors.squares + m * SQUARES + lane * 4, base + STAGE_BYTES + m * SQUARES_PITCH);
+  }
   floatx4 acc[MI][NI];
   if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, false>(lds, row_of, first, last, K, acc)) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4, wm = wave % WM, wn = wave / WM;
+  if constexpr (SCALED) {
+    // Lane (r, q) adds up a quarter of row r's squares.  A wave's loads arrive in order, so its rows were there before its first
+    // step of K, and behind that step's barrier everyone's.
+    if (first < last) {
+      const floatx4* from = (const floatx4*)((const char*)lds + STAGE_BYTES + min(r, M - 1) * SQUARES_PITCH) + q * (SQUARES / 16);
+      floatx4 sum = from[0];
+#pragma unroll
+      for (int j = 1; j < SQUARES / 16; ++j) sum += from[j];
+      const float factor = rsqrtf(sum_xor32(sum_xor16((sum[0] + sum[1]) + (sum[2] + sum[3]))) / factors.width + factors.eps);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[0][j] *= factor;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int m = m0 + (wm * MI + i) * 16 + r;
@@ -116,21 +145,23 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
   }
 }
 
-template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END>
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END, bool SCALED = false>
 static int launch_tile(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int parts,
-                       long long part_stride, GateAct act, hipStream_t stream) {
+                       long long part_stride, GateAct act, hipStream_t stream, RowFactors factors = {}) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, COLUMNS = END == END_GATED ? BN / 2 : BN;
-  constexpr size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES;
+  const size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? (M <= 8 ? 8 : 16) * SQUARES_PITCH : 0);
   static std::atomic<bool> raised{false};
-  auto kernel = gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END>;
-  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, bytes, &raised);
+  auto kernel = gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED>;
+  static_assert(!SCALED || lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + 16 * SQUARES_PITCH <= 160 * 1024, "LDS of a CU");
+  const int limit_raised = lds_tile::raise_lds_limit(
+      (const void*)kernel, lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? 16 * SQUARES_PITCH : 0), &raised);
   if (limit_raised != FE_OK) return limit_raised;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + COLUMNS - 1) / COLUMNS;
   if (tiles_m * tiles_n * parts > 0x7fffffffLL) return FE_BAD_ARGUMENT;
   const int steps = K / KSTEP, per_part = (steps + parts - 1) / parts;
   kernel<<<(unsigned)(tiles_m * tiles_n * parts), 64 * WM * WN * KG, bytes, stream>>>(
       (const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldw, ldo, (int)tiles_m, (int)tiles_n, parts, per_part, part_stride,
-      (long long)N * ldw, act);
+      (long long)N * ldw, act, factors);
   return fe_check_launch();
 }
 
@@ -160,6 +191,28 @@ static int launch(const void* x, const void* w, void* out, int M, int N, int K, 
     FE_TILE(10, 1, 1, 1, 2, 2, 12)
     FE_TILE(11, 1, 1, 1, 3, 2, 9)
     FE_TILE(12, 1, 1, 1, 4, 2, 8)
+    FE_TILE(13, 1, 1, 1, 5, 2, 10)
+  }
+#undef FE_TILE
+#undef FE_END
+  return FE_BAD_ARGUMENT;
+}
+
+// The same for up to 16 rows of x with row factors: tiles 9 to 13, endings parts and gated.  Two buffers fewer where two blocks
+// share a CU's LDS, which the squares would keep from it.
+static int launch_scaled(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
+                         int parts, long long part_stride, int tile, GateAct act, hipStream_t stream, RowFactors factors) {
+#define FE_END(END, ...) return launch_tile<__VA_ARGS__, END, true>(x, w, out, M, N, K, ldw, ldo, parts, part_stride, act, stream, factors)
+#define FE_TILE(I, ...)                                                \
+  case I:                                                              \
+    if (ending == END_PARTS) FE_END(END_PARTS, __VA_ARGS__);           \
+    else if (ending == END_GATED) FE_END(END_GATED, __VA_ARGS__);      \
+    break;
+  switch (tile) {
+    FE_TILE(9, 1, 1, 1, 1, 2, 12)
+    FE_TILE(10, 1, 1, 1, 2, 2, 10)
+    FE_TILE(11, 1, 1, 1, 3, 2, 7)
+    FE_TILE(12, 1, 1, 1, 4, 2, 6)
     FE_TILE(13, 1, 1, 1, 5, 2, 10)
   }
 #undef FE_TILE

@@ -307,3 +307,18 @@ extern "C" int fe_gemm_wide(const void* x, const void* w, void* out, int M, int 
 #undef FE_LAUNCH
   return fe_check_launch();
 }
+
+// Endings 0 and 2 through LDS for up to 16 rows of x whose norm's factors were left out: `squares` [M][256] float32 (fe_gemm_update_norm),
+// the sums of row m are multiplied by rsqrt(sum of squares[m] / width + eps).  lds_tile 9 to 13.
+extern "C" int fe_gemm_lds_scaled(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo,
+                                  int ending, int parts, long long part_stride, int lds_tile, int activation, const float* squares,
+                                  float width, float eps, hipStream_t stream) {
+  if (M < 1) return FE_OK;
+  GateAct act;
+  if (!gate_act(activation, &act)) return FE_BAD_ARGUMENT;
+  if (M > 16 || N < 1 || K < WSTEP || K % WSTEP || ldw < K || ldw % 8 || ldo < N) return FE_BAD_ARGUMENT;
+  if (!squares || !(width > 0.f) || !(eps > 0.f) || ((((uintptr_t)x) | ((uintptr_t)w) | ((uintptr_t)squares)) & 15)) return FE_BAD_ARGUMENT;
+  if ((ending != EPI_PARTS && ending != EPI_SWIGLU) || parts < 1 || parts > 64 || (ending != EPI_PARTS && parts != 1)) return FE_BAD_ARGUMENT;
+  if (parts > 1 && part_stride < (long long)M * ldo) return FE_BAD_ARGUMENT;
+  return through_lds::launch_scaled(x, w, out, M, N, K, ldw, ldo, ending, parts, part_stride, lds_tile, act, stream, {squares, width, eps});
+}

@@ -11,6 +11,7 @@ from __future__ import annotations
 import functools
 import threading
 from ctypes import c_double, c_float, c_int, c_longlong, c_void_p
+from typing import NamedTuple
 
 import numpy as np
 import torch
@@ -299,7 +300,11 @@ FEW_ROWS_LIBRARY_MIN_K = 4097   # ... unless K is short enough for the blocks of
 def _few_rows_to_library(x: Tensor, weight: Tensor) -> bool:
     """A product that stores bfloat16 (q/k/v), 5 to 16 rows, a weight too large for the kernels of
     few rows to win: the matrix library."""
-    return (FEW_ROWS_IN_PARTS < x.shape[0] <= SKINNY_MAX_ROWS and weight.shape[1] >= FEW_ROWS_LIBRARY_MIN_K
+    return _few_rows_library_pays(x.shape[0], weight)
+
+
+def _few_rows_library_pays(rows: int, weight: Tensor) -> bool:
+    return (FEW_ROWS_IN_PARTS < rows <= SKINNY_MAX_ROWS and weight.shape[1] >= FEW_ROWS_LIBRARY_MIN_K
             and weight.shape[0] * weight.shape[1] * weight.element_size() > IN_PARTS_MAX_WEIGHT_BYTES)
 
 
@@ -476,6 +481,7 @@ LDS_HEAD_MIN_K = 2048
 LDS_GATE_MAX_ROWS = 1536       # gate/up: measured up to here (4,096 rows, 256 columns of K = 4,096: 28.6 against 43.0 us)
 LDS_MIN_K = 1024               # measured from this K on ...
 LDS_MIN_WEIGHT_ROWS = 512      # ... and for weights of at least this many rows
+UPDATE_NORM_MAX_WIDTH = 8192   # 32 weight rows a block
 
 
 def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, summed: bool = False,
@@ -636,6 +642,91 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     return rows * columns <= 600_000 or large_tiles >= 180
 
 
+class UpdateProduct(NamedTuple):
+    """An update of the residual stream that has not been multiplied out: x @ weight^T."""
+
+    x: Tensor
+    weight: Tensor
+
+
+class UnscaledRows(NamedTuple):
+    """Rows of a norm without its factors: bfloat16(h * weight) [M, N], and what the factor of row m is made of:
+    rsqrt(sum of squares[m] / N + eps), squares [M, 256] float32."""
+
+    rows: Tensor
+    squares: Tensor
+    eps: float
+
+    @property
+    def shape(self) -> torch.Size:
+        return self.rows.shape
+
+
+def update_norm_fits(x: Tensor, weight: Tensor) -> bool:
+    """Whether a product back to the residual stream may be left to ``update_norm``.  us in a captured graph, product and norm in two
+    launches -> one: 1,024 x 2,048 at 1 / 16 rows 5.4 -> 3.2 / 6.1 -> 3.9, 2,048 x 6,144 9.5 -> 7.0 / 9.9 -> 8.6, 2,560 x 9,728 13.7 ->
+    11.2 / 13.8 -> 13.3, 5,120 x 25,600 51 -> 48 / 50 -> 49, 8,192 x 4,096 18.6 -> 15.9 / 22 -> 16 (wider ones would need more
+    rows a block; 8,192 x 8,192 at 1 row alone is slower, 30.8 -> 32.5, at 8 38.6 -> 31.0)."""
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+            and 0 < x.shape[0] <= SKINNY_MAX_ROWS and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
+            and weight.shape[0] <= UPDATE_NORM_MAX_WIDTH and x.shape[1] % 64 == 0 and weight.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def update_norm(h: Tensor, product: UpdateProduct, norm_weight: Tensor, eps: float) -> UnscaledRows:
+    """h += x @ weight^T (float32, in place), and the rows bfloat16(h * norm_weight) with their sums of squares, in one launch."""
+    x, weight = product
+    _gpu(h, "h", torch.float32)
+    _gpu(norm_weight, "norm_weight", torch.float32)
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(weight, "weight", torch.bfloat16, contiguous=False)
+    if not update_norm_fits(x, weight) or h.shape != (x.shape[0], weight.shape[0]) or norm_weight.shape != (weight.shape[0],) or not eps > 0.0:
+        raise KernelError(f"no product with a norm behind it for {tuple(x.shape)} x {tuple(weight.shape)} into {tuple(h.shape)}")
+    m, n = h.shape
+    rows = torch.empty((m, n), dtype=torch.bfloat16, device=h.device)
+    squares = torch.empty((m, 256), dtype=torch.float32, device=h.device)
+    _call("gemm_update", "fe_gemm_update_norm", _ptr(x), _ptr(weight), _ptr(h), _ptr(norm_weight), _ptr(rows), _ptr(squares),
+          c_int(m), c_int(n), c_int(x.shape[1]), c_longlong(weight.stride(0)), _stream())
+    return UnscaledRows(rows, squares, float(eps))
+
+
+def _weight_fits_lds(weight: Tensor) -> bool:
+    return (weight.dtype == torch.bfloat16 and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] >= LDS_MIN_K
+            and weight.shape[1] % 64 == 0 and weight.shape[0] >= LDS_MIN_WEIGHT_ROWS and weight.stride(0) % 8 == 0
+            and weight.data_ptr() % 16 == 0)
+
+
+def unscaled_in_parts(rows: int, weight: Tensor) -> bool:
+    """Whether ``linear_in_parts`` takes ``UnscaledRows``: where it takes the product through LDS."""
+    return (0 < rows <= SKINNY_MAX_ROWS and _weight_fits_lds(weight) and not _few_rows_library_pays(rows, weight)
+            and _lds_in_parts(rows, *weight.shape) is not None)
+
+
+def unscaled_swiglu(rows: int, gate_up_weight: Tensor) -> bool:
+    """Whether ``linear_swiglu`` takes ``UnscaledRows``: where it takes the product through LDS."""
+    return (0 < rows <= SKINNY_MAX_ROWS and _weight_fits_lds(gate_up_weight) and gate_up_weight.shape[0] % 2 == 0
+            and not (rows > 1 and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS)
+            and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1]))
+
+
+def _gemm_lds_unscaled(x: UnscaledRows, weight: Tensor, ending: str, parts: int, tile: int, act: str) -> Tensor:
+    rows, squares, eps = x
+    _gpu(rows, "x", torch.bfloat16)
+    _gpu(squares, "squares", torch.float32)
+    m, k = rows.shape
+    n = weight.shape[0]
+    if squares.shape != (m, 256) or not 0 < m <= SKINNY_MAX_ROWS or LDS_TILES[tile][0] != 16 or ending not in ("parts", "gated"):
+        raise KernelError("rows without their norm's factors: up to 16, with 256 sums of squares each, float32 parts or a gated product")
+    if ending == "parts":
+        out, cols = torch.empty((parts, m, n), dtype=torch.float32, device=rows.device), n
+    else:
+        out, cols = torch.empty((m, n // 2), dtype=torch.bfloat16, device=rows.device), n // 2
+    _call("gemm_wide", "fe_gemm_lds_scaled", _ptr(rows), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
+          c_longlong(weight.stride(0)), c_longlong(cols), c_int(0 if ending == "parts" else 2), c_int(parts), c_longlong(m * cols),
+          c_int(tile), _gate_act(act), _ptr(squares), c_float(k), c_float(eps), _stream())
+    return out
+
+
 def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu") -> Tensor:
     """x @ weight^T for bfloat16 rows: ``"parts"`` float32 partial sums [parts, M, N] over runs of whole 64-steps of K,
     ``"bf16"`` [M, N], or ``"gated"``: act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first; ``act`` as in
@@ -733,10 +824,15 @@ def _lds_in_parts(rows: int, weight_rows: int, k: int) -> tuple[int, int] | None
     return lds_plan(rows, weight_rows, k, 4 * weight_rows, 4, summed=True, one_round=True)
 
 
-def linear_in_parts(x: Tensor, weight: Tensor) -> Tensor | None:
+def linear_in_parts(x: Tensor | UnscaledRows, weight: Tensor) -> Tensor | None:
     """x @ weight^T as float32 partial sums [parts <= 4, M, N] over parts of K, for a consumer that
     adds them up itself (the decode attention kernel that prepares its own queries and keys);
     None where the plain product is the better choice or the sizes do not fit."""
+    if isinstance(x, UnscaledRows):
+        if not unscaled_in_parts(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
+            raise KernelError("rows without their norm's factors are for the product through LDS only")
+        tile, parts = _lds_in_parts(x.shape[0], *weight.shape)
+        return _gemm_lds_unscaled(x, weight, "parts", parts, tile, "silu")
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     steps = -(-weight.shape[1] // 128)
@@ -801,8 +897,13 @@ GATED_TILE_MAX_ROWS = 4096
 GATED_TILE_MAX_K = 3072
 
 
-def linear_swiglu(x: Tensor, gate_up_weight: Tensor, act: str = "silu") -> Tensor:
+def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "silu") -> Tensor:
     """act(x Wg^T) * (x Wu^T) for the fused weight [2I, K] (gate rows first); ``act`` as in ``swiglu``."""
+    if isinstance(x, UnscaledRows):
+        if not unscaled_swiglu(x.shape[0], gate_up_weight) or gate_up_weight.shape[1] != x.shape[1]:
+            raise KernelError("rows without their norm's factors are for the product through LDS only")
+        tile, _ = lds_plan(x.shape[0], *gate_up_weight.shape, gate_up_weight.shape[0])
+        return _gemm_lds_unscaled(x, gate_up_weight, "gated", 1, tile, act)
     _gpu(x, "x")
     _gpu(gate_up_weight, "gate_up_weight")
     rows = x.shape[0]
@@ -1354,7 +1455,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_update", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

@@ -319,27 +319,36 @@ class GroupedQueryAttention(Mixer):
     CONV_STATE = "conv"
 
     takes_stream = True
+    leaves_product = True
 
-    def forward(self, x: Tensor, batch, cache: CacheView, writes_cache: bool = True,
-                stream: Tensor | None = None) -> Tensor | None:
+    def takes_unscaled(self, tokens: int, batch, cache: CacheView, writes_cache: bool = True) -> bool:
+        rotary = self.position.rotary()
+        return (not self.general and writes_cache and self.qkv_bias is None
+                and self._single_tokens_only(batch, tokens, cache, 0 if rotary is None else rotary[1])
+                and ops.unscaled_in_parts(tokens, self.qkv_weight))
+
+    def forward(self, x: Tensor | ops.UnscaledRows, batch, cache: CacheView, writes_cache: bool = True,
+                stream: Tensor | None = None, product: bool = False) -> Tensor | ops.UpdateProduct | None:
         rotary = self.position.rotary()
         inv_freq, rotary_dim = rotary if rotary is not None else (None, 0)
         if self.general:
             return self._forward_general(x, batch, cache, writes_cache, stream, inv_freq, rotary_dim)
         eps = self.qk_norm_eps if self.qk_norm_eps is not None else 1.0
         if writes_cache:
-            if self._single_tokens_only(batch, x, cache, rotary_dim):
+            if self._single_tokens_only(batch, x.shape[0], cache, rotary_dim):
                 # norms, rotation, cache write and attention in one launch, which also adds up
                 # the projection's partial sums where the product is faster with K in parts
                 qkv = ops.linear_in_parts(x, self.qkv_weight) if self.qkv_bias is None else None
                 if qkv is None:
                     qkv = ops.linear(x, self.qkv_weight, self.qkv_bias)
-                attn = torch.empty((x.shape[0], self.q_size), dtype=x.dtype, device=x.device)
+                attn = torch.empty((x.shape[0], self.q_size), dtype=self.ctx.dtype, device=qkv.device)
                 ops.decode_attention_prepare(
                     qkv, self.q_norm, self.k_norm, inv_freq, cache.key_pages, cache.value_pages, attn,
                     batch.cu_q, batch.ctx_len, cache.block_table, q_heads=self.num_heads,
                     kv_heads=self.num_kv_heads, head_dim=self.head_dim, eps=eps, scale=self.scale,
                     window=self.window, max_ctx=batch.max_ctx)
+                if product and self.o_bias is None and ops.update_norm_fits(attn, self.o_weight):
+                    return ops.UpdateProduct(attn, self.o_weight)
                 return ops.linear_update(attn, self.o_weight, self.o_bias, stream)
             qkv = ops.linear(x, self.qkv_weight, self.qkv_bias)
         else:  # another call wrote the keys and values this one reads: only q is needed
@@ -428,12 +437,12 @@ class GroupedQueryAttention(Mixer):
             norm_weight_k=self.k_norm if self.qk_norm_eps is not None else None,
             norm_first=self.qk_norm_eps is not None, q_temp=self.query_temperature, **mixing)
 
-    def _single_tokens_only(self, batch, x: Tensor, cache: CacheView, rotary_dim: int) -> bool:
+    def _single_tokens_only(self, batch, tokens: int, cache: CacheView, rotary_dim: int) -> bool:
         """Every sequence of the step brings one token, and the sizes are ones that the
         decode kernel prepares queries and keys for itself."""
-        return (batch.num_decode is not None and batch.num_decode == batch.num_seqs == x.shape[0]
+        return (batch.num_decode is not None and batch.num_decode == batch.num_seqs == tokens
                 and ops.decode_prepare_supported(
-                    x.dtype, q_heads=self.num_heads, kv_heads=self.num_kv_heads, head_dim=self.head_dim,
+                    self.ctx.dtype, q_heads=self.num_heads, kv_heads=self.num_kv_heads, head_dim=self.head_dim,
                     rotary_dim=rotary_dim, block_size=cache.key_pages.shape[2]))
 
     def token_inputs(self):
@@ -442,7 +451,7 @@ class GroupedQueryAttention(Mixer):
     def kernel_libraries(self):
         if self.general:
             return {"whole_norm_rope" if self.whole_norm_eps is not None else "conv_rope", "attention_masked", "attention_decode", "attention_prefill", "stream_ops", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide"}
-        return {"qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide"}
+        return {"qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_update"}
 
 
 register_part("mixer", "gqa_attention", GroupedQueryAttention)

@@ -65,7 +65,7 @@ class Residual:
 
     def __init__(self, h: Tensor) -> None:
         self.h = h
-        self.pending: Tensor | None = None
+        self.pending = None
         self.streams: Tensor | None = None
         self.pending_mix: tuple[Tensor, Tensor] | None = None    # (mix [S, S] indexed [from, to], share [S])
         self.pending_bias: Tensor | None = None                   # float32 [W]: added with the pending update, or alone
@@ -73,8 +73,28 @@ class Residual:
         self.pending_norm: tuple[Tensor, float] | None = None    # (weight, eps): the update is RMS-normed before it is added
         self.in_compute_dtype: Tensor | None = None               # the stream as a norm of updates last stored it beside h (the same values)
 
-    def add(self, update: Tensor | None, bias: Tensor | None = None) -> None:
-        """Leave an update pending; None: the part has added it into the stream itself.  ``bias``: one number a
+    @property
+    def pending(self) -> Tensor | None:
+        """The update that has not been added yet; one that was left as a product is multiplied out now."""
+        if isinstance(self._pending, ops.UpdateProduct):
+            self._pending = ops.linear_update(self._pending.x, self._pending.weight)
+        return self._pending
+
+    @pending.setter
+    def pending(self, update: Tensor | ops.UpdateProduct | None) -> None:
+        self._pending = update
+
+    def take_product(self) -> ops.UpdateProduct | None:
+        """A pending update that is still a product, if nothing else is pending: the caller makes and adds it itself."""
+        if (not isinstance(self._pending, ops.UpdateProduct) or self.streams is not None or self.pending_other is not None
+                or self.pending_bias is not None or self.pending_norm is not None):
+            return None
+        product, self._pending = self._pending, None
+        return product
+
+    def add(self, update: Tensor | ops.UpdateProduct | None, bias: Tensor | None = None) -> None:
+        """Leave an update pending, as a tensor or as a product that the next norm may make in its own launch (``take_product``;
+        everyone else finds the tensor in ``pending``); None: the part has added it into the stream itself.  ``bias``: one number a
         channel that comes on top."""
         self.flush()
         self.in_compute_dtype = None
@@ -279,6 +299,12 @@ class Mixer(Part):
     # it may add its update into the stream itself, where its last product can do so for free, and
     # then returns None instead of the update.
     takes_stream = False
+    # True for a part whose forward takes ``product=True``: it may then return its update as an ``ops.UpdateProduct``.
+    leaves_product = False
+
+    def takes_unscaled(self, tokens: int, batch, cache: CacheView | None, writes_cache: bool = True) -> bool:
+        """Whether ``forward`` takes, for this step, rows whose norm left its factors out (``ops.UnscaledRows``)."""
+        return False
 
     def joint_ends(self) -> JointEnds | None:
         """The part's outer matrices, if it can run between products that it shares with others (``forward_joint``)."""
@@ -302,7 +328,11 @@ class Mixer(Part):
 class FeedForward(Part):
     role = "feed_forward"
     takes_stream = False   # as for a mixer
+    leaves_product = False
     takes_extra = False    # True: ``forward`` takes ``extra=``, an update of the same tokens that joins its own
+
+    def takes_unscaled(self, tokens: int) -> bool:
+        return False       # as for a mixer
 
     def joint_ends(self) -> JointEnds | None:
         return None        # as for a mixer

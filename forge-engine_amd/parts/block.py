@@ -21,18 +21,24 @@ class PreNormBlock(Block):
     NORMS = ("input", "post_mixer")
 
     def forward(self, residual: Residual, batch, cache: CacheView | None, writes_cache: bool = True) -> None:
-        x = self.norms["input"].forward(residual)
-        if self.mixer.takes_stream:
-            residual.add(self.mixer.forward(x, batch, cache, writes_cache, stream=residual.open()))
-        else:
-            residual.add(self.mixer.forward(x, batch, cache, writes_cache))
+        x = self._normed("input", residual, lambda rows: self.mixer.takes_unscaled(rows, batch, cache, writes_cache))
+        residual.add(self.mixer.forward(x, batch, cache, writes_cache, **self._ways(self.mixer, residual)))
         if self.feed_forward is None:
             return
-        y = self.norms["post_mixer"].forward(residual)
-        if self.feed_forward.takes_stream:
-            residual.add(self.feed_forward.forward(y, batch, stream=residual.open()))
-        else:
-            residual.add(self.feed_forward.forward(y, batch))
+        y = self._normed("post_mixer", residual, self.feed_forward.takes_unscaled)
+        residual.add(self.feed_forward.forward(y, batch, **self._ways(self.feed_forward, residual)))
+
+    def _normed(self, role: str, residual: Residual, takes_unscaled) -> Tensor:
+        norm = self.norms[role]
+        if getattr(norm, "leaves_factors", False):
+            return norm.forward(residual, unscaled=takes_unscaled(residual.h.shape[0]))
+        return norm.forward(residual)
+
+    @staticmethod
+    def _ways(part, residual: Residual) -> dict:
+        """How the part may hand over its update beside returning it: into the stream itself, or as a product."""
+        ways = {"stream": residual.open()} if part.takes_stream else {}
+        return dict(ways, product=True) if part.leaves_product else ways
 
 
 class OutputNormBlock(Block):

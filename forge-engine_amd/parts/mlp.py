@@ -51,9 +51,15 @@ class SwiGLU(FeedForward):
             raise KeyError(name)
 
     takes_stream = True
+    leaves_product = True
 
-    def forward(self, x: Tensor, batch=None, stream: Tensor | None = None) -> Tensor | None:
+    def takes_unscaled(self, tokens: int) -> bool:
+        return ops.unscaled_swiglu(tokens, self.gate_up_weight)
+
+    def forward(self, x: Tensor | ops.UnscaledRows, batch=None, stream: Tensor | None = None, product: bool = False) -> Tensor | ops.UpdateProduct | None:
         act = ops.linear_swiglu(x, self.gate_up_weight, self.activation)
+        if product and ops.update_norm_fits(act, self.down_weight):
+            return ops.UpdateProduct(act, self.down_weight)
         return ops.linear_update(act, self.down_weight, stream=stream)   # the update stays float32 for the residual sum
 
     def joint_ends(self) -> JointEnds:
@@ -66,7 +72,7 @@ class SwiGLU(FeedForward):
         ops.swiglu(z, out, self.activation)
 
     def kernel_libraries(self):
-        return {"rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_tile"}
+        return {"rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_update", "gemm_tile"}
 
 
 class PolyNormMLP(FeedForward):

@@ -37,7 +37,15 @@ class RMSNorm(Norm):
             raise KeyError(name)
         self.weight = tensor + self.offset if self.offset else tensor
 
-    def forward(self, residual: Residual, rows: Tensor | None = None) -> Tensor:
+    leaves_factors = True
+
+    def forward(self, residual: Residual, rows: Tensor | None = None, unscaled: bool = False) -> Tensor | ops.UnscaledRows:
+        """``unscaled``: who reads the rows can multiply by the norm's factors itself, so a pending product may be added and
+        normed in one launch up to those."""
+        if unscaled and rows is None:
+            product = residual.take_product()
+            if product is not None:
+                return ops.update_norm(residual.h, product, self.weight, self.eps)
         if residual.pending_norm is not None:    # a norm behind the sublayer before: both norms in one pass over the row
             if rows is not None:                 # the chosen rows alone; stream and pending update are left as they are
                 update, (weight, eps) = residual.pending, residual.pending_norm
@@ -56,7 +64,7 @@ class RMSNorm(Norm):
         return ops.add_rmsnorm(residual.h, update, self.weight, self.eps, out, other=other, shift=shift)
 
     def kernel_libraries(self):
-        return {"rowwise", "stream_ops"}
+        return {"rowwise", "stream_ops", "gemm_update"}
 
 
 class UpdateRMSNorm(RMSNorm):
@@ -64,6 +72,8 @@ class UpdateRMSNorm(RMSNorm):
     ``u * rsqrt(mean(u^2) + eps) * w``, and added into the stream, all in float32 and in one
     kernel.  Returns the new stream in the compute dtype (what the next sublayer reads: the
     sublayers of such a layer see the stream itself)."""
+
+    leaves_factors = False
 
     def forward(self, residual: Residual, rows: Tensor | None = None) -> Tensor:
         if rows is not None:

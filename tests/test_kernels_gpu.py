@@ -961,6 +961,53 @@ def test_gemm_lds(ops, tile, m, n, k, parts):
     assert torch.equal(one_row[:, 0], got[:, 0])                 # a row's sums do not depend on the rows beside it
 
 
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(1, 64), (255, 448), (256, 512), (1024, 2048), (2049, 1088), (2568, 8256), (4097, 640), (6400, 4096), (8192, 1024)])
+def test_update_with_the_next_norm(ops, m, n, k):
+    """One to thirty-two weight rows a block, last blocks with fewer, waves without chunks to walks longer than their buffers, a
+    weight that is a slice of a wider one.  The stream against the exact products: |error| <= (2 k + 32) 2^-24 (|h| + sum |a||b|);
+    the rows are its rounded product with the norm's weight, the squares its own to the last bits of a sum of n."""
+    g = torch.Generator().manual_seed(m * n + k)
+    x = rand(g, m, k, dtype=torch.bfloat16).to(DEV)
+    w = rand(g, n, k + 64, dtype=torch.bfloat16, scale=0.05).to(DEV)[:, :k]
+    h, gain = rand(g, m, n).to(DEV), rand(g, n).to(DEV)
+    exact = h.double() + x.double() @ w.double().t()
+    bound = (h.double().abs() + x.double().abs() @ w.double().abs().t()) * (2 * k + 32) * 2.0 ** -24
+    got = h.clone()
+    out = ops.update_norm(got, ops.UpdateProduct(x, w), gain, 1e-6)
+    assert bool(((got.double() - exact).abs() <= bound).all())
+    assert torch.equal(out.rows, (got * gain).bfloat16())
+    squares = got.double().pow(2).sum(1)
+    assert bool(((out.squares.double().sum(1) - squares).abs() <= squares * 64 * 2.0 ** -24).all())
+    assert out.squares.shape == (m, 256) and bool((out.squares[:, -(-n // -(-n // 256)):] == 0).all())
+    again = h.clone()
+    assert torch.equal(ops.update_norm(again, ops.UpdateProduct(x, w), gain, 1e-6).rows, out.rows) and torch.equal(again, got)
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+@pytest.mark.parametrize("tile", range(9, 14))
+def test_rows_without_their_factors(ops, m, tile):
+    """What a norm in one launch gives and what reads it beside the same rows normed in float32 ahead of the product: the row
+    factor is one number, so both differ from the exact result by one rounding of each operand (2^-8) and the sums'."""
+    g = torch.Generator().manual_seed(tile)
+    n, k = 330, 1344
+    gain = rand(g, k).to(DEV)
+    h = rand(g, m, k).to(DEV) * torch.logspace(-3, 3, m, device=DEV)[:, None]
+    squares = torch.zeros(m, 256, device=DEV)
+    squares[:, :21] = h.pow(2).view(m, 21, 64).sum(2)
+    rows = ops.UnscaledRows((h * gain).bfloat16(), squares, 1e-6)
+    w = rand(g, 2 * n, k, dtype=torch.bfloat16, scale=0.05).to(DEV)
+    y = h.double() * torch.rsqrt(h.double().pow(2).mean(1, keepdim=True) + 1e-6) * gain.double()
+    exact, size = y @ w.double().t(), y.abs() @ w.double().abs().t()
+    for parts in (1, 4, 30):      # the last with parts that have no steps
+        got = ops._gemm_lds_unscaled(rows, w, "parts", parts, tile, "silu")
+        assert bool(((got.double().sum(0) - exact).abs() <= size * 2.0 ** -8).all())
+    gated = ops._gemm_lds_unscaled(rows, w, "gated", 1, tile, "silu").double()
+    want = torch.nn.functional.silu(exact[:, :n]) * exact[:, n:]
+    bound = (size[:, :n] * (exact[:, n:].abs() + size[:, n:] * 2.0 ** -8) * 1.1 + size[:, n:] * exact[:, :n].abs()) * 2.0 ** -8 + want.abs() * 2.0 ** -8
+    assert bool(((gated - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("tile", range(14))
 def test_gemm_lds_walks_of_every_length(ops, tile):
     """Walks over K of one step to more than two rounds of the buffers (3 to 12 stages), whose last steps are written out one by one:

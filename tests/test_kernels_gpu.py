@@ -1218,6 +1218,24 @@ def test_decode_attention_kernel_every_count_of_key_splits(ops, q_heads, kv_head
             torch.testing.assert_close(out.cpu().float(), want, atol=2e-2, rtol=2e-2, msg=lambda m: f"{splits} splits: {m}")
 
 
+@pytest.mark.parametrize("window", [None, 100, 128, 129])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(4, 2, 128), (8, 1, 64), (2, 2, 256)])
+def test_decode_attention_that_needs_no_splits(ops, q_heads, kv_heads, head_dim, window):
+    """Contexts and windows about the four blocks of 32 keys up to which a sequence takes none of the launch's splits, beside longer
+    ones that take them all, several times on the same counters."""
+    g = torch.Generator().manual_seed(64)
+    seqs = [(n - 1, 1) for n in (1, 32, 127, 128, 129, 160, 161, 700, 2, 96)]
+    q, kp, vp, cu, ctx, table = _attention_case(g, torch.bfloat16, seqs, q_heads, kv_heads, head_dim, 16)
+    kw = dict(q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, scale=head_dim ** -0.5, window=window)
+    want = refs.paged_attention_by_matrices(q, kp, vp, cu, ctx, table, **kw)
+    dev = [t.to(DEV) for t in (kp, vp, cu, ctx, table)]
+    for splits in (8, 3, 8):
+        out = torch.full((len(seqs), q_heads * head_dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.paged_attention(q.to(DEV), dev[0], dev[1], out, dev[2], dev[3], dev[4], num_seqs=len(seqs), max_q_len=1,
+                            num_decode=len(seqs), max_ctx=700, splits=splits, **kw)
+        torch.testing.assert_close(out.cpu().float(), want, atol=2e-2, rtol=2e-2, msg=lambda m: f"{splits} splits: {m}")
+
+
 @pytest.mark.parametrize("splits", [9, 12, 16, 17, 32, 64])
 @pytest.mark.parametrize("q_heads,kv_heads,head_dim,block_size", [(4, 2, 128, 16), (8, 1, 64, 32)])
 def test_decode_attention_that_prepares_with_many_key_splits(ops, q_heads, kv_heads, head_dim, block_size, splits):

@@ -43,7 +43,7 @@ using lds_tile::KSTEP;
 constexpr int XCDS = 8;
 constexpr int END_PARTS = 0, END_BF16 = 1, END_GATED = 2;
 
-// Rows whose norm's factor was left out (gemm_update.hip): the sums of row m are multiplied by rsqrt(sum of squares[m][.] / width +
+// Rows whose norm's factor was left out (gemm_ring.hip): the sums of row m are multiplied by rsqrt(sum of squares[m][.] / width +
 // eps) before anything else is done with them.  The factors are made from LDS, where the row's 256 partial sums of squares went
 // ahead of the walk over K.
 struct RowFactors {

@@ -330,8 +330,11 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
     to_library = out_dtype == torch.bfloat16 and _few_rows_to_library(x, weight)
     if (bias is None and out_dtype == torch.bfloat16 and not to_library and _lds_fits(x, weight)
             and _lds_store_pays(x.shape[0], *weight.shape)):
-        tile, _ = lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])
+        tile = None if _ring_store_pays(x.shape[0], *weight.shape) else lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])[0]
         return gemm_lds(x, weight, "bf16", tile=tile)
+    ending = {torch.float32: "f32", torch.bfloat16: "bf16"}.get(out_dtype)
+    if bias is None and not to_library and _ring_fits(x, weight, ending) and _ring_store_pays(x.shape[0], *weight.shape):
+        return gemm_ring(x, weight, ending)
     if bias is None and out_dtype == torch.float32 and _lds_fits(x, weight) and _lds_head_pays(x.shape[0], *weight.shape):
         rows = x.shape[0]          # (hundreds of tiles a CU: the cheapest tile whatever the rounds, not the plan's)
         return gemm_lds(x, weight, "parts", tile=10 if rows <= 8 else 12 if rows <= 16 else 8 if rows <= 32 else 4)[0]
@@ -685,9 +688,57 @@ def update_norm(h: Tensor, product: UpdateProduct, norm_weight: Tensor, eps: flo
     m, n = h.shape
     rows = torch.empty((m, n), dtype=torch.bfloat16, device=h.device)
     squares = torch.empty((m, 256), dtype=torch.float32, device=h.device)
-    _call("gemm_update", "fe_gemm_update_norm", _ptr(x), _ptr(weight), _ptr(h), _ptr(norm_weight), _ptr(rows), _ptr(squares),
+    _call("gemm_ring", "fe_gemm_update_norm", _ptr(x), _ptr(weight), _ptr(h), _ptr(norm_weight), _ptr(rows), _ptr(squares),
           c_int(m), c_int(n), c_int(x.shape[1]), c_longlong(weight.stride(0)), _stream())
     return UnscaledRows(rows, squares, float(eps))
+
+
+# The product with a ring for each wave (``gemm_ring``) beside what took a size before, measured over 420 random products of 1 to 16
+# rows (weights of 128 to 8,192 rows or 6,144 columns of two, K of 256 to 10,240; us, before -> this).
+RING_STORE_ROWS = 6144         # weight rows
+RING_GATE_COLUMNS = 6144
+RING_PARTS_ROWS = 2048
+
+
+def _ring_store_pays(rows: int, weight_rows: int, k: int) -> bool:
+    """Stored products: 1.36 times as fast on the average (2,048 x 2,048 at 1 / 8 / 16 rows 4.9 -> 3.8, 4.6 -> 3.9, 4.9 -> 4.3; 6,144 x 2,048
+    8.3 -> 6.9, 6.9 -> 6.6, 7.2 -> 6.8; 1,024 x 4,096 6.7 -> 4.4, 6.7 -> 4.5, 7.1 -> 5.3).  Not at a K of 256 (four of eight waves have
+    a chunk: 2.31 against 2.46), not beyond 6,144 weight rows (8,192 x 4,096 at 8 rows 13.9 against 15.2), nor through some 4,096 rows
+    at K >= 4,096 from five rows on, whose tiles of sixteen rows the other product fills too (7.6 against 7.8)."""
+    return rows <= SKINNY_MAX_ROWS and k >= 320 and weight_rows <= RING_STORE_ROWS and not (rows > 4 and k >= 4096 and 3584 < weight_rows <= 4096)
+
+
+def _ring_parts_pays(weight_rows: int, k: int) -> bool:
+    """q/k/v: from 2,048 weight rows on (6,144 x 2,560 at 1 / 8 rows 7.8 -> 7.7, 7.5 -> 7.4, x 4,096 11.8 -> 11.1, 11.8 -> 10.7; 4,096 x
+    2,048 5.2 against 5.5, but one sum instead of two for who adds them up); fewer rows have too few bytes a block at a long K
+    (1,024 x 4,608 at 16 rows 4.1 against 4.8)."""
+    return RING_PARTS_ROWS <= weight_rows <= RING_STORE_ROWS or (weight_rows < RING_PARTS_ROWS and k <= 2048)
+
+
+def gemm_ring(x: Tensor | UnscaledRows, weight: Tensor, ending: str, act: str = "silu") -> Tensor:
+    """x @ weight^T for up to 16 bfloat16 rows, whole sums in a block: ``"f32"`` or ``"bf16"`` [M, N] (N up to 8,192), or ``"gated"``:
+    act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first, up to 12,288 of both)."""
+    rows, squares, eps = x if isinstance(x, UnscaledRows) else (x, None, 0.0)
+    _gpu(rows, "x", torch.bfloat16)
+    _gpu(weight, "weight", torch.bfloat16, contiguous=False)
+    if not _ring_fits(rows, weight, ending):
+        raise KernelError(f"no product with a ring for each wave for {tuple(rows.shape)} x {tuple(weight.shape)}, {ending!r}")
+    m, k = rows.shape
+    if squares is not None and _gpu(squares, "squares", torch.float32).shape != (m, 256):
+        raise KernelError("rows without their norm's factors come with 256 sums of squares each")
+    n = weight.shape[0] // 2 if ending == "gated" else weight.shape[0]
+    out = torch.empty((m, n), dtype=torch.float32 if ending == "f32" else torch.bfloat16, device=rows.device)
+    _call("gemm_ring", "fe_gemm_ring", _ptr(rows), _ptr(weight), _ptr(out), c_int(m), c_int(n), c_int(k), c_longlong(weight.stride(0)),
+          c_int({"f32": 1, "bf16": 2, "gated": 3}[ending]), _gate_act(act), _ptr(squares), c_float(eps), _stream())
+    return out
+
+
+def _ring_fits(x: Tensor, weight: Tensor, ending: str) -> bool:
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+            and 0 < x.shape[0] <= SKINNY_MAX_ROWS and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
+            and x.shape[1] > 0 and x.shape[1] % 64 == 0 and weight.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0 and ending in ("f32", "bf16", "gated")
+            and 0 < weight.shape[0] <= (2 * RING_GATE_COLUMNS if ending == "gated" else UPDATE_NORM_MAX_WIDTH) and (ending != "gated" or weight.shape[0] % 2 == 0))
 
 
 def _weight_fits_lds(weight: Tensor) -> bool:
@@ -697,16 +748,17 @@ def _weight_fits_lds(weight: Tensor) -> bool:
 
 
 def unscaled_in_parts(rows: int, weight: Tensor) -> bool:
-    """Whether ``linear_in_parts`` takes ``UnscaledRows``: where it takes the product through LDS."""
+    """Whether ``linear_in_parts`` takes ``UnscaledRows``: where it takes a product through LDS."""
     return (0 < rows <= SKINNY_MAX_ROWS and _weight_fits_lds(weight) and not _few_rows_library_pays(rows, weight)
-            and _lds_in_parts(rows, *weight.shape) is not None)
+            and (_ring_parts_pays(*weight.shape) or _lds_in_parts(rows, *weight.shape) is not None))
 
 
 def unscaled_swiglu(rows: int, gate_up_weight: Tensor) -> bool:
-    """Whether ``linear_swiglu`` takes ``UnscaledRows``: where it takes the product through LDS."""
+    """Whether ``linear_swiglu`` takes ``UnscaledRows``: where it takes a product through LDS."""
     return (0 < rows <= SKINNY_MAX_ROWS and _weight_fits_lds(gate_up_weight) and gate_up_weight.shape[0] % 2 == 0
             and not (rows > 1 and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS)
-            and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1]))
+            and (gate_up_weight.shape[0] <= 2 * RING_GATE_COLUMNS
+                 or _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])))
 
 
 def _gemm_lds_unscaled(x: UnscaledRows, weight: Tensor, ending: str, parts: int, tile: int, act: str) -> Tensor:
@@ -727,10 +779,15 @@ def _gemm_lds_unscaled(x: UnscaledRows, weight: Tensor, ending: str, parts: int,
     return out
 
 
-def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int = 2, act: str = "silu") -> Tensor:
+def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int | None = 2, act: str = "silu") -> Tensor:
     """x @ weight^T for bfloat16 rows: ``"parts"`` float32 partial sums [parts, M, N] over runs of whole 64-steps of K,
     ``"bf16"`` [M, N], or ``"gated"``: act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first; ``act`` as in
-    ``swiglu``).  ``tile``: the block's, see ``LDS_TILES``."""
+    ``swiglu``).  ``tile``: the block's, see ``LDS_TILES``, or None: a ring for each wave (``gemm_ring``), whole sums."""
+    if tile is None:
+        if parts != 1:
+            raise KernelError("a ring for each wave makes whole sums")
+        out = gemm_ring(x, weight, {"parts": "f32"}.get(ending, ending), act)
+        return out.unsqueeze(0) if ending == "parts" else out
     _gpu(x, "x", torch.bfloat16)
     _gpu(weight, "weight", torch.bfloat16, contiguous=False)
     if (x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1] or x.shape[1] % 64 or weight.stride(1) != 1
@@ -830,7 +887,9 @@ def linear_in_parts(x: Tensor | UnscaledRows, weight: Tensor) -> Tensor | None:
     None where the plain product is the better choice or the sizes do not fit."""
     if isinstance(x, UnscaledRows):
         if not unscaled_in_parts(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
-            raise KernelError("rows without their norm's factors are for the product through LDS only")
+            raise KernelError("rows without their norm's factors are for the products through LDS only")
+        if _ring_parts_pays(*weight.shape):
+            return gemm_ring(x, weight, "f32").unsqueeze(0)
         tile, parts = _lds_in_parts(x.shape[0], *weight.shape)
         return _gemm_lds_unscaled(x, weight, "parts", parts, tile, "silu")
     _gpu(x, "x")
@@ -842,8 +901,11 @@ def linear_in_parts(x: Tensor | UnscaledRows, weight: Tensor) -> Tensor | None:
     if _few_rows_to_library(x, weight):
         return None
     plan = _lds_in_parts(rows, *weight.shape) if _lds_fits(x, weight) else None
+    ring = rows <= SKINNY_MAX_ROWS and _lds_fits(x, weight) and _ring_parts_pays(*weight.shape)
     if plan is not None:
-        return gemm_lds(x, weight, "parts", plan[1], plan[0])
+        return gemm_lds(x, weight, "parts", *((1, None) if ring else (plan[1], plan[0])))
+    if ring:
+        return gemm_ring(x, weight, "f32").unsqueeze(0)
     if FEW_ROWS_IN_PARTS < rows <= SKINNY_MAX_ROWS and _wide_fits(x, weight, SKINNY_MAX_ROWS, 1):
         # (what the product through LDS does not take: K of 960, fewer than 512 weight rows) blocks of 32 weight rows in up
         # to four parts of K
@@ -901,7 +963,9 @@ def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "
     """act(x Wg^T) * (x Wu^T) for the fused weight [2I, K] (gate rows first); ``act`` as in ``swiglu``."""
     if isinstance(x, UnscaledRows):
         if not unscaled_swiglu(x.shape[0], gate_up_weight) or gate_up_weight.shape[1] != x.shape[1]:
-            raise KernelError("rows without their norm's factors are for the product through LDS only")
+            raise KernelError("rows without their norm's factors are for the products through LDS only")
+        if gate_up_weight.shape[0] <= 2 * RING_GATE_COLUMNS:
+            return gemm_ring(x, gate_up_weight, "gated", act)
         tile, _ = lds_plan(x.shape[0], *gate_up_weight.shape, gate_up_weight.shape[0])
         return _gemm_lds_unscaled(x, gate_up_weight, "gated", 1, tile, act)
     _gpu(x, "x")
@@ -915,10 +979,15 @@ def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "
         return gemm_gated(x, gate_up_weight, shape=3, act=act)
     to_library = (2 <= rows <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
                   and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
+    # Up to 16 rows and 6,144 columns: a ring for each wave (1.41 times what took 140 random sizes before; 3,072 columns of K = 1,024 at
+    # 1 row 5.0 -> 4.8 us, 6,144 of 2,048 12.4 -> 11.8, of 4,096 25.1 -> 20.1; one of them slower by more than 1 %)
+    ring = rows <= SKINNY_MAX_ROWS and _lds_fits(x, gate_up_weight) and _ring_fits(x, gate_up_weight, "gated")
     if (not to_library and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
             and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])):
-        tile, _ = lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])
+        tile = None if ring else lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])[0]
         return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
+    if ring and not to_library:
+        return gemm_ring(x, gate_up_weight, "gated", act)
     paired_fits = (rows <= MID_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16
                    and x.is_contiguous() and gate_up_weight.is_contiguous() and x.shape[1] % 64 == 0
                    and x.shape[1] <= WIDE_GATE_MAX_K and gate_up_weight.shape[0] % 2 == 0
@@ -1455,7 +1524,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_update", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

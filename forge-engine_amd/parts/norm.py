@@ -64,7 +64,7 @@ class RMSNorm(Norm):
         return ops.add_rmsnorm(residual.h, update, self.weight, self.eps, out, other=other, shift=shift)
 
     def kernel_libraries(self):
-        return {"rowwise", "stream_ops", "gemm_update"}
+        return {"rowwise", "stream_ops", "gemm_ring"}
 
 
 class UpdateRMSNorm(RMSNorm):

@@ -985,11 +985,46 @@ def test_update_with_the_next_norm(ops, m, n, k):
 
 
 @pytest.mark.parametrize("m", [1, 8, 9, 16])
-@pytest.mark.parametrize("tile", range(9, 14))
+@pytest.mark.parametrize("n,k", [(1, 64), (255, 448), (256, 512), (1024, 2048), (2049, 1088), (2568, 8256), (4097, 640), (6144, 1024), (8192, 1024)])
+def test_gemm_ring(ops, m, n, k):
+    """One to thirty-two weight rows a block, last blocks with fewer, waves without chunks to walks longer than their buffers, a
+    weight that is a slice of a wider one: |error| <= (2 k + 32) 2^-24 sum |a||b|, and one rounding on top where bfloat16 is stored."""
+    g = torch.Generator().manual_seed(m * n + k)
+    x = rand(g, m, k, dtype=torch.bfloat16).to(DEV)
+    w = rand(g, 2 * n, k + 64, dtype=torch.bfloat16, scale=0.05).to(DEV)[:, :k]
+    exact = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * (2 * k + 32) * 2.0 ** -24 + 1e-30
+    assert bool(((ops.gemm_ring(x, w[n:], "f32").double() - exact[:, n:]).abs() <= bound[:, n:]).all())
+    stored = ops.gemm_ring(x, w[:n], "bf16").double()
+    assert bool(((stored - exact[:, :n]).abs() <= bound[:, :n] + exact[:, :n].abs() * 2.0 ** -8).all())
+    if n <= 6144:
+        for act in ("silu", "gelu_tanh"):
+            gated = ops.gemm_ring(x, w, "gated", act).float()
+            torch.testing.assert_close(gated, ops.swiglu(exact.float().contiguous(), torch.empty(m, n, device=DEV), act), atol=2e-2, rtol=2e-2)
+    one_row = ops.gemm_ring(x[:1].contiguous(), w[n:], "f32")
+    assert torch.equal(one_row[0], ops.gemm_ring(x, w[n:], "f32")[0])      # a row's sums do not depend on the rows beside it
+
+
+def test_gemm_ring_refuses(ops):
+    x = torch.zeros(16, 1024, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(16384, 1024, dtype=torch.bfloat16, device=DEV)
+    few = ops.UnscaledRows(x, torch.zeros(16, 255, device=DEV), 1e-6)
+    for bad in (lambda: ops.gemm_ring(x, w, "f32"), lambda: ops.gemm_ring(x, w[:12290], "gated"), lambda: ops.gemm_ring(x, w[:1023], "gated"),
+                lambda: ops.gemm_ring(x, w[:1024], "parts"), lambda: ops.gemm_ring(x[:, :1000].contiguous(), w[:8, :1000].contiguous(), "f32"),
+                lambda: ops.gemm_ring(torch.zeros(17, 1024, dtype=torch.bfloat16, device=DEV), w[:8], "f32"),
+                lambda: ops.gemm_ring(few, w[:1024], "f32"), lambda: ops.gemm_ring(x, w[:1024].float(), "f32"),
+                lambda: ops.gemm_lds(x, w[:1024], "parts", 2, None),
+                lambda: ops.update_norm(torch.zeros(16, 1024, device=DEV), ops.UpdateProduct(x, w[:1000]), torch.ones(1024, device=DEV), 1e-6)):
+        with pytest.raises(ops.KernelError):
+            bad()
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+@pytest.mark.parametrize("tile", [*range(9, 14), None])
 def test_rows_without_their_factors(ops, m, tile):
     """What a norm in one launch gives and what reads it beside the same rows normed in float32 ahead of the product: the row
     factor is one number, so both differ from the exact result by one rounding of each operand (2^-8) and the sums'."""
-    g = torch.Generator().manual_seed(tile)
+    g = torch.Generator().manual_seed(tile or 0)
     n, k = 330, 1344
     gain = rand(g, k).to(DEV)
     h = rand(g, m, k).to(DEV) * torch.logspace(-3, 3, m, device=DEV)[:, None]
@@ -999,10 +1034,10 @@ def test_rows_without_their_factors(ops, m, tile):
     w = rand(g, 2 * n, k, dtype=torch.bfloat16, scale=0.05).to(DEV)
     y = h.double() * torch.rsqrt(h.double().pow(2).mean(1, keepdim=True) + 1e-6) * gain.double()
     exact, size = y @ w.double().t(), y.abs() @ w.double().abs().t()
-    for parts in (1, 4, 30):      # the last with parts that have no steps
-        got = ops._gemm_lds_unscaled(rows, w, "parts", parts, tile, "silu")
+    for parts in (1, 4, 30) if tile is not None else (1,):      # 30: with parts that have no steps
+        got = ops.gemm_ring(rows, w, "f32")[None] if tile is None else ops._gemm_lds_unscaled(rows, w, "parts", parts, tile, "silu")
         assert bool(((got.double().sum(0) - exact).abs() <= size * 2.0 ** -8).all())
-    gated = ops._gemm_lds_unscaled(rows, w, "gated", 1, tile, "silu").double()
+    gated = (ops.gemm_ring(rows, w, "gated") if tile is None else ops._gemm_lds_unscaled(rows, w, "gated", 1, tile, "silu")).double()
     want = torch.nn.functional.silu(exact[:, :n]) * exact[:, n:]
     bound = (size[:, :n] * (exact[:, n:].abs() + size[:, n:] * 2.0 ** -8) * 1.1 + size[:, n:] * exact[:, :n].abs()) * 2.0 ** -8 + want.abs() * 2.0 ** -8
     assert bool(((gated - want).abs() <= bound).all())

@@ -198,9 +198,68 @@ def stream_read(data: Tensor, sink: Tensor) -> None:
 
 # ------------------------------------------------------------ matrix products
 
+# The float32 product on the matrix cores' bfloat16 instruction (``gemm_split``): its tiles (rows of a, rows of b, K a step) with the
+# microseconds a step takes a CU that holds one block (and, of the last tile, two).
+SPLIT_TILES = ((128, 160, 64, 3.7), (128, 128, 64, 3.1), (96, 128, 64, 2.45), (128, 64, 64, 1.87), (96, 64, 64, 1.52), (64, 64, 128, 2.0),
+               (32, 32, 128, 0.80))
+SPLIT_TWO_SMALL = 1.55
+SPLIT_MIN_K = 256
+SPLIT_MIN_ROWS_F32 = 64        # ``gemm_nt_f32`` keeps the rows of decode steps, whose sums do not depend on how many they are
+SPLIT_MIN_ROWS = 16            # layers take it from here on: 17 rows read the weight three times otherwise
+SPLIT_MOST_PARTS = 6
+
+
+def _split_fits(a: Tensor, b: Tensor) -> bool:
+    return (a.dtype == torch.float32 and b.dtype == torch.float32 and a.dim() == 2 and b.dim() == 2 and a.shape[0] > 0
+            and a.shape[1] == b.shape[1] and a.shape[1] >= SPLIT_MIN_K and a.shape[1] % 4 == 0 and a.stride(1) == 1 and b.stride(1) == 1
+            and a.stride(0) % 4 == 0 and b.stride(0) % 4 == 0 and a.stride(0) >= a.shape[1] and b.stride(0) >= b.shape[1]
+            and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _split_plan(m: int, n: int, k: int, most_parts: int) -> tuple[int, int]:
+    """(tile, parts of K) for ``gemm_split``: the least of what a launch is predicted to take, which is the steps of the fullest CU or
+    the weight's bytes at 4.5 TB/s, and what each part more costs who adds them up.  Over 1,715 launches (7 weights of 640 to 6,144
+    rows, 20 to 1,024 rows of a, every tile, 1 to 6 parts) the picks take 2 % longer than the best.  us, what took the size before ->
+    this: 700 x 4,096 x 1,024 62 -> 47, x 6,144 x 1,024 98 -> 69, x 1,024 x 2,048 in two parts 40 -> 31, x 2,048 x 6,144 in two 189 -> 129;
+    60 x 4,096 x 2,048 62 -> 19, in four parts 15; 20 x 1,024 x 3,072 in four parts 33 -> 9; 100 x 1,024 x 2,048 15.8 -> 17.3, in four 10.6."""
+    best = None
+    for tile, (rows, columns, step_k, step) in enumerate(SPLIT_TILES):
+        for parts in range(1, max(1, min(most_parts, k // (2 * step_k))) + 1):
+            tiles = -(-m // rows) * -(-n // columns) * parts
+            if rows == 32:
+                full, rest = divmod(tiles, 512)
+                one = full * SPLIT_TWO_SMALL + (0.0 if rest == 0 else step if rest <= 256 else SPLIT_TWO_SMALL)
+            else:
+                one = -(-tiles // 256) * step
+            us = 4.5 + max(-(-(-(-k // step_k)) // parts) * one, n * k * 4 / 4.5e6) + (parts - 1) * (m * n * 8 / 4.5e6 + 0.5)
+            if best is None or us < best[0]:
+                best = (us, tile, parts)
+    return best[1], best[2]
+
+
+def gemm_split(a: Tensor, b: Tensor, parts: int, tile: int, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+    """float32 partial sums [parts, M, N] of a[M, K] @ b[N, K]^T over runs of whole steps of K (given ``out`` [M, N], the product with
+    the bias there), each operand as three bfloat16 numbers whose sum it is.  ``tile``: the block's, see ``SPLIT_TILES``."""
+    _gpu(a, "a", torch.float32, contiguous=False)
+    _gpu(b, "b", torch.float32, contiguous=False)
+    if not _split_fits(a, b) or not 0 <= tile < len(SPLIT_TILES) or not 1 <= parts <= 64 or (parts > 1 and (bias is not None or out is not None)):
+        raise KernelError("the product of split operands takes float32 rows 16 bytes aligned, K a multiple of four from 256, and a bias or a place in one part")
+    m, k = a.shape
+    n = b.shape[0]
+    if out is not None and _gpu(out, "out", torch.float32).shape != (m, n):
+        raise KernelError(f"out must be [{m}, {n}], got {tuple(out.shape)}")
+    if bias is not None and _gpu(bias, "bias", torch.float32).shape != (n,):
+        raise KernelError(f"bias must be [{n}]")
+    result = torch.empty((parts, m, n), dtype=torch.float32, device=a.device) if out is None else out
+    _call("gemm_split", "fe_gemm_split", _ptr(a), _ptr(b), _ptr(bias), _ptr(result), c_int(m), c_int(n), c_int(k),
+          c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile), _stream())
+    return result
+
+
 def gemm_nt_f32(a: Tensor, b: Tensor, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
     """out[M, N] = a[M, K] @ b[N, K]^T (+ bias), true float32: FMAs, and beyond the rows of a decode step
-    the matrix cores' float32 instruction, whose products and sums stay in 32 bits."""
+    the matrix cores, whose products and sums stay in 32 bits (``gemm_split``, or for a short K the float32 instruction)."""
     _gpu(a, "a", torch.float32, contiguous=False)
     _gpu(b, "b", torch.float32, contiguous=False)
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[1]:
@@ -218,6 +277,8 @@ def gemm_nt_f32(a: Tensor, b: Tensor, bias: Tensor | None = None, out: Tensor | 
         _gpu(bias, "bias", torch.float32)
         if bias.shape != (n,):
             raise KernelError(f"bias must be [{n}]")
+    if m > SPLIT_MIN_ROWS_F32 and _split_fits(a, b) and out.data_ptr() % 4 == 0:
+        return gemm_split(a, b, 1, _split_plan(m, n, k, 1)[0], bias, out)
     lda = a.stride(0) if m > 1 else max(k, a.stride(0))
     ldb = b.stride(0) if n > 1 else max(k, b.stride(0))
     _call("gemm_f32", "fe_gemm_nt_f32", _ptr(a), _ptr(b), _ptr(bias), _ptr(out), c_int(m), c_int(n),
@@ -323,7 +384,12 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
     _gpu(weight, "weight", contiguous=False)
     out_dtype = x.dtype if out_dtype is None else out_dtype
     if weight.dtype == torch.float32:
-        y = gemm_nt_f32(x if x.dtype == torch.float32 else x.float(), weight, bias)
+        x = x if x.dtype == torch.float32 else x.float()
+        if SPLIT_MIN_ROWS < x.shape[0] <= SPLIT_MIN_ROWS_F32 and _split_fits(x, weight) and (bias is None or bias.dtype == torch.float32):
+            y = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
+            gemm_split(x, weight, 1, _split_plan(x.shape[0], *weight.shape, 1)[0], bias, y)
+        else:
+            y = gemm_nt_f32(x, weight, bias)
         return y if out_dtype == torch.float32 else y.to(out_dtype)
     if x.dtype != weight.dtype:
         raise KernelError(f"activation {x.dtype} does not match weight {weight.dtype}")
@@ -820,6 +886,9 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
     sum in the same order, stream + (x @ weight^T)."""
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
+    if bias is None and x.shape[0] > SPLIT_MIN_ROWS and _split_fits(x, weight):
+        tile, parts = _split_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS)
+        return gemm_split(x, weight, parts, tile)
     plain_bf16 = bias is None and weight.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
     if plain_bf16 and _lds_fits(x, weight):
         plan = _lds_update(x.shape[0], *weight.shape)
@@ -1524,7 +1593,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

@@ -178,6 +178,65 @@ def test_gemm_f32_tiles(ops, m, n, k, tile):
     assert torch.equal(got, again)
 
 
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("m,n,k,parts", [(1, 1, 256, 1), (31, 33, 260, 1), (97, 161, 316, 2), (129, 65, 1028, 3), (128, 320, 576, 4), (193, 129, 260, 30)])
+def test_gemm_split(ops, tile, m, n, k, parts):
+    """Operands as three bfloat16 numbers each: edges of every tile, K that ends inside a step, inside one's half and with one, parts
+    without steps, rows with a stride.  The sums of 32 products and the sums of those are float32: |error| <= 2 k 2^-24 sum |a||b|
+    as for any order of float32 products; a row with infinities, NaN, or numbers that round to an infinity of bfloat16 spoils itself
+    only and is what float32 makes it."""
+    g = torch.Generator().manual_seed(m * 31 + n)
+    a, b, bias = rand(g, m, k + 4).to(DEV), rand(g, n, k + 8).to(DEV), rand(g, n).to(DEV)
+    a *= torch.logspace(-3, 3, m, device=DEV)[:, None]
+    if m > 4:
+        a[1, k - 1], a[2, 3], a[3, 0], a[4, 7] = math.inf, math.nan, 3.4e38, -3.4028234e38
+        b[:, 0] *= 1e-3
+        b[:, 7] *= 1e-3
+    x, y = a[:, :k], b[:, :k]
+    got = ops.gemm_split(x, y, parts, tile)
+    assert got.shape == (parts, m, n)
+    want = x.double() @ y.double().t()
+    most = (x.double().abs() @ y.double().abs().t()) * (2 * k + 2 * parts) * 2.0 ** -24
+    total = got.double().sum(0)
+    plain = torch.ones(m, dtype=torch.bool, device=DEV)
+    if m > 4:
+        plain[1:3] = False
+        assert torch.equal(total[1], want[1].float().double()) and bool(total[2].isnan().all())
+    assert bool(((total - want).abs() <= most)[plain].all())
+    assert torch.equal(got, ops.gemm_split(x, y, parts, tile)) or m > 4
+    if parts == 1:
+        out = torch.empty(m, n, device=DEV)
+        ops.gemm_split(x, y, 1, tile, bias, out)
+        assert bool(((out.double() - want - bias.double()).abs() <= most + (want.abs() + bias.double().abs()) * 2.0 ** -24)[plain].all())
+
+
+def test_gemm_split_loses_nothing_of_an_operand(ops):
+    """Numbers whose 24 bits all count, times one, over fourteen orders of magnitude: the number itself."""
+    g = torch.Generator().manual_seed(5)
+    a = (rand(g, 70, 256) * 10.0 ** (torch.arange(256) % 15 - 7)).to(DEV)
+    assert torch.equal(ops.gemm_split(a, torch.eye(256, device=DEV), 1, 4)[0], a)
+    assert torch.equal(ops.gemm_split(torch.eye(256, device=DEV), a, 1, 1)[0], a.t())
+
+
+def test_gemm_split_refuses_and_routes(ops, monkeypatch):
+    a, b = torch.zeros(70, 1024, device=DEV), torch.zeros(512, 1024, device=DEV)
+    for bad in (lambda: ops.gemm_split(a, b, 1, 7), lambda: ops.gemm_split(a, b, 65, 0), lambda: ops.gemm_split(a, b, 2, 0, torch.zeros(512, device=DEV)),
+                lambda: ops.gemm_split(a[:, 1:1021], b[:, :1020], 1, 0), lambda: ops.gemm_split(a[:, :252], b[:, :252], 1, 0),
+                lambda: ops.gemm_split(a, b.bfloat16(), 1, 0), lambda: ops.gemm_split(a, b, 1, 0, None, torch.zeros(70, 511, device=DEV))):
+        with pytest.raises(ops.KernelError):
+            bad()
+    taken = []
+    real = ops.gemm_split
+    monkeypatch.setattr(ops, "gemm_split", lambda *args, **kw: taken.append("split") or real(*args, **kw))
+    for rows, k, kind, own in ((65, 256, "nt", True), (64, 256, "nt", False), (65, 252, "nt", False), (65, 258, "nt", False), (17, 1024, "linear", True),
+                               (16, 1024, "linear", False), (64, 1024, "linear", True), (17, 1024, "update", True), (16, 1024, "update", False)):
+        x, w = torch.randn(rows, k, device=DEV), torch.randn(300, k, device=DEV)
+        taken.clear()
+        got = {"nt": ops.gemm_nt_f32, "linear": ops.linear, "update": ops.linear_update}[kind](x, w)
+        assert bool(taken) == own, (rows, k, kind)
+        torch.testing.assert_close((got.sum(0) if got.dim() == 3 else got).double(), x.double() @ w.double().t(), atol=1e-3, rtol=1e-5)
+
+
 def test_gemm_f32_is_true_float32(ops):
     # operands whose product needs more than bfloat16's or tf32's mantissa
     a = torch.tensor([[1.0 + 2**-20, 1.0]])

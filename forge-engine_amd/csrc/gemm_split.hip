@@ -1,9 +1,5 @@
 // float32 matrix product C[M,N] = A[M,K] * B[N,K]^T (+ bias[N]) of more rows than a decode step, on the matrix cores' bfloat16
-// instruction: every operand is the sum of three bfloat16 numbers, x = x0 + x1 + x2 exactly (24 bits of a float32 are three times
-// eight; each part the rounding of what the parts before leave), and of the nine products of the parts the six largest are
-// added up in float32, x0 y0 + x0 y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0.  The three left out are below 2^-25 of |x y| together,
-// half a last bit, where a product rounded to float32 itself is off by as much; what a sum loses otherwise is the rounding of
-// the sums, of which there are fewer: six of 32 products each for 32 of K, where the float32 instruction makes eight of four.
+// instruction, each operand in three bfloat16 parts (split_f32.h).
 //
 // The float32 MFMA does 154 TFLOP/s here, the bfloat16 one 1,440, which six products make 240.  What bounds this kernel is that, the
 // splitting (3.5 instructions an element: a conversion of two, and a dot product with (-1, 0) that subtracts a part exactly) and
@@ -14,12 +10,10 @@
 // `global_load_lds_dwordx4` straight from memory as float32, waited for by count; a wave splits the fragments that it reads.
 // Large tiles have two groups that alternate, one splitting while the other multiplies (96 x 128 tiles of the product above 49 -> 43
 // us); small ones, bound by latency, four groups that do the same at the same time (32 x 32, 20 rows: 12.2 -> 10.5).
-// Measured on one MI355X against the float32 MFMA: 700 x 4,096 x 1,024 63 -> 43 us, 700 x 12,288 x 2,048 333 -> 239, 1,024 x 4,096 x
-// 2,048 152 -> 103 (167 TFLOP/s), and against the weight streamed past registers once for every eight rows 60 x 4,096 x 1,024
-// 52 -> 11.  Error against 64 bits 3.4e-7 of 4.1e-7 (700 x 4,096 x 1,024).
-//
-// A part of a number that is infinite, or rounds to that, is no number, and so is every sum that it is part of: a result that is not
-// finite is made again in float32 alone, product by product.  Numbers below 2^-110 lose bits of their last part.
+// Measured on one MI355X against the float32 MFMA: 700 x 4,096 x 1,024 63 -> 48 us, 700 x 6,144 x 1,024 98 -> 71, 1,024 x 4,096 x
+// 2,048 152 -> 110 (156 TFLOP/s), and against the weight streamed past registers once for every eight rows 60 x 4,096 x 1,024
+// 52 -> 11.  Error against 64 bits 1.5e-7 of 4.1e-7 (700 x 4,096 x 1,024).
+#include "split_f32.h"
 #include "lds_tile.h"
 
 namespace {
@@ -29,34 +23,8 @@ using lds_tile::floatx4;
 using lds_tile::uintx4;
 using lds_tile::load_to_lds;
 using lds_tile::wait_loads;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 
 constexpr int XCDS = 8;
-
-// two floats as three pairs of bfloat16; minus: (-1, 0) and (0, -1), which the compiler must not see (it takes -1.0 for a pair of them)
-__device__ __forceinline__ void split2(float x0, float x1, bf16x2 minus0, bf16x2 minus1, unsigned& high, unsigned& middle, unsigned& low) {
-  const bf16x2 h = {(__bf16)x0, (__bf16)x1};
-  const float r0 = __builtin_amdgcn_fdot2_f32_bf16(h, minus0, x0, false), r1 = __builtin_amdgcn_fdot2_f32_bf16(h, minus1, x1, false);
-  const bf16x2 m = {(__bf16)r0, (__bf16)r1};
-  const float s0 = __builtin_amdgcn_fdot2_f32_bf16(m, minus0, r0, false), s1 = __builtin_amdgcn_fdot2_f32_bf16(m, minus1, r1, false);
-  const bf16x2 l = {(__bf16)s0, (__bf16)s1};
-  high = __builtin_bit_cast(unsigned, h);
-  middle = __builtin_bit_cast(unsigned, m);
-  low = __builtin_bit_cast(unsigned, l);
-}
-__device__ __forceinline__ void split8(floatx4 u, floatx4 v, bf16x2 minus0, bf16x2 minus1, bf16x8 (&parts)[3]) {
-  uintx4 p[3];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    unsigned a, b, c;
-    split2(u[2 * e], u[2 * e + 1], minus0, minus1, a, b, c);
-    p[0][e] = a; p[1][e] = b; p[2][e] = c;
-    split2(v[2 * e], v[2 * e + 1], minus0, minus1, a, b, c);
-    p[0][2 + e] = a; p[1][2 + e] = b; p[2][2 + e] = c;
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) parts[i] = __builtin_bit_cast(bf16x8, p[i]);
-}
 
 template <int MI, int NI, int WM, int WN, int STAGES, int KG>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_split_kernel(
@@ -98,10 +66,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_split_kernel(
   };
 
   const int r = lane & 15, q = lane >> 4, group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  unsigned low_minus = 0x0000bf80u, high_minus = 0xbf800000u;
-  asm("" : "+s"(low_minus));
-  asm("" : "+s"(high_minus));
-  const bf16x2 minus0 = __builtin_bit_cast(bf16x2, low_minus), minus1 = __builtin_bit_cast(bf16x2, high_minus);
+  const split_f32::Minus minus = split_f32::minus();
   floatx4 acc[MI][NI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -119,28 +84,16 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_split_kernel(
         if (step * BK + c * 4 >= K) u = floatx4{0.f, 0.f, 0.f, 0.f};
         if (step * BK + c * 4 + 16 >= K) v = floatx4{0.f, 0.f, 0.f, 0.f};
       }
-      split8(u, v, minus0, minus1, parts);
+      split_f32::split8(u, v, minus, parts);
     };
 #pragma unroll
     for (int i = 0; i < MI; ++i) fragment((wm * MI + i) * 16 + r, a[i]);
 #pragma unroll
     for (int j = 0; j < NI; ++j) fragment(BM + (wn * NI + j) * 16 + r, b[j]);
   };
-  // The products of 32 of K are added up by themselves first, the smallest at first, so that the long sum is rounded once for them
-  // and not six times (700 x 4,096 x 1,024: error 3.4e-7 without, 1.6e-7).
   auto multiply = [&]() {
-    constexpr int OF_A[6] = {2, 0, 1, 1, 0, 0}, OF_B[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      floatx4 sum[MI];
-#pragma unroll
-      for (int p = 0; p < 6; ++p)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-          sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j][OF_B[p]], a[i][OF_A[p]], p == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : sum[i], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < MI; ++i) acc[i][j] += sum[i];
-    }
+    for (int j = 0; j < NI; ++j) split_f32::add_products<MI>(a, b[j], [&](int i) -> floatx4& { return acc[i][j]; });
   };
   auto barrier = []() {
     __builtin_amdgcn_sched_barrier(0);
@@ -222,15 +175,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_split_kernel(
     for (int j = 0; j < NI; ++j) {
       const int n = n0 + (wn * NI + j) * 16 + 4 * q;
       floatx4 v = acc[i][j];
-      const float largest = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-      if (!(largest <= 3.4028234663852886e38f) || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]) {
-        for (int e = 0; e < 4 && n + e < N; ++e) {
-          const float *x = A + (size_t)m * lda, *y = B + (size_t)(n + e) * ldb;
-          float sum = 0.f;
-          for (int k = first * BK; k < min(K, steps * BK); ++k) sum = __fmaf_rn(x[k], y[k], sum);
-          v[e] = sum;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!split_f32::finite(v[e]) && n + e < N) {
+          const int k = first * BK;
+          v[e] = split_f32::dot(A + (size_t)m * lda + k, B + (size_t)(n + e) * ldb + k, min(K, steps * BK) - k);
         }
-      }
       float* dst = C + (size_t)part * part_stride + (size_t)m * ldc + n;
       if (bias)
         for (int e = 0; e < 4; ++e) if (n + e < N) v[e] += bias[n + e];

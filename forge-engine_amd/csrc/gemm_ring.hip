@@ -20,11 +20,17 @@
 // 2,048 x 2,048 stored at 8 rows 4.6 -> 3.9 us, 6,144 x 2,048 gated 12.4 -> 11.8, of K = 4,096 25.1 -> 20.1; the same steps 793 -> 768 us
 // and 2,297 -> 2,262.
 //
+// float32 operands go through the same rings, 32 of K a chunk, and through the bfloat16 instruction in three parts each (split_f32.h).
+// At 4 rows, product, norm or gate in launches of their own before: 2,048 x 2,048 with its norm 11 -> 7.5 us, 2,048 x 6,144 17 -> 16 (the
+// splitting of 16 rows where 8 are a block's), 3,072 gated columns of K = 1,024 12.3 -> 7.9, 6,144 of 2,048 24 -> 20.7; 16 rows, which
+// took the weight twice, 42 -> 20.7.
+//
 // MFMA 16x16x32 bf16 with A = W, B = x^T: lane l (r = l % 16, q = l / 16) supplies row r, k = 8 q .. + 8 of either and receives
 // D[weight row 4 q + i][row of x r].  Rows of either tile that the block has not (weight rows of its neighbour, rows of x beyond
 // M) are not fetched: what lies in LDS there only reaches sums that are not stored.
 #include "gate_act.h"
 #include "lds_tile.h"
+#include "split_f32.h"
 
 namespace {
 
@@ -34,7 +40,7 @@ using lds_tile::uintx4;
 using lds_tile::load_to_lds;
 using lds_tile::wait_loads;
 
-constexpr int WAVES = 8, CHUNK = 64, SQUARES = 256;
+constexpr int WAVES = 8, SQUARES = 256;
 constexpr int UPDATE = 0, FLOAT = 1, BFLOAT = 2, GATED = 3;
 
 // XI, WI: requests of eight rows a chunk for x and for the weight
@@ -47,9 +53,9 @@ struct Ring {
 };
 
 struct Ending {
-  float* h;                 // UPDATE: the stream, the norm's weight, what is left of the norm
+  float* h;                 // UPDATE: the stream, the norm's weight, what is left of the norm (of the operands' type)
   const float* weight;
-  bf16_t* y;
+  void* y;
   float* squares;
   void* out;                // the others: [M, N], row stride N
   const float* row_squares; // SCALED: [M][256], the factors' row length and eps
@@ -57,10 +63,12 @@ struct Ending {
   GateAct act;
 };
 
-template <int XI, int WI, int END, bool SCALED>
+template <typename T, int XI, int WI, int END, bool SCALED>
 __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, Ending ending, int M, int N, int K, long long ldw, int block_rows) {
+    const T* __restrict__ x, const T* __restrict__ w, Ending ending, int M, int N, int K, long long ldw, int block_rows) {
   using R = Ring<XI, WI, SCALED>;
+  constexpr bool WIDE = sizeof(T) == 4;
+  constexpr int CHUNK = 128 / sizeof(T), PIECE = 16 / sizeof(T);      // elements of a row's 128 bytes, and of 16
   constexpr int TILES = R::TILES, PAIR = END == GATED ? 2 : 1;
   constexpr int VALUES = TILES * 256 / PAIR;          // results of a block, one a thread
   static_assert(VALUES <= 64 * WAVES && (END != GATED || WI % 2 == 0), "a thread a result");
@@ -95,8 +103,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   const int chunks = K / CHUNK, count = (chunks - wave + WAVES - 1) / WAVES;       // this wave's chunks: wave, wave + 8, ..
   const unsigned int base = lds_at + wave * R::WAVE_BYTES;
   // a request: eight rows of 128 bytes, 16-byte piece c of a row at c ^ (row % 8)
-  const int of_group = lane >> 3, at = wave * CHUNK + ((lane & 7) ^ of_group) * 8;
-  const bf16_t *x_from[XI], *w_from[WI];
+  const int of_group = lane >> 3, at = wave * CHUNK + ((lane & 7) ^ of_group) * PIECE;
+  const T *x_from[XI], *w_from[WI];
   bool x_has[XI], w_has[WI];
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
@@ -124,7 +132,14 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   floatx4 acc[TILES];
 #pragma unroll
   for (int t = 0; t < TILES; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // float32 operands: the products of the first parts, added to the whole every four chunks, and all others, a 2^8th of their size: so
+  // the long sum is rounded a quarter as often and a long K costs no accuracy
+  floatx4 large[TILES], small[TILES];
+  int turn = 0;
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) large[t] = small[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   const uintx4* ring = lds + wave * (R::WAVE_BYTES / 16);
+  const split_f32::Minus minus = split_f32::minus();
   uintx4 a[2], b[TILES][2];
   auto fragments = [&](int stage) {
     const uintx4* from = ring + stage * R::LOADS * 64;
@@ -138,6 +153,21 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before the buffer is filled again
   };
   auto multiply = [&]() {
+    if constexpr (WIDE) {       // the two pieces are a lane's eight elements of 32
+      bf16x8 x_parts[1][3], w_parts[3];
+      split_f32::split8(__builtin_bit_cast(floatx4, a[0]), __builtin_bit_cast(floatx4, a[1]), minus, x_parts[0]);
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        split_f32::split8(__builtin_bit_cast(floatx4, b[t][0]), __builtin_bit_cast(floatx4, b[t][1]), minus, w_parts);
+        split_f32::add_products_apart(x_parts[0], w_parts, large[t], small[t]);
+        if (turn == 3) {
+          acc[t] += large[t];
+          large[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      turn = (turn + 1) & 3;
+      return;
+    }
 #pragma unroll
     for (int half = 0; half < 2; ++half)
 #pragma unroll
@@ -183,13 +213,17 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   // the waves' sums meet, each in its wave's own ring, which nobody else reads and which it has emptied
   floatx4* meet = (floatx4*)(lds + wave * (R::WAVE_BYTES / 16));
 #pragma unroll
-  for (int t = 0; t < TILES; ++t) meet[t * 64 + lane] = acc[t];
+  for (int t = 0; t < TILES; ++t) meet[t * 64 + lane] = WIDE ? acc[t] + (large[t] + small[t]) : acc[t];
   __syncthreads();
-  auto total = [&](int lane_group) {
+  auto total = [&](int lane_group) {       // of the eight columns' gate or up rows, or of all sixteen: lane group of the tile
     const float* from = (const float*)lds + tile * 256 + (lane_group * 16 + row) * 4 + (tid & 3);
     float sum = 0.f;
 #pragma unroll
     for (int v = 0; v < WAVES; ++v) sum += from[v * (R::WAVE_BYTES / 4)];
+    if constexpr (WIDE) {
+      if (!split_f32::finite(sum) && mine)
+        sum = split_f32::dot(x + (size_t)row * K, w + (size_t)(n0 + column + (lane_group != group ? N : 0)) * ldw, K);
+    }
     return sum;
   };
   if constexpr (END == UPDATE) {
@@ -201,7 +235,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
       if ((tid & 3) == 0) per_row[tid >> 6][row] = square;
       if (mine) {
         ending.h[place] = sum;
-        ending.y[place] = float_to_bf16(sum * gain);
+        store_from_float((T*)ending.y + place, sum * gain);
       }
     }
     __syncthreads();
@@ -220,7 +254,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
     if constexpr (END == GATED) {
       float up = total(group + 2);
       if (SCALED) up *= factor;
-      ((bf16_t*)ending.out)[place] = float_to_bf16(gate_times(sum, up, ending.act));
+      if constexpr (WIDE) ((float*)ending.out)[place] = gate_times_exact(sum, up, ending.act);
+      else ((bf16_t*)ending.out)[place] = float_to_bf16(gate_times(sum, up, ending.act));
     } else if constexpr (END == FLOAT) {
       ((float*)ending.out)[place] = sum;
     } else {
@@ -229,21 +264,21 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   }
 }
 
-template <int XI, int WI, int END, bool SCALED>
+template <typename T, int XI, int WI, int END, bool SCALED>
 int launch(const void* x, const void* w, const Ending& ending, int M, int N, int K, long long ldw, int block_rows, hipStream_t stream) {
   static std::atomic<bool> raised{false};
-  auto kernel = gemm_ring_kernel<XI, WI, END, SCALED>;
+  auto kernel = gemm_ring_kernel<T, XI, WI, END, SCALED>;
   const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, Ring<XI, WI, SCALED>::BYTES, &raised);
   if (limit_raised != FE_OK) return limit_raised;
   kernel<<<(N + block_rows - 1) / block_rows, 64 * WAVES, Ring<XI, WI, SCALED>::BYTES, stream>>>(
-      (const bf16_t*)x, (const bf16_t*)w, ending, M, N, K, ldw, block_rows);
+      (const T*)x, (const T*)w, ending, M, N, K, ldw, block_rows);
   return fe_check_launch();
 }
 
-template <int END, bool SCALED>
+template <typename T, int END, bool SCALED>
 int pick(const void* x, const void* w, const Ending& ending, int M, int N, int K, long long ldw, hipStream_t stream) {
   const int block_rows = (N + SQUARES - 1) / SQUARES;
-#define FE_PICK(XI, WI) return launch<XI, WI, END, SCALED>(x, w, ending, M, N, K, ldw, block_rows, stream)
+#define FE_PICK(XI, WI) return launch<T, XI, WI, END, SCALED>(x, w, ending, M, N, K, ldw, block_rows, stream)
   const int groups = (block_rows + 7) / 8;
   if constexpr (END == GATED) {
     switch (groups) {
@@ -263,41 +298,48 @@ int pick(const void* x, const void* w, const Ending& ending, int M, int N, int K
   return FE_BAD_ARGUMENT;
 }
 
-bool operands_fit(const void* x, const void* w, int M, int N, int K, long long ldw) {
-  return M <= 16 && N >= 1 && K >= CHUNK && K % CHUNK == 0 && ldw >= K && ldw % 8 == 0 && x && w && ((((uintptr_t)x) | ((uintptr_t)w)) & 15) == 0;
+bool operands_fit(const void* x, const void* w, int dtype, int M, int N, int K, long long ldw) {
+  if (dtype != FE_F32 && dtype != FE_BF16) return false;
+  const int chunk = dtype == FE_F32 ? 32 : 64, piece = dtype == FE_F32 ? 4 : 8;
+  return M <= 16 && N >= 1 && K >= chunk && K % chunk == 0 && ldw >= K && ldw % piece == 0 && x && w && ((((uintptr_t)x) | ((uintptr_t)w)) & 15) == 0;
 }
 
 }  // namespace
 
-// x [M, K] bfloat16, contiguous, 1 <= M <= 16, K a multiple of 64; w [N, K] bfloat16 with row stride ldw, rows 16-byte aligned, N up to
-// 8,192; h [M, N] float32, contiguous, is replaced by h + x w^T; weight [N] float32; y [M, N] bfloat16; squares [M][256] float32,
-// whose sum over a row is that row's sum of squares of the new h (entries beyond the blocks are zero).
-extern "C" int fe_gemm_update_norm(const void* x, const void* w, float* h, const float* weight, void* y, float* squares, int M,
-                                   int N, int K, long long ldw, hipStream_t stream) {
+// x [M, K], contiguous, 1 <= M <= 16, and w [N, K] with row stride ldw, rows 16-byte aligned, N up to 8,192: bfloat16, K a multiple of
+// 64, or float32, K a multiple of 32; h [M, N] float32, contiguous, is replaced by h + x w^T; weight [N] float32; y [M, N] of x's type;
+// squares [M][256] float32, whose sum over a row is that row's sum of squares of the new h (entries beyond the blocks are zero).
+extern "C" int fe_gemm_update_norm(const void* x, const void* w, int dtype, float* h, const float* weight, void* y, float* squares,
+                                   int M, int N, int K, long long ldw, hipStream_t stream) {
   if (M < 1) return FE_OK;
-  if (!operands_fit(x, w, M, N, K, ldw) || N > 32 * SQUARES || !h || !weight || !y || !squares) return FE_BAD_ARGUMENT;
-  return pick<UPDATE, false>(x, w, {h, weight, (bf16_t*)y, squares, nullptr, nullptr, 0.f, 0.f, {}}, M, N, K, ldw, stream);
+  if (!operands_fit(x, w, dtype, M, N, K, ldw) || N > 32 * SQUARES || !h || !weight || !y || !squares) return FE_BAD_ARGUMENT;
+  const Ending how = {h, weight, y, squares, nullptr, nullptr, 0.f, 0.f, {}};
+  if (dtype == FE_F32) return pick<float, UPDATE, false>(x, w, how, M, N, K, ldw, stream);
+  return pick<bf16_t, UPDATE, false>(x, w, how, M, N, K, ldw, stream);
 }
 
-// The same operands; ending 1: out [M, N] float32, 2: bfloat16 (N up to 8,192), 3: out [M, N] bfloat16 = act(x gate^T) * (x up^T) for a
-// fused weight [2 N, K], gate rows first (N up to 6,144; act by `activation`, gate_act.h).  squares (null: none) [M][256] float32: the
-// sums of row m are multiplied by rsqrt(sum of squares[m] / K + eps) before anything else is done with them.
-extern "C" int fe_gemm_ring(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, int ending, int activation,
-                            const float* squares, float eps, hipStream_t stream) {
+// The same operands; ending 1: out [M, N] float32, 2: bfloat16, of bfloat16 operands (N up to 8,192), 3: out [M, N] of x's type =
+// act(x gate^T) * (x up^T) for a fused weight [2 N, K], gate rows first (N up to 6,144; act by `activation`, gate_act.h).  squares
+// (null: none) [M][256] float32: the sums of row m are multiplied by rsqrt(sum of squares[m] / K + eps) before anything else is done
+// with them.
+extern "C" int fe_gemm_ring(const void* x, const void* w, int dtype, void* out, int M, int N, int K, long long ldw, int ending,
+                            int activation, const float* squares, float eps, hipStream_t stream) {
   if (M < 1) return FE_OK;
   GateAct act;
   if (!gate_act(activation, &act)) return FE_BAD_ARGUMENT;
-  if (!operands_fit(x, w, M, N, K, ldw) || !out || N > (ending == GATED ? 24 : 32) * SQUARES) return FE_BAD_ARGUMENT;
+  if (!operands_fit(x, w, dtype, M, N, K, ldw) || !out || N > (ending == GATED ? 24 : 32) * SQUARES) return FE_BAD_ARGUMENT;
   if (squares && (!(eps > 0.f) || (((uintptr_t)squares) & 15))) return FE_BAD_ARGUMENT;
   const Ending how = {nullptr, nullptr, nullptr, nullptr, out, squares, (float)K, eps, act};
-#define FE_PICK(END)                                                             \
-  if (ending == END) {                                                           \
-    if (squares) return pick<END, true>(x, w, how, M, N, K, ldw, stream);        \
-    return pick<END, false>(x, w, how, M, N, K, ldw, stream);                    \
+#define FE_PICK(TYPE, T, END)                                                       \
+  if (dtype == TYPE && ending == END) {                                             \
+    if (squares) return pick<T, END, true>(x, w, how, M, N, K, ldw, stream);        \
+    return pick<T, END, false>(x, w, how, M, N, K, ldw, stream);                    \
   }
-  FE_PICK(FLOAT)
-  FE_PICK(BFLOAT)
-  FE_PICK(GATED)
+  FE_PICK(FE_BF16, bf16_t, FLOAT)
+  FE_PICK(FE_BF16, bf16_t, BFLOAT)
+  FE_PICK(FE_BF16, bf16_t, GATED)
+  FE_PICK(FE_F32, float, FLOAT)
+  FE_PICK(FE_F32, float, GATED)
 #undef FE_PICK
   return FE_BAD_ARGUMENT;
 }

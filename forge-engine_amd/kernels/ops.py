@@ -369,7 +369,7 @@ def _few_rows_library_pays(rows: int, weight: Tensor) -> bool:
             and weight.shape[0] * weight.shape[1] * weight.element_size() > IN_PARTS_MAX_WEIGHT_BYTES)
 
 
-def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None) -> Tensor:
+def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None, out_dtype=None) -> Tensor:
     """y = x @ weight^T (+ bias) for a weight in [out, in] layout; float32
     accumulation; y in ``out_dtype`` (default: x's dtype).
 
@@ -380,12 +380,18 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, out_dtype=None
     rest is the platform's matrix library's, which the reference uses for every
     projection (its nn.Linear calls, qwen3.py:115-122,215-223).
     """
+    if isinstance(x, UnscaledRows):
+        if bias is not None or out_dtype not in (None, x.rows.dtype) or not unscaled_linear(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
+            raise KernelError("rows without their norm's factors are for the products through LDS only")
+        return gemm_ring(x, weight, "f32" if weight.dtype == torch.float32 else "bf16")
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     out_dtype = x.dtype if out_dtype is None else out_dtype
     if weight.dtype == torch.float32:
         x = x if x.dtype == torch.float32 else x.float()
-        if SPLIT_MIN_ROWS < x.shape[0] <= SPLIT_MIN_ROWS_F32 and _split_fits(x, weight) and (bias is None or bias.dtype == torch.float32):
+        if bias is None and _ring_fits(x, weight, "f32") and _ring_float32_pays(x.shape[0], *weight.shape):
+            y = gemm_ring(x, weight, "f32")
+        elif SPLIT_MIN_ROWS < x.shape[0] <= SPLIT_MIN_ROWS_F32 and _split_fits(x, weight) and (bias is None or bias.dtype == torch.float32):
             y = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
             gemm_split(x, weight, 1, _split_plan(x.shape[0], *weight.shape, 1)[0], bias, y)
         else:
@@ -719,7 +725,7 @@ class UpdateProduct(NamedTuple):
 
 
 class UnscaledRows(NamedTuple):
-    """Rows of a norm without its factors: bfloat16(h * weight) [M, N], and what the factor of row m is made of:
+    """Rows of a norm without its factors: h * weight [M, N] in the compute dtype, and what the factor of row m is made of:
     rsqrt(sum of squares[m] / N + eps), squares [M, 256] float32."""
 
     rows: Tensor
@@ -736,10 +742,18 @@ def update_norm_fits(x: Tensor, weight: Tensor) -> bool:
     launches -> one: 1,024 x 2,048 at 1 / 16 rows 5.4 -> 3.2 / 6.1 -> 3.9, 2,048 x 6,144 9.5 -> 7.0 / 9.9 -> 8.6, 2,560 x 9,728 13.7 ->
     11.2 / 13.8 -> 13.3, 5,120 x 25,600 51 -> 48 / 50 -> 49, 8,192 x 4,096 18.6 -> 15.9 / 22 -> 16 (wider ones would need more
     rows a block; 8,192 x 8,192 at 1 row alone is slower, 30.8 -> 32.5, at 8 38.6 -> 31.0)."""
-    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
-            and 0 < x.shape[0] <= SKINNY_MAX_ROWS and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
-            and weight.shape[0] <= UPDATE_NORM_MAX_WIDTH and x.shape[1] % 64 == 0 and weight.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+    return _ring_operands_fit(x, weight) and weight.shape[0] <= UPDATE_NORM_MAX_WIDTH
+
+
+def _ring_operands_fit(x: Tensor, weight: Tensor) -> bool:
+    return (x.dtype == weight.dtype and x.dim() == 2 and x.is_contiguous() and 0 < x.shape[0] <= SKINNY_MAX_ROWS
+            and weight.dim() == 2 and weight.shape[1] == x.shape[1] and _ring_weight_fits(weight) and x.data_ptr() % 16 == 0)
+
+
+def _ring_weight_fits(weight: Tensor) -> bool:
+    piece = {torch.bfloat16: 8, torch.float32: 4}.get(weight.dtype)
+    return (piece is not None and weight.dim() == 2 and weight.shape[0] > 0 and weight.shape[1] > 0 and weight.shape[1] % (8 * piece) == 0
+            and weight.stride(1) == 1 and weight.stride(0) % piece == 0 and weight.data_ptr() % 16 == 0)
 
 
 def update_norm(h: Tensor, product: UpdateProduct, norm_weight: Tensor, eps: float) -> UnscaledRows:
@@ -747,14 +761,14 @@ def update_norm(h: Tensor, product: UpdateProduct, norm_weight: Tensor, eps: flo
     x, weight = product
     _gpu(h, "h", torch.float32)
     _gpu(norm_weight, "norm_weight", torch.float32)
-    _gpu(x, "x", torch.bfloat16)
-    _gpu(weight, "weight", torch.bfloat16, contiguous=False)
+    _gpu(x, "x")
+    _gpu(weight, "weight", contiguous=False)
     if not update_norm_fits(x, weight) or h.shape != (x.shape[0], weight.shape[0]) or norm_weight.shape != (weight.shape[0],) or not eps > 0.0:
         raise KernelError(f"no product with a norm behind it for {tuple(x.shape)} x {tuple(weight.shape)} into {tuple(h.shape)}")
     m, n = h.shape
-    rows = torch.empty((m, n), dtype=torch.bfloat16, device=h.device)
+    rows = torch.empty((m, n), dtype=x.dtype, device=h.device)
     squares = torch.empty((m, 256), dtype=torch.float32, device=h.device)
-    _call("gemm_ring", "fe_gemm_update_norm", _ptr(x), _ptr(weight), _ptr(h), _ptr(norm_weight), _ptr(rows), _ptr(squares),
+    _call("gemm_ring", "fe_gemm_update_norm", _ptr(x), _ptr(weight), c_int(_code(x.dtype)), _ptr(h), _ptr(norm_weight), _ptr(rows), _ptr(squares),
           c_int(m), c_int(n), c_int(x.shape[1]), c_longlong(weight.stride(0)), _stream())
     return UnscaledRows(rows, squares, float(eps))
 
@@ -774,6 +788,13 @@ def _ring_store_pays(rows: int, weight_rows: int, k: int) -> bool:
     return rows <= SKINNY_MAX_ROWS and k >= 320 and weight_rows <= RING_STORE_ROWS and not (rows > 4 and k >= 4096 and 3584 < weight_rows <= 4096)
 
 
+def _ring_float32_pays(rows: int, weight_rows: int, k: int) -> bool:
+    """float32, beside the weight streamed past registers once for every eight rows: 9 to 16 rows always (6,144 x 2,048 23.9 -> 12.5 us,
+    2,048 x 6,144 24.2 -> 16.5), to eight at a short K (4,096 x 1,024 7.7 -> 5.8; 2,048 x 2,048 6.9 against 7.3, x 6,144 13.0 against 16.7).
+    Error against 64 bits 0.9 to 1.0e-7 of 0.9 to 1.1e-7."""
+    return k >= SPLIT_MIN_K and (rows > 8 or (k <= 1152 and weight_rows >= 2048))
+
+
 def _ring_parts_pays(weight_rows: int, k: int) -> bool:
     """q/k/v: from 2,048 weight rows on (6,144 x 2,560 at 1 / 8 rows 7.8 -> 7.7, 7.5 -> 7.4, x 4,096 11.8 -> 11.1, 11.8 -> 10.7; 4,096 x
     2,048 5.2 against 5.5, but one sum instead of two for who adds them up); fewer rows have too few bytes a block at a long K
@@ -782,29 +803,31 @@ def _ring_parts_pays(weight_rows: int, k: int) -> bool:
 
 
 def gemm_ring(x: Tensor | UnscaledRows, weight: Tensor, ending: str, act: str = "silu") -> Tensor:
-    """x @ weight^T for up to 16 bfloat16 rows, whole sums in a block: ``"f32"`` or ``"bf16"`` [M, N] (N up to 8,192), or ``"gated"``:
-    act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first, up to 12,288 of both)."""
+    """x @ weight^T for up to 16 rows, whole sums in a block: ``"f32"`` or, of bfloat16, ``"bf16"`` [M, N] (N up to 8,192), or
+    ``"gated"``: act(gate) * up [M, N / 2] in x's dtype for a fused gate/up weight (gate rows first, up to 12,288 of both)."""
     rows, squares, eps = x if isinstance(x, UnscaledRows) else (x, None, 0.0)
-    _gpu(rows, "x", torch.bfloat16)
-    _gpu(weight, "weight", torch.bfloat16, contiguous=False)
+    _gpu(rows, "x")
+    _gpu(weight, "weight", contiguous=False)
     if not _ring_fits(rows, weight, ending):
         raise KernelError(f"no product with a ring for each wave for {tuple(rows.shape)} x {tuple(weight.shape)}, {ending!r}")
     m, k = rows.shape
     if squares is not None and _gpu(squares, "squares", torch.float32).shape != (m, 256):
         raise KernelError("rows without their norm's factors come with 256 sums of squares each")
     n = weight.shape[0] // 2 if ending == "gated" else weight.shape[0]
-    out = torch.empty((m, n), dtype=torch.float32 if ending == "f32" else torch.bfloat16, device=rows.device)
-    _call("gemm_ring", "fe_gemm_ring", _ptr(rows), _ptr(weight), _ptr(out), c_int(m), c_int(n), c_int(k), c_longlong(weight.stride(0)),
+    out = torch.empty((m, n), dtype=torch.float32 if ending == "f32" else rows.dtype, device=rows.device)
+    _call("gemm_ring", "fe_gemm_ring", _ptr(rows), _ptr(weight), c_int(_code(rows.dtype)), _ptr(out), c_int(m), c_int(n), c_int(k), c_longlong(weight.stride(0)),
           c_int({"f32": 1, "bf16": 2, "gated": 3}[ending]), _gate_act(act), _ptr(squares), c_float(eps), _stream())
     return out
 
 
-def _ring_fits(x: Tensor, weight: Tensor, ending: str) -> bool:
-    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
-            and 0 < x.shape[0] <= SKINNY_MAX_ROWS and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
-            and x.shape[1] > 0 and x.shape[1] % 64 == 0 and weight.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and weight.data_ptr() % 16 == 0 and ending in ("f32", "bf16", "gated")
-            and 0 < weight.shape[0] <= (2 * RING_GATE_COLUMNS if ending == "gated" else UPDATE_NORM_MAX_WIDTH) and (ending != "gated" or weight.shape[0] % 2 == 0))
+def _ring_fits(x: Tensor, weight: Tensor, ending: str | None) -> bool:
+    return _ring_operands_fit(x, weight) and _ring_ending_fits(weight, ending)
+
+
+def _ring_ending_fits(weight: Tensor, ending: str | None) -> bool:
+    if ending == "gated":
+        return weight.shape[0] % 2 == 0 and weight.shape[0] <= 2 * RING_GATE_COLUMNS
+    return weight.shape[0] <= UPDATE_NORM_MAX_WIDTH and (ending == "f32" or (ending == "bf16" and weight.dtype == torch.bfloat16))
 
 
 def _weight_fits_lds(weight: Tensor) -> bool:
@@ -819,12 +842,29 @@ def unscaled_in_parts(rows: int, weight: Tensor) -> bool:
             and (_ring_parts_pays(*weight.shape) or _lds_in_parts(rows, *weight.shape) is not None))
 
 
+def unscaled_linear(rows: int, weight: Tensor) -> bool:
+    """Whether ``linear`` takes ``UnscaledRows`` for a product without a bias, stored in the compute dtype."""
+    if not (0 < rows <= SKINNY_MAX_ROWS and _ring_weight_fits(weight) and weight.shape[1] >= LDS_MIN_K):
+        return False
+    if weight.dtype == torch.float32:
+        return weight.shape[0] <= UPDATE_NORM_MAX_WIDTH
+    return not _few_rows_library_pays(rows, weight) and _ring_store_pays(rows, *weight.shape)
+
+
 def unscaled_swiglu(rows: int, gate_up_weight: Tensor) -> bool:
     """Whether ``linear_swiglu`` takes ``UnscaledRows``: where it takes a product through LDS."""
+    if gate_up_weight.dtype == torch.float32:
+        return 0 < rows <= SKINNY_MAX_ROWS and _ring_gate_float32(gate_up_weight)
     return (0 < rows <= SKINNY_MAX_ROWS and _weight_fits_lds(gate_up_weight) and gate_up_weight.shape[0] % 2 == 0
             and not (rows > 1 and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS)
             and (gate_up_weight.shape[0] <= 2 * RING_GATE_COLUMNS
                  or _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])))
+
+
+def _ring_gate_float32(weight: Tensor) -> bool:
+    """Gated products of float32: wherever they fit (with the gate's kernel behind them before: 3,072 columns of K = 1,024 at 4 rows 12.3 ->
+    7.9 us, 6,144 of 2,048 23.7 -> 20.7, at 16 rows 42 -> 21)."""
+    return _ring_weight_fits(weight) and _ring_ending_fits(weight, "gated") and weight.shape[1] >= SPLIT_MIN_K
 
 
 def _gemm_lds_unscaled(x: UnscaledRows, weight: Tensor, ending: str, parts: int, tile: int, act: str) -> Tensor:
@@ -1046,6 +1086,8 @@ def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "
             and x.data_ptr() % 16 == 0 and gate_up_weight.data_ptr() % 16 == 0
             and gate_up_weight.shape[0] * gate_up_weight.stride(0) < 2 ** 32 and rows * x.shape[1] < 2 ** 32):
         return gemm_gated(x, gate_up_weight, shape=3, act=act)
+    if gate_up_weight.dtype == torch.float32 and _ring_fits(x, gate_up_weight, "gated") and _ring_gate_float32(gate_up_weight):
+        return gemm_ring(x, gate_up_weight, "gated", act)
     to_library = (2 <= rows <= SKINNY_MAX_ROWS and gate_up_weight.shape[0] > GATE_LIBRARY_WEIGHT_ROWS
                   and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16)
     # Up to 16 rows and 6,144 columns: a ring for each wave (1.41 times what took 140 random sizes before; 3,072 columns of K = 1,024 at

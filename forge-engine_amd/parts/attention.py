@@ -322,10 +322,12 @@ class GroupedQueryAttention(Mixer):
     leaves_product = True
 
     def takes_unscaled(self, tokens: int, batch, cache: CacheView, writes_cache: bool = True) -> bool:
+        if self.general or not writes_cache or self.qkv_bias is not None:
+            return False
         rotary = self.position.rotary()
-        return (not self.general and writes_cache and self.qkv_bias is None
-                and self._single_tokens_only(batch, tokens, cache, 0 if rotary is None else rotary[1])
-                and ops.unscaled_in_parts(tokens, self.qkv_weight))
+        if self._single_tokens_only(batch, tokens, cache, 0 if rotary is None else rotary[1]):
+            return ops.unscaled_in_parts(tokens, self.qkv_weight)
+        return ops.unscaled_linear(tokens, self.qkv_weight)
 
     def forward(self, x: Tensor | ops.UnscaledRows, batch, cache: CacheView, writes_cache: bool = True,
                 stream: Tensor | None = None, product: bool = False) -> Tensor | ops.UpdateProduct | None:
@@ -359,12 +361,14 @@ class GroupedQueryAttention(Mixer):
             cache.block_table, cache.key_pages, cache.value_pages, q_heads=self.num_heads,
             kv_heads=self.num_kv_heads, head_dim=self.head_dim, rotary_dim=rotary_dim, eps=eps,
             write_kv=writes_cache)
-        attn = torch.empty((x.shape[0], self.q_size), dtype=x.dtype, device=x.device)
+        attn = torch.empty((x.shape[0], self.q_size), dtype=self.ctx.dtype, device=qkv.device)
         ops.paged_attention(
             qkv, cache.key_pages, cache.value_pages, attn, batch.cu_q, batch.ctx_len, cache.block_table,
             num_seqs=batch.num_seqs, max_q_len=batch.max_q_len, q_heads=self.num_heads,
             kv_heads=self.num_kv_heads, head_dim=self.head_dim, scale=self.scale, window=self.window,
             num_decode=batch.num_decode, max_ctx=batch.max_ctx)
+        if product and self.o_bias is None and ops.update_norm_fits(attn, self.o_weight):
+            return ops.UpdateProduct(attn, self.o_weight)
         return ops.linear_update(attn, self.o_weight, self.o_bias, stream)   # float32 update for the residual sum
 
     def _forward_general(self, x: Tensor, batch, cache: CacheView, writes_cache: bool, stream, inv_freq,

@@ -1022,20 +1022,21 @@ def test_gemm_lds(ops, tile, m, n, k, parts):
 
 @pytest.mark.parametrize("m", [1, 8, 9, 16])
 @pytest.mark.parametrize("n,k", [(1, 64), (255, 448), (256, 512), (1024, 2048), (2049, 1088), (2568, 8256), (4097, 640), (6400, 4096), (8192, 1024)])
-def test_update_with_the_next_norm(ops, m, n, k):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_update_with_the_next_norm(ops, m, n, k, dtype):
     """One to thirty-two weight rows a block, last blocks with fewer, waves without chunks to walks longer than their buffers, a
     weight that is a slice of a wider one.  The stream against the exact products: |error| <= (2 k + 32) 2^-24 (|h| + sum |a||b|);
     the rows are its rounded product with the norm's weight, the squares its own to the last bits of a sum of n."""
     g = torch.Generator().manual_seed(m * n + k)
-    x = rand(g, m, k, dtype=torch.bfloat16).to(DEV)
-    w = rand(g, n, k + 64, dtype=torch.bfloat16, scale=0.05).to(DEV)[:, :k]
+    x = rand(g, m, k, dtype=dtype).to(DEV)
+    w = rand(g, n, k + 64, dtype=dtype, scale=0.05).to(DEV)[:, :k]
     h, gain = rand(g, m, n).to(DEV), rand(g, n).to(DEV)
     exact = h.double() + x.double() @ w.double().t()
     bound = (h.double().abs() + x.double().abs() @ w.double().abs().t()) * (2 * k + 32) * 2.0 ** -24
     got = h.clone()
     out = ops.update_norm(got, ops.UpdateProduct(x, w), gain, 1e-6)
     assert bool(((got.double() - exact).abs() <= bound).all())
-    assert torch.equal(out.rows, (got * gain).bfloat16())
+    assert torch.equal(out.rows, (got * gain).to(dtype))
     squares = got.double().pow(2).sum(1)
     assert bool(((out.squares.double().sum(1) - squares).abs() <= squares * 64 * 2.0 ** -24).all())
     assert out.squares.shape == (m, 256) and bool((out.squares[:, -(-n // -(-n // 256)):] == 0).all())
@@ -1062,6 +1063,54 @@ def test_gemm_ring(ops, m, n, k):
             torch.testing.assert_close(gated, ops.swiglu(exact.float().contiguous(), torch.empty(m, n, device=DEV), act), atol=2e-2, rtol=2e-2)
     one_row = ops.gemm_ring(x[:1].contiguous(), w[n:], "f32")
     assert torch.equal(one_row[0], ops.gemm_ring(x, w[n:], "f32")[0])      # a row's sums do not depend on the rows beside it
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(1, 32), (255, 224), (256, 512), (1024, 2048), (2049, 1088), (2568, 4128), (4097, 640), (6144, 1024), (8192, 96)])
+def test_gemm_ring_of_float32(ops, m, n, k):
+    """The same in float32: |error| <= (2 k + 32) 2^-24 sum |a||b| as for any order of float32 products, gated results in float32; rows with
+    an infinity, NaN or a number that rounds to an infinity of bfloat16 spoil themselves only and are what float32 makes them."""
+    g = torch.Generator().manual_seed(m * n + k)
+    x = rand(g, m, k).to(DEV) * torch.logspace(-3, 3, m, device=DEV)[:, None]
+    w = rand(g, 2 * n, k + 64, scale=0.05).to(DEV)[:, :k]
+    plain = torch.ones(m, dtype=torch.bool, device=DEV)
+    if m > 3:
+        x[1, k - 1], x[2, 3], x[3, 0] = math.inf, math.nan, 3.4e38
+        w[:, 0] *= 1e-3
+        plain[1:3] = False
+    exact = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * (2 * k + 32) * 2.0 ** -24 + 1e-37
+    got = ops.gemm_ring(x, w[n:], "f32")
+    assert bool(((got.double() - exact[:, n:]).abs() <= bound[:, n:])[plain].all())
+    if m > 3:
+        assert torch.equal(got[1], exact[1, n:].float()) and bool(got[2].isnan().all())
+        plain[3] = False        # its gate times its up leaves float32's range
+    if n <= 6144:
+        gated = ops.gemm_ring(x, w, "gated")
+        want = torch.nn.functional.silu(exact[:, :n]) * exact[:, n:]
+        slack = bound[:, :n] * (exact[:, n:].abs() + bound[:, n:]) * 1.1 + bound[:, n:] * exact[:, :n].abs() + want.abs() * 8 * 2.0 ** -24 + 1e-30
+        assert gated.dtype == torch.float32 and bool(((gated.double() - want).abs() <= slack)[plain].all())
+    if m > 1:
+        assert torch.equal(ops.gemm_ring(x[:1].contiguous(), w[n:], "f32")[0], got[0])
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+def test_float32_rows_without_their_factors(ops, m):
+    """A norm up to its factors and its readers, all in float32, beside the exact result."""
+    g = torch.Generator().manual_seed(m)
+    n, k = 2050, 1056
+    gain, h = rand(g, k).to(DEV), rand(g, m, k).to(DEV) * torch.logspace(-3, 3, m, device=DEV)[:, None]
+    squares = torch.zeros(m, 256, device=DEV)
+    squares[:, :33] = h.pow(2).view(m, 33, 32).sum(2)
+    rows = ops.UnscaledRows(h * gain, squares, 1e-6)
+    w = rand(g, 2 * n, k, scale=0.05).to(DEV)
+    y = h.double() * torch.rsqrt(h.double().pow(2).mean(1, keepdim=True) + 1e-6) * gain.double()
+    exact, bound = y @ w.double().t(), (y.abs() @ w.double().abs().t()) * (2 * k + 64) * 2.0 ** -24
+    assert ops.unscaled_linear(m, w[:n]) and ops.unscaled_swiglu(m, w)
+    assert bool(((ops.linear(rows, w[:n]).double() - exact[:, :n]).abs() <= bound[:, :n]).all())
+    want = torch.nn.functional.silu(exact[:, :n]) * exact[:, n:]
+    slack = bound[:, :n] * (exact[:, n:].abs() + bound[:, n:]) * 1.1 + bound[:, n:] * exact[:, :n].abs() + want.abs() * 8 * 2.0 ** -24 + 1e-30
+    assert bool(((ops.linear_swiglu(rows, w).double() - want).abs() <= slack).all())
 
 
 def test_gemm_ring_refuses(ops):

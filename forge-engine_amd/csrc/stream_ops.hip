@@ -17,40 +17,29 @@ static inline int row_threads(int rows, int width) { return rows <= FEW_ROWS && 
 // sequence, the sequence's state row for its first token of the step.
 template <typename TX, typename TO>
 __global__ __launch_bounds__(ROW_THREADS_FEW) void token_shift_kernel(
-    const TX* __restrict__ x, const float* __restrict__ w, const float* __restrict__ state,
+    const TX* __restrict__ x, const float* __restrict__ w, float* __restrict__ state,
     const int* __restrict__ cu_q, const int* __restrict__ token_seq, const int* __restrict__ state_slots,
     TO* __restrict__ out, int tokens, int width, int count, int slots) {
   const int t = blockIdx.x;
   const int seq = token_seq[t];
   const bool first = cu_q[seq] == t;
-  const int slot = state_slots[seq];
+  const int slot = state_slots[seq], last = cu_q[seq + 1] - 1;
   const TX* row = x + (size_t)t * width;
   const TX* before = first ? row : row - width;   // never an address before the buffer
-  const float* kept = state + (size_t)min(max(slot, 0), slots - 1) * width;
+  float* kept = state + (size_t)min(max(slot, 0), slots - 1) * width;
+  const bool saves = first && last >= t && last < tokens && slot >= 0 && slot < slots;
+  const TX* final = saves ? x + (size_t)last * width : row;
   for (int c = threadIdx.x; c < width; c += blockDim.x) {
     const float v = load_as_float(row + c);
     const float p = first ? kept[c] : load_as_float(before + c);
     const float d = p - v;
     for (int s = 0; s < count; ++s)
       store_from_float(out + ((size_t)s * tokens + t) * width + c, v + d * w[(size_t)s * width + c]);
+    if (saves) kept[c] = load_as_float(final + c);
   }
 }
 
-// state[slot[s]] = x[last row of sequence s], for sequences that bring tokens.  One block per sequence.
-template <typename TX>
-__global__ __launch_bounds__(ROW_THREADS) void save_last_rows_kernel(
-    const TX* __restrict__ x, float* __restrict__ state, const int* __restrict__ cu_q,
-    const int* __restrict__ state_slots, int width, int slots, int tokens) {
-  const int seq = blockIdx.x;
-  const int begin = cu_q[seq], end = cu_q[seq + 1];
-  const int slot = state_slots[seq];
-  if (end <= begin || end > tokens || slot < 0 || slot >= slots) return;
-  const TX* row = x + (size_t)(end - 1) * width;
-  float* kept = state + (size_t)slot * width;
-  for (int c = threadIdx.x; c < width; c += ROW_THREADS) kept[c] = load_as_float(row + c);
-}
-
-extern "C" int fe_token_shift(const void* x, int x_dtype, const float* weights, const float* state, const int* cu_q,
+extern "C" int fe_token_shift(const void* x, int x_dtype, const float* weights, float* state, const int* cu_q,
                               const int* token_seq, const int* state_slots, void* out, int out_dtype, int tokens,
                               int width, int count, int slots, hipStream_t stream) {
   if (tokens <= 0) return FE_OK;
@@ -64,18 +53,6 @@ extern "C" int fe_token_shift(const void* x, int x_dtype, const float* weights, 
   else if (x_dtype == FE_BF16 && out_dtype == FE_F32) LAUNCH(bf16_t, float);
   else return FE_BAD_ARGUMENT;
 #undef LAUNCH
-  return fe_check_launch();
-}
-
-extern "C" int fe_save_last_rows(const void* x, int x_dtype, float* state, const int* cu_q, const int* state_slots,
-                                 int num_seqs, int width, int slots, int tokens, hipStream_t stream) {
-  if (num_seqs <= 0 || tokens <= 0) return FE_OK;
-  if (width <= 0 || slots < 1) return FE_BAD_ARGUMENT;
-  if (x_dtype == FE_F32)
-    save_last_rows_kernel<float><<<num_seqs, ROW_THREADS, 0, stream>>>((const float*)x, state, cu_q, state_slots, width, slots, tokens);
-  else if (x_dtype == FE_BF16)
-    save_last_rows_kernel<bf16_t><<<num_seqs, ROW_THREADS, 0, stream>>>((const bf16_t*)x, state, cu_q, state_slots, width, slots, tokens);
-  else return FE_BAD_ARGUMENT;
   return fe_check_launch();
 }
 

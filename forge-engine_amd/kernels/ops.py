@@ -1682,8 +1682,6 @@ def token_shift(x: Tensor, weights: Tensor, state: Tensor, cu_q: Tensor, token_s
     _call("stream_ops", "fe_token_shift", _ptr(x), c_int(_code(x.dtype)), _ptr(weights), _ptr(state), _ptr(cu_q),
           _ptr(token_seq), _ptr(state_slots), _ptr(out), c_int(_code(out.dtype)), c_int(tokens), c_int(width),
           c_int(weights.shape[0]), c_int(state.shape[0]), _stream())
-    _call("stream_ops", "fe_save_last_rows", _ptr(x), c_int(_code(x.dtype)), _ptr(state), _ptr(cu_q), _ptr(state_slots),
-          c_int(num_seqs), c_int(width), c_int(state.shape[0]), c_int(tokens), _stream())
     return out
 
 

@@ -247,6 +247,181 @@ extern "C" int fe_linear_recurrence(const void* q, const void* k, const void* v,
   return fe_check_launch();
 }
 
+// ---------------------------------------------------------------- a step of single tokens, with its ending
+// The same recurrence for one token a sequence, with the gates before it and the norm and gate behind it in the one launch: decays are
+// transformed and an mLSTM's stabilised gates made where they are used, and a head's read-out, which lies in LDS, becomes
+//     out = o / rms(o) * weight * act(gate)       (with a normaliser column: o / (max(|n|, exp(-m)) + 1e-6) in the place of o).
+// What bounds it: latency, and for large states a CU's share of their bytes (a head's state is read and written once).  So a block is one
+// head of one sequence (the norm needs the whole head), a column belongs to the L lanes that hold its key channels four by four, and a
+// thread asks for all its U pieces of the state (one pass of them, for up to 9 x 32 columns of 128 keys) before it uses the first.
+// Six sequences in a captured step, transform, gates, walk and norm in launches of their own -> this: 32 heads of 64 x 64
+// 11.3 -> 5.8, 16 of 64 x 128 11.7 -> 7.6, 8 of 128 x 257 22.6 -> 9.2 us.
+struct StepEnding {
+  const float* gates; const float* gate_bias; float* maximum;      // an mLSTM's: [T][2 heads], [2 heads], [slots][heads]
+  const float* decay_bias;
+  const float* weight; const void* gate; void* out;
+  size_t gate_stride, out_stride;
+  float cap, tau, eps;
+  int decay_kind, weight_len, act;
+};
+
+template <int L>
+__device__ __forceinline__ float sum_lanes(float v) {
+  static_assert(L == 4 || L == 8 || L == 16 || L == 32 || L == 64, "a power of two from four");
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));                  // lane ^ 1
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));                  // lane ^ 2
+  if (L >= 8) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));     // 7 - lane within 8
+  if (L >= 16) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));    // 15 - lane within 16
+  if (L >= 32) v = sum_xor16(v);
+  if (L >= 64) v = sum_xor32(v);
+  return v;
+}
+
+constexpr int STEP_MAX_VALUES = 512;
+
+template <typename T, int L, int U, int THREADS>
+__global__ __launch_bounds__(THREADS) void recurrence_step_kernel(RecurrenceArgs p, StepEnding e) {
+  constexpr int COLS = THREADS / L;
+  __shared__ float read_out[STEP_MAX_VALUES + 1];
+  const int h = blockIdx.x, seq = blockIdx.y;
+  const int t = p.cu_q[seq], slot = p.state_slots[seq];
+  if (p.cu_q[seq + 1] <= t || t < 0 || t >= p.tokens || slot < 0 || slot >= p.slots) return;
+  const int tid = threadIdx.x, lane = tid & 63, rg = tid % L, jl = tid / L;
+  const int Dk = p.key_dim, Dv = p.value_dim, H = p.heads, columns = Dv + p.ones_column;
+  const bool channels = rg * 4 < Dk;
+  const int i0 = channels ? rg * 4 : 0;        // lanes beyond the key channels read the first ones and add nothing
+  float4* state = (float4*)(p.state + ((size_t)slot * H + h) * columns * Dk + i0);      // column c: state[c * Dk / 4]
+  const T* v_row = (const T*)p.v + (size_t)t * p.v_stride + (size_t)h * Dv;
+
+  float4 piece[U];
+  float value[U];
+  auto fetch = [&](int first) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int col = min(first + u * COLS + jl, columns - 1);
+      piece[u] = state[(size_t)col * (Dk / 4)];
+      value[u] = load_as_float(v_row + min(col, Dv - 1));
+    }
+  };
+  fetch(0);
+
+  float q[4], k[4], a[4], bonus[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const size_t c = (size_t)h * Dk + i0 + j;
+    const float qv = load_as_float((const T*)p.q + (size_t)t * p.q_stride + c) * p.q_scale;
+    const float kv = load_as_float((const T*)p.k + (size_t)t * p.k_stride + c);
+    q[j] = channels ? qv : 0.f;
+    k[j] = channels ? kv : 0.f;
+    bonus[j] = p.bonus ? p.bonus[c] : 0.f;
+    a[j] = 1.f;
+    if (p.decay) {
+      const float z = p.decay[(size_t)t * H * Dk + c] + e.decay_bias[c];
+      a[j] = e.decay_kind == 1 ? expf(-expf(z)) : expf(log_sigmoid(z) / e.tau);
+    }
+  }
+  float in_scale = 1.f, floor_ = 0.f, m = 0.f;
+  if (e.gates) {       // the formulas of mlstm_gate_scan_kernel for one token
+    const float gi = e.cap * tanhf((e.gates[(size_t)t * 2 * H + h] + e.gate_bias[h]) / e.cap);
+    const float gf = log_sigmoid(e.cap * tanhf((e.gates[(size_t)t * 2 * H + H + h] + e.gate_bias[H + h]) / e.cap));
+    const float m_in = e.maximum[(size_t)slot * H + h];
+    m = fmaxf(m_in + gf, gi);
+    in_scale = expf(gi - m);
+    floor_ = expf(-m);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = expf(gf + m_in - m);
+  }
+
+  for (int first = 0;;) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int col = first + u * COLS + jl;
+      const float vj = (col < Dv ? value[u] : 1.f) * in_scale;
+      float s[4] = {piece[u].x, piece[u].y, piece[u].z, piece[u].w}, sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float kv = k[j] * vj;
+        if (p.bonus) sum = fmaf(fmaf(bonus[j], kv, s[j]), q[j], sum);
+        s[j] = fmaf(s[j], a[j], kv);
+        if (!p.bonus) sum = fmaf(s[j], q[j], sum);
+      }
+      sum = sum_lanes<L>(sum);
+      if (col < columns) {
+        if (channels) state[(size_t)col * (Dk / 4)] = make_float4(s[0], s[1], s[2], s[3]);
+        if (rg == 0) read_out[col] = sum;
+      }
+    }
+    first += U * COLS;
+    if (first >= columns) break;
+    fetch(first);
+  }
+  __syncthreads();
+  if (e.gates && tid == 0) e.maximum[(size_t)slot * H + h] = m;      // everyone has read the one before
+  const float scale = e.gates ? 1.f / (fmaxf(fabsf(read_out[Dv]), floor_) + 1e-6f) : 1.f;
+  float squares = 0.f;
+  for (int c = lane; c < Dv; c += 64) squares += read_out[c] * scale * (read_out[c] * scale);       // every wave the whole head's
+  const float inv = rsqrtf(wave_sum(squares) / (float)Dv + e.eps) * scale;
+  for (int c = tid; c < Dv; c += THREADS) {
+    float y = read_out[c] * inv;
+    if (e.weight) y *= e.weight[e.weight_len == Dv ? c : h * Dv + c];
+    const float g = load_as_float((const T*)e.gate + (size_t)t * e.gate_stride + (size_t)h * Dv + c);
+    y *= e.act == 1 ? g / (1.f + expf(-g)) : 1.f / (1.f + expf(-g));
+    store_from_float((T*)e.out + (size_t)t * e.out_stride + (size_t)h * Dv + c, y);
+  }
+}
+
+template <typename T, int L>
+static void launch_step(const RecurrenceArgs& p, const StepEnding& e, int columns, int num_seqs, hipStream_t stream) {
+  const dim3 grid(p.heads, num_seqs);
+  // four pieces of the state a thread where 256 or 512 threads hold it so, else nine of 1,024 threads
+  if (columns * L <= 4 * 256) recurrence_step_kernel<T, L, 4, 256><<<grid, 256, 0, stream>>>(p, e);
+  else if (columns * L <= 4 * 512) recurrence_step_kernel<T, L, 4, 512><<<grid, 512, 0, stream>>>(p, e);
+  else recurrence_step_kernel<T, L, 9, 1024><<<grid, 1024, 0, stream>>>(p, e);
+}
+
+template <typename T>
+static void launch_step_keys(const RecurrenceArgs& p, const StepEnding& e, int columns, int num_seqs, hipStream_t stream) {
+  if (p.key_dim <= 16) launch_step<T, 4>(p, e, columns, num_seqs, stream);
+  else if (p.key_dim <= 32) launch_step<T, 8>(p, e, columns, num_seqs, stream);
+  else if (p.key_dim <= 64) launch_step<T, 16>(p, e, columns, num_seqs, stream);
+  else if (p.key_dim <= 128) launch_step<T, 32>(p, e, columns, num_seqs, stream);
+  else launch_step<T, 64>(p, e, columns, num_seqs, stream);
+}
+
+// A step in which every sequence brings one token (or none).  key_dim a multiple of four up to 256, value_dim up to 512; q, k, v, gate and
+// out of one dtype, rows of any stride; `decay` [tokens][heads * key_dim] stays as it is (kinds as above, 1 or 2), or gates, gate_bias and
+// maximum are an mLSTM's (then a normaliser column follows the values), or neither.  act 1: silu(gate), 2: sigmoid(gate).
+extern "C" int fe_linear_recurrence_step(const void* q, const void* k, const void* v, int dtype, long long q_stride, long long k_stride,
+                                         long long v_stride, const float* decay, int decay_kind, const float* decay_bias, float tau,
+                                         const float* gates, const float* gate_bias, float cap, float* maximum, float q_scale,
+                                         const float* bonus, float* state, int slots, const float* weight, int weight_len,
+                                         const void* gate, long long gate_stride, int act, float eps, void* out, long long out_stride,
+                                         const int* cu_q, const int* state_slots, int num_seqs, int heads, int key_dim, int value_dim,
+                                         int tokens, hipStream_t stream) {
+  if (tokens <= 0 || num_seqs <= 0) return FE_OK;
+  if (heads <= 0 || key_dim < 4 || key_dim > 256 || key_dim % 4 || value_dim < 1 || value_dim > STEP_MAX_VALUES || slots < 1 ||
+      num_seqs > 65535 || (dtype != FE_F32 && dtype != FE_BF16) || decay_kind < 0 || decay_kind > 2 ||
+      (decay_kind != 0) != (decay != nullptr) || (decay && !decay_bias) || !(tau > 0.f) || !(eps > 0.f) || (act != 1 && act != 2) || !gate ||
+      !out || !state || (((uintptr_t)state) & 15) || (gates && (decay || !gate_bias || !maximum || !(cap > 0.f))))
+    return FE_BAD_ARGUMENT;
+  const long long keys = (long long)heads * key_dim, values = (long long)heads * value_dim;
+  if (q_stride < keys || k_stride < keys || v_stride < values || gate_stride < values || out_stride < values) return FE_BAD_ARGUMENT;
+  if (weight && weight_len != value_dim && weight_len != values) return FE_BAD_ARGUMENT;
+  RecurrenceArgs p = {};
+  p.q = q; p.k = k; p.v = v;
+  p.q_stride = (size_t)q_stride; p.k_stride = (size_t)k_stride; p.v_stride = (size_t)v_stride;
+  p.decay = decay; p.bonus = bonus; p.state = state; p.cu_q = cu_q; p.state_slots = state_slots;
+  p.q_scale = q_scale;
+  p.ones_column = gates ? 1 : 0; p.slots = slots;
+  p.heads = heads; p.key_dim = key_dim; p.value_dim = value_dim; p.tokens = tokens;
+  const StepEnding e = {gates, gate_bias, maximum, decay_bias, weight, gate, out, (size_t)gate_stride, (size_t)out_stride,
+                        cap, tau, eps, decay_kind, weight_len, act};
+  const int columns = value_dim + p.ones_column;
+  if (dtype == FE_F32) launch_step_keys<float>(p, e, columns, num_seqs, stream);
+  else launch_step_keys<bf16_t>(p, e, columns, num_seqs, stream);
+  return fe_check_launch();
+}
+
 // ---------------------------------------------------------------- stabilised gates of an mLSTM
 // Per sequence and head, along the tokens:  i = cap tanh((g_i + b_i) / cap),
 // f = logsigmoid(cap tanh((g_f + b_f) / cap)),  m_t = max(f + m_(t-1), i);

@@ -2409,6 +2409,61 @@ def linear_recurrence(q: Tensor, k: Tensor, v: Tensor, out: Tensor, state: Tenso
     return out
 
 
+STEP_MAX_VALUES = 512
+
+
+def linear_recurrence_step_fits(state: Tensor, *, key_dim: int, value_dim: int) -> bool:
+    """Whether ``linear_recurrence_step`` takes heads of these sizes."""
+    return key_dim % 4 == 0 and 4 <= key_dim <= 256 and 1 <= value_dim <= STEP_MAX_VALUES and state.data_ptr() % 16 == 0
+
+
+def linear_recurrence_step(q: Tensor, k: Tensor, v: Tensor, gate: Tensor, out: Tensor, state: Tensor, cu_q: Tensor, state_slots: Tensor, *,
+                           num_seqs: int, heads: int, key_dim: int, value_dim: int, eps: float, act: str, weight: Tensor | None = None,
+                           decay: Tensor | None = None, decay_kind: str = "none", decay_bias: Tensor | None = None, tau: float = 1.0,
+                           gates: Tensor | None = None, gate_bias: Tensor | None = None, cap: float = 1.0, maximum: Tensor | None = None,
+                           q_scale: float = 1.0, bonus: Tensor | None = None) -> Tensor:
+    """``linear_recurrence`` for a step of single tokens with what lies around it in the same launch: the decays' transform
+    (``decay`` stays as it is) or, given ``gates``, ``mlstm_gate_scan`` (head decay, input scale and a normaliser column), and
+    ``head_norm_gate`` behind it, into ``out`` [T, heads * value_dim] (q's dtype, rows of any stride).  Six sequences, us: see the kernel."""
+    columns, tokens = value_dim + (0 if gates is None else 1), q.shape[0]
+    strides = [_strided_rows(q, "q", heads * key_dim), _strided_rows(k, "k", heads * key_dim), _strided_rows(v, "v", heads * value_dim)]
+    gate_stride, out_stride = _strided_rows(gate, "gate", heads * value_dim), _strided_rows(out, "out", heads * value_dim)
+    if any(t.dtype != q.dtype or t.shape[0] != tokens for t in (k, v, gate, out)) or tokens != num_seqs:
+        raise KernelError("q, k, v, gate and out must share dtype and hold one token a sequence")
+    _gpu(state, "state", torch.float32)
+    _sequences(cu_q, state_slots, num_seqs)
+    if state.dim() != 4 or state.shape[1:] != (heads, columns, key_dim):
+        raise KernelError(f"state must be [slots, {heads}, {columns}, {key_dim}], got {tuple(state.shape)}")
+    if not linear_recurrence_step_fits(state, key_dim=key_dim, value_dim=value_dim):
+        raise KernelError(f"key sizes in fours up to 256 and up to {STEP_MAX_VALUES} values, a state 16 bytes aligned")
+    if decay_kind not in _DECAY_KINDS or (decay is None) != (decay_kind == "none") or (decay is None) != (decay_bias is None):
+        raise KernelError("decay, its kind and its bias go together")
+    if act not in ("silu", "sigmoid"):
+        raise KernelError(f"unknown gate activation '{act}'")
+    if gates is not None and (decay is not None or gate_bias is None or maximum is None or not cap > 0.0):
+        raise KernelError("gates come with their bias, a positive cap and the maximum, and without a decay per channel")
+    for name, t, shape in (("decay", decay, (tokens, heads * key_dim)), ("decay_bias", decay_bias, (heads * key_dim,)),
+                           ("gates", gates, (tokens, 2 * heads)), ("gate_bias", gate_bias, (2 * heads,)),
+                           ("maximum", maximum, (state.shape[0], heads)), ("bonus", bonus, None), ("weight", weight, None)):
+        if t is not None:
+            _gpu(t, name, torch.float32)
+            if shape is not None and tuple(t.shape) != shape:
+                raise KernelError(f"{name} must be {shape}, got {tuple(t.shape)}")
+    if bonus is not None and bonus.numel() != heads * key_dim:
+        raise KernelError(f"bonus must hold {heads * key_dim} entries")
+    if weight is not None and weight.numel() not in (value_dim, heads * value_dim):
+        raise KernelError(f"weight must hold {value_dim} or {heads * value_dim} entries")
+    if not tau > 0.0 or not eps > 0.0:
+        raise KernelError("tau and eps must be positive")
+    _call("linear_recurrence", "fe_linear_recurrence_step", _ptr(q), _ptr(k), _ptr(v), c_int(_code(q.dtype)), *(c_longlong(s) for s in strides),
+          _ptr(decay), c_int(_DECAY_KINDS[decay_kind]), _ptr(decay_bias), c_float(tau), _ptr(gates), _ptr(gate_bias), c_float(cap),
+          _ptr(maximum), c_float(q_scale), _ptr(bonus), _ptr(state), c_int(state.shape[0]), _ptr(weight),
+          c_int(0 if weight is None else weight.numel()), _ptr(gate), c_longlong(gate_stride), c_int(_ACTS[act]), c_float(eps), _ptr(out),
+          c_longlong(out_stride), _ptr(cu_q), _ptr(state_slots), c_int(num_seqs), c_int(heads), c_int(key_dim), c_int(value_dim),
+          c_int(tokens), _stream())
+    return out
+
+
 def mlstm_gate_scan(gates: Tensor, bias: Tensor, cap: float, maximum: Tensor, cu_q: Tensor, state_slots: Tensor,
                     out: Tensor, *, num_seqs: int, heads: int) -> Tensor:
     """The stabilised gates of an mLSTM, per sequence and head along the tokens: with i = cap tanh((g_i +

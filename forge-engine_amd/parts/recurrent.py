@@ -97,6 +97,14 @@ class _RecurrentMixer(Mixer):
         _, at, rows = self._fused[key]
         return product[:, at:at + rows]
 
+    def single_tokens(self, tokens: int, batch, cache: CacheView) -> bool:
+        """Every sequence of the step brings one token, and gates, recurrence and norm may be one launch."""
+        return (batch.num_decode is not None and batch.num_decode == batch.num_seqs == tokens
+                and ops.linear_recurrence_step_fits(cache.states[self.STATE], key_dim=self.key_dim, value_dim=self.value_dim))
+
+    def sizes(self, batch) -> dict:
+        return {"num_seqs": batch.num_seqs, "heads": self.heads, "key_dim": self.key_dim, "value_dim": self.value_dim, "eps": self.eps}
+
     def state_shape(self) -> tuple[int, ...]:
         return (self.heads, self.value_dim, self.key_dim)      # value-major: a thread's key channels lie together
 
@@ -152,12 +160,16 @@ class RWKVTimeMix(_RecurrentMixer):
         gate = ops.linear(mixes[3], t["g"])
         low = ops.tanh_rows(ops.linear(mixes[4], t["w1"]))
         decay = ops.linear(low, t["w2"], out_dtype=torch.float32)
+        y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
+        if self.single_tokens(x.shape[0], batch, cache):
+            ops.linear_recurrence_step(r, k, v, gate, y, cache.states[self.STATE], batch.cu_q, batch.state_slots, **self.sizes(batch),
+                                       decay=decay, decay_kind="exp_neg_exp", decay_bias=t["w0"], bonus=t["u"], weight=t["norm"], act="silu")
+            return ops.linear_update(y, t["o"])
         out = torch.empty((x.shape[0], self.heads, self.value_dim), dtype=torch.float32, device=x.device)
         ops.linear_recurrence(r, k, v, out, cache.states[self.STATE], batch.cu_q, batch.state_slots,
                               num_seqs=batch.num_seqs, max_q_len=batch.max_q_len, heads=self.heads,
                               key_dim=self.key_dim, value_dim=self.value_dim, decay=decay,
                               decay_kind="exp_neg_exp", decay_bias=t["w0"], bonus=t["u"])
-        y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
         ops.head_norm_gate(out, t["norm"], gate, y, heads=self.heads, dim=self.value_dim, eps=self.eps, act="silu")
         return ops.linear_update(y, t["o"])
 
@@ -186,13 +198,18 @@ class GatedLinearAttention(_RecurrentMixer):
         t = self.tensors
         qkvg = ops.linear(x, t["qkvg"])
         decay = ops.linear(ops.linear(x, t["a1"]), t["a2"], out_dtype=torch.float32)
+        y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
+        if self.single_tokens(x.shape[0], batch, cache):
+            ops.linear_recurrence_step(*(self.columns(qkvg, key) for key in ("q", "k", "v", "g")), y, cache.states[self.STATE], batch.cu_q,
+                                       batch.state_slots, **self.sizes(batch), decay=decay, decay_kind="sigmoid_root",
+                                       decay_bias=t["a2_bias"], tau=self.tau, q_scale=self.key_dim ** -0.5, weight=t["norm"], act="silu")
+            return ops.linear_update(y, t["o"])
         out = torch.empty((x.shape[0], self.heads, self.value_dim), dtype=torch.float32, device=x.device)
         ops.linear_recurrence(self.columns(qkvg, "q"), self.columns(qkvg, "k"), self.columns(qkvg, "v"), out,
                               cache.states[self.STATE], batch.cu_q, batch.state_slots, num_seqs=batch.num_seqs,
                               max_q_len=batch.max_q_len, heads=self.heads, key_dim=self.key_dim,
                               value_dim=self.value_dim, decay=decay, decay_kind="sigmoid_root",
                               decay_bias=t["a2_bias"], tau=self.tau, q_scale=self.key_dim ** -0.5)
-        y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
         ops.head_norm_gate(out, t["norm"], self.columns(qkvg, "g"), y, heads=self.heads, dim=self.value_dim,
                            eps=self.eps, act="silu")
         return ops.linear_update(y, t["o"])
@@ -239,6 +256,12 @@ class MLSTM(_RecurrentMixer):
         t = self.tensors
         qkvg = ops.linear(x, t["qkvg"])
         gates = ops.linear(x, t["gates"], out_dtype=torch.float32)
+        y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
+        if self.single_tokens(x.shape[0], batch, cache):
+            ops.linear_recurrence_step(*(self.columns(qkvg, key) for key in ("q", "k", "v", "g")), y, cache.states[self.STATE], batch.cu_q,
+                                       batch.state_slots, **self.sizes(batch), gates=gates, gate_bias=self.gate_bias, cap=self.gate_cap,
+                                       maximum=cache.states[self.MAXIMUM], q_scale=self.key_dim ** -0.5, weight=t["norm"], act="sigmoid")
+            return ops.linear_update(y, t["o"])
         scanned = torch.empty((3, x.shape[0], self.heads), dtype=torch.float32, device=x.device)
         ops.mlstm_gate_scan(gates, self.gate_bias, self.gate_cap, cache.states[self.MAXIMUM], batch.cu_q,
                             batch.state_slots, scanned, num_seqs=batch.num_seqs, heads=self.heads)
@@ -248,7 +271,6 @@ class MLSTM(_RecurrentMixer):
                               max_q_len=batch.max_q_len, heads=self.heads, key_dim=self.key_dim,
                               value_dim=self.value_dim, head_decay=scanned[0], in_scale=scanned[1],
                               q_scale=self.key_dim ** -0.5, ones_column=True)
-        y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
         ops.head_norm_gate(out, t["norm"], self.columns(qkvg, "g"), y, heads=self.heads, dim=self.value_dim,
                            eps=self.eps, act="sigmoid", extra=1, floor=scanned[2])
         return ops.linear_update(y, t["o"])

@@ -557,6 +557,22 @@ def mlstm_gate_scan(gates, bias, cap, maximum, cu_q, state_slots, out, *, num_se
     return out
 
 
+def linear_recurrence_step_fits(state, *, key_dim, value_dim):
+    return key_dim % 4 == 0 and value_dim <= 512
+
+
+def linear_recurrence_step(q, k, v, gate, out, state, cu_q, state_slots, *, num_seqs, heads, key_dim, value_dim, eps, act, weight=None,
+                           gates=None, gate_bias=None, cap=1.0, maximum=None, **options):
+    extra, floor = 0 if gates is None else 1, None
+    if gates is not None:
+        scanned = mlstm_gate_scan(gates, gate_bias, cap, maximum, cu_q, state_slots, torch.zeros(3, q.shape[0], heads), num_seqs=num_seqs, heads=heads)
+        options.update(head_decay=scanned[0], in_scale=scanned[1], ones_column=True)
+        floor = scanned[2]
+    o = linear_recurrence(q, k, v, torch.zeros(q.shape[0], heads, value_dim + extra), state, cu_q, state_slots, num_seqs=num_seqs,
+                          max_q_len=1, heads=heads, key_dim=key_dim, value_dim=value_dim, **options)
+    return head_norm_gate(o, weight, gate, out, heads=heads, dim=value_dim, eps=eps, act=act, extra=extra, floor=floor)
+
+
 def hyper_norm(streams, update, mix, share, read, weight, bias, eps, out, rows=None, store=True, rms=False, shift=None):
     count = streams.shape[0]
     x = streams
@@ -956,7 +972,7 @@ DECODE_SPLITS_TESTED = tuple(range(1, 65))
 NAMES = ("cap_rows", "gate_heads", "latent_row_sizes", "latent_step_fits", "latent_query_step", "latent_value_step", "decode_prepare_supported", "linear_in_parts", "embed_rows", "add_rmsnorm", "add_rows", "swiglu", "gemm_nt_f32", "linear", "linear_update", "linear_swiglu", "gemm_skinny",
          "qk_norm_rope_write", "paged_attention", "argmax_rows", "sample_filtered_rows",
          "cast_rows", "add_bias", "token_shift", "rmsnorm_update", "rmsnorm_mean", "polynorm", "tanh_rows", "head_norm_gate",
-         "conv_rope_norm_write", "masked_attention", "linear_recurrence", "mlstm_gate_scan",
+         "conv_rope_norm_write", "masked_attention", "linear_recurrence", "linear_recurrence_step_fits", "linear_recurrence_step", "mlstm_gate_scan",
          "hyper_norm", "embed_token_pairs", "scale_rows", "whole_norm_rope_write", "moe_route", "moe_experts", "linear_gated",
          "relu_squared", "causal_conv_act", "selective_scan", "rmsnorm_update_norm", "layernorm_update", "activate", "gate_rows",
          "latent_norm_rope_write", "latent_query_pack", "latent_attention", "heads_product", "moe_route_grouped",

@@ -276,6 +276,41 @@ def test_linear_recurrence(ops, dtype, form, heads, key_dim, value_dim):
     torch.testing.assert_close(state_d.cpu(), state_ref, atol=1e-4, rtol=1e-4)
 
 
+# one and several passes of a block's columns, key sizes that leave lanes of a column without channels, the smallest and largest heads
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", ["rwkv", "gla", "mlstm", "plain"])
+@pytest.mark.parametrize("heads,key_dim,value_dim", [(3, 64, 64), (2, 64, 128), (2, 128, 256), (5, 4, 1), (2, 48, 80), (2, 20, 50), (1, 128, 16),
+                                                     (2, 200, 24), (1, 256, 512), (2, 32, 511)])
+def test_linear_recurrence_step(ops, dtype, form, heads, key_dim, value_dim):
+    g = torch.Generator().manual_seed(12)
+    cu, _, slots = layout([1] * 4, [4, 1, 0, 5])
+    tokens, keys, values = 4, heads * key_dim, heads * value_dim
+    wide = rand(g, tokens, 2 * keys + 2 * values + 3, dtype=dtype)
+    cut = lambda t: (t[:, 3:3 + keys], t[:, 3 + keys:3 + 2 * keys], t[:, 3 + 2 * keys:3 + 2 * keys + values], t[:, 3 + 2 * keys + values:])
+    columns = value_dim + (1 if form == "mlstm" else 0)
+    state, maximum = rand(g, 7, heads, columns, key_dim), rand(g, 7, heads, scale=2.0)
+    tensors = {"weight": rand(g, value_dim if form == "gla" else values)}
+    numbers = dict(num_seqs=tokens, heads=heads, key_dim=key_dim, value_dim=value_dim, eps=1e-6, act="sigmoid" if form == "mlstm" else "silu")
+    if form == "rwkv":
+        tensors.update(decay=rand(g, tokens, keys), decay_bias=rand(g, keys) - 1.0, bonus=rand(g, heads, key_dim))
+        numbers.update(decay_kind="exp_neg_exp")
+    elif form == "gla":
+        tensors.update(decay=rand(g, tokens, keys, scale=2.0), decay_bias=rand(g, keys))
+        numbers.update(decay_kind="sigmoid_root", tau=7.0, q_scale=key_dim ** -0.5)
+    elif form == "mlstm":
+        tensors.update(gates=rand(g, tokens, 2 * heads, scale=6.0), gate_bias=rand(g, 2 * heads), maximum=maximum)
+        numbers.update(cap=12.0, q_scale=key_dim ** -0.5)
+    state_d, wide_d, cu_d, slots_d = dev(state, wide, cu, slots)
+    tensors_d = {n: t.to(DEV) for n, t in tensors.items()}
+    got = ops.linear_recurrence_step(*cut(wide_d), torch.zeros(tokens, values + 5, dtype=dtype, device=DEV)[:, 5:], state_d, cu_d, slots_d,
+                                     **tensors_d, **numbers)
+    want = refs.linear_recurrence_step(*cut(wide), torch.zeros(tokens, values, dtype=dtype), state, cu, slots, **tensors, **numbers)
+    torch.testing.assert_close(got.cpu().float(), want.float(), **tol(dtype))
+    torch.testing.assert_close(state_d.cpu(), state, atol=1e-4, rtol=1e-4)
+    if form == "mlstm":
+        torch.testing.assert_close(tensors_d["maximum"].cpu(), maximum, atol=1e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("heads", [1, 2, 5])
 def test_mlstm_gate_scan(ops, heads):
     g = torch.Generator().manual_seed(11)

@@ -17,8 +17,7 @@
 //
 // The grouped products tile the sorted rows within an expert (a tile never spans two experts).  float32, and
 // bfloat16 with K no multiple of 32: 32 rows x 64 columns a block, K through LDS in steps of 32, FMA.  bfloat16:
-// MFMA 16x16x32 over tiles of 32 x 64 to 256 x 128 with rows and weight straight from memory in LDS, or, for few rows, a ring of
-// buffers a wave.  A launch of tiles has as many row-tile slots as the pairs could need at worst (pairs /
+// MFMA 16x16x32 over tiles of 32 x 64 to 256 x 128 with rows and weight straight from memory in LDS.  A launch has as many row-tile slots as the pairs could need at worst (pairs /
 // rows a tile + experts); a block whose slot lies beyond the tiles there are returns at once.
 #include "common.h"
 #include "lds_tile.h"
@@ -467,211 +466,6 @@ static int launch_moe_tile(const bf16_t* a, const bf16_t* w, const int* offsets,
   return fe_check_launch();
 }
 
-// The two products of few rows (a decode step): the row tile is 8 XI rows (an expert rarely has more of 16 tokens'), and one block a CU
-// takes an even share of all the weight rows that are read at all, in runs of eight columns (MODE 0: eight gate and eight up rows), in
-// order, UNIT runs of one expert at a time.  Eight waves take chunks of 64 of K in turn, each with a ring of its own in LDS that it
-// fills straight from memory and that runs on over the units, so that the weight keeps coming while a unit's sums meet.
-// What bounds it: the bytes of the experts that have rows, and the starts of the two launches.  Both products in a captured step, us,
-// experts as wide as the model, weights that no cache holds, in tiles of 32 x 64 (two rounds of blocks, each with a start of its own) ->
-// this (time of those bytes at 6.4 TB/s): 8 experts of 2,048, 2 a token, 1 / 2 / 8 / 16 / 48 tokens 22.6 -> 14.1 (7.9), 27.7 -> 23.1
-// (15.7), 49.3 -> 43.0 (31.5), 54.0 -> 43.1, 52.8 -> 43.5; of 1,024 13.9 -> 9.5 (2.0), 14.0 -> 12.3, 17.3 -> 16.1 (7.9), 19.9 -> 16.3; 32
-// experts of 2,048, 4 a token, 1 / 8 / 48 tokens 30.0 -> 21.7 (15.7), 106.4 -> 89.3 (70.8), 154.0 -> 149.1.  A unit of half the runs (twice
-// the reads of the rows) was up to 1.5 us slower from 6 tokens on.
-template <int XI, int MODE, int UNIT>
-struct MoeRing {
-  static constexpr int WAVES = 8, WI = MODE == 0 ? 2 * UNIT : UNIT, LOADS = XI + WI, TILES = (WI + 1) / 2;
-  static constexpr int MEET = WAVES * TILES * 1024;                     // sums of a unit, of which two lie there
-  static constexpr int STAGES = (152 * 1024 - 2 * MEET) / (WAVES * LOADS * 1024);
-  static constexpr int WAVE_BYTES = STAGES * LOADS * 1024, BYTES = WAVES * WAVE_BYTES + 2 * MEET;
-  static constexpr int ROWS = 8 * XI, MAX_PAIRS = 256;
-  static_assert(STAGES >= 2 && LOADS * (STAGES - 1) < 64, "a ring");
-};
-
-template <int XI, int MODE, int UNIT>
-__global__ __launch_bounds__(512) void moe_ring_kernel(
-    const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ offsets, const int* __restrict__ order,
-    const float* __restrict__ pair_weight, bf16_t* __restrict__ act, float* __restrict__ out, int E, int N, int K, int top, int tokens,
-    float limit, float alpha, int form, const float* __restrict__ extra, int extra_parts) {
-  using R = MoeRing<XI, MODE, UNIT>;
-  using lds_tile::bf16x8;
-  constexpr int PAIR = MODE == 0 ? 2 : 1, VALUES = R::TILES * 256 / PAIR, COLUMNS = 8 * UNIT, CHUNK = 64;
-  extern __shared__ __attribute__((aligned(16))) uintx4 lds[];
-  __shared__ int tile_expert[R::MAX_PAIRS], tile_first[R::MAX_PAIRS], tile_end[R::MAX_PAIRS], pair_of[R::MAX_PAIRS], row_tiles;
-  __shared__ float weight_of[R::MAX_PAIRS];        // of a pair, by its place in the order
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, q = lane >> 4, pairs = tokens * top;
-  if (tid < pairs && tid < offsets[E]) {
-    const int pair = order[tid];
-    pair_of[tid] = pair;
-    weight_of[tid] = pair_weight ? pair_weight[pair] : 1.f;
-  }
-  if (wave == 7) {       // the row tiles there are, experts 64 at a time
-    int before = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = min(e0 + lane, E - 1), begin = offsets[e], end = offsets[e + 1];
-      const int mine = e0 + lane < E ? (end - begin + R::ROWS - 1) / R::ROWS : 0;
-      int upto = mine;
-#pragma unroll
-      for (int offset = 1; offset < 64; offset <<= 1) {
-        const int below = __shfl_up(upto, offset, FE_WAVE);
-        if (lane >= offset) upto += below;
-      }
-      for (int j = 0; j < mine; ++j) {
-        const int at = before + upto - mine + j;
-        if (at >= R::MAX_PAIRS) break;
-        tile_expert[at] = e;
-        tile_first[at] = begin + j * R::ROWS;
-        tile_end[at] = min(end, begin + (j + 1) * R::ROWS);
-      }
-      before += __shfl(upto, 63, FE_WAVE);
-    }
-    if (lane == 0) row_tiles = min(before, R::MAX_PAIRS);
-  }
-  __syncthreads();
-  const int runs = (N + 7) / 8, all = row_tiles * runs;
-  const int from = (int)((long long)all * blockIdx.x / gridDim.x), upto = (int)((long long)all * (blockIdx.x + 1) / gridDim.x);
-  if (from >= upto) return;
-
-  const int chunks = K / CHUNK, count = (chunks - wave + R::WAVES - 1) / R::WAVES;      // this wave's chunks of a unit: wave, wave + 8, ..
-  const unsigned int base = __builtin_amdgcn_readfirstlane((unsigned int)(size_t)(const __attribute__((address_space(3))) char*)&lds[0]) +
-                            wave * R::WAVE_BYTES;
-  const int of_group = lane >> 3, piece_at = wave * CHUNK + ((lane & 7) ^ of_group) * 8;
-  // a place in the work: run `run` of row tile `tile`, `left` runs before the block's end
-  struct Place {
-    int tile, run, left;
-  };
-  auto runs_at = [&](const Place& p) { return min(min(UNIT, p.left), runs - p.run); };
-  auto advance = [&](Place& p) {
-    const int by = runs_at(p);
-    p.left -= by;
-    p.run += by;
-    if (p.run == runs) {
-      p.run = 0;
-      ++p.tile;
-    }
-  };
-  const Place start = {__builtin_amdgcn_readfirstlane(from / runs), __builtin_amdgcn_readfirstlane(from % runs), upto - from};
-
-  // what is asked for runs STAGES chunks ahead of what is multiplied
-  Place next = start;
-  int next_chunk = 0, ahead = 0, fill = 0;      // chunks asked for and not yet multiplied; the buffer to fill
-  const bf16_t *x_from[XI], *w_from[R::WI];
-  bool x_has[XI], w_has[R::WI];
-  auto aim = [&]() {
-    const int expert = __builtin_amdgcn_readfirstlane(tile_expert[next.tile]), first = __builtin_amdgcn_readfirstlane(tile_first[next.tile]);
-    const int end = __builtin_amdgcn_readfirstlane(tile_end[next.tile]), has = runs_at(next);
-    const bf16_t* w_expert = w + (size_t)expert * (PAIR * (size_t)N) * K;
-#pragma unroll
-    for (int i = 0; i < XI; ++i) {
-      const int row = first + i * 8 + of_group, sorted = min(row, end - 1);
-      x_has[i] = row < end;
-      x_from[i] = a + (size_t)(MODE != 1 ? pair_of[sorted] / top : sorted) * K + piece_at;
-    }
-#pragma unroll
-    for (int i = 0; i < R::WI; ++i) {        // MODE 0: eight gate rows, then the eight up rows of the same columns
-      const int run = min(i / PAIR, has - 1);
-      w_has[i] = i / PAIR < has;
-      w_from[i] = w_expert + ((size_t)min((next.run + run) * 8 + of_group, N - 1) + (MODE == 0 && i % 2 ? N : 0)) * K + piece_at;
-    }
-  };
-  // every request is issued whatever the rows, so that the waits can count: of rows that there are not, the first lanes' only
-  auto load = [&]() {
-    if (next.left <= 0 || count <= 0) return;
-    const int k = next_chunk * R::WAVES * CHUNK;
-    const unsigned int to = base + fill * R::LOADS * 1024;
-#pragma unroll
-    for (int i = 0; i < XI; ++i)
-      if (x_has[i] || of_group == 0) lds_tile::load_to_lds(x_from[i] + k, to + i * 1024);
-#pragma unroll
-    for (int i = 0; i < R::WI; ++i)
-      if (w_has[i] || of_group == 0) lds_tile::load_to_lds(w_from[i] + k, to + (XI + i) * 1024);
-    fill = fill + 1 == R::STAGES ? 0 : fill + 1;
-    ++ahead;
-    if (++next_chunk == count) {
-      next_chunk = 0;
-      advance(next);
-      if (next.left > 0) aim();
-    }
-  };
-  aim();
-#pragma unroll
-  for (int s = 0; s < R::STAGES; ++s) load();
-
-  const uintx4* ring = lds + wave * (R::WAVE_BYTES / 16);
-  int stage = 0, unit = 0;
-  for (Place at = start; at.left > 0; advance(at), ++unit) {
-    floatx4 acc[R::TILES];
-#pragma unroll
-    for (int t = 0; t < R::TILES; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int c = 0; c < count; ++c) {
-      if (ahead == R::STAGES) lds_tile::wait_loads<R::LOADS*(R::STAGES - 1)>();
-      else lds_tile::wait_steps<R::LOADS, R::STAGES - 1>(ahead - 1);
-      const uintx4* buffer = ring + stage * R::LOADS * 64;
-      uintx4 x_half[2], w_half[R::TILES][2];
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const int piece = (4 * half + q) ^ (r & 7);
-        x_half[half] = buffer[(XI == 1 ? r & 7 : r) * 8 + piece];
-#pragma unroll
-        for (int t = 0; t < R::TILES; ++t) w_half[t][half] = buffer[XI * 64 + min(t * 16 + r, R::WI * 8 - 8 + (r & 7)) * 8 + piece];
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before the buffer is filled again
-      --ahead;
-      load();
-#pragma unroll
-      for (int half = 0; half < 2; ++half)
-#pragma unroll
-        for (int t = 0; t < R::TILES; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w_half[t][half]), __builtin_bit_cast(bf16x8, x_half[half]), acc[t], 0, 0, 0);
-      stage = stage + 1 == R::STAGES ? 0 : stage + 1;
-    }
-    // the waves' sums meet, in one of two places in turn: whoever writes there again has passed the next unit's barrier
-    float* meet = (float*)((char*)lds + R::WAVES * R::WAVE_BYTES + (unit & 1) * R::MEET);
-#pragma unroll
-    for (int t = 0; t < R::TILES; ++t) ((floatx4*)meet)[(wave * R::TILES + t) * 64 + lane] = acc[t];
-    lds_tile::reads_done_barrier();
-    // value v: of tile v / 256 (MODE 0: v / 128), element v % 4 of lane group v / 64 % 4 (MODE 0: % 2), row v / 4 % 16; other waves each time
-    const int v = (tid + unit * VALUES) & 511;
-    if (v >= VALUES) continue;
-    const int tile = v / (256 / PAIR), group = (v >> 6) & (4 / PAIR - 1), row = (v >> 2) & 15;
-    const int column = tile * (16 / PAIR) + group * 4 + (v & 3), n = at.run * 8 + column;
-    const int sorted = tile_first[at.tile] + row;
-    if (sorted >= tile_end[at.tile] || column >= 8 * runs_at(at) || n >= N) continue;
-    auto total = [&](int lane_group) {
-      const float* parts = meet + (tile * 64 + lane_group * 16 + row) * 4 + (v & 3);
-      float sum = 0.f;
-#pragma unroll
-      for (int o = 0; o < R::WAVES; ++o) sum += parts[o * R::TILES * 256];
-      return sum;
-    };
-    const float sum = total(group);
-    if constexpr (MODE != 1) {
-      float up = 0.f;
-      if constexpr (MODE == 0) up = total(group + 2);
-      act[(size_t)sorted * N + n] = float_to_bf16(gated(sum, up, limit, alpha, form, weight_of[sorted]));
-    } else {
-      const int pair = pair_of[sorted], token = pair / top, choice = pair - token * top;
-      out[((size_t)choice * tokens + token) * N + n] =
-          with_extra(sum * weight_of[sorted], choice, extra, extra_parts, (size_t)tokens * N, (size_t)token * N + n);
-    }
-  }
-}
-
-template <int XI, int MODE, int UNIT>
-static int launch_moe_ring(const bf16_t* a, const bf16_t* w, const int* offsets, const int* order, const float* pair_weight,
-                           bf16_t* act, float* out, int experts, int N, int K, int top, int tokens, float limit, float alpha,
-                           int form, const float* extra, int extra_parts, hipStream_t stream) {
-  using R = MoeRing<XI, MODE, UNIT>;
-  static std::atomic<bool> raised{false};
-  auto kernel = moe_ring_kernel<XI, MODE, UNIT>;
-  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, R::BYTES, &raised);
-  if (limit_raised != FE_OK) return limit_raised;
-  const long long units = (long long)tokens * top * ((N + 8 * UNIT - 1) / (8 * UNIT));
-  kernel<<<(unsigned)std::min(256LL, units), 512, R::BYTES, stream>>>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top,
-                                                                     tokens, limit, alpha, form, extra, extra_parts);
-  return fe_check_launch();
-}
-
 // Which tile (rows x weight rows) a launch takes, by the rows an expert gets on average: few rows want many blocks with deep
 // buffers, each streaming its part of the weight (what bounds them is the weight's bytes), many rows want every weight row read
 // for more of them (what bounds them is the lines that a CU's L1 can wait for, see gemm_lds.h).  Measured on one MI355X, both
@@ -701,27 +495,10 @@ extern "C" int fe_moe_tile(int gated, int tokens, int top, int experts, int N, i
   return 32064;
 }
 
-// Rows of a tile of the ring kernel for few rows (8 or 16), or 0: the tiles above.  Few: the experts get 12 rows or fewer on average (at 16
-// most of them read their weight twice: 8 experts of 2,048, 48 tokens 52.8 -> 43.5 us, 64 tokens 53.2 -> 63.3), and all pairs fit the
-// block's lists.  Short sums leave its eight waves a chunk each: 64 experts of 512, 8 a token, 1 token 12.0 -> 8.9, but 4 tokens
-// 15.9 -> 16.4.
-extern "C" int fe_moe_ring_rows(int tokens, int top, int experts, int K) {
-  const long long pairs = (long long)tokens * top;
-  if (K % 64 != 0 || pairs > 256 || pairs > 12LL * experts || (K < 1024 && pairs > 8)) return 0;
-  return tokens <= 8 ? 8 : 16;
-}
-
 template <int MODE>
 static int launch_moe(const bf16_t* a, const bf16_t* w, const int* offsets, const int* order, const float* pair_weight,
                       bf16_t* act, float* out, int experts, int N, int K, int top, int tokens, float limit, float alpha,
                       int form, const float* extra, int extra_parts, hipStream_t stream) {
-  if (const int rows = fe_moe_ring_rows(tokens, top, experts, K)) {
-    constexpr int UNIT = MODE == 0 ? 2 : 4;
-    if (rows == 8) return launch_moe_ring<1, MODE, UNIT>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens, limit,
-                                                         alpha, form, extra, extra_parts, stream);
-    return launch_moe_ring<2, MODE, UNIT>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens, limit, alpha, form,
-                                          extra, extra_parts, stream);
-  }
 #define FE_GO(...) return launch_moe_tile<__VA_ARGS__, MODE>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens, \
                                                              limit, alpha, form, extra, extra_parts, stream)
   switch (fe_moe_tile(MODE == 0, tokens, top, experts, N, K)) {

@@ -211,56 +211,6 @@ def test_grouped_products_tiles(tokens, hidden, experts, top, inner, weight_inpu
     assert float((got.double() - want).norm() / want.norm()) < 1e-3
 
 
-@pytest.mark.parametrize("tokens,hidden,experts,top,inner,form", [
-    (1, 1024, 3, 1, 1028, "bounded"), (8, 1024, 7, 2, 1024, "silu"), (4, 64, 130, 2, 64, "bounded"),        # tiles of eight rows
-    (9, 1088, 3, 2, 1091, "bounded"), (16, 2112, 2, 1, 1024, "relu_squared"), (48, 1024, 8, 2, 1088, "bounded"),  # of sixteen
-    (32, 1024, 22, 8, 1152, "silu")])                                                                       # 256 pairs
-@pytest.mark.parametrize("spread", [False, True])
-def test_grouped_products_of_few_rows(tokens, hidden, experts, top, inner, form, spread):
-    """Rings of buffers a wave: rows beside a tile's edges, an expert with several tiles (all tokens take the same experts), units that
-    end with an expert or a block, columns beside a run of eight: against the same products in 64 bits, the middle in bfloat16."""
-    from forge_engine_amd.kernels import library, ops
-    assert library.load("moe").fe_moe_ring_rows(tokens, top, experts, hidden) == (8 if tokens <= 8 else 16)
-    g = torch.Generator(device=DEV).manual_seed(tokens + inner)
-
-    def draw(*shape, scale=1.0):
-        return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
-
-    matrices = 1 if form == "relu_squared" else 2
-    x, first, down = draw(tokens, hidden), draw(experts, matrices * inner, hidden, scale=hidden ** -0.5), draw(experts, hidden, inner, scale=inner ** -0.5)
-    chosen = torch.rand(tokens, experts, generator=g, device=DEV).argsort(1)[:, :top].int() if spread else \
-        torch.arange(top, device=DEV).int().repeat(tokens, 1)
-    weights, extra = torch.rand(tokens, top, generator=g, device=DEV), torch.randn(2, tokens, hidden, generator=g, device=DEV)
-    got = ops.moe_experts(x, chosen, weights, first, down, torch.full((top, tokens, hidden), float("nan"), device=DEV), limit=2.0,
-                          alpha=1.702, extra=extra, form=form)
-    want = torch.zeros(top, tokens, hidden, dtype=torch.float64, device=DEV)
-    for k in range(top):
-        for e in chosen[:, k].unique().tolist():
-            mine = (chosen[:, k] == e).nonzero().flatten()
-            both = x[mine].double() @ first[e].double().t()
-            if form == "relu_squared":
-                act = both.clamp(min=0.0).square()
-            elif form == "silu":
-                act = torch.nn.functional.silu(both[:, :inner]) * both[:, inner:]
-            else:
-                gate, up = both[:, :inner].clamp(max=2.0), both[:, inner:].clamp(-2.0, 2.0)
-                act = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
-            want[k, mine] = act.float().bfloat16().double() @ down[e].double().t() * weights[mine, k, None].double()
-    want[0] += extra.double().sum(0)
-    # the middle may round the other way where a float32 sum lies beside a tie: 2^-8 of one of `inner` terms of size inner^-0.5 each
-    torch.testing.assert_close(got.double(), want, atol=2e-2, rtol=1e-3)
-    assert float((got.double() - want).norm() / want.norm()) < 1e-3
-
-
-def test_when_grouped_products_take_rings():
-    """Both sides of the lines: rows an expert, pairs, steps of K."""
-    from forge_engine_amd.kernels import library
-    rows = library.load("moe").fe_moe_ring_rows
-    assert [rows(t, 2, 8, 2048) for t in (1, 8, 9, 48, 49)] == [8, 8, 16, 16, 0]
-    assert rows(32, 8, 64, 1024) == 16 and rows(33, 8, 64, 1024) == 0
-    assert rows(1, 8, 64, 512) == 8 and rows(2, 8, 64, 512) == 0 and rows(1, 2, 8, 1024 + 32) == 0
-
-
 def test_which_tile_a_grouped_product_takes():
     """Both sides of every line: rows an expert, blocks, steps, for the gated product and the other; and that the sizes above
     reach every tile."""

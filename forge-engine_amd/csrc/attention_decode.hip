@@ -205,9 +205,13 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     // The launch has splits for the longest context that may come; one that four waves read in one step needs none, and no merge
     // (1 sequence of 60 keys in a launch of 8 splits 7.5 -> 5.6 us, 8 of 100 in one of 4 9.0 -> 7.1.  Beyond, two steps without a
     // merge tie with one and the merge where the pages come from memory: 217 keys 7.6 against 7.9, in a step 0.3 slower).
-    const KeyRange range = key_range(run.ctx, PREPARE ? run.ctx - 1 : run.ctx, window, chunk);
-    if (range.last - range.first <= WAVES) run.splits = 1;
-    if (run.split >= run.splits) return;
+    // Finished queries keep their splits, and with them the order of every sum: the designs that bring them have routers, whose choice
+    // among experts at a near tie another rounding changes.
+    if constexpr (PREPARE) {
+      const KeyRange range = key_range(run.ctx, run.ctx - 1, window, chunk);
+      if (range.last - range.first <= WAVES) run.splits = 1;
+      if (run.split >= run.splits) return;
+    }
   }
   const int seq = run.seq, split = run.split, splits = run.splits;
   const size_t first_part = (size_t)run.part * kv_heads + (size_t)hk * splits;

@@ -369,7 +369,7 @@ def _few_rows_library_pays(rows: int, weight: Tensor) -> bool:
             and weight.shape[0] * weight.shape[1] * weight.element_size() > IN_PARTS_MAX_WEIGHT_BYTES)
 
 
-def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None, out_dtype=None) -> Tensor:
+def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None, out_dtype=None, ring: bool = True) -> Tensor:
     """y = x @ weight^T (+ bias) for a weight in [out, in] layout; float32
     accumulation; y in ``out_dtype`` (default: x's dtype).
 
@@ -378,7 +378,8 @@ def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None,
     bfloat16: up to 16 rows take the weight-streaming kernel or, like up to 256 rows, the
     product for portions, where the measurements above and below say they win; the
     rest is the platform's matrix library's, which the reference uses for every
-    projection (its nn.Linear calls, qwen3.py:115-122,215-223).
+    projection (its nn.Linear calls, qwen3.py:115-122,215-223).  ``ring`` False: bfloat16 rows do not go to ``gemm_ring``, whose sums are
+    rounded in another order than those of the products beside it, which a router's choice at a near tie answers to.
     """
     if isinstance(x, UnscaledRows):
         if bias is not None or out_dtype not in (None, x.rows.dtype) or not unscaled_linear(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
@@ -402,10 +403,10 @@ def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None,
     to_library = out_dtype == torch.bfloat16 and _few_rows_to_library(x, weight)
     if (bias is None and out_dtype == torch.bfloat16 and not to_library and _lds_fits(x, weight)
             and _lds_store_pays(x.shape[0], *weight.shape)):
-        tile = None if _ring_store_pays(x.shape[0], *weight.shape) else lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])[0]
+        tile = None if ring and _ring_store_pays(x.shape[0], *weight.shape) else lds_plan(x.shape[0], *weight.shape, 2 * weight.shape[0])[0]
         return gemm_lds(x, weight, "bf16", tile=tile)
     ending = {torch.float32: "f32", torch.bfloat16: "bf16"}.get(out_dtype)
-    if bias is None and not to_library and _ring_fits(x, weight, ending) and _ring_store_pays(x.shape[0], *weight.shape):
+    if ring and bias is None and not to_library and _ring_fits(x, weight, ending) and _ring_store_pays(x.shape[0], *weight.shape):
         return gemm_ring(x, weight, ending)
     if bias is None and out_dtype == torch.float32 and _lds_fits(x, weight) and _lds_head_pays(x.shape[0], *weight.shape):
         rows = x.shape[0]          # (hundreds of tiles a CU: the cheapest tile whatever the rounds, not the plan's)
@@ -2666,7 +2667,7 @@ def moe_route(x: Tensor, router_weight: Tensor, router_bias: Tensor | None, top:
         _gpu(router_bias, "router_bias", torch.float32)
         if router_bias.shape != (experts,):
             raise KernelError(f"router_bias must be [{experts}]")
-    logits = linear(x, router_weight, out_dtype=torch.float32)     # float32 accumulation, float32 logits
+    logits = linear(x, router_weight, out_dtype=torch.float32, ring=False)     # float32 accumulation, float32 logits
     chosen = torch.empty((tokens, top), dtype=torch.int32, device=x.device)
     weights = torch.empty((tokens, top), dtype=torch.float32, device=x.device)
     _call("moe", "fe_moe_select", _ptr(logits), _ptr(router_bias), _ptr(chosen), _ptr(weights), c_int(tokens), c_int(experts),
@@ -2696,7 +2697,7 @@ def moe_route_grouped(x: Tensor, router_weight: Tensor, correction: Tensor | Non
         _gpu(correction, "correction", torch.float32)
         if correction.shape != (experts,):
             raise KernelError(f"correction must be [{experts}]")
-    logits = linear(x, router_weight, out_dtype=torch.float32)
+    logits = linear(x, router_weight, out_dtype=torch.float32, ring=False)
     chosen = torch.empty((tokens, top), dtype=torch.int32, device=x.device)
     weights = torch.empty((tokens, top), dtype=torch.float32, device=x.device)
     _call("moe", "fe_moe_select_grouped", _ptr(logits), c_longlong(logits.shape[1]), _ptr(correction), _ptr(chosen), _ptr(weights),
@@ -2782,7 +2783,7 @@ def moe_experts(x: Tensor, chosen: Tensor | None, weights: Tensor, gate_up: Tens
 def linear_gated(x: Tensor, gate_up_weight: Tensor, *, limit: float, alpha: float) -> Tensor:
     """``min(g, limit) * sigmoid(alpha * min(g, limit)) * (clamp(u, -limit, limit) + 1)`` with g and u the two
     halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype."""
-    gate_up = linear(x, gate_up_weight)
+    gate_up = linear(x, gate_up_weight, ring=False)
     tokens, width = gate_up.shape
     if width % 2 or not limit > 0.0:
         raise KernelError("a gated weight needs an even number of rows and a positive limit")

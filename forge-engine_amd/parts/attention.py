@@ -376,7 +376,7 @@ class GroupedQueryAttention(Mixer):
         if writes_cache != self.own_kv or (not writes_cache and self.whole_norm_eps is None):
             raise ValueError("the general attention path writes its own keys and values, except for a layer that "
                              "has none and reads another call's")
-        qkv = ops.linear(x, self.qkv_weight)        # [T, q | k | v (| gate)]; the bias is added by the kernel below
+        qkv = ops.linear(x, self.qkv_weight, ring=False)        # [T, q | k | v (| gate)]; the bias is added by the kernel below
         out_size = self.out_size if self.output_gate else self.num_heads * self.value_row
         attn = torch.empty((x.shape[0], out_size), dtype=x.dtype, device=x.device)
         self._attend(qkv, attn, batch, cache, writes_cache, inv_freq, rotary_dim)

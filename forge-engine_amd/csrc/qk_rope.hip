@@ -138,20 +138,50 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_kernel(
   }
 }
 
-// The same for bfloat16 heads of 16 * 2^n elements that are rotated whole (rotary_dim == head_dim):
-// head_dim / 8 lanes share a head, each with 8 consecutive elements (one 16-byte load and store),
-// so a wave works on 512 / head_dim heads at once; the partner of element j, j + head_dim / 2,
-// sits in the lane head_dim / 16 further on (one shuffle per element).
-#define VEC_ROUNDS 3   // rounds of 2048 / head_dim heads that a block of the kernel below takes at most
-template <int LPH>    // lanes per head
+// 16 bytes of a head: eight bfloat16 elements, in the arithmetic of rope_math.h, or four float32 ones.
+__device__ __forceinline__ void unpack(const uint4& raw, float (&v)[8]) {
+  const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+  unpack_bf16x8(w4, v);
+}
+__device__ __forceinline__ void unpack(const uint4& raw, float (&v)[4]) {
+  v[0] = __uint_as_float(raw.x); v[1] = __uint_as_float(raw.y); v[2] = __uint_as_float(raw.z); v[3] = __uint_as_float(raw.w);
+}
+__device__ __forceinline__ uint4 pack(const float (&v)[8]) {
+  uint32_t w4[4];
+  pack_bf16x8(v, w4);
+  return make_uint4(w4[0], w4[1], w4[2], w4[3]);
+}
+__device__ __forceinline__ uint4 pack(const float (&v)[4]) {
+  return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
+}
+__device__ __forceinline__ float sum_squares(const float (&v)[8]) { return sum_squares8(v); }
+__device__ __forceinline__ float sum_squares(const float (&v)[4]) {
+  return __fmaf_rn(v[3], v[3], __fmaf_rn(v[2], v[2], __fmaf_rn(v[1], v[1], v[0] * v[0])));
+}
+__device__ __forceinline__ bf16_t element(const uint4& raw, int e, bf16_t) {
+  const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+  return (bf16_t)(e & 1 ? w4[e >> 1] >> 16 : w4[e >> 1] & 0xffffu);
+}
+__device__ __forceinline__ float element(const uint4& raw, int e, float) {
+  const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+  return __uint_as_float(w4[e]);
+}
+
+// The same for heads of 64, 128 or 256 elements that are rotated whole (rotary_dim == head_dim): LPH lanes share a head, each with
+// 16 bytes of consecutive elements (one load and store), so a block works on 256 / LPH heads at once; the partner of element j,
+// j + head_dim / 2, sits in the lane LPH / 2 further on (one shuffle per element).
+// Bound by latency with few tokens, by the rows' bytes with many.  float32, an element a lane and values token by token -> this: 700
+// tokens of 32 heads of 128 15.4 -> 7.3 us, 2,048 30.9 -> 16.8, 64 3.9 -> 3.1.
+#define VEC_ROUNDS 3   // rounds of 256 / LPH heads that a block of the kernel below takes at most
+template <typename T, int LPH>    // lanes per head
 __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
-    bf16_t* __restrict__ qkv, const float* __restrict__ q_weight, const float* __restrict__ k_weight,
+    T* __restrict__ qkv, const float* __restrict__ q_weight, const float* __restrict__ k_weight,
     const float* __restrict__ inv_freq, const int* __restrict__ positions,
     const int* __restrict__ token_seq, const int* __restrict__ block_table, int table_stride,
-    bf16_t* __restrict__ key_pages, bf16_t* __restrict__ value_pages, int q_heads, int kv_heads,
+    T* __restrict__ key_pages, T* __restrict__ value_pages, int q_heads, int kv_heads,
     int block_size, int num_blocks, float eps, int write_kv, int heads_per_block, int groups_per_token,
     int tokens, int values_apart) {
-  constexpr int D = LPH * 8;
+  constexpr int E = 16 / sizeof(T), D = LPH * E;
   constexpr int HALF = D / 2;
   constexpr int HEADS_AT_ONCE = 256 / LPH;
   const int heads_all = q_heads + 2 * kv_heads;
@@ -161,8 +191,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
     // by token every element is a 2-byte store of its own, 2 * block_size bytes from the next.
     // Here 16 lanes write 16 neighbouring slots of one dim (tokens of one sequence follow one
     // another in the batch), which the memory system takes as one piece.
-    constexpr int PITCH = D + 8;            // elements; rows stay 16-byte aligned, columns spread over the banks
-    __shared__ __attribute__((aligned(16))) bf16_t rows[16][PITCH];
+    constexpr int PITCH = D + E;            // elements; rows stay 16-byte aligned, columns spread over the banks
+    __shared__ __attribute__((aligned(16))) T rows[16][PITCH];
     __shared__ long long slot_at[16];       // element offset of [page][kv_head][0][slot], or -1
     const int vb = blockIdx.x - tokens * groups_per_token;
     const int kv_head = vb % kv_heads;
@@ -181,8 +211,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
     for (int piece = threadIdx.x; piece < 16 * LPH; piece += 256) {
       const int row = piece / LPH, sub = piece % LPH;
       const int t = min(t0 + row, tokens - 1);
-      *(uint4*)&rows[row][sub * 8] =
-          *(const uint4*)(qkv + ((size_t)t * heads_all + q_heads + kv_heads + kv_head) * D + sub * 8);
+      *(uint4*)&rows[row][sub * E] =
+          *(const uint4*)(qkv + ((size_t)t * heads_all + q_heads + kv_heads + kv_head) * D + sub * E);
     }
     __syncthreads();
     const int row = threadIdx.x & 15;
@@ -195,8 +225,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
   const int t = blockIdx.x / groups_per_token;
   const int group = blockIdx.x - t * groups_per_token;
   const int head_end = min(values_apart ? q_heads + kv_heads : heads_all, (group + 1) * heads_per_block);
-  const int sub = threadIdx.x % LPH;          // which 8 elements of the head
-  const int first = sub * 8;
+  const int sub = threadIdx.x % LPH;          // which E elements of the head
+  const int first = sub * E;
   const bool low = first < HALF;              // elements of the first half pair with the second
   // A block's time is a chain of trips to memory, not bytes: the heads' elements, which depend on
   // nothing, are asked for before the position is (and with it the sines and cosines), for all of the
@@ -224,7 +254,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
   for (int round = 0; round < ROUNDS; ++round) {
     const int head = head_first + round * HEADS_AT_ONCE;
     if (head >= head_end) break;
-    bf16_t* x = qkv + ((size_t)t * heads_all + head) * D + first;
+    T* x = qkv + ((size_t)t * heads_all + head) * D + first;
     const bool is_q = head < q_heads;
     const bool is_k = !is_q && head < q_heads + kv_heads;
     if (!is_q && !write_kv) continue;
@@ -237,39 +267,32 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
       page = ((size_t)block * kv_heads + kv_head) * block_size * D;
       slot = pos % block_size;
       if (!is_k) {   // value: into the transposed page, element d at [d][slot]
-        const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
-        bf16_t* vdst = value_pages + page + slot;
+        T* vdst = value_pages + page + slot;
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          vdst[(size_t)(first + e) * block_size] = (bf16_t)(e & 1 ? w4[e >> 1] >> 16 : w4[e >> 1] & 0xffffu);
+        for (int e = 0; e < E; ++e) vdst[(size_t)(first + e) * block_size] = element(raw, e, T());
         continue;
       }
     }
-    float v[8];
-    {
-      const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
-      unpack_bf16x8(w4, v);
-    }
+    float v[E];
+    unpack(raw, v);
     const float* w = is_q ? q_weight : k_weight;
     if (w) {
-      float sumsq = sum_squares8(v);
+      float sumsq = sum_squares(v);
 #pragma unroll
       for (int offset = LPH / 2; offset > 0; offset >>= 1) sumsq += __shfl_xor(sumsq, offset, FE_WAVE);
       const float inv = inverse_rms(sumsq, D, eps);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = normalise(v[e], inv, w[first + e]);
+      for (int e = 0; e < E; ++e) v[e] = normalise(v[e], inv, w[first + e]);
     }
-    uint32_t o4[4];
-    float r[8];
+    float r[E];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < E; ++e) {
       const float other = __shfl_xor(v[e], LPH / 2, FE_WAVE);     // element first + e -/+ HALF
       const int j = (first + e) & (HALF - 1);
       r[e] = low ? rotate_low(v[e], other, cos_s[j], sin_s[j]) : rotate_high(v[e], other, cos_s[j], sin_s[j]);
     }
-    pack_bf16x8(r, o4);
-    bf16_t* dst = is_q ? x : key_pages + page + (size_t)slot * D + first;
-    *(uint4*)dst = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+    T* dst = is_q ? x : key_pages + page + (size_t)slot * D + first;
+    *(uint4*)dst = pack(r);
   }
 }
 
@@ -288,29 +311,33 @@ extern "C" int fe_qk_norm_rope_write(void* qkv, int dtype, const float* q_weight
   if (work <= 0 || work > 0x7fffffffLL) return FE_BAD_ARGUMENT;
   // few tokens: four heads a block, so that the launch has many blocks; many tokens: a block per
   // token, so that the angles' sines and cosines are computed once per token (the vector kernel:
-  // one round of heads a block with few tokens, with many up to VEC_ROUNDS rounds, 48 heads of 128)
+  // one round of heads a block with few tokens, with many up to VEC_ROUNDS rounds, 48 heads of 128 in bfloat16)
   const int heads_all = q_heads + 2 * kv_heads;
-  const bool vec = dtype == FE_BF16 && rotary_dim == head_dim && (head_dim == 64 || head_dim == 128 || head_dim == 256) &&
+  const bool vec = (dtype == FE_BF16 || dtype == FE_F32) && rotary_dim == head_dim && (head_dim == 64 || head_dim == 128 || head_dim == 256) &&
                    ((((uintptr_t)qkv) | ((uintptr_t)key_pages)) & 15) == 0;
-  // the vector kernel works on 2048 / head_dim heads at once
-  const int heads_per_block = vec ? std::min(heads_all, (tokens >= 256 ? VEC_ROUNDS : 1) * (2048 / head_dim))
+  // the vector kernel works on 256 / LPH heads at once
+  const int heads_per_block = vec ? std::min(heads_all, (tokens >= 256 ? VEC_ROUNDS : 1) * ((dtype == FE_BF16 ? 2048 : 1024) / head_dim))
                                   : (tokens >= 256 ? heads_all : 4);
   const int groups_per_token = (heads_all + heads_per_block - 1) / heads_per_block;
   long long blocks = (long long)tokens * groups_per_token;
   if (blocks > 0x7fffffffLL) return FE_BAD_ARGUMENT;
   if (vec) {
-    // with many tokens the values go to blocks of their own that write 16 slots of a page at a time
-    const int values_apart = write_kv && kv_heads > 0 && tokens >= 256;
+    // with many tokens the values go to blocks of their own that write 16 slots of a page at a time (float32, whose element by element
+    // stores are twice as many for the same bytes, from the second such block on: 20 tokens tie, 255 7.6 -> 4.2 us)
+    const int values_apart = write_kv && kv_heads > 0 && tokens >= (dtype == FE_F32 ? 17 : 256);
     if (values_apart) blocks += (long long)((tokens + 15) / 16) * kv_heads;
     if (blocks > 0x7fffffffLL) return FE_BAD_ARGUMENT;
-#define FE_GO(LPH)                                                                                          \
-  qk_norm_rope_write_vec_kernel<LPH><<<(unsigned)blocks, 256, 0, stream>>>(                                   \
-      (bf16_t*)qkv, q_weight, k_weight, inv_freq, positions, token_seq, block_table, table_stride,            \
-      (bf16_t*)key_pages, (bf16_t*)value_pages, q_heads, kv_heads, block_size, num_blocks, eps, write_kv,     \
+#define FE_GO(T, LPH)                                                                                       \
+  qk_norm_rope_write_vec_kernel<T, LPH><<<(unsigned)blocks, 256, 0, stream>>>(                                \
+      (T*)qkv, q_weight, k_weight, inv_freq, positions, token_seq, block_table, table_stride,                 \
+      (T*)key_pages, (T*)value_pages, q_heads, kv_heads, block_size, num_blocks, eps, write_kv,               \
       heads_per_block, groups_per_token, tokens, values_apart)
-    if (head_dim == 64) FE_GO(8);
-    else if (head_dim == 128) FE_GO(16);
-    else FE_GO(32);
+    if (dtype == FE_F32 && head_dim == 64) FE_GO(float, 16);
+    else if (dtype == FE_F32 && head_dim == 128) FE_GO(float, 32);
+    else if (dtype == FE_F32) FE_GO(float, 64);
+    else if (head_dim == 64) FE_GO(bf16_t, 8);
+    else if (head_dim == 128) FE_GO(bf16_t, 16);
+    else FE_GO(bf16_t, 32);
 #undef FE_GO
     return fe_check_launch();
   }

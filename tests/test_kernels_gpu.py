@@ -265,7 +265,7 @@ def _qk_case(g, dtype, tokens, q_heads, kv_heads, head_dim, block_size, num_bloc
     (2, 1, 48, 5, 0), (4, 2, 64, 8, 64), (32, 8, 128, 16, 128),
     (64, 16, 128, 16, 128), (20, 4, 256, 32, 256),       # more heads than a block of the vector kernel takes: two blocks a token
 ])
-@pytest.mark.parametrize("tokens", [11, 300])       # few tokens: four heads a block; many: a block per token
+@pytest.mark.parametrize("tokens", [11, 17, 300])   # few tokens: four heads a block; many: a block per token; 17: float32 values in blocks of their own
 def test_qk_norm_rope_write(ops, dtype, q_heads, kv_heads, head_dim, block_size, rotary_dim, tokens):
     g = torch.Generator().manual_seed(5)
     num_blocks = 2 * ((tokens + 5) // block_size + 2)

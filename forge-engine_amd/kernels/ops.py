@@ -2653,10 +2653,7 @@ _SCORINGS = {"softmax": 0, "sigmoid": 1}
 _GATED_FORMS = {"bounded": 0, "silu": 1, "relu_squared": 2}
 
 
-def moe_route(x: Tensor, router_weight: Tensor, router_bias: Tensor | None, top: int, scoring: str = "softmax") -> tuple[Tensor, Tensor]:
-    """Router logits ``x W^T + b`` in float32; for every token the ``top`` experts with the largest logits
-    (int32 [T, top], largest first, the lowest index among equals) and their weights (float32 [T, top]): the
-    softmax over the chosen logits alone, or (``scoring`` "sigmoid") each chosen logit's own sigmoid."""
+def _router_logits(x: Tensor, router_weight: Tensor, router_bias: Tensor | None, top: int) -> Tensor:
     _gpu(x, "x")
     _gpu(router_weight, "router_weight", x.dtype)
     tokens, hidden = x.shape
@@ -2667,12 +2664,36 @@ def moe_route(x: Tensor, router_weight: Tensor, router_bias: Tensor | None, top:
         _gpu(router_bias, "router_bias", torch.float32)
         if router_bias.shape != (experts,):
             raise KernelError(f"router_bias must be [{experts}]")
-    logits = linear(x, router_weight, out_dtype=torch.float32, ring=False)     # float32 accumulation, float32 logits
+    return linear(x, router_weight, out_dtype=torch.float32, ring=False)     # float32 accumulation, float32 logits
+
+
+def moe_route(x: Tensor, router_weight: Tensor, router_bias: Tensor | None, top: int, scoring: str = "softmax") -> tuple[Tensor, Tensor]:
+    """Router logits ``x W^T + b`` in float32; for every token the ``top`` experts with the largest logits
+    (int32 [T, top], largest first, the lowest index among equals) and their weights (float32 [T, top]): the
+    softmax over the chosen logits alone, or (``scoring`` "sigmoid") each chosen logit's own sigmoid."""
+    logits = _router_logits(x, router_weight, router_bias, top)
+    tokens, experts = logits.shape
     chosen = torch.empty((tokens, top), dtype=torch.int32, device=x.device)
     weights = torch.empty((tokens, top), dtype=torch.float32, device=x.device)
     _call("moe", "fe_moe_select", _ptr(logits), _ptr(router_bias), _ptr(chosen), _ptr(weights), c_int(tokens), c_int(experts),
           c_int(top), c_int(_SCORINGS[scoring]), _stream())
     return chosen, weights
+
+
+def moe_route_plan(x: Tensor, router_weight: Tensor, router_bias: Tensor | None, top: int,
+                   scoring: str = "softmax") -> tuple[Tensor | None, Tensor, tuple[Tensor, Tensor] | None]:
+    """``moe_route`` with the plan that ``moe_experts`` takes, (offsets, order): (chosen, weights, None), or where the step has few enough
+    tokens and experts for one launch to choose and sort, (None, weights, plan)."""
+    tokens, experts = x.shape[0], router_weight.shape[0]
+    if not (0 < tokens <= 64 and experts <= 64 and 1 <= top <= min(experts, 16) and tokens * top <= 256):
+        return *moe_route(x, router_weight, router_bias, top, scoring), None
+    logits = _router_logits(x, router_weight, router_bias, top)
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device=x.device)
+    order = torch.empty(tokens * top, dtype=torch.int32, device=x.device)
+    weights = torch.empty((tokens, top), dtype=torch.float32, device=x.device)
+    _call("moe", "fe_moe_select_plan", _ptr(logits), _ptr(router_bias), _ptr(offsets), _ptr(order), _ptr(weights), c_int(tokens),
+          c_int(experts), c_int(top), c_int(_SCORINGS[scoring]), _stream())
+    return None, weights, (offsets, order)
 
 
 def moe_route_grouped(x: Tensor, router_weight: Tensor, correction: Tensor | None, *, experts: int, top: int, groups: int = 1,

@@ -201,7 +201,7 @@ class RoutedExperts(FeedForward):
                 top=self.top, groups=self.groups, keep=self.keep_groups, scale=self.route_scale)
             gate_logits, gate_column = logits, self.experts
         else:
-            chosen, weights = ops.moe_route(x, self.router_weight, self.router_bias, self.top, self.scoring)
+            chosen, weights, plan = ops.moe_route_plan(x, self.router_weight, self.router_bias, self.top, self.scoring)
             if self.shared_gate:
                 gate_logits = ops.linear(x, self.router_rows[self.experts:], out_dtype=torch.float32)
         shared = None

@@ -669,6 +669,16 @@ def moe_route(x, router_weight, router_bias, top, scoring="softmax"):
     return best.indices.to(torch.int32), weights
 
 
+def moe_route_plan(x, router_weight, router_bias, top, scoring="softmax"):
+    chosen, weights = moe_route(x, router_weight, router_bias, top, scoring)
+    if x.shape[0] > 64 or router_weight.shape[0] > 64 or chosen.numel() > 256:
+        return chosen, weights, None
+    flat = chosen.reshape(-1).long()
+    counts = torch.bincount(flat, minlength=router_weight.shape[0])
+    offsets = torch.cat([torch.zeros(1, dtype=torch.long), torch.cumsum(counts, 0)]).to(torch.int32)
+    return None, weights, (offsets, torch.argsort(flat, stable=True).to(torch.int32))
+
+
 def _gated(g, u, limit, alpha, form="bounded"):
     if form == "silu":
         return g * torch.sigmoid(g) * u
@@ -973,7 +983,7 @@ NAMES = ("cap_rows", "gate_heads", "latent_row_sizes", "latent_step_fits", "late
          "qk_norm_rope_write", "paged_attention", "argmax_rows", "sample_filtered_rows",
          "cast_rows", "add_bias", "token_shift", "rmsnorm_update", "rmsnorm_mean", "polynorm", "tanh_rows", "head_norm_gate",
          "conv_rope_norm_write", "masked_attention", "linear_recurrence", "linear_recurrence_step_fits", "linear_recurrence_step", "mlstm_gate_scan",
-         "hyper_norm", "embed_token_pairs", "scale_rows", "whole_norm_rope_write", "moe_route", "moe_experts", "linear_gated",
+         "hyper_norm", "embed_token_pairs", "scale_rows", "whole_norm_rope_write", "moe_route", "moe_route_plan", "moe_experts", "linear_gated",
          "relu_squared", "causal_conv_act", "selective_scan", "rmsnorm_update_norm", "layernorm_update", "activate", "gate_rows",
          "latent_norm_rope_write", "latent_query_pack", "latent_attention", "heads_product", "moe_route_grouped",
          "rotary_table", "head_recurrence", "head_recurrence_gated", "gated_group_norm", "stream_sum_cast", "moe_plan_table")

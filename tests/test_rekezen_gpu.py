@@ -170,6 +170,28 @@ def test_mixture_of_experts_kernels(tokens, hidden, experts, top, inner, dtype):
     close(ops.linear_gated(x.to(DEV), shared.to(DEV), limit=0.8, alpha=1.702), refs.linear_gated(x, shared, limit=0.8, alpha=1.702), dtype)
 
 
+# the smallest, most tokens, experts, pairs and choices, and one of each too many
+@pytest.mark.parametrize("scoring,biased", [("softmax", True), ("sigmoid", False)])
+@pytest.mark.parametrize("tokens,experts,top", [(1, 1, 1), (8, 8, 2), (64, 64, 4), (16, 17, 16), (64, 3, 3), (65, 8, 2), (8, 65, 2), (33, 64, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_routing_with_its_plan_chooses_as_without(tokens, experts, top, scoring, biased, dtype):
+    from forge_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(tokens + experts)
+    x, router = torch.randn(tokens, 128, generator=g).to(DEV, dtype), torch.randn(experts, 128, generator=g).to(DEV, dtype)
+    router[experts // 2] = router[0]           # equal logits: the lowest index
+    bias = torch.randn(experts, generator=g).to(DEV) if biased else None
+    chosen, weights = ops.moe_route(x, router, bias, top, scoring)
+    none, got_weights, plan = ops.moe_route_plan(x, router, bias, top, scoring)
+    assert torch.equal(got_weights, weights)
+    if tokens > 64 or experts > 64 or tokens * top > 256:
+        assert plan is None and torch.equal(none, chosen)
+        return
+    flat = chosen.reshape(-1).long()
+    counts = torch.bincount(flat, minlength=experts)
+    assert none is None and torch.equal(plan[0][1:], torch.cumsum(counts, 0).int()) and int(plan[0][0]) == 0
+    assert torch.equal(plan[1], torch.argsort(flat, stable=True).int())
+
+
 @pytest.mark.parametrize("tokens,hidden,experts,top,inner", [
     (3, 96, 130, 2, 33), (40, 128, 70, 3, 100),                 # more experts than a wave has lanes, few rows each
     (65, 160, 2, 1, 70), (150, 64, 3, 2, 130),                  # 32 to 100 rows an expert

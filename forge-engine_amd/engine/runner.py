@@ -212,6 +212,7 @@ class ModelRunner:
         self.embedding_states: dict[str, Tensor] = {
             name: torch.zeros((num_state_slots + 1, *state.shape), dtype=state.dtype or torch.float32, device=self.device)
             for name, state in model.embedding_needs().states().items()}
+        self._slot_states = ops.SlotStates([state for states in [*self.states, self.embedding_states] for state in states.values()])
         self.pad_state_slot = num_state_slots
         self.steps_run = 0
         self.workspace = ops.Workspace()    # scratch that this runner's launches (and its captured graphs) share
@@ -221,9 +222,8 @@ class ModelRunner:
         """Lease a state slot and empty tables for the request.  The slot's fixed-size state starts
         at zero: the runner clears it here, so a mixer never has to know a request's first step."""
         record = self.cache.begin(request_id)
-        for states in [*self.states, self.embedding_states]:
-            for state in states.values():
-                state[record.state_slot].zero_()
+        if self._slot_states.states:
+            self._slot_states.zero(record.state_slot)
 
     def end(self, request_id: str) -> None:
         self.cache.end(request_id)

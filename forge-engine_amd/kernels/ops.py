@@ -1663,6 +1663,28 @@ def _parts_of(update: Tensor, rows: int, width: int, name: str) -> int:
     raise KernelError(f"{name} must be [{rows}, {width}] or [parts <= 64, {rows}, {width}], got {tuple(update.shape)}")
 
 
+class SlotStates:
+    """The fixed-size states of a runner, [slots, ...] each, one row of which a request begins with at zero."""
+
+    def __init__(self, states: list[Tensor]) -> None:
+        self.states = states
+        rows = [(t.data_ptr(), t[0].numel() * t.element_size()) for t in states]
+        self.slots = min((t.shape[0] for t in states), default=0)
+        self.together = bool(states) and all(t.is_cuda and t.is_contiguous() and size % 4 == 0 and at % 4 == 0 for t, (at, size) in zip(states, rows))
+        if self.together:
+            self.most = max(size for _, size in rows)
+            self.table = torch.tensor(rows, dtype=torch.int64).to(states[0].device)
+
+    def zero(self, slot: int) -> None:
+        if not 0 <= slot < max(1, self.slots):
+            raise KernelError(f"slot {slot} of {self.slots}")
+        if self.together:
+            _call("stream_ops", "fe_zero_slots", _ptr(self.table), c_int(len(self.states)), c_longlong(self.most), c_int(slot), _stream())
+        else:
+            for state in self.states:
+                state[slot].zero_()
+
+
 def token_shift(x: Tensor, weights: Tensor, state: Tensor, cu_q: Tensor, token_seq: Tensor, state_slots: Tensor, *,
                 num_seqs: int, out_dtype) -> Tensor:
     """out[s, t] = x[t] + (x'[t] - x[t]) * weights[s]: x' is the row before within the token's

@@ -327,3 +327,22 @@ def test_mlstm_gate_scan(ops, heads):
                               num_seqs=len(lengths), heads=heads)
     torch.testing.assert_close(got.cpu(), want, atol=1e-5, rtol=1e-4)
     torch.testing.assert_close(maximum_d.cpu(), maximum_ref, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("together", [True, False])
+def test_a_requests_states_from_zero(ops, together):
+    """Rows of one word, of words that end no 16-byte piece and start on none, of more pieces than a launch has threads; with a row of
+    an odd number of bytes among them, one by one."""
+    states = [torch.ones(5, device=DEV, dtype=torch.int32), torch.ones(5, 3, 7, device=DEV), torch.ones(5, 8, 129, 128, device=DEV),
+              torch.ones(5, 600, 4000, device=DEV), torch.ones(5, 6, device=DEV, dtype=torch.bfloat16)]
+    if not together:
+        states.append(torch.ones(5, 3, device=DEV, dtype=torch.bfloat16))
+    slots = ops.SlotStates(states)
+    assert slots.together == together
+    for slot in (4, 0):
+        slots.zero(slot)
+    for state in states:
+        assert not state[[0, 4]].any() and bool((state[1:4] == 1).all())
+    for slot in (-1, 5):
+        with pytest.raises(ops.KernelError):
+            slots.zero(slot)

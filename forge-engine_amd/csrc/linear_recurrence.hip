@@ -9,7 +9,7 @@
 // step may hold portions of prompts beside single tokens.
 //
 // Work split: block = 256 threads that share a head's staged tokens; a column of the state belongs to
-// L lanes (16 for key sizes up to 64, a whole wave of 64 beyond), each holding R key channels of it
+// L lanes (16 for key sizes up to 64, 32 up to 128, a whole wave of 64 beyond), each holding R key channels of it
 // in registers for the whole walk, so a block owns 16 or 4 columns and the lanes of a column meet by
 // lane permutes.  Tokens are staged 16 at a time through LDS (q, k, the decay per key channel, v
 // times the input scale, the per-head decay); the next chunk's loads are issued into registers
@@ -27,11 +27,15 @@
 #define LR_THREADS 256
 #define LR_CHUNK 16
 
-__device__ __forceinline__ float sum_16_lanes(float v) {
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));    // lane ^ 1
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));    // lane ^ 2
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));   // 7 - lane within 8
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));   // 15 - lane within 16
+template <int L>
+__device__ __forceinline__ float sum_lanes(float v) {
+  static_assert(L == 4 || L == 8 || L == 16 || L == 32 || L == 64, "a power of two from four");
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));                  // lane ^ 1
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));                  // lane ^ 2
+  if (L >= 8) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));     // 7 - lane within 8
+  if (L >= 16) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));    // 15 - lane within 16
+  if (L >= 32) v = sum_xor16(v);
+  if (L >= 64) v = sum_xor32(v);
   return v;
 }
 
@@ -164,7 +168,7 @@ __global__ __launch_bounds__(LR_THREADS) void linear_recurrence_kernel(Recurrenc
           acc = fmaf(S[m], Qs[tt][i], acc);
         }
       }
-      return L == 16 ? sum_16_lanes(acc) : wave_sum_dpp(acc);
+      return sum_lanes<L>(acc);
     };
     const int count = min(CH, end - t0);
     if (count == CH) {      // a whole chunk, unrolled: the LDS reads of later tokens overlap the sums of earlier ones
@@ -241,7 +245,10 @@ extern "C" int fe_linear_recurrence(const void* q, const void* k, const void* v,
   else if (key_dim <= 32) launch_recurrence<16, 2>(p, columns, num_seqs, stream);
   else if (key_dim <= 48) launch_recurrence<16, 3>(p, columns, num_seqs, stream);
   else if (key_dim <= 64) launch_recurrence<16, 4>(p, columns, num_seqs, stream);
-  else if (key_dim <= 128) launch_recurrence<64, 2>(p, columns, num_seqs, stream);
+  // 32 lanes: ten instructions a column and token instead of fifteen for 64 (nine for 16, whose longer chain a token costs more where few walks
+  // run).  us, 64 -> 32 lanes (16): 8 heads of 128 x 257, 500, 338, .. 70 tokens 156 -> 102 (97), 1 x 500 96 -> 78 (89), 16 x 100 177 -> 113
+  // (111); 4 heads 82 -> 68 (90), 77 -> 66 (87), 95 -> 61 (66); 4 heads of 100 x 64 63 -> 65 (87).
+  else if (key_dim <= 128) launch_recurrence<32, 4>(p, columns, num_seqs, stream);
   else if (key_dim <= 192) launch_recurrence<64, 3>(p, columns, num_seqs, stream);
   else launch_recurrence<64, 4>(p, columns, num_seqs, stream);
   return fe_check_launch();
@@ -264,18 +271,6 @@ struct StepEnding {
   float cap, tau, eps;
   int decay_kind, weight_len, act;
 };
-
-template <int L>
-__device__ __forceinline__ float sum_lanes(float v) {
-  static_assert(L == 4 || L == 8 || L == 16 || L == 32 || L == 64, "a power of two from four");
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));                  // lane ^ 1
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));                  // lane ^ 2
-  if (L >= 8) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));     // 7 - lane within 8
-  if (L >= 16) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));    // 15 - lane within 16
-  if (L >= 32) v = sum_xor16(v);
-  if (L >= 64) v = sum_xor32(v);
-  return v;
-}
 
 constexpr int STEP_MAX_VALUES = 512;
 

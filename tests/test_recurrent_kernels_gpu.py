@@ -311,6 +311,30 @@ def test_linear_recurrence_step(ops, dtype, form, heads, key_dim, value_dim):
         torch.testing.assert_close(tensors_d["maximum"].cpu(), maximum, atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("lengths", [[40] * 10 + [0, 1], [400, 1, 5]])     # chunks of 16 tokens whole and not, columns that fill no block
+@pytest.mark.parametrize("form", ["plain", "mlstm", "rwkv"])
+@pytest.mark.parametrize("key_dim,value_dim", [(128, 256), (96, 250), (65, 251)])
+def test_linear_recurrence_of_many_and_few_walks(ops, lengths, form, key_dim, value_dim):
+    g = torch.Generator().manual_seed(13)
+    heads, tokens, ones = 2, sum(lengths), form == "mlstm"
+    cu, _, slots = layout(lengths, list(range(len(lengths))))
+    q, k, v = (rand(g, tokens, heads * n) for n in (key_dim, key_dim, value_dim))
+    state = rand(g, len(lengths) + 1, heads, value_dim + ones, key_dim)
+    options = dict(num_seqs=len(lengths), max_q_len=max(lengths), heads=heads, key_dim=key_dim, value_dim=value_dim, q_scale=key_dim ** -0.5,
+                   ones_column=ones)
+    extra = dict(head_decay=torch.rand(tokens, heads, generator=g), in_scale=torch.rand(tokens, heads, generator=g))
+    if form == "rwkv":
+        extra = dict(decay=rand(g, tokens, heads * key_dim), decay_kind="exp_neg_exp", decay_bias=rand(g, heads * key_dim) - 1.0,
+                     bonus=rand(g, heads, key_dim))
+    state_d, cu_d, slots_d = dev(state, cu, slots)
+    extra_d = {n: (t.to(DEV) if isinstance(t, torch.Tensor) else t) for n, t in extra.items()}
+    got = ops.linear_recurrence(q.to(DEV), k.to(DEV), v.to(DEV), torch.zeros(tokens, heads, value_dim + ones, device=DEV), state_d, cu_d, slots_d,
+                                **options, **extra_d)
+    want = refs.linear_recurrence(q, k, v, torch.zeros(tokens, heads, value_dim + ones), state, cu, slots, **options, **extra)
+    torch.testing.assert_close(got.cpu(), want, atol=1e-4, rtol=1e-4)
+    torch.testing.assert_close(state_d.cpu(), state, atol=1e-4, rtol=1e-4)
+
+
 @pytest.mark.parametrize("heads", [1, 2, 5])
 def test_mlstm_gate_scan(ops, heads):
     g = torch.Generator().manual_seed(11)

@@ -15,7 +15,9 @@ static inline int row_threads(int rows, int width) { return rows <= FEW_ROWS && 
 // ---------------------------------------------------------------- token shift
 // out[s][t][c] = x[t][c] + (prev[t][c] - x[t][c]) * w[s][c]; prev = x[t - 1] inside the token's
 // sequence, the sequence's state row for its first token of the step.
-template <typename TX, typename TO>
+// COUNT: the blends of a call, if the kernel was made for them (0: any): their weights then arrive in one trip (six rows of 2,048, five
+// blends, in a captured step 5.80 -> 3.08 us; 1,393 rows 21.05 -> 11.18).
+template <typename TX, typename TO, int COUNT>
 __global__ __launch_bounds__(ROW_THREADS_FEW) void token_shift_kernel(
     const TX* __restrict__ x, const float* __restrict__ w, float* __restrict__ state,
     const int* __restrict__ cu_q, const int* __restrict__ token_seq, const int* __restrict__ state_slots,
@@ -33,8 +35,16 @@ __global__ __launch_bounds__(ROW_THREADS_FEW) void token_shift_kernel(
     const float v = load_as_float(row + c);
     const float p = first ? kept[c] : load_as_float(before + c);
     const float d = p - v;
-    for (int s = 0; s < count; ++s)
-      store_from_float(out + ((size_t)s * tokens + t) * width + c, v + d * w[(size_t)s * width + c]);
+    if constexpr (COUNT > 0) {
+      float weights[COUNT];
+#pragma unroll
+      for (int s = 0; s < COUNT; ++s) weights[s] = w[(size_t)s * width + c];
+#pragma unroll
+      for (int s = 0; s < COUNT; ++s) store_from_float(out + ((size_t)s * tokens + t) * width + c, v + d * weights[s]);
+    } else {
+      for (int s = 0; s < count; ++s)
+        store_from_float(out + ((size_t)s * tokens + t) * width + c, v + d * w[(size_t)s * width + c]);
+    }
     if (saves) kept[c] = load_as_float(final + c);
   }
 }
@@ -44,15 +54,17 @@ extern "C" int fe_token_shift(const void* x, int x_dtype, const float* weights, 
                               int width, int count, int slots, hipStream_t stream) {
   if (tokens <= 0) return FE_OK;
   if (width <= 0 || count < 1 || count > 8 || slots < 1) return FE_BAD_ARGUMENT;
-#define LAUNCH(TX, TO)                                                                                       \
-  token_shift_kernel<TX, TO><<<tokens, row_threads(tokens, width), 0, stream>>>((const TX*)x, weights, state, cu_q, token_seq, \
-                                                                  state_slots, (TO*)out, tokens, width, count, slots)
+#define GO(TX, TO, COUNT)                                                                                                              \
+  token_shift_kernel<TX, TO, COUNT><<<tokens, row_threads(tokens, width), 0, stream>>>((const TX*)x, weights, state, cu_q, token_seq,    \
+                                                                         state_slots, (TO*)out, tokens, width, count, slots)
+#define LAUNCH(TX, TO) do { if (count == 1) GO(TX, TO, 1); else if (count == 5) GO(TX, TO, 5); else GO(TX, TO, 0); } while (0)
   if (x_dtype == FE_F32 && out_dtype == FE_F32) LAUNCH(float, float);
   else if (x_dtype == FE_F32 && out_dtype == FE_BF16) LAUNCH(float, bf16_t);
   else if (x_dtype == FE_BF16 && out_dtype == FE_BF16) LAUNCH(bf16_t, bf16_t);
   else if (x_dtype == FE_BF16 && out_dtype == FE_F32) LAUNCH(bf16_t, float);
   else return FE_BAD_ARGUMENT;
 #undef LAUNCH
+#undef GO
   return fe_check_launch();
 }
 

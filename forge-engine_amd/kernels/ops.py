@@ -426,6 +426,25 @@ def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None,
     return y
 
 
+def linear_several(x: Tensor, weights: list[Tensor]) -> list[Tensor]:
+    """``linear`` of rows x[i] [M, K] and weight i, in one launch where they are few bfloat16 rows and two to four equal weights that a round of
+    blocks holds (see ``fe_gemm_ring_several`` for both sides' times)."""
+    first = weights[0]
+    n, k = first.shape
+    together = (2 <= len(weights) <= 4 and x.dim() == 3 and x.shape[0] == len(weights) and x.is_contiguous() and n * len(weights) <= UPDATE_NORM_MAX_WIDTH
+                and first.dtype == torch.bfloat16 and all(w.shape == first.shape and w.is_contiguous() for w in weights)
+                and all(_ring_operands_fit(x[i], w) for i, w in enumerate(weights)) and _ring_store_pays(x.shape[1], n, k))
+    if not together:
+        return [linear(x[i], w) for i, w in enumerate(weights)]
+    _gpu(x, "x", torch.bfloat16)
+    for w in weights:
+        _gpu(w, "weight", torch.bfloat16)
+    out = torch.empty((len(weights), x.shape[1], n), dtype=x.dtype, device=x.device)
+    _call("gemm_ring", "fe_gemm_ring_several", _ptr(x), (c_void_p * len(weights))(*(w.data_ptr() for w in weights)), _ptr(out), c_int(len(weights)),
+          c_int(x.shape[1]), c_int(n), c_int(k), _stream())
+    return list(out.unbind(0))
+
+
 # Measured on MI355X: a weight with few row tiles and a long K (the output and down projections: 160
 # tiles, K = 4096 and 9728) leaves CUs idle; parts of K of about twelve 128-steps each (three and
 # six parts), of equal length, summed by blocks of four waves, take 6.9 instead of 9.0 us and 13.1

@@ -970,6 +970,10 @@ def decode_prepare_supported(*args, **kwargs):
     return False        # on the CPU a step of single tokens takes the two references below in turn
 
 
+def linear_several(x, weights):
+    return [linear(x[i], w) for i, w in enumerate(weights)]
+
+
 def linear_in_parts(x, weight):
     return None
 
@@ -979,7 +983,7 @@ def linear_in_parts(x, weight):
 DECODE_SPLITS_TESTED = tuple(range(1, 65))
 
 
-NAMES = ("cap_rows", "gate_heads", "latent_row_sizes", "latent_step_fits", "latent_query_step", "latent_value_step", "decode_prepare_supported", "linear_in_parts", "embed_rows", "add_rmsnorm", "add_rows", "swiglu", "gemm_nt_f32", "linear", "linear_update", "linear_swiglu", "gemm_skinny",
+NAMES = ("cap_rows", "gate_heads", "latent_row_sizes", "latent_step_fits", "latent_query_step", "latent_value_step", "decode_prepare_supported", "linear_in_parts", "embed_rows", "add_rmsnorm", "add_rows", "swiglu", "gemm_nt_f32", "linear", "linear_several", "linear_update", "linear_swiglu", "gemm_skinny",
          "qk_norm_rope_write", "paged_attention", "argmax_rows", "sample_filtered_rows",
          "cast_rows", "add_bias", "token_shift", "rmsnorm_update", "rmsnorm_mean", "polynorm", "tanh_rows", "head_norm_gate",
          "conv_rope_norm_write", "masked_attention", "linear_recurrence", "linear_recurrence_step_fits", "linear_recurrence_step", "mlstm_gate_scan",

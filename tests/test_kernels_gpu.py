@@ -2042,3 +2042,19 @@ def test_prefill_attention_far_key_and_tile_edges(ops, row_sets, monkeypatch):
                               cu.to(DEV), ctx.to(DEV), table.to(DEV), num_seqs=1, max_q_len=length, q_heads=2, kv_heads=1,
                               head_dim=head_dim, scale=head_dim ** -0.5, num_decode=0).cpu().float()
     assert float((got[query, :head_dim] - vp[page, 0, :, slot].float()).abs().max()) > 0.1
+
+
+# rows of the last block of each weight beyond its columns, one to four groups of eight rows a block, fewer chunks of K than waves
+@pytest.mark.parametrize("weights", [2, 3, 4])
+@pytest.mark.parametrize("rows,n,k", [(1, 2048, 2048), (6, 1024, 1024), (8, 2047, 320), (9, 2048, 1088), (16, 700, 4096), (16, 130, 320), (3, 1, 512)])
+def test_several_products_in_one_launch(ops, rows, n, k, weights, monkeypatch):
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn(weights, rows, k, generator=g).bfloat16()
+    w = [(torch.randn(n, k, generator=g) * k ** -0.5).bfloat16() for _ in range(weights)]
+    taken, real_call = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda lib, name, *a: taken.append(name) or real_call(lib, name, *a))
+    got = ops.linear_several(x.to(DEV), [t.to(DEV) for t in w])
+    assert taken == ["fe_gemm_ring_several"]
+    for i in range(weights):
+        # float32 sums of up to 4,096 products of order one, rounded to bfloat16: a unit in the last place of eight bits
+        torch.testing.assert_close(got[i].cpu().float(), x[i].float() @ w[i].float().T, rtol=2 ** -7, atol=2e-3)

@@ -135,6 +135,22 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_split_kernel(
     }
     if (group == 0) barrier();
   } else {
+    // The small tiles are what up to 64 rows take, whose sums were FMAs before: theirs go into the whole every four steps, so that the
+    // instruction's cutting off stays small (20 rows through the 1.7B sizes: error against 64 bits 6.5e-7 -> 4.9e-7, with FMAs 4.9e-7).
+    floatx4 whole_sum[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) whole_sum[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto gather = [&]() {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          whole_sum[i][j] += acc[i][j];
+          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
       if (first + s < steps) load(first + s, s);
@@ -144,9 +160,15 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_split_kernel(
       if (step + STAGES - 1 < steps) load(step + STAGES - 1, before);
       take(step, stage);
       multiply();
+      if ((step - first) % 4 == 3) gather();
       before = stage;
       stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
+    gather();
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[i][j] = whole_sum[i][j];
   }
   if constexpr (KG > 1) {       // the groups' sums, added in the order of the groups
     __syncthreads();

@@ -1022,6 +1022,64 @@ def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int |
     return out
 
 
+def gemm_big(x: Tensor, weight: Tensor, ending: str, parts: int = 1, act: str = "silu") -> Tensor:
+    """x @ weight^T for bfloat16 rows in tiles of 256 x 256 (csrc/gemm_big.hip): ``"parts"`` float32 partial sums [parts, M, N] over
+    runs of whole 64-steps of K, or ``"gated"``: act(gate) * up [M, N / 2] for a fused gate/up weight (gate rows first; ``act`` as in
+    ``swiglu``)."""
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(weight, "weight", torch.bfloat16, contiguous=False)
+    gated = ending == "gated"
+    if not _big_fits(x, weight, gated):
+        raise KernelError("tiles of 256 x 256 take contiguous bfloat16 rows, K a multiple of 64, a multiple of four columns, aligned rows")
+    m, k = x.shape
+    if ending not in ("parts", "gated") or not 1 <= parts <= (1 if gated else min(64, k // 64)):
+        raise KernelError(f"no ending {ending!r} with {parts} parts")
+    n = weight.shape[0] // 2 if gated else weight.shape[0]
+    out = torch.empty((m, n) if gated else (parts, m, n), dtype=torch.bfloat16 if gated else torch.float32, device=x.device)
+    _call("gemm_big", "fe_gemm_big", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(n), c_int(k), c_longlong(weight.stride(0)),
+          c_longlong(n), c_int(int(gated)), c_int(parts), c_longlong(m * n), _gate_act(act), _stream())
+    return out
+
+
+def _big_fits(x: Tensor, weight: Tensor, gated: bool) -> bool:
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and x.shape[0] > 0
+            and weight.dim() == 2 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1] and x.shape[1] % 64 == 0
+            and x.shape[1] > 0 and weight.shape[0] % (8 if gated else 4) == 0 and weight.shape[0] > 0
+            and weight.stride(0) % 8 == 0 and weight.stride(0) < 1 << 22
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _big_gate_pays(rows: int, columns: int, k: int) -> bool:
+    """Whether tiles of 256 x 256 are the better ones for the gate/up product: where they fill their rounds of one a CU (a round of
+    tiles of 128 rows counted as 0.62), the more the longer K is.  Drawn over 7,093 random sizes of 200 to 8,192 rows in captured
+    graphs beside what takes them otherwise.  Time of the others over this one's, by the share of the rounds that is filled: K under 1,024 .86 at .1,
+    1.25 at .3, 1.4 from .4 on; to 2,048 1.05 at .45, 1.12 at .6, 1.2 from .75 on; to 4,096 .96 at .55, 1.07 at .65, 1.15 from .8 on.
+    Longer ones, which the library's tiles of the same size cut alike, from .8 on in more than one round 1.11, in one round .96."""
+    if k < 512:
+        return False
+    whole, halves, across = -(-rows // 256), -(-rows // 128), -(-columns // 128)
+
+    def rounds(tiles: int) -> int:
+        return -(-tiles // WIDE_CUS)
+
+    full = whole * across // WIDE_CUS * WIDE_CUS // whole
+    cost = min(rounds(whole * across), rounds(whole * full) + 0.62 * rounds(halves * (across - full)))
+    filled = rows * 2 * columns / (256 * 256 * WIDE_CUS * cost)
+    if k >= 4096:
+        return filled >= 0.8 and cost > 1.0
+    return filled >= (0.3 if k < 1024 else 0.57 if k < 2048 else 0.65)
+
+
+def _big_update_parts(rows: int, weight_rows: int, k: int) -> int:
+    """Parts of K in which tiles of 256 x 256 make an update faster than the rest does, or 0: a long K in two to seven parts that
+    fill three quarters of one round of the CUs (3,898 random updates with their norms in captured graphs: from K = 8,192 on 1.07 to 1.29
+    times as fast, 2,560 x 9,728 at 2,048 rows 117 -> 100 us; at K = 4,096 to 8,192 .88 to 1.01; in one part, where the library adds into the stream, 1.0)."""
+    tiles = -(-rows // 256) * -(-weight_rows // 256)
+    parts = WIDE_CUS // tiles if k >= 8192 else 0
+    return parts if 2 <= parts <= 7 and rows * weight_rows * parts >= 0.75 * WIDE_CUS * 256 * 256 else 0
+
+
 def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream: Tensor | None = None) -> Tensor | None:
     """The float32 product x @ weight^T (+ bias) as an update of the residual stream: [M, N], or
     partial sums [parts, M, N] that ``add_rmsnorm`` / ``add_rows`` add up.  Given the float32
@@ -1034,6 +1092,10 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
         tile, parts = _split_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS)
         return gemm_split(x, weight, parts, tile)
     plain_bf16 = bias is None and weight.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
+    if plain_bf16 and x.shape[0] > MID_ROWS and _big_fits(x, weight, False):
+        parts = _big_update_parts(x.shape[0], *weight.shape)
+        if parts:
+            return gemm_big(x, weight, "parts", parts)
     if plain_bf16 and _lds_fits(x, weight):
         plan = _lds_update(x.shape[0], *weight.shape)
         if plan is not None:
@@ -1166,7 +1228,8 @@ def _gate_block_columns(columns: int) -> int:
 # against the matrix library followed by `fe_swiglu`, microseconds at Qwen3-4B's widths (K = 2560, 9728 columns):
 # 1,024 rows 134 / 126, 1,536: 157 / 148, 2,048: 199 / 224, 2,560: 264 / 310, 3,072: 297 / 272, 4,096: 377 / 438,
 # 8,192: 793 / 755; at K = 4096 (12,288 columns) the library wins at every row count but one (2,048: 329 / 306,
-# 4,096: 683 / 590).  So: a short K, and the row counts of a prompt portion of 2,048 to 4,096 tokens.
+# 4,096: 683 / 590).  So: a short K, and the row counts of a prompt portion of 2,048 to 4,096 tokens, of the sizes that tiles of
+# 256 x 256 leave: those that fill too little of their rounds, K under 512 and columns that are no multiple of four.
 GATED_TILE_MIN_ROWS = 2048
 GATED_TILE_MAX_ROWS = 4096
 GATED_TILE_MAX_K = 3072
@@ -1184,6 +1247,8 @@ def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "
     _gpu(x, "x")
     _gpu(gate_up_weight, "gate_up_weight")
     rows = x.shape[0]
+    if rows > MID_ROWS and _big_fits(x, gate_up_weight, True) and _big_gate_pays(rows, gate_up_weight.shape[0] // 2, x.shape[1]):
+        return gemm_big(x, gate_up_weight, "gated", act=act)
     if (GATED_TILE_MIN_ROWS <= rows <= GATED_TILE_MAX_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16
             and x.is_contiguous() and x.shape[1] % 64 == 0 and x.shape[1] <= GATED_TILE_MAX_K and gate_up_weight.shape[0] % 2 == 0
             and gate_up_weight.dim() == 2 and gate_up_weight.stride(1) == 1 and gate_up_weight.stride(0) % 8 == 0
@@ -1752,7 +1817,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "gemm_big", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

@@ -466,3 +466,16 @@ def test_no_read_of_lds_is_under_way_at_a_barrier_behind_which_its_buffer_is_fil
     found = _reads_in_flight_at_barriers(listing.read_text())
     assert any(found.values())
     assert {name: at for name, at in found.items() if any(at)} == {}
+
+
+def test_large_tiles_leave_m0_to_their_loads(tmp_path):
+    """Nothing but the loads into LDS touches m0, which they leave as it is, and nothing goes to scratch memory."""
+    listing = tmp_path / "gemm_big.s"
+    flags = [flag for flag in build.HIPCC_FLAGS if flag != "-shared"]
+    subprocess.run([build.find_hipcc(), *flags, "-S", "--cuda-device-only", "-o", str(listing), str(build.SOURCE_DIR / "gemm_big.hip")],
+                   check=True, capture_output=True)
+    text = listing.read_text()
+    lines = [line.split(";")[0].strip() for line in text.splitlines()]
+    uses = [line for line in lines if re.search(r"\bm0\b", line)]
+    assert uses and all(line.startswith("s_mov_b32 m0, s") for line in uses)
+    assert not any(line.startswith(("scratch_", "buffer_store", "buffer_load")) for line in lines)

@@ -209,11 +209,49 @@ SPLIT_MIN_ROWS = 16            # layers take it from here on where ``_split_pays
 SPLIT_MOST_PARTS = 6
 
 
+# The same with a split ahead, by a launch of its own (csrc/gemm_planes.hip), for more than 64 rows: 16 rows of a, 64 rows of b a block takes, and
+# the microseconds of a round of one block a CU (of the first tile, whose blocks share a CU in pairs, also of two) and of a step of 64 of K in it.
+PLANES_TILES = {(4, 1): (4.0, 0.69, 1.19), (4, 2): (4.9, 1.18, None), (5, 2): (5.7, 1.32, None), (6, 1): (4.3, 0.95, None),
+                (6, 2): (6.3, 1.41, None), (7, 2): (7.1, 1.58, None), (8, 1): (5.0, 1.02, None), (8, 2): (7.3, 1.72, None),
+                (9, 1): (5.3, 1.11, None), (10, 1): (5.5, 1.26, None)}
+
+
 def _split_fits(a: Tensor, b: Tensor) -> bool:
     return (a.dtype == torch.float32 and b.dtype == torch.float32 and a.dim() == 2 and b.dim() == 2 and a.shape[0] > 0
             and a.shape[1] == b.shape[1] and a.shape[1] >= SPLIT_MIN_K and a.shape[1] % 4 == 0 and a.stride(1) == 1 and b.stride(1) == 1
             and a.stride(0) % 4 == 0 and b.stride(0) % 4 == 0 and a.stride(0) >= a.shape[1] and b.stride(0) >= b.shape[1]
             and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0)
+
+
+def _planes_fit(a: Tensor, b: Tensor) -> bool:
+    return 6 * a.shape[0] * (a.shape[1] + 63) < 1 << 32 and b.stride(0) < 1 << 22
+
+
+@functools.lru_cache(maxsize=4096)
+def _product_plan(m: int, n: int, k: int, most_parts: int, planes: bool) -> tuple[int | tuple[int, int], int]:
+    """(tile, parts of K) for ``gemm_split``: its own, or for more than 64 rows the tile of planes that is predicted to take less, the pass over
+    a and what adds the parts up with it.  Over 2,272 random products of 65 to 1,400 rows (512 to 12,288 weight rows, K 256 to 8,192) the
+    prediction is within 7 % for nine in ten, the pick of a tile the best one, and the 1,437 products that go to planes take 0.80 of the
+    others' time (one in 200 more than 1.03)."""
+    tile, parts = _split_plan(m, n, k, most_parts)
+    if m <= SPLIT_MIN_ROWS_F32 or not planes:
+        return tile, parts
+    us, planes_tile, planes_parts = min(
+        (_planes_us(m, n, k, shape, p) + (p - 1) * (m * n * 8 / 4.5e6 + 0.5), shape, p)
+        for shape in PLANES_TILES for p in range(1, max(1, min(most_parts, k // 128)) + 1))
+    return (planes_tile, planes_parts) if us < _split_us(m, n, k, tile, parts) else (tile, parts)
+
+
+def _planes_us(m: int, n: int, k: int, shape: tuple[int, int], parts: int) -> float:
+    round_us, step_us, pair_us = PLANES_TILES[shape]
+    tiles, steps = -(-m // (16 * shape[0])) * -(-n // (64 * shape[1])) * parts, -(-(-(-k // 64)) // parts)
+    one, pair = round_us + steps * step_us, round_us + steps * (pair_us or 0.0)
+    if pair_us is None:
+        rounds = -(-tiles // 256) * one
+    else:
+        full, rest = divmod(tiles, 512)
+        rounds = full * pair + (0.0 if rest == 0 else one if rest <= 256 else pair)
+    return 3.6 + 2.2e-6 * m * k + max(rounds, n * k * 4 / 4.5e6)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -266,13 +304,15 @@ def _split_pays(m: int, n: int, k: int, most_parts: int) -> bool:
     return us < 1.25 * _tiles_f32_us(m, n, k)
 
 
-def gemm_split(a: Tensor, b: Tensor, parts: int, tile: int, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+def gemm_split(a: Tensor, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
     """float32 partial sums [parts, M, N] of a[M, K] @ b[N, K]^T over runs of whole steps of K (given ``out`` [M, N], the product with
     the bias there), each operand as three bfloat16 numbers whose sum it is (a number below 2^-110: up to 2^-134 beside it).  ``tile``: the
-    block's, see ``SPLIT_TILES``."""
+    block's, of ``SPLIT_TILES`` by its number, or of ``PLANES_TILES`` (a split ahead)."""
     _gpu(a, "a", torch.float32, contiguous=False)
     _gpu(b, "b", torch.float32, contiguous=False)
-    if not _split_fits(a, b) or not 0 <= tile < len(SPLIT_TILES) or not 1 <= parts <= 64 or (parts > 1 and (bias is not None or out is not None)):
+    planes = isinstance(tile, tuple)
+    known = tile in PLANES_TILES and _planes_fit(a, b) and parts <= -(-a.shape[1] // 64) if planes else 0 <= tile < len(SPLIT_TILES)
+    if not _split_fits(a, b) or not known or not 1 <= parts <= 64 or (parts > 1 and (bias is not None or out is not None)):
         raise KernelError("the product of split operands takes float32 rows 16 bytes aligned, K a multiple of four from 256, and a bias or a place in one part")
     m, k = a.shape
     n = b.shape[0]
@@ -281,6 +321,11 @@ def gemm_split(a: Tensor, b: Tensor, parts: int, tile: int, bias: Tensor | None 
     if bias is not None and _gpu(bias, "bias", torch.float32).shape != (n,):
         raise KernelError(f"bias must be [{n}]")
     result = torch.empty((parts, m, n), dtype=torch.float32, device=a.device) if out is None else out
+    if planes:
+        scratch = torch.empty(3 * m * (-(-k // 64) * 64), dtype=torch.bfloat16, device=a.device)
+        _call("gemm_planes", "fe_gemm_planes", _ptr(a), _ptr(scratch), _ptr(b), _ptr(bias), _ptr(result), c_int(m), c_int(n), c_int(k),
+              c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile[0]), c_int(tile[1]), _stream())
+        return result
     _call("gemm_split", "fe_gemm_split", _ptr(a), _ptr(b), _ptr(bias), _ptr(result), c_int(m), c_int(n), c_int(k),
           c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile), _stream())
     return result
@@ -309,7 +354,7 @@ def gemm_nt_f32(a: Tensor, b: Tensor, bias: Tensor | None = None, out: Tensor | 
         if bias.shape != (n,):
             raise KernelError(f"bias must be [{n}]")
     if m > SPLIT_MIN_ROWS_F32 and _split_fits(a, b) and out.data_ptr() % 4 == 0 and _split_pays(m, n, k, 1):
-        return gemm_split(a, b, 1, _split_plan(m, n, k, 1)[0], bias, out)
+        return gemm_split(a, b, 1, _product_plan(m, n, k, 1, _planes_fit(a, b))[0], bias, out)
     lda = a.stride(0) if m > 1 else max(k, a.stride(0))
     ldb = b.stride(0) if n > 1 else max(k, b.stride(0))
     _call("gemm_f32", "fe_gemm_nt_f32", _ptr(a), _ptr(b), _ptr(bias), _ptr(out), c_int(m), c_int(n),
@@ -1089,7 +1134,7 @@ def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream:
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     if bias is None and x.shape[0] > SPLIT_MIN_ROWS and _split_fits(x, weight) and _split_pays(x.shape[0], *weight.shape, SPLIT_MOST_PARTS):
-        tile, parts = _split_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS)
+        tile, parts = _product_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS, _planes_fit(x, weight))
         return gemm_split(x, weight, parts, tile)
     plain_bf16 = bias is None and weight.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
     if plain_bf16 and x.shape[0] > MID_ROWS and _big_fits(x, weight, False):
@@ -1817,7 +1862,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "gemm_big", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "gemm_big", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

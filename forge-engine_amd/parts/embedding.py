@@ -134,7 +134,7 @@ class LMHead(Head):
         return logits if self.scale == 1.0 else ops.scale_rows(logits, self.scale)
 
     def kernel_libraries(self):
-        return {"gemm_f32", "gemm_split", "gemm_skinny", "gemm_ring"} | ({"hyper"} if self.scale != 1.0 or self.softcap is not None else set())
+        return {"gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_ring"} | ({"hyper"} if self.scale != 1.0 or self.softcap is not None else set())
 
 
 register_part("embedding", "token_embedding", TokenEmbedding)

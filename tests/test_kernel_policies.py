@@ -454,7 +454,7 @@ def _reads_in_flight_at_barriers(listing: str) -> dict[str, list[int]]:
     return found
 
 
-@pytest.mark.parametrize("source", ["gemm_split", "gemm_f32", "moe"])
+@pytest.mark.parametrize("source", ["gemm_split", "gemm_planes", "gemm_f32", "moe"])
 def test_no_read_of_lds_is_under_way_at_a_barrier_behind_which_its_buffer_is_filled(source, tmp_path):
     """A wave that passes such a barrier requests loads into the buffer that it or another has just read: the compiler keeps reads before
     the barrier, but waits for them only where they are used, which it may move behind it.  (``gemm_tile``, whose buffers are filled two
@@ -468,11 +468,12 @@ def test_no_read_of_lds_is_under_way_at_a_barrier_behind_which_its_buffer_is_fil
     assert {name: at for name, at in found.items() if any(at)} == {}
 
 
-def test_large_tiles_leave_m0_to_their_loads(tmp_path):
+@pytest.mark.parametrize("source", ["gemm_big", "gemm_planes"])
+def test_loads_into_lds_have_m0_to_themselves(source, tmp_path):
     """Nothing but the loads into LDS touches m0, which they leave as it is, and nothing goes to scratch memory."""
-    listing = tmp_path / "gemm_big.s"
+    listing = tmp_path / f"{source}.s"
     flags = [flag for flag in build.HIPCC_FLAGS if flag != "-shared"]
-    subprocess.run([build.find_hipcc(), *flags, "-S", "--cuda-device-only", "-o", str(listing), str(build.SOURCE_DIR / "gemm_big.hip")],
+    subprocess.run([build.find_hipcc(), *flags, "-S", "--cuda-device-only", "-o", str(listing), str(build.SOURCE_DIR / f"{source}.hip")],
                    check=True, capture_output=True)
     text = listing.read_text()
     lines = [line.split(";")[0].strip() for line in text.splitlines()]

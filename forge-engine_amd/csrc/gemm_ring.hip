@@ -44,13 +44,13 @@ using lds_tile::wait_loads;
 constexpr int WAVES = 8, SQUARES = 256;
 constexpr int UPDATE = 0, FLOAT = 1, BFLOAT = 2, GATED = 3, SEVERAL = 4;
 
-// XI, WI: requests of eight rows a chunk for x and for the weight
-template <int XI, int WI, bool SCALED>
+// XI, WI: requests of eight rows a chunk for x and for the weight; PAIRED: a buffer holds two chunks
+template <int XI, int WI, bool SCALED, bool PAIRED>
 struct Ring {
-  static constexpr int LOADS = XI + WI, STAGES = (SCALED ? 17 : 19) / LOADS, TILES = (WI + 1) / 2;
+  static constexpr int LOADS = (PAIRED ? 2 : 1) * (XI + WI), STAGES = (SCALED ? 17 : 19) / LOADS, TILES = (WI + 1) / 2;
   static constexpr int WAVE_BYTES = STAGES * LOADS * 1024;
   static constexpr int BYTES = WAVES * (WAVE_BYTES + (SCALED ? XI * 1024 : 0));      // behind the rings, the rows' squares
-  static_assert(TILES * 1024 <= WAVE_BYTES && STAGES >= 2 && BYTES <= 152 * 1024, "LDS of a CU");
+  static_assert((PAIRED ? 2 : 1) * TILES * 1024 <= WAVE_BYTES && STAGES >= 2 && BYTES <= 152 * 1024, "LDS of a CU");
 };
 
 struct Ending {
@@ -66,11 +66,21 @@ struct Ending {
   int each;
 };
 
+// float32, up to eight weight rows a block: they and up to eight rows of x fill a quarter of the instruction's tile, whose operands are split
+// whatever they hold.  So it takes two chunks at a time, the second one's rows in its rows 8 to 15: sums [n][m] and [8 + n][8 + m]
+// are the result's halves, the others are nobody's.  4 rows: 2,048 x 6,144 with its norm 17.0 -> 12.6 us, 2,048 x 2,048 8.4 -> 6.9, 1 row: 1,024 x
+// 3,072 9.6 -> 7.3.  With 9 to 16 rows of x two sets of sums take the chunks in turn, so that a row's sums stay the same.
+template <typename T, int WI>
+constexpr bool pairs() {
+  return sizeof(T) == 4 && WI == 1;
+}
+
 template <typename T, int XI, int WI, int END, bool SCALED>
 __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
     const T* __restrict__ x, const T* __restrict__ w, Ending ending, int M, int N, int K, long long ldw, int block_rows) {
-  using R = Ring<XI, WI, SCALED>;
-  constexpr bool WIDE = sizeof(T) == 4;
+  constexpr bool WIDE = sizeof(T) == 4, PAIRED = pairs<T, WI>(), FOLD = PAIRED && XI == 1;
+  constexpr int CHUNKS = PAIRED ? 2 : 1, SETS = PAIRED && !FOLD ? 2 : 1;      // chunks of a buffer, sets of sums
+  using R = Ring<XI, WI, SCALED, PAIRED>;
   constexpr int CHUNK = 128 / sizeof(T), PIECE = 16 / sizeof(T);      // elements of a row's 128 bytes, and of 16
   constexpr int TILES = R::TILES, PAIR = END == GATED ? 2 : 1;
   constexpr int VALUES = TILES * 256 / PAIR;          // results of a block, one a thread
@@ -111,7 +121,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
       load_to_lds(ending.row_squares + min(wave + WAVES * i, M - 1) * SQUARES + lane * 4, lds_at + squares_at + i * 1024);
   }
 
-  const int chunks = K / CHUNK, count = (chunks - wave + WAVES - 1) / WAVES;       // this wave's chunks: wave, wave + 8, ..
+  const int chunks = K / CHUNK, own = (chunks - wave + WAVES - 1) / WAVES;       // this wave's chunks: wave, wave + 8, ..
+  const int count = (own + CHUNKS - 1) / CHUNKS;      // buffers full of them
   const unsigned int base = lds_at + wave * R::WAVE_BYTES;
   // a request: eight rows of 128 bytes, 16-byte piece c of a row at c ^ (row % 8)
   const int of_group = lane >> 3, at = wave * CHUNK + ((lane & 7) ^ of_group) * PIECE;
@@ -131,52 +142,55 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   // every request is issued whatever the rows, so that the waits can count: where all eight rows lie beyond the block's last one (the
   // last block's), that one is fetched again
   auto load = [&](int index, int stage) {
-    const int k = index * WAVES * CHUNK;
-    const unsigned int to = base + stage * R::LOADS * 1024;
 #pragma unroll
-    for (int i = 0; i < XI; ++i)
-      if (x_has[i] || of_group == 0) load_to_lds(x_from[i] + k, to + i * 1024);
+    for (int part = 0; part < CHUNKS; ++part) {
+      const int k = (PAIRED ? min(2 * index + part, own - 1) : index) * WAVES * CHUNK;      // a chunk too few: the last one again
+      const unsigned int to = base + (stage * R::LOADS + part * (XI + WI)) * 1024;
 #pragma unroll
-    for (int i = 0; i < WI; ++i)
-      if (w_has[i] || of_group == 0) load_to_lds(w_from[i] + k, to + (XI + i) * 1024);
+      for (int i = 0; i < XI; ++i)
+        if (x_has[i] || of_group == 0) load_to_lds(x_from[i] + k, to + i * 1024);
+#pragma unroll
+      for (int i = 0; i < WI; ++i)
+        if (w_has[i] || of_group == 0) load_to_lds(w_from[i] + k, to + (XI + i) * 1024);
+    }
   };
-  floatx4 acc[TILES];
+  floatx4 acc[SETS * TILES];
 #pragma unroll
-  for (int t = 0; t < TILES; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < SETS * TILES; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   // float32 operands: the products of the first parts, added to the whole every four chunks, and all others, a 2^8th of their size: so
   // the long sum is rounded a quarter as often and a long K costs no accuracy
-  floatx4 large[TILES], small[TILES];
+  floatx4 large[SETS * TILES], small[SETS * TILES];
   int turn = 0;
 #pragma unroll
-  for (int t = 0; t < TILES; ++t) large[t] = small[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < SETS * TILES; ++t) large[t] = small[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   const uintx4* ring = lds + wave * (R::WAVE_BYTES / 16);
   const split_f32::Minus minus = split_f32::minus();
   uintx4 a[2], b[TILES][2];
-  auto fragments = [&](int stage) {
-    const uintx4* from = ring + stage * R::LOADS * 64;
+  auto fragments = [&](int stage, int part) {
+    const uintx4* from = ring + (stage * R::LOADS + (FOLD ? r >> 3 : part) * (XI + WI)) * 64;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int piece = (4 * half + q) ^ (r & 7);
       a[half] = from[(XI == 1 ? r & 7 : r) * 8 + piece];
 #pragma unroll
-      for (int t = 0; t < TILES; ++t) b[t][half] = from[XI * 64 + min(t * 16 + r, WI * 8 - 8 + (r & 7)) * 8 + piece];
+      for (int t = 0; t < TILES; ++t) b[t][half] = from[XI * 64 + (FOLD ? r & 7 : min(t * 16 + r, WI * 8 - 8 + (r & 7))) * 8 + piece];
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before the buffer is filled again
   };
-  auto multiply = [&]() {
+  auto multiply = [&](int set) {
     if constexpr (WIDE) {       // the two pieces are a lane's eight elements of 32
       bf16x8 x_parts[1][3], w_parts[3];
       split_f32::split8(__builtin_bit_cast(floatx4, a[0]), __builtin_bit_cast(floatx4, a[1]), minus, x_parts[0]);
 #pragma unroll
       for (int t = 0; t < TILES; ++t) {
         split_f32::split8(__builtin_bit_cast(floatx4, b[t][0]), __builtin_bit_cast(floatx4, b[t][1]), minus, w_parts);
-        split_f32::add_products_apart(x_parts[0], w_parts, large[t], small[t]);
+        split_f32::add_products_apart(x_parts[0], w_parts, large[set * TILES + t], small[set * TILES + t]);
         if (turn == 3) {
-          acc[t] += large[t];
-          large[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+          acc[set * TILES + t] += large[set * TILES + t];
+          large[set * TILES + t] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
       }
-      turn = (turn + 1) & 3;
+      if (set == SETS - 1) turn = (turn + 1) & 3;
       return;
     }
 #pragma unroll
@@ -200,9 +214,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   int stage = 0, i = 0;
   for (; count - i > R::STAGES; ++i) {
     wait_loads<R::LOADS*(R::STAGES - 1)>();
-    fragments(stage);
+    if constexpr (SETS == 2) {
+      fragments(stage, 0);
+      multiply(0);
+    }
+    fragments(stage, SETS - 1);
     load(i + R::STAGES, stage);
-    multiply();
+    multiply(SETS - 1);
     stage = stage + 1 == R::STAGES ? 0 : stage + 1;
   }
   // the last chunks, with fewer and fewer requests under way: each with its own wait
@@ -212,8 +230,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
     if constexpr (L > 0) {
       if (rest >= L) {
         wait_loads<R::LOADS*(L - 1)>();
-        fragments(stage);
-        multiply();
+        if constexpr (SETS == 2) {
+          fragments(stage, 0);
+          multiply(0);
+        }
+        fragments(stage, SETS - 1);
+        if (PAIRED && L == 1 && own % 2 && (!FOLD || r >= 8)) a[0] = a[1] = uintx4{0, 0, 0, 0};      // an odd chunk, here twice
+        multiply(SETS - 1);
         stage = stage + 1 == R::STAGES ? 0 : stage + 1;
       }
       self(self, std::integral_constant<int, L - 1>{});
@@ -224,13 +247,18 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
   // the waves' sums meet, each in its wave's own ring, which nobody else reads and which it has emptied
   floatx4* meet = (floatx4*)(lds + wave * (R::WAVE_BYTES / 16));
 #pragma unroll
-  for (int t = 0; t < TILES; ++t) meet[t * 64 + lane] = WIDE ? acc[t] + (large[t] + small[t]) : acc[t];
+  for (int t = 0; t < SETS * TILES; ++t) meet[t * 64 + lane] = WIDE ? acc[t] + (large[t] + small[t]) : acc[t];
   __syncthreads();
   auto total = [&](int lane_group) {       // of the eight columns' gate or up rows, or of all sixteen: lane group of the tile
     const float* from = (const float*)lds + tile * 256 + (lane_group * 16 + row) * 4 + (tid & 3);
     float sum = 0.f;
+    if constexpr (FOLD) from = (const float*)lds + ((lane_group & 1) * 16 + (row & 7)) * 4 + (tid & 3);
+    constexpr int OTHER = FOLD ? (2 * 16 + 8) * 4 : 256;      // from the first chunks' sum to the second ones'
 #pragma unroll
-    for (int v = 0; v < WAVES; ++v) sum += from[v * (R::WAVE_BYTES / 4)];
+    for (int v = 0; v < WAVES; ++v) {
+      if constexpr (PAIRED) sum += from[v * (R::WAVE_BYTES / 4)] + from[v * (R::WAVE_BYTES / 4) + OTHER];
+      else sum += from[v * (R::WAVE_BYTES / 4)];
+    }
     if constexpr (WIDE) {
       if (!split_f32::finite(sum) && mine)
         sum = split_f32::dot(x + (size_t)row * K, w + (size_t)(n0 + column + (lane_group != group ? N : 0)) * ldw, K);
@@ -278,10 +306,11 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
 template <typename T, int XI, int WI, int END, bool SCALED>
 int launch(const void* x, const void* w, const Ending& ending, int M, int N, int K, long long ldw, int block_rows, int weights, hipStream_t stream) {
   static std::atomic<bool> raised{false};
+  using R = Ring<XI, WI, SCALED, pairs<T, WI>()>;
   auto kernel = gemm_ring_kernel<T, XI, WI, END, SCALED>;
-  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, Ring<XI, WI, SCALED>::BYTES, &raised);
+  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, R::BYTES, &raised);
   if (limit_raised != FE_OK) return limit_raised;
-  kernel<<<ending.each * weights, 64 * WAVES, Ring<XI, WI, SCALED>::BYTES, stream>>>(
+  kernel<<<ending.each * weights, 64 * WAVES, R::BYTES, stream>>>(
       (const T*)x, (const T*)w, ending, M, N, K, ldw, block_rows);
   return fe_check_launch();
 }

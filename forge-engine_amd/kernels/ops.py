@@ -861,9 +861,9 @@ def _update_norm_pays(rows: int, weight_rows: int, k: int) -> bool:
 def _update_norm_float32_pays(rows: int, weight_rows: int, k: int) -> bool:
     """float32: 9 to 16 rows, for which the weight would be read twice, always (512 x 2,048 1.3 times as fast, x 25,600 1.04); to eight rows
     through more than 2,048 weight rows (2,560 x 9,728 28 -> 27 us, 4,096 x 12,288 44 -> 41), and through fewer, which fill half of a tile
-    of sixteen, to a K of three times theirs (2,048 x 2,048 9.6 -> 7.9; the two launches alone are some 6 % faster at the line, 2,048 x 6,144
-    15.7 and 17.1, which a step does not show: 1.7B at 4 requests 2,297 and 2,300, 0.6B, 1,024 x 3,072, 1,575 -> 1,555; but 1,024 x 4,096 .85 of
-    the speed, x 8,192 .81, 512 x 25,600 .5) or just beyond 6,144, where the other kernel takes another pass (2,048 x 8,192 1.1)."""
+    of sixteen, to a K of three times theirs (2,048 x 2,048 9.5 -> 6.9, x 6,144 15.0 -> 12.6, 1,024 x 3,072 8.8 -> 7.3) or just beyond 6,144,
+    where the other kernel takes another pass (2,048 x 8,192 22.3 -> 15.9).  The lines were drawn when a tile took one chunk of K at a time; with
+    two, sizes beyond them come to 0.6 (256 x 4,096) to 1.4 (2,048 x 12,288) of the two launches' speed, 1,024 x 4,096 to 1.07."""
     return rows > 8 or weight_rows > 2048 or k <= 3 * weight_rows or (weight_rows >= 1792 and 6144 < k <= 9728)
 
 

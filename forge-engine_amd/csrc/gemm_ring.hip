@@ -42,7 +42,7 @@ using lds_tile::load_to_lds;
 using lds_tile::wait_loads;
 
 constexpr int WAVES = 8, SQUARES = 256;
-constexpr int UPDATE = 0, FLOAT = 1, BFLOAT = 2, GATED = 3, SEVERAL = 4;
+constexpr int UPDATE = 0, FLOAT = 1, BFLOAT = 2, GATED = 3, SEVERAL = 4, TANH = 5;      // TANH: BFLOAT and `Ending::tanh`
 
 // XI, WI: requests of eight rows a chunk for x and for the weight; PAIRED: a buffer holds two chunks
 template <int XI, int WI, bool SCALED, bool PAIRED>
@@ -64,6 +64,7 @@ struct Ending {
   GateAct act;
   const void* more[3];      // SEVERAL: the weights behind the first, and each one's blocks; x and out [weights][M][.]
   int each;
+  bool tanh;                // BFLOAT: tanh of what is stored otherwise, rounded again
 };
 
 // float32, up to eight weight rows a block: they and up to eight rows of x fill a quarter of the instruction's tile, whose operands are split
@@ -298,7 +299,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
     } else if constexpr (END == FLOAT) {
       ((float*)ending.out)[place] = sum;
     } else {
-      ((bf16_t*)ending.out)[place] = float_to_bf16(sum);
+      bf16_t y = float_to_bf16(sum);
+      if (END == BFLOAT && ending.tanh) y = float_to_bf16(tanhf(bf16_to_float(y)));      // the bits of a launch of its own behind this one
+      ((bf16_t*)ending.out)[place] = y;
     }
   }
 }
@@ -354,13 +357,13 @@ extern "C" int fe_gemm_update_norm(const void* x, const void* w, int dtype, floa
                                    int M, int N, int K, long long ldw, hipStream_t stream) {
   if (M < 1) return FE_OK;
   if (!operands_fit(x, w, dtype, M, N, K, ldw) || N > 32 * SQUARES || !h || !weight || !y || !squares) return FE_BAD_ARGUMENT;
-  const Ending how = {h, weight, y, squares, nullptr, nullptr, 0.f, 0.f, {}, {}, 0};
+  const Ending how = {h, weight, y, squares, nullptr, nullptr, 0.f, 0.f, {}, {}, 0, false};
   if (dtype == FE_F32) return pick<float, UPDATE, false>(x, w, how, M, N, K, ldw, stream);
   return pick<bf16_t, UPDATE, false>(x, w, how, M, N, K, ldw, stream);
 }
 
 // The same operands; ending 1: out [M, N] float32, 2: bfloat16, of bfloat16 operands (N up to 8,192), 3: out [M, N] of x's type =
-// act(x gate^T) * (x up^T) for a fused weight [2 N, K], gate rows first (N up to 6,144; act by `activation`, gate_act.h).  squares
+// act(x gate^T) * (x up^T) for a fused weight [2 N, K], gate rows first (N up to 6,144; act by `activation`, gate_act.h), 5: tanh of ending 2.  squares
 // (null: none) [M][256] float32: the sums of row m are multiplied by rsqrt(sum of squares[m] / K + eps) before anything else is done
 // with them.
 extern "C" int fe_gemm_ring(const void* x, const void* w, int dtype, void* out, int M, int N, int K, long long ldw, int ending,
@@ -370,7 +373,9 @@ extern "C" int fe_gemm_ring(const void* x, const void* w, int dtype, void* out, 
   if (!gate_act(activation, &act)) return FE_BAD_ARGUMENT;
   if (!operands_fit(x, w, dtype, M, N, K, ldw) || !out || N > (ending == GATED ? 24 : 32) * SQUARES) return FE_BAD_ARGUMENT;
   if (squares && (!(eps > 0.f) || (((uintptr_t)squares) & 15))) return FE_BAD_ARGUMENT;
-  const Ending how = {nullptr, nullptr, nullptr, nullptr, out, squares, (float)K, eps, act, {}, 0};
+  const bool tanh = ending == TANH;
+  if (tanh) ending = BFLOAT;
+  const Ending how = {nullptr, nullptr, nullptr, nullptr, out, squares, (float)K, eps, act, {}, 0, tanh};
 #define FE_PICK(TYPE, T, END)                                                       \
   if (dtype == TYPE && ending == END) {                                             \
     if (squares) return pick<T, END, true>(x, w, how, M, N, K, ldw, stream);        \
@@ -391,7 +396,7 @@ extern "C" int fe_gemm_ring(const void* x, const void* w, int dtype, void* out, 
 extern "C" int fe_gemm_ring_several(const void* x, const void* const* w, void* out, int weights, int M, int N, int K, hipStream_t stream) {
   if (M < 1) return FE_OK;
   if (weights < 2 || weights > 4 || !w || !out || N < 1 || (long long)N * weights > 32 * SQUARES) return FE_BAD_ARGUMENT;
-  Ending how = {nullptr, nullptr, nullptr, nullptr, out, nullptr, 0.f, 0.f, {}, {}, 0};
+  Ending how = {nullptr, nullptr, nullptr, nullptr, out, nullptr, 0.f, 0.f, {}, {}, 0, false};
   for (int i = 0; i < weights; ++i) {
     if (!operands_fit(x, w[i], FE_BF16, M, N, K, K)) return FE_BAD_ARGUMENT;
     if (i > 0) how.more[i - 1] = w[i];

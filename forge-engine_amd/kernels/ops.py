@@ -935,7 +935,7 @@ def _ring_parts_pays(rows: int, weight_rows: int, k: int) -> bool:
 
 
 def gemm_ring(x: Tensor | UnscaledRows, weight: Tensor, ending: str, act: str = "silu") -> Tensor:
-    """x @ weight^T for up to 16 rows, whole sums in a block: ``"f32"`` or, of bfloat16, ``"bf16"`` [M, N] (N up to 8,192), or
+    """x @ weight^T for up to 16 rows, whole sums in a block: ``"f32"`` or, of bfloat16, ``"bf16"`` or its ``"tanh"`` [M, N] (N up to 8,192), or
     ``"gated"``: act(gate) * up [M, N / 2] in x's dtype for a fused gate/up weight (gate rows first, up to 12,288 of both)."""
     rows, squares, eps = x if isinstance(x, UnscaledRows) else (x, None, 0.0)
     _gpu(rows, "x")
@@ -948,7 +948,7 @@ def gemm_ring(x: Tensor | UnscaledRows, weight: Tensor, ending: str, act: str = 
     n = weight.shape[0] // 2 if ending == "gated" else weight.shape[0]
     out = torch.empty((m, n), dtype=torch.float32 if ending == "f32" else rows.dtype, device=rows.device)
     _call("gemm_ring", "fe_gemm_ring", _ptr(rows), _ptr(weight), c_int(_code(rows.dtype)), _ptr(out), c_int(m), c_int(n), c_int(k), c_longlong(weight.stride(0)),
-          c_int({"f32": 1, "bf16": 2, "gated": 3}[ending]), _gate_act(act), _ptr(squares), c_float(eps), _stream())
+          c_int({"f32": 1, "bf16": 2, "gated": 3, "tanh": 5}[ending]), _gate_act(act), _ptr(squares), c_float(eps), _stream())
     return out
 
 
@@ -959,7 +959,7 @@ def _ring_fits(x: Tensor, weight: Tensor, ending: str | None) -> bool:
 def _ring_ending_fits(weight: Tensor, ending: str | None) -> bool:
     if ending == "gated":
         return weight.shape[0] % 2 == 0 and weight.shape[0] <= 2 * RING_GATE_COLUMNS
-    return weight.shape[0] <= UPDATE_NORM_MAX_WIDTH and (ending == "f32" or (ending == "bf16" and weight.dtype == torch.bfloat16))
+    return weight.shape[0] <= UPDATE_NORM_MAX_WIDTH and (ending == "f32" or (ending in ("bf16", "tanh") and weight.dtype == torch.bfloat16))
 
 
 def _weight_fits_lds(weight: Tensor) -> bool:
@@ -1954,6 +1954,40 @@ def rmsnorm_update(h: Tensor, update: Tensor, weight: Tensor, eps: float, out: T
     return out
 
 
+UPDATE_SHIFT_MAX_WIDTH = 8192      # a row's elements stay in the registers of 1,024 threads
+UPDATE_SHIFT_MAX_ROWS = 512        # ... which a row has up to here
+
+
+def update_shift_fits(h: Tensor) -> bool:
+    """Whether ``rmsnorm_update_shift`` takes a stream: on the GPU, its rows in registers."""
+    return h.is_cuda and h.shape[0] <= UPDATE_SHIFT_MAX_ROWS and h.shape[1] <= UPDATE_SHIFT_MAX_WIDTH
+
+
+def rmsnorm_update_shift(h: Tensor, update: Tensor, weight: Tensor, eps: float, shift: Tensor, state: Tensor, token_seq: Tensor,
+                         state_slots: Tensor, *, out_dtype) -> Tensor:
+    """``rmsnorm_update`` followed by ``token_shift`` with one blend (``shift`` [1, W]) in a step whose sequences bring one token each: the same
+    bits in h, the state and the result [1, T, W], in one launch for up to UPDATE_SHIFT_MAX_ROWS rows of UPDATE_SHIFT_MAX_WIDTH."""
+    _gpu(h, "h", torch.float32)
+    _gpu(weight, "weight", torch.float32)
+    _gpu(shift, "shift", torch.float32)
+    _gpu(state, "state", torch.float32)
+    _gpu(token_seq, "token_seq", torch.int32)
+    _gpu(state_slots, "state_slots", torch.int32)
+    rows, width = h.shape
+    parts = _parts_of(update, rows, width, "update")
+    if weight.shape != (width,) or shift.shape != (1, width) or state.dim() != 2 or state.shape[1] != width:
+        raise KernelError(f"weight must be [{width}], shift [1, {width}] and state [slots, {width}]")
+    if token_seq.numel() != rows or state_slots.numel() != rows or not update_shift_fits(h):
+        raise KernelError("one token a sequence, up to 512 rows of 8,192")
+    if not eps > 0.0:
+        raise KernelError("eps must be positive")
+    out = torch.empty((1, rows, width), dtype=out_dtype, device=h.device)
+    _call("stream_ops", "fe_rmsnorm_update_shift", _ptr(h), _ptr(update), c_int(parts), c_longlong(h.numel()), _ptr(weight), c_float(eps),
+          _ptr(shift), _ptr(state), _ptr(token_seq), _ptr(state_slots), _ptr(out), c_int(_code(out.dtype)), c_int(rows), c_int(width),
+          c_int(state.shape[0]), _stream())
+    return out
+
+
 def layernorm_update(h: Tensor, update: Tensor, weight: Tensor, eps: float, factor: float = 1.0,
                      out: Tensor | None = None) -> Tensor | None:
     """h += factor * (u - mean(u)) * rsqrt(var(u) + eps) * weight, u the update (float32, [parts, T, W] added up
@@ -2062,6 +2096,15 @@ def tanh_rows(x: Tensor) -> Tensor:
     return x
 
 
+def linear_tanh(x: Tensor, weight: Tensor) -> Tensor:
+    """tanh of ``linear``'s result: in the product's own launch where few bfloat16 rows go through a ring, with the same bits (six
+    rows in a captured graph: 5.4 -> 4.0 us)."""
+    if (x.is_cuda and x.dtype == torch.bfloat16 and _ring_fits(x, weight, "bf16") and _ring_store_pays(x.shape[0], *weight.shape)
+            and not _few_rows_to_library(x, weight)):
+        return gemm_ring(x, weight, "tanh")
+    return tanh_rows(linear(x, weight))
+
+
 _ACTS = {"none": 0, "silu": 1, "sigmoid": 2}
 
 
@@ -2115,7 +2158,7 @@ def conv_rope_norm_write(qkv: Tensor, bias: Tensor | None, conv_weight: Tensor |
                          kv_heads: int, head_dim: int, value_dim: int, rotary_dim: int, unit_norm_eps: float | None,
                          taps: int, v_from: Tensor | None = None, v_mix: float = 0.0, v_keep: Tensor | None = None,
                          norm_weight_q: Tensor | None = None, norm_weight_k: Tensor | None = None,
-                         norm_first: bool = False, q_temp: tuple[float, float] | None = None) -> None:
+                         norm_first: bool = False, q_temp: tuple[float, float] | None = None, single: bool = False) -> None:
     """From the projection's output to queries and cached keys and values in one kernel: a short
     projection's bias (float32 [channels] or None: the product before has none), a short causal
     convolution over time on every q, k and v channel (``taps`` > 0: y_t = sum_j c[:, j] *
@@ -2130,7 +2173,8 @@ def conv_rope_norm_write(qkv: Tensor, bias: Tensor | None, conv_weight: Tensor |
     (float32 [head_dim], shared by the heads): the unit norm's result times a weight per dim, an RMS norm;
     ``norm_first``: the norm comes before the rotation instead of behind it.  ``q_temp`` (coef, every): queries at
     position p are multiplied by ``1 + coef * ln(floor((p + 1) / every) + 1)`` last of all.  Pages whose rows are wider than
-    a head (``masked_attention`` says why): q_out has the key pages' row width, q and key rows are filled up with zeros."""
+    a head (``masked_attention`` says why): q_out has the key pages' row width, q and key rows are filled up with zeros.
+    ``single``: every sequence brings one token (the caller knows), and the state is moved on in the same launch."""
     channels = (q_heads + kv_heads) * head_dim + kv_heads * value_dim
     for name, w in (("norm_weight_q", norm_weight_q), ("norm_weight_k", norm_weight_k)):
         if w is not None:
@@ -2186,6 +2230,8 @@ def conv_rope_norm_write(qkv: Tensor, bias: Tensor | None, conv_weight: Tensor |
             _gpu(dense, name, qkv.dtype)
             if dense.shape != (tokens, kv_heads * value_dim):
                 raise KernelError(f"{name} must be [{tokens}, {kv_heads * value_dim}], got {tuple(dense.shape)}")
+    if single and tokens != num_seqs:
+        raise KernelError("one token a sequence")
     stride = qkv.stride(0) if tokens > 1 else max(qkv.stride(0), qkv.shape[1])
     slots = conv_state.shape[0] if taps > 1 else 0
     _call("conv_rope", "fe_conv_rope_norm_write", _ptr(qkv), c_int(_code(qkv.dtype)), c_longlong(stride), _ptr(bias),
@@ -2196,8 +2242,8 @@ def conv_rope_norm_write(qkv: Tensor, bias: Tensor | None, conv_weight: Tensor |
           c_int(1 if unit_norm_eps is not None else 0), c_int(taps), c_int(block_size), c_int(num_blocks), c_int(slots),
           _ptr(v_from), c_float(v_mix), _ptr(v_keep), _ptr(norm_weight_q), _ptr(norm_weight_k), c_int(1 if norm_first else 0),
           c_float(q_temp[0] if q_temp is not None else 0.0), c_double(q_temp[1] if q_temp is not None else 0.0),
-          c_int(key_row), c_int(value_pages.shape[2]), _stream())
-    if taps > 1:
+          c_int(key_row), c_int(value_pages.shape[2]), c_int(int(single)), _stream())
+    if taps > 1 and not single:
         _call("conv_rope", "fe_conv_state_update", _ptr(qkv), c_int(_code(qkv.dtype)), c_longlong(stride), _ptr(bias), _ptr(conv_state),
               _ptr(cu_q), _ptr(state_slots), c_int(num_seqs), c_int(channels), c_int(taps), c_int(slots), c_int(tokens),
               _stream())

@@ -432,6 +432,8 @@ class GroupedQueryAttention(Mixer):
             if self.value_mix_key not in batch.carry:
                 raise ValueError(f"{self.prefix}: no earlier layer of the step left the values '{self.value_mix_key}'")
             mixing = {"v_from": batch.carry[self.value_mix_key], "v_mix": self.mix_weight}
+        if qkv.is_cuda and batch.num_decode is not None and batch.num_decode == batch.num_seqs == qkv.shape[0]:
+            mixing["single"] = True
         ops.conv_rope_norm_write(
             qkv, self.conv_bias, self.conv_weight, cache.states[self.CONV_STATE] if self.conv_taps > 1 else None, inv_freq,
             batch.positions, batch.token_seq, batch.cu_q, batch.state_slots, cache.block_table,

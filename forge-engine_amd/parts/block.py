@@ -81,20 +81,39 @@ class OutputNormBlock(Block):
         return CacheNeeds(paged=needs.paged, state=states)
 
     def forward(self, residual: Residual, batch, cache: CacheView | None, writes_cache: bool = True) -> None:
-        h = residual.flush()
         if self.token_shift:
-            s = ops.token_shift(h, self.shift, cache.states[self.SHIFT_STATE], batch.cu_q, batch.token_seq,
-                                batch.state_slots, num_seqs=batch.num_seqs, out_dtype=self.ctx.dtype)[0]
+            s = self._shifted(residual, batch, cache.states[self.SHIFT_STATE])
             mixer_cache = dataclasses.replace(
                 cache, states={n: t for n, t in cache.states.items() if n != self.SHIFT_STATE})
         else:       # the layer before has left the stream in the compute dtype as well, unless this is the first
+            h = residual.flush()
             s = residual.in_compute_dtype if residual.in_compute_dtype is not None else ops.cast_rows(h, self.ctx.dtype)
             mixer_cache = cache
         residual.add(self.mixer.forward(s, batch, mixer_cache, writes_cache))
+        if self.feed_forward is None:
+            self._last_norm("mixer_out", residual)
+            return
         x = self.norms["mixer_out"].forward(residual)
-        if self.feed_forward is not None:
-            residual.add(self.feed_forward.forward(x, batch))
-            self.norms["ff_out"].forward(residual)
+        residual.add(self.feed_forward.forward(x, batch))
+        self._last_norm("ff_out", residual)
+
+    def _last_norm(self, role: str, residual: Residual) -> None:
+        """Layers with a token shift leave their last norm pending: the next one's shift applies it in the same launch, or the model's last norm."""
+        norm = self.norms[role]
+        if self.token_shift and getattr(norm, "waits", False):
+            update, residual.pending = residual.pending, None
+            residual.add_normed(update, norm.weight, norm.eps)
+        else:
+            norm.forward(residual)
+
+    def _shifted(self, residual: Residual, batch, state: Tensor) -> Tensor:
+        if (residual.pending_norm is not None and batch.num_decode is not None
+                and batch.num_decode == batch.num_seqs == residual.h.shape[0] and ops.update_shift_fits(residual.h)):
+            update, weight, eps = residual.take_normed()
+            return ops.rmsnorm_update_shift(residual.h, update, weight, eps, self.shift, state, batch.token_seq, batch.state_slots,
+                                            out_dtype=self.ctx.dtype)[0]
+        return ops.token_shift(residual.flush(), self.shift, state, batch.cu_q, batch.token_seq, batch.state_slots,
+                               num_seqs=batch.num_seqs, out_dtype=self.ctx.dtype)[0]
 
     def kernel_libraries(self):
         return {"stream_ops"}

@@ -157,7 +157,7 @@ class RWKVTimeMix(_RecurrentMixer):
         mixes = ops.token_shift(x, self.mu, cache.states[self.PREVIOUS], batch.cu_q, batch.token_seq,
                                 batch.state_slots, num_seqs=batch.num_seqs, out_dtype=x.dtype)
         r, k, v, gate = ops.linear_several(mixes[:4], [t[key] for key in ("r", "k", "v", "g")])
-        low = ops.tanh_rows(ops.linear(mixes[4], t["w1"]))
+        low = ops.linear_tanh(mixes[4], t["w1"])
         decay = ops.linear(low, t["w2"], out_dtype=torch.float32)
         y = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=x.dtype, device=x.device)
         if self.single_tokens(x.shape[0], batch, cache):

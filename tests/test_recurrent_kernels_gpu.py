@@ -64,6 +64,39 @@ def test_token_shift(ops, x_dtype, out_dtype, lengths, width, count):
     torch.testing.assert_close(sd.cpu(), state_ref, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("parts", [1, 4, 5])
+@pytest.mark.parametrize("rows,width", [(1, 24), (3, 256), (6, 1024), (6, 2048), (7, 2049), (512, 4097), (300, 2048), (2, 8192)])
+def test_update_and_shift_in_one_launch(ops, out_dtype, parts, rows, width):
+    """Every count of elements a thread holds, tokens in another order than their sequences, and a token without a slot of its own: the
+    bits of the norm of the update and the token shift behind it."""
+    g = torch.Generator().manual_seed(rows + width)
+    h, update, w = rand(g, rows, width).to(DEV), rand(g, parts, rows, width).to(DEV), (1.0 + rand(g, width, scale=0.1)).to(DEV)
+    shift, state = torch.rand(1, width, generator=g).to(DEV), rand(g, rows + 3, width).to(DEV)
+    seq = torch.arange(rows, dtype=torch.int32, device=DEV)
+    slots = (1 + torch.randperm(rows + 1, generator=g)[:rows]).int().to(DEV)      # the first and the last row are nobody's
+    if rows > 2:
+        slots[1] = rows + 9
+    want_h, want_state = h.clone(), state.clone()
+    ops.rmsnorm_update(want_h, update, w, 1e-6, None)
+    want = ops.token_shift(want_h, shift, want_state, torch.arange(rows + 1, dtype=torch.int32, device=DEV), seq, slots, num_seqs=rows, out_dtype=out_dtype)
+    got = ops.rmsnorm_update_shift(h, update, w, 1e-6, shift, state, seq, slots, out_dtype=out_dtype)
+    assert torch.equal(got, want) and torch.equal(h, want_h) and torch.equal(state, want_state)
+    with pytest.raises(ops.KernelError):
+        ops.rmsnorm_update_shift(h[:, :width - 1].contiguous(), update, w, 1e-6, shift, state, seq, slots, out_dtype=out_dtype)
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 64, 2048), (6, 64, 2048), (16, 2050, 1024), (17, 64, 2048), (3, 40, 72)])
+def test_product_with_its_tanh(ops, rows, n, k):
+    """In the product's launch or behind it: the same bits."""
+    g = torch.Generator().manual_seed(rows + n)
+    x, w = rand(g, rows, k, dtype=torch.bfloat16).to(DEV), rand(g, n, k, dtype=torch.bfloat16, scale=0.1).to(DEV)
+    x[0, :8] = torch.tensor([float("nan"), 3e38, 1.0, -1.0, 0.0, 1e-30, -1e-3, 2.0]).bfloat16().to(DEV) if rows > 1 else x[0, :8]
+    want = ops.tanh_rows(ops.linear(x, w))
+    got = ops.linear_tanh(x, w)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(9.0), want.nan_to_num(9.0))
+
+
 @pytest.mark.parametrize("out_dtype", [None, torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("parts", [0, 3])
 @pytest.mark.parametrize("rows,width", [(7, 24), (33, 200), (300, 2050)])
@@ -210,6 +243,28 @@ def test_conv_rope_norm_write(ops, dtype, sizes):
     torch.testing.assert_close(values_d.cpu().float(), values_ref.float(), **tol(dtype))
     if taps > 1:
         torch.testing.assert_close(state_d.cpu(), state_ref, atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [2, 4, 8])
+def test_convolution_state_of_single_tokens(ops, dtype, taps):
+    """Moved on by the launch that reads it, or by one of its own: the same bits everywhere; a slot that is no slot stays out of it."""
+    g = torch.Generator().manual_seed(taps)
+    seqs, geometry = 5, dict(q_heads=6, kv_heads=2, head_dim=72, value_dim=40)
+    cu, seq, slots = layout([1] * seqs, [2, 4, 0, 9, 3])
+    ctx, table, keys, values = attention_case(g, dtype, [1] * seqs, [0, 7, 9, 14, 3], block_size=8, **geometry)
+    channels = 8 * 72 + 2 * 40
+    qkv, bias, conv_w, state = rand(g, seqs, channels, dtype=dtype), rand(g, channels), rand(g, channels, taps), rand(g, 6, taps - 1, channels)
+    inv_freq = 1.0 / 10000.0 ** (torch.arange(0, 32, 2).float() / 32)
+    found = []
+    for single in (False, True):
+        held = dev(qkv, bias, conv_w, state, inv_freq, torch.tensor([0, 7, 9, 14, 3], dtype=torch.int32), seq, cu, slots, table, keys, values)
+        q = torch.empty(seqs, 6 * 72, dtype=dtype, device=DEV)
+        ops.conv_rope_norm_write(*held, q, num_seqs=seqs, rotary_dim=32, unit_norm_eps=1e-6, taps=taps, single=single, **geometry)
+        found.append((q, held[3], held[10], held[11]))
+    assert all(torch.equal(a, b) for a, b in zip(*found))
+    with pytest.raises(ops.KernelError):
+        ops.conv_rope_norm_write(*held, q, num_seqs=seqs - 1, rotary_dim=32, unit_norm_eps=1e-6, taps=taps, single=True, **geometry)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

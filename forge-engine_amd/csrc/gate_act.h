@@ -23,3 +23,9 @@ __device__ __forceinline__ float gate_exponent(float g, GateAct act) { return -g
 // with the fast exponential, where the result is rounded to bfloat16
 __device__ __forceinline__ float gate_times(float g, float u, GateAct act) { return g / (1.f + __expf(gate_exponent(g, act))) * u; }
 __device__ __forceinline__ float gate_times_exact(float g, float u, GateAct act) { return g / (1.f + expf(gate_exponent(g, act))) * u; }
+// the bounded form: min(g, limit) * sigmoid(alpha min(g, limit)) * (clamp(u, -limit, limit) + 1)
+__device__ __forceinline__ float gate_bounded(float g, float u, float limit, float alpha) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g / (1.f + expf(-alpha * g)) * (u + 1.f);
+}

@@ -308,6 +308,15 @@ extern "C" int fe_gemm_wide(const void* x, const void* w, void* out, int M, int 
   return fe_check_launch();
 }
 
+// The bounded gate (gate_act.h) of a fused weight [2 N, K], gate rows first: out [M, N] bfloat16, ldo its row stride; lds_tile 9 to 13.
+extern "C" int fe_gemm_lds_bounded(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo,
+                                   int lds_tile, float limit, float alpha, hipStream_t stream) {
+  if (M < 1) return FE_OK;
+  if (N < 1 || K < WSTEP || K % WSTEP || ldw < K || ldw % 8 || ldo < N || !(limit > 0.f)) return FE_BAD_ARGUMENT;
+  if ((((uintptr_t)x) & 15) || (((uintptr_t)w) & 15)) return FE_BAD_ARGUMENT;
+  return through_lds::launch_bounded(x, w, out, M, N, K, ldw, ldo, lds_tile, limit, alpha, stream);
+}
+
 // Endings 0 and 2 through LDS for up to 16 rows of x whose norm's factors were left out: `squares` [M][256] float32 (fe_gemm_update_norm),
 // the sums of row m are multiplied by rsqrt(sum of squares[m] / width + eps).  lds_tile 9 to 13.
 extern "C" int fe_gemm_lds_scaled(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo,

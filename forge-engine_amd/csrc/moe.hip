@@ -21,6 +21,7 @@
 // MFMA 16x16x32 over tiles of 32 x 64 to 256 x 128 with rows and weight straight from memory in LDS.  A launch has as many row-tile slots as the pairs could need at worst (pairs /
 // rows a tile + experts); a block whose slot lies beyond the tiles there are returns at once.
 #include "common.h"
+#include "gate_act.h"
 #include "lds_tile.h"
 #include <algorithm>
 
@@ -277,9 +278,7 @@ __device__ __forceinline__ float gated(float g, float u, float limit, float alph
   u *= w;
   if (form == 2) return fmaxf(g, 0.f) * fmaxf(g, 0.f);      // one matrix an expert: g alone
   if (form == 1) return g / (1.f + expf(-g)) * u;
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g / (1.f + expf(-alpha * g)) * (u + 1.f);
+  return gate_bounded(g, u, limit, alpha);
 }
 
 // A token's first choice also takes what every token gets beside its experts (a shared expert's output,

@@ -1542,8 +1542,12 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
                     window: int | None = None, num_decode: int | None = None,
                     max_ctx: int | None = None, splits: int | None = None, chunk: int | None = None,
                     sink: Tensor | None = None, softcap: float | None = None, slopes: Tensor | None = None,
-                    dist_bias: Tensor | None = None, by_length: int | None = None) -> Tensor:
+                    dist_bias: Tensor | None = None, by_length: int | None = None,
+                    gate: tuple[Tensor, int, float] | None = None) -> Tensor:
     """Attention of every query token of a mixed batch over its paged keys.
+
+    ``gate`` (gate, share, factor): the output times sigmoid(gate) * factor, a gate for every ``share`` elements of a row; for
+    steps of single tokens alone (``num_decode`` = ``num_seqs``) of a bfloat16 cache.
 
     ``splits``: key runs of every single token's sequence; ``by_length``: runs by length instead, this many a kv head beyond the
     sequences (at most 64 of them); neither: ``decode_runs``.  Both are for the matrix-core decode kernel; another ignores them.
@@ -1563,7 +1567,7 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
     go to the streaming decode kernel and the others to the general kernel.
     """
     _gpu(q, "q", contiguous=False)
-    _gpu(out, "out", q.dtype)
+    _gpu(out, "out", q.dtype, contiguous=gate is None)
     _gpu(key_pages, "key_pages", q.dtype)
     _gpu(value_pages, "value_pages", q.dtype)
     _gpu(cu_q, "cu_q", torch.int32)
@@ -1572,7 +1576,7 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
     tokens = q.shape[0]
     if q.dim() != 2 or q.stride(1) != 1 or q.shape[1] < q_heads * head_dim:
         raise KernelError(f"q must be [T, >= {q_heads * head_dim}] with unit inner stride")
-    if out.shape != (tokens, q_heads * head_dim):
+    if out.shape != (tokens, q_heads * head_dim) or out.stride(1) != 1:
         raise KernelError(f"out must be [{tokens}, {q_heads * head_dim}], got {tuple(out.shape)}")
     if q_heads % kv_heads:
         raise KernelError("query heads must be a multiple of kv heads")
@@ -1593,11 +1597,15 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
         any_single, any_longer, num_decode = True, max_q_len > 1, num_seqs
     else:
         any_single, any_longer = num_decode > 0, num_decode < num_seqs
+    if gate is not None and (any_longer or q.dtype != torch.bfloat16 or gate[0].dtype != q.dtype or gate[0].shape[0] != tokens):
+        raise KernelError("a gate is for single tokens of a bfloat16 cache, in rows of the queries' type")
     bf16_pages = (q.dtype == torch.bfloat16 and block_size >= 16 and block_size & (block_size - 1) == 0
                   and q.data_ptr() % 16 == 0 and q_stride % 8 == 0)      # the fast kernels read 16 bytes at a time
     fast_decode = bf16_pages and head_dim in (64, 128, 256) and groups <= 8
     fast_prefill = bf16_pages and head_dim in (64, 128)
     masked = chunk is not None or sink is not None or softcap is not None or slopes is not None or dist_bias is not None
+    if gate is not None and not fast_decode:
+        raise KernelError("a gate is served by the matrix-core decode kernel only")
     if masked:
         if dist_bias is not None:     # a table of biases by distance, float32 [Hq, span]: entry min(position - j, span - 1) joins the score
             _gpu(dist_bias, "dist_bias", torch.float32)
@@ -1648,6 +1656,18 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
         if dist_bias is not None:
             mask = (c_int(chunk or 0), _ptr(sink), _ptr(dist_bias), c_int(dist_bias.shape[1]))
         cap = (c_float(softcap),) if softcap is not None else ()
+        if gate is not None:
+            values, share, factor = gate
+            if slopes is not None and softcap is not None:
+                raise KernelError("slopes do not go with a soft cap")
+            _call("attention_decode", "fe_paged_attention_decode_gated", _ptr(q), c_longlong(q_stride),
+                  _ptr(key_pages), _ptr(value_pages), _ptr(out), c_longlong(out.stride(0)), _ptr(part_o),
+                  _ptr(part_ml), _ptr(counters), _ptr(cu_q), _ptr(ctx_len), _ptr(block_table), c_int(block_table.stride(0)),
+                  c_int(num_seqs), c_int(kv_heads), c_int(groups), c_int(head_dim), c_int(block_size),
+                  c_int(num_blocks), c_int(window or 0), c_int(chunk or 0), _ptr(sink), _ptr(dist_bias if dist_bias is not None else slopes),
+                  c_int(dist_bias.shape[1] if dist_bias is not None else 0), c_float(scale), c_float(softcap or 0.0), c_int(splits),
+                  _ptr(values), c_longlong(_strided_rows(values, "gate", q_heads * head_dim // share)), c_int(share), c_float(factor), _stream())
+            return out
         name = ("fe_paged_attention_decode_biased" if dist_bias is not None else "fe_paged_attention_decode_sloped" if slopes is not None else "fe_paged_attention_decode_capped" if cap
                 else "fe_paged_attention_decode_masked" if masked else "fe_paged_attention_decode")
         _call("attention_decode", name, _ptr(q), c_longlong(q_stride),
@@ -2268,7 +2288,8 @@ def masked_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor | None, o
     filled up to sizes that the matrix-core kernels take): with a gate alone, whose kernel then leaves the rest out.  Scores and softmax
     float32.  A bfloat16 cache with keys and values of 64 or 128 elements, groups up to 8 and pages of
     a power of two >= 16 goes to the matrix-core kernels of ``paged_attention`` (single tokens and
-    portions each to its own), with the gate in a small kernel behind them; everything else, and
+    portions each to its own), with the gate in the single tokens' own kernel where a step has nothing else, in a small one behind
+    them where it has; everything else, and
     the float32 mode, to the vector-ALU kernel that does all of it in one launch."""
     _gpu(q, "q", contiguous=False)
     _gpu(key_pages, "key_pages", q.dtype)
@@ -2336,6 +2357,12 @@ def masked_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor | None, o
             and not (slopes is not None and softcap is not None) and value_pages is not None
             and not (dist_bias is not None and (slopes is not None or softcap is not None))
             and block_size >= 16 and block_size & (block_size - 1) == 0 and q.data_ptr() % 16 == 0 and q_stride % 8 == 0):
+        if gate is not None and num_decode == num_seqs and tokens <= num_seqs and out_stride % 2 == 0 and out.data_ptr() % 4 == 0:
+            # single tokens alone: the decode kernel multiplies what it stores
+            return paged_attention(q, key_pages, value_pages, out, cu_q, ctx_len, block_table, num_seqs=num_seqs, max_q_len=max_q_len,
+                                   q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, scale=scale, window=window,
+                                   num_decode=num_decode, max_ctx=max_ctx, chunk=chunk, sink=sink, softcap=softcap, slopes=slopes,
+                                   dist_bias=dist_bias, gate=(gate, value_dim if head_gate else 1, factor))
         attended = out if out.is_contiguous() else torch.empty_like(out, memory_format=torch.contiguous_format)
         paged_attention(q, key_pages, value_pages, attended, cu_q, ctx_len, block_table, num_seqs=num_seqs, max_q_len=max_q_len,
                         q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, scale=scale, window=window,
@@ -3112,7 +3139,17 @@ def moe_experts(x: Tensor, chosen: Tensor | None, weights: Tensor, gate_up: Tens
 
 def linear_gated(x: Tensor, gate_up_weight: Tensor, *, limit: float, alpha: float) -> Tensor:
     """``min(g, limit) * sigmoid(alpha * min(g, limit)) * (clamp(u, -limit, limit) + 1)`` with g and u the two
-    halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype."""
+    halves of ``x @ gate_up_weight^T`` ([2F, H]: gate rows first); the result [T, F] in x's dtype.  Up to 16 bfloat16 rows that go
+    through LDS: in the product's launch, with the bits of the two."""
+    if (isinstance(x, Tensor) and x.is_cuda and _lds_fits(x, gate_up_weight) and gate_up_weight.shape[0] % 2 == 0 and limit > 0.0
+            and not _few_rows_to_library(x, gate_up_weight) and _lds_store_pays(x.shape[0], *gate_up_weight.shape)):
+        (tokens, k), rows = x.shape, gate_up_weight.shape[0]
+        tile = lds_plan(tokens, rows, k, 2 * rows)[0]       # as `linear` takes it: the tile's sums are its, bit for bit
+        if tile is not None and tile >= 9:
+            out = torch.empty((tokens, rows // 2), dtype=x.dtype, device=x.device)
+            _call("gemm_wide", "fe_gemm_lds_bounded", _ptr(x), _ptr(gate_up_weight), _ptr(out), c_int(tokens), c_int(rows // 2), c_int(k),
+                  c_longlong(gate_up_weight.stride(0)), c_longlong(rows // 2), c_int(tile), c_float(limit), c_float(alpha), _stream())
+            return out
     gate_up = linear(x, gate_up_weight, ring=False)
     tokens, width = gate_up.shape
     if width % 2 or not limit > 0.0:

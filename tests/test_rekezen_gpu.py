@@ -170,6 +170,57 @@ def test_mixture_of_experts_kernels(tokens, hidden, experts, top, inner, dtype):
     close(ops.linear_gated(x.to(DEV), shared.to(DEV), limit=0.8, alpha=1.702), refs.linear_gated(x, shared, limit=0.8, alpha=1.702), dtype)
 
 
+# one row, a tile's last, columns that fill no tile of gate and up rows, the shortest K, every tile
+@pytest.mark.parametrize("rows,columns,k", [(5, 1024, 2048), (8, 2048, 2048), (16, 2047, 1024), (9, 2500, 1024), (16, 1030, 4096), (12, 4100, 1088), (13, 8192, 1024)])
+def test_bounded_gate_in_its_product(rows, columns, k, monkeypatch):
+    """The bits of the product and a launch of the activation."""
+    from forge_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + columns)
+    x = torch.randn(rows, k, generator=g).bfloat16().to(DEV)
+    weight = (torch.randn(2 * columns, k, generator=g) * 2 * k ** -0.5).bfloat16().to(DEV)
+    calls = []
+    real = ops._call
+    monkeypatch.setattr(ops, "_call", lambda library, name, *args: (calls.append(name), real(library, name, *args)))
+    got = ops.linear_gated(x, weight, limit=1.5, alpha=1.702)
+    assert calls == ["fe_gemm_lds_bounded"]
+    monkeypatch.setattr(ops, "_lds_store_pays", lambda *sizes: False)
+    calls.clear()
+    both = ops.gemm_lds(x, weight, "bf16", tile=ops.lds_plan(rows, 2 * columns, k, 4 * columns)[0])
+    monkeypatch.setattr(ops, "linear", lambda *args, **how: both)
+    want = ops.linear_gated(x, weight, limit=1.5, alpha=1.702)
+    assert calls[-1] == "fe_gated_act" and torch.equal(got, want)
+
+
+# keys in one run, a few, more than sixteen; a gate a head and one an element; rows of q, gate and output of other strides
+@pytest.mark.parametrize("form", ["plain", "capped", "sloped", "table", "sink"])
+@pytest.mark.parametrize("dim,per_head,contexts", [(128, True, (1, 33, 700, 16)), (64, False, (40, 3, 1, 257, 90)), (128, False, (4000,)), (64, True, (9,) * 20)])
+def test_gate_in_the_decode_kernel(dim, per_head, contexts, form):
+    """Single tokens: the bits of the attention and a launch of the gate."""
+    from forge_engine_amd.kernels import ops
+    n, heads, kv_heads, page = len(contexts), 8, 2, 16
+    g = torch.Generator().manual_seed(dim + n)
+    pages = [-(-c // page) for c in contexts]
+    table = torch.zeros(n, max(pages), dtype=torch.int32)
+    order = torch.randperm(sum(pages), generator=g).int()
+    for i, count in enumerate(pages):
+        table[i, :count] = order[sum(pages[:i]):sum(pages[:i]) + count]
+    keys = torch.randn(sum(pages), kv_heads, page, dim, generator=g).bfloat16().to(DEV)
+    values = torch.randn(sum(pages), kv_heads, dim, page, generator=g).bfloat16().to(DEV)
+    q = torch.randn(n, heads * dim + 64, generator=g).bfloat16().to(DEV)[:, :heads * dim]
+    gate = torch.randn(n, heads * (1 if per_head else dim) + 3, generator=g).bfloat16().to(DEV)[:, 3:]
+    kinds = {"plain": {}, "capped": {"softcap": 20.0}, "sloped": {"slopes": torch.rand(heads, generator=g).to(DEV) * 0.1},
+             "table": {"dist_bias": torch.randn(heads, 50, generator=g).to(DEV)}, "sink": {"sink": torch.randn(heads, generator=g).to(DEV)}}
+    where = (torch.arange(n + 1, dtype=torch.int32, device=DEV), torch.tensor(contexts, dtype=torch.int32, device=DEV), table.to(DEV))
+    how = dict(num_seqs=n, max_q_len=1, q_heads=heads, kv_heads=kv_heads, head_dim=dim, value_dim=dim, scale=dim ** -0.5, num_decode=n,
+               max_ctx=max(contexts), **kinds[form])
+    got = torch.empty(n, heads * dim + 2, dtype=torch.bfloat16, device=DEV)[:, :heads * dim]
+    ops.masked_attention(q, keys, values, got, *where, gate=gate, head_gate=per_head, factor=1.25, **how)
+    apart, want = (torch.empty(n, heads * dim, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.masked_attention(q, keys, values, apart, *where, **how)
+    ops._sigmoid_gate(apart, gate, want, heads, dim, dim, per_head, 1.25)
+    assert torch.equal(got, want)
+
+
 # the smallest, most tokens, experts, pairs and choices, and one of each too many
 @pytest.mark.parametrize("scoring,biased", [("softmax", True), ("sigmoid", False)])
 @pytest.mark.parametrize("tokens,experts,top", [(1, 1, 1), (8, 8, 2), (64, 64, 4), (16, 17, 16), (64, 3, 3), (65, 8, 2), (8, 65, 2), (33, 64, 8)])

@@ -1,6 +1,3 @@
-#ifndef SPREAD
-#define SPREAD 3
-#endif
 // float32 matrix product C[M,N] = A[M,K] * B[N,K]^T (+ bias[N]) of the rows of prompts, each operand in three bfloat16 parts (split_f32.h) and
 // A split ahead, by a launch of its own: [3][M][K] planes of bfloat16, which a block then fetches like any bfloat16 operand.
 // (gemm_split splits a fragment wherever it is used: every element of A by every block of its rows, in two waves of each.)
@@ -23,6 +20,8 @@ namespace {
 
 using split_f32::bf16x2;
 using split_f32::bf16x8;
+using split_f32::split2;
+using split_f32::split8;
 using lds_tile::floatx4;
 using lds_tile::wait_loads;
 
@@ -32,31 +31,6 @@ constexpr int XCDS = 8, KSTEP = 64, GROUPS = 2, WAVES = 8;
 // vector register, and nothing else in these kernels uses m0, so it is left as it is.
 __device__ __forceinline__ void load_to_lds(const void* base, unsigned int offset, unsigned int at) {
   asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(at) : "memory", "m0");
-}
-
-// Two floats as three pairs of bfloat16, each part the rounding of what the parts before leave: 5.5 instructions each, of the kind that runs
-// beside the matrix cores.  (split_f32's dot product with (-1, 0) takes a part off its number in one instruction instead of two, but holds
-// those up: a step of 128 x 128 2.25 -> 2.08 us.  Where splitting itself is the bound, as in gemm_split, that form is the faster one.)
-__device__ __forceinline__ void split2(float x0, float x1, unsigned& high, unsigned& middle, unsigned& low) {
-  high = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x0, (__bf16)x1});
-  const float r0 = x0 - __uint_as_float(high << 16), r1 = x1 - __uint_as_float(high & 0xffff0000u);
-  middle = __builtin_bit_cast(unsigned, bf16x2{(__bf16)r0, (__bf16)r1});
-  const float s0 = r0 - __uint_as_float(middle << 16), s1 = r1 - __uint_as_float(middle & 0xffff0000u);
-  low = __builtin_bit_cast(unsigned, bf16x2{(__bf16)s0, (__bf16)s1});
-}
-__device__ __forceinline__ void split8(floatx4 u, floatx4 v, bf16x8 (&parts)[3]) {
-  typedef __attribute__((ext_vector_type(4))) unsigned int uintx4;
-  uintx4 p[3];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    unsigned a, b, c;
-    split2(u[2 * e], u[2 * e + 1], a, b, c);
-    p[0][e] = a; p[1][e] = b; p[2][e] = c;
-    split2(v[2 * e], v[2 * e + 1], a, b, c);
-    p[0][2 + e] = a; p[1][2 + e] = b; p[2][2 + e] = c;
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) parts[i] = __builtin_bit_cast(bf16x8, p[i]);
 }
 
 // A [M, K] float32 as planes [3][M][KP] bfloat16, zeros beyond K: eight elements a thread
@@ -286,18 +260,21 @@ int launch(const bf16_t* planes, const float* A, const float* B, const float* bi
 // A [M, K], B [N, K] float32, rows 16-byte aligned (strides lda, ldb), K a multiple of four; planes: room for 3 M bfloat16 rows of K rounded up
 // to 64, less than 4 GB; bias [N] or null; C holds `parts` matrices [M, N] (row stride ldc) part_stride floats apart, each the sum over a run of whole
 // steps of K, whose sum is the product; with a bias one.  A block takes 16 rows16 rows of A x 64 columns64 rows of B.
+// ready: the planes hold A's parts already (who made A stored them beside it).
 extern "C" int fe_gemm_planes(const float* A, void* planes, const float* B, const float* bias, float* C, int M, int N, int K, long long lda,
-                              long long ldb, long long ldc, int parts, long long part_stride, int rows16, int columns64, hipStream_t stream) {
+                              long long ldb, long long ldc, int parts, long long part_stride, int rows16, int columns64, int ready, hipStream_t stream) {
   if (M < 1 || N < 1) return FE_OK;
   if (K < 4 || K % 4 || lda < K || ldb < K || ldc < N || lda % 4 || ldb % 4 || ldb >= (1 << 22)) return FE_BAD_ARGUMENT;
   if ((((uintptr_t)planes) | ((uintptr_t)A) | ((uintptr_t)B)) & 15) return FE_BAD_ARGUMENT;
   const int KP = (K + KSTEP - 1) / KSTEP * KSTEP;
   if (parts < 1 || parts > 64 || parts > KP / KSTEP || (parts > 1 && (bias || part_stride < (long long)M * ldc))) return FE_BAD_ARGUMENT;
   if (6LL * M * KP >= (1LL << 32)) return FE_BAD_ARGUMENT;
-  const long long blocks = ((long long)M * (KP / 8) + 255) / 256;
-  split_rows_kernel<<<(unsigned)blocks, 256, 0, stream>>>(A, (bf16_t*)planes, M, K, KP, lda);
-  const int split = fe_check_launch();
-  if (split != FE_OK) return split;
+  if (!ready) {
+    const long long blocks = ((long long)M * (KP / 8) + 255) / 256;
+    split_rows_kernel<<<(unsigned)blocks, 256, 0, stream>>>(A, (bf16_t*)planes, M, K, KP, lda);
+    const int split = fe_check_launch();
+    if (split != FE_OK) return split;
+  }
 #define FE_TILE(MI, NI) \
   if (rows16 == MI && columns64 == NI) return launch<MI, NI>((const bf16_t*)planes, A, B, bias, C, M, N, K, lda, ldb, ldc, parts, part_stride, stream);
   FE_TILE(4, 1) FE_TILE(4, 2) FE_TILE(5, 2) FE_TILE(6, 1) FE_TILE(6, 2) FE_TILE(7, 2) FE_TILE(8, 1) FE_TILE(8, 2) FE_TILE(9, 1) FE_TILE(10, 1)

@@ -3,6 +3,7 @@
 // products are float32 or bfloat16.
 #include "common.h"
 #include "gate_act.h"
+#include "split_f32.h"
 
 // ---------------------------------------------------------------- embedding
 // out[t, :] = float(table[ids[t], :]) * scale.  One block per token.
@@ -208,12 +209,26 @@ __device__ __forceinline__ void store4_from_float(bf16_t* p, float4 v) {
   *(uint2*)p = u;
 }
 
-template <typename TD, typename TO, int VEC, int THREADS>
+// Four floats as their three parts (split_f32.h), in planes [3][rows][width]
+__device__ __forceinline__ void store4_split(bf16_t* planes, size_t rows, size_t row, int width, int at, float4 v) {
+  // (the parts are those of the rounded numbers: the compiler must not join the product that made one with the subtraction here)
+  asm("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
+  uint2 p[3];
+  split_f32::split2(v.x, v.y, p[0].x, p[1].x, p[2].x);
+  split_f32::split2(v.z, v.w, p[0].y, p[1].y, p[2].y);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *(uint2*)(planes + (i * rows + row) * width + at) = p[i];
+}
+
+// SPLIT: the result's parts go into `planes` as well, for a product that takes them (gemm_planes.hip), which saves the launch that would read the
+// result again to make them (us, 700 rows of 1,024: 3.7 -> 4.5, and the product of 4,096 columns behind it 42 -> 35; with the gate below, of
+// 3,072 columns: 6.9 -> 7.2, and the product of 1,024 behind it 36 -> 27)
+template <typename TD, typename TO, int VEC, int THREADS, bool SPLIT = false>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_regs_kernel(
     float* __restrict__ h, const TD* __restrict__ delta, const float* __restrict__ other, const float* __restrict__ shift,
     const float* __restrict__ w,
     TO* __restrict__ out, const int* __restrict__ rows, int hidden, float eps, int store_sum,
-    int parts, size_t part_stride) {
+    int parts, size_t part_stride, bf16_t* __restrict__ planes) {
   __shared__ float scratch[16];
   const int r = blockIdx.x;
   const int s = rows ? rows[r] : r;
@@ -260,31 +275,35 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_regs_kernel(
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
     const int i = (threadIdx.x + j * THREADS) * 4;
-    if (i < hidden)
-      store4_from_float(orow + i, make_float4(v[j].x * inv * ww[j].x, v[j].y * inv * ww[j].y,
-                                              v[j].z * inv * ww[j].z, v[j].w * inv * ww[j].w));
+    if (i < hidden) {
+      const float4 y = make_float4(v[j].x * inv * ww[j].x, v[j].y * inv * ww[j].y, v[j].z * inv * ww[j].z, v[j].w * inv * ww[j].w);
+      store4_from_float(orow + i, y);
+      if constexpr (SPLIT) store4_split(planes, gridDim.x, r, hidden, i, y);
+    }
   }
 }
 
-template <typename TD, typename TO>
-static void launch_add_rmsnorm_typed(float* h, const TD* delta, const float* other, const float* shift, const float* w, TO* out, const int* rows,
+template <typename TD, typename TO, bool SPLIT = false>
+static bool launch_add_rmsnorm_typed(float* h, const TD* delta, const float* other, const float* shift, const float* w, TO* out, const int* rows,
                                      int n_rows, int hidden, float eps, int store_sum, int parts,
-                                     size_t part_stride, hipStream_t stream) {
+                                     size_t part_stride, hipStream_t stream, bf16_t* planes = nullptr) {
   const bool aligned = hidden % 4 == 0 && part_stride % 4 == 0 && (((uintptr_t)h | (uintptr_t)delta | (uintptr_t)other | (uintptr_t)shift | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
   if (aligned && n_rows <= 512 && hidden > 1024 && hidden <= 4096)   // up to a few hundred rows: a whole row in flight at once
-    add_rmsnorm_regs_kernel<TD, TO, 1, 1024><<<n_rows, 1024, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride);
+    add_rmsnorm_regs_kernel<TD, TO, 1, 1024, SPLIT><<<n_rows, 1024, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride, planes);
   else if (aligned && n_rows <= 512 && hidden > 4096 && hidden <= 8192)
-    add_rmsnorm_regs_kernel<TD, TO, 2, 1024><<<n_rows, 1024, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride);
+    add_rmsnorm_regs_kernel<TD, TO, 2, 1024, SPLIT><<<n_rows, 1024, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride, planes);
   else if (aligned && hidden <= 1024)
-    add_rmsnorm_regs_kernel<TD, TO, 1, 256><<<n_rows, 256, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride);
+    add_rmsnorm_regs_kernel<TD, TO, 1, 256, SPLIT><<<n_rows, 256, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride, planes);
   else if (aligned && hidden <= 4096)
-    add_rmsnorm_regs_kernel<TD, TO, 4, 256><<<n_rows, 256, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride);
+    add_rmsnorm_regs_kernel<TD, TO, 4, 256, SPLIT><<<n_rows, 256, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride, planes);
   else if (aligned && hidden <= 8192)
-    add_rmsnorm_regs_kernel<TD, TO, 8, 256><<<n_rows, 256, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride);
+    add_rmsnorm_regs_kernel<TD, TO, 8, 256, SPLIT><<<n_rows, 256, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride, planes);
+  else if (SPLIT) return false;
   else {
     const int threads = hidden >= 2048 ? 512 : (hidden >= 512 ? 256 : 64);
     add_rmsnorm_kernel<TD, TO><<<n_rows, threads, 0, stream>>>(h, delta, other, shift, w, out, rows, hidden, eps, store_sum, parts, part_stride);
   }
+  return true;
 }
 
 template <typename TD>
@@ -314,6 +333,20 @@ extern "C" int fe_add_rmsnorm(float* h, const void* delta, int delta_dtype, cons
   if (delta_dtype == FE_BF16)
     return launch_add_rmsnorm<bf16_t>(h, (const bf16_t*)delta, other, shift, w, out, out_dtype, rows, n_rows, hidden, eps, store_sum, delta_parts, (size_t)part_stride, stream);
   return FE_BAD_ARGUMENT;
+}
+
+// The same of float32 rows in order, with the result's parts beside it: planes [3][n_rows][hidden] bfloat16; up to 8,192 columns, a multiple of
+// 64, everything 16-byte aligned.
+extern "C" int fe_add_rmsnorm_split(float* h, const float* delta, const float* other, const float* shift, const float* w, float* out, void* planes,
+                                    int n_rows, int hidden, float eps, int store_sum, int delta_parts, long long part_stride,
+                                    hipStream_t stream) {
+  if (n_rows <= 0) return FE_OK;
+  if (hidden <= 0 || hidden % 64 || !planes || (((uintptr_t)planes) & 15) || !(eps > 0.f) || delta_parts < 1 || delta_parts > 64 || part_stride < 0)
+    return FE_BAD_ARGUMENT;
+  if (!launch_add_rmsnorm_typed<float, float, true>(h, delta, other, shift, w, out, nullptr, n_rows, hidden, eps, store_sum, delta_parts,
+                                                    (size_t)part_stride, stream, (bf16_t*)planes))
+    return FE_BAD_ARGUMENT;
+  return fe_check_launch();
 }
 
 // h[t] += delta[t] + other[t] + shift for all rows (flushes what is pending without a norm; any of the three
@@ -410,6 +443,31 @@ extern "C" int fe_swiglu(const void* gate_up, long long in_stride, void* out, lo
     swiglu_kernel<bf16_t><<<blocks, threads, 0, stream>>>((const bf16_t*)gate_up, (size_t)in_stride, (bf16_t*)out, (size_t)out_stride, inter, total, act);
   else
     return FE_BAD_ARGUMENT;
+  return fe_check_launch();
+}
+
+// The same for float32, four elements a thread, with the result's parts beside it: planes [3][tokens][inter] bfloat16
+__global__ __launch_bounds__(256) void swiglu_split_kernel(const float* __restrict__ gate_up, size_t in_stride, float* __restrict__ out,
+                                                           bf16_t* __restrict__ planes, int inter, size_t tokens, GateAct act) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, t = i / inter;
+  const int c = (int)(i - t * inter);
+  if (t >= tokens) return;
+  const float4 g = *(const float4*)(gate_up + t * in_stride + c), u = *(const float4*)(gate_up + t * in_stride + inter + c);
+  const float4 y = make_float4(gate_times_exact(g.x, u.x, act), gate_times_exact(g.y, u.y, act), gate_times_exact(g.z, u.z, act), gate_times_exact(g.w, u.w, act));
+  *(float4*)(out + i) = y;
+  store4_split(planes, tokens, t, inter, c, y);
+}
+
+extern "C" int fe_swiglu_split(const float* gate_up, long long in_stride, float* out, void* planes, int tokens, int inter, int activation,
+                               hipStream_t stream) {
+  if (tokens <= 0) return FE_OK;
+  GateAct act;
+  if (!gate_act(activation, &act)) return FE_BAD_ARGUMENT;
+  if (inter <= 0 || inter % 64 || in_stride < 2LL * inter || in_stride % 4 || !planes) return FE_BAD_ARGUMENT;
+  if ((((uintptr_t)gate_up) | ((uintptr_t)out) | ((uintptr_t)planes)) & 15) return FE_BAD_ARGUMENT;
+  const long long blocks = ((long long)tokens * inter / 4 + 255) / 256;
+  if (blocks > 0x7fffffffLL) return FE_BAD_ARGUMENT;
+  swiglu_split_kernel<<<(unsigned)blocks, 256, 0, stream>>>(gate_up, (size_t)in_stride, out, (bf16_t*)planes, inter, (size_t)tokens, act);
   return fe_check_launch();
 }
 

@@ -56,6 +56,29 @@ __device__ __forceinline__ void split8(floatx4 u, floatx4 v, const Minus& minus,
   for (int i = 0; i < 3; ++i) parts[i] = __builtin_bit_cast(bf16x8, p[i]);
 }
 
+// The same, the same bits, in 5.5 instructions each of the kind that runs beside the matrix cores.  (The dot product with (-1, 0) takes a part off its number in one instruction instead of two, but holds
+// those up: a step of 128 x 128 2.25 -> 2.08 us.  Where splitting itself is the bound, as in gemm_split, that form is the faster one.)
+__device__ __forceinline__ void split2(float x0, float x1, unsigned& high, unsigned& middle, unsigned& low) {
+  high = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x0, (__bf16)x1});
+  const float r0 = x0 - __uint_as_float(high << 16), r1 = x1 - __uint_as_float(high & 0xffff0000u);
+  middle = __builtin_bit_cast(unsigned, bf16x2{(__bf16)r0, (__bf16)r1});
+  const float s0 = r0 - __uint_as_float(middle << 16), s1 = r1 - __uint_as_float(middle & 0xffff0000u);
+  low = __builtin_bit_cast(unsigned, bf16x2{(__bf16)s0, (__bf16)s1});
+}
+__device__ __forceinline__ void split8(floatx4 u, floatx4 v, bf16x8 (&parts)[3]) {
+  uintx4 p[3];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    unsigned a, b, c;
+    split2(u[2 * e], u[2 * e + 1], a, b, c);
+    p[0][e] = a; p[1][e] = b; p[2][e] = c;
+    split2(v[2 * e], v[2 * e + 1], a, b, c);
+    p[0][2 + e] = a; p[1][2 + e] = b; p[2][2 + e] = c;
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) parts[i] = __builtin_bit_cast(bf16x8, p[i]);
+}
+
 // acc(i) += first operand b x second operands a[i], i < COUNT, over 32 of K.  The products of the first parts go into the long sum; the
 // others, a 2^8th of their size, are added up by themselves first, so that the long sum is rounded twice for all six and not six
 // times.  (The instruction cuts off what an addend has below the last bit of a larger one, downwards: a sum that the small products

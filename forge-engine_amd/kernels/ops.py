@@ -95,11 +95,11 @@ def embed_rows(ids: Tensor, table: Tensor, out: Tensor, scale: float = 1.0, norm
 
 def add_rmsnorm(h: Tensor, delta: Tensor | None, weight: Tensor, eps: float, out: Tensor,
                 rows: Tensor | None = None, store_sum: bool = True, other: Tensor | None = None,
-                shift: Tensor | None = None) -> Tensor:
+                shift: Tensor | None = None, planes: Tensor | None = None) -> Tensor:
     """sum = h[s] + delta[s] + other[s] + shift (float32, written back to h if store_sum);
     out[r] = sum * rsqrt(mean(sum^2) + eps) * weight, s = rows[r] or r.
     delta may be [parts, rows, hidden]: the parts are added up in order first.  other: float32 like h, shift: float32
-    [hidden]; any of the three may be None."""
+    [hidden]; any of the three may be None.  planes [3, rows, hidden] bfloat16: takes the result's parts (``SplitRows``)."""
     _gpu(h, "h", torch.float32)
     _gpu(weight, "weight", torch.float32)
     _gpu(out, "out")
@@ -121,6 +121,14 @@ def add_rmsnorm(h: Tensor, delta: Tensor | None, weight: Tensor, eps: float, out
         raise KernelError(f"out must be [{n_rows}, {hidden}], got {tuple(out.shape)}")
     if not eps > 0.0:
         raise KernelError("eps must be positive")
+    if planes is not None:
+        _gpu(planes, "planes", torch.bfloat16)
+        if rows is not None or out.dtype != torch.float32 or planes.shape != (3, *out.shape) or (delta is not None and delta.dtype != torch.float32):
+            raise KernelError("the parts of a norm's rows come of float32 rows in order")
+        _call("rowwise", "fe_add_rmsnorm_split", _ptr(h), _ptr(delta), _ptr(other), _ptr(shift), _ptr(weight), _ptr(out), _ptr(planes),
+              c_int(n_rows), c_int(hidden), c_float(eps), c_int(1 if store_sum and not (delta is None and other is None and shift is None) else 0),
+              c_int(parts), c_longlong(h.numel()), _stream())
+        return out
     _call("rowwise", "fe_add_rmsnorm", _ptr(h), _ptr(delta),
           c_int(_code(delta.dtype) if delta is not None else FE_F32), _ptr(other), _ptr(shift), _ptr(weight), _ptr(out),
           c_int(_code(out.dtype)), _ptr(rows), c_int(n_rows), c_int(hidden), c_float(eps),
@@ -172,14 +180,21 @@ def _gate_act(act: str) -> c_int:
     return c_int(GATE_ACTS[act])
 
 
-def swiglu(gate_up: Tensor, out: Tensor, act: str = "silu") -> Tensor:
+def swiglu(gate_up: Tensor, out: Tensor, act: str = "silu", planes: Tensor | None = None) -> Tensor:
     """out[t, i] = act(gate_up[t, i]) * gate_up[t, I + i]; rows of any stride.  ``act``: ``silu`` or ``gelu_tanh``
-    (0.5 z (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))))."""
+    (0.5 z (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3)))).  ``planes``: as ``add_rmsnorm``'s."""
     tokens, two_inter = gate_up.shape
     in_stride = _strided_rows(gate_up, "gate_up", two_inter)
     if two_inter % 2 or out.shape != (tokens, two_inter // 2) or out.dtype != gate_up.dtype:
         raise KernelError(f"out must be [{tokens}, {two_inter // 2}] in gate_up's dtype, got {tuple(out.shape)}")
     out_stride = _strided_rows(out, "out", two_inter // 2)
+    if planes is not None:
+        _gpu(planes, "planes", torch.bfloat16)
+        if out.dtype != torch.float32 or not out.is_contiguous() or planes.shape != (3, *out.shape):
+            raise KernelError("the parts of a gate's rows come of dense float32 rows")
+        _call("rowwise", "fe_swiglu_split", _ptr(gate_up), c_longlong(in_stride), _ptr(out), _ptr(planes), c_int(tokens), c_int(two_inter // 2),
+              _gate_act(act), _stream())
+        return out
     _call("rowwise", "fe_swiglu", _ptr(gate_up), c_longlong(in_stride), _ptr(out), c_longlong(out_stride), c_int(_code(out.dtype)),
           c_int(tokens), c_int(two_inter // 2), _gate_act(act), _stream())
     return out
@@ -304,10 +319,46 @@ def _split_pays(m: int, n: int, k: int, most_parts: int) -> bool:
     return us < 1.25 * _tiles_f32_us(m, n, k)
 
 
-def gemm_split(a: Tensor, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+class SplitRows(NamedTuple):
+    """Rows [M, K] float32 and, made with them, their parts in bfloat16 (planes [3, M, K]) for the products that take them ahead: the same
+    products of the same tiles, without the pass that makes the parts."""
+
+    rows: Tensor
+    planes: Tensor
+
+    @classmethod
+    def empty(cls, m: int, k: int, device) -> SplitRows:
+        return cls(torch.empty((m, k), dtype=torch.float32, device=device), torch.empty((3, m, k), dtype=torch.bfloat16, device=device))
+
+    @property
+    def shape(self) -> torch.Size:
+        return self.rows.shape
+
+
+SPLIT_AHEAD_MAX_K = 8192        # the widest rows that the norm's kernel holds in registers
+
+
+def takes_split(rows: int, weight: Tensor, update: bool = False) -> bool:
+    """Whether ``linear`` (``linear_update``) takes ``SplitRows`` of so many rows: where it takes planes for their float32 rows."""
+    if not weight.is_cuda or weight.dtype != torch.float32 or weight.dim() != 2 or rows <= SPLIT_MIN_ROWS_F32:
+        return False
+    n, k = weight.shape
+    if (k % 64 or k < SPLIT_MIN_K or (k > SPLIT_AHEAD_MAX_K and not update) or weight.stride(1) != 1 or weight.stride(0) % 4 or not k <= weight.stride(0) < 1 << 22
+            or weight.data_ptr() % 16 or 6 * rows * (k + 63) >= 1 << 32):
+        return False
+    most_parts = SPLIT_MOST_PARTS if update else 1
+    return _split_pays(rows, n, k, most_parts) and isinstance(_product_plan(rows, n, k, most_parts, True)[0], tuple)
+
+
+def gemm_split(a: Tensor | SplitRows, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
     """float32 partial sums [parts, M, N] of a[M, K] @ b[N, K]^T over runs of whole steps of K (given ``out`` [M, N], the product with
     the bias there), each operand as three bfloat16 numbers whose sum it is (a number below 2^-110: up to 2^-134 beside it).  ``tile``: the
-    block's, of ``SPLIT_TILES`` by its number, or of ``PLANES_TILES`` (a split ahead)."""
+    block's, of ``SPLIT_TILES`` by its number, or of ``PLANES_TILES`` (a split ahead, here or by who made a)."""
+    made = None
+    if isinstance(a, SplitRows):
+        a, made = a
+        if not isinstance(tile, tuple) or a.shape[1] % 64 or not a.is_contiguous() or _gpu(made, "planes", torch.bfloat16).shape != (3, *a.shape):
+            raise KernelError("parts made ahead are for the tiles of planes, dense rows and K a multiple of 64")
     _gpu(a, "a", torch.float32, contiguous=False)
     _gpu(b, "b", torch.float32, contiguous=False)
     planes = isinstance(tile, tuple)
@@ -322,9 +373,9 @@ def gemm_split(a: Tensor, b: Tensor, parts: int, tile: int | tuple[int, int], bi
         raise KernelError(f"bias must be [{n}]")
     result = torch.empty((parts, m, n), dtype=torch.float32, device=a.device) if out is None else out
     if planes:
-        scratch = torch.empty(3 * m * (-(-k // 64) * 64), dtype=torch.bfloat16, device=a.device)
+        scratch = torch.empty(3 * m * (-(-k // 64) * 64), dtype=torch.bfloat16, device=a.device) if made is None else made
         _call("gemm_planes", "fe_gemm_planes", _ptr(a), _ptr(scratch), _ptr(b), _ptr(bias), _ptr(result), c_int(m), c_int(n), c_int(k),
-              c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile[0]), c_int(tile[1]), _stream())
+              c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile[0]), c_int(tile[1]), c_int(int(made is not None)), _stream())
         return result
     _call("gemm_split", "fe_gemm_split", _ptr(a), _ptr(b), _ptr(bias), _ptr(result), c_int(m), c_int(n), c_int(k),
           c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile), _stream())
@@ -445,7 +496,7 @@ def _few_rows_library_pays(rows: int, weight: Tensor) -> bool:
             and weight.shape[0] * weight.shape[1] * weight.element_size() > IN_PARTS_MAX_WEIGHT_BYTES)
 
 
-def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None, out_dtype=None, ring: bool = True) -> Tensor:
+def linear(x: Tensor | UnscaledRows | SplitRows, weight: Tensor, bias: Tensor | None = None, out_dtype=None, ring: bool = True) -> Tensor:
     """y = x @ weight^T (+ bias) for a weight in [out, in] layout; float32
     accumulation; y in ``out_dtype`` (default: x's dtype).
 
@@ -464,6 +515,11 @@ def linear(x: Tensor | UnscaledRows, weight: Tensor, bias: Tensor | None = None,
         if bias is not None or out_dtype not in (None, x.rows.dtype) or not unscaled_linear(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
             raise KernelError("rows without their norm's factors are for the products through LDS only")
         return gemm_ring(x, weight, "f32" if weight.dtype == torch.float32 else "bf16")
+    if isinstance(x, SplitRows):
+        if out_dtype not in (None, torch.float32) or not takes_split(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
+            raise KernelError("rows with their parts are for the products of planes only")
+        y = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=weight.device)
+        return gemm_split(x, weight, 1, _product_plan(x.shape[0], *weight.shape, 1, True)[0], bias, y)
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     out_dtype = x.dtype if out_dtype is None else out_dtype
@@ -1125,12 +1181,17 @@ def _big_update_parts(rows: int, weight_rows: int, k: int) -> int:
     return parts if 2 <= parts <= 7 and rows * weight_rows * parts >= 0.75 * WIDE_CUS * 256 * 256 else 0
 
 
-def linear_update(x: Tensor, weight: Tensor, bias: Tensor | None = None, stream: Tensor | None = None) -> Tensor | None:
+def linear_update(x: Tensor | SplitRows, weight: Tensor, bias: Tensor | None = None, stream: Tensor | None = None) -> Tensor | None:
     """The float32 product x @ weight^T (+ bias) as an update of the residual stream: [M, N], or
     partial sums [parts, M, N] that ``add_rmsnorm`` / ``add_rows`` add up.  Given the float32
     ``stream`` [M, N] itself, the matrix library's product (more than 64 rows) adds into it as it
     stores, which saves the next norm the update's bytes, and None is returned: the same float32
     sum in the same order, stream + (x @ weight^T)."""
+    if isinstance(x, SplitRows):
+        if bias is not None or not takes_split(x.shape[0], weight, update=True) or weight.shape[1] != x.shape[1]:
+            raise KernelError("rows with their parts are for the products of planes only")
+        tile, parts = _product_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS, True)
+        return gemm_split(x, weight, parts, tile)
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     if bias is None and x.shape[0] > SPLIT_MIN_ROWS and _split_fits(x, weight) and _split_pays(x.shape[0], *weight.shape, SPLIT_MOST_PARTS):
@@ -1280,8 +1341,11 @@ GATED_TILE_MAX_ROWS = 4096
 GATED_TILE_MAX_K = 3072
 
 
-def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "silu") -> Tensor:
-    """act(x Wg^T) * (x Wu^T) for the fused weight [2I, K] (gate rows first); ``act`` as in ``swiglu``."""
+def linear_swiglu(x: Tensor | UnscaledRows | SplitRows, gate_up_weight: Tensor, act: str = "silu", split: bool = False) -> Tensor | SplitRows:
+    """act(x Wg^T) * (x Wu^T) for the fused weight [2I, K] (gate rows first); ``act`` as in ``swiglu``.  ``split``: float32 rows that
+    were not gated in the product's own launch come as ``SplitRows``."""
+    if isinstance(x, SplitRows):
+        return _swiglu_rows(linear(x, gate_up_weight), act, split)
     if isinstance(x, UnscaledRows):
         if not unscaled_swiglu(x.shape[0], gate_up_weight) or gate_up_weight.shape[1] != x.shape[1]:
             raise KernelError("rows without their norm's factors are for the products through LDS only")
@@ -1326,9 +1390,16 @@ def linear_swiglu(x: Tensor | UnscaledRows, gate_up_weight: Tensor, act: str = "
         return gemm_wide(x, gate_up_weight, "swiglu_half", block_rows=_gate_block_columns(gate_up_weight.shape[0] // 2), act=act)
     if _skinny_fits(x, gate_up_weight) and not to_library:
         return gemm_skinny(x, gate_up_weight, "swiglu", act=act)
-    gate_up = torch.matmul(x, gate_up_weight.t()) if to_library else linear(x, gate_up_weight)
-    out = torch.empty((x.shape[0], gate_up_weight.shape[0] // 2), dtype=gate_up.dtype, device=x.device)
-    return swiglu(gate_up, out, act)
+    return _swiglu_rows(torch.matmul(x, gate_up_weight.t()) if to_library else linear(x, gate_up_weight), act, split)
+
+
+def _swiglu_rows(gate_up: Tensor, act: str, split: bool) -> Tensor | SplitRows:
+    rows, columns = gate_up.shape[0], gate_up.shape[1] // 2
+    if split and gate_up.dtype == torch.float32 and columns % 64 == 0:
+        out = SplitRows.empty(rows, columns, gate_up.device)
+        swiglu(gate_up, out.rows, act, out.planes)
+        return out
+    return swiglu(gate_up, torch.empty((rows, columns), dtype=gate_up.dtype, device=gate_up.device), act)
 
 
 # ------------------------------------------------------------------ attention

@@ -329,7 +329,13 @@ class GroupedQueryAttention(Mixer):
             return ops.unscaled_in_parts(tokens, self.qkv_weight)
         return ops.unscaled_linear(tokens, self.qkv_weight)
 
-    def forward(self, x: Tensor | ops.UnscaledRows, batch, cache: CacheView, writes_cache: bool = True,
+    def takes_split(self, tokens: int, batch, cache: CacheView, writes_cache: bool = True) -> bool:
+        if self.general or not writes_cache or self.ctx.dtype != torch.float32 or not ops.takes_split(tokens, self.qkv_weight):
+            return False
+        rotary = self.position.rotary()
+        return not self._single_tokens_only(batch, tokens, cache, 0 if rotary is None else rotary[1])
+
+    def forward(self, x: Tensor | ops.UnscaledRows | ops.SplitRows, batch, cache: CacheView, writes_cache: bool = True,
                 stream: Tensor | None = None, product: bool = False) -> Tensor | ops.UpdateProduct | None:
         rotary = self.position.rotary()
         inv_freq, rotary_dim = rotary if rotary is not None else (None, 0)

@@ -306,6 +306,10 @@ class Mixer(Part):
         """Whether ``forward`` takes, for this step, rows whose norm left its factors out (``ops.UnscaledRows``)."""
         return False
 
+    def takes_split(self, tokens: int, batch, cache: CacheView | None, writes_cache: bool = True) -> bool:
+        """Whether ``forward`` takes, for this step, rows with their parts (``ops.SplitRows``)."""
+        return False
+
     def joint_ends(self) -> JointEnds | None:
         """The part's outer matrices, if it can run between products that it shares with others (``forward_joint``)."""
         return None
@@ -332,6 +336,9 @@ class FeedForward(Part):
     takes_extra = False    # True: ``forward`` takes ``extra=``, an update of the same tokens that joins its own
 
     def takes_unscaled(self, tokens: int) -> bool:
+        return False       # as for a mixer
+
+    def takes_split(self, tokens: int) -> bool:
         return False       # as for a mixer
 
     def joint_ends(self) -> JointEnds | None:

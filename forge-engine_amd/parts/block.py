@@ -21,17 +21,17 @@ class PreNormBlock(Block):
     NORMS = ("input", "post_mixer")
 
     def forward(self, residual: Residual, batch, cache: CacheView | None, writes_cache: bool = True) -> None:
-        x = self._normed("input", residual, lambda rows: self.mixer.takes_unscaled(rows, batch, cache, writes_cache))
+        x = self._normed("input", residual, self.mixer, batch, cache, writes_cache)
         residual.add(self.mixer.forward(x, batch, cache, writes_cache, **self._ways(self.mixer, residual)))
         if self.feed_forward is None:
             return
-        y = self._normed("post_mixer", residual, self.feed_forward.takes_unscaled)
+        y = self._normed("post_mixer", residual, self.feed_forward)
         residual.add(self.feed_forward.forward(y, batch, **self._ways(self.feed_forward, residual)))
 
-    def _normed(self, role: str, residual: Residual, takes_unscaled) -> Tensor:
-        norm = self.norms[role]
+    def _normed(self, role: str, residual: Residual, part, *step) -> Tensor:
+        norm, rows = self.norms[role], residual.h.shape[0]
         if getattr(norm, "leaves_factors", False):
-            return norm.forward(residual, unscaled=takes_unscaled(residual.h.shape[0]))
+            return norm.forward(residual, unscaled=part.takes_unscaled(rows, *step), split=part.takes_split(rows, *step))
         return norm.forward(residual)
 
     @staticmethod

@@ -56,9 +56,16 @@ class SwiGLU(FeedForward):
     def takes_unscaled(self, tokens: int) -> bool:
         return self.gate_up_weight.dtype == self.ctx.dtype and ops.unscaled_swiglu(tokens, self.gate_up_weight)
 
-    def forward(self, x: Tensor | ops.UnscaledRows, batch=None, stream: Tensor | None = None, product: bool = False) -> Tensor | ops.UpdateProduct | None:
-        act = ops.linear_swiglu(x, self.gate_up_weight, self.activation)
-        if product and ops.update_norm_pays(act, self.down_weight):
+    def takes_split(self, tokens: int) -> bool:
+        return self.ctx.dtype == torch.float32 and ops.takes_split(tokens, self.gate_up_weight)
+
+    def forward(self, x: Tensor | ops.UnscaledRows | ops.SplitRows, batch=None, stream: Tensor | None = None,
+                product: bool = False) -> Tensor | ops.UpdateProduct | None:
+        if self.ctx.dtype == torch.float32 and ops.takes_split(x.shape[0], self.down_weight, update=True):
+            act = ops.linear_swiglu(x, self.gate_up_weight, self.activation, split=True)
+        else:
+            act = ops.linear_swiglu(x, self.gate_up_weight, self.activation)
+        if product and not isinstance(act, ops.SplitRows) and ops.update_norm_pays(act, self.down_weight):
             return ops.UpdateProduct(act, self.down_weight)
         return ops.linear_update(act, self.down_weight, stream=stream)   # the update stays float32 for the residual sum
 

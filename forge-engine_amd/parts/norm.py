@@ -39,9 +39,10 @@ class RMSNorm(Norm):
 
     leaves_factors = True
 
-    def forward(self, residual: Residual, rows: Tensor | None = None, unscaled: bool = False) -> Tensor | ops.UnscaledRows:
+    def forward(self, residual: Residual, rows: Tensor | None = None, unscaled: bool = False,
+                split: bool = False) -> Tensor | ops.UnscaledRows | ops.SplitRows:
         """``unscaled``: who reads the rows can multiply by the norm's factors itself, so a pending product may be added and
-        normed in one launch up to those."""
+        normed in one launch up to those.  ``split``: who reads float32 rows takes them with their parts."""
         if unscaled and rows is None:
             product = residual.take_product()
             if product is not None:
@@ -60,6 +61,11 @@ class RMSNorm(Norm):
             return ops.add_rmsnorm(h, residual.pending, self.weight, self.eps, out, rows=rows, store_sum=False,
                                    other=residual.pending_other, shift=residual.pending_bias)
         update, other, shift = residual.take_joined()
+        if split and (update is None or update.dtype == torch.float32) and all(
+                t is None or t.data_ptr() % 16 == 0 for t in (residual.h, update, other, shift, self.weight)):
+            x = ops.SplitRows.empty(residual.h.shape[0], self.size, residual.h.device)
+            ops.add_rmsnorm(residual.h, update, self.weight, self.eps, x.rows, other=other, shift=shift, planes=x.planes)
+            return x
         out = torch.empty((residual.h.shape[0], self.size), dtype=self.ctx.dtype, device=residual.h.device)
         return ops.add_rmsnorm(residual.h, update, self.weight, self.eps, out, other=other, shift=shift)
 

@@ -18,7 +18,8 @@
 // 26.7 -> 24.1, at 256 54 -> 42 (the matrix library and the gate kernel); q/k/v of 6,144 x 2,560 at 256 rows
 // 21 -> 15; down projection of 2,560 x 9,728 at 64 / 256 / 512 rows 14.6 -> 12, 25.5 -> 22, 48 -> 32; gate/up of
 // 3,072 x 1,024 at 384 rows 18.0 -> 13.5.  Starting the blocks' walks over K at different places changes nothing (no
-// memory channel is hot), nor do four stages instead of three.  From 1,500 rows on the matrix library is ahead.
+// memory channel is hot), nor do four stages instead of three, nor loads that go out one by one between the MFMAs; without loads that product
+// takes 25 of its 41.5 us, with lines that the L2 holds 34.  From 1,500 rows on tiles of 256 x 256 (gemm_big.hip) and the matrix library are ahead.
 //
 // Up to 16 rows of x, tiles of 16 rows with one fragment a wave: the weight's bytes are nearly all of the tile's, so the widths
 // (16 to 80 weight rows) only choose how evenly the CUs share them, and 8 to 12 stages keep 64 KB and more of a CU's share in
@@ -56,7 +57,7 @@ constexpr int SQUARES = 256, SQUARES_PITCH = SQUARES * 4 + 16;      // bytes fro
 // the bfloat16 ending and a launch of the activation behind it (8 rows of 2,048 through 4,096 in a captured graph:
 // 6.6 -> 5.0 us).
 // With a gated ending a fragment of sixteen weight rows is eight gate rows and the eight up rows of the same columns.
-template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END, bool SCALED>
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, int END, bool SCALED, bool ONCE>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
     long long ldw, long long ldo, int tiles_m, int tiles_n, int parts, int steps_per_part, long long part_stride,
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
   // save (us, written out -> fetched again: gate/up of 512 columns, K = 2,048 at 25 rows 6.95 -> 6.58, 768 of 2,560 at 53 8.09 -> 7.59, of K =
   // 12,288 27.5 -> 27.0; every other tile 1 to 7 % the other way).
   constexpr bool REFETCH = MI == 1 && NI == 2 && WM == 2 && WN == 1;
-  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, false, REFETCH>(lds, row_of, first, last, K, acc)) return;
+  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, false, REFETCH>(lds, row_of, first, last, K, acc, std::integral_constant<bool, ONCE>())) return;
   if constexpr (SCALED) {
     // Lane (r, q) adds up a quarter of row r's squares.  A wave's loads arrive in order, so its rows were there before its first
     // step of K, and behind that step's barrier everyone's.
@@ -161,14 +162,16 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
                        long long part_stride, GateAct act, hipStream_t stream, RowFactors factors = {}) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, COLUMNS = END == END_GATED || END == END_BOUNDED ? BN / 2 : BN;
   const size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? (M <= 8 ? 8 : 16) * SQUARES_PITCH : 0);
-  static std::atomic<bool> raised{false};
-  auto kernel = gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED>;
   static_assert(!SCALED || lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + 16 * SQUARES_PITCH <= 160 * 1024, "LDS of a CU");
-  const int limit_raised = lds_tile::raise_lds_limit(
-      (const void*)kernel, lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? 16 * SQUARES_PITCH : 0), &raised);
-  if (limit_raised != FE_OK) return limit_raised;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + COLUMNS - 1) / COLUMNS;
   if (tiles_m * tiles_n * parts > 0x7fffffffLL) return FE_BAD_ARGUMENT;
+  // one tile of x: no block reads another's weight rows (an instance of its own: asked at every load it cost prompts of 361 rows .3 %)
+  static std::atomic<bool> raised[2];
+  const bool once = tiles_m == 1;
+  auto kernel = once ? gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, true> : gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, SCALED>;
+  const int limit_raised = lds_tile::raise_lds_limit(
+      (const void*)kernel, lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? 16 * SQUARES_PITCH : 0), &raised[once]);
+  if (limit_raised != FE_OK) return limit_raised;
   const int steps = K / KSTEP, per_part = (steps + parts - 1) / parts;
   kernel<<<(unsigned)(tiles_m * tiles_n * parts), 64 * WM * WN * KG, bytes, stream>>>(
       (const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldw, ldo, (int)tiles_m, (int)tiles_n, parts, per_part, part_stride,

@@ -23,6 +23,14 @@ __device__ __forceinline__ void load_to_lds(const void* global, unsigned int at)
   asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off\n s_mov_b32 m0, %0"
                : "=&s"(m0) : "v"(global), "s"(at) : "memory");
 }
+// The same for lines that no other block reads (and this one not again): they pass the caches without staying there, which leaves a CU more
+// of the lines that its L1 waits for (8 rows x 19,456 x 2,560 19.5 -> 18.6 us, x 2,560 x 9,728 10.7 -> 10.0; where two blocks share a weight
+// row it is the wrong way: 250 rows 41.3 -> 46.4).
+__device__ __forceinline__ void load_to_lds_once(const void* global, unsigned int at) {
+  unsigned int m0;
+  asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off nt\n s_mov_b32 m0, %0"
+               : "=&s"(m0) : "v"(global), "s"(at) : "memory");
+}
 // wait until at most PENDING of this wave's loads are outstanding (PENDING < 64; loads of the compiler's in between only make it longer)
 template <int PENDING>
 __device__ __forceinline__ void wait_loads() {
@@ -52,7 +60,8 @@ struct Shape {
 // Fills acc[i][j] of lane (r = lane % 16, q = lane / 16) of wave (wm, wn) with the products of row 16 (MI wm + i) + r of the first
 // operand and rows 16 (NI wn + j) + 4 q .. + 3 of the second, over 64-steps [first, last) of K (a multiple of 64, or, with
 // HALF_END, of 32).  row_of(j): where row j of the tile begins, the first operand's BM rows, then the second's BN.  Returns
-// whether this wave holds the sums (those of group 0 do); every thread of the block must call it.
+// whether this wave holds the sums (those of group 0 do); every thread of the block must call it.  once (a bool or a constant): no other
+// block reads the rows of the second operand.
 //
 // LDS holds a step of a tile as [row][8 chunks of 16 bytes], chunk c of row j at position c ^ (j % 8): the lanes that a 16-byte
 // read serves in one cycle then hit different bank groups (no conflicts counted).  Both operands go there straight from memory
@@ -63,8 +72,8 @@ struct Shape {
 // 4,245; counting the way down at run time, a chain of branches a step, cost more than it saved (1,058 at 1 request).  REFETCH: they
 // do fetch the last step again, in a walk of half the instructions, for a tile whose short walks are over before the written out steps
 // have been fetched (gemm_lds.h).
-template <int MI, int NI, int WM, int WN, int KG, int STAGES, bool HALF_END, bool REFETCH = false, typename RowOf>
-__device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, int last, int K, floatx4 (&acc)[MI][NI]) {
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, bool HALF_END, bool REFETCH = false, typename Once = std::false_type, typename RowOf>
+__device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, int last, int K, floatx4 (&acc)[MI][NI], Once once = {}) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, WAVES = WM * WN * KG, T = 2 / KG;
   constexpr int GROUPS = (BM + BN) / 8, LOADS = GROUPS / WAVES, MORE = GROUPS % WAVES;   // groups of eight rows: one load of a wave each
   constexpr int STAGE = (BM + BN) * 8;              // 16-byte units of a stage
@@ -78,9 +87,13 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
   auto load = [&](int step, int stage) {
     const int k0 = (REFETCH ? min(step, last - 1) : step) * KSTEP;
     const int at = k0 + (HALF_END && k0 + KSTEP > K ? my_chunk & 3 : my_chunk) * 8;
+    auto load_one = [&](int i) {
+      if (once && (wave + WAVES * i) * 8 >= BM) load_to_lds_once(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
+      else load_to_lds(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
+    };
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_to_lds(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
-    if (MORE > 0 && wave < MORE) load_to_lds(from[LOADS] + at, base + (stage * STAGE + (wave + WAVES * LOADS) * 64) * 16);
+    for (int i = 0; i < LOADS; ++i) load_one(i);
+    if (MORE > 0 && wave < MORE) load_one(LOADS);
   };
   const int r = lane & 15, q = lane >> 4, group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
   const uintx4* x_at = lds + (wm * 16 * MI + r) * 8;

@@ -458,7 +458,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void moe_lds_kernel(
     return w_expert + (size_t)min(n0 + j, N - 1) * K;
   };
   floatx4 acc[MI][NI];
-  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, true>(lds, row_of, 0, (K + lds_tile::KSTEP - 1) / lds_tile::KSTEP, K, acc)) return;
+  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, true>(lds, row_of, 0, (K + lds_tile::KSTEP - 1) / lds_tile::KSTEP, K, acc,
+                                                             offsets[expert + 1] - offsets[expert] <= TILE_ROWS)) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4, wm = wave % WM, wn = wave / WM;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {

@@ -18,7 +18,8 @@
 //   * softmax statistics per query row in float32 (a row's keys sit in four
 //     lanes: two shuffles), base-2 exponent with the scale folded in;
 //   * output transposed, O^T = V^T P^T: A = 16 dims x 32 keys from the value
-//     pages, which are stored transposed ([D][slot]) for this, B = P^T.
+//     pages, which are stored transposed ([D][slot]) for this, B = P^T.  The values are loaded past the caches (64 sequences of 130 to
+//     2,000 keys 59.0 -> 53.7 us, 8 of 1,025 13.2 -> 12.7, two of 30,000 and 20,000 43.7 -> 40.8; the keys as well: 54.3, 13.0, 41.7).
 // Exactness: scores, max, sum and the weighted value sum are float32; P is
 // rounded to bfloat16 for the second product; one rounding at the final store.
 //
@@ -31,6 +32,7 @@
 // holds the same bits whichever kernel wrote them.
 #include "common.h"
 #include "rope_math.h"
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
@@ -180,7 +182,7 @@ __device__ __forceinline__ bool find_run(const int* cu_q, const int* ctx_len, in
 // (1, or a head's width), rows `stride` apart; no gate: null.  The output is rounded before and after, as by a launch of its own
 // behind this one, whose bits these are (8 tokens of 16 heads of 128
 // behind 300 keys in a captured graph: 10.2 -> 8.5 us).
-struct OutGate {
+struct OutGate : Prepare {
   const bf16_t* gate;
   size_t stride;
   int share;
@@ -194,15 +196,16 @@ struct OutGate {
 
 // MODE 0: finished queries; 1: PREPARE from the projection's bfloat16 output; 2: PREPARE from its
 // float32 partial sums.
-template <int D, int MODE, bool CAP = false, int DIST = 0>
+// GATED: MODE 0 alone, with an OutGate in the place of Prepare (an argument more and a branch at the stores cost the others .1 us a launch)
+template <int D, int MODE, bool CAP = false, int DIST = 0, bool GATED = false>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     const bf16_t* __restrict__ q, long long q_stride, const bf16_t* key_pages,
     const bf16_t* value_pages, bf16_t* __restrict__ out, long long out_stride,
     float* part_o, float* part_ml, int* __restrict__ counters, const int* __restrict__ cu_q,
     const int* __restrict__ ctx_len, const int* __restrict__ block_table, int table_stride,
     int kv_heads, int groups, int block_shift, int num_blocks, int window, float scale_log2,
-    Prepare prep, int chunk, const float* __restrict__ sink, float cap_ratio, const float* __restrict__ slopes,
-    int bias_span, int num_seqs, int more, OutGate gate) {
+    std::conditional_t<GATED, OutGate, Prepare> prep, int chunk, const float* __restrict__ sink, float cap_ratio, const float* __restrict__ slopes,
+    int bias_span, int num_seqs, int more) {
   constexpr bool PREPARE = MODE != 0, FROM_SUMS = MODE == 2;
   const int block_size = 1 << block_shift, block_mask = block_size - 1;
   constexpr int KC = D / 32;        // MFMA k-steps over the head dim (scores)
@@ -351,7 +354,8 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     const bf16_t* vbase = value_pages + ((((size_t)vpage * kv_heads + hk) * D) << block_shift) + (vkey & block_mask);
     uintx4 va[DT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t) va[t] = *(const uintx4*)(vbase + ((size_t)(t * 16 + lr) << block_shift));
+    for (int t = 0; t < DT; ++t)      // (an instruction takes whole lines, once: past the caches; a line of keys takes two instructions)
+      va[t] = __builtin_nontemporal_load((const uintx4*)(vbase + ((size_t)(t * 16 + lr) << block_shift)));
     __builtin_amdgcn_sched_barrier(0);
     fetch_keys(b + WAVES, checked(knext_raw, (b + WAVES) * KEYS + krow), knext);
     vraw = raw_page((b + 2 * WAVES) * KEYS + 8 * lq);
@@ -635,7 +639,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       // a sink per query head: exp(sink) joins the denominator, with no key and no value
       if (sink) l += __builtin_amdgcn_exp2f(sink[hk * groups + g] * 1.4426950408889634f - m_tot);
       bf16_t y = float_to_bf16(l > 0.f ? ov / l : 0.f);
-      if (!PREPARE && gate.gate) y = gate.times(y, gate.at(q0, (hk * groups + g) * D + d));
+      if constexpr (GATED) y = prep.times(y, prep.at(q0, (hk * groups + g) * D + d));
       out[(size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d] = y;
     } else {
       const size_t slot = first_part + split;
@@ -666,11 +670,13 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   // a thread's first two gates come in the meantime
   float g0 = 0.f, g1 = 0.f;
   auto load_gates = [&](int e) {
-    const int g = e / D, d = e - g * D;
-    g0 = gate.at(q0, (hk * groups + g) * D + d);
-    g1 = gate.at(q0, (hk * groups + g) * D + d + 1);
+    if constexpr (GATED) {
+      const int g = e / D, d = e - g * D;
+      g0 = prep.at(q0, (hk * groups + g) * D + d);
+      g1 = prep.at(q0, (hk * groups + g) * D + d + 1);
+    }
   };
-  if (!PREPARE && gate.gate && 2 * tid < groups * D) load_gates(2 * tid);
+  if (GATED && 2 * tid < groups * D) load_gates(2 * tid);
   __shared__ int is_last;
   __builtin_amdgcn_s_waitcnt((0x0) | (0x7 << 4) | (0xF << 8));    // vmcnt(0): this wave's stores have been acknowledged
   __syncthreads();
@@ -696,9 +702,9 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
       if (splits <= 4) y = merge_few<4>(part_o, part_ml, first_part, splits, groups, g, D, d, sink2);
       else if (splits <= 8) y = merge_few<8>(part_o, part_ml, first_part, splits, groups, g, D, d, sink2);
       else y = merge_few<16>(part_o, part_ml, first_part, splits, groups, g, D, d, sink2);
-      if (!PREPARE && gate.gate) {
+      if constexpr (GATED) {
         if (e != 2 * tid) load_gates(e);
-        y = gate.times(y, g0, g1);
+        y = prep.times(y, g0, g1);
       }
       *dst = y;
     }
@@ -738,9 +744,9 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     if (sink) l_tot += __builtin_amdgcn_exp2f(sink[hk * groups + g] * 1.4426950408889634f - m_tot);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     unsigned int y = (unsigned int)float_to_bf16(ov0 * inv) | ((unsigned int)float_to_bf16(ov1 * inv) << 16);
-    if (!PREPARE && gate.gate) {
+    if constexpr (GATED) {
       if (e != 2 * tid) load_gates(e);
-      y = gate.times(y, g0, g1);
+      y = prep.times(y, g0, g1);
     }
     *(unsigned int*)(out + (size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d) = y;
   }
@@ -753,9 +759,9 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
                          int num_seqs, int kv_heads, int groups, int head_dim, int block_size,
                          int num_blocks, int window, float scale, int splits, const Prepare* prep,
                          int chunk, const float* sink, hipStream_t stream, float softcap = 0.f, const float* slopes = nullptr,
-                         int bias_span = 0, OutGate gate = {nullptr, 0, 1, 1.f}) {
+                         int bias_span = 0, const OutGate* gate = nullptr) {
   if (num_seqs <= 0) return FE_OK;
-  if (gate.gate && (prep || gate.share < 1)) return FE_BAD_ARGUMENT;
+  if (gate && (prep || gate->share < 1)) return FE_BAD_ARGUMENT;
   if (softcap < 0.f || (softcap > 0.f && (prep || !(scale > 0.f)))) return FE_BAD_ARGUMENT;
   if (slopes && (prep || softcap > 0.f)) return FE_BAD_ARGUMENT;
   if (bias_span < 0 || (bias_span > 0 && !slopes)) return FE_BAD_ARGUMENT;
@@ -774,22 +780,20 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
   dim3 grid(more > 0 ? 1 : splits, kv_heads, num_seqs + more);
   const float scale_log2 = scale * 1.4426950408889634f;
   const Prepare none = {nullptr, nullptr, nullptr, 0.f, nullptr, 0, 0};
-#define FE_GO(DD, MODE)                                                                                    \
-  paged_decode_kernel<DD, MODE><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
+#define FE_GO_AS(DD, MODE, CAP, DIST, GATED, EXTRA, RATIO, SLOPES, SPAN)                                            \
+  paged_decode_kernel<DD, MODE, CAP, DIST, GATED><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
       (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, MODE ? *prep : none, chunk, sink, 0.f, nullptr, 0, num_seqs, more, gate)
-#define FE_GO_CAPPED(DD)                                                                                   \
-  paged_decode_kernel<DD, 0, true><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
-      (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, softcap / scale, nullptr, 0, num_seqs, more, gate)
-#define FE_GO_SLOPED(DD)                                                                                   \
-  paged_decode_kernel<DD, 0, false, 1><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
-      (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, 0.f, slopes, 0, num_seqs, more, gate)
-#define FE_GO_TABLE(DD)                                                                                    \
-  paged_decode_kernel<DD, 0, false, 2><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
-      (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
-      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, none, chunk, sink, 0.f, slopes, bias_span, num_seqs, more, gate)
+      table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, EXTRA, chunk, sink, RATIO, SLOPES, SPAN, num_seqs, more)
+#define FE_GO(DD, MODE) FE_GO_AS(DD, MODE, false, 0, false, MODE ? *prep : none, 0.f, nullptr, 0)
+#define FE_GO_FORM(DD, CAP, DIST, RATIO, SLOPES, SPAN)                                \
+  do {                                                                                \
+    if (gate) FE_GO_AS(DD, 0, CAP, DIST, true, *gate, RATIO, SLOPES, SPAN);           \
+    else FE_GO_AS(DD, 0, CAP, DIST, false, none, RATIO, SLOPES, SPAN);                \
+  } while (0)
+#define FE_GO_PLAIN(DD) FE_GO_FORM(DD, false, 0, 0.f, nullptr, 0)
+#define FE_GO_CAPPED(DD) FE_GO_FORM(DD, true, 0, softcap / scale, nullptr, 0)
+#define FE_GO_SLOPED(DD) FE_GO_FORM(DD, false, 1, 0.f, slopes, 0)
+#define FE_GO_TABLE(DD) FE_GO_FORM(DD, false, 2, 0.f, slopes, bias_span)
   if (slopes && bias_span > 0) {
     if (head_dim == 64) FE_GO_TABLE(64);
     else if (head_dim == 128) FE_GO_TABLE(128);
@@ -811,11 +815,14 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
     else if (head_dim == 128) FE_GO(128, 1);
     else FE_GO(256, 1);
   } else {
-    if (head_dim == 64) FE_GO(64, 0);
-    else if (head_dim == 128) FE_GO(128, 0);
-    else FE_GO(256, 0);
+    if (head_dim == 64) FE_GO_PLAIN(64);
+    else if (head_dim == 128) FE_GO_PLAIN(128);
+    else FE_GO_PLAIN(256);
   }
+#undef FE_GO_AS
 #undef FE_GO
+#undef FE_GO_FORM
+#undef FE_GO_PLAIN
 #undef FE_GO_CAPPED
 #undef FE_GO_SLOPED
 #undef FE_GO_TABLE
@@ -917,11 +924,15 @@ extern "C" int fe_paged_attention_decode_gated(const void* q, long long q_stride
                                                int splits, const void* gate, long long gate_stride, int share, float factor,
                                                hipStream_t stream) {
   const long long width = (long long)kv_heads * groups * head_dim;
+  OutGate how = {};
+  how.gate = (const bf16_t*)gate;
+  how.stride = (size_t)gate_stride;
+  how.share = share;
+  how.factor = factor;
   if (!gate || share < 1 || width % share || gate_stride < width / share) return FE_BAD_ARGUMENT;
   return launch_decode(q, q_stride, key_pages, value_pages, out, out_stride, part_o, part_ml, counters, cu_q,
                        ctx_len, block_table, table_stride, num_seqs, kv_heads, groups, head_dim, block_size,
-                       num_blocks, window, scale, splits, nullptr, chunk, sink, stream, softcap, slopes, span,
-                       {(const bf16_t*)gate, (size_t)gate_stride, share, factor});
+                       num_blocks, window, scale, splits, nullptr, chunk, sink, stream, softcap, slopes, span, &how);
 }
 
 // The same for a batch in which EVERY sequence brings one token, straight from the fused

@@ -75,10 +75,11 @@ class Residual:
 
     @property
     def pending(self) -> Tensor | None:
-        """The update that has not been added yet; one that was left as a product is multiplied out now."""
-        if isinstance(self._pending, ops.UpdateProduct):
-            self._pending = ops.linear_update(self._pending.x, self._pending.weight)
-        return self._pending
+        """The update that has not been added yet; one that was left as a product is multiplied out now.  One that is to be normed
+        first is applied now, and nothing is pending any more: only who asks for it with its norm (``take_normed``) gets it."""
+        if self.pending_norm is not None:
+            self._apply_normed()
+        return self._multiplied_out()
 
     @pending.setter
     def pending(self, update: Tensor | ops.UpdateProduct | None) -> None:
@@ -128,7 +129,7 @@ class Residual:
         """The stream is another tensor from here on (nothing of the old one, or pending on it, counts any more)."""
         self.h = h
         self.in_compute_dtype = None
-        self.pending, self.pending_bias, self.pending_other = update, None, None
+        self.pending, self.pending_bias, self.pending_other, self.pending_norm = update, None, None, None
 
     def add_normed(self, update: Tensor, weight: Tensor, eps: float) -> None:
         """Leave ``h += update * rsqrt(mean(update^2) + eps) * weight`` pending (a norm behind a
@@ -139,11 +140,24 @@ class Residual:
         self.in_compute_dtype = None
         self.pending, self.pending_norm = update, (weight, float(eps))
 
+    def normed(self):
+        """(update, weight, eps) of a pending update that is to be normed; it stays pending."""
+        return (self._multiplied_out(), *self.pending_norm)
+
     def take_normed(self):
-        """(update, weight, eps) of a pending update that is to be normed, which the caller now applies."""
-        update, (weight, eps) = self.pending, self.pending_norm
+        """The same, which the caller now applies."""
+        taken = self.normed()
         self.pending = self.pending_norm = None
-        return update, weight, eps
+        return taken
+
+    def _multiplied_out(self) -> Tensor | None:
+        if isinstance(self._pending, ops.UpdateProduct):
+            self._pending = ops.linear_update(self._pending.x, self._pending.weight)
+        return self._pending
+
+    def _apply_normed(self) -> None:
+        update, weight, eps = self.take_normed()
+        ops.rmsnorm_update(self.h, update, weight, eps, None)
 
     def add_mixed(self, update: Tensor, mix: Tensor, share: Tensor) -> None:
         """Several streams: leave ``x_t <- sum_s mix[s, t] x_s + share[t] * update`` pending."""
@@ -184,13 +198,12 @@ class Residual:
             if self.streams is not None:
                 raise ValueError("a bias on an update needs a model with one residual stream")
             ops.add_rows(self.h, *self.take_joined())
+        elif self.pending_norm is not None:
+            self._apply_normed()
         elif self.pending is not None:
             if self.streams is not None:
                 update, mix, share = self.take_pending()
                 ops.hyper_norm(self.streams, update, mix, share, None, None, None, 0.0, None)
-            elif self.pending_norm is not None:
-                update, weight, eps = self.take_normed()
-                ops.rmsnorm_update(self.h, update, weight, eps, None)
             else:
                 ops.add_rows(self.h, self.pending)
                 self.pending = None

@@ -49,7 +49,7 @@ class RMSNorm(Norm):
                 return ops.update_norm(residual.h, product, self.weight, self.eps)
         if residual.pending_norm is not None:    # a norm behind the sublayer before: both norms in one pass over the row
             if rows is not None:                 # the chosen rows alone; stream and pending update are left as they are
-                update, (weight, eps) = residual.pending, residual.pending_norm
+                update, weight, eps = residual.normed()
                 out = torch.empty((rows.numel(), self.size), dtype=self.ctx.dtype, device=residual.h.device)
                 return ops.rmsnorm_update_norm(residual.h, update, weight, eps, self.weight, self.eps, out, rows=rows)
             update, weight, eps = residual.take_normed()

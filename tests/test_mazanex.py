@@ -134,3 +134,84 @@ def test_greedy_generation_through_the_scheduler(folders, monkeypatch):
     engine.run_until_idle()
     for request_id, prompt in zip(ids, prompts):
         assert list(engine.request(request_id).output_token_ids) == mu.plain_greedy(folders["A"], prompt, 6)
+
+
+class _Matrix:
+    """A mixer or a feed-forward that is one matrix."""
+
+    takes_stream = leaves_product = False
+
+    def __init__(self, g, width):
+        self.matrix = torch.randn(width, width, generator=g)
+
+    def forward(self, x, *step):
+        return x @ self.matrix.T
+
+
+@pytest.mark.parametrize("chosen", [None, [2, 0]])
+@pytest.mark.parametrize("last", ["layer_norm", "rms_norm", "own"])
+@pytest.mark.parametrize("arrangement", ["shifted", "shifted_alone", "sandwich"])
+def test_a_norm_left_pending_reaches_whoever_reads_the_stream(arrangement, last, chosen, monkeypatch):
+    """Two layers that leave their last norm pending, and a last norm that applies it, one that knows none, and one of a program's own, for
+    whole steps and for chosen rows: the formulas in 64 bits."""
+    from types import SimpleNamespace
+
+    from forge_engine_amd.cache.spec import CacheView
+    from forge_engine_amd.parts.base import BuildContext, Residual
+    from forge_engine_amd.parts.block import OutputNormBlock, SandwichNormBlock
+    from forge_engine_amd.parts.norm import LayerNorm, RMSNorm, UpdateRMSNorm
+    kernel_refs.install(monkeypatch)
+    ctx, width, g = BuildContext(torch.device("cpu"), torch.float32), 6, torch.Generator().manual_seed(5)
+
+    class OwnNorm(RMSNorm):
+        leaves_factors = False
+
+        def forward(self, residual, rows=None):
+            if residual.pending is not None:
+                residual.h += residual.pending
+                residual.pending = None
+            z = residual.h if rows is None else residual.h[rows.long()]
+            return kernel_refs._unit(z, self.eps) * self.weight
+
+    def norm(kind, **how):
+        made = kind(ctx, "n", size=width, eps=1e-3, **how)
+        for name, spec in made.param_specs().items():
+            made.set_param(name, 1.0 + 0.3 * torch.randn(spec.shape, generator=g))
+        return made
+
+    def unit(x):
+        return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-3)
+
+    x0 = torch.randn(4, width, generator=g)
+    residual, want = Residual(x0.clone()), x0.double()
+    batch = SimpleNamespace(cu_q=torch.tensor([0, 3, 4], dtype=torch.int32), token_seq=torch.tensor([0, 0, 0, 1], dtype=torch.int32),
+                            state_slots=torch.tensor([1, 0], dtype=torch.int32), num_seqs=2, num_decode=1, carry={})
+    for _ in range(2):
+        mixer, feed_forward = _Matrix(g, width), None if arrangement == "shifted_alone" else _Matrix(g, width)
+        if arrangement == "sandwich":
+            norms = {role: norm(RMSNorm) for role in SandwichNormBlock.NORMS}
+            SandwichNormBlock(ctx, mixer, feed_forward, norms).forward(residual, batch, None)
+            w = {role: n.weight.double() for role, n in norms.items()}
+            want = want + unit((unit(want) * w["input"]) @ mixer.matrix.T.double()) * w["mixer_out"]
+            want = want + unit((unit(want) * w["post_mixer"]) @ feed_forward.matrix.T.double()) * w["ff_out"]
+            continue
+        norms = {role: norm(UpdateRMSNorm) for role in OutputNormBlock.NORMS}
+        block = OutputNormBlock(ctx, mixer, feed_forward, norms, hidden_size=width, token_shift=True)
+        block.set_param(block.name("shift"), torch.rand(width, generator=g))
+        state = torch.zeros(2, width)
+        block.forward(residual, batch, CacheView(states={OutputNormBlock.SHIFT_STATE: state}))
+        before = torch.cat([torch.zeros(1, width), want[:2], torch.zeros(1, width)])
+        mixed = (want + (before - want) * block.shift.double()) @ mixer.matrix.T.double()
+        want = want + unit(mixed) * norms["mixer_out"].weight.double()
+        if feed_forward is not None:
+            want = want + unit(want @ feed_forward.matrix.T.double()) * norms["ff_out"].weight.double()
+    final = norm({"layer_norm": LayerNorm, "rms_norm": RMSNorm, "own": OwnNorm}[last])
+    rows = None if chosen is None else torch.tensor(chosen, dtype=torch.int32)
+    got = final.forward(residual, rows=rows)
+    if last == "layer_norm":
+        centred = want - want.mean(-1, keepdim=True)
+        expected = unit(centred) * final.weight + final.bias
+    else:
+        expected = unit(want) * final.weight
+    assert torch.allclose(got.double(), expected if rows is None else expected[chosen], atol=2e-5)
+    assert torch.allclose(residual.flush().double(), want, atol=2e-5) and residual.pending is None and residual.pending_norm is None

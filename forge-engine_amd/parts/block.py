@@ -98,10 +98,13 @@ class OutputNormBlock(Block):
         self._last_norm("ff_out", residual)
 
     def _last_norm(self, role: str, residual: Residual) -> None:
-        """Layers with a token shift leave their last norm pending: the next one's shift applies it in the same launch, or the model's last norm."""
+        """Layers with a token shift leave their last norm pending: the next one's shift applies it in the same launch, or the model's last norm
+        (a reader of the stream that knows no pending norm finds it applied)."""
         norm = self.norms[role]
         if self.token_shift and getattr(norm, "waits", False):
             update, residual.pending = residual.pending, None
+            if update is None:
+                raise ValueError("a norm of updates needs a pending update")
             residual.add_normed(update, norm.weight, norm.eps)
         else:
             norm.forward(residual)

@@ -215,3 +215,18 @@ def test_a_norm_left_pending_reaches_whoever_reads_the_stream(arrangement, last,
         expected = unit(want) * final.weight
     assert torch.allclose(got.double(), expected if rows is None else expected[chosen], atol=2e-5)
     assert torch.allclose(residual.flush().double(), want, atol=2e-5) and residual.pending is None and residual.pending_norm is None
+
+
+def test_a_norm_of_updates_needs_an_update(monkeypatch):
+    """A part that has added its update into the stream itself leaves nothing to norm: refused, with the norm left pending as without."""
+    from forge_engine_amd.parts.base import BuildContext, Residual
+    from forge_engine_amd.parts.block import OutputNormBlock
+    from forge_engine_amd.parts.norm import UpdateRMSNorm
+    kernel_refs.install(monkeypatch)
+    ctx = BuildContext(torch.device("cpu"), torch.float32)
+    for shift in (True, False):
+        block = OutputNormBlock(ctx, None, None, {"mixer_out": UpdateRMSNorm(ctx, "n", size=4, eps=1e-3)}, hidden_size=4, token_shift=shift)
+        residual = Residual(torch.ones(2, 4))
+        residual.add(None)
+        with pytest.raises(ValueError, match="pending update"):
+            block._last_norm("mixer_out", residual)

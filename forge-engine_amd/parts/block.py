@@ -11,6 +11,7 @@ from ..cache.spec import CacheNeeds, CacheView, FixedState
 from ..kernels import ops
 from ..registry import register_part
 from .base import Block, BuildContext, ParamSpec, Residual
+from .norm import RMSNorm, UpdateRMSNorm
 
 
 class PreNormBlock(Block):
@@ -31,7 +32,10 @@ class PreNormBlock(Block):
     def _normed(self, role: str, residual: Residual, part, *step) -> Tensor:
         norm, rows = self.norms[role], residual.h.shape[0]
         if getattr(norm, "leaves_factors", False):
-            return norm.forward(residual, unscaled=part.takes_unscaled(rows, *step), split=part.takes_split(rows, *step))
+            unscaled = part.takes_unscaled(rows, *step)
+            if type(norm).forward is RMSNorm.forward:       # a norm with a way of its own may know nothing of the parts
+                return norm.forward(residual, unscaled=unscaled, split=part.takes_split(rows, *step))
+            return norm.forward(residual, unscaled=unscaled)
         return norm.forward(residual)
 
     @staticmethod
@@ -101,7 +105,7 @@ class OutputNormBlock(Block):
         """Layers with a token shift leave their last norm pending: the next one's shift applies it in the same launch, or the model's last norm
         (a reader of the stream that knows no pending norm finds it applied)."""
         norm = self.norms[role]
-        if self.token_shift and getattr(norm, "waits", False):
+        if self.token_shift and type(norm).forward is UpdateRMSNorm.forward:
             update, residual.pending = residual.pending, None
             if update is None:
                 raise ValueError("a norm of updates needs a pending update")

@@ -80,7 +80,6 @@ class UpdateRMSNorm(RMSNorm):
     sublayers of such a layer see the stream itself)."""
 
     leaves_factors = False
-    waits = True            # an arrangement may leave the norm pending with its update (``Residual.add_normed``)
 
     def forward(self, residual: Residual, rows: Tensor | None = None) -> Tensor:
         if rows is not None:

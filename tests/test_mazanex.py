@@ -230,3 +230,40 @@ def test_a_norm_of_updates_needs_an_update(monkeypatch):
         residual.add(None)
         with pytest.raises(ValueError, match="pending update"):
             block._last_norm("mixer_out", residual)
+
+
+@pytest.mark.parametrize("knows_parts", [False, True])
+def test_norms_of_their_own_way_are_called_as_before(knows_parts, monkeypatch):
+    """A norm that takes over another's ``forward`` is not asked for rows with their parts, nor is its way left out where it norms updates."""
+    from forge_engine_amd.parts.base import BuildContext, FeedForward, Residual
+    from forge_engine_amd.parts.block import OutputNormBlock, PreNormBlock
+    from forge_engine_amd.parts.norm import RMSNorm, UpdateRMSNorm
+    kernel_refs.install(monkeypatch)
+    ctx, asked = BuildContext(torch.device("cpu"), torch.float32), []
+
+    class Before(RMSNorm):
+        if not knows_parts:
+            def forward(self, residual, rows=None, unscaled=False):
+                asked.append(unscaled)
+                return super().forward(residual, rows)
+
+    class Takes(FeedForward):
+        def takes_split(self, tokens):
+            return True
+
+    monkeypatch.setattr(RMSNorm, "forward", RMSNorm.forward if not knows_parts else lambda self, residual, rows=None, unscaled=False, split=False: asked.append(split))
+    norm = Before(ctx, "n", size=4, eps=1e-3)
+    norm.weight = torch.ones(4)
+    block = PreNormBlock(ctx, None, Takes(ctx, "f"), {"input": norm})
+    block._normed("input", Residual(torch.ones(2, 4)), block.feed_forward)
+    assert asked == [knows_parts]
+
+    class Doubled(UpdateRMSNorm):
+        def forward(self, residual, rows=None):
+            residual.pending = residual.pending * 2.0
+            residual.flush()
+
+    residual = Residual(torch.ones(2, 4))
+    residual.add(torch.ones(2, 4))
+    OutputNormBlock(ctx, None, None, {"mixer_out": Doubled(ctx, "n", size=4, eps=1e-3)}, hidden_size=4, token_shift=True)._last_norm("mixer_out", residual)
+    assert torch.equal(residual.flush(), torch.full((2, 4), 3.0))

@@ -53,6 +53,14 @@ struct RowFactors {
 };
 constexpr int SQUARES = 256, SQUARES_PITCH = SQUARES * 4 + 16;      // bytes from row to row in LDS: sixteen rows in different banks
 
+// The tile of 32 x 32, of which a CU holds two: its last ten steps written out cost walks of 16 to 48 steps more than the requests that they
+// save (us, written out -> fetched again: gate/up of 512 columns, K = 2,048 at 25 rows 6.95 -> 6.58, 768 of 2,560 at 53 8.09 -> 7.59, of K =
+// 12,288 27.5 -> 27.0; every other tile 1 to 7 % the other way).
+template <int MI, int NI, int WM, int WN>
+constexpr bool refetches() {
+  return MI == 1 && NI == 2 && WM == 2 && WN == 1;
+}
+
 // END_BOUNDED: `gate_bounded` of gate and up, both rounded to bfloat16 first, with the limit in act.cubic and alpha in act.linear: the bits of
 // the bfloat16 ending and a launch of the activation behind it (8 rows of 2,048 through 4,096 in a captured graph:
 // 6.6 -> 5.0 us).
@@ -92,11 +100,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_lds_kernel(
       lds_tile::load_to_lds(factors.squares + m * SQUARES + lane * 4, base + STAGE_BYTES + m * SQUARES_PITCH);
   }
   floatx4 acc[MI][NI];
-  // The tile of 32 x 32, of which a CU holds two: its last ten steps written out cost walks of 16 to 48 steps more than the requests that they
-  // save (us, written out -> fetched again: gate/up of 512 columns, K = 2,048 at 25 rows 6.95 -> 6.58, 768 of 2,560 at 53 8.09 -> 7.59, of K =
-  // 12,288 27.5 -> 27.0; every other tile 1 to 7 % the other way).
-  constexpr bool REFETCH = MI == 1 && NI == 2 && WM == 2 && WN == 1;
-  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, false, REFETCH>(lds, row_of, first, last, K, acc, std::integral_constant<bool, ONCE>())) return;
+  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, false, refetches<MI, NI, WM, WN>()>(lds, row_of, first, last, K, acc,
+                                                                                         std::integral_constant<bool, ONCE>())) return;
   if constexpr (SCALED) {
     // Lane (r, q) adds up a quarter of row r's squares.  A wave's loads arrive in order, so its rows were there before its first
     // step of K, and behind that step's barrier everyone's.
@@ -165,10 +170,15 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
   static_assert(!SCALED || lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + 16 * SQUARES_PITCH <= 160 * 1024, "LDS of a CU");
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + COLUMNS - 1) / COLUMNS;
   if (tiles_m * tiles_n * parts > 0x7fffffffLL) return FE_BAD_ARGUMENT;
-  // one tile of x: no block reads another's weight rows (an instance of its own: asked at every load it cost prompts of 361 rows .3 %)
+  // one tile of x: no block reads another's weight rows (an instance of its own: asked at every load it cost prompts of 361 rows .3 %), and
+  // unless the tile fetches a walk's last step again, neither does this one.  (Its walks of eight steps request eighteen: with those past the
+  // caches decode steps of 17 to 32 requests took, us, 0.6B 1,114 -> 1,139 and 1,156 -> 1,188, 1.7B 1,591 -> 1,607; as it is 1,118, 1,164 and 1,581.
+  // Prompts of so many tokens alone, 0.6B, gained 30 of 1,155 by it: the weights then left the head's rows in the last cache.)
+  constexpr bool AGAIN = refetches<MI, NI, WM, WN>();
+  static_assert(!(SCALED && AGAIN), "rows with factors are one tile of x");
   static std::atomic<bool> raised[2];
-  const bool once = tiles_m == 1;
-  auto kernel = once ? gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, true> : gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, SCALED>;
+  const bool once = tiles_m == 1 && !AGAIN;
+  auto kernel = once ? gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, !AGAIN> : gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, SCALED>;
   const int limit_raised = lds_tile::raise_lds_limit(
       (const void*)kernel, lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? 16 * SQUARES_PITCH : 0), &raised[once]);
   if (limit_raised != FE_OK) return limit_raised;

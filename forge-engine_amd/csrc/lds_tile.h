@@ -74,6 +74,7 @@ struct Shape {
 // have been fetched (gemm_lds.h).
 template <int MI, int NI, int WM, int WN, int KG, int STAGES, bool HALF_END, bool REFETCH = false, typename Once = std::false_type, typename RowOf>
 __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, int last, int K, floatx4 (&acc)[MI][NI], Once once = {}) {
+  static_assert(!(REFETCH && std::is_same_v<Once, std::true_type>), "lines that are fetched again stay in the caches");
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, WAVES = WM * WN * KG, T = 2 / KG;
   constexpr int GROUPS = (BM + BN) / 8, LOADS = GROUPS / WAVES, MORE = GROUPS % WAVES;   // groups of eight rows: one load of a wave each
   constexpr int STAGE = (BM + BN) * 8;              // 16-byte units of a stage

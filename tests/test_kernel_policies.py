@@ -480,3 +480,21 @@ def test_loads_into_lds_have_m0_to_themselves(source, tmp_path):
     uses = [line for line in lines if re.search(r"\bm0\b", line)]
     assert uses and all(line.startswith("s_mov_b32 m0, s") for line in uses)
     assert not any(line.startswith(("scratch_", "buffer_store", "buffer_load")) for line in lines)
+
+
+def test_lines_that_are_fetched_again_stay_in_the_caches(tmp_path):
+    """Loads of the products through LDS pass the caches (nt) where a line is read once, in an instance of each tile for one tile of x, and
+    never in the tile that fetches a walk's last step again."""
+    listing = tmp_path / "gemm_wide.s"
+    flags = [flag for flag in build.HIPCC_FLAGS if flag != "-shared"]
+    subprocess.run([build.find_hipcc(), *flags, "-S", "--cuda-device-only", "-o", str(listing), str(build.SOURCE_DIR / "gemm_wide.hip")],
+                   check=True, capture_output=True)
+    kernels = re.findall(r"^(_Z\w*gemm_lds_kernel\w+):(.*?)^\.Lfunc_end", listing.read_text(), re.M | re.S)
+    assert kernels
+    past = {}
+    for name, code in kernels:
+        mi, ni, wm, wn, *_ = (int(v) for v in re.findall(r"Li(\d+)E", name))
+        assert "global_load_lds_dwordx4" in code
+        past.setdefault((mi, ni, wm, wn), set()).add(bool(re.search(r"global_load_lds_dwordx4 .*\bnt\b", code)))
+    assert past.pop((1, 2, 2, 1)) == {False}
+    assert len(past) == 13 and all(kinds == {False, True} for kinds in past.values())

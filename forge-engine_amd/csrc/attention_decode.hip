@@ -18,8 +18,11 @@
 //   * softmax statistics per query row in float32 (a row's keys sit in four
 //     lanes: two shuffles), base-2 exponent with the scale folded in;
 //   * output transposed, O^T = V^T P^T: A = 16 dims x 32 keys from the value
-//     pages, which are stored transposed ([D][slot]) for this, B = P^T.  The values are loaded past the caches (64 sequences of 130 to
-//     2,000 keys 59.0 -> 53.7 us, 8 of 1,025 13.2 -> 12.7, two of 30,000 and 20,000 43.7 -> 40.8; the keys as well: 54.3, 13.0, 41.7).
+//     pages, which are stored transposed ([D][slot]) for this, B = P^T.  In pages of 16 and 32 keys an instruction takes whole lines,
+//     once, and the values are loaded past the caches (64 sequences of 130 to 2,000 keys 59.0 -> 53.7 us, 8 of 1,025 13.2 -> 12.7, two
+//     of 30,000 and 20,000 43.7 -> 40.8; the keys, a line of which takes two instructions, as well: 54.3, 13.0, 41.7).  From 64 on a
+//     dim's row is a line or more, of which two waves take a half each: past the caches they would both fetch it (60 sequences of
+//     1,585 keys 126 -> 142 us, 14 of 14,614 in pages of 128 106 -> 120).
 // Exactness: scores, max, sum and the weighted value sum are float32; P is
 // rounded to bfloat16 for the second product; one rounding at the final store.
 //
@@ -197,7 +200,8 @@ struct OutGate : Prepare {
 // MODE 0: finished queries; 1: PREPARE from the projection's bfloat16 output; 2: PREPARE from its
 // float32 partial sums.
 // GATED: MODE 0 alone, with an OutGate in the place of Prepare (an argument more and a branch at the stores cost the others .1 us a launch)
-template <int D, int MODE, bool CAP = false, int DIST = 0, bool GATED = false>
+// PAST: values are loaded past the caches
+template <int D, int MODE, bool CAP = false, int DIST = 0, bool GATED = false, bool PAST = true>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     const bf16_t* __restrict__ q, long long q_stride, const bf16_t* key_pages,
     const bf16_t* value_pages, bf16_t* __restrict__ out, long long out_stride,
@@ -354,8 +358,11 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
     const bf16_t* vbase = value_pages + ((((size_t)vpage * kv_heads + hk) * D) << block_shift) + (vkey & block_mask);
     uintx4 va[DT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t)      // (an instruction takes whole lines, once: past the caches; a line of keys takes two instructions)
-      va[t] = __builtin_nontemporal_load((const uintx4*)(vbase + ((size_t)(t * 16 + lr) << block_shift)));
+    for (int t = 0; t < DT; ++t) {
+      const uintx4* from = (const uintx4*)(vbase + ((size_t)(t * 16 + lr) << block_shift));
+      if constexpr (PAST) va[t] = __builtin_nontemporal_load(from);
+      else va[t] = *from;
+    }
     __builtin_amdgcn_sched_barrier(0);
     fetch_keys(b + WAVES, checked(knext_raw, (b + WAVES) * KEYS + krow), knext);
     vraw = raw_page((b + 2 * WAVES) * KEYS + 8 * lq);
@@ -780,8 +787,13 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
   dim3 grid(more > 0 ? 1 : splits, kv_heads, num_seqs + more);
   const float scale_log2 = scale * 1.4426950408889634f;
   const Prepare none = {nullptr, nullptr, nullptr, 0.f, nullptr, 0, 0};
-#define FE_GO_AS(DD, MODE, CAP, DIST, GATED, EXTRA, RATIO, SLOPES, SPAN)                                            \
-  paged_decode_kernel<DD, MODE, CAP, DIST, GATED><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
+#define FE_GO_AS(...)                            \
+  do {                                           \
+    if (block_size <= 32) FE_GO_WITH(true, __VA_ARGS__); \
+    else FE_GO_WITH(false, __VA_ARGS__);         \
+  } while (0)
+#define FE_GO_WITH(PAST, DD, MODE, CAP, DIST, GATED, EXTRA, RATIO, SLOPES, SPAN)                                    \
+  paged_decode_kernel<DD, MODE, CAP, DIST, GATED, PAST><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (const bf16_t*)key_pages, \
       (const bf16_t*)value_pages, (bf16_t*)out, out_stride, part_o, part_ml, counters, cu_q, ctx_len, block_table,     \
       table_stride, kv_heads, groups, block_shift, num_blocks, window, scale_log2, EXTRA, chunk, sink, RATIO, SLOPES, SPAN, num_seqs, more)
 #define FE_GO(DD, MODE) FE_GO_AS(DD, MODE, false, 0, false, MODE ? *prep : none, 0.f, nullptr, 0)
@@ -820,6 +832,7 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
     else FE_GO_PLAIN(256);
   }
 #undef FE_GO_AS
+#undef FE_GO_WITH
 #undef FE_GO
 #undef FE_GO_FORM
 #undef FE_GO_PLAIN

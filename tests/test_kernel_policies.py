@@ -498,3 +498,20 @@ def test_lines_that_are_fetched_again_stay_in_the_caches(tmp_path):
         past.setdefault((mi, ni, wm, wn), set()).add(bool(re.search(r"global_load_lds_dwordx4 .*\bnt\b", code)))
     assert past.pop((1, 2, 2, 1)) == {False}
     assert len(past) == 13 and all(kinds == {False, True} for kinds in past.values())
+
+
+def test_values_of_long_pages_stay_in_the_caches(tmp_path):
+    """The decode attention has instances whose values pass the caches, for pages in which an instruction takes whole lines of them, and
+    others whose loads all stay there, for pages in which two waves share a line."""
+    listing = tmp_path / "attention_decode.s"
+    flags = [flag for flag in build.HIPCC_FLAGS if flag != "-shared"]
+    subprocess.run([build.find_hipcc(), *flags, "-S", "--cuda-device-only", "-o", str(listing), str(build.SOURCE_DIR / "attention_decode.hip")],
+                   check=True, capture_output=True)
+    kernels = re.findall(r"^(_Z\w*paged_decode_kernel\w+):(.*?)^\.Lfunc_end", listing.read_text(), re.M | re.S)
+    forms = {}
+    for name, code in kernels:
+        head, past = re.match(r"(.*)Lb([01])EEv", name).groups()
+        loads = len(re.findall(r"global_load_dwordx4 .*\bnt\b", code))
+        assert loads == (2 * int(re.search(r"ILi(\d+)E", name).group(1)) // 16 if past == "1" else 0)      # the two register sets' steps
+        forms.setdefault(head, set()).add(past)
+    assert forms and all(kinds == {"0", "1"} for kinds in forms.values())

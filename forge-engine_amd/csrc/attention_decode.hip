@@ -768,7 +768,8 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
                          int chunk, const float* sink, hipStream_t stream, float softcap = 0.f, const float* slopes = nullptr,
                          int bias_span = 0, const OutGate* gate = nullptr) {
   if (num_seqs <= 0) return FE_OK;
-  if (gate && (prep || gate->share < 1)) return FE_BAD_ARGUMENT;
+  constexpr int GATED_DIM = 128;      // gates come with heads of up to so many elements
+  if (gate && (prep || gate->share < 1 || head_dim > GATED_DIM)) return FE_BAD_ARGUMENT;
   if (softcap < 0.f || (softcap > 0.f && (prep || !(scale > 0.f)))) return FE_BAD_ARGUMENT;
   if (slopes && (prep || softcap > 0.f)) return FE_BAD_ARGUMENT;
   if (bias_span < 0 || (bias_span > 0 && !slopes)) return FE_BAD_ARGUMENT;
@@ -799,8 +800,9 @@ static int launch_decode(const void* q, long long q_stride, const void* key_page
 #define FE_GO(DD, MODE) FE_GO_AS(DD, MODE, false, 0, false, MODE ? *prep : none, 0.f, nullptr, 0)
 #define FE_GO_FORM(DD, CAP, DIST, RATIO, SLOPES, SPAN)                                \
   do {                                                                                \
-    if (gate) FE_GO_AS(DD, 0, CAP, DIST, true, *gate, RATIO, SLOPES, SPAN);           \
-    else FE_GO_AS(DD, 0, CAP, DIST, false, none, RATIO, SLOPES, SPAN);                \
+    if constexpr (DD <= GATED_DIM)                                                    \
+      if (gate) { FE_GO_AS(DD, 0, CAP, DIST, true, *gate, RATIO, SLOPES, SPAN); break; } \
+    FE_GO_AS(DD, 0, CAP, DIST, false, none, RATIO, SLOPES, SPAN);                     \
   } while (0)
 #define FE_GO_PLAIN(DD) FE_GO_FORM(DD, false, 0, 0.f, nullptr, 0)
 #define FE_GO_CAPPED(DD) FE_GO_FORM(DD, true, 0, softcap / scale, nullptr, 0)
@@ -926,7 +928,7 @@ extern "C" int fe_paged_attention_decode_biased(const void* q, long long q_strid
 }
 
 // Any of the forms above (softcap 0, slopes null and span 0 for the ones without; `slopes` is the table where span > 0), the
-// output times sigmoid(gate) * factor: gate [tokens] rows gate_stride apart, a number for every `share` elements of a row.
+// output times sigmoid(gate) * factor: gate [tokens] rows gate_stride apart, a number for every `share` elements of a row; heads of 64 or 128.
 extern "C" int fe_paged_attention_decode_gated(const void* q, long long q_stride, const void* key_pages,
                                                const void* value_pages, void* out, long long out_stride,
                                                float* part_o, float* part_ml, int* counters, const int* cu_q,

@@ -1618,7 +1618,7 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
     """Attention of every query token of a mixed batch over its paged keys.
 
     ``gate`` (gate, share, factor): the output times sigmoid(gate) * factor, a gate for every ``share`` elements of a row; for
-    steps of single tokens alone (``num_decode`` = ``num_seqs``) of a bfloat16 cache.
+    steps of single tokens alone (``num_decode`` = ``num_seqs``) of a bfloat16 cache with heads of 64 or 128.
 
     ``splits``: key runs of every single token's sequence; ``by_length``: runs by length instead, this many a kv head beyond the
     sequences (at most 64 of them); neither: ``decode_runs``.  Both are for the matrix-core decode kernel; another ignores them.
@@ -1675,8 +1675,8 @@ def paged_attention(q: Tensor, key_pages: Tensor, value_pages: Tensor, out: Tens
     fast_decode = bf16_pages and head_dim in (64, 128, 256) and groups <= 8
     fast_prefill = bf16_pages and head_dim in (64, 128)
     masked = chunk is not None or sink is not None or softcap is not None or slopes is not None or dist_bias is not None
-    if gate is not None and not fast_decode:
-        raise KernelError("a gate is served by the matrix-core decode kernel only")
+    if gate is not None and not (fast_decode and head_dim <= 128):
+        raise KernelError("a gate is served by the matrix-core decode kernel only, for heads of 64 and 128")
     if masked:
         if dist_bias is not None:     # a table of biases by distance, float32 [Hq, span]: entry min(position - j, span - 1) joins the score
             _gpu(dist_bias, "dist_bias", torch.float32)

@@ -221,6 +221,17 @@ def test_gate_in_the_decode_kernel(dim, per_head, contexts, form):
     assert torch.equal(got, want)
 
 
+def test_gate_of_wide_heads_is_for_a_launch_of_its_own():
+    """Heads of 256 have no gated decode kernel: refused before a launch, whatever else the call has."""
+    from forge_engine_amd.kernels import ops
+    q, pages = torch.zeros(2, 512, dtype=torch.bfloat16, device=DEV), torch.zeros(2, 1, 16, 256, dtype=torch.bfloat16, device=DEV)
+    cu, ctx, table = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in ([0, 1, 2], [3, 9], [[0], [1]]))
+    how = dict(num_seqs=2, max_q_len=1, q_heads=2, kv_heads=1, head_dim=256, scale=1.0, num_decode=2, max_ctx=9)
+    for more in ({}, {"softcap": 5.0}, {"slopes": torch.zeros(2, device=DEV)}):
+        with pytest.raises(ops.KernelError, match="heads of 64 and 128"):
+            ops.paged_attention(q, pages, pages.transpose(2, 3).contiguous(), torch.empty_like(q), cu, ctx, table, gate=(q, 1, 1.0), **how, **more)
+
+
 # the smallest, most tokens, experts, pairs and choices, and one of each too many
 @pytest.mark.parametrize("scoring,biased", [("softmax", True), ("sigmoid", False)])
 @pytest.mark.parametrize("tokens,experts,top", [(1, 1, 1), (8, 8, 2), (64, 64, 4), (16, 17, 16), (64, 3, 3), (65, 8, 2), (8, 65, 2), (33, 64, 8)])

@@ -9,6 +9,7 @@ implementation: without a GPU or without the compiled library a call raises.
 from __future__ import annotations
 
 import functools
+import math
 import threading
 from ctypes import c_double, c_float, c_int, c_longlong, c_void_p
 from typing import NamedTuple
@@ -225,10 +226,12 @@ SPLIT_MOST_PARTS = 6
 
 
 # The same with a split ahead, by a launch of its own (csrc/gemm_planes.hip), for more than 64 rows: 16 rows of a, 64 rows of b a block takes, and
-# the microseconds of a round of one block a CU (of the first tile, whose blocks share a CU in pairs, also of two) and of a step of 64 of K in it.
-PLANES_TILES = {(4, 1): (4.0, 0.69, 1.19), (4, 2): (4.9, 1.18, None), (5, 2): (5.7, 1.32, None), (6, 1): (4.3, 0.95, None),
-                (6, 2): (6.3, 1.41, None), (7, 2): (7.1, 1.58, None), (8, 1): (5.0, 1.02, None), (8, 2): (7.3, 1.72, None),
-                (9, 1): (5.3, 1.11, None), (10, 1): (5.5, 1.26, None)}
+# the microseconds of a round of one block a CU (of the first tile, whose blocks share a CU in pairs, also of two) and of a step of 64 of K in it,
+# the weight coming from memory as it does in a model (from the caches a step takes .83 of this: fitted to such times, the picks took one
+# product in ten more than 1.03 of gemm_split's time).
+PLANES_TILES = {(4, 1): (4.1, 0.92, 1.97), (4, 2): (5.4, 1.41, None), (5, 2): (6.0, 1.59, None), (6, 1): (4.5, 1.16, None),
+                (6, 2): (6.3, 1.63, None), (7, 2): (7.0, 1.80, None), (8, 1): (5.1, 1.21, None), (8, 2): (7.3, 1.88, None),
+                (9, 1): (5.5, 1.28, None), (10, 1): (5.6, 1.46, None)}
 
 
 def _split_fits(a: Tensor, b: Tensor) -> bool:
@@ -242,31 +245,45 @@ def _planes_fit(a: Tensor, b: Tensor) -> bool:
     return 6 * a.shape[0] * (a.shape[1] + 63) < 1 << 32 and b.stride(0) < 1 << 22
 
 
-@functools.lru_cache(maxsize=4096)
-def _product_plan(m: int, n: int, k: int, most_parts: int, planes: bool) -> tuple[int | tuple[int, int], int]:
+def _product_plan(m: int, n: int, k: int, most_parts: int, planes: bool, made: bool = False) -> tuple[int | tuple[int, int], int]:
     """(tile, parts of K) for ``gemm_split``: its own, or for more than 64 rows the tile of planes that is predicted to take less, the pass over
-    a and what adds the parts up with it.  Over 2,272 random products of 65 to 1,400 rows (512 to 12,288 weight rows, K 256 to 8,192) the
-    prediction is within 7 % for nine in ten, the pick of a tile the best one, and the 1,437 products that go to planes take 0.80 of the
-    others' time (one in 200 more than 1.03)."""
+    a (``made``: what its maker takes longer to store the planes) and what adds the parts up with it.  Over 1,877 random products of 65 to 1,400
+    rows (256 to 24,576 weight rows, K 256 to 12,800; 45,000 launches) the picks take 0.4 % longer than the best, and those that go to planes
+    0.81 of the others' time (``made``: 0.78), none more than 1.03.
+
+    A plan takes 20 (whole) to 70 us (in parts) to find; a length makes as many tiles as the next multiple of 16, the rows of a fragment, so
+    that is what plans are kept by."""
+    return _product_plan_of(m if m <= SPLIT_MIN_ROWS_F32 else -(-m // 16) * 16, n, k, most_parts, planes, made)
+
+
+@functools.lru_cache(maxsize=4096)
+def _product_plan_of(m: int, n: int, k: int, most_parts: int, planes: bool, made: bool) -> tuple[int | tuple[int, int], int]:
     tile, parts = _split_plan(m, n, k, most_parts)
     if m <= SPLIT_MIN_ROWS_F32 or not planes:
         return tile, parts
-    us, planes_tile, planes_parts = min(
-        (_planes_us(m, n, k, shape, p) + (p - 1) * (m * n * 8 / 4.5e6 + 0.5), shape, p)
-        for shape in PLANES_TILES for p in range(1, max(1, min(most_parts, k // 128)) + 1))
+    us, planes_tile, planes_parts = _planes_plan(m, n, k, most_parts)
+    us += 0.8 if made else 3.8 + 1.9e-6 * m * k
     return (planes_tile, planes_parts) if us < _split_us(m, n, k, tile, parts) else (tile, parts)
 
 
-def _planes_us(m: int, n: int, k: int, shape: tuple[int, int], parts: int) -> float:
-    round_us, step_us, pair_us = PLANES_TILES[shape]
-    tiles, steps = -(-m // (16 * shape[0])) * -(-n // (64 * shape[1])) * parts, -(-(-(-k // 64)) // parts)
-    one, pair = round_us + steps * step_us, round_us + steps * (pair_us or 0.0)
-    if pair_us is None:
-        rounds = -(-tiles // 256) * one
-    else:
-        full, rest = divmod(tiles, 512)
-        rounds = full * pair + (0.0 if rest == 0 else one if rest <= 256 else pair)
-    return 3.6 + 2.2e-6 * m * k + max(rounds, n * k * 4 / 4.5e6)
+def _planes_plan(m: int, n: int, k: int, most_parts: int) -> tuple[float, tuple[int, int] | None, int]:
+    """(us, tile, parts of K): the least of what a launch on planes is predicted to take."""
+    steps_of_k, most = -(-k // 64), max(1, min(most_parts, k // 128))
+    weight_us, part_us = n * k * 4 / 4.5e6, m * n * 8 / 4.5e6 + 0.5
+    best = (math.inf, None, 0)
+    for shape, (round_us, step_us, pair_us) in PLANES_TILES.items():
+        tiles_of_part = -(-m // (16 * shape[0])) * -(-n // (64 * shape[1]))
+        for parts in range(1, most + 1):
+            tiles, steps = tiles_of_part * parts, -(-steps_of_k // parts)
+            us = round_us + steps * step_us
+            if pair_us is None:
+                us *= -(-tiles // 256)
+            elif tiles > 256:
+                us = -(-tiles // 512) * (round_us + steps * pair_us) - (steps * (pair_us - step_us) if 0 < tiles % 512 <= 256 else 0.0)
+            us = max(us, weight_us) + (parts - 1) * part_us
+            if us < best[0]:
+                best = (us, shape, parts)
+    return best
 
 
 @functools.lru_cache(maxsize=4096)
@@ -339,7 +356,7 @@ SPLIT_AHEAD_MAX_K = 8192        # the widest rows that the norm's kernel holds i
 
 
 def takes_split(rows: int, weight: Tensor, update: bool = False) -> bool:
-    """Whether ``linear`` (``linear_update``) takes ``SplitRows`` of so many rows: where it takes planes for their float32 rows."""
+    """Whether ``linear`` (``linear_update``) takes ``SplitRows`` of so many rows: where planes that are there already take the product."""
     if not weight.is_cuda or weight.dtype != torch.float32 or weight.dim() != 2 or rows <= SPLIT_MIN_ROWS_F32:
         return False
     n, k = weight.shape
@@ -347,7 +364,7 @@ def takes_split(rows: int, weight: Tensor, update: bool = False) -> bool:
             or weight.data_ptr() % 16 or 6 * rows * (k + 63) >= 1 << 32):
         return False
     most_parts = SPLIT_MOST_PARTS if update else 1
-    return _split_pays(rows, n, k, most_parts) and isinstance(_product_plan(rows, n, k, most_parts, True)[0], tuple)
+    return _split_pays(rows, n, k, most_parts) and isinstance(_product_plan(rows, n, k, most_parts, True, True)[0], tuple)
 
 
 def gemm_split(a: Tensor | SplitRows, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
@@ -519,7 +536,7 @@ def linear(x: Tensor | UnscaledRows | SplitRows, weight: Tensor, bias: Tensor | 
         if out_dtype not in (None, torch.float32) or not takes_split(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
             raise KernelError("rows with their parts are for the products of planes only")
         y = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=weight.device)
-        return gemm_split(x, weight, 1, _product_plan(x.shape[0], *weight.shape, 1, True)[0], bias, y)
+        return gemm_split(x, weight, 1, _product_plan(x.shape[0], *weight.shape, 1, True, True)[0], bias, y)
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     out_dtype = x.dtype if out_dtype is None else out_dtype
@@ -1190,7 +1207,7 @@ def linear_update(x: Tensor | SplitRows, weight: Tensor, bias: Tensor | None = N
     if isinstance(x, SplitRows):
         if bias is not None or not takes_split(x.shape[0], weight, update=True) or weight.shape[1] != x.shape[1]:
             raise KernelError("rows with their parts are for the products of planes only")
-        tile, parts = _product_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS, True)
+        tile, parts = _product_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS, True, True)
         return gemm_split(x, weight, parts, tile)
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)

@@ -515,3 +515,20 @@ def test_values_of_long_pages_stay_in_the_caches(tmp_path):
         assert loads == (2 * int(re.search(r"ILi(\d+)E", name).group(1)) // 16 if past == "1" else 0)      # the two register sets' steps
         forms.setdefault(head, set()).add(past)
     assert forms and all(kinds == {"0", "1"} for kinds in forms.values())
+
+
+@pytest.mark.parametrize("rows,weight_rows,k,most_parts,split,planes,made", [
+    (768, 1024, 1024, 1, 21.6, 25.9, 20.0), (560, 6976, 512, 1, 38.5, 46.9, None), (403, 1024, 2048, 6, 25.9, 29.6, 23.1), (92, 2560, 2560, 6, 21.1, 24.9, None),
+    (934, 1536, 512, 1, 17.0, 19.9, 14.5), (78, 3828, 3828, 1, 54.9, 63.9, 64.0), (700, 6144, 1024, 1, 68.0, 59.0, 52.0), (700, 2048, 6144, 6, 130.0, 100.0, 96.0)])
+def test_float32_products_of_prompts_take_planes_where_they_were_measured_to_be_faster(rows, weight_rows, k, most_parts, split, planes, made):
+    """us, the weight coming from memory: through gemm_split, through planes with the pass over the rows, and without it."""
+    assert isinstance(ops._product_plan(rows, weight_rows, k, most_parts, True)[0], tuple) == (planes < split)
+    assert made is None or isinstance(ops._product_plan(rows, weight_rows, k, most_parts, True, made=True)[0], tuple) == (made < split)
+
+
+def test_float32_plans_are_shared_by_the_lengths_of_a_fragment_of_rows():
+    before = ops._product_plan_of.cache_info().misses
+    for rows in range(497, 513):
+        assert ops._product_plan(rows, 2056, 4104, 6, True) == ops._product_plan(512, 2056, 4104, 6, True)
+    assert ops._product_plan_of.cache_info().misses - before == 1
+    assert ops._product_plan(64, 2056, 4104, 6, True) == ops._split_plan(64, 2056, 4104, 6) and ops._product_plan(512, 2056, 4104, 6, False) == ops._split_plan(512, 2056, 4104, 6)

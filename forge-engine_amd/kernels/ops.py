@@ -248,8 +248,9 @@ def _planes_fit(a: Tensor, b: Tensor) -> bool:
 def _product_plan(m: int, n: int, k: int, most_parts: int, planes: bool, made: bool = False) -> tuple[int | tuple[int, int], int]:
     """(tile, parts of K) for ``gemm_split``: its own, or for more than 64 rows the tile of planes that is predicted to take less, the pass over
     a (``made``: what its maker takes longer to store the planes) and what adds the parts up with it.  Over 1,877 random products of 65 to 1,400
-    rows (256 to 24,576 weight rows, K 256 to 12,800; 45,000 launches) the picks take 0.4 % longer than the best, and those that go to planes
-    0.81 of the others' time (``made``: 0.78), none more than 1.03.
+    rows (256 to 24,576 weight rows, K 256 to 12,800; 45,000 launches) the picks take 0.3 % longer than the best, and those that go to planes
+    0.81 of the others' time (``made``: 0.78), seven of 2,459 more than 1.03.  Among the planes are only those whose sums are as exact as the ones
+    of ``gemm_split``'s own plan (``_sum_error``).
 
     A plan takes 20 (whole) to 70 us (in parts) to find; a length makes as many tiles as the next multiple of 16, the rows of a fragment, so
     that is what plans are kept by."""
@@ -261,26 +262,42 @@ def _product_plan_of(m: int, n: int, k: int, most_parts: int, planes: bool, made
     tile, parts = _split_plan(m, n, k, most_parts)
     if m <= SPLIT_MIN_ROWS_F32 or not planes:
         return tile, parts
-    us, planes_tile, planes_parts = _planes_plan(m, n, k, most_parts)
-    us += 0.8 if made else 3.8 + 1.9e-6 * m * k
-    return (planes_tile, planes_parts) if us < _split_us(m, n, k, tile, parts) else (tile, parts)
+    error = 1.02 * _sum_error("split gathered" if SPLIT_TILES[tile][2] == 128 else "split", k / parts)
+    found = _planes_plan(m, n, k, most_parts, error)
+    us = (0.8 if made else 3.8 + 1.9e-6 * m * k) + found[0]
+    return found[1:] if us < 1.03 * _split_us(m, n, k, tile, parts) else (tile, parts)      # (where they take the same, the more exact one)
 
 
-def _planes_plan(m: int, n: int, k: int, most_parts: int) -> tuple[float, tuple[int, int] | None, int]:
-    """(us, tile, parts of K): the least of what a launch on planes is predicted to take."""
+def _sum_error(kind: str, products: float) -> float:
+    """What a float32 sum of so many products is off by against 64 bits, in 1e-7 of the sums' root mean square (parts, which are added up in
+    float32, by a part's): within 5 % for K of 1,024 to 6,144 in one to six parts.  What goes into the whole every four steps stays
+    near the rounding of the result, and so do short sums; long ones of the tiles that have no registers for that do not (K = 2,048, 6,144 in
+    one part: 0.9 and 1.2 gathered, 1.9 and 3.4 of planes, 2.1 and 3.8 of gemm_split's larger tiles)."""
+    long = products / 1024
+    if kind == "planes gathered":
+        return 0.80 + 0.06 * long
+    if kind == "split gathered":
+        return 0.89 + 0.03 * long
+    return (1.13 if kind == "split" else 1.0) * math.sqrt(0.15 + 1.62 * long + 0.04 * long * long)
+
+
+def _planes_plan(m: int, n: int, k: int, most_parts: int, error: float) -> tuple[float, tuple[int, int] | None, int]:
+    """(us, tile, parts of K): the least of what a launch on planes is predicted to take whose sums are off by at most ``error``."""
     steps_of_k, most = -(-k // 64), max(1, min(most_parts, k // 128))
     weight_us, part_us = n * k * 4 / 4.5e6, m * n * 8 / 4.5e6 + 0.5
+    fewest = {kind: next((parts for parts in range(1, most + 1) if _sum_error(kind, k / parts) <= error), most + 1) for kind in ("planes", "planes gathered")}
     best = (math.inf, None, 0)
     for shape, (round_us, step_us, pair_us) in PLANES_TILES.items():
         tiles_of_part = -(-m // (16 * shape[0])) * -(-n // (64 * shape[1]))
-        for parts in range(1, most + 1):
+        gathered = shape[0] * shape[1] <= 10
+        for parts in range(fewest["planes gathered" if gathered else "planes"], most + 1):
             tiles, steps = tiles_of_part * parts, -(-steps_of_k // parts)
             us = round_us + steps * step_us
             if pair_us is None:
                 us *= -(-tiles // 256)
             elif tiles > 256:
                 us = -(-tiles // 512) * (round_us + steps * pair_us) - (steps * (pair_us - step_us) if 0 < tiles % 512 <= 256 else 0.0)
-            us = max(us, weight_us) + (parts - 1) * part_us
+            us = (max(us, weight_us) + (parts - 1) * part_us) * (1.0 if gathered else 1.04)
             if us < best[0]:
                 best = (us, shape, parts)
     return best

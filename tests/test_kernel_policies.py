@@ -532,3 +532,15 @@ def test_float32_plans_are_shared_by_the_lengths_of_a_fragment_of_rows():
         assert ops._product_plan(rows, 2056, 4104, 6, True) == ops._product_plan(512, 2056, 4104, 6, True)
     assert ops._product_plan_of.cache_info().misses - before == 1
     assert ops._product_plan(64, 2056, 4104, 6, True) == ops._split_plan(64, 2056, 4104, 6) and ops._product_plan(512, 2056, 4104, 6, False) == ops._split_plan(512, 2056, 4104, 6)
+
+
+def test_float32_plans_of_planes_lose_no_precision():
+    """Over the sizes of prompts: never the long sums of the largest tiles where gemm_split's plan gathers its own, and never longer ones than its."""
+    for rows in (66, 96, 130, 250, 333, 500, 700, 1400):
+        for n, k, most_parts in ((4096, 1024, 1), (6144, 1024, 1), (12288, 2048, 1), (4096, 2048, 1), (1024, 2048, 6), (1024, 3072, 6), (2048, 6144, 6), (2560, 9728, 6)):
+            for made in (False, True):
+                (tile, parts), (split, split_parts) = ops._product_plan(rows, n, k, most_parts, True, made), ops._split_plan(rows, n, k, most_parts)
+                if not isinstance(tile, tuple):
+                    assert (tile, parts) == ops._split_plan(-(-rows // 16) * 16, n, k, most_parts)
+                elif tile[0] * tile[1] > 10:
+                    assert ops.SPLIT_TILES[split][2] == 64 and 0.75 * k / parts <= k / split_parts

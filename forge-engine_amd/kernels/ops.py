@@ -253,19 +253,20 @@ def _product_plan(m: int, n: int, k: int, most_parts: int, planes: bool, made: b
     of ``gemm_split``'s own plan (``_sum_error``).
 
     A plan takes 20 (whole) to 70 us (in parts) to find; a length makes as many tiles as the next multiple of 16, the rows of a fragment, so
-    that is what plans are kept by."""
-    return _product_plan_of(m if m <= SPLIT_MIN_ROWS_F32 else -(-m // 16) * 16, n, k, most_parts, planes, made)
+    that is what those of planes are kept by."""
+    own = _split_plan(m, n, k, most_parts)
+    if m <= SPLIT_MIN_ROWS_F32 or not planes:
+        return own
+    return _planes_instead(-(-m // 16) * 16, n, k, most_parts, made) or own
 
 
 @functools.lru_cache(maxsize=4096)
-def _product_plan_of(m: int, n: int, k: int, most_parts: int, planes: bool, made: bool) -> tuple[int | tuple[int, int], int]:
+def _planes_instead(m: int, n: int, k: int, most_parts: int, made: bool) -> tuple[tuple[int, int], int] | None:
     tile, parts = _split_plan(m, n, k, most_parts)
-    if m <= SPLIT_MIN_ROWS_F32 or not planes:
-        return tile, parts
     error = 1.02 * _sum_error("split gathered" if SPLIT_TILES[tile][2] == 128 else "split", k / parts)
     found = _planes_plan(m, n, k, most_parts, error)
     us = (0.8 if made else 3.8 + 1.9e-6 * m * k) + found[0]
-    return found[1:] if us < 1.03 * _split_us(m, n, k, tile, parts) else (tile, parts)      # (where they take the same, the more exact one)
+    return found[1:] if us < 1.03 * _split_us(m, n, k, tile, parts) else None      # (where they take the same, the more exact one)
 
 
 def _sum_error(kind: str, products: float) -> float:

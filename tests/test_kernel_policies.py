@@ -526,12 +526,13 @@ def test_float32_products_of_prompts_take_planes_where_they_were_measured_to_be_
     assert made is None or isinstance(ops._product_plan(rows, weight_rows, k, most_parts, True, made=True)[0], tuple) == (made < split)
 
 
-def test_float32_plans_are_shared_by_the_lengths_of_a_fragment_of_rows():
-    before = ops._product_plan_of.cache_info().misses
+def test_float32_plans_of_planes_are_shared_by_the_lengths_of_a_fragment_of_rows():
+    before = ops._planes_instead.cache_info().misses
     for rows in range(497, 513):
         assert ops._product_plan(rows, 2056, 4104, 6, True) == ops._product_plan(512, 2056, 4104, 6, True)
-    assert ops._product_plan_of.cache_info().misses - before == 1
-    assert ops._product_plan(64, 2056, 4104, 6, True) == ops._split_plan(64, 2056, 4104, 6) and ops._product_plan(512, 2056, 4104, 6, False) == ops._split_plan(512, 2056, 4104, 6)
+    assert ops._planes_instead.cache_info().misses - before == 1
+    for rows, planes in ((64, True), (81, True), (512, False)):      # ... and gemm_split's own by the length itself
+        assert ops._product_plan(rows, 1024, 4096, 6, planes) == ops._split_plan(rows, 1024, 4096, 6)
 
 
 def test_float32_plans_of_planes_lose_no_precision():
@@ -541,6 +542,6 @@ def test_float32_plans_of_planes_lose_no_precision():
             for made in (False, True):
                 (tile, parts), (split, split_parts) = ops._product_plan(rows, n, k, most_parts, True, made), ops._split_plan(rows, n, k, most_parts)
                 if not isinstance(tile, tuple):
-                    assert (tile, parts) == ops._split_plan(-(-rows // 16) * 16, n, k, most_parts)
+                    assert (tile, parts) == (split, split_parts)
                 elif tile[0] * tile[1] > 10:
                     assert ops.SPLIT_TILES[split][2] == 64 and 0.75 * k / parts <= k / split_parts

@@ -89,7 +89,11 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
     const int k0 = (REFETCH ? min(step, last - 1) : step) * KSTEP;
     const int at = k0 + (HALF_END && k0 + KSTEP > K ? my_chunk & 3 : my_chunk) * 8;
     auto load_one = [&](int i) {
-      if (once && (wave + WAVES * i) * 8 >= BM) load_to_lds_once(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
+      // a row of the second operand: known here but for the share that may begin inside the first.  (A branch at every load cost tiles of 16 rows,
+      // us, 11 x 4,096 x 4,096 8.0 -> 8.7, now 7.5; gate/up of 64 x 19,456 x 2,560 3 %.)
+      constexpr int WHOLE = BM / 8 / WAVES, MIXED = BM / 8 % WAVES;
+      const bool second = i > WHOLE || (i == WHOLE && (MIXED == 0 || wave >= MIXED));
+      if (once && second) load_to_lds_once(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
       else load_to_lds(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);
     };
 #pragma unroll

@@ -267,6 +267,7 @@ extern "C" int fe_moe_select_plan(const float* logits, const float* bias, int* o
   return fe_check_launch();
 }
 
+#define CUS 256
 #define BM 32
 #define BN 64
 #define BK 32
@@ -403,9 +404,10 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
 using lds_tile::floatx4;
 using lds_tile::uintx4;
 
-// find_tile by the lanes of a wave: experts 64 at a time, a lane one of them; every lane gets the answer
+// find_tile by the lanes of a wave: experts 64 at a time, a lane one of them; every lane gets the answer, and whether the tile has all of the
+// expert's rows
 template <int ROWS>
-__device__ __forceinline__ bool find_tile_by_lanes(const int* __restrict__ offsets, int E, int slot, int& expert, int& row0, int& row_end) {
+__device__ __forceinline__ bool find_tile_by_lanes(const int* __restrict__ offsets, int E, int slot, int& expert, int& row0, int& row_end, bool& alone) {
   const int lane = threadIdx.x & 63;
   int before = 0;
   for (int e0 = 0; e0 < E; e0 += 64) {
@@ -425,6 +427,7 @@ __device__ __forceinline__ bool find_tile_by_lanes(const int* __restrict__ offse
       const int first = __shfl(begin, at, FE_WAVE), tile = slot - before - (__shfl(upto, at, FE_WAVE) - __shfl(mine, at, FE_WAVE));
       row0 = first + tile * ROWS;
       row_end = __shfl(end, at, FE_WAVE);
+      alone = __builtin_amdgcn_readfirstlane(row_end - first) <= ROWS;
       return true;
     }
     before += __shfl(upto, 63, FE_WAVE);
@@ -432,7 +435,10 @@ __device__ __forceinline__ bool find_tile_by_lanes(const int* __restrict__ offse
   return false;
 }
 
-template <int MI, int NI, int WM, int WN, int KG, int STAGES, int MODE>
+// PAST: weight rows of experts whose pairs are one tile pass the caches.  That is worth it where the blocks are at least one a CU (16 experts of
+// 2,048 x 2,048, two of them, eight tokens 117 -> 107 us; a loss of 2 to 5 % where one or two experts are a few dozen blocks, which wait for
+// single lines: 1 token of 2,048 x 1,024 19.7 -> 20.8), and not where experts have more tiles, whose blocks share the rows.
+template <int MI, int NI, int WM, int WN, int KG, int STAGES, int MODE, bool PAST>
 __global__ __launch_bounds__(64 * WM * WN * KG) void moe_lds_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ offsets,
     const int* __restrict__ order, const float* __restrict__ pair_weight, bf16_t* __restrict__ act,
@@ -445,7 +451,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void moe_lds_kernel(
   const int item = (int)(blockIdx.x % 8) * per_die + (int)(blockIdx.x / 8);
   if (item >= items) return;
   int expert, row0, row_end;
-  if (!find_tile_by_lanes<TILE_ROWS>(offsets, E, item % slots, expert, row0, row_end)) return;
+  bool alone;
+  if (!find_tile_by_lanes<TILE_ROWS>(offsets, E, item % slots, expert, row0, row_end, alone)) return;
   const int n0 = (item / slots) * COLUMNS;
   const bf16_t* w_expert = w + (size_t)expert * (MODE == 0 ? 2 * (size_t)N : (size_t)N) * K;
   auto row_of = [&](int row) -> const bf16_t* {      // rows beyond the expert's and columns beyond N: the last again, never stored
@@ -458,8 +465,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void moe_lds_kernel(
     return w_expert + (size_t)min(n0 + j, N - 1) * K;
   };
   floatx4 acc[MI][NI];
-  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, true>(lds, row_of, 0, (K + lds_tile::KSTEP - 1) / lds_tile::KSTEP, K, acc,
-                                                             offsets[expert + 1] - offsets[expert] <= TILE_ROWS)) return;
+  if (!lds_tile::product<MI, NI, WM, WN, KG, STAGES, true>(lds, row_of, 0, (K + lds_tile::KSTEP - 1) / lds_tile::KSTEP, K, acc, PAST && alone)) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4, wm = wave % WM, wn = wave / WM;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
@@ -514,13 +520,14 @@ static int launch_moe_tile(const bf16_t* a, const bf16_t* w, const int* offsets,
                            int form, const float* extra, int extra_parts, hipStream_t stream) {
   constexpr int TILE_ROWS = 16 * MI * WM, TILE_COLS = 16 * NI * WN, COLUMNS = MODE == 0 ? TILE_COLS / 2 : TILE_COLS;
   constexpr size_t bytes = lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES;
-  static std::atomic<bool> raised{false};
-  auto kernel = moe_lds_kernel<MI, NI, WM, WN, KG, STAGES, MODE>;
-  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, bytes, &raised);
-  if (limit_raised != FE_OK) return limit_raised;
   const long long pairs = (long long)tokens * top, slots = pairs / TILE_ROWS + experts, tiles = ((long long)N + COLUMNS - 1) / COLUMNS;
   const long long blocks = (slots * tiles + 7) / 8 * 8;
   if (blocks > 0x7fffffffLL) return FE_BAD_ARGUMENT;
+  static std::atomic<bool> raised[2];
+  const bool past = std::min<long long>(experts, pairs) * tiles >= CUS && pairs <= (long long)experts * TILE_ROWS;
+  auto kernel = past ? moe_lds_kernel<MI, NI, WM, WN, KG, STAGES, MODE, true> : moe_lds_kernel<MI, NI, WM, WN, KG, STAGES, MODE, false>;
+  const int limit_raised = lds_tile::raise_lds_limit((const void*)kernel, bytes, &raised[past]);
+  if (limit_raised != FE_OK) return limit_raised;
   kernel<<<(unsigned)blocks, 64 * WM * WN * KG, bytes, stream>>>(a, w, offsets, order, pair_weight, act, out, experts, N, K, top, tokens,
                                                                  limit, alpha, form, extra, extra_parts, (int)slots, (int)tiles);
   return fe_check_launch();

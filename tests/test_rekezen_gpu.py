@@ -295,6 +295,32 @@ def test_grouped_products_tiles(tokens, hidden, experts, top, inner, weight_inpu
     assert float((got.double() - want).norm() / want.norm()) < 1e-3
 
 
+# blocks for less than all CUs and for just as many, pairs an expert up to a tile's rows and one more, and all but a few with one expert,
+# whose tiles then share its weight rows beside experts that are one tile
+@pytest.mark.parametrize("tokens,experts,top,hidden,inner,most", [(1, 8, 1, 320, 1024, 1), (1, 8, 1, 320, 8160, 1), (1, 8, 1, 320, 8192, 1), (2, 4, 2, 4096, 288, 2), (64, 4, 2, 1024, 2048, 64),
+                                                                  (65, 4, 2, 1024, 2048, 65), (60, 8, 2, 1088, 1024, 60), (250, 8, 2, 1024, 2080, 250)])
+def test_grouped_products_whose_weights_pass_the_caches(tokens, experts, top, hidden, inner, most):
+    from forge_engine_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(tokens + inner)
+    x = torch.randn(tokens, hidden, generator=g, device=DEV).bfloat16()
+    gate_up = (torch.randn(experts, 2 * inner, hidden, generator=g, device=DEV) * hidden ** -0.5).bfloat16()
+    down = (torch.randn(experts, hidden, inner, generator=g, device=DEV) * inner ** -0.5).bfloat16()
+    chosen = torch.zeros(tokens, top, dtype=torch.int32, device=DEV)       # the first expert takes `most` tokens, a second choice goes round
+    if top > 1:
+        chosen[:, 1] = 1 + torch.arange(tokens, device=DEV).int() % (experts - 1)
+    weights = torch.rand(tokens, top, generator=g, device=DEV)
+    got = ops.moe_experts(x, chosen, weights, gate_up, down, torch.full((top, tokens, hidden), float("nan"), device=DEV), limit=2.0, alpha=1.702)
+    for k in range(top):
+        mine = chosen[:, k].long()
+        both = torch.stack([x[i].double() @ gate_up[e].double().t() for i, e in enumerate(mine.tolist())])
+        gate, up = both[:, :inner].clamp(max=2.0), both[:, inner:].clamp(-2.0, 2.0)
+        act = (gate * torch.sigmoid(1.702 * gate) * (up + 1.0)).float().bfloat16().double()
+        want = torch.stack([act[i] @ down[e].double().t() for i, e in enumerate(mine.tolist())]) * weights[:, k, None].double()
+        torch.testing.assert_close(got[k].double(), want, atol=2e-2, rtol=1e-3)
+        assert float((got[k].double() - want).norm() / want.norm()) < 1e-3
+    assert int((chosen == 0).sum()) == most
+
+
 def test_which_tile_a_grouped_product_takes():
     """Both sides of every line: rows an expert, blocks, steps, for the gated product and the other; and that the sizes above
     reach every tile."""

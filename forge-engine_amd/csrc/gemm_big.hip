@@ -30,11 +30,13 @@
 // k = 8 q .. + 8 of either and receives D[weight row 4 q + i][row of x r]: four neighbouring output columns of a row.
 #include "common.h"
 #include "gate_act.h"
+#include "lds_load.h"
 #include "lds_tile.h"
 #include <algorithm>
 
 namespace {
 
+using lds_load::load_to_lds;
 using lds_tile::bf16x8;
 using lds_tile::floatx4;
 using lds_tile::uintx4;
@@ -44,11 +46,6 @@ constexpr int CUS = 256, XCDS = 8, KSTEP = 64, THREADS = 512;
 constexpr int HALF = 128, PART_BYTES = HALF * 128;
 constexpr int END_PARTS = 0, END_GATED = 1;
 
-// 16 bytes a lane from `base` + `offset` to LDS byte address `at` + 16 * lane (`at` the same in every lane).  The statement writes no
-// vector register, and nothing else in these kernels uses m0, so it is left as it is.
-__device__ __forceinline__ void load_to_lds(const void* base, unsigned int offset, unsigned int at) {
-  asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(at) : "memory", "m0");
-}
 __device__ __forceinline__ void barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" ::: "memory");

@@ -14,10 +14,12 @@
 // 4,096 x 1,024 48 -> 42, x 6,144 x 1,024 68 -> 59, x 12,288 x 2,048 257 -> 190, x 2,048 x 6,144 130 -> 100.  Error against 64 bits
 // 8.2e-8 of 1.49e-7 (700 x 6,144 x 1,024): the products of the first parts and the others' are summed apart, to the end.
 #include "split_f32.h"
+#include "lds_load.h"
 #include "lds_tile.h"
 
 namespace {
 
+using lds_load::load_to_lds;
 using split_f32::bf16x2;
 using split_f32::bf16x8;
 using split_f32::split2;
@@ -26,12 +28,6 @@ using lds_tile::floatx4;
 using lds_tile::wait_loads;
 
 constexpr int XCDS = 8, KSTEP = 64, GROUPS = 2, WAVES = 8;
-
-// 16 bytes a lane from `base` + `offset` to LDS byte address `at` + 16 * lane (`at` the same in every lane).  The statement writes no
-// vector register, and nothing else in these kernels uses m0, so it is left as it is.
-__device__ __forceinline__ void load_to_lds(const void* base, unsigned int offset, unsigned int at) {
-  asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(at) : "memory", "m0");
-}
 
 // A [M, K] float32 as planes [3][M][KP] bfloat16, zeros beyond K: eight elements a thread
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ A, bf16_t* __restrict__ planes, int M, int K, int KP, long long lda) {

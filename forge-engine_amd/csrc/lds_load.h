@@ -1,0 +1,18 @@
+// Loads from memory straight into LDS for kernels in which nothing else uses m0: it is left as it is, not saved and put back around
+// every load (lds_tile.h), which is two scalar instructions less.  Whoever includes this keeps to that; the compiler, which takes m0 as
+// its own, is told of the clobber and warns that it may not honour it, here alone.
+#pragma once
+#include "common.h"
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+namespace lds_load {
+
+// 16 bytes a lane from `base` + `offset` to LDS byte address `at` + 16 * lane (`at` the same in every lane).  The statement writes no
+// vector register.
+__device__ __forceinline__ void load_to_lds(const void* base, unsigned int offset, unsigned int at) {
+  asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(at) : "memory", "m0");
+}
+
+}  // namespace lds_load
+#pragma clang diagnostic pop

@@ -26,7 +26,7 @@ HIPCC_FLAGS = (
     f"--offload-arch={TARGET_ARCH}", "-O3", "-std=c++17", "-shared", "-fPIC",
     # packed float32 instructions are kept off: the compiler must not form them
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-Wno-unused-command-line-argument", "-Wno-inline-asm",
+    "-Wno-unused-command-line-argument",
 )
 
 

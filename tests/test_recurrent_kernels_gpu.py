@@ -86,14 +86,18 @@ def test_update_and_shift_in_one_launch(ops, out_dtype, parts, rows, width):
         ops.rmsnorm_update_shift(h[:, :width - 1].contiguous(), update, w, 1e-6, shift, state, seq, slots, out_dtype=out_dtype)
 
 
-@pytest.mark.parametrize("rows,n,k", [(1, 64, 2048), (6, 64, 2048), (16, 2050, 1024), (17, 64, 2048), (3, 40, 72)])
-def test_product_with_its_tanh(ops, rows, n, k):
+@pytest.mark.parametrize("rows,n,k,launches", [(1, 64, 2048, 1), (6, 64, 2048, 1), (16, 2050, 1024, 1), (17, 64, 2048, 2), (3, 40, 72, 2)])
+def test_product_with_its_tanh(ops, rows, n, k, launches, monkeypatch):
     """In the product's launch or behind it: the same bits."""
     g = torch.Generator().manual_seed(rows + n)
     x, w = rand(g, rows, k, dtype=torch.bfloat16).to(DEV), rand(g, n, k, dtype=torch.bfloat16, scale=0.1).to(DEV)
     x[0, :8] = torch.tensor([float("nan"), 3e38, 1.0, -1.0, 0.0, 1e-30, -1e-3, 2.0]).bfloat16().to(DEV) if rows > 1 else x[0, :8]
     want = ops.tanh_rows(ops.linear(x, w))
+    calls = []
+    real = ops._call
+    monkeypatch.setattr(ops, "_call", lambda library, name, *args: (calls.append(name), real(library, name, *args)))
     got = ops.linear_tanh(x, w)
+    assert calls == ["fe_gemm_ring"] if launches == 1 else (len(calls) == 2 and calls[0] != "fe_gemm_ring" and calls[1] != "fe_gemm_ring")
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(9.0), want.nan_to_num(9.0))
 
 

@@ -170,11 +170,16 @@ def test_mixture_of_experts_kernels(tokens, hidden, experts, top, inner, dtype):
     close(ops.linear_gated(x.to(DEV), shared.to(DEV), limit=0.8, alpha=1.702), refs.linear_gated(x, shared, limit=0.8, alpha=1.702), dtype)
 
 
-# one row, a tile's last, columns that fill no tile of gate and up rows, the shortest K, every tile
-@pytest.mark.parametrize("rows,columns,k", [(5, 1024, 2048), (8, 2048, 2048), (16, 2047, 1024), (9, 2500, 1024), (16, 1030, 4096), (12, 4100, 1088), (13, 8192, 1024)])
-def test_bounded_gate_in_its_product(rows, columns, k, monkeypatch):
-    """The bits of the product and a launch of the activation."""
+# (rows, columns, K, the tile): one of every tile, columns that fill no tile of gate and up rows, K of an odd count of steps
+BOUNDED = [(5, 1024, 2048, 9), (8, 2048, 2048, 9), (16, 2047, 1024, 9), (9, 2500, 1024, 10), (16, 1030, 4096, 9), (12, 4100, 1088, 11), (13, 8192, 1024, 12), (9, 9728, 1024, 13),
+           (16, 10001, 1088, 13)]
+
+
+@pytest.mark.parametrize("rows,columns,k,tile", BOUNDED)
+def test_bounded_gate_in_its_product(rows, columns, k, tile, monkeypatch):
+    """The bits of the product as ``linear`` makes it and a launch of the activation behind it."""
     from forge_engine_amd.kernels import ops
+    assert {case[3] for case in BOUNDED} == {9, 10, 11, 12, 13} and ops.lds_plan(rows, 2 * columns, k, 4 * columns)[0] == tile
     g = torch.Generator().manual_seed(rows + columns)
     x = torch.randn(rows, k, generator=g).bfloat16().to(DEV)
     weight = (torch.randn(2 * columns, k, generator=g) * 2 * k ** -0.5).bfloat16().to(DEV)
@@ -183,19 +188,37 @@ def test_bounded_gate_in_its_product(rows, columns, k, monkeypatch):
     monkeypatch.setattr(ops, "_call", lambda library, name, *args: (calls.append(name), real(library, name, *args)))
     got = ops.linear_gated(x, weight, limit=1.5, alpha=1.702)
     assert calls == ["fe_gemm_lds_bounded"]
-    monkeypatch.setattr(ops, "_lds_store_pays", lambda *sizes: False)
     calls.clear()
-    both = ops.gemm_lds(x, weight, "bf16", tile=ops.lds_plan(rows, 2 * columns, k, 4 * columns)[0])
-    monkeypatch.setattr(ops, "linear", lambda *args, **how: both)
-    want = ops.linear_gated(x, weight, limit=1.5, alpha=1.702)
-    assert calls[-1] == "fe_gated_act" and torch.equal(got, want)
+    both, want = ops.linear(x, weight, ring=False), torch.empty_like(got)
+    ops._call("moe", "fe_gated_act", ops._ptr(both), ops._ptr(want), ops.c_int(ops._code(both.dtype)), ops.c_int(rows), ops.c_int(columns),
+              ops.c_float(1.5), ops.c_float(1.702), ops._stream())
+    assert calls == ["fe_gemm_wide", "fe_gated_act"] and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tile", [9, 10, 11, 12, 13])
+@pytest.mark.parametrize("rows,columns,k", [(1, 1, 64), (1, 7, 64), (16, 9, 128), (15, 33, 1024), (2, 130, 832)])
+def test_bounded_gate_of_the_smallest_products(rows, columns, k, tile):
+    """One row, one step of K, fewer columns than a fragment has, a weight of rows further apart: every tile against the bits of its own
+    bfloat16 product and a launch of the activation."""
+    from forge_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + columns)
+    x = torch.randn(rows, k, generator=g).bfloat16().to(DEV)
+    weight = (torch.randn(2 * columns, k + 8, generator=g) * 2 * k ** -0.5).bfloat16().to(DEV)[:, :k]
+    c_int, ptr = ops.c_int, ops._ptr
+    got = torch.full((rows + 1, columns), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops._call("gemm_wide", "fe_gemm_lds_bounded", ptr(x), ptr(weight), ptr(got), c_int(rows), c_int(columns), c_int(k), ops.c_longlong(weight.stride(0)),
+              ops.c_longlong(columns), c_int(tile), ops.c_float(1.5), ops.c_float(1.702), ops._stream())
+    both, want = ops.gemm_lds(x, weight, "bf16", tile=tile), torch.empty(rows, columns, dtype=torch.bfloat16, device=DEV)
+    ops._call("moe", "fe_gated_act", ptr(both), ptr(want), c_int(ops._code(both.dtype)), c_int(rows), c_int(columns), ops.c_float(1.5), ops.c_float(1.702),
+              ops._stream())
+    assert torch.equal(got[:rows], want) and bool(got[rows].isnan().all())
 
 
 # keys in one run, a few, more than sixteen; a gate a head and one an element; rows of q, gate and output of other strides
 @pytest.mark.parametrize("form", ["plain", "capped", "sloped", "table", "sink"])
 @pytest.mark.parametrize("dim,per_head,contexts", [(128, True, (1, 33, 700, 16)), (64, False, (40, 3, 1, 257, 90)), (128, False, (4000,)), (64, True, (9,) * 20)])
-def test_gate_in_the_decode_kernel(dim, per_head, contexts, form):
-    """Single tokens: the bits of the attention and a launch of the gate."""
+def test_gate_in_the_decode_kernel(dim, per_head, contexts, form, monkeypatch):
+    """Single tokens: the bits of the attention and a launch of the gate, in one."""
     from forge_engine_amd.kernels import ops
     n, heads, kv_heads, page = len(contexts), 8, 2, 16
     g = torch.Generator().manual_seed(dim + n)
@@ -214,7 +237,11 @@ def test_gate_in_the_decode_kernel(dim, per_head, contexts, form):
     how = dict(num_seqs=n, max_q_len=1, q_heads=heads, kv_heads=kv_heads, head_dim=dim, value_dim=dim, scale=dim ** -0.5, num_decode=n,
                max_ctx=max(contexts), **kinds[form])
     got = torch.empty(n, heads * dim + 2, dtype=torch.bfloat16, device=DEV)[:, :heads * dim]
+    calls = []
+    real = ops._call
+    monkeypatch.setattr(ops, "_call", lambda library, name, *args: (calls.append(name), real(library, name, *args)))
     ops.masked_attention(q, keys, values, got, *where, gate=gate, head_gate=per_head, factor=1.25, **how)
+    assert calls == ["fe_paged_attention_decode_gated"]
     apart, want = (torch.empty(n, heads * dim, dtype=torch.bfloat16, device=DEV) for _ in range(2))
     ops.masked_attention(q, keys, values, apart, *where, **how)
     ops._sigmoid_gate(apart, gate, want, heads, dim, dim, per_head, 1.25)

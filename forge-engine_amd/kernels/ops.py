@@ -375,20 +375,29 @@ SPLIT_AHEAD_MAX_K = 8192        # the widest rows that the norm's kernel holds i
 
 def takes_split(rows: int, weight: Tensor, update: bool = False) -> bool:
     """Whether ``linear`` (``linear_update``) takes ``SplitRows`` of so many rows: where planes that are there already take the product."""
-    if not weight.is_cuda or weight.dtype != torch.float32 or weight.dim() != 2 or rows <= SPLIT_MIN_ROWS_F32:
+    if rows <= SPLIT_MIN_ROWS_F32 or not weight.is_cuda or weight.dtype != torch.float32 or weight.dim() != 2 or _made_plan(rows, *weight.shape, update) is None:
         return False
-    n, k = weight.shape
-    if (k % 64 or k < SPLIT_MIN_K or (k > SPLIT_AHEAD_MAX_K and not update) or weight.stride(1) != 1 or weight.stride(0) % 4 or not k <= weight.stride(0) < 1 << 22
-            or weight.data_ptr() % 16 or 6 * rows * (k + 63) >= 1 << 32):
-        return False
+    return weight.stride(1) == 1 and weight.stride(0) % 4 == 0 and weight.shape[1] <= weight.stride(0) < 1 << 22 and weight.data_ptr() % 16 == 0
+
+
+@functools.lru_cache(maxsize=4096)
+def _made_plan(rows: int, n: int, k: int, update: bool) -> tuple[tuple[int, int], int] | None:
+    """The plan of a product with ``SplitRows``, or None where they are not taken."""
+    if rows <= SPLIT_MIN_ROWS_F32 or k % 64 or k < SPLIT_MIN_K or (k > SPLIT_AHEAD_MAX_K and not update) or 6 * rows * (k + 63) >= 1 << 32:
+        return None
     most_parts = SPLIT_MOST_PARTS if update else 1
-    return _split_pays(rows, n, k, most_parts) and isinstance(_product_plan(rows, n, k, most_parts, True, True)[0], tuple)
+    plan = _product_plan(rows, n, k, most_parts, True, True)
+    return plan if isinstance(plan[0], tuple) and _split_pays(rows, n, k, most_parts) else None
 
 
-def gemm_split(a: Tensor | SplitRows, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+def gemm_split(a: Tensor | SplitRows, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None,
+               checked: bool = False) -> Tensor:
     """float32 partial sums [parts, M, N] of a[M, K] @ b[N, K]^T over runs of whole steps of K (given ``out`` [M, N], the product with
     the bias there), each operand as three bfloat16 numbers whose sum it is (a number below 2^-110: up to 2^-134 beside it).  ``tile``: the
-    block's, of ``SPLIT_TILES`` by its number, or of ``PLANES_TILES`` (a split ahead, here or by who made a)."""
+    block's, of ``SPLIT_TILES`` by its number, or of ``PLANES_TILES`` (a split ahead, here or by who made a).
+    ``checked``: the caller has looked the operands over and made the plan for them."""
+    if checked:
+        return _launch_split(a, None, b, parts, tile, bias, out)
     made = None
     if isinstance(a, SplitRows):
         a, made = a
@@ -406,8 +415,15 @@ def gemm_split(a: Tensor | SplitRows, b: Tensor, parts: int, tile: int | tuple[i
         raise KernelError(f"out must be [{m}, {n}], got {tuple(out.shape)}")
     if bias is not None and _gpu(bias, "bias", torch.float32).shape != (n,):
         raise KernelError(f"bias must be [{n}]")
+    return _launch_split(a, made, b, parts, tile, bias, out)
+
+
+def _launch_split(a: Tensor, made: Tensor | None, b: Tensor, parts: int, tile: int | tuple[int, int], bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+    """``gemm_split`` of operands that have been looked over and the plan that was made for them."""
+    m, k = a.shape
+    n = b.shape[0]
     result = torch.empty((parts, m, n), dtype=torch.float32, device=a.device) if out is None else out
-    if planes:
+    if isinstance(tile, tuple):
         scratch = torch.empty(3 * m * (-(-k // 64) * 64), dtype=torch.bfloat16, device=a.device) if made is None else made
         _call("gemm_planes", "fe_gemm_planes", _ptr(a), _ptr(scratch), _ptr(b), _ptr(bias), _ptr(result), c_int(m), c_int(n), c_int(k),
               c_longlong(a.stride(0)), c_longlong(b.stride(0)), c_longlong(n), c_int(parts), c_longlong(m * n), c_int(tile[0]), c_int(tile[1]), c_int(int(made is not None)), _stream())
@@ -440,7 +456,7 @@ def gemm_nt_f32(a: Tensor, b: Tensor, bias: Tensor | None = None, out: Tensor | 
         if bias.shape != (n,):
             raise KernelError(f"bias must be [{n}]")
     if m > SPLIT_MIN_ROWS_F32 and _split_fits(a, b) and out.data_ptr() % 4 == 0 and _split_pays(m, n, k, 1):
-        return gemm_split(a, b, 1, _product_plan(m, n, k, 1, _planes_fit(a, b))[0], bias, out)
+        return gemm_split(a, b, 1, _product_plan(m, n, k, 1, _planes_fit(a, b))[0], bias, out, checked=True)
     lda = a.stride(0) if m > 1 else max(k, a.stride(0))
     ldb = b.stride(0) if n > 1 else max(k, b.stride(0))
     _call("gemm_f32", "fe_gemm_nt_f32", _ptr(a), _ptr(b), _ptr(bias), _ptr(out), c_int(m), c_int(n),
@@ -551,10 +567,11 @@ def linear(x: Tensor | UnscaledRows | SplitRows, weight: Tensor, bias: Tensor | 
             raise KernelError("rows without their norm's factors are for the products through LDS only")
         return gemm_ring(x, weight, "f32" if weight.dtype == torch.float32 else "bf16")
     if isinstance(x, SplitRows):
-        if out_dtype not in (None, torch.float32) or not takes_split(x.shape[0], weight) or weight.shape[1] != x.shape[1]:
+        plan = _made_plan(x.shape[0], *weight.shape, False) if weight.dim() == 2 else None
+        if plan is None or out_dtype not in (None, torch.float32):
             raise KernelError("rows with their parts are for the products of planes only")
         y = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=weight.device)
-        return gemm_split(x, weight, 1, _product_plan(x.shape[0], *weight.shape, 1, True, True)[0], bias, y)
+        return gemm_split(x, weight, 1, plan[0], bias, y)      # (which looks the operands over)
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     out_dtype = x.dtype if out_dtype is None else out_dtype
@@ -1207,12 +1224,16 @@ def _big_gate_pays(rows: int, columns: int, k: int) -> bool:
     return filled >= (0.3 if k < 1024 else 0.57 if k < 2048 else 0.65)
 
 
+BIG_UPDATE_MIN_K = 8192
+
+
 def _big_update_parts(rows: int, weight_rows: int, k: int) -> int:
     """Parts of K in which tiles of 256 x 256 make an update faster than the rest does, or 0: a long K in two to seven parts that
     fill three quarters of one round of the CUs (3,898 random updates with their norms in captured graphs: from K = 8,192 on 1.07 to 1.29
     times as fast, 2,560 x 9,728 at 2,048 rows 117 -> 100 us; at K = 4,096 to 8,192 .88 to 1.01; in one part, where the library adds into the stream, 1.0)."""
-    tiles = -(-rows // 256) * -(-weight_rows // 256)
-    parts = WIDE_CUS // tiles if k >= 8192 else 0
+    if k < BIG_UPDATE_MIN_K:
+        return 0
+    parts = WIDE_CUS // (-(-rows // 256) * -(-weight_rows // 256))
     return parts if 2 <= parts <= 7 and rows * weight_rows * parts >= 0.75 * WIDE_CUS * 256 * 256 else 0
 
 
@@ -1223,19 +1244,19 @@ def linear_update(x: Tensor | SplitRows, weight: Tensor, bias: Tensor | None = N
     stores, which saves the next norm the update's bytes, and None is returned: the same float32
     sum in the same order, stream + (x @ weight^T)."""
     if isinstance(x, SplitRows):
-        if bias is not None or not takes_split(x.shape[0], weight, update=True) or weight.shape[1] != x.shape[1]:
+        plan = _made_plan(x.shape[0], *weight.shape, True) if weight.dim() == 2 else None
+        if plan is None or bias is not None:
             raise KernelError("rows with their parts are for the products of planes only")
-        tile, parts = _product_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS, True, True)
-        return gemm_split(x, weight, parts, tile)
+        return gemm_split(x, weight, plan[1], plan[0])
     _gpu(x, "x")
     _gpu(weight, "weight", contiguous=False)
     if bias is None and x.shape[0] > SPLIT_MIN_ROWS and _split_fits(x, weight) and _split_pays(x.shape[0], *weight.shape, SPLIT_MOST_PARTS):
         tile, parts = _product_plan(x.shape[0], *weight.shape, SPLIT_MOST_PARTS, _planes_fit(x, weight))
-        return gemm_split(x, weight, parts, tile)
+        return gemm_split(x, weight, parts, tile, checked=True)
     plain_bf16 = bias is None and weight.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
-    if plain_bf16 and x.shape[0] > MID_ROWS and _big_fits(x, weight, False):
+    if plain_bf16 and x.shape[0] > MID_ROWS and x.shape[1] >= BIG_UPDATE_MIN_K:
         parts = _big_update_parts(x.shape[0], *weight.shape)
-        if parts:
+        if parts and _big_fits(x, weight, False):
             return gemm_big(x, weight, "parts", parts)
     if plain_bf16 and _lds_fits(x, weight):
         plan = _lds_update(x.shape[0], *weight.shape)
@@ -1391,7 +1412,7 @@ def linear_swiglu(x: Tensor | UnscaledRows | SplitRows, gate_up_weight: Tensor, 
     _gpu(x, "x")
     _gpu(gate_up_weight, "gate_up_weight")
     rows = x.shape[0]
-    if rows > MID_ROWS and _big_fits(x, gate_up_weight, True) and _big_gate_pays(rows, gate_up_weight.shape[0] // 2, x.shape[1]):
+    if rows > MID_ROWS and x.dtype == torch.bfloat16 and _big_gate_pays(rows, gate_up_weight.shape[0] // 2, x.shape[1]) and _big_fits(x, gate_up_weight, True):
         return gemm_big(x, gate_up_weight, "gated", act=act)
     if (GATED_TILE_MIN_ROWS <= rows <= GATED_TILE_MAX_ROWS and x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16
             and x.is_contiguous() and x.shape[1] % 64 == 0 and x.shape[1] <= GATED_TILE_MAX_K and gate_up_weight.shape[0] % 2 == 0

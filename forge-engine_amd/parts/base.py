@@ -79,7 +79,7 @@ class Residual:
         first is applied now, and nothing is pending any more: only who asks for it with its norm (``take_normed``) gets it."""
         if self.pending_norm is not None:
             self._apply_normed()
-        return self._multiplied_out()
+        return self._multiplied_out() if isinstance(self._pending, ops.UpdateProduct) else self._pending
 
     @pending.setter
     def pending(self, update: Tensor | ops.UpdateProduct | None) -> None:
@@ -142,7 +142,7 @@ class Residual:
 
     def normed(self):
         """(update, weight, eps) of a pending update that is to be normed; it stays pending."""
-        return (self._multiplied_out(), *self.pending_norm)
+        return (self._multiplied_out() if isinstance(self._pending, ops.UpdateProduct) else self._pending, *self.pending_norm)
 
     def take_normed(self):
         """The same, which the caller now applies."""
@@ -150,9 +150,8 @@ class Residual:
         self.pending = self.pending_norm = None
         return taken
 
-    def _multiplied_out(self) -> Tensor | None:
-        if isinstance(self._pending, ops.UpdateProduct):
-            self._pending = ops.linear_update(self._pending.x, self._pending.weight)
+    def _multiplied_out(self) -> Tensor:
+        self._pending = ops.linear_update(self._pending.x, self._pending.weight)
         return self._pending
 
     def _apply_normed(self) -> None:

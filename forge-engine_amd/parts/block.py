@@ -33,7 +33,7 @@ class PreNormBlock(Block):
         norm, rows = self.norms[role], residual.h.shape[0]
         if getattr(norm, "leaves_factors", False):
             unscaled = part.takes_unscaled(rows, *step)
-            if type(norm).forward is RMSNorm.forward:       # a norm with a way of its own may know nothing of the parts
+            if self.ctx.dtype == torch.float32 and type(norm).forward is RMSNorm.forward:       # (a norm with a way of its own may know nothing of parts)
                 return norm.forward(residual, unscaled=unscaled, split=part.takes_split(rows, *step))
             return norm.forward(residual, unscaled=unscaled)
         return norm.forward(residual)

@@ -563,3 +563,13 @@ def test_float32_plans_of_planes_lose_no_precision():
                     assert (tile, parts) == (split, split_parts)
                 elif tile[0] * tile[1] > 10:
                     assert ops.SPLIT_TILES[split][2] == 64 and 0.75 * k / parts <= k / split_parts
+
+
+def test_rows_of_decode_steps_are_turned_away_unseen():
+    """Whether rows come with their parts is asked of every part of every layer: by the rows first, which say no for any decode step."""
+    for rows in (1, 17, 64):
+        assert not ops.takes_split(rows, None) and not ops.takes_split(rows, None, update=True) and ops._made_plan(rows, 4096, 1024, False) is None
+    assert ops._made_plan(700, 4096, 1024, False) == ops._product_plan(700, 4096, 1024, 1, True, made=True)
+    assert ops._made_plan(700, 1024, 3072, True) == ops._product_plan(700, 1024, 3072, ops.SPLIT_MOST_PARTS, True, made=True)
+    assert ops._made_plan(700, 1024, 1000, False) is None and ops._made_plan(700, 4096, 8256, False) is None
+    assert ops._big_update_parts(2048, 2560, 8128) == 0 and ops._big_update_parts(2048, 2560, 8192) == 3

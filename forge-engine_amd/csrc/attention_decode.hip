@@ -19,10 +19,10 @@
 //     lanes: two shuffles), base-2 exponent with the scale folded in;
 //   * output transposed, O^T = V^T P^T: A = 16 dims x 32 keys from the value
 //     pages, which are stored transposed ([D][slot]) for this, B = P^T.  In pages of 16 and 32 keys an instruction takes whole lines,
-//     once, and the values are loaded past the caches (64 sequences of 130 to 2,000 keys 59.0 -> 53.7 us, 8 of 1,025 13.2 -> 12.7, two
-//     of 30,000 and 20,000 43.7 -> 40.8; the keys, a line of which takes two instructions, as well: 54.3, 13.0, 41.7).  From 64 on a
-//     dim's row is a line or more, of which two waves take a half each: past the caches they would both fetch it (60 sequences of
-//     1,585 keys 126 -> 142 us, 14 of 14,614 in pages of 128 106 -> 120).
+//     once, and the values are loaded past the caches (64 sequences of 130 to 2,000 keys 52.0 -> 48.4 us, 8 of 1,025 12.3 -> 12.1, two
+//     of 30,000 and 20,000 42.8 -> 39.7; the keys, a line of which takes two instructions, as well: 1 to 2 % more again).  From 64 on a
+//     dim's row is a line or more, of which two waves take a half each: past the caches they would both fetch it (the 64 sequences in pages
+//     of 64 57.4 -> 60.9, 14 of 14,614 in pages of 128 158 -> 178).
 // Exactness: scores, max, sum and the weighted value sum are float32; P is
 // rounded to bfloat16 for the second product; one rounding at the final store.
 //

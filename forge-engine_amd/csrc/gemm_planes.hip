@@ -8,11 +8,12 @@
 // read two ahead, the step's loads go out one after the other over the first rows (their addresses pass one by one: issued at once they held
 // everything up), and between two MFMAs stand two vector instructions of the sums of the row before or of the splitting.
 //
-// What bounds it: a step of 128 x 128 takes 1.7 us of 1.28 that its MFMAs do (2.1 with the small products added to the long sum at every step
+// What bounds it: a step of 128 x 128 takes 1.7 us (1.9 with the weight coming from memory) of 1.28 that its MFMAs do (2.1 with the small products added to the long sum at every step
 // and loads issued at once; without loads .16 less, without the planes' reads .3, without splitting .2), a round of tiles another 4 to 7 us:
 // the first loads' way, the groups' meeting, the stores.  Measured on one MI355X against gemm_split, us, both with the pass over A: 700 x
 // 4,096 x 1,024 48 -> 42, x 6,144 x 1,024 68 -> 59, x 12,288 x 2,048 257 -> 190, x 2,048 x 6,144 130 -> 100.  Error against 64 bits
-// 8.2e-8 of 1.49e-7 (700 x 6,144 x 1,024): the products of the first parts and the others' are summed apart, to the end.
+// 8.2e-8 of 1.49e-7 (700 x 6,144 x 1,024; 1.31e-7 in the tiles that do not gather, below): the products of the first parts and the others'
+// are summed apart, to the end.
 #include "split_f32.h"
 #include "lds_load.h"
 #include "lds_tile.h"

@@ -15,7 +15,7 @@
 // before the sums meet at the end, in the waves' order.
 //
 // What bounds it: the weight's bytes, and latency at the small sizes.  No block reads another's weight rows, so they pass the caches
-// (lds_tile::load_to_lds_once; 1 to 16 rows, us: 12,288 x 2,048 gated 12.0 -> 10.9, 6,144 x 2,560 7.7 -> 7.3, 4,096 x 1,024 3.8 -> 3.7).  What the update ending saves is the norm's launch (4.0 to 4.7
+// (lds_tile::load_to_lds_once; us: 4 rows x 12,288 x 2,048 gated 11.4 -> 10.6, 8 x 6,144 x 2,560 7.4 -> 7.1, 1 x 4,096 x 1,024 3.7 either way).  What the update ending saves is the norm's launch (4.0 to 4.7
 // us in a captured step) and the parts that went through memory: 2,560 x 9,728 with its norm 13.7 -> 11.2 us at 8 rows (4.5 TB/s),
 // 2,560 x 4,096 9.2 -> 6.5, 1,024 x 2,048 at 1 row 5.4 -> 3.2; a decode step of 0.6B at 1 request 909 -> 799 us, of 4B at 8 requests
 // 2,464 -> 2,300.  The stored endings beside what took such sizes before (420 random products): bfloat16 1.36 times as fast, gated 1.41;

@@ -23,9 +23,9 @@ __device__ __forceinline__ void load_to_lds(const void* global, unsigned int at)
   asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off\n s_mov_b32 m0, %0"
                : "=&s"(m0) : "v"(global), "s"(at) : "memory");
 }
-// The same for lines that no other block reads (and this one not again): they pass the caches without staying there, which leaves a CU more
-// of the lines that its L1 waits for (8 rows x 19,456 x 2,560 19.5 -> 18.6 us, x 2,560 x 9,728 10.7 -> 10.0; where two blocks share a weight
-// row it is the wrong way: 250 rows 41.3 -> 46.4).
+// The same for lines that no other block reads (and this one not again): they pass the caches without staying there (us, weights from memory,
+// with the caches full of something else before: 8 rows x 19,456 x 2,560 19.4 -> 17.9, x 2,560 x 9,728 11.1 -> 10.8, 64 rows x 19,456 x 2,560
+// 23.8 -> 22.7; where two blocks share a weight row it is the wrong way: 250 rows 41.3 -> 46.4).
 __device__ __forceinline__ void load_to_lds_once(const void* global, unsigned int at) {
   unsigned int m0;
   asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off nt\n s_mov_b32 m0, %0"
@@ -89,8 +89,8 @@ __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, in
     const int k0 = (REFETCH ? min(step, last - 1) : step) * KSTEP;
     const int at = k0 + (HALF_END && k0 + KSTEP > K ? my_chunk & 3 : my_chunk) * 8;
     auto load_one = [&](int i) {
-      // a row of the second operand: known here but for the share that may begin inside the first.  (A branch at every load cost tiles of 16 rows,
-      // us, 11 x 4,096 x 4,096 8.0 -> 8.7, now 7.5; gate/up of 64 x 19,456 x 2,560 3 %.)
+      // a row of the second operand: known here but for the share that may begin inside the first.  (Loads past the caches with a branch at
+      // every load, us: 11 x 4,096 x 4,096 7.7 -> 8.5, 5 x 3,776 x 4,480 7.8 -> 9.1; without it 7.5 and 7.6.)
       constexpr int WHOLE = BM / 8 / WAVES, MIXED = BM / 8 % WAVES;
       const bool second = i > WHOLE || (i == WHOLE && (MIXED == 0 || wave >= MIXED));
       if (once && second) load_to_lds_once(from[i] + at, base + (stage * STAGE + (wave + WAVES * i) * 64) * 16);

@@ -435,9 +435,10 @@ __device__ __forceinline__ bool find_tile_by_lanes(const int* __restrict__ offse
   return false;
 }
 
-// PAST: weight rows of experts whose pairs are one tile pass the caches.  That is worth it where the blocks are at least one a CU (16 experts of
-// 2,048 x 2,048, two of them, eight tokens 117 -> 107 us; a loss of 2 to 5 % where one or two experts are a few dozen blocks, which wait for
-// single lines: 1 token of 2,048 x 1,024 19.7 -> 20.8), and not where experts have more tiles, whose blocks share the rows.
+// PAST: weight rows of experts whose pairs are one tile pass the caches.  That is worth it where the blocks are at least one a CU (both products,
+// two choices a token, width 2,048, us: 8 tokens, 8 / 16 experts 53.0 -> 48.9 / 69.5 -> 64.9, 32 tokens 54.7 -> 51.8), not where one or two
+// experts are a few dozen blocks, which only wait longer (1 token, 2,048 x 1,024 19.7 -> 20.8), nor where experts have more tiles, whose blocks
+// share the rows (300 tokens 73.7 -> 75.3, by asking alone).
 template <int MI, int NI, int WM, int WN, int KG, int STAGES, int MODE, bool PAST>
 __global__ __launch_bounds__(64 * WM * WN * KG) void moe_lds_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ offsets,

@@ -170,15 +170,14 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
   static_assert(!SCALED || lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + 16 * SQUARES_PITCH <= 160 * 1024, "LDS of a CU");
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + COLUMNS - 1) / COLUMNS;
   if (tiles_m * tiles_n * parts > 0x7fffffffLL) return FE_BAD_ARGUMENT;
-  // one tile of x: no block reads another's weight rows (an instance of its own: asked at every load it cost prompts of 361 rows .3 %), and
-  // unless the tile fetches a walk's last step again, neither does this one.  (Its walks of eight steps request eighteen: with those past the
-  // caches decode steps of 17 to 32 requests took, us, 0.6B 1,114 -> 1,139 and 1,156 -> 1,188, 1.7B 1,591 -> 1,607; as it is 1,118, 1,164 and 1,581.
-  // Prompts of so many tokens alone, 0.6B, gained 30 of 1,155 by it: the weights then left the head's rows in the last cache.)
-  constexpr bool AGAIN = refetches<MI, NI, WM, WN>();
-  static_assert(!(SCALED && AGAIN), "rows with factors are one tile of x");
+  // one tile of x: no block reads another's weight rows (an instance of its own: asked at every load it cost prompts of 361 rows .3 %).  The
+  // tile that fetches a walk's last step again does so past the caches too: by itself its walks of 4 to 16 steps are .3 to 3 % slower for it
+  // in the mean and those of 32 2 % faster, but whole prompts gain (32 steps of 17 to 32 rows, its rows past the caches to in them, mean
+  // ratio of the times at 0.6B, 1.7B and 4B: prompts .951, 1.004 and .967; decode 1.004, 1.007 and .999, at most 1.009).  Likely because the
+  // last cache is left to rows that are read again; at 0.6B all of a layer's products have to pass, at 4B the first one is enough.
   static std::atomic<bool> raised[2];
-  const bool once = tiles_m == 1 && !AGAIN;
-  auto kernel = once ? gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, !AGAIN> : gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, SCALED>;
+  const bool once = tiles_m == 1;
+  auto kernel = once ? gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, true> : gemm_lds_kernel<MI, NI, WM, WN, KG, STAGES, END, SCALED, SCALED>;
   const int limit_raised = lds_tile::raise_lds_limit(
       (const void*)kernel, lds_tile::Shape<MI, NI, WM, WN, KG, STAGES>::BYTES + (SCALED ? 16 * SQUARES_PITCH : 0), &raised[once]);
   if (limit_raised != FE_OK) return limit_raised;

@@ -23,7 +23,7 @@ __device__ __forceinline__ void load_to_lds(const void* global, unsigned int at)
   asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off\n s_mov_b32 m0, %0"
                : "=&s"(m0) : "v"(global), "s"(at) : "memory");
 }
-// The same for lines that no other block reads (and this one not again): they pass the caches without staying there (us, weights from memory,
+// The same for lines that no other block reads: they pass the caches without staying there (us, weights from memory,
 // with the caches full of something else before: 8 rows x 19,456 x 2,560 19.4 -> 17.9, x 2,560 x 9,728 11.1 -> 10.8, 64 rows x 19,456 x 2,560
 // 23.8 -> 22.7; where two blocks share a weight row it is the wrong way: 250 rows 41.3 -> 46.4).
 __device__ __forceinline__ void load_to_lds_once(const void* global, unsigned int at) {
@@ -74,7 +74,6 @@ struct Shape {
 // have been fetched (gemm_lds.h).
 template <int MI, int NI, int WM, int WN, int KG, int STAGES, bool HALF_END, bool REFETCH = false, typename Once = std::false_type, typename RowOf>
 __device__ __forceinline__ bool product(uintx4* lds, RowOf row_of, int first, int last, int K, floatx4 (&acc)[MI][NI], Once once = {}) {
-  static_assert(!(REFETCH && std::is_same_v<Once, std::true_type>), "lines that are fetched again stay in the caches");
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, WAVES = WM * WN * KG, T = 2 / KG;
   constexpr int GROUPS = (BM + BN) / 8, LOADS = GROUPS / WAVES, MORE = GROUPS % WAVES;   // groups of eight rows: one load of a wave each
   constexpr int STAGE = (BM + BN) * 8;              // 16-byte units of a stage

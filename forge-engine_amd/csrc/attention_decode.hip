@@ -253,14 +253,16 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
   } else {
     const int z = blockIdx.z, q = cu_q[z];
     run = {z, (int)blockIdx.x, (int)gridDim.x, z * (int)gridDim.x, q, cu_q[z + 1] - q, ctx_len[z]};
-    // The launch has splits for the longest context that may come; one that four waves read in two blocks each needs none, and no merge (us,
-    // splits and merge -> one run: 1 sequence of 60 keys in a launch of 8 splits 7.5 -> 5.6, of 150 7.3 -> 6.3, of 217 7.3 -> 6.6, of 250 7.5 ->
-    // 7.0, 8 of 200 in one of 4 8.2 -> 7.4; with three blocks each it takes as long as the merge).
+    // The launch has splits for the longest context that may come; one that four waves read in one block each needs none, and no merge (us,
+    // splits and merge -> one run: 1 sequence of 60 keys in a launch of 8 splits 7.5 -> 5.6, 8 of 100 in one of 4 9.0 -> 7.1).
+    // Beyond, one run would save more (1 of 217 keys 7.1 -> 5.9), but a wave's second block would be rounded against another maximum than its
+    // split's, and so the results of all contexts of 129 to 256 keys; one run that keeps its blocks apart and sums them as the splits do
+    // takes as long as they (7.2).
     // Finished queries keep their splits, and with them the order of every sum: they come by the general attention path, which the designs
     // with routers take, whose choice among experts at a near tie another rounding changes (and some without one, for whom it is time left).
     if constexpr (PREPARE) {
       const KeyRange range = key_range(run.ctx, run.ctx - 1, window, chunk);
-      if (range.last - range.first <= 2 * WAVES) run.splits = 1;
+      if (range.last - range.first <= WAVES) run.splits = 1;
       if (run.split >= run.splits) return;
     }
   }

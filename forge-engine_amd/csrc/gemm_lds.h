@@ -26,12 +26,6 @@
 // stored in 96 x 64 9.8 -> 8.9, 2,048 x 6,144 in parts in 96 x 128 22.6 -> 18.5; 80 rows: gate/up of 9,728 x 2,560, the library and
 // the gate kernel before, 35.0 -> 26.0).
 //
-// A gate/up weight has many rows, so that hundreds of rows of x make several rounds of 128 x 160: tiles of 128 x 192 to 192 x 160 make
-// one round of what those cut into one and a half, and pull fewer bytes a product (882 sizes of 192 to 1,024 rows: 8 % faster in the
-// mean; 9,728 columns, K = 2,560 at 320 rows, the library and the gate kernel before, 54.4 -> 44, at 361 50 -> 46).  128 x 256 is wider
-// than its registers (16 of 256 go to memory and back once a step) and wins all the same where it makes one round.  The other endings
-// gain 1 to 2 %, which is not worth their code.
-//
 // Up to 16 rows of x, tiles of 16 rows with one fragment a wave: the weight's bytes are nearly all of the tile's, so the widths
 // (16 to 80 weight rows) only choose how evenly the CUs share them, and 8 to 12 stages keep 64 KB and more of a CU's share in
 // flight; the kernels with the weight in registers had a wave's two to four steps, and read x again for every 16 weight rows
@@ -201,8 +195,7 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
 
 // Operands and endings as fe_gemm_wide's (ending 0: parts, 1: bfloat16, 2: gated); the caller has checked them.
 // tile: rows of x x weight rows a block takes: 0: 32 x 32, 1: 64 x 32, 2: 64 x 64, 3: 64 x 80, 4: 64 x 96, 5: 128 x 64,
-//   6: 128 x 128, 7: 128 x 160, 8: 32 x 64, 9 to 13: 16 x 16, 32, 48, 64, 80; 96064, 96096, 96128: 96 x 64, 96, 128;
-//   gated only 128192, 128256, 160160, 192128, 192160: 128 x 192, 256, 160 x 160, 192 x 128, 160.
+//   6: 128 x 128, 7: 128 x 160, 8: 32 x 64, 9 to 13: 16 x 16, 32, 48, 64, 80; 96064, 96096, 96128: 96 x 64, 96, 128.
 static int launch(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
                   int parts, long long part_stride, int tile, GateAct act, hipStream_t stream) {
 #define FE_END(END, ...) return launch_tile<__VA_ARGS__, END>(x, w, out, M, N, K, ldw, ldo, parts, part_stride, act, stream)
@@ -211,10 +204,6 @@ static int launch(const void* x, const void* w, void* out, int M, int N, int K, 
     if (ending == END_PARTS) FE_END(END_PARTS, __VA_ARGS__);           \
     else if (ending == END_BF16) FE_END(END_BF16, __VA_ARGS__);        \
     else if (ending == END_GATED) FE_END(END_GATED, __VA_ARGS__);      \
-    break;
-#define FE_GATED(I, ...)                                               \
-  case I:                                                              \
-    if (ending == END_GATED) FE_END(END_GATED, __VA_ARGS__);           \
     break;
   switch (tile) {
     FE_TILE(0, 1, 2, 2, 1, 2, 10)
@@ -234,13 +223,7 @@ static int launch(const void* x, const void* w, void* out, int M, int N, int K, 
     FE_TILE(96064, 3, 2, 2, 2, 2, 4)
     FE_TILE(96096, 3, 3, 2, 2, 2, 4)
     FE_TILE(96128, 3, 4, 2, 2, 2, 4)
-    FE_GATED(128192, 4, 6, 2, 2, 2, 3)
-    FE_GATED(128256, 4, 8, 2, 2, 2, 3)
-    FE_GATED(160160, 5, 5, 2, 2, 2, 3)
-    FE_GATED(192128, 6, 4, 2, 2, 2, 3)
-    FE_GATED(192160, 6, 5, 2, 2, 2, 3)
   }
-#undef FE_GATED
 #undef FE_TILE
 #undef FE_END
   return FE_BAD_ARGUMENT;

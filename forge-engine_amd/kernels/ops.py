@@ -761,9 +761,6 @@ LDS_TILES = dict(enumerate((
     (64, 96, 2, 0.302, 0.6041), (128, 64, 1, 0.3322, 0.6643), (128, 128, 1, 0.5162, 1.0325), (128, 160, 1, 0.6269, 1.2538), (32, 64, 2, 0.1891, 0.35),
     (16, 16, 2, 0.073, 0.117), (16, 32, 2, 0.116, 0.247), (16, 48, 2, 0.143, 0.334), (16, 64, 2, 0.168, 0.444), (16, 80, 1, 0.220, 0.440))))
 LDS_TILES.update({96064: (96, 64, 1, 0.3087, 0.6173), 96096: (96, 96, 1, 0.3728, 0.7456), 96128: (96, 128, 1, 0.4775, 0.955)})
-# Beside them, for gate/up products only
-LDS_GATE_TILES = {**LDS_TILES, 128192: (128, 192, 1, 0.6899, 1.3798), 128256: (128, 256, 1, 0.8844, 1.7688), 160160: (160, 160, 1, 0.7983, 1.5966),
-                  192128: (192, 128, 1, 0.6386, 1.2772), 192160: (192, 160, 1, 0.8, 1.6)}
 LDS_HEAD_WEIGHT_ROWS = 131072  # float32 logits: see _lds_head_pays
 LDS_HEAD_MIN_K = 2048
 LDS_GATE_MAX_ROWS = 1536       # gate/up: measured up to here (4,096 rows, 256 columns of K = 4,096: 28.6 against 43.0 us)
@@ -773,7 +770,7 @@ UPDATE_NORM_MAX_WIDTH = 8192   # 32 weight rows a block
 
 
 def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, summed: bool = False,
-             one_round: bool = False, gated: bool = False) -> tuple[int, int]:
+             one_round: bool = False) -> tuple[int, int]:
     """(tile, parts of K) for ``gemm_lds``: the least of what a launch is predicted to take.  A block's steps take its CU
     what the table says, the chip reads the weight at 9.1 TB/s (slower with fewer blocks than CUs: half of them, 6.7) and pulls
     31 TB/s of tiles at best; the fourth powers of the three add up.  Fitted to 35,000 launches (90 weights of 512 to 19,456 rows,
@@ -784,23 +781,22 @@ def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int =
     the reading rate, the tiles' rate and the cost of a part have values of their own (4,500 launches, 27 weights of 512 to
     34,816 rows, 1 to 16 rows of x: the picks take 2 % longer than the best in parts, 0.3 % whole).
     ``summed``: with what each part costs the consumer that adds them up (its reads at 5 TB/s).  ``one_round``: at most a block a CU
-    (the prediction is kind to a second round that is not whole).  ``gated``: a gate/up product's, which has tiles of its own (fitted
-    to 882 sizes of 192 to 1,024 rows: the picks take 0.7 % longer than the best, 8 % less than without them).
+    (the prediction is kind to a second round that is not whole).
 
     A plan takes 20 (whole) to 60 us (in parts) to find, which a portion of a new length would pay for every weight; a length
     makes as many tiles as the next multiple of 32, the smallest tile beyond 16 rows, so that is what plans are kept by (one
     length in 90 gets another plan than its own, by the prediction 1 % longer)."""
-    return _lds_plan(m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32, weight_rows, k, bytes_out, most_parts, summed, one_round, gated)
+    return _lds_plan(m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32, weight_rows, k, bytes_out, most_parts, summed, one_round)
 
 
 @functools.lru_cache(maxsize=4096)
-def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool, one_round: bool, gated: bool) -> tuple[int, int]:
+def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool, one_round: bool) -> tuple[int, int]:
     steps = k // 64
     best = None
     few = m <= SKINNY_MAX_ROWS
     consumer_us = 0.15 + m * weight_rows * 8e-7 if summed else 0.0
     read, alone, pull, store = (1.74e-7, 0.27, 8.8e-8, 1.33e-6) if few else (1.1e-7, 0.45, 3.27e-8, 3.05e-7)
-    for tile, (rows, columns, held, one, two) in (LDS_GATE_TILES if gated else LDS_TILES).items():
+    for tile, (rows, columns, held, one, two) in LDS_TILES.items():
         if few != (rows == 16):
             continue
         for parts in range(1, max(1, min(most_parts, steps // 4)) + 1):
@@ -922,39 +918,31 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     columns 56.5 against 60.5);
     17 to 64 rows one round (64 rows: 9,728 of 2,560 28.0 -> 25.2; 11,008 of 2,048 in 230 blocks of 64 x 96 26.5 -> 21.3), from K = 8,192
     and 8,192 columns on more (32 rows: 14,336 of 8,192 120 -> 92);
-    beyond, up to 1,536 rows, one round of the plan's blocks (1,700 sizes of 65 to 1,500 rows, 768 to 14,336 columns, K of 1,024 to 5,120;
-    time over that of what took them: one round .85 in the mean, more 1.17).  K up to 2,048: all of them (.81; 3,072 of 1,024 at 768 rows
-    23.4 -> 18.6 us, 6,144 of 2,048 at 480 rows 38.6 -> 31.5).  To 4,096: but for blocks of 128 x 256 (1.09) and, beyond 256 rows, up to
-    192 of at least 128 x 128 (512 rows: 3,072 of 2,560 1.04, 569: 4,096 of 2,560 1.10); the others .89 (9,728 of 2,560 at 80 rows 35.0
-    -> 26.0, at 256 52.5 -> 43.0, at 320 54.4 -> 44.5; 12,288 of 4,096 at 96 53.8 -> 41.8); nor, to 128 rows, under 160 blocks of 128 x
-    128 (9,728 of 2,560 at 128 rows ties alone, 36.0 against 34.9, and a whole prompt is 1 % slower).  To 5,120: beyond 256 rows only tiles that pull
-    little a column or leave the library's badly filled: not 96 x 128, 128 x 128, nor any of more than 128 rows or 160 weight rows
-    but 160 x 160 and 192 x 160 (the others .90, these 1.02 with up to 1.15).  Longer K, by the tiles of 128 x 160: to 256 rows from 512
-    columns on (256 of 8,192 at 80 rows 13.5 against 15.5), beyond that products too small for the library to fill the chip (1,536 of
-    4,096 at 320 rows 25.1 -> 21.3) or where these tiles nearly do (1,024 of 8,192 at 1,536 rows 59.5 against 70.8)."""
+    beyond, where tiles of 128 x 160 would make one round, up to 1,536 rows.  K up to 2,048: all of them (3,072 of 1,024 at 768 rows
+    23.4 -> 20.3, 256 of 1,024 at 1,100 rows 11.5 -> 6.6).  Larger K: to 256 rows one round of the plan's blocks (9,728 of 2,560 at
+    256 rows 52.5 -> 43.0, at 80 rows in 203 blocks of 96 x 96 35.0 -> 26.0; 12,288 of 4,096 at 96 rows 53.8 -> 41.8), but for few
+    columns at K > 5,120 (256 of 8,192 at 80 rows 13.5 against 15.5) and, to 128 rows, for under 160 blocks of 128 x 128, which tie
+    (128 rows: 9,728 of 2,560 36.0 against 34.9, 9,984 of 5,120 58.5 against 61.6; 184 blocks: 11,776 of 4,096 56.7 -> 49.9);
+    beyond that either products too small for the library to fill the chip (1,536 of 4,096 at 320 rows 25.1 -> 21.3) or
+    tiles of 128 x 160 that nearly do (4,864 of 4,096 at 320 rows 44.3 -> 39.9; 3,072 of 4,096 at 320 rows 33.6 against 37.7,
+    1,024 of 8,192 at 1,536 rows 59.5 against 70.8)."""
     weight_rows = 2 * columns
-    tile, _ = lds_plan(rows, weight_rows, k, weight_rows, gated=True)
-    blocks = -(-rows // LDS_GATE_TILES[tile][0]) * -(-weight_rows // LDS_GATE_TILES[tile][1])
+    tile, _ = lds_plan(rows, weight_rows, k, weight_rows)
+    blocks = -(-rows // LDS_TILES[tile][0]) * -(-weight_rows // LDS_TILES[tile][1])
     if rows <= SKINNY_MAX_ROWS:
         if GATE_HALF_FEW_ROWS_MAX_K < k <= 4096 and columns >= 4096 and (rows <= 4 or columns > 12288):
             return False
         return LDS_TILES[tile][2] == 2 or blocks <= WIDE_CUS or blocks > 1.6 * WIDE_CUS      # (a CU holds one block of the widest tile)
+    large_tiles = -(-rows // 128) * -(-weight_rows // 160)
+    if rows > LDS_GATE_MAX_ROWS or large_tiles > WIDE_CUS:
+        return False
     if rows <= MID_ROWS:
         return blocks <= WIDE_CUS or (k >= 8192 and columns >= 8192)
-    large_tiles = -(-rows // 128) * -(-weight_rows // 160)
-    if rows > LDS_GATE_MAX_ROWS or (blocks > WIDE_CUS and large_tiles > WIDE_CUS):
-        return False
     if k <= 2048 or not _library_fits(weight_rows, k):
         return True
-    if blocks > WIDE_CUS:
-        return False
-    if k > 5120:
-        return large_tiles <= WIDE_CUS and (columns >= 512 if rows <= 256 else rows * columns <= 600_000 or large_tiles >= 180)
     if rows <= 256:
-        return (k > 4096 or tile != 128256) and not (rows <= 128 and blocks < 160 and tile == 6)
-    if k <= 4096:
-        return tile != 128256 and (blocks > 192 or LDS_GATE_TILES[tile][0] * LDS_GATE_TILES[tile][1] < 128 * 128)
-    return tile not in (96128, 6, 128192, 128256, 192128)
+        return blocks <= WIDE_CUS and (columns >= 512 or k <= 5120) and not (rows <= 128 and blocks < 160 and LDS_TILES[tile][:2] == (128, 128))
+    return rows * columns <= 600_000 or large_tiles >= 180
 
 
 class UpdateProduct(NamedTuple):
@@ -1199,7 +1187,7 @@ def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int |
         code = 1 if ending == "bf16" else 2
     else:
         raise KernelError(f"no ending {ending!r} with {parts} parts")
-    if tile not in (LDS_GATE_TILES if ending == "gated" else LDS_TILES):
+    if tile not in LDS_TILES:
         raise KernelError(f"no tile {tile}")
     _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
           c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
@@ -1461,7 +1449,7 @@ def linear_swiglu(x: Tensor | UnscaledRows | SplitRows, gate_up_weight: Tensor, 
     ring = rows <= SKINNY_MAX_ROWS and _lds_fits(x, gate_up_weight) and _ring_fits(x, gate_up_weight, "gated")
     if (not to_library and gate_up_weight.shape[0] % 2 == 0 and _lds_fits(x, gate_up_weight)
             and _lds_gate_pays(rows, gate_up_weight.shape[0] // 2, gate_up_weight.shape[1])):
-        tile = None if ring else lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0], gated=True)[0]
+        tile = None if ring else lds_plan(rows, *gate_up_weight.shape, gate_up_weight.shape[0])[0]
         return gemm_lds(x, gate_up_weight, "gated", tile=tile, act=act)
     if ring and not to_library:
         return gemm_ring(x, gate_up_weight, "gated", act)

@@ -253,11 +253,10 @@ def test_which_gated_products_go_through_lds():
     taken = ((1, 3072, 1024), (8, 9728, 2560), (2, 2064, 2432), (983, 960, 2880), (128, 9728, 2496), (8, 17408, 5120), (16, 12288, 5120), (5, 4096, 4096), (5, 12288, 4096),
              (17, 9728, 2560), (64, 9728, 2560), (32, 14336, 8192), (65, 17408, 5120), (128, 6144, 2048), (256, 9728, 2560), (192, 9728, 2560),
              (384, 3072, 1024), (700, 3072, 1024), (1536, 256, 1024), (80, 512, 5184), (320, 1536, 4096), (320, 4864, 4096),
-             (64, 11008, 2048), (80, 9728, 2560), (96, 12288, 4096), (320, 9728, 2560), (320, 3072, 4096), (769, 3072, 1024),
-             (190, 14336, 2048), (480, 6144, 2048), (345, 9728, 5120))
+             (64, 11008, 2048), (80, 9728, 2560), (96, 12288, 4096), (128, 11776, 4096))
     left = ((8, 13824, 2560), (1, 14336, 2048), (4, 4096, 4096), (8, 17408, 4096), (64, 12352, 2048), (32, 16384, 4096),
-            (128, 9728, 2560), (640, 6144, 4096), (506, 3072, 2560), (80, 256, 8192), (640, 9728, 2560), (378, 4096, 5120), (1536, 1024, 8192),
-            (1537, 256, 1024), (4096, 256, 4096), (8192, 256, 8192), (1536, 4096, 1024))
+            (128, 9728, 2560), (128, 8448, 4096), (80, 256, 8192), (320, 9728, 2560), (320, 3072, 4096), (1536, 1024, 8192),
+            (1537, 256, 1024), (4096, 256, 4096), (8192, 256, 8192), (769, 3072, 1024))
     for size in taken:
         assert pays(*size), size
     for size in left:
@@ -527,7 +526,7 @@ def test_which_loads_pass_the_caches_is_known_when_a_product_is_compiled(tmp_pat
         if 2 * mi * wm % (wm * wn * kg) == 0:
             shapes.setdefault(re.match(r"(.*)Lb[01]EEE", name).group(1), set()).add((code.count("global_load_lds_dwordx4"), code.count("s_cbranch")))
     assert shapes and all(len(kinds) == 1 for kinds in shapes.values())
-    assert len(past) == 22 and all(kinds == {False, True} for kinds in past.values())
+    assert len(past) == 17 and all(kinds == {False, True} for kinds in past.values())
 
 
 def test_values_of_long_pages_stay_in_the_caches(tmp_path):

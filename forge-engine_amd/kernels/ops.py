@@ -867,26 +867,15 @@ def _lds_store_pays(rows: int, weight_rows: int, k: int) -> bool:
     """Products that store bfloat16.  Up to 8 rows where K is 2,048 and more and the weight has up to 8,192 rows, from five rows
     (8 rows: 6,144 x 2,048 9.2 -> 7.7 us, 2,048 x 2,048 5.5 -> 5.4, but 4,096 x 1,024 4.23 -> 4.28 and 12,288 x 2,048 12.4 ->
     12.8; 4 rows: 2,048 x 2,048 5.2 -> 5.4), 9 to 16 rows always (1,024 x 1,024 3.9 -> 3.7, 6,144 x 2,560 14.7 -> 9.6).
-    Beyond, up to 256 rows, 512 through weights of up to 4,096 rows, weights of 2,048 rows (1,024: 7.7 against 8.4 us at 192 rows) to
+    Beyond, up to 256 rows, 512 through weights of up to 4,096 rows (beyond, the library ties or
+    wins: 6,144 x 2,560 at 320 rows 18.6 against 19.9 us), weights of 2,048 rows (1,024: 7.7 against 8.4 us at 192 rows) to
     50 MB (10,240 x 5,120 at 64 rows 32.6 against 33.9).  Not through fewer than 3,584 rows at K > 5,120 beyond 192 rows
     (3,072 x 6,144 at 256 rows 28.8 against 31.4), nor through more at K >= 2,048 and 321 to 384 rows, which fill the library's
-    tiles (time over the library's: 3,584 x 2,560 at 356 rows 1.04, 4,096 x 2,048 .99, at 380 .94; at 320 and 448 rows .91 and .88).
-    Beyond these row counts, where the library's tiles of 128 and 256 rows are filled worst (time over the library's, 1,080 sizes):
-    through 3,072 to 4,096 rows up to 640 rows, 768 where K <= 2,048 or the weight has up to 3,584 rows (.66 to 1.02, mean .87; 4,096 x
-    2,048 at 576 rows 23.5 -> 19.0 us; to 1,024 rows .95 with 1.09 among them); through more 289 to 384 rows up to 7,168 rows, 10,240
-    where K <= 2,048 (.65 to 1.02, mean .85; 6,144 x 2,560 at 361 rows 27.9 -> 23.0; but 8,192 x 3,072 at 380 rows 1.08, 12,288 x 1,024
-    1.07 to 1.33), and where K <= 2,048 to 512 rows up to 8,192 and to 640 up to 6,144 (.78 to 1.03, mean .92; but 6,144 x 2,560 at 400 to
-    512 rows 1.04 to 1.09, 6,144 x 1,024 at 680 rows 1.33)."""
+    tiles (4,096 x 2,048 at 384 rows 14.8 against 16.7; at 320 and 448 rows 15.3 -> 14.8 and 17.1 -> 14.9)."""
     if rows <= SKINNY_MAX_ROWS:
         return rows > 8 or (rows > 4 and k >= 2048 and weight_rows <= 8192)
-    if weight_rows < 2048 or weight_rows * k > 26_000_000:
+    if weight_rows < 2048 or weight_rows * k > 26_000_000 or rows > (512 if weight_rows <= 4096 else 256):
         return False
-    if rows > (512 if weight_rows <= 4096 else 256):
-        if weight_rows <= 4096:
-            return weight_rows >= 3072 and k <= 4096 and rows <= (768 if k <= 2048 or weight_rows <= 3584 else 640)
-        if rows <= 384:
-            return rows > 288 and (weight_rows <= 7168 or (weight_rows <= 10240 and k <= 2048))
-        return k <= 2048 and rows <= (640 if weight_rows <= 6144 else 512 if weight_rows <= 8192 else 0)
     if not _library_fits(weight_rows, k):
         return True
     if weight_rows >= 3584:

@@ -293,12 +293,11 @@ def test_which_stored_products_go_through_lds():
 
 
 def test_which_products_of_portions_leave_the_library():
-    """Both sides of every line beyond 256 and 512 rows (rows, weight rows, K), see the rules."""
-    for size in ((513, 4096, 1024), (768, 4096, 2048), (640, 4096, 2560), (768, 3584, 4096), (513, 3072, 4096), (289, 6144, 2560), (384, 7168, 3072),
-                 (384, 10240, 2048), (385, 8192, 2048), (512, 8192, 1024), (640, 6144, 2048)):
+    """Both sides of the lines of 256 and 512 rows (rows, weight rows, K): beyond them all of these are the library's."""
+    for size in ((512, 4096, 1024), (512, 4096, 2560), (512, 3072, 4096), (256, 6144, 2560), (256, 10240, 2048)):
         assert ops._lds_store_pays(*size), size
-    for size in ((769, 4096, 2048), (641, 4096, 2560), (769, 3584, 4096), (513, 3056, 2048), (513, 3072, 4160), (288, 6144, 2560), (385, 6144, 2560),
-                 (384, 7424, 2560), (384, 10496, 1024), (513, 8192, 2048), (641, 6144, 1024), (400, 8448, 1024)):
+    for size in ((513, 4096, 1024), (768, 4096, 2048), (640, 4096, 2560), (768, 3584, 4096), (513, 3072, 4096), (257, 6144, 2560), (289, 6144, 2560),
+                 (384, 7168, 3072), (384, 10240, 2048), (385, 8192, 2048), (512, 8192, 1024), (640, 6144, 2048)):
         assert not ops._lds_store_pays(*size), size
 
 

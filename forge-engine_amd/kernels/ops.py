@@ -761,6 +761,11 @@ LDS_TILES = dict(enumerate((
     (64, 96, 2, 0.302, 0.6041), (128, 64, 1, 0.3322, 0.6643), (128, 128, 1, 0.5162, 1.0325), (128, 160, 1, 0.6269, 1.2538), (32, 64, 2, 0.1891, 0.35),
     (16, 16, 2, 0.073, 0.117), (16, 32, 2, 0.116, 0.247), (16, 48, 2, 0.143, 0.334), (16, 64, 2, 0.168, 0.444), (16, 80, 1, 0.220, 0.440))))
 LDS_TILES.update({96064: (96, 64, 1, 0.3087, 0.6173), 96096: (96, 96, 1, 0.3728, 0.7456), 96128: (96, 128, 1, 0.4775, 0.955)})
+# The same times as they stood when the parts of K and the gate/up products' line were drawn: see ``_lds_order``.
+LDS_ORDER_TILES = {**dict(enumerate((
+    (32, 32, 2, 0.151, 0.256), (64, 32, 1, 0.191, 0.382), (64, 64, 2, 0.212, 0.348), (64, 80, 1, 0.303, 0.606), (64, 96, 2, 0.292, 0.451),
+    (128, 64, 1, 0.317, 0.634), (128, 128, 1, 0.510, 1.02), (128, 160, 1, 0.630, 1.26), (32, 64, 2, 0.202, 0.378)))),
+    **{tile: LDS_TILES[tile] for tile in range(9, 14)}}
 LDS_HEAD_WEIGHT_ROWS = 131072  # float32 logits: see _lds_head_pays
 LDS_HEAD_MIN_K = 2048
 LDS_GATE_MAX_ROWS = 1536       # gate/up: measured up to here (4,096 rows, 256 columns of K = 4,096: 28.6 against 43.0 us)
@@ -771,50 +776,70 @@ UPDATE_NORM_MAX_WIDTH = 8192   # 32 weight rows a block
 
 def lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int = 1, summed: bool = False,
              one_round: bool = False) -> tuple[int, int]:
-    """(tile, parts of K) for ``gemm_lds``: the least of what a launch is predicted to take.  A block's steps take its CU
+    """(tile, parts of K) for ``gemm_lds``.  The parts are those of ``_lds_order``: they settle the order of a product's sums, and so its
+    bits.  The tile settles nothing but the time, and is the one with the least that a launch is predicted to take.  A block's steps take its CU
     what the table says, the chip reads the weight at 9.1 TB/s (slower with fewer blocks than CUs: half of them, 6.7) and pulls
     31 TB/s of tiles at best; the fourth powers of the three add up.  Fitted to 35,000 launches (90 weights of 512 to 19,456 rows,
     17 to 1,024 rows of x, every tile, 1 to 8 parts; as picks, one that takes more than 1 % longer than the one before counted three
-    times): the picks take 0.8 % longer than the best of these tiles, fitted to half of the weights 1.3 to 1.9 % in the other half.
-    Without the tiles of 96 rows the best would take 1.8 % longer, and the table and rates of before picked 1.8 % beside it (mean of
-    1,146 sizes; 25 % gain more than 2 %, 1.7 % lose as much).  Up to 16 rows
-    the reading rate, the tiles' rate and the cost of a part have values of their own (4,500 launches, 27 weights of 512 to
-    34,816 rows, 1 to 16 rows of x: the picks take 2 % longer than the best in parts, 0.3 % whole).
+    times): with parts of its own choice the picks take 0.8 % longer than the best of these tiles, fitted to half of the weights 1.3 to 1.9 %
+    in the other half.  Without the tiles of 96 rows the best would take 1.8 % longer.  Up to 16 rows the plan is that of ``_lds_order``.
     ``summed``: with what each part costs the consumer that adds them up (its reads at 5 TB/s).  ``one_round``: at most a block a CU
     (the prediction is kind to a second round that is not whole).
 
-    A plan takes 20 (whole) to 60 us (in parts) to find, which a portion of a new length would pay for every weight; a length
+    A plan takes 25 (whole) to 70 us (in parts) to find, which a portion of a new length would pay for every weight; a length
     makes as many tiles as the next multiple of 32, the smallest tile beyond 16 rows, so that is what plans are kept by (one
     length in 90 gets another plan than its own, by the prediction 1 % longer)."""
-    return _lds_plan(m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32, weight_rows, k, bytes_out, most_parts, summed, one_round)
+    return _lds_plan(_lds_length(m), weight_rows, k, bytes_out, most_parts, summed, one_round)
 
 
-@functools.lru_cache(maxsize=4096)
-def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool, one_round: bool) -> tuple[int, int]:
-    steps = k // 64
-    best = None
-    few = m <= SKINNY_MAX_ROWS
-    consumer_us = 0.15 + m * weight_rows * 8e-7 if summed else 0.0
-    read, alone, pull, store = (1.74e-7, 0.27, 8.8e-8, 1.33e-6) if few else (1.1e-7, 0.45, 3.27e-8, 3.05e-7)
-    for tile, (rows, columns, held, one, two) in LDS_TILES.items():
-        if few != (rows == 16):
+def _lds_length(m: int) -> int:
+    return m if m <= SKINNY_MAX_ROWS else -(-m // 32) * 32
+
+
+def _lds_least(tiles: dict, m: int, weight_rows: int, k: int, rates: tuple, parts_of, added_of, step_of, one_round: bool) -> tuple[int, int]:
+    """(tile, parts) with the least predicted time."""
+    steps, (read, alone, pull), best = k // 64, rates, None
+    for tile, (rows, columns, held, one, two) in tiles.items():
+        if (m <= SKINNY_MAX_ROWS) != (rows == 16):
             continue
-        for parts in range(1, max(1, min(most_parts, steps // 4)) + 1):
-            tiles = -(-m // rows) * -(-weight_rows // columns) * parts
-            if one_round and tiles > 256:
+        for parts in parts_of:
+            blocks = -(-m // rows) * -(-weight_rows // columns) * parts
+            if one_round and blocks > 256:
                 continue
-            rounds = -(-tiles // 256)
-            step = two * -(-rounds // 2) if few and held == 2 and rounds > 1 else one * (rounds % 2) + two * (rounds // 2)
-            walk = -(-steps // parts) * step
-            added = parts * (m * bytes_out * store + consumer_us + 0.05 * few)
+            part_steps, added = -(-steps // parts), added_of(parts)
+            walk = part_steps * step_of(-(-blocks // 256), held, one, two)
             if best is not None and walk + added >= best[0]:         # (the sum of powers is no less than its largest)
                 continue
-            bounds = (walk, weight_rows * k * 2 * read * (256 / min(256, tiles)) ** alone,
-                      tiles * -(-steps // parts) * (rows + columns) * 128 * pull)
+            bounds = (walk, weight_rows * k * 2 * read * (256 / min(256, blocks)) ** alone, blocks * part_steps * (rows + columns) * 128 * pull)
             us = sum(b ** 4 for b in bounds) ** 0.25 + added
             if best is None or us < best[0]:
                 best = (us, tile, parts)
     return best[1], best[2]
+
+
+@functools.lru_cache(maxsize=4096)
+def _lds_order(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool, one_round: bool) -> tuple[int, int]:
+    """(tile, parts) of a launch as the time of its steps was first fitted: 3,300 launches (25 weights of 1,024 to 17,408 rows, 17 to 1,024
+    rows of x, the tiles of 32 to 128 rows, 1 to 8 parts), the weight read at 5.4 TB/s, tiles pulled at 20; up to 16 rows the reading
+    rate, the tiles' rate and the cost of a part have values of their own (4,500 launches, 27 weights of 512 to 34,816 rows: the picks take 2 %
+    longer than the best in parts, 0.3 % whole).  What depends on it is what a result's bits depend on: how many parts of K a
+    product is summed in, and which gate/up products are rounded before the gate (``_lds_gate_pays``).  A better fit of the times moves both at
+    hundreds of sizes for 1 or 2 % of a launch, and every prompt's logits with them, so it chooses among tiles only."""
+    few = m <= SKINNY_MAX_ROWS
+    store = 1.33e-6 if few else 3.1e-7
+    consumer_us = 0.15 + m * weight_rows * 8e-7 if summed else 0.0
+    return _lds_least(LDS_ORDER_TILES, m, weight_rows, k, (1.74e-7, 0.27, 8.8e-8) if few else (1.84e-7, 0.35, 4.9e-8),
+                      range(1, max(1, min(most_parts, k // 64 // 4)) + 1), lambda parts: parts * (m * bytes_out * store + consumer_us + 0.05 * few),
+                      lambda rounds, held, one, two: one * rounds if held == 1 or rounds == 1 else two * -(-rounds // 2), one_round)
+
+
+@functools.lru_cache(maxsize=4096)
+def _lds_plan(m: int, weight_rows: int, k: int, bytes_out: int, most_parts: int, summed: bool, one_round: bool) -> tuple[int, int]:
+    order = _lds_order(m, weight_rows, k, bytes_out, most_parts, summed, one_round)
+    if m <= SKINNY_MAX_ROWS:
+        return order
+    return _lds_least(LDS_TILES, m, weight_rows, k, (1.1e-7, 0.45, 3.27e-8), order[1:], lambda parts: 0.0,
+                      lambda rounds, held, one, two: one * (rounds % 2) + two * (rounds // 2), one_round)
 
 
 def _lds_fits(x: Tensor, weight: Tensor) -> bool:
@@ -905,18 +930,19 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     70.9 -> 65.2; 346 blocks: 13,824 of 2,560 at 8 rows 28.9 against 33.4), and the weights of K = 4,096 from 4,096 columns at up to
     four rows and beyond 12,288 at more, whose blocks keep x in registers (1 row: 12,288 columns 37.4 against 38.9, 8 rows: 17,408
     columns 56.5 against 60.5);
-    17 to 64 rows one round (64 rows: 9,728 of 2,560 28.0 -> 25.2; 11,008 of 2,048 in 230 blocks of 64 x 96 26.5 -> 21.3), from K = 8,192
+    17 to 64 rows one round (64 rows: 9,728 of 2,560 28.0 -> 25.2; 344 blocks: 11,008 of 2,048 24.0 against 27.5), from K = 8,192
     and 8,192 columns on more (32 rows: 14,336 of 8,192 120 -> 92);
     beyond, where tiles of 128 x 160 would make one round, up to 1,536 rows.  K up to 2,048: all of them (3,072 of 1,024 at 768 rows
     23.4 -> 20.3, 256 of 1,024 at 1,100 rows 11.5 -> 6.6).  Larger K: to 256 rows one round of the plan's blocks (9,728 of 2,560 at
-    256 rows 52.5 -> 43.0, at 80 rows in 203 blocks of 96 x 96 35.0 -> 26.0; 12,288 of 4,096 at 96 rows 53.8 -> 41.8), but for few
-    columns at K > 5,120 (256 of 8,192 at 80 rows 13.5 against 15.5) and, to 128 rows, for under 160 blocks of 128 x 128, which tie
-    (128 rows: 9,728 of 2,560 36.0 against 34.9, 9,984 of 5,120 58.5 against 61.6; 184 blocks: 11,776 of 4,096 56.7 -> 49.9);
+    256 rows 52.5 -> 43.0; at 128 rows, 406 blocks, 35.3 against 40.3), but for few columns at K > 5,120 (256 of 8,192 at 80 rows
+    13.5 against 15.5);
     beyond that either products too small for the library to fill the chip (1,536 of 4,096 at 320 rows 25.1 -> 21.3) or
     tiles of 128 x 160 that nearly do (4,864 of 4,096 at 320 rows 44.3 -> 39.9; 3,072 of 4,096 at 320 rows 33.6 against 37.7,
-    1,024 of 8,192 at 1,536 rows 59.5 against 70.8)."""
+    1,024 of 8,192 at 1,536 rows 59.5 against 70.8).
+    The blocks are those of ``_lds_order``.  Tiles of 96 rows, or of 64 x 96, would bring more sizes into one round (9,728 of 2,560 at 80 rows 35.0
+    -> 26.0, 11,008 of 2,048 at 64 26.5 -> 21.3), but what takes them now rounds gate and up before the gate, so their results would change."""
     weight_rows = 2 * columns
-    tile, _ = lds_plan(rows, weight_rows, k, weight_rows)
+    tile, _ = _lds_order(_lds_length(rows), weight_rows, k, weight_rows, 1, False, False)
     blocks = -(-rows // LDS_TILES[tile][0]) * -(-weight_rows // LDS_TILES[tile][1])
     if rows <= SKINNY_MAX_ROWS:
         if GATE_HALF_FEW_ROWS_MAX_K < k <= 4096 and columns >= 4096 and (rows <= 4 or columns > 12288):
@@ -930,7 +956,7 @@ def _lds_gate_pays(rows: int, columns: int, k: int) -> bool:
     if k <= 2048 or not _library_fits(weight_rows, k):
         return True
     if rows <= 256:
-        return blocks <= WIDE_CUS and (columns >= 512 or k <= 5120) and not (rows <= 128 and blocks < 160 and LDS_TILES[tile][:2] == (128, 128))
+        return blocks <= WIDE_CUS and (columns >= 512 or k <= 5120)
     return rows * columns <= 600_000 or large_tiles >= 180
 
 

@@ -252,10 +252,9 @@ def test_which_gated_products_go_through_lds():
     pays = ops._lds_gate_pays
     taken = ((1, 3072, 1024), (8, 9728, 2560), (2, 2064, 2432), (983, 960, 2880), (128, 9728, 2496), (8, 17408, 5120), (16, 12288, 5120), (5, 4096, 4096), (5, 12288, 4096),
              (17, 9728, 2560), (64, 9728, 2560), (32, 14336, 8192), (65, 17408, 5120), (128, 6144, 2048), (256, 9728, 2560), (192, 9728, 2560),
-             (384, 3072, 1024), (700, 3072, 1024), (1536, 256, 1024), (80, 512, 5184), (320, 1536, 4096), (320, 4864, 4096),
-             (64, 11008, 2048), (80, 9728, 2560), (96, 12288, 4096), (128, 11776, 4096))
-    left = ((8, 13824, 2560), (1, 14336, 2048), (4, 4096, 4096), (8, 17408, 4096), (64, 12352, 2048), (32, 16384, 4096),
-            (128, 9728, 2560), (128, 8448, 4096), (80, 256, 8192), (320, 9728, 2560), (320, 3072, 4096), (1536, 1024, 8192),
+             (384, 3072, 1024), (700, 3072, 1024), (1536, 256, 1024), (80, 512, 5184), (320, 1536, 4096), (320, 4864, 4096))
+    left = ((8, 13824, 2560), (1, 14336, 2048), (4, 4096, 4096), (8, 17408, 4096), (64, 11008, 2048), (32, 16384, 4096),
+            (128, 9728, 2560), (96, 12288, 4096), (80, 256, 8192), (320, 9728, 2560), (320, 3072, 4096), (1536, 1024, 8192),
             (1537, 256, 1024), (4096, 256, 4096), (8192, 256, 8192), (769, 3072, 1024))
     for size in taken:
         assert pays(*size), size
@@ -299,6 +298,23 @@ def test_which_products_of_portions_leave_the_library():
     for size in ((513, 4096, 1024), (768, 4096, 2048), (640, 4096, 2560), (768, 3584, 4096), (513, 3072, 4096), (257, 6144, 2560), (289, 6144, 2560),
                  (384, 7168, 3072), (384, 10240, 2048), (385, 8192, 2048), (512, 8192, 1024), (640, 6144, 2048)):
         assert not ops._lds_store_pays(*size), size
+
+
+def test_parts_of_products_do_not_move_with_the_tiles_times(monkeypatch):
+    """How many parts of K a product is summed in settles its bits: pinned, and the same whatever the tiles are said to take."""
+    sizes = (((110, 1024, 2048), 4), ((130, 1024, 2048), 4), ((160, 1024, 3072), 4), ((256, 1024, 3072), 3), ((90, 2048, 2048), 3), ((300, 2048, 6144), 2),
+             ((700, 2048, 6144), 3), ((110, 2560, 9728), 3), ((130, 2560, 9728), 3), ((160, 2560, 9728), 3), ((64, 2560, 9728), ops._lds_update(64, 2560, 9728)[1]))
+    gates = ((80, 9728, 2560), (96, 12288, 4096), (64, 11008, 2048), (256, 9728, 2560), (361, 3072, 1024), (900, 3072, 1024))
+    routes = [ops._lds_gate_pays(*size) for size in gates]
+    assert routes == [False, False, False, True, True, False]
+    for times in (1.0, 0.5, 2.0):
+        monkeypatch.setattr(ops, "LDS_TILES", {tile: (rows, columns, held, one * times, two * (times if rows > 64 else 1.0))
+                                               for tile, (rows, columns, held, one, two) in ops.LDS_TILES.items()})
+        ops._lds_plan.cache_clear()
+        assert all(ops._lds_update(*size)[1] == parts for size, parts in sizes)
+        assert [ops._lds_gate_pays(*size) for size in gates] == routes
+    monkeypatch.undo()
+    ops._lds_plan.cache_clear()
 
 
 def test_plans_are_found_once_for_all_lengths_of_as_many_tiles():

@@ -194,10 +194,6 @@ static int launch_tile(const void* x, const void* w, void* out, int M, int N, in
 }
 
 // Operands and endings as fe_gemm_wide's (ending 0: parts, 1: bfloat16, 2: gated); the caller has checked them.
-// tile: rows of x x weight rows a block takes: 0: 32 x 32, 1: 64 x 32, 2: 64 x 64, 3: 64 x 80, 4: 64 x 96, 5: 128 x 64,
-//   6: 128 x 128, 7: 128 x 160, 8: 32 x 64, 9 to 13: 16 x 16, 32, 48, 64, 80; 96064, 96096, 96128: 96 x 64, 96, 128.
-static int launch(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
-                  int parts, long long part_stride, int tile, GateAct act, hipStream_t stream) {
 #define FE_END(END, ...) return launch_tile<__VA_ARGS__, END>(x, w, out, M, N, K, ldw, ldo, parts, part_stride, act, stream)
 #define FE_TILE(I, ...)                                                \
   case I:                                                              \
@@ -205,6 +201,11 @@ static int launch(const void* x, const void* w, void* out, int M, int N, int K, 
     else if (ending == END_BF16) FE_END(END_BF16, __VA_ARGS__);        \
     else if (ending == END_GATED) FE_END(END_GATED, __VA_ARGS__);      \
     break;
+// tile: rows of x x weight rows a block takes: 0: 32 x 32, 1: 64 x 32, 2: 64 x 64, 3: 64 x 80, 4: 64 x 96, 5: 128 x 64,
+//   6: 128 x 128, 7: 128 x 160, 8: 32 x 64, 9 to 13: 16 x 16, 32, 48, 64, 80.  (Templates: a source holds the tiles that it launches.)
+template <typename T>
+static int launch(const T* x, const T* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
+                  int parts, long long part_stride, int tile, GateAct act, hipStream_t stream) {
   switch (tile) {
     FE_TILE(0, 1, 2, 2, 1, 2, 10)
     FE_TILE(1, 2, 2, 2, 1, 2, 8)
@@ -220,17 +221,27 @@ static int launch(const void* x, const void* w, void* out, int M, int N, int K, 
     FE_TILE(11, 1, 1, 1, 3, 2, 9)
     FE_TILE(12, 1, 1, 1, 4, 2, 8)
     FE_TILE(13, 1, 1, 1, 5, 2, 10)
+  }
+  return FE_BAD_ARGUMENT;
+}
+
+// tile: 96064, 96096, 96128: 96 x 64, 96, 128.
+template <typename T>
+static int launch_96(const T* x, const T* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
+                     int parts, long long part_stride, int tile, GateAct act, hipStream_t stream) {
+  switch (tile) {
     FE_TILE(96064, 3, 2, 2, 2, 2, 4)
     FE_TILE(96096, 3, 3, 2, 2, 2, 4)
     FE_TILE(96128, 3, 4, 2, 2, 2, 4)
   }
-#undef FE_TILE
-#undef FE_END
   return FE_BAD_ARGUMENT;
 }
+#undef FE_TILE
+#undef FE_END
 
 // The bounded ending: tiles 9 to 13.
-static int launch_bounded(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int tile,
+template <typename T>
+static int launch_bounded(const T* x, const T* w, void* out, int M, int N, int K, long long ldw, long long ldo, int tile,
                           float limit, float alpha, hipStream_t stream) {
 #define FE_TILE(I, ...) \
   case I: return launch_tile<__VA_ARGS__, END_BOUNDED>(x, w, out, M, N, K, ldw, ldo, 1, 0, GateAct{alpha, limit}, stream);
@@ -247,7 +258,8 @@ static int launch_bounded(const void* x, const void* w, void* out, int M, int N,
 
 // The same for up to 16 rows of x with row factors: tiles 9 to 13, endings parts and gated.  Two buffers fewer where two blocks
 // share a CU's LDS, which the squares would keep from it.
-static int launch_scaled(const void* x, const void* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
+template <typename T>
+static int launch_scaled(const T* x, const T* w, void* out, int M, int N, int K, long long ldw, long long ldo, int ending,
                          int parts, long long part_stride, int tile, GateAct act, hipStream_t stream, RowFactors factors) {
 #define FE_END(END, ...) return launch_tile<__VA_ARGS__, END, true>(x, w, out, M, N, K, ldw, ldo, parts, part_stride, act, stream, factors)
 #define FE_TILE(I, ...)                                                \

@@ -261,7 +261,7 @@ extern "C" int fe_gemm_wide(const void* x, const void* w, void* out, int M, int 
   if (parts > 1 && part_stride < (long long)M * ldo) return FE_BAD_ARGUMENT;
   if (lds_tile >= 0) {
     if (ending == EPI_SWIGLU_HALF) return FE_BAD_ARGUMENT;
-    return through_lds::launch(x, w, out, M, N, K, ldw, ldo, ending, parts, part_stride, lds_tile, act, stream);
+    return through_lds::launch((const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldw, ldo, ending, parts, part_stride, lds_tile, act, stream);
   }
   const int steps = K / WSTEP;
   const int per_part = (steps + parts - 1) / parts;
@@ -314,7 +314,7 @@ extern "C" int fe_gemm_lds_bounded(const void* x, const void* w, void* out, int 
   if (M < 1) return FE_OK;
   if (N < 1 || K < WSTEP || K % WSTEP || ldw < K || ldw % 8 || ldo < N || !(limit > 0.f)) return FE_BAD_ARGUMENT;
   if ((((uintptr_t)x) & 15) || (((uintptr_t)w) & 15)) return FE_BAD_ARGUMENT;
-  return through_lds::launch_bounded(x, w, out, M, N, K, ldw, ldo, lds_tile, limit, alpha, stream);
+  return through_lds::launch_bounded((const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldw, ldo, lds_tile, limit, alpha, stream);
 }
 
 // Endings 0 and 2 through LDS for up to 16 rows of x whose norm's factors were left out: `squares` [M][256] float32 (fe_gemm_update_norm),
@@ -329,5 +329,5 @@ extern "C" int fe_gemm_lds_scaled(const void* x, const void* w, void* out, int M
   if (!squares || !(width > 0.f) || !(eps > 0.f) || ((((uintptr_t)x) | ((uintptr_t)w) | ((uintptr_t)squares)) & 15)) return FE_BAD_ARGUMENT;
   if ((ending != EPI_PARTS && ending != EPI_SWIGLU) || parts < 1 || parts > 64 || (ending != EPI_PARTS && parts != 1)) return FE_BAD_ARGUMENT;
   if (parts > 1 && part_stride < (long long)M * ldo) return FE_BAD_ARGUMENT;
-  return through_lds::launch_scaled(x, w, out, M, N, K, ldw, ldo, ending, parts, part_stride, lds_tile, act, stream, {squares, width, eps});
+  return through_lds::launch_scaled((const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldw, ldo, ending, parts, part_stride, lds_tile, act, stream, {squares, width, eps});
 }

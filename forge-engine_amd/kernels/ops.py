@@ -1204,9 +1204,12 @@ def gemm_lds(x: Tensor, weight: Tensor, ending: str, parts: int = 1, tile: int |
         raise KernelError(f"no ending {ending!r} with {parts} parts")
     if tile not in LDS_TILES:
         raise KernelError(f"no tile {tile}")
-    _call("gemm_wide", "fe_gemm_wide", _ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k),
-          c_longlong(weight.stride(0)), c_longlong(cols), c_int(code), c_int(parts), c_longlong(m * cols),
-          c_int(64), c_int(64), c_int(tile), _gate_act(act), _stream())
+    sizes = (_ptr(x), _ptr(weight), _ptr(out), c_int(m), c_int(cols), c_int(k), c_longlong(weight.stride(0)), c_longlong(cols), c_int(code),
+             c_int(parts), c_longlong(m * cols))
+    if LDS_TILES[tile][0] == 96:
+        _call("gemm_lds96", "fe_gemm_lds96", *sizes, c_int(tile), _gate_act(act), _stream())
+    else:
+        _call("gemm_wide", "fe_gemm_wide", *sizes, c_int(64), c_int(64), c_int(tile), _gate_act(act), _stream())
     return out
 
 
@@ -2106,7 +2109,7 @@ def sample_filtered_rows(logits: Tensor, params: Tensor, tokens: Tensor, status:
           _stream())
 
 
-LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_tile", "gemm_big", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
+LIBRARIES = ("rowwise", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_tile", "gemm_big", "qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_prefill", "sample")
 
 
 # ------------------------------------------------- ops on the stream, beside the matrix products

@@ -480,8 +480,8 @@ class GroupedQueryAttention(Mixer):
 
     def kernel_libraries(self):
         if self.general:
-            return {"whole_norm_rope" if self.whole_norm_eps is not None else "conv_rope", "attention_masked", "attention_decode", "attention_prefill", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
-        return {"qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_decode_f32", "attention_prefill", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+            return {"whole_norm_rope" if self.whole_norm_eps is not None else "conv_rope", "attention_masked", "attention_decode", "attention_prefill", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
+        return {"qk_rope", "attention_generic", "attention_f32", "attention_decode", "attention_decode_f32", "attention_prefill", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 register_part("mixer", "gqa_attention", GroupedQueryAttention)

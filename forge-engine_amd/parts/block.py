@@ -209,7 +209,7 @@ class ParallelBlock(Block):
         residual.add(update if self.feed_forward is None else self._with_feed_forward(x, update, batch))
 
     def kernel_libraries(self):
-        return {"gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big", "rowwise"}
+        return {"gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big", "rowwise"}
 
 
 def _side_by_side(a: Tensor | None, b: Tensor | None) -> Tensor | None:

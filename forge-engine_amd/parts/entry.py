@@ -55,7 +55,7 @@ class ConcatProjection(StreamEntry):
             residual.replace(fresh[0], fresh[1:] if fresh.shape[0] > 1 else None)
 
     def kernel_libraries(self):
-        return {"stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 class PassVectors(StreamEntry):

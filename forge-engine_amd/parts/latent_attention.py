@@ -224,7 +224,7 @@ class LatentAttention(Mixer):
         return self.position.token_inputs()
 
     def kernel_libraries(self):
-        return {"latent", "attention_latent", "attention_masked", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"latent", "attention_latent", "attention_masked", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 register_part("mixer", "latent_attention", LatentAttention)

@@ -79,7 +79,7 @@ class SwiGLU(FeedForward):
         ops.swiglu(z, out, self.activation)
 
     def kernel_libraries(self):
-        return {"rowwise", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big", "gemm_tile"}
+        return {"rowwise", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big", "gemm_tile"}
 
 
 class PolyNormMLP(FeedForward):
@@ -123,7 +123,7 @@ class PolyNormMLP(FeedForward):
         return ops.linear_update(act, self.down_weight)
 
     def kernel_libraries(self):
-        return {"stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 class ActivatedMLP(FeedForward):
@@ -164,7 +164,7 @@ class ActivatedMLP(FeedForward):
         return ops.linear_update(act, self.down_weight)
 
     def kernel_libraries(self):
-        return {"stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 register_part("feed_forward", "activated_mlp", ActivatedMLP)

@@ -222,7 +222,7 @@ class RoutedExperts(FeedForward):
                                extra=extra, form=self.form, weight_input=self.weight_input, plan=plan)
 
     def kernel_libraries(self):
-        return {"moe", "rowwise", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big", "gemm_tile"}
+        return {"moe", "rowwise", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big", "gemm_tile"}
 
 
 register_part("feed_forward", "routed_experts", RoutedExperts)

@@ -114,7 +114,7 @@ class _RecurrentMixer(Mixer):
         return CacheNeeds(state={self.STATE: FixedState(self.state_shape(), torch.float32)})
 
     def kernel_libraries(self):
-        return {"linear_recurrence", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"linear_recurrence", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 class RWKVTimeMix(_RecurrentMixer):
@@ -323,7 +323,7 @@ class Retention(_RecurrentMixer):
         return self.position.token_inputs()
 
     def kernel_libraries(self):
-        return {"head_recurrence", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"head_recurrence", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 register_part("mixer", "retention", Retention)

@@ -91,7 +91,7 @@ class SelectiveScanMixer(Mixer):
         return ops.linear_update(y, t["o"])
 
     def kernel_libraries(self):
-        return {"selective_scan", "conv_rope", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"selective_scan", "conv_rope", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 register_part("mixer", "selective_scan", SelectiveScanMixer)

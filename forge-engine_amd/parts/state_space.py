@@ -107,7 +107,7 @@ class StateSpaceMixer(Mixer):
         ops.gated_group_norm(y.view(-1, inner), z[:, :inner], t["norm"], out, groups=self.norm_groups, eps=self.eps)
 
     def kernel_libraries(self):
-        return {"head_recurrence", "selective_scan", "conv_rope", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_ring", "gemm_big"}
+        return {"head_recurrence", "selective_scan", "conv_rope", "stream_ops", "gemm_f32", "gemm_split", "gemm_planes", "gemm_skinny", "gemm_mid", "gemm_wide", "gemm_lds96", "gemm_ring", "gemm_big"}
 
 
 register_part("mixer", "state_space_duality", StateSpaceMixer)

@@ -541,7 +541,21 @@ def test_which_loads_pass_the_caches_is_known_when_a_product_is_compiled(tmp_pat
         if 2 * mi * wm % (wm * wn * kg) == 0:
             shapes.setdefault(re.match(r"(.*)Lb[01]EEE", name).group(1), set()).add((code.count("global_load_lds_dwordx4"), code.count("s_cbranch")))
     assert shapes and all(len(kinds) == 1 for kinds in shapes.values())
-    assert len(past) == 17 and all(kinds == {False, True} for kinds in past.values())
+    assert len(past) == 14 and all(kinds == {False, True} for kinds in past.values())
+
+
+def test_tiles_of_96_rows_pass_the_caches_for_one_tile_of_x_too(tmp_path):
+    """Every tile and ending of the library of these tiles has both instances, whose weight rows pass the caches and whose all stay."""
+    listing = tmp_path / "gemm_lds96.s"
+    flags = [flag for flag in build.HIPCC_FLAGS if flag != "-shared"]
+    subprocess.run([build.find_hipcc(), *flags, "-S", "--cuda-device-only", "-o", str(listing), str(build.SOURCE_DIR / "gemm_lds96.hip")],
+                   check=True, capture_output=True)
+    past = {}
+    for name, code in re.findall(r"^(_Z\w*gemm_lds_kernel\w+):(.*?)^\.Lfunc_end", listing.read_text(), re.M | re.S):
+        mi, ni, wm, wn, _, _, ending = (int(v) for v in re.findall(r"Li(\d+)E", name))
+        past.setdefault((16 * mi * wm, 16 * ni * wn, ending), set()).add(bool(re.search(r"global_load_lds_dwordx4 .*\bnt\b", code)))
+    assert set(past) == {tuple(ops.LDS_TILES[tile][:2]) + (ending,) for tile in ops.LDS_TILES if ops.LDS_TILES[tile][0] == 96 for ending in (0, 1, 2)}
+    assert all(kinds == {False, True} for kinds in past.values())
 
 
 def test_values_of_long_pages_stay_in_the_caches(tmp_path):

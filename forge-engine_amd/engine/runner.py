@@ -7,8 +7,6 @@ trace replay all go through ``ModelRunner.step``.
 
 from __future__ import annotations
 
-import time
-
 import numpy as np
 import torch
 from torch import Tensor
@@ -33,10 +31,13 @@ PORTION_GRAPH_SIGHTINGS = 2       # a shape is captured on this sighting ...
 PORTION_GRAPH_SIGHTINGS_PER = 128  # ... plus one for every so many tokens of the step
 # A step whose kernels take much longer than the host takes to launch them has little to gain: its launches are hidden behind the GPU's work
 # (a replay still saves some of the gaps between kernels, 250 us of 230 to 330 launches), and a capture in the middle of a queue waits for
-# it and then leaves the GPU idle while it records.  4B, 2,048 tokens: 16.4 ms of kernels against 6 of launches; a replay takes 16.2, a
-# capture costs 30 ms (runs of queued prompts in which captures fall 18.7 ms a pass, eager 16.5).  0.6B in float32, 700 tokens: 6.4
-# against 4.4, replays take 6.2.  Measured on a shape's last eager run, by the GPU's clock and the host's.
-PORTION_GRAPH_MAX_GPU_SHARE = 2.0
+# it and then leaves the GPU idle while it records (4B, 2,048 tokens: a replay takes 16.2 ms, eager 16.4, the step with the capture 45).
+# Known by the step's tokens times the matrix elements that a call multiplies a token with (``DecoderModel.products_per_token``), so that a step of a
+# shape is the same one wherever and whenever it runs.  Drawn where the GPU takes about twice as long as the host (ms, host and GPU; work): 4B 1,024 tokens 5.3, 10.6
+# (1.0e11), 1,536 5.3, 13.1 (1.6e11), 1.7B 2,560 tokens 4.9, 9.3 (1.3e11), 3,072 4.9, 11.2, 0.6B 4,096 tokens 4.9, 8.0 (6e10), two other designs at a width
+# of 2,048 1.8, 3.3 and 2.1, 4.0 (1.0e11), at twice the tokens 1.8, 5.7 and 2.1, 7.3; float32 0.6B 700 tokens 4.7, 6.5 (1.1e10), 1,500 4.3, 13.5 (2.4e10),
+# 1.7B 300 4.5, 7.8 (1.5e10), 500 4.5, 10.1 (2.5e10).
+PORTION_GRAPH_MAX_WORK = {torch.bfloat16: 1.3e11, torch.float32: 2e10}
 
 
 class _DecodeGraph:
@@ -173,48 +174,13 @@ class _PortionGraph:
             table_rows[n:] = -1
 
 
-class _PortionSeen:
-    """How often a shape of a step with prompt portions has come, and what its last eager run before a capture took: the host to launch it,
-    the GPU to run it (from its first kernel on, so a GPU that waits for launches takes as long as the host)."""
-
-    def __init__(self) -> None:
-        self.count = 0
-        self.host_ms = 0.0
-        self.events = None            # the GPU's times, once they have passed
-        self._hidden: bool | None = None
-
-    def run(self, forward):
-        """``forward()``, timed."""
-        stream, events = torch.cuda.current_stream(), [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        events[0].record(stream)
-        began = time.perf_counter()
-        result = forward()
-        self.host_ms = (time.perf_counter() - began) * 1e3
-        events[1].record(stream)
-        self.events = events
-        return result
-
-    def launches_hidden(self) -> bool:
-        """Whether the GPU hides the step's launches.  As long as it has not come to the end of the run that is timed, however often the
-        shape is back, it has work ahead of it."""
-        if self._hidden is None:
-            if self.events is None:
-                return False
-            begin, end = self.events
-            if not end.query():
-                return True
-            self._hidden = begin.elapsed_time(end) > PORTION_GRAPH_MAX_GPU_SHARE * self.host_ms
-            self.events = None
-        return self._hidden
-
-
 class ModelRunner:
     def __init__(self, model: DecoderModel, *, block_size: int, block_capacity: int | list[int] | tuple[int, ...],
                  num_state_slots: int, use_graphs: bool = True, eager_sightings: int | None = None) -> None:
         """``block_capacity``: pages of every cache group's pool, or one count per group (a group
         whose window bounds what a request holds needs fewer).  ``eager_sightings``: how often a shape of a step with prompt portions runs eagerly before
-        it is captured (None: by the step's size, see ``PORTION_GRAPH_SIGHTINGS``, and only if the GPU does not hide
-        its launches; a loop that repeats one shape, a benchmark for instance, passes 1)."""
+        it is captured (None: by the step's size, see ``PORTION_GRAPH_SIGHTINGS``, and not at all where the GPU hides its
+        launches, see ``PORTION_GRAPH_MAX_WORK``; a loop that repeats one shape, a benchmark for instance, passes 1)."""
         self.model = model
         self.eager_sightings = eager_sightings
         self.use_graphs = use_graphs and model.ctx.device.type == "cuda" and model.graph_safe
@@ -222,12 +188,12 @@ class ModelRunner:
         self._steady: _SteadyDecode | None = None
         self.steady_steps = 0
         self._portion_graphs: dict[tuple, _PortionGraph] = {}
-        self._portion_seen: dict[tuple, _PortionSeen] = {}
-        self._timed: _PortionSeen | None = None      # the eager step to come is timed for this shape
+        self._portion_seen: dict[tuple, int] = {}
         self.graph_replays = 0
         self.portion_graph_replays = 0
         self.device = model.ctx.device
         self.dtype = model.ctx.dtype
+        self._products_per_token = model.products_per_token()
         self.block_size = block_size
         self.token_inputs = model.token_inputs()     # per-token integers beside the positions, name -> width
         needs = model.cache_needs()
@@ -449,12 +415,16 @@ class ModelRunner:
             self._forward(batch, views, scratch_state=True)
         torch.cuda.current_stream(self.device).wait_stream(side)
 
+    def _launches_hidden(self, tokens: int) -> bool:
+        """Whether the GPU hides the launches of a step of so many tokens."""
+        return tokens * self._products_per_token > PORTION_GRAPH_MAX_WORK[self.dtype]
+
     def _portion_key(self, entries: list[StepEntry]):
         """The shape under which a step with prompt portions may be captured, or None."""
         if not self.use_graphs or len(entries) > GRAPH_MAX_REQUESTS:
             return None
         tokens = sum(len(e.tokens) for e in entries)
-        if tokens > PORTION_GRAPH_MAX_TOKENS:
+        if tokens > PORTION_GRAPH_MAX_TOKENS or (self.eager_sightings is None and self._launches_hidden(tokens)):
             return None
         seqs = -(-len(entries) // PORTION_GRAPH_SEQ_STEP) * PORTION_GRAPH_SEQ_STEP
         wanted = sum(len(e.want) for e in entries)
@@ -478,19 +448,14 @@ class ModelRunner:
         key = (*shape, widths)
         slot = self._portion_graphs.pop(key, None)
         if slot is None:
-            seen = self._portion_seen.pop(key, None) or _PortionSeen()
+            seen = self._portion_seen.pop(key, 0)
             if len(self._portion_seen) >= 4 * GRAPH_LIMIT:
                 self._portion_seen.pop(next(iter(self._portion_seen)))
-            self._portion_seen[key] = seen
+            self._portion_seen[key] = seen + 1
             eager = self.eager_sightings
             if eager is None:
                 eager = PORTION_GRAPH_SIGHTINGS - 1 + shape[0] // PORTION_GRAPH_SIGHTINGS_PER
-            if seen.count < eager:
-                seen.count += 1
-                if seen.count == eager and self.eager_sightings is None:
-                    self._timed = seen
-                return None
-            if self.eager_sightings is None and seen.launches_hidden():
+            if seen < eager:
                 return None
             if len(self._portion_graphs) >= GRAPH_LIMIT:
                 self._portion_graphs.pop(next(iter(self._portion_graphs)))
@@ -552,10 +517,8 @@ class ModelRunner:
             logits = self._portion_graph_step(entries, shape)
             if logits is not None:
                 return logits
-        timed, self._timed = self._timed, None
         batch = self.prepare(entries)
-        views = self.cache_views(batch)
-        logits = self._forward(batch, views) if timed is None else timed.run(lambda: self._forward(batch, views))
+        logits = self._forward(batch, self.cache_views(batch))
         for i, entry in enumerate(entries):
             self.cache.commit(entry.request_id, batch.ctx_before_host[i] + batch.q_lens[i])
         self.steps_run += 1

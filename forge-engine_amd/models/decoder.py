@@ -96,6 +96,11 @@ class DecoderModel:
                     raise ValueError(f"parts ask for the token input '{name}' at widths {asked[name]} and {width}")
         return asked
 
+    def products_per_token(self) -> float:
+        """Matrix elements that a token is multiplied with in a layer's call, the mean over a step's calls."""
+        each = [sum(part.products_per_token() for part in layer.children()) for layer in self.layers]
+        return sum(each[call.layer] for call in self.schedule) / max(1, len(self.schedule))
+
     def cache_needs(self) -> list[CacheNeeds]:
         """One entry per schedule call (what its mixer asks of the cache)."""
         return [self.layers[call.layer].cache_needs() for call in self.schedule]

@@ -16,6 +16,7 @@ which model it is in.  Roles:
 
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 from typing import Any
 
@@ -230,6 +231,10 @@ class Part:
         """Checkpoint name -> spec, for every tensor this part (and its
         sub-parts) reads."""
         return {}
+
+    def products_per_token(self) -> int:
+        """Elements of the matrices that a token is multiplied with in one call."""
+        return sum(math.prod(spec.shape) for spec in self.param_specs().values() if spec.kind == "matrix")
 
     def set_param(self, name: str, tensor: Tensor) -> None:
         """Receive one loaded tensor (already on the device, already in the

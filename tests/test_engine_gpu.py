@@ -393,6 +393,38 @@ def test_steps_with_portions_replay_captured_graphs(name, dtype, folders):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_steps_whose_launches_the_gpu_hides_stay_eager(dtype, folders, monkeypatch):
+    """The same prompt over and over without a wait between the steps, on both sides of the line that decides about its capture: below it the
+    shape is captured on its second sighting, beyond it never, and whoever runs it (twice each) finds the same bits, the same
+    lengths in the cache and as many replays.  A step that repeats one shape on purpose is captured beyond it too."""
+    from forge_engine_amd.engine import runner as engine_runner
+
+    config, weights = TINY["C"], folder_weights(folders["C"])
+    prompt = ru.make_requests(config, 44, (40,))
+    want = {k: plain.forward(weights, config, v)[-1] for k, v in prompt.items()}
+    (name, tokens), = prompt.items()
+    _, model = load_model(folders["C"], dtype=dtype, device=DEV)
+    work = len(tokens) * model.products_per_token()
+    scale = float(want[name].abs().max())
+    bound = 1e-4 * scale + 1e-5 if dtype == "float32" else ru.BF16_FRACTION * scale
+    for line, sightings, replays in ((work, None, 5), (work - 1, None, 0), (work - 1, 1, 5)):
+        monkeypatch.setitem(engine_runner.PORTION_GRAPH_MAX_WORK, getattr(torch, dtype), line)
+        runs = []
+        for _ in range(2):
+            runner = ModelRunner(model, block_size=16, block_capacity=8, num_state_slots=2, eager_sightings=sightings)
+            logits = []
+            for _ in range(6):
+                runner.begin(name)
+                logits.append(runner.step([StepEntry(name, tokens, [len(tokens) - 1])]).clone())
+                assert runner.length(name) == len(tokens)
+                runner.end(name)
+            assert runner.portion_graph_replays == replays and runner.steps_run == 6 and runner.cache.allocated_pages == 0
+            runs.append(torch.cat(logits).cpu())
+        assert torch.equal(*runs)
+        assert float((runs[0] - want[name]).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_steps_of_a_hundred_requests_with_portions_replay_captured_graphs(dtype, folders):
     """Steps of more than 64 requests that hold prompt portions beside decoded tokens are captured
     too: 90 requests, ten of which bring portions of 5 tokens in every step while the others bring

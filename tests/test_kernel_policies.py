@@ -615,26 +615,36 @@ def test_rows_of_decode_steps_are_turned_away_unseen():
     assert ops._big_update_parts(2048, 2560, 8128) == 0 and ops._big_update_parts(2048, 2560, 8192) == 3
 
 
-@pytest.mark.parametrize("gpu_ms,host_ms,hidden", [(16.2, 6.0, True), (12.1, 6.0, True), (11.9, 6.0, False), (5.2, 6.0, False)])
-def test_steps_whose_launches_the_gpu_hides_are_not_captured(gpu_ms, host_ms, hidden):
-    """Both sides of the line; while the GPU has not come to the end of the timed run nothing is decided, and what was found once is kept."""
-    class Event:
-        passed = False
+@pytest.mark.parametrize("elements,dtype,captured,hidden", [
+    (100_925_440, "bfloat16", 1288, 1289), (50_331_648, "bfloat16", 2582, 2583), (15_728_640, "bfloat16", 4096, 8266),
+    (15_728_640, "float32", 1271, 1272), (50_331_648, "float32", 397, 398)])
+def test_steps_whose_launches_the_gpu_hides_are_known_by_their_size(elements, dtype, captured, hidden):
+    """Both sides of the line, by the tokens and the model alone: no clock has a say in which of two forms of a step runs."""
+    import types
 
-        def query(self):
-            return self.passed
+    import torch
 
-        def elapsed_time(self, end):
-            return gpu_ms
+    step = types.SimpleNamespace(_products_per_token=elements, dtype=getattr(torch, dtype))
+    assert not runner.ModelRunner._launches_hidden(step, captured) and runner.ModelRunner._launches_hidden(step, hidden)
 
-    seen, events = runner._PortionSeen(), [Event(), Event()]
-    assert not seen.launches_hidden()            # never run
-    seen.host_ms, seen.events = host_ms, events
-    assert seen.launches_hidden() and seen.launches_hidden()
-    events[1].passed = True
-    assert seen.launches_hidden() == hidden
-    seen.events = None
-    assert seen.launches_hidden() == hidden
+
+def test_products_per_token_count_what_a_token_is_multiplied_with():
+    """A layer's matrices, of the experts those that a token is sent to; no lookups, no norms, no head."""
+    import torch
+
+    from forge_engine_amd.config import load_model_config
+    from forge_engine_amd.engine import build_model
+    from forge_engine_amd.parts.base import BuildContext
+    from forge_engine_amd.parts.moe import RoutedExperts
+
+    dense = {"architectures": ["Qwen3ForCausalLM"], "model_type": "qwen3", "hidden_act": "silu", "vocab_size": 320, "hidden_size": 96,
+             "intermediate_size": 160, "num_hidden_layers": 3, "num_attention_heads": 6, "num_key_value_heads": 2, "head_dim": 64,
+             "max_position_embeddings": 128, "rms_norm_eps": 1e-6, "rope_theta": 10000.0, "tie_word_embeddings": False, "eos_token_id": None}
+    model = build_model(load_model_config(dense), dtype="bfloat16", device=torch.device("cpu"))
+    assert model.products_per_token() == 96 * (6 + 2 + 2) * 64 + 6 * 64 * 96 + 3 * 96 * 160
+    ctx = BuildContext(torch.device("cpu"), torch.bfloat16)
+    experts = RoutedExperts(ctx, "m", hidden_size=48, experts=8, top=2, intermediate_size=80, limit=1.0, shared_size=32)
+    assert experts.products_per_token() == 8 * 48 + 2 * 3 * 48 * 80 + 3 * 48 * 32
 
 
 def test_float32_decode_attention_sizes_and_splits():

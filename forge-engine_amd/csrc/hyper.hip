@@ -235,7 +235,8 @@ static void launch_hyper(float* streams, long long stream_stride, const float* u
   const size_t lds = out ? (size_t)W * sizeof(float) : 0;
   const bool vec = W % 4 == 0 && ((uintptr_t)streams % 16 == 0) && stream_stride % 4 == 0 &&
                    (!update || ((uintptr_t)update % 16 == 0 && part_stride % 4 == 0));
-  // (the threads of a row, and with them the order of its sums, are those of the launches below)
+  // (The order of a row's sums is that of the launches below.  A row of 2,048 in few rows has 512 threads here and 1,024 there: theirs beyond find
+  // nothing behind the row's end, and what their waves add to the sums are zeros behind the others.)
   const bool few = n_rows <= 512 && W >= 2048;
   if (vec && parts <= EARLY_PARTS && W <= (few ? 4096 : 2048)) {
 #define FE_EARLY(THREADS, ROUNDS)                                                                                              \

@@ -337,7 +337,9 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_early_kernel(
 }
 constexpr int EARLY_PARTS = 8;
 
-// Rows of up to 4,096 elements in the threads, and with them the order of sums, of the launches below.
+// Rows of up to 4,096 elements.  The order of a row's sums is that of the launches below: an element belongs to the same lane, wave and round as there, and
+// where those have more threads (256 or 1,024 for a row of fewer fours) or rounds (four for 2,560), they find nothing behind the row's end and
+// add zeros behind the others.
 template <typename TO, bool SPLIT>
 static void launch_add_rmsnorm_early(float* h, const float* delta, const float* w, TO* out, const int* rows, int n_rows, int hidden, float eps,
                                      int store_sum, int parts, size_t part_stride, hipStream_t stream, bf16_t* planes) {

@@ -60,6 +60,41 @@ def test_hyper_norm_kernel(streams, width, parts, dtype):
         close(got_x, want_x, torch.float32)
 
 
+@pytest.mark.parametrize("rows", [8, 37, 513, 600])          # up to 512 rows of 2,048 and more take more threads a row
+@pytest.mark.parametrize("streams,width", [(1, 1024), (4, 1024), (4, 1028), (3, 2044), (1, 2048), (4, 2048), (4, 2052), (2, 4096), (4, 4096), (2, 4100)])
+def test_hyper_norm_has_the_bits_of_the_general_kernel(streams, width, rows):
+    """Rows with an update in up to four parts go to a kernel that requests all of a row's operands before it uses any; with a fifth part
+    (of zeros here) they go to the general one.  The same bits in the streams and in the rows, on both sides of every line between
+    instances, with and without each operand that may be absent; and the plain reference's values, five parts of numbers among them."""
+    from forge_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(streams * 10000 + width + rows)
+    mix = torch.eye(streams) + 0.2 * torch.randn(streams, streams, generator=g)
+    share, read = torch.randn(streams, generator=g), torch.randn(streams, generator=g)
+    weight, bias, shift = 1 + 0.1 * torch.randn(width, generator=g), 0.1 * torch.randn(width, generator=g), torch.randn(width, generator=g)
+    dev = lambda t: None if t is None else t.to(DEV)
+    for parts in (0, 1, 2, 4, 5):
+        x = torch.randn(streams, rows, width, generator=g) * 3
+        update = torch.randn(parts, rows, width, generator=g) if parts else None
+        five = torch.zeros(5, rows, width)
+        if parts:
+            five[:parts] = update
+        for use_mix, use_read, rms, use_shift, dtype in ((True, True, False, False, torch.bfloat16), (False, False, True, True, torch.float32),
+                                                         (True, False, False, True, torch.float32), (False, True, True, False, torch.bfloat16)):
+            use_mix = use_mix and (parts > 0 or use_shift)      # without either the streams are left as they are
+            rest = (mix if use_mix else None, share if use_mix else None, read if use_read else None, weight, None if rms else bias)
+            results = []
+            for brought in (update, five):
+                got_x, out = dev(x).clone(), torch.full((rows, width), float("nan"), dtype=dtype, device=DEV)
+                ops.hyper_norm(got_x, dev(brought), *(dev(t) for t in rest), 1e-5, out, rms=rms, shift=dev(shift if use_shift else None))
+                results.append((got_x, out))
+            for here, there in zip(*results):
+                assert torch.equal(here.view(torch.int16), there.view(torch.int16)), (parts, use_mix, use_read, rms, use_shift)
+            want_x = x.clone()
+            want = refs.hyper_norm(want_x, update, *rest, 1e-5, torch.empty(rows, width, dtype=dtype), rms=rms, shift=shift if use_shift else None)
+            close(results[0][1], want, dtype)
+            close(results[0][0], want_x, torch.float32)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_token_pair_embedding_kernel(dtype):
     from forge_engine_amd.kernels import ops

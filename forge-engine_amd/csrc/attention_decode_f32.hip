@@ -5,8 +5,16 @@
 // wave has for one block (requests of whole lines, waits counted by hand).  Scores transposed, S^T = K Q^T, and output transposed,
 // O^T = V^T P^T, on the float32 MFMA 16x16x4 with the group's query rows padded to 16: lane (r = l % 16, q = l / 16) supplies a
 // key's dims 16 i + 4 q + e (of the keys and of the queries: which four dims an instruction takes does not matter), receives the scores of keys
-// 4 q .. + 3 of row r, and these are, after the softmax, what it supplies to the second product.  A dot product is four chains of
-// D / 16 instructions each.
+// 4 q .. + 3 of row r, and these are, after the softmax, what it supplies to the second product.
+//
+// An error that grows with the length of a chain of sums is what separates this from the kernel for all sizes, whose dot products are trees over
+// lanes: so a dot product is sixteen chains of D / 64 instructions, added up as a tree, a block's share of the output is summed from zero and joins the
+// run's in one rounding, the exponent takes the scale and the maximum in one, and waves and splits are added up as trees too.  Relative error of 24 launches each of 1 to 8 sequences, 16 heads on
+// 8, against 64 bits, the kernel for all sizes -> this: 60 to 200 keys 1.54e-7 -> 1.52e-7, 200 to 1,000 1.64 -> 1.61, 1,000 to 8,000 2.07 ->
+// 1.84, with scores four times as large 2.69 -> 2.56, 3.52 -> 3.07, 4.15 -> 3.80.  Heads of 64, whose dot products are short (and whose shares are
+// two chains for it), 8 on one, 1.34 -> 1.42, 1.54 -> 1.48, 1.96 -> 1.73, 2.52 -> 2.62, 2.77 -> 2.87, 3.66 -> 3.53.  (Dot products in four chains and
+// everything else in a row: 1.95, 2.11, 2.67, 3.64, 4.40, 5.48 with heads of 128, and 4 sequences of 90 to 600 keys 10.0 us where this
+// takes 10.3, 1 of 8,000 18.6 and 19.5.)
 //
 // On the way the block's heads are normalised and rotated, in the arithmetic of the stand-alone kernel (rope_math.h), four elements a
 // lane, and the last split's last wave writes the new key and value to their pages and treats them as a partial result of their own.
@@ -15,8 +23,8 @@
 //
 // Bound by latency where contexts are short (start, keys and values, merge one after the other), by the cache's bytes where they are long.
 // What it saves are two launches and the trips between them (rotation 4.8, attention 9 and its merge 6.6 us at 4 sequences of 90 to 600
-// keys): float32 steps of 1.7B at 4 requests of 90 to 600 tokens 2,087 -> 1,826 us, at 1 of 8,000 2,690 -> 2,058, of 0.6B at 1 of 217 1,349 ->
-// 1,139, 8 of 300 to 800 1,658 -> 1,344, 2 of 2,000 to 4,000 2,041 -> 1,400.
+// keys): float32 steps of 1.7B at 4 requests of 90 to 600 tokens 2,090 -> 1,845 us, at 1 of 8,000 2,684 -> 2,089, of 0.6B at 1 of 217 1,349 -> 1,151, 8 of 300 to 800
+// 1,714 -> 1,406, 2 of 2,000 to 4,000 2,117 -> 1,422.
 #include "agent_access.h"
 #include "common.h"
 #include "lds_load.h"
@@ -30,6 +38,7 @@ using lds_tile::floatx4;
 using lds_tile::uintx4;
 
 constexpr int KEYS = 16, WAVES = 4, GMAX = 8;
+constexpr int CHAINS = 16;      // that a dot product is summed in
 constexpr int ROUND = 8;        // splits that the merge reads at a time
 
 template <int D>
@@ -37,6 +46,7 @@ struct Slot {
   static constexpr int LPH = D / 4;                                  // lanes that share a head
   static constexpr int ROUNDS = ((GMAX + 2) * LPH + 255) / 256;      // how often the block's lanes take heads
   static constexpr int LOADS = D / 16;                               // requests of 1,024 bytes: a block's keys, and its values
+  static constexpr int SHARES = D == 64 ? 2 : 1;                     // chains that a block's share of the output is summed in
   static constexpr int VALUES_AT = LOADS * 1024, BYTES = 2 * VALUES_AT;      // the heads come to the values' place before them
   static_assert(ROUNDS <= LOADS, "heads in the values' place");
 };
@@ -223,15 +233,22 @@ __global__ __launch_bounds__(256, 2) void paged_decode_f32_kernel(
     for (int i = 0; i < LOADS; ++i) k4[i] = __builtin_bit_cast(floatx4, slot[lr * CPR + ((4 * i + lq) ^ (lr & 7))]);
     reads_done();
     if (goes_on) request_keys(b + WAVES, next);
-    floatx4 st[4];
+    floatx4 st[CHAINS];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) st[e] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < CHAINS; ++c) st[c] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) st[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[i][e], qb[i][e], st[e], 0, 0, 0);
+      for (int e = 0; e < 4; ++e) {
+        floatx4& sum = st[(4 * i + e) % CHAINS];
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[i][e], qb[i][e], sum, 0, 0, 0);
+      }
     // lane (lr = query row, lq): score of key b * 16 + 4 lq + i
-    const floatx4 scores = (st[0] + st[1]) + (st[2] + st[3]);
+#pragma unroll
+    for (int half = CHAINS / 2; half > 0; half >>= 1)
+#pragma unroll
+      for (int c = 0; c < half; ++c) st[c] += st[c + half];
+    const floatx4 scores = st[0];
     const int key0 = b * KEYS + 4 * lq;
     float s[4], mx = -INFINITY;
     bool owned[4];
@@ -247,7 +264,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_f32_kernel(
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      s[i] = expf(s[i] - m_use);
+      s[i] = owned[i] ? expf(fmaf(scores[i], scale, -m_use)) : 0.f;
       sum += s[i];
     }
     l_run = fmaf(l_run, corr, sum_xor32(sum_xor16(sum)));
@@ -264,10 +281,17 @@ __global__ __launch_bounds__(256, 2) void paged_decode_f32_kernel(
     }
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-      o[t] *= corr;
+      floatx4 share[S::SHARES];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)       // slots that no key in reach owns may hold anything: their values count as zero
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(owned[i] ? va[t][i] : 0.f, s[i], o[t], 0, 0, 0);
+      for (int i = 0; i < S::SHARES; ++i) share[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {     // slots that no key in reach owns may hold anything: their values count as zero
+        floatx4& sum = share[i * S::SHARES / 4];
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(owned[i] ? va[t][i] : 0.f, s[i], sum, 0, 0, 0);
+      }
+      if constexpr (S::SHARES == 2) share[0] += share[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[t][i] = fmaf(o[t][i], corr, share[0][i]);
     }
   }
   if (splits == 1) write_pages();
@@ -286,12 +310,14 @@ __global__ __launch_bounds__(256, 2) void paged_decode_f32_kernel(
     for (int w = 0; w < WAVES; ++w) m_tot = fmaxf(m_tot, Ms[w][g]);
     float ov = 0.f, l = 0.f;
     if (m_tot > -INFINITY) {
+      float f[WAVES], part[WAVES];
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) {
-        const float f = expf(Ms[w][g] - m_tot);
-        ov += f * ((const float*)(slots + w * (S::BYTES / 16)))[g * D + d];
-        l += f * Ls[w][g];
+        f[w] = expf(Ms[w][g] - m_tot);
+        part[w] = ((const float*)(slots + w * (S::BYTES / 16)))[g * D + d];
       }
+      ov = fmaf(f[0], part[0], f[1] * part[1]) + fmaf(f[2], part[2], f[3] * part[3]);
+      l = fmaf(f[0], Ls[0][g], f[1] * Ls[1][g]) + fmaf(f[2], Ls[2][g], f[3] * Ls[3][g]);
       if (extra) {
         const float f = expf(Ms[WAVES][g] - m_tot);
         ov += f * heads_s[(groups + 1) * PITCH + d];
@@ -338,14 +364,21 @@ __global__ __launch_bounds__(256, 2) void paged_decode_f32_kernel(
 #pragma unroll
         for (int i = 0; i < ROUND; ++i) m_new = fmaxf(m_new, m[i]);
         const float m_use = m_new > -INFINITY ? m_new : 0.f, corr = expf(m_tot - m_use);
-        l_tot *= corr;
-        ov *= corr;
 #pragma unroll
         for (int i = 0; i < ROUND; ++i) {
           const float f = base + i < splits ? expf(m[i] - m_use) : 0.f;
-          l_tot = fmaf(f, l[i], l_tot);
-          ov = fmaf(f, part[i], ov);
+          l[i] *= f;
+          part[i] *= f;
         }
+#pragma unroll
+        for (int half = ROUND / 2; half > 0; half >>= 1)
+#pragma unroll
+          for (int i = 0; i < half; ++i) {
+            l[i] += l[i + half];
+            part[i] += part[i + half];
+          }
+        l_tot = fmaf(l_tot, corr, l[0]);
+        ov = fmaf(ov, corr, part[0]);
         m_tot = m_new;
       }
       out[(size_t)q0 * out_stride + (size_t)(hk * groups + g) * D + d] = l_tot > 0.f ? ov / l_tot : 0.f;

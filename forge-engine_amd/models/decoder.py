@@ -34,8 +34,11 @@ class DecoderModel:
             self.head.tie(self.embedding)
         self._owners: dict[str, Part] = {}
         self._specs: dict[str, ParamSpec] = {}
+        self._products: dict[Part, int] = {}      # matrix elements that a token is multiplied with in the part
         for part in self.parts():
-            for name, spec in part.param_specs().items():
+            specs = part.param_specs()
+            self._products[part] = part.products_per_token(specs)
+            for name, spec in specs.items():
                 if name in self._owners:
                     raise ValueError(f"tensor name '{name}' is claimed by two parts")
                 self._owners[name] = part
@@ -98,7 +101,7 @@ class DecoderModel:
 
     def products_per_token(self) -> float:
         """Matrix elements that a token is multiplied with in a layer's call, the mean over a step's calls."""
-        each = [sum(part.products_per_token() for part in layer.children()) for layer in self.layers]
+        each = [sum(self._products[part] for part in layer.children()) for layer in self.layers]
         return sum(each[call.layer] for call in self.schedule) / max(1, len(self.schedule))
 
     def cache_needs(self) -> list[CacheNeeds]:

@@ -232,9 +232,9 @@ class Part:
         sub-parts) reads."""
         return {}
 
-    def products_per_token(self) -> int:
-        """Elements of the matrices that a token is multiplied with in one call."""
-        return sum(math.prod(spec.shape) for spec in self.param_specs().values() if spec.kind == "matrix")
+    def products_per_token(self, specs: dict[str, ParamSpec]) -> int:
+        """Elements of the matrices that a token is multiplied with in one call; ``specs``: what ``param_specs`` gave."""
+        return sum(math.prod(spec.shape) for spec in specs.values() if spec.kind == "matrix")
 
     def set_param(self, name: str, tensor: Tensor) -> None:
         """Receive one loaded tensor (already on the device, already in the

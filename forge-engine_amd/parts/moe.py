@@ -125,10 +125,10 @@ class RoutedExperts(FeedForward):
                 self._owners[self._expert_name(expert, which)] = (expert, which)
         return specs
 
-    def products_per_token(self) -> int:
+    def products_per_token(self, specs) -> int:
         """Of the experts those that a token is sent to."""
         expert = (self.matrices + 1) * self.intermediate_size * self.hidden_size
-        return super().products_per_token() - (self.experts - self.top) * expert
+        return super().products_per_token(specs) - (self.experts - self.top) * expert
 
     def set_param(self, name: str, tensor: Tensor) -> None:
         f, h = self.intermediate_size, self.hidden_size

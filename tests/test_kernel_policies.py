@@ -644,7 +644,7 @@ def test_products_per_token_count_what_a_token_is_multiplied_with():
     assert model.products_per_token() == 96 * (6 + 2 + 2) * 64 + 6 * 64 * 96 + 3 * 96 * 160
     ctx = BuildContext(torch.device("cpu"), torch.bfloat16)
     experts = RoutedExperts(ctx, "m", hidden_size=48, experts=8, top=2, intermediate_size=80, limit=1.0, shared_size=32)
-    assert experts.products_per_token() == 8 * 48 + 2 * 3 * 48 * 80 + 3 * 48 * 32
+    assert experts.products_per_token(experts.param_specs()) == 8 * 48 + 2 * 3 * 48 * 80 + 3 * 48 * 32
 
 
 def test_float32_decode_attention_sizes_and_splits():

@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
 
   // PREPARE: the block's query heads, key head and value head are finished once, eight elements a lane, and handed to all waves through
   // LDS (every wave for itself, all of the heads in the layout of its operand: .7 us a launch where this is .4; 1 sequence of 1,000 keys
-  // 9.5 -> 8.6 us, 8 of 100 7.4 -> 6.4, the step of 0.6B at 1 request 768 -> 756).
+  // 9.5 -> 8.6 us, 8 of 100 7.4 -> 6.4, the step of 0.6B at 1 request, with the keys through LDS, 769 -> 760).
   constexpr int LPH = Slot::LPH, ROUNDS = Slot::ROUNDS, LOADS = Slot::LOADS;
   constexpr int PITCH = D + 8;                       // of a finished head in LDS: neighbouring heads' chunks in different banks
   __shared__ float cos_s[PREPARE ? D / 2 : 1], sin_s[PREPARE ? D / 2 : 1];
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void paged_decode_kernel(
 
   // The new token's key and value go to their pages behind the last load that this wave waits for: its loads and stores are counted
   // together, so it would wait for these stores (a value's elements lie in as many lines) as well.  That is behind the merge, or, where
-  // there is none, behind the keys, so that the stores are under way while the waves meet (1 sequence of 217 keys 6.55 -> 6.30 us; with a
+  // there is none, behind the keys, so that the stores are under way while the waves meet (217 keys as one run 6.55 -> 6.30 us; with a
   // merge to come 8 of 300 keys 8.4 -> 8.6).
   auto write_pages = [&]() {
     if constexpr (PREPARE) {

@@ -21,10 +21,9 @@
 // memory channel is hot), nor do four stages instead of three, nor loads that go out one by one between the MFMAs; without loads that product
 // takes 25 of its 41.5 us, with lines that the L2 holds 34.  From 1,500 rows on tiles of 256 x 256 (gemm_big.hip) and the matrix library are ahead.
 //
-// Tiles of 96 rows stand between those of 64 and 128: they are the ones that fill a round with the fewest bytes where 64 make too
-// many blocks and 128 too few (361 rows: 3,072 columns of gate/up, K = 1,024, 256 blocks of 96 x 96, 14.4 -> 12.0 us, 4,096 x 1,024
-// stored in 96 x 64 9.8 -> 8.9, 2,048 x 6,144 in parts in 96 x 128 22.6 -> 18.5; 80 rows: gate/up of 9,728 x 2,560, the library and
-// the gate kernel before, 35.0 -> 26.0).
+// Tiles of 96 rows (gemm_lds96.hip) stand between those of 64 and 128: they are the ones that fill a round with the fewest bytes where 64 make
+// too many blocks and 128 too few (361 rows: 3,072 columns of gate/up, K = 1,024, 256 blocks of 96 x 96, 14.4 -> 12.0 us, 4,096 x 1,024
+// stored in 96 x 64 9.8 -> 8.9, 2,048 x 6,144 in four parts in 96 x 128 22.6 -> 18.5).
 //
 // Up to 16 rows of x, tiles of 16 rows with one fragment a wave: the weight's bytes are nearly all of the tile's, so the widths
 // (16 to 80 weight rows) only choose how evenly the CUs share them, and 8 to 12 stages keep 64 KB and more of a CU's share in
